@@ -7,17 +7,16 @@
 // 68,76-80) and the tied head (mlx_lm/models/gpt2.py:167).
 //
 // Two kernels:
-//  * gemm_bf16_tile: 128x128x64 block tile, 4 waves in 2x2, each wave a 64x64
-//    tile of four v_mfma_f32_32x32x16_bf16 accumulators (or 256x256x64 with 8
-//    waves); two k-blocks in LDS, two more in registers; each die gets a run
-//    of neighbouring tiles that share their operands in its L2; K may be
-//    split over blocks where rows are few.  Any M, N; K % 8 == 0.
+//  * gemm_bf16_tile: block tiles of 32 x 128 to 256 x 256 outputs, k-blocks of 64 columns
+//    copied from memory straight into a ring in LDS, several ahead; waves of 32 x 32
+//    v_mfma_f32_32x32x16_bf16 tiles; each die gets a run of neighbouring tiles that share
+//    their operands in its L2; K may be split over blocks where rows are few.  Any M, N; K % 8 == 0.
 //  * gemm_bf16_skinny: M <= 64 rows (decode).  A block of four waves owns 16
 //    output features and splits K among its waves; W streams from HBM once
 //    as the MFMA A-operand, the activations are the B-operand.
 #include "common.h"
+#include "lds_copy.h"
 
-#include <algorithm>
 #include <type_traits>
 
 #define FLAG_GELU FLAG_ACT_GELU
@@ -27,9 +26,9 @@
 #define FLAG_KV 8  // columns from q_width on are keys, then values: they go to their cache pages, not to out
 #define FLAG_THROUGH 16  // (set here) out and ws are below 4 GB: the tile kernels' stores go through to memory
 
-// Out-of-range loads read a clamped address and are zeroed afterwards with this
-// constant: selecting between an address and a zero kept in a variable turns
-// the load into a flat load through scratch memory.
+// Out-of-range loads (of the kernel for few rows) read a clamped address and are zeroed afterwards
+// with this constant: selecting between an address and a zero kept in a variable turns the load
+// into a flat load through scratch memory.
 #define ZERO4 make_uint4(0u, 0u, 0u, 0u)
 
 struct GemmArgs {
@@ -40,7 +39,7 @@ struct GemmArgs {
   int M, N, K;
   int lda, ldw, ldo;
   int flags;
-  // K split over blockIdx.y (tile kernel, 128 x 128): partial sums [n_splits][M][N] go to ws
+  // K split over blockIdx.y (tiles 128 columns wide): partial sums [n_splits][M][N] go to ws
   float* ws;
   int n_splits, blocks_per_split;
   // key/value scatter (FLAG_KV): row m is token m of the step, at positions[m] of request token_req[m]
@@ -94,15 +93,7 @@ __device__ __forceinline__ void store_out(const GemmArgs& p, int m, int n, float
 
 // ---------------------------------------------------------------------------
 
-// Rows of a tile beyond the matrix read some row inside it (what they give is
-// never stored), and not all the same one: a tile of which only a few rows
-// exist would read that one row from hundreds of lanes at once, as would every
-// block of that row of tiles, and the cache channel that holds it serves them
-// one after another (a step of 2,056 rows took half as long again as one of 2,048).
-__device__ __forceinline__ int row_inside(int r, int n) { return r < n ? r : r % n; }
-
 #define BK 64
-#define LDS_STRIDE (BK + 8)  // 144 bytes a row: 16-byte reads of 16 rows hit distinct banks
 
 // Which tile a block works on.  Blocks go to the eight dies (each with an L2 of
 // its own) in turn, so block b runs on die b % 8.  The tiles are put in an
@@ -127,53 +118,51 @@ __device__ __forceinline__ bool tile_of_block(int tiles_m, int tiles_n, int& tm,
   return true;
 }
 
-// The shape of a block: WAVES_M x WAVES_N waves, each with TM x TN MFMA tiles of
-// 32 x 32.  What bounds this kernel is how fast a CU is fed from the L2s, so
-// the larger the block's tile, the fewer bytes per product: 128 x 128 (two
-// blocks a CU) where the matrix gives few tiles, 256 x 256 (one block a CU,
-// half the bytes) where it gives enough of them.
-template <int WAVES_M_, int WAVES_N_, int TM_, int TN_, int PANEL_, int BLOCKS_PER_CU_>
+// The shape of a block: WAVES_M x WAVES_N waves, each with TM x TN MFMA tiles of 32 x 32, and a ring of STAGES k-blocks
+// in LDS.  What bounds this kernel is how fast a CU is fed from the L2s (some 32 to 39 bytes a cycle arrive, measured with
+// the products taken out), so the larger the tile, the fewer bytes per product: 256 x 256 where the matrix gives a tile
+// to every CU, smaller ones where it does not; `price` below chooses.  Eight waves (but for 32 rows): two a SIMD cover each
+// other's waits for LDS; four waves of 64 x 64 were level or up to 12 % behind.
+template <int WAVES_M_, int WAVES_N_, int TM_, int TN_, int STAGES_, int PANEL_, int WAVES_PER_SIMD_>
 struct TileShape {
-  static constexpr int WAVES_M = WAVES_M_, WAVES_N = WAVES_N_, TM = TM_, TN = TN_;
-  static constexpr int PANEL = PANEL_, BLOCKS_PER_CU = BLOCKS_PER_CU_;  // PANEL: rows of tiles that share a die's L2
-  static constexpr int THREADS = 64 * WAVES_M * WAVES_N;
+  static constexpr int WAVES_M = WAVES_M_, WAVES_N = WAVES_N_, TM = TM_, TN = TN_, STAGES = STAGES_;
+  static constexpr int PANEL = PANEL_, WAVES_PER_SIMD = WAVES_PER_SIMD_;  // PANEL: rows of tiles that share a die's L2
+  static constexpr int WAVES = WAVES_M * WAVES_N, THREADS = 64 * WAVES;
   static constexpr int BM = WAVES_M * TM * 32, BN = WAVES_N * TN * 32;
-  static constexpr int PA = BM * 8 / THREADS, PB = BN * 8 / THREADS;  // 16-byte pieces a thread moves per k-block
-  static constexpr int ROW_STEP = THREADS / 8;                          // rows between a thread's pieces
+  static constexpr int PA = BM / 8 / WAVES, PB = BN / 8 / WAVES;  // copies of 1 KB a wave asks for per k-block
+  static constexpr int COPIES = PA + PB;
+  static constexpr int STAGE_BYTES = (BM + BN) * BK * 2;
+  static_assert(BM % (8 * WAVES) == 0 && BN % (8 * WAVES) == 0, "a wave copies whole kilobytes");
+  static_assert(STAGES * STAGE_BYTES <= 160 * 1024, "the ring fits a CU's LDS");
 };
-using Tile128 = TileShape<2, 2, 2, 2, 8, 2>;
-using Tile256 = TileShape<2, 4, 4, 2, 4, 1>;
-using Tile256x192 = TileShape<4, 2, 2, 3, 4, 1>;
-using Tile64x128 = TileShape<1, 4, 2, 1, 8, 2>;
-using Tile32x128 = TileShape<1, 4, 1, 1, 8, 2>;
-using Tile128x8 = TileShape<2, 4, 2, 1, 8, 1>;  // the same tile with eight waves, for a block that has its CU alone
+using Tile256 = TileShape<2, 4, 4, 2, 2, 4, 2>;
+using Tile256x192 = TileShape<4, 2, 2, 3, 2, 4, 2>;
+using Tile256x128 = TileShape<4, 2, 2, 2, 3, 4, 2>;
+using Tile128 = TileShape<2, 4, 2, 1, 4, 8, 2>;
+using Tile64x128 = TileShape<2, 4, 1, 1, 3, 8, 4>;  // two blocks a CU, as the next
+using Tile32x128 = TileShape<1, 4, 1, 1, 4, 8, 2>;
 
-// Pipeline: LDS holds two k-blocks; registers hold two more on their way.  In
-// iteration i the loads of k-block i+2 are issued and k-block i is multiplied
-// out of LDS; between the MFMAs of its four steps k-block i+1 (loaded an
-// iteration ago) goes from registers to the other half of LDS, a quarter at a
-// time (all at the end, the LDS writes of all waves came in one burst with the
-// MFMA units idle: 8 % slower); one barrier an iteration.
+// Pipeline: k-block kb is multiplied out of one slot of the ring while those up to kb + STAGES - 1 are on their way into
+// the others (lds_copy.h); one wait by count and one barrier a k-block.  Nothing passes through registers but the operands,
+// which are read a quarter of a k-block (16 columns) ahead of their products: left to the compiler, each read stood next
+// to its product (2,048 x 4,800 x 1,600: 36.0 us, 34.0 read ahead; 8,000 x 1,600 x 6,400: 178.7 and 167.0).  Before, the k-blocks went through
+// registers into LDS two ahead: 42.6 and 192 us for these, 65 against 58.6 for 2,048 x 1,600 x 6,400, and where few
+// rows give few tiles, so that a tile's own walk is the time, 39.0 against 14.0 for 333 x 1,600 x 6,400 and 14.8 against
+// 7.1 for 333 x 1,600 x 1,600 (K in three parts; rows x features x K, weights from memory, on an MI355X).
 // SPLIT: K is shared out over blockIdx.y and the partial sums go to the workspace (a kernel of
 // its own, so that the unsplit one carries none of it).
-// PACKED: W lies in the decode kernels' packed order.  A wave's load is then half a tile of 16
-// features x 64 k, 1 KB of consecutive bytes: lane l gets the 8 values k = 16 (l / 16) + 8 h + 0..7
-// of feature l % 16, and load g of the block's BN / 8 covers feature block g / 2, half h = g % 2.
-// (Reading the packed order with the row-major kernel's lanes, eight pieces of one row to eight
-// neighbouring lanes, touched eight lines with every eight lanes: 14 % slower.)
+// PACKED: W lies in the decode kernels' packed order.
 template <typename S, bool SPLIT, bool PACKED>
-__global__ __launch_bounds__(S::THREADS, S::BLOCKS_PER_CU) void gemm_bf16_tile_kernel(GemmArgs p) {
-  constexpr int BM = S::BM, BN = S::BN, TM = S::TM, TN = S::TN, PA = S::PA, PB = S::PB;
+__global__ __launch_bounds__(S::THREADS, S::WAVES_PER_SIMD) void gemm_bf16_tile_kernel(GemmArgs p) {
+  constexpr int BM = S::BM, BN = S::BN, TM = S::TM, TN = S::TN, PA = S::PA, PB = S::PB, STAGES = S::STAGES;
   // (one buffer: the epilogue uses it again for the output tiles)
-  __shared__ __attribute__((aligned(16))) uint16_t smem[2 * (BM + BN) * LDS_STRIDE];
-  uint16_t* const As[2] = {smem, smem + BM * LDS_STRIDE};
-  uint16_t* const Bs[2] = {smem + 2 * BM * LDS_STRIDE, smem + (2 * BM + BN) * LDS_STRIDE};
+  __shared__ __attribute__((aligned(1024))) uint16_t smem[STAGES * S::STAGE_BYTES / 2];
 
   int tm, tn;
   if (!tile_of_block<S::PANEL>((p.M + BM - 1) / BM, (p.N + BN - 1) / BN, tm, tn)) return;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
-  const int wave = tid >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / S::WAVES_N, wn = wave % S::WAVES_N;
   const int m0 = tm * BM;
   const int n0 = tn * BN;
@@ -186,72 +175,56 @@ __global__ __launch_bounds__(S::THREADS, S::BLOCKS_PER_CU) void gemm_bf16_tile_k
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
 
-  // each thread moves PA 16-byte pieces of A and PB of W per k-block: piece c
-  // is row c / 8, columns (c % 8) * 8 ..; rows beyond the matrix read rows
-  // inside it (their products land in rows or columns that are never stored)
-  // (32-bit element offsets and one LDS offset: registers are scarce here)
-  constexpr int ROW_STEP = S::ROW_STEP;
-  int a_off[PA], b_off[PB];
-  const int lds_off0 = (tid >> 3) * LDS_STRIDE + (tid & 7) * 8;  // piece i lies ROW_STEP rows further down
-#pragma unroll
-  for (int i = 0; i < PA; ++i) a_off[i] = row_inside(m0 + (tid >> 3) + ROW_STEP * i, p.M) * p.lda + (tid & 7) * 8;
-  // (packed weights: a k-block further on is 1024 elements further on, not 64)
-  constexpr int wmul = PACKED ? 16 : 1;
-  int lds_b[PB];  // where the thread's pieces of W go in a stage of LDS
-#pragma unroll
-  for (int i = 0; i < PB; ++i) {
-    if constexpr (PACKED) {
-      const int g = wave * PB + i, fb = g >> 1, h = g & 1;
-      const int nb = min(n0 / 16 + fb, (p.N + 15) / 16 - 1);  // (blocks beyond the matrix read its last one)
-      b_off[i] = nb * p.w_kblocks * 1024 + h * 512 + lane * 8;
-      lds_b[i] = (fb * 16 + (lane & 15)) * LDS_STRIDE + (2 * (lane >> 4) + h) * 8;
-    } else {
-      b_off[i] = row_inside(n0 + (tid >> 3) + ROW_STEP * i, p.N) * p.ldw + (tid & 7) * 8;
-      lds_b[i] = lds_off0 + i * ROW_STEP * LDS_STRIDE;
-    }
-  }
-  const int kc_mine = (tid & 7) * 8;
-  // this split's k-blocks (all of them without a split); the offsets start at its first column
+  // this split's k-blocks (all of them without a split)
   const int kb_lo = SPLIT ? blockIdx.y * p.blocks_per_split : 0;
   const int n_blocks = SPLIT ? min((p.K + BK - 1) / BK, kb_lo + p.blocks_per_split) - kb_lo : (p.K + BK - 1) / BK;
-  const int k_lo = kb_lo * BK;
-  if constexpr (SPLIT) {
+
+  // What this wave copies: rows of 128 bytes, eight of them a copy.  Row r's piece s of 16 bytes in LDS is piece
+  // s ^ (r / 2 % 8) of the row in memory, so that lanes which read one piece of sixteen neighbouring rows meet sixteen
+  // different groups of banks (s ^ (r % 8), which gives only eight, made a read take twice as long).  Packed weights need none of that: half a tile of 16 features x 64 k is a copy as it lies, and
+  // sixteen lanes read 256 bytes in a row.  Rows beyond the matrix lie beyond the buffer's end, columns beyond K are
+  // sent there.
+  const i32x4_t a_buf = copy_buffer(p.A, ((size_t)(p.M - 1) * p.lda + p.K) * 2);
+  const i32x4_t b_buf = copy_buffer(p.W, PACKED ? (size_t)((p.N + 15) / 16) * p.w_kblocks * 2048
+                                                : ((size_t)(p.N - 1) * p.ldw + p.K) * 2);
+  const int row8 = lane >> 3;
+  auto piece_of = [&](int copy) __attribute__((always_inline)) { return (lane & 7) ^ ((copy & 1) * 4 + (row8 >> 1)); };
+  uint32_t a_from[PA], b_from[PB];
 #pragma unroll
-    for (int i = 0; i < PA; ++i) a_off[i] += k_lo;
-#pragma unroll
-    for (int i = 0; i < PB; ++i) b_off[i] += k_lo * wmul;
+  for (int i = 0; i < PA; ++i) {
+    const int row = m0 + (wave * PA + i) * 8 + row8;
+    a_from[i] = row < p.M ? (uint32_t)(((size_t)row * p.lda + piece_of(wave * PA + i) * 8) * 2) : COPY_NOTHING;
   }
-
-  uint4 ra[2][PA], rb[2][PB];
-  auto load_global = [&](uint4 (&xa)[PA], uint4 (&xb)[PB], int k0) {
-    // a piece beyond K is read from the row's last eight columns instead (K may be
-    // smaller than a k-block, so no earlier k-block is sure to hold this piece's
-    // columns) and zeroed when it goes to LDS: zeroing it here would make the
-    // loads wait at once
-    const int kk = (k_lo + k0 + kc_mine < p.K) ? k0 : p.K - 8 - kc_mine - k_lo;
-    const int kw = PACKED ? k0 * 16 : kk;  // (packed weights are padded with zeros to whole k-blocks)
 #pragma unroll
-    for (int i = 0; i < PA; ++i) xa[i] = *(const uint4*)(p.A + a_off[i] + kk);
+  for (int i = 0; i < PB; ++i) {
+    const int g = wave * PB + i;
+    if constexpr (PACKED) {
+      const int fb = n0 / 16 + (g >> 1);
+      b_from[i] = fb < (p.N + 15) / 16 ? (uint32_t)(((size_t)fb * p.w_kblocks * 1024 + (g & 1) * 512 + lane * 8) * 2) : COPY_NOTHING;
+    } else {
+      const int row = n0 + g * 8 + row8;
+      b_from[i] = row < p.N ? (uint32_t)(((size_t)row * p.ldw + piece_of(g) * 8) * 2) : COPY_NOTHING;
+    }
+  }
+  const uint32_t ring = lds_address(smem);
+  const uint32_t a_to = ring + wave * PA * 1024, b_to = ring + BM * BK * 2 + wave * PB * 1024;
+  // (k-blocks beyond the last are asked for too, as nothing: the waits then count the same copies in every round)
+  auto ask = [&](int kb, int slot) __attribute__((always_inline)) {
+    const bool live = kb < n_blocks;
+    const int k_left = live ? p.K - (kb_lo + kb) * BK : 0;  // columns from this k-block on
+    const uint32_t at = (uint32_t)slot * S::STAGE_BYTES;
+    const uint32_t k2 = (uint32_t)(kb_lo + kb) * (BK * 2), w2 = PACKED ? k2 * 16 : k2;
 #pragma unroll
-    for (int i = 0; i < PB; ++i) xb[i] = *(const uint4*)(p.W + b_off[i] + kw);
+    for (int i = 0; i < PA; ++i) copy16_to_lds(a_buf, piece_of(wave * PA + i) * 8 < k_left ? a_from[i] : COPY_NOTHING, k2, a_to + at + i * 1024);
+#pragma unroll
+    for (int i = 0; i < PB; ++i) 
+      copy16_to_lds(b_buf, (PACKED ? live : piece_of(wave * PB + i) * 8 < k_left) ? b_from[i] : COPY_NOTHING, w2, b_to + at + i * 1024);
   };
-  auto store_lds = [&](int stage, const uint4 (&xa)[PA], const uint4 (&xb)[PB], int k0) {
-    const bool in = k_lo + k0 + kc_mine < p.K;
-#pragma unroll
-    for (int i = 0; i < PA; ++i) *(uint4*)(As[stage] + lds_off0 + i * ROW_STEP * LDS_STRIDE) = in ? xa[i] : ZERO4;
-#pragma unroll
-    for (int i = 0; i < PB; ++i) *(uint4*)(Bs[stage] + lds_b[i]) = (PACKED || in) ? xb[i] : ZERO4;
-  };
 
-  load_global(ra[0], rb[0], 0);
-  if (n_blocks > 1) load_global(ra[1], rb[1], BK);
-  store_lds(0, ra[0], rb[0], 0);
-  __syncthreads();
-
-  const int frag_row = lane & 31;
-  const int frag_k = (lane >> 5) * 8;
-  const uint16_t* a_frag = As[0] + (wm * TM * 32 + frag_row) * LDS_STRIDE + frag_k;
-  const uint16_t* b_frag = Bs[0] + (wn * TN * 32 + frag_row) * LDS_STRIDE + frag_k;
+  const int row32 = lane & 31, hi = lane >> 5;
+  const char* const a_row = (const char*)smem + (wm * TM * 32 + row32) * 128;
+  const char* const b_row = (const char*)smem + BM * BK * 2 +
+                            (PACKED ? ((wn * TN * 2 + (row32 >> 4)) * 2 + hi) * 1024 + (row32 & 15) * 16 : (wn * TN * 32 + row32) * 128);
 
   // Without a split the tiles are accumulated transposed (the weights' rows as the MFMA's rows):
   // a lane then holds four neighbouring columns of one output row, which the epilogue wants.
@@ -261,84 +234,46 @@ __global__ __launch_bounds__(S::THREADS, S::BLOCKS_PER_CU) void gemm_bf16_tile_k
     else
       return __builtin_amdgcn_mfma_f32_32x32x16_bf16(b, a, c, 0, 0, 0);
   };
-  auto multiply = [&](int stage) {
-    const uint16_t* af = a_frag + stage * (BM * LDS_STRIDE);
-    const uint16_t* bf = b_frag + stage * (BN * LDS_STRIDE);
+  // The operands of 16 columns (a quarter of a k-block) go to registers one quarter ahead of their products, also
+  // across the barrier: a k-block's last quarter is multiplied after the barrier that lets the next one be read.
+  bf16x8_t fa[2][TM], fb[2][TN];
+  auto read_quarter = [&](int set, int slot, int q) __attribute__((always_inline)) {
+    const char* af = a_row + slot * S::STAGE_BYTES;
+    const char* bf = b_row + slot * S::STAGE_BYTES;
+    const int s = ((2 * q + hi) ^ ((row32 >> 1) & 7)) * 16;
 #pragma unroll
-    for (int ks = 0; ks < BK; ks += 16) {
-      bf16x8_t a[TM], b[TN];
+    for (int i = 0; i < TM; ++i) fa[set][i] = *(const bf16x8_t*)(af + i * 32 * 128 + s);
 #pragma unroll
-      for (int i = 0; i < TM; ++i) a[i] = *(const bf16x8_t*)(af + i * 32 * LDS_STRIDE + ks);
+    for (int j = 0; j < TN; ++j) fb[set][j] = *(const bf16x8_t*)(PACKED ? bf + j * 4096 + q * 256 : bf + j * 32 * 128 + s);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto multiply = [&](int set) __attribute__((always_inline)) {
 #pragma unroll
-      for (int j = 0; j < TN; ++j) b[j] = *(const bf16x8_t*)(bf + j * 32 * LDS_STRIDE + ks);
+    for (int i = 0; i < TM; ++i)
 #pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-          acc[i][j] = mfma_tile(a[i], b[j], acc[i][j]);
-    }
+      for (int j = 0; j < TN; ++j) acc[i][j] = mfma_tile(fa[set][i], fb[set][j], acc[i][j]);
+    __builtin_amdgcn_sched_barrier(0);
   };
 
-  // Two k-blocks an iteration, so that the register sets are named statically.
-  // The steady part has no branch and no select inside: only then does the
-  // compiler count exactly how many loads may stay in flight at each wait
-  // (a conditional load makes it wait for all of them).
-  auto load_whole = [&](uint4 (&xa)[PA], uint4 (&xb)[PB], int k0) {  // a k-block that lies inside K
 #pragma unroll
-    for (int i = 0; i < PA; ++i) xa[i] = *(const uint4*)(p.A + a_off[i] + k0);
-#pragma unroll
-    for (int i = 0; i < PB; ++i) xb[i] = *(const uint4*)(p.W + b_off[i] + k0 * wmul);
-  };
-  // multiply out of `stage` and, a quarter with each 16 columns, move the next k-block (in
-  // registers since the iteration before) into the other stage, which nobody reads any more
-  auto multiply_store = [&](int stage, const uint4 (&xa)[PA], const uint4 (&xb)[PB]) {
-    const uint16_t* af = a_frag + stage * (BM * LDS_STRIDE);
-    const uint16_t* bf = b_frag + stage * (BN * LDS_STRIDE);
-    uint16_t* an = As[stage ^ 1] + lds_off0;
-    uint16_t* bn = Bs[stage ^ 1];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int ks = q * 16;
-      bf16x8_t a[TM], b[TN];
-#pragma unroll
-      for (int i = 0; i < TM; ++i) a[i] = *(const bf16x8_t*)(af + i * 32 * LDS_STRIDE + ks);
-#pragma unroll
-      for (int j = 0; j < TN; ++j) b[j] = *(const bf16x8_t*)(bf + j * 32 * LDS_STRIDE + ks);
-#pragma unroll
-      for (int i = q * PA / 4; i < (q + 1) * PA / 4; ++i) *(uint4*)(an + i * ROW_STEP * LDS_STRIDE) = xa[i];
-#pragma unroll
-      for (int i = q * PB / 4; i < (q + 1) * PB / 4; ++i) *(uint4*)(bn + lds_b[i]) = xb[i];
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-          acc[i][j] = mfma_tile(a[i], b[j], acc[i][j]);
-    }
-  };
-  int kb = 0;
-  const int whole_blocks = SPLIT ? min(n_blocks, p.K / BK - kb_lo) : p.K / BK;  // k-blocks that need no masking
-  for (; kb + 4 <= whole_blocks; kb += 2) {
-    load_whole(ra[0], rb[0], (kb + 2) * BK);
-    __builtin_amdgcn_sched_barrier(0);  // the loads go out before the arithmetic, not after it
-    multiply_store(0, ra[1], rb[1]);
-    __syncthreads();
-    load_whole(ra[1], rb[1], (kb + 3) * BK);
-    __builtin_amdgcn_sched_barrier(0);
-    multiply_store(1, ra[0], rb[0]);
-    __syncthreads();
-  }
-  // the last few k-blocks, with every guard
-  for (; kb < n_blocks; kb += 2) {
-    if (kb + 2 < n_blocks) load_global(ra[0], rb[0], (kb + 2) * BK);
+  for (int s = 0; s < STAGES - 1; ++s) ask(s, s);
+  int slot = 0;
+  for (int kb = 0; kb < n_blocks; ++kb) {
+    copies_arrived<(STAGES - 2) * S::COPIES>();
+    ring_barrier();  // k-block kb is whole, and nobody reads the slot of k-block kb - 1 any more
+    read_quarter(0, slot, 0);
+    ask(kb + STAGES - 1, slot == 0 ? STAGES - 1 : slot - 1);
+    if (kb > 0) multiply(1);
+    read_quarter(1, slot, 1);
     multiply(0);
-    if (kb + 1 < n_blocks) store_lds(1, ra[1], rb[1], (kb + 1) * BK);
-    __syncthreads();
-    if (kb + 1 >= n_blocks) break;
-    if (kb + 3 < n_blocks) load_global(ra[1], rb[1], (kb + 3) * BK);
+    read_quarter(0, slot, 2);
     multiply(1);
-    if (kb + 2 < n_blocks) store_lds(0, ra[0], rb[0], (kb + 2) * BK);
-    __syncthreads();
+    read_quarter(1, slot, 3);
+    multiply(0);
+    slot = slot == STAGES - 1 ? 0 : slot + 1;
   }
+  multiply(1);
+  copies_arrived<0>();  // (what was asked for beyond the end: the epilogue writes where it goes)
 
   if constexpr (SPLIT) {  // the partial sums as they are; sum_partials adds them and runs the epilogue
     float* ws = p.ws + (size_t)blockIdx.y * p.M * p.N;
@@ -520,11 +455,9 @@ __global__ __launch_bounds__(S::THREADS, S::BLOCKS_PER_CU) void gemm_bf16_tile_k
 
 #define SK_WAVES 4
 #define SK_MAXM 64
-// From 17 rows on this file's kernels take the product: tiles of 32 x 128 up to 32 rows and of
-// 64 x 128 up to 64 (and beyond where 128 x 128 tiles would be few), with K split over blocks
-// where the tiles alone do not fill the GPU.  (A kernel that streamed the weights once for 17 to
-// 64 rows, 64 features a block, was 3 to 17 % slower than these at GPT-2 XL's projections and
-// twice as slow at the vocabulary's head.)
+// From 17 rows on the tile kernel takes the product, with K split over blocks where the tiles alone
+// do not fill the GPU.  (A kernel that streamed the weights once for 17 to 64 rows, 64 features a
+// block, was 3 to 17 % slower at GPT-2 XL's projections and twice as slow at the vocabulary's head.)
 #define TILE_MIN_ROWS 17
 
 template <int MT>  // number of 16-row groups of activations (1..4)
@@ -619,107 +552,96 @@ static int check_args(const GemmArgs& p) {
   return 0;
 }
 
-template <typename S>
+template <typename S, bool CAN_SPLIT>
 static void launch_tiles(const GemmArgs& p, hipStream_t stream) {
   const long tiles = (long)((p.M + S::BM - 1) / S::BM) * ((p.N + S::BN - 1) / S::BN);
   dim3 grid((unsigned)((tiles + 7) / 8 * 8), p.n_splits), block(S::THREADS);  // a run of tiles for each die
-  if (p.n_splits > 1) {
-    if (p.w_packed)
-      hipLaunchKernelGGL((gemm_bf16_tile_kernel<S, true, true>), grid, block, 0, stream, p);
-    else
-      hipLaunchKernelGGL((gemm_bf16_tile_kernel<S, true, false>), grid, block, 0, stream, p);
-  } else {
-    if (p.w_packed)
-      hipLaunchKernelGGL((gemm_bf16_tile_kernel<S, false, true>), grid, block, 0, stream, p);
-    else
-      hipLaunchKernelGGL((gemm_bf16_tile_kernel<S, false, false>), grid, block, 0, stream, p);
+  if constexpr (CAN_SPLIT) {
+    if (p.n_splits > 1) {
+      if (p.w_packed)
+        hipLaunchKernelGGL((gemm_bf16_tile_kernel<S, true, true>), grid, block, 0, stream, p);
+      else
+        hipLaunchKernelGGL((gemm_bf16_tile_kernel<S, true, false>), grid, block, 0, stream, p);
+      return;
+    }
   }
+  if (p.w_packed)
+    hipLaunchKernelGGL((gemm_bf16_tile_kernel<S, false, true>), grid, block, 0, stream, p);
+  else
+    hipLaunchKernelGGL((gemm_bf16_tile_kernel<S, false, false>), grid, block, 0, stream, p);
 }
 
-// How many tiles a die gets (tile_of_block shares them out evenly).
-template <typename S>
-static int busiest_die(int M, int N) {
-  const long tiles = (long)((M + S::BM - 1) / S::BM) * ((N + S::BN - 1) / S::BN);
-  return (int)((tiles + 7) / 8);
+// What a shape costs, in microseconds: `tile` for each round of tiles on a CU and `kblock` for each k-block of it, `pair`
+// a k-block where two blocks share the CU (shapes that fit twice), `launch` once.  Fitted to the times of 16 numbers of
+// rows from 20 to 8,000 against 18 matrices of widths from 768 to 2,048, K up to 6,400, each with K in 1 to 8 parts; the
+// shape and parts chosen from these prices are within 1 % of the best on average (at worst 1.3 times: 20 to 64 rows to
+// 10,880 features, which only one kind of design asks of these kernels).
+struct TilePrice {
+  int variant, bm, bn, per_cu;
+  double launch, tile, kblock, pair;
+  bool splits;  // K may be split over blocks
+};
+static const TilePrice TILE_PRICES[] = {
+    {3, Tile256::BM, Tile256::BN, 1, 0.0, 7.78, 1.39, 0.0, false},
+    {4, Tile256x192::BM, Tile256x192::BN, 1, 0.0, 7.26, 1.17, 0.0, false},
+    {8, Tile256x128::BM, Tile256x128::BN, 1, 0.0, 7.6, 0.7, 0.0, false},
+    {1, Tile128::BM, Tile128::BN, 1, 0.0, 4.33, 0.49, 0.0, true},
+    {5, Tile64x128::BM, Tile64x128::BN, 2, 0.52, 2.81, 0.41, 0.77, true},
+    {6, Tile32x128::BM, Tile32x128::BN, 2, 1.81, 1.98, 0.3, 0.52, true},
+};
+static double price(const TilePrice& s, int M, int N, int K, int n_splits) {
+  const long tiles = (long)((M + s.bm - 1) / s.bm) * ((N + s.bn - 1) / s.bn);
+  const int cus = n_compute_units();
+  // the busiest CU: of a die's run of tiles, or of all blocks where K is split
+  const long n = n_splits > 1 ? (tiles * n_splits + cus - 1) / cus
+                              : ((tiles + N_DIES - 1) / N_DIES + cus / N_DIES - 1) / (cus / N_DIES);
+  const int k_blocks = ((K + BK - 1) / BK + n_splits - 1) / n_splits;
+  if (s.per_cu == 1) return s.launch + n * (s.tile + k_blocks * s.kblock);
+  return s.launch + (n / 2) * (s.tile + k_blocks * s.pair) + (n % 2) * (s.tile + k_blocks * s.kblock);
 }
-
-// Microseconds per k-block of the busiest die, from what was measured at GPT-2 XL
-// sizes: two 128 x 128 blocks on a CU finish a k-block each in 1.15 us, one
-// alone in 1.3 us (its fetching and its arithmetic take turns; two blocks
-// overlap each other's), a 256 x 256 block (four times the work) in 2.0 us.  A
-// die has 32 CUs.
-static double cost_128(int M, int N) {
-  const int per_die = n_compute_units() / N_DIES;  // CUs of a die: two of these blocks fit each
-  const int tiles = busiest_die<Tile128>(M, N);
-  const int rest = tiles % (2 * per_die);
-  // (a last round of few blocks finds the L2 idle: 1.0)
-  return (double)(tiles / (2 * per_die)) * 1.15 +
-         (rest == 0 ? 0.0 : rest <= per_die / 2 ? 1.0 : rest <= per_die ? 1.3 : 1.15);
-}
-static double cost_256(int M, int N) {
-  const int per_die = n_compute_units() / N_DIES;
-  return (double)((busiest_die<Tile256>(M, N) + per_die - 1) / per_die) * 2.0;
-}
-// (256 x 192: three quarters of the arithmetic, seven eighths of the bytes; its tiles fit N = 4800)
-static double cost_256x192(int M, int N) {
-  const int per_die = n_compute_units() / N_DIES;
-  return (double)((busiest_die<Tile256x192>(M, N) + per_die - 1) / per_die) * 1.6;
-}
-
-// Tiles of 64 x 128 instead of 128 x 128 where the latter would be few (up to 128): twice the
-// blocks, each with half the arithmetic and three quarters of the bytes.  Measured at widths
-// from 768 to 2,048: ahead by up to a quarter while the 128 x 128 tiles leave half the CUs idle,
-// level at 144 tiles, behind from 160 on (2,048 rows of a projection to 1,280 features with
-// K = 5,120: 59 us against 51), where what the tiles fetch from the L2s counts for more.
-static bool small_tiles(int M, int N) { return (long)((M + 127) / 128) * ((N + 127) / 128) <= 128; }
-
-// Microseconds a CU takes per k-block when it holds `n` blocks of tiles `rows` x 128 (measured at
-// widths 768 to 2,048): a block alone waits for its fetches most of the time, so a second block
-// on the CU costs little; from the third on they take turns.
-static double kblock_us(int rows, int n) {
-  const double alone = rows <= 32 ? 0.37 : rows <= 64 ? 0.52 : 0.62;
-  const double pair = rows <= 32 ? 0.56 : rows <= 64 ? 0.80 : 1.14;
-  return (n / 2) * pair + (n % 2) * alone;
+// The cheapest shape for K in so many parts, and its price.
+static int cheapest_shape(int M, int N, int K, int n_splits, double* us) {
+  int variant = 0;
+  for (const TilePrice& s : TILE_PRICES) {
+    if (n_splits > 1 && !s.splits) continue;
+    const double t = price(s, M, N, K, n_splits);
+    if (!variant || t < *us) variant = s.variant, *us = t;
+  }
+  return variant;
 }
 
 // Into how many parts the kernels with tiles 128 wide should split K (1: no split).  Few rows
 // give few tiles (up to 128 rows of GPT-2 XL's projections are 13 to 50 tiles for 256 CUs), and a
 // tile's walk through K takes the same time whether 50 or 500 of them run; a split shortens the
 // walk and costs a second kernel that reads the partial sums ([parts][M][N] floats).  Both sides
-// are priced from what was measured (65 to 768 rows, widths 768 to 2,048, K up to 8,192): the walk
-// as k-blocks times the time per k-block of the busiest CU, the second kernel as a launch plus
-// its bytes at 3 TB/s.  `fused`: the second kernel stands in for one that would run anyway (the
-// norm that follows a sum into the residual stream, the write of keys and values into their
-// pages), so it costs only the extra bytes.  A part keeps three k-blocks or more.
+// are priced: the walk as above, the second kernel as a launch plus its bytes at 3 TB/s.
+// `fused`: the second kernel stands in for one that would run anyway (the norm that follows a
+// sum into the residual stream, the write of keys and values into their pages), so it costs only
+// the extra bytes.  A part keeps three k-blocks or more, and more parts have to be 5 % cheaper
+// (with no such margin the choices were 0.4 % further from the best).
 // `force` > 0 asks for that many parts wherever K has them (for tests of small sizes).
 extern "C" int gemm_bf16_splits(int M, int N, int K, int fused, int force) {
   if (M < TILE_MIN_ROWS) return 1;
-  const long cols = (N + 127) / 128;
-  const int rows = M <= 32 ? 32 : small_tiles(M, N) ? 64 : 128;
-  const long tiles = (long)((M + rows - 1) / rows) * cols;
   const int n_blocks = (K + BK - 1) / BK;
   int best = 1;
   if (force > 0) {
     best = force < n_blocks ? force : n_blocks;
   } else {
-    double best_us = 0.0, whole_us = 0.0;
+    double best_us = 0.0;
     for (int s = 1; s <= 16 && s <= (n_blocks >= 3 ? n_blocks / 3 : 1); ++s) {
-      const int per = (n_blocks + s - 1) / s;
-      const int on_cu = (int)((tiles * s + n_compute_units() - 1) / n_compute_units());
-      double us = kblock_us(rows, on_cu) * per;
+      double us = 0.0;
+      cheapest_shape(M, N, K, s, &us);
       if (s > 1) us += (fused ? 1.0 : 2.5) + 8.0 * (fused ? s - 1 : s) * (double)M * N / 3e6;
-      if (s == 1) whole_us = us;
-      if (s == 1 || us < best_us) best = s, best_us = us;
+      if (s == 1 || us < 0.95 * best_us) best = s, best_us = us;
     }
-    if (best_us > 0.9 * whole_us) best = 1;  // (the prices are good to a tenth)
   }
   if (best <= 1) return 1;
   const int per = (n_blocks + best - 1) / best;
   return (n_blocks + per - 1) / per;  // no empty part
 }
 
-// variant: 0 = choose, 1 = 128 x 128 tiles, 2 = skinny kernel, 3 = 256 x 256 tiles, 4 = 256 x 192
-// tiles, 5 = 64 x 128 tiles, 6 = 32 x 128 tiles.  n_splits > 1 (variants 1, 5 and 6 only): no
+// variant: 0 = choose, 1 (and 7) = 128 x 128 tiles, 2 = skinny kernel, 3 = 256 x 256 tiles, 4 = 256 x 192
+// tiles, 5 = 64 x 128 tiles, 6 = 32 x 128 tiles, 8 = 256 x 128 tiles.  n_splits > 1 (variants 1, 5 and 6 only): no
 // epilogue, the partial sums go to ws.  ldw == 0: W is in the decode kernels' packed order
 // (tiles of 16 features x 64 k, zero padded), which all kernels here read as well as rows.
 extern "C" int gemm_bf16_scatter(void* out, const void* A, const void* W, const float* bias, int M, int N,
@@ -779,28 +701,18 @@ extern "C" int gemm_bf16_scatter(void* out, const void* A, const void* W, const 
   p.ws = ws, p.n_splits = n_splits, p.blocks_per_split = (n_blocks + n_splits - 1) / n_splits;
   if (fits_through_buffer((size_t)M * ldo * 4) && fits_through_buffer((size_t)M * N * 4)) p.flags |= FLAG_THROUGH;
   if (n_splits > 1) {
-    if (variant == 0) variant = M <= 32 ? 6 : small_tiles(M, N) ? 5 : 1;
+    double us = 0.0;
+    if (variant == 0) variant = cheapest_shape(M, N, K, n_splits, &us);
     if (variant != 1 && variant != 5 && variant != 6) FAIL("gemm_bf16: only the tiles of 128, 64 and 32 rows by 128 split K");
     if (p.blocks_per_split * (n_splits - 1) >= n_blocks) FAIL("gemm_bf16: %d splits of K=%d leave one empty", n_splits, K);
     if (!ws || ((uintptr_t)ws & 15) || ws_floats < (size_t)n_splits * M * N)
       FAIL("gemm_bf16: %d splits of %d x %d need an aligned workspace of that many floats", n_splits, M, N);
   }
   if (variant == 0) {
-    if (M < TILE_MIN_ROWS)
-      variant = 2;
-    else if (M <= 32)
-      variant = 6;
-    else if (M <= 64 || small_tiles(M, N))
-      variant = 5;
-    else {
-      const double c1 = cost_128(M, N), c3 = cost_256(M, N), c4 = cost_256x192(M, N);
-      variant = c4 < c3 && c4 < c1 ? 4 : c3 < c1 ? 3 : 1;
-      // No more tiles of 128 x 128 than CUs: a block alone on its CU hides more of its waits with eight
-      // waves of 64 x 32 than with four of 64 x 64 (2,048 rows to 1,600 features: 24.0 us against 26.4 at
-      // K = 1,600, 65.1 against 67.6 at 6,400; with two blocks a CU the four waves are level or ahead).
-      if (variant == 1 && n_splits == 1 && busiest_die<Tile128>(M, N) <= n_compute_units() / N_DIES) variant = 7;
-    }
+    double us = 0.0;
+    variant = M < TILE_MIN_ROWS ? 2 : cheapest_shape(M, N, K, 1, &us);
   }
+  if (variant == 7) variant = 1;
   if (variant == 2) {
     if (M > SK_MAXM) FAIL("gemm_bf16: the skinny kernel takes at most %d rows, got %d", SK_MAXM, M);
     dim3 grid((N + 15) / 16), block(256);
@@ -813,20 +725,18 @@ extern "C" int gemm_bf16_scatter(void* out, const void* A, const void* W, const 
       hipLaunchKernelGGL(gemm_bf16_skinny_kernel<3>, grid, block, 0, stream, p);
     else
       hipLaunchKernelGGL(gemm_bf16_skinny_kernel<4>, grid, block, 0, stream, p);
-  } else if (variant == 7) {
-    launch_tiles<Tile128x8>(p, stream);
-
-  } else if (variant == 1 || variant == 3 || variant == 4 || variant == 5 || variant == 6) {
-    if (variant == 1)
-      launch_tiles<Tile128>(p, stream);
-    else if (variant == 3)
-      launch_tiles<Tile256>(p, stream);
-    else if (variant == 4)
-      launch_tiles<Tile256x192>(p, stream);
-    else if (variant == 5)
-      launch_tiles<Tile64x128>(p, stream);
-    else
-      launch_tiles<Tile32x128>(p, stream);
+  } else if (variant == 1) {
+    launch_tiles<Tile128, true>(p, stream);
+  } else if (variant == 5) {
+    launch_tiles<Tile64x128, true>(p, stream);
+  } else if (variant == 6) {
+    launch_tiles<Tile32x128, true>(p, stream);
+  } else if (variant == 3) {
+    launch_tiles<Tile256, false>(p, stream);
+  } else if (variant == 4) {
+    launch_tiles<Tile256x192, false>(p, stream);
+  } else if (variant == 8) {
+    launch_tiles<Tile256x128, false>(p, stream);
   } else {
     FAIL("gemm_bf16: unknown variant %d", variant);
   }

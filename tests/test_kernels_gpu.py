@@ -885,6 +885,31 @@ def test_gemm_bf16_reads_weights_kept_in_packed_order_only(M, N, K):
         assert torch.allclose(outs[1].double().cpu(), plain.gelu_tanh(ref), rtol=2**-7, atol=1e-3), (variant, splits)
 
 
+@pytest.mark.parametrize("M,N,K", [(17, 16, 8), (129, 128, 64), (65, 130, 72), (255, 257, 192), (257, 120, 256), (31, 384, 328), (300, 200, 520)])
+@pytest.mark.parametrize("packed", [False, True])
+def test_gemm_bf16_tiles_at_the_ring_s_edges(M, N, K, packed):
+    """Tiles with a row or column more or less than whole ones, and K of fewer k-blocks than a tile's
+    ring has slots, as many, and more, whole or not.  What lies around the operands is NaN: rows,
+    columns and k-blocks that do not exist must come in as zeros.  (Sums of K products of bfloat16
+    values in 32 bits: K roundings of the largest partial sum at most, here against 64 bits.)"""
+    k = _k()
+    a_all = torch.full((M + 40, K + 24), float("nan"), dtype=torch.bfloat16, device=DEV)
+    w_all = torch.full((N + 40, K + 24), float("nan"), dtype=torch.bfloat16, device=DEV)
+    a, w = a_all[:M, :K], w_all[:N, :K]
+    a.copy_(_rand((M, K), torch.bfloat16, 10))
+    w.copy_(_rand((N, K), torch.bfloat16, 11, 0.1))
+    bias = _rand((N,), torch.float32, 12)
+    ref = plain.linear(a.double().cpu(), w.double().cpu(), bias.double().cpu())
+    tol = K * 2.0**-24 * (a.double().abs() @ w.double().abs().t()).max().item() + 1e-6
+    weights = k.PackedWeight(w.contiguous(), keep_rows=False) if packed else w
+    parts = [s for s in (2, 3) if s <= (K + 63) // 64]
+    for variant, splits in [(v, None) for v in (1, 3, 4, 5, 6, 8)] + [(v, s) for v in (1, 5, 6) for s in parts]:
+        out = torch.full((M, N), 7.0, dtype=torch.float32, device=DEV)
+        k.linear(out, a, weights, bias, variant=variant, splits=splits)
+        err = (out.double().cpu() - ref).abs().max().item()
+        assert err < tol, (variant, splits, err)
+
+
 @pytest.mark.parametrize("M,N,K", [(17, 48, 64), (33, 257, 384), (64, 4800, 1600), (40, 1600, 6400), (64, 333, 1608),
                                    (48, 80, 200), (20, 100, 520), (32, 4800, 1600), (24, 1600, 6400), (30, 333, 1608)])
 @pytest.mark.parametrize("mode", ["plain", "gelu", "accumulate", "f32out"])
