@@ -137,7 +137,7 @@ static Entry<fn_embed> k_embed("embed", "embed_scale_add");
 static Entry<fn_layernorm> k_layernorm("norm", "layernorm");
 static Entry<int (*)(void*, const float*, int, const int*, const float*, float, int, int, int, hipStream_t)> k_rmsnorm("rmsnorm", "rmsnorm");
 static Entry<fn_gemm_f32> k_gemm_f32("gemm_f32", "gemm_f32");
-static Entry<fn_int4> k_gemm_f32_splits("gemm_f32", "gemm_f32_splits");
+static Entry<fn_int5> k_gemm_f32_splits("gemm_f32", "gemm_f32_splits");
 static Entry<fn_gemm_bf16> k_gemm_bf16("gemm_bf16", "gemm_bf16_scatter");
 static Entry<fn_int5> k_gemm_bf16_splits("gemm_bf16", "gemm_bf16_splits");
 static Entry<fn_gemm_decode> k_gemm_decode("gemm_bf16_decode", "gemm_bf16_decode");
@@ -491,12 +491,13 @@ static int linear(EngCtx* ctx, const EngMat& out, const EngValue& a, const EngWe
     }
   }
   if (w.dtype == DT_F32) {
-    // Few rows of a narrow matrix give the kernel for them fewer blocks than there are compute
-    // units: K goes in parts then, and the same second kernels add them up as for bfloat16.
+    // Where a matrix gives fewer blocks than there are compute units, or a last round of few, K goes
+    // in parts, and the same second kernels add them up as for bfloat16.
     int n_splits = 1;
-    if ((variant == 0 || variant == 3) && M <= F32_FEW_ROWS) {
+    if (variant == 0 || (variant == 3 && M <= F32_FEW_ROWS) || splits != 0) {
+      const int fused = (accumulate && pending && pending->allowed) ? 1 : 0;
       if (splits == 0)
-        QUERY(k_gemm_f32_splits, n_splits, M, N, K, ctx->force_splits);
+        QUERY(k_gemm_f32_splits, n_splits, M, N, K, fused, ctx->force_splits);
       else
         n_splits = split_count((K + 63) / 64, splits);
       if (n_splits > 1) {

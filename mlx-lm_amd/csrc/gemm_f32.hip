@@ -13,6 +13,7 @@
 // without a block.  Where 16 features a block still give fewer blocks than
 // units, K goes in parts and a second kernel (the caller's) adds them up.
 #include "common.h"
+#include "lds_copy.h"
 
 #define FLAG_GELU FLAG_ACT_GELU
 #define FLAG_RELU2 FLAG_ACT_RELU2  // the square of the ReLU instead
@@ -26,128 +27,163 @@ struct GemmArgs {
   int M, N, K;
   int lda, ldw, ldo;
   int flags;
-  // the kernel for few rows: blockIdx.y takes part y of K's chunks and leaves its sums in
-  // ws[y][M][N], without bias or epilogue
-  int n_splits;
+  // blockIdx.y takes part y of K's chunks of 64 columns (`per_split` of them) and leaves its sums
+  // in ws[y][M][N], without bias or epilogue
+  int n_splits, per_split;
   float* ws;
 };
 
-// Rows of a tile beyond the matrix read a row inside it (their products are
-// never stored): the row one tile back where there is one, so that they do not
-// all read the matrix's last row at once, which one cache channel would have
-// to serve to every block of that row of tiles.
-__device__ __forceinline__ int row_inside(int r, int n, int tile) {
-  return r < n ? r : (r - tile >= 0 && r - tile < n ? r - tile : n - 1);
-}
+// Many rows: WAVES_M x WAVES_N waves a block, each with TM x TN tiles of 16 x 16 outputs.
+// v_mfma_f32_16x16x4_f32 computes D = A B for A 16 x 4 and B 4 x 16: lane l brings A[l % 16][l / 16] and
+// B[l / 16][l % 16] and gets D[4 * (l / 16) + r][l % 16] in accumulator r.  Here A is the weights' tile and B the
+// rows', so that a lane holds four neighbouring features of one row.  Which column of k an instruction's four slots
+// stand for is free as long as both operands agree, so a lane reads 16 bytes, columns 4 * (l / 16) .. + 3 of each 16,
+// and the four floats go to four instructions.
+//
+// Steps of 32 columns (rows of 128 bytes) are copied straight into a ring of slots in LDS, two ahead (lds_copy.h); a
+// row's 16-byte pieces lie permuted as in gemm_bf16.hip, so that sixteen neighbouring rows meet sixteen groups of banks.
+// At 32-bit speed (a sixteenth of bfloat16's) a step of 64 x 128 outputs is 2,048 cycles of each SIMD's matrix unit and
+// 24 KB of copies: the matrix units are the bound, and what is lost is lost to CUs that hold fewer tiles than others.
+// Hence small tiles, two blocks a CU, and K in parts where that evens the blocks out (`price`).  (The kernel before
+// this one read its operands from the L2s in the instruction's layout, sixteen pieces of 64 bytes a load, and had no
+// parts: 1,050 rows against GPT-2 large's four matrices took 178, 76, 179 and 287 us, now 87, 36, 117 and 113, the last
+// with K in three; the library's rate for a large product would make them 68, 22, 90 and 90.)
+template <int WAVES_M_, int WAVES_N_, int TM_, int TN_>
+struct F32Shape {
+  static constexpr int WAVES_M = WAVES_M_, WAVES_N = WAVES_N_, TM = TM_, TN = TN_;
+  static constexpr int WAVES = WAVES_M * WAVES_N, THREADS = 64 * WAVES, STAGES = 3, STEP = 32;
+  static constexpr int BM = WAVES_M * TM * 16, BN = WAVES_N * TN * 16;
+  static constexpr int PA = BM / 8 / WAVES, PB = BN / 8 / WAVES, COPIES = PA + PB;  // copies of eight rows a wave and step
+  static constexpr int STAGE_BYTES = (BM + BN) * STEP * 4;
+  static_assert(BM % (8 * WAVES) == 0 && BN % (8 * WAVES) == 0, "a wave copies whole kilobytes");
+};
+using F32Tile64x128 = F32Shape<2, 2, 2, 4>;
+using F32Tile64 = F32Shape<2, 2, 2, 2>;
+using F32Tile32x64 = F32Shape<2, 2, 1, 2>;
 
-// Many rows: 2 x 2 waves a block, each with RT x RT tiles of 16 x 16 outputs (a block tile of
-// 128 x 128 or 64 x 64).  v_mfma_f32_16x16x4_f32 computes D = A B for A 16 x 4 and B 4 x 16: lane
-// l brings A[l % 16][l / 16] and B[l / 16][l % 16] and gets D[4 * (l / 16) + r][l % 16] in
-// accumulator r.  Which column of k an instruction's four slots stand for is free as long as both
-// operands agree, so a lane loads 16 bytes, columns 4 * (l / 16) .. + 3 of each 16, of row l % 16
-// of a tile of A and of feature l % 16 of a tile of W, and the four floats go to four
-// instructions.  The operands come straight from memory (the L2s, mostly) in that layout: no LDS
-// and no barrier; the next 32 columns are asked for before this step's products begin.  At 32-bit
-// speed of the matrix cores (a sixteenth of bfloat16's) the L1 carries that easily.
-template <int RT>
-__global__ __launch_bounds__(256) void gemm_f32_kernel(GemmArgs p) {
-  constexpr int WT = 16 * RT;  // a wave's tile
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+template <typename S>
+__global__ __launch_bounds__(S::THREADS, 2) void gemm_f32_tile_kernel(GemmArgs p) {
+  constexpr int BM = S::BM, BN = S::BN, TM = S::TM, TN = S::TN, PA = S::PA, PB = S::PB, STAGES = S::STAGES;
+  __shared__ __attribute__((aligned(1024))) float smem[STAGES * S::STAGE_BYTES / 4];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int x = lane & 15, g = lane >> 4;
-  const int m0 = blockIdx.y * (2 * WT) + (wave >> 1) * WT;
-  const int n0 = blockIdx.x * (2 * WT) + (wave & 1) * WT;
-  // rows and features beyond the matrix read one inside it; their products are never stored
-  const float* arow[RT];
-  const float* wrow[RT];
-#pragma unroll
-  for (int i = 0; i < RT; ++i) {
-    arow[i] = p.A + (size_t)row_inside(m0 + 16 * i + x, p.M, 2 * WT) * p.lda + 4 * g;
-    wrow[i] = p.W + (size_t)row_inside(n0 + 16 * i + x, p.N, 2 * WT) * p.ldw + 4 * g;
-  }
-  f32x4_t acc[RT][RT];
-#pragma unroll
-  for (int i = 0; i < RT; ++i)
-#pragma unroll
-    for (int j = 0; j < RT; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  const int wm = wave / S::WAVES_N, wn = wave % S::WAVES_N;
+  const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
+  const int k_lo = blockIdx.z * p.per_split * 64, k_end = min(p.K, k_lo + p.per_split * 64);
+  const int n_steps = (k_end - k_lo + S::STEP - 1) / S::STEP;
 
-  // a step: 32 columns, two 16-byte pieces a lane of each row and feature (a whole 128-byte line
-  // of each by the lane's group of four).  The rows' values beyond K count as zero.
-  f32x4_t a0[2][RT], w0[2][RT], a1[2][RT], w1[2][RT];
-  auto ask = [&](int k0, f32x4_t (&ad)[2][RT], f32x4_t (&wd)[2][RT]) {
+  // the block's rows and features, each a buffer of its own from the block's first on: what lies beyond the matrix lies
+  // beyond the buffer, or is sent there
+  const int a_rows = min(BM, p.M - m0), b_rows = min(BN, p.N - n0);
+  const i32x4_t a_buf = copy_buffer(p.A + (size_t)m0 * p.lda, ((size_t)(a_rows - 1) * p.lda + p.K) * 4);
+  const i32x4_t b_buf = copy_buffer(p.W + (size_t)n0 * p.ldw, ((size_t)(b_rows - 1) * p.ldw + p.K) * 4);
+  const int row8 = lane >> 3;
+  auto piece_of = [&](int copy) __attribute__((always_inline)) { return (lane & 7) ^ ((copy & 1) * 4 + (row8 >> 1)); };
+  uint32_t a_from[PA], b_from[PB];
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int col = min(k0 + 16 * h, p.K - 4 - 4 * g);  // (+ 4 * g is in the pointers)
+  for (int i = 0; i < PA; ++i) {
+    const int c = wave * PA + i, row = c * 8 + row8;
+    a_from[i] = row < a_rows ? (uint32_t)(((size_t)row * p.lda + piece_of(c) * 4) * 4) : COPY_NOTHING;
+  }
 #pragma unroll
-      for (int i = 0; i < RT; ++i) {
-        ad[h][i] = *(const f32x4_t*)(arow[i] + col);
-        wd[h][i] = *(const f32x4_t*)(wrow[i] + col);
+  for (int i = 0; i < PB; ++i) {
+    const int c = wave * PB + i, row = c * 8 + row8;
+    b_from[i] = row < b_rows ? (uint32_t)(((size_t)row * p.ldw + piece_of(c) * 4) * 4) : COPY_NOTHING;
+  }
+  const uint32_t ring = lds_address(smem);
+  // (steps beyond the last are asked for too, as nothing: the waits then count the same copies in every round)
+  auto ask = [&](int t, int slot) __attribute__((always_inline)) {
+    const int k = k_lo + t * S::STEP, left = t < n_steps ? k_end - k : 0;
+    const uint32_t k4 = t < n_steps ? (uint32_t)k * 4u : 0u, at = ring + (uint32_t)slot * S::STAGE_BYTES;
+#pragma unroll
+    for (int i = 0; i < PA; ++i)
+      copy16_to_lds(a_buf, piece_of(wave * PA + i) * 4 < left ? a_from[i] : COPY_NOTHING, k4, at + (wave * PA + i) * 1024);
+#pragma unroll
+    for (int i = 0; i < PB; ++i)
+      copy16_to_lds(b_buf, piece_of(wave * PB + i) * 4 < left ? b_from[i] : COPY_NOTHING, k4, at + BM * 128 + (wave * PB + i) * 1024);
+  };
+
+  f32x4_t acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  const char* const a_row = (const char*)smem + (wm * TM * 16 + x) * 128;
+  const char* const b_row = (const char*)smem + BM * 128 + (wn * TN * 16 + x) * 128;
+  // the operands of 16 columns go to registers that many columns ahead of their products, also across the barrier
+  f32x4_t fa[2][TM], fb[2][TN];
+  auto read_half = [&](int h, int slot) __attribute__((always_inline)) {
+    const int s = ((4 * h + g) ^ (x >> 1)) * 16;
+#pragma unroll
+    for (int i = 0; i < TM; ++i) fa[h][i] = *(const f32x4_t*)(a_row + slot * S::STAGE_BYTES + i * 2048 + s);
+#pragma unroll
+    for (int j = 0; j < TN; ++j) fb[h][j] = *(const f32x4_t*)(b_row + slot * S::STAGE_BYTES + j * 2048 + s);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto multiply = [&](int h) __attribute__((always_inline)) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(fb[h][j][c], fa[h][i][c], acc[i][j], 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+#pragma unroll
+  for (int t = 0; t < STAGES - 1; ++t) ask(t, t);
+  int slot = 0;
+  for (int t = 0; t < n_steps; ++t) {
+    copies_arrived<(STAGES - 2) * S::COPIES>();
+    ring_barrier();  // step t is whole, and nobody reads the slot of step t - 1 any more
+    read_half(0, slot);
+    ask(t + STAGES - 1, slot == 0 ? STAGES - 1 : slot - 1);
+    if (t > 0) multiply(1);
+    read_half(1, slot);
+    multiply(0);
+    slot = slot == STAGES - 1 ? 0 : slot + 1;
+  }
+  multiply(1);
+
+  // Epilogue.  Accumulator r of tile (i, j): row 16 * i + x, feature 16 * j + 4 * g + r.  What is read (bias, the
+  // residual stream to add to) is read for a row of tiles before anything of it is stored: a load that comes after a
+  // store to memory it might alias waits for it.
+  const bool parts = p.n_splits > 1;
+  float* const out = parts ? p.ws + (size_t)blockIdx.z * p.M * p.N : p.out;
+  const int ldo = parts ? p.N : p.ldo;
+  const bool vec = ldo % 4 == 0 && ((uintptr_t)out & 15) == 0;
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+    const int m = m0 + (wm * TM + i) * 16 + x;
+    if (m >= p.M) continue;
+    f32x4_t v[TN];
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      const int n = n0 + (wn * TN + j) * 16 + 4 * g;
+      v[j] = acc[i][j];
+      if (parts) continue;
+      const bool add = p.flags & FLAG_ACCUMULATE, whole = vec && n + 4 <= p.N;
+      f32x4_t old = {0.f, 0.f, 0.f, 0.f};
+      if (add && whole) old = *(const f32x4_t*)(p.out + (size_t)m * ldo + n);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int nc = min(n + r, p.N - 1);
+        const float b = p.bias ? p.bias[nc] : 0.f;
+        if (add)
+          v[j][r] = (whole ? old[r] : p.out[(size_t)m * ldo + nc]) + (v[j][r] + b);
+        else
+          v[j][r] = activate<false>(p.flags, v[j][r] + b);
       }
     }
-  };
-  auto multiply = [&](int k0, const f32x4_t (&as)[2][RT], const f32x4_t (&ws)[2][RT]) {
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const float live = k0 + 16 * h + 4 * g < p.K ? 1.f : 0.f;
-#pragma unroll
-      for (int i = 0; i < RT; ++i) {
-        const f32x4_t av = as[h][i] * live;
-#pragma unroll
-        for (int j = 0; j < RT; ++j) {
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av.x, ws[h][j].x, acc[i][j], 0, 0, 0);
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av.y, ws[h][j].y, acc[i][j], 0, 0, 0);
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av.z, ws[h][j].z, acc[i][j], 0, 0, 0);
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av.w, ws[h][j].w, acc[i][j], 0, 0, 0);
-        }
-      }
-    }
-  };
-  // Two steps a round, their operands in two sets of registers by turns.  A step's loads are
-  // issued on one path whether its columns exist or not (beyond K they read inside the matrix),
-  // and stay ahead of the products before them: the wait is then for the older set only.
-  ask(0, a0, w0);
-  for (int k0 = 0; k0 < p.K; k0 += 64) {
-    ask(k0 + 32, a1, w1);
-    __builtin_amdgcn_sched_barrier(0);
-    multiply(k0, a0, w0);
-    __builtin_amdgcn_sched_barrier(0);
-    ask(k0 + 64, a0, w0);
-    __builtin_amdgcn_sched_barrier(0);
-    if (k0 + 32 < p.K) multiply(k0 + 32, a1, w1);  // (uniform)
-    __builtin_amdgcn_sched_barrier(0);
-  }
-
-  // Epilogue.  Accumulator r of tile (i, j): row 16 * i + 4 * g + r, feature 16 * j + x.  What is
-  // read (bias, the residual stream to add to) is read for a row of tiles before anything of it is
-  // stored: a load that comes after a store to memory it might alias waits for it.
-#pragma unroll
-  for (int i = 0; i < RT; ++i) {
-    const int mb = m0 + 16 * i + 4 * g;
-    f32x4_t v[RT];
-#pragma unroll
-    for (int j = 0; j < RT; ++j) {
-      const int n = n0 + 16 * j + x;
-      const int nc = min(n, p.N - 1);
-      const float bias = p.bias ? p.bias[nc] : 0.f;
-      if (p.flags & FLAG_ACCUMULATE) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) v[j][r] = p.out[(size_t)min(mb + r, p.M - 1) * p.ldo + nc];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) v[j][r] += acc[i][j][r] + bias;
+    for (int j = 0; j < TN; ++j) {
+      const int n = n0 + (wn * TN + j) * 16 + 4 * g;
+      if (vec && n + 4 <= p.N) {
+        *(f32x4_t*)(out + (size_t)m * ldo + n) = v[j];
       } else {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          v[j][r] = acc[i][j][r] + bias;
-          v[j][r] = activate<false>(p.flags, v[j][r]);
-        }
+        for (int r = 0; r < 4; ++r)
+          if (n + r < p.N) out[(size_t)m * ldo + n + r] = v[j][r];
       }
-    }
-#pragma unroll
-    for (int j = 0; j < RT; ++j) {
-      const int n = n0 + 16 * j + x;
-      if (n >= p.N) continue;
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        if (mb + r < p.M) p.out[(size_t)(mb + r) * p.ldo + n] = v[j][r];
     }
   }
 }
@@ -267,21 +303,56 @@ __global__ __launch_bounds__(64 * SKF_MAX_WAVES) void gemm_f32_skinny_kernel(Gem
 
 DEFINE_LAST_ERROR(mlxlm_last_error)
 
-// In how many parts the kernel for few rows should take K so that its blocks fill the GPU: one
-// and a half blocks a compute unit, eight chunks of 64 columns a part at least.  1 where the
-// matrix gives a block to every unit anyway, or is so small that a second kernel costs more
-// than the split gains.
-extern "C" int gemm_f32_splits(int M, int N, int K, int force) {
+// What a tile shape costs in microseconds: its products at the speed of a CU's matrix units (2.5e-4 an output and 64
+// columns; a block alone on its CU, one wave a SIMD, a fifth more), blocks that share a CU one after another, and a
+// fixed part for the first step's way and the epilogue.  Against the times of 6 numbers of rows from 80 to 2,048 and ten
+// matrices of widths 768 to 1,600, each with K in 1 to 8 parts, the choice is within 3 % of the best on average.
+struct F32Price {
+  int variant, bm, bn;
+};
+static const F32Price F32_PRICES[] = {
+    {1, F32Tile64x128::BM, F32Tile64x128::BN}, {2, F32Tile64::BM, F32Tile64::BN}, {4, F32Tile32x64::BM, F32Tile32x64::BN}};
+static double price(const F32Price& s, int M, int N, int K, int n_splits) {
+  const long tiles = (long)((M + s.bm - 1) / s.bm) * ((N + s.bn - 1) / s.bn);
+  const long n = (tiles * n_splits + n_compute_units() - 1) / n_compute_units();
+  const int chunks = ((K + 63) / 64 + n_splits - 1) / n_splits;
+  return 4.0 + (n == 1 ? 1.2 : 1.0) * n * chunks * (2.5e-4 * s.bm * s.bn);
+}
+static int cheapest_shape(int M, int N, int K, int n_splits, double* us) {
+  int variant = 0;
+  for (const F32Price& s : F32_PRICES) {
+    const double t = price(s, M, N, K, n_splits);
+    if (!variant || t < *us) variant = s.variant, *us = t;
+  }
+  return variant;
+}
+
+// In how many parts K should go.  Up to 64 rows (the kernel for few rows): so that its blocks fill
+// the GPU, one and a half blocks a compute unit, eight chunks of 64 columns a part at least; 1 where
+// the matrix gives a block to every unit anyway, or is so small that a second kernel costs more
+// than the split gains.  More rows: by the prices above and the second kernel's, a launch plus the
+// bytes of the partial sums at 3 TB/s.  `fused`: it stands in for one that would run anyway (the norm
+// that follows a sum into the residual stream), so it costs only the extra bytes.
+extern "C" int gemm_f32_splits(int M, int N, int K, int fused, int force) {
   const int n_chunks = (K + SKF_CHUNK - 1) / SKF_CHUNK;
-  if (M < 1 || M > SKF_MAX_ROWS) return 1;
+  if (M < 1) return 1;
   int want;
   if (force > 0) {
     want = force;
-  } else {
+  } else if (M <= SKF_MAX_ROWS) {
     const int n_blocks = (N + 15) / 16;
     if (n_blocks >= n_compute_units() || (long)N * K < SKF_SPLIT_FROM) return 1;
     want = (3 * n_compute_units() / 2 + n_blocks - 1) / n_blocks;
     if (want > n_chunks / 8) want = n_chunks / 8;
+  } else {
+    double best_us = 0.0;
+    want = 1;
+    for (int s = 1; s <= 8 && s <= n_chunks / 2; ++s) {
+      double us = 0.0;
+      cheapest_shape(M, N, K, s, &us);
+      if (s > 1) us += (fused ? 1.0 : 2.5) + 8.0 * (fused ? s - 1 : s) * (double)M * N / 3e6;
+      if (s == 1 || us < 0.95 * best_us) want = s, best_us = us;
+    }
   }
   if (want < 1) want = 1;
   if (want > n_chunks) want = n_chunks;
@@ -289,9 +360,14 @@ extern "C" int gemm_f32_splits(int M, int N, int K, int force) {
   return (n_chunks + per - 1) / per;  // no empty part
 }
 
-// variant: 0 = choose, 1 = 128x128 block tile, 2 = 64x64 block tile, 3 = the kernel for up to 64 rows.
-// n_splits > 1 (the kernel for few rows only): K in that many parts, whose sums go to
-// ws[part][M][N] (ws_floats floats at least) for sum_partials of gemm_bf16_decode.hip to add up
+template <typename S>
+static void launch_tiles(const GemmArgs& p, hipStream_t stream) {
+  dim3 grid((p.N + S::BN - 1) / S::BN, (p.M + S::BM - 1) / S::BM, p.n_splits), block(S::THREADS);
+  hipLaunchKernelGGL(gemm_f32_tile_kernel<S>, grid, block, 0, stream, p);
+}
+
+// variant: 0 = choose, 1 = tiles of 64 x 128, 2 = of 64 x 64, 4 = of 32 x 64, 3 = the kernel for up to
+// 64 rows.  n_splits > 1: K in that many parts, whose sums go to ws[part][M][N] (ws_floats floats at least) for sum_partials of gemm_bf16_decode.hip to add up
 // and finish; out is not written then.
 extern "C" int gemm_f32(void* out, const void* A, const void* W, const float* bias, int M, int N,
                         int K, int lda, int ldw, int ldo, int flags, int variant, int n_splits, float* ws,
@@ -304,7 +380,7 @@ extern "C" int gemm_f32(void* out, const void* A, const void* W, const float* bi
   p.M = M, p.N = N, p.K = K;
   p.lda = lda, p.ldw = ldw, p.ldo = ldo;
   p.flags = flags;
-  p.n_splits = 1, p.ws = nullptr;
+  p.n_splits = 1, p.per_split = (K + SKF_CHUNK - 1) / SKF_CHUNK, p.ws = nullptr;
   if (M < 0 || N <= 0 || K <= 0) FAIL("gemm_f32: bad sizes M=%d N=%d K=%d", M, N, K);
   if (K % 4 != 0) FAIL("gemm_f32: K=%d must be a multiple of 4", K);
   if (lda % 4 != 0 || ldw % 4 != 0)
@@ -318,19 +394,22 @@ extern "C" int gemm_f32(void* out, const void* A, const void* W, const float* bi
   if (M == 0) return 0;
   if (n_splits < 1) FAIL("gemm_f32: n_splits=%d", n_splits);
   if (n_splits > 1) {
-    if (variant == 0 && M <= SKF_MAX_ROWS) variant = 3;
-    if (variant != 3) FAIL("gemm_f32: only the kernel for up to %d rows takes K in parts", SKF_MAX_ROWS);
-    if (n_splits > (K + SKF_CHUNK - 1) / SKF_CHUNK) FAIL("gemm_f32: %d parts of K=%d", n_splits, K);
+    const int n_chunks = (K + SKF_CHUNK - 1) / SKF_CHUNK, per = (n_chunks + n_splits - 1) / n_splits;
+    if (n_splits > n_chunks) FAIL("gemm_f32: %d parts of K=%d", n_splits, K);
     if (!ws || ws_floats < (size_t)n_splits * M * N) FAIL("gemm_f32: the parts' workspace is too small");
-    p.n_splits = n_splits, p.ws = ws;
+    p.n_splits = n_splits, p.per_split = per, p.ws = ws;
   }
-  if (variant == 0) variant = M <= SKF_MAX_ROWS ? 3 : (size_t)M * N < (size_t)128 * 128 * 128 ? 2 : 1;
+  double us = 0.0;
+  if (variant == 0) variant = M <= SKF_MAX_ROWS ? 3 : cheapest_shape(M, N, K, n_splits, &us);
+  if (variant != 3 && p.per_split * (n_splits - 1) * SKF_CHUNK >= K) FAIL("gemm_f32: %d parts of K=%d leave one empty", n_splits, K);
+  if (variant != 3 && !(fits_copy_buffer(((size_t)127 * lda + K) * 4) && fits_copy_buffer(((size_t)127 * ldw + K) * 4)))
+    FAIL("gemm_f32: rows of K=%d floats, %d and %d apart, are too long", K, lda, ldw);
   if (variant == 1) {
-    dim3 grid((N + 127) / 128, (M + 127) / 128), block(256);
-    hipLaunchKernelGGL(gemm_f32_kernel<4>, grid, block, 0, stream, p);
+    launch_tiles<F32Tile64x128>(p, stream);
   } else if (variant == 2) {
-    dim3 grid((N + 63) / 64, (M + 63) / 64), block(256);
-    hipLaunchKernelGGL(gemm_f32_kernel<2>, grid, block, 0, stream, p);
+    launch_tiles<F32Tile64>(p, stream);
+  } else if (variant == 4) {
+    launch_tiles<F32Tile32x64>(p, stream);
   } else if (variant == 3) {
     if (M > SKF_MAX_ROWS) FAIL("gemm_f32: the kernel for few rows takes at most %d, got %d", SKF_MAX_ROWS, M);
     // where the blocks are fewer than the compute units, more waves each

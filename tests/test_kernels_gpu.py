@@ -104,6 +104,32 @@ def test_gemm_f32(M, N, K, mode):
         assert err < 1e-5 * math.sqrt(K) * 4, (variant, err)
 
 
+@pytest.mark.parametrize("M,N,K", [(65, 60, 4), (33, 64, 32), (64, 129, 64), (31, 127, 100), (97, 65, 192), (129, 257, 520)])
+def test_gemm_f32_tiles_at_the_ring_s_edges(M, N, K):
+    """Tiles with a row or feature more or less than whole ones, K of fewer steps of 32 columns than a
+    tile's ring has slots, as many, and more, whole and in parts.  What lies around the operands is NaN:
+    rows, features and columns that do not exist must come in as zeros, and nothing beyond the
+    output's columns is written.  (K roundings of the largest partial sum at most, against 64 bits.)"""
+    k = _k()
+    a = torch.full((M + 40, K + 12), float("nan"), device=DEV)[:M, :K]
+    w = torch.full((N + 40, K + 12), float("nan"), device=DEV)[:N, :K]
+    a.copy_(_rand((M, K), torch.float32, 10))
+    w.copy_(_rand((N, K), torch.float32, 11, 0.1))
+    bias = _rand((N,), torch.float32, 12)
+    ref = plain.linear(a.double().cpu(), w.double().cpu(), bias.double().cpu())
+    tol = (K + 4) * 2.0**-24 * ((a.double().abs() @ w.double().abs().t()).max().item() + bias.abs().max().item() + 1)
+    chunks = (K + 63) // 64
+    for variant in (1, 2, 4):
+        for splits in [None] + [s for s in (2, 3) if s <= chunks]:
+            for pad in (0, 3):  # (rows of the output whose pieces of four are aligned, or not)
+                wide = torch.full((M, N + pad), 0.5, device=DEV)
+                out = wide[:, :N]
+                k.linear(out, a, w, bias, accumulate=True, variant=variant, splits=splits)
+                err = (out.double().cpu() - ref - 0.5).abs().max().item()
+                assert err < tol, (variant, splits, pad, err)
+                assert (wide[:, N:] == 0.5).all()
+
+
 @pytest.mark.parametrize("N,K", [(1, 4), (7, 508), (9, 512), (17, 516), (40, 1024), (33, 1028), (100, 1600),
                                  (24, 2052), (4100, 520), (4097, 1600)])
 def test_gemm_f32_few_rows(N, K):
