@@ -9,8 +9,8 @@
 // (mlx_lm/models/base.py:132-139 with mask=None, mlx_lm/generate.py:1414).
 //
 // Work split: grid (rows, heads, n_splits), 1 to 16 waves a block.  The row's
-// keys [k_lo, k_hi) are cut into tiles of 32 or 64; the tiles are dealt to the splits
-// in runs and, inside a block, to the waves in turn.  With few rows in a step
+// keys [k_lo, k_hi) are cut into tiles of 16; the tiles are dealt to the splits
+// in runs and, inside a block, to the waves in turn; a wave asks for its next tile before it takes one.  With few rows in a step
 // it is the many waves of a block, joined through LDS, that give the GPU
 // enough to do; the parts of splits are joined by the block of a (row, head) that
 // finishes last, or by a second kernel.  A wave reads a tile as
@@ -49,6 +49,7 @@ struct DecodeArgs {
   // request brings one token), so neither `rows` nor `token_req` has to be read.
   // table_in_lds: the request's page numbers are copied to LDS once (max_blocks of them fit).
   int rows_are_requests, table_in_lds;
+  int page_shift;  // page_size is two to this power, or -1
   int out_head_dim;
   // 1 or 2: the blocks that share a row's keys join their sums themselves: the one that arrives
   // last at the (row, head)'s counter adds them in the order of the parts (no second kernel);
@@ -87,6 +88,12 @@ __device__ __forceinline__ float gate_at(const DecodeArgs& p, int row, int col) 
 
 #define MAX_WAVES 16
 
+// Sixteen bytes that nobody on this die asks for again
+__device__ __forceinline__ uint4 load_once(const void* at) {
+  const u32x4_t v = __builtin_nontemporal_load((const u32x4_t*)at);
+  return make_uint4(v.x, v.y, v.z, v.w);
+}
+
 union Frag8g {
   uint4 u;
   bf16x8_t v;
@@ -97,10 +104,13 @@ __device__ __forceinline__ size_t out_at(const DecodeArgs& p, int row, int col) 
   return p.ldo != 0 ? (size_t)row * p.ldo + col : packed_at(row, col, (p.n_heads * p.out_head_dim + 63) / 64);
 }
 
-// Keys a wave takes at a time: 32 or 64, the caller's choice.  With 64, a context of 530 gave nine
-// of a block's waves a tile and the others none: 9.3 us for 8 rows of 25 heads against 7.3 with 32.
-// Where rows x heads are several blocks a CU and the walk is long, the larger tile's sixteen
-// loads a lane in flight are ahead (32 rows at contexts of 512 to 1,022: 2 % of the step).
+// What bounds this kernel: the keys and values come from memory once, and at many rows or long contexts that is the
+// time (64 rows of 25 heads of 64 at contexts of 300 to 1,001 are 266 MB: 49 us, 5.4 TB/s; a plain stream reads 6.4, with
+// the streaming hint 7.2).  So they are read with that hint (8 to 10 % here); a tile is small and the next one
+// on its way while it is taken, so that a wave's registers are few and many waves have something in flight (tiles of
+// 32 or 64 keys, one at a time, with a lookup and two divisions a lane and key: 54 to 58 us, 13.4 against 12.2 for 8 rows,
+// 25.3 against 22.1 for 16 rows of 16 heads of 128, 16.9 against 14.9 for 8 rows of float keys).  At few rows and short
+// contexts what is left is the chain: table and query, keys, the waves' join.
 
 // 16 bytes of a row as floats, and a float back as an element
 __device__ __forceinline__ void unpack(const uint4& v, float (&f)[8], const uint16_t*) {
@@ -143,19 +153,20 @@ __device__ __forceinline__ bool last_to_arrive(unsigned* counter, unsigned n_par
   return *s_last != 0;
 }
 
-// T: uint16_t (bfloat16 bits) or float.  CPK lanes per key: head_dim = EPL * CPK.  TILE: keys a wave at a time.
-template <typename T, int CPK, int TILE>
+// T: uint16_t (bfloat16 bits) or float.  CPK lanes per key: head_dim = EPL * CPK.
+template <typename T, int CPK>
 __global__ __launch_bounds__(64 * (CPK >= 16 ? MAX_WAVES / 2 : MAX_WAVES)) void attn_decode_kernel(DecodeArgs p) {
   constexpr int EPL = 16 / sizeof(T);  // elements a lane holds of a key
   constexpr int HD = EPL * CPK;
+  constexpr int TILE = ATTN_DECODE_TILE_KEYS;
   constexpr int KPL = 64 / CPK;    // keys per load instruction
-  constexpr int NL = TILE / KPL;   // loads per tile (= CPK)
+  constexpr int NL = TILE / KPL;   // loads per tile
   __shared__ float Ms[MAX_WAVES], Ls[MAX_WAVES];
   __shared__ float Os[MAX_WAVES][HD];
   __shared__ int s_last;
   extern __shared__ int page_of[];  // [max_blocks] with table_in_lds
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n_waves = blockDim.x >> 6;
   if (blockIdx.y >= p.n_heads) {  // a reading block (uniform)
     if (blockIdx.z != 0) return;
@@ -196,7 +207,7 @@ __global__ __launch_bounds__(64 * (CPK >= 16 ? MAX_WAVES / 2 : MAX_WAVES)) void 
   if (p.table_in_lds) {
     for (int i = tid; i < p.max_blocks; i += blockDim.x) page_of[i] = table[i];
   }
-  const int pos = p.positions[row];
+  const int pos = __builtin_amdgcn_readfirstlane(p.positions[row]);
   const int sub = lane % CPK;  // which EPL columns of the key
   const int kin = lane / CPK;  // which key of a load
   const T* k_pages = (const T*)p.k_pages;
@@ -219,13 +230,13 @@ __global__ __launch_bounds__(64 * (CPK >= 16 ? MAX_WAVES / 2 : MAX_WAVES)) void 
   const int sink_hi = min(p.keep_first, k_lo);
   const int n_sink_tiles = (sink_hi + TILE - 1) / TILE;
   const int n_tiles = n_sink_tiles + (k_hi - kt0 + TILE - 1) / TILE;
-  // Joined here, a row may take fewer splits than the launch has: as many as leave a wave a tile
-  // of 32 keys, and one if a wave has fewer than 96 keys anyway (joining costs about a tile's
+  // Joined here, a row may take fewer splits than the launch has: as many as leave a wave
+  // ATTN_DECODE_KEYS_A_PART keys, and one if a wave has few anyway (joining costs about 32 keys'
   // time).  Blocks of the splits it does not take have nothing to do.
   int n_splits = p.n_splits;
   if (p.join_here == 2) {
     const int keys_a_wave = (k_hi - kt0 + n_sink_tiles * TILE) / n_waves;
-    n_splits = keys_a_wave >= 96 ? min(n_splits, keys_a_wave / 32) : 1;
+    n_splits = keys_a_wave >= ATTN_DECODE_SPLIT_KEYS_A_WAVE ? min(n_splits, keys_a_wave / ATTN_DECODE_KEYS_A_PART) : 1;
     if (split >= n_splits) return;  // (the whole block)
   }
   const int per_split = (n_tiles + n_splits - 1) / n_splits;
@@ -239,23 +250,41 @@ __global__ __launch_bounds__(64 * (CPK >= 16 ? MAX_WAVES / 2 : MAX_WAVES)) void 
   const size_t head_off = (size_t)kv_head * p.page_size * HD;
   if (p.table_in_lds) __syncthreads();  // (uniform over the block)
 
-  for (int t = t_begin + wave; t < t_end; t += n_waves) {
+  // A tile's loads.  A load's keys lie in one page (a page holds whole loads), so the page, found through scalar
+  // arithmetic, is the wave's and only the place within the load a lane's own.  Keys outside the run are pulled
+  // inside, loads too (their scores are masked below).
+  const int lane_off = kin * HD + sub * EPL;
+  auto tile_of = [&](int t, int& kt, int& t_lo, int& t_hi) __attribute__((always_inline)) {
     const bool sink = t < n_sink_tiles;
-    const int kt = sink ? t * TILE : kt0 + (t - n_sink_tiles) * TILE;
-    const int t_lo = sink ? 0 : k_lo, t_hi = sink ? sink_hi : k_hi;  // the run of keys this tile is of
-    uint4 kv[NL], vv[NL];
-    // all loads of the tile first; addresses of keys outside the run are
-    // pulled inside (their scores are masked below)
+    kt = sink ? t * TILE : kt0 + (t - n_sink_tiles) * TILE;
+    t_lo = sink ? 0 : k_lo, t_hi = sink ? sink_hi : k_hi;  // the run of keys this tile is of
+  };
+  auto ask = [&](int t, uint4 (&kv)[NL], uint4 (&vv)[NL]) __attribute__((always_inline)) {
+    int kt, t_lo, t_hi;
+    tile_of(t, kt, t_lo, t_hi);
+    const int first = t_lo - t_lo % KPL, last = t_hi - 1 - (t_hi - 1) % KPL;  // the run's first and last load
+    const bool whole = kt >= t_lo && kt + TILE <= t_hi;
+    int page[NL], in_page[NL];
 #pragma unroll
     for (int j = 0; j < NL; ++j) {
-      int key = kt + j * KPL + kin;
-      key = min(max(key, t_lo), t_hi - 1);
-      const int page = p.table_in_lds ? page_of[key / p.page_size] : table[key / p.page_size];
-      const size_t off = (size_t)page * p.page_stride + head_off +
-                         (size_t)(key % p.page_size) * HD + sub * EPL;
-      kv[j] = *(const uint4*)(k_pages + off);
-      vv[j] = *(const uint4*)(v_pages + off);
+      const int b = min(max(kt + j * KPL, first), last);
+      const int in_table = p.page_shift >= 0 ? b >> p.page_shift : b / p.page_size;
+      in_page[j] = (b - in_table * p.page_size) * HD + (whole ? lane_off : (min(max(b + kin, t_lo), t_hi - 1) - b) * HD + sub * EPL);
+      if (p.table_in_lds)  // (pointers that say where they point: one for both would make a flat load)
+        page[j] = ((const __attribute__((address_space(3))) int*)page_of)[in_table];
+      else
+        page[j] = ((const __attribute__((address_space(1))) int*)table)[in_table];
     }
+#pragma unroll
+    for (int j = 0; j < NL; ++j) {
+      const size_t at = (size_t)page[j] * p.page_stride + head_off + in_page[j];
+      kv[j] = load_once(k_pages + at);
+      vv[j] = load_once(v_pages + at);
+    }
+  };
+  auto take = [&](int t, const uint4 (&kv)[NL], const uint4 (&vv)[NL]) __attribute__((always_inline)) {
+    int kt, t_lo, t_hi;
+    tile_of(t, kt, t_lo, t_hi);
     float s[NL];
     float tmax = -INFINITY;
 #pragma unroll
@@ -289,6 +318,22 @@ __global__ __launch_bounds__(64 * (CPK >= 16 ? MAX_WAVES / 2 : MAX_WAVES)) void 
       for (int i = 0; i < EPL; ++i) o[i] += pj * vf[i];
     }
     m = m_new;
+  };
+  // the next tile is on its way while one is taken, in two sets of registers by turns
+  uint4 k0[NL], v0[NL], k1[NL], v1[NL];
+  int t = t_begin + wave;
+  if (t < t_end) {
+    ask(t, k0, v0);
+    for (; t + 2 * n_waves < t_end; t += 2 * n_waves) {
+      ask(t + n_waves, k1, v1);
+      take(t, k0, v0);
+      ask(t + 2 * n_waves, k0, v0);
+      take(t + n_waves, k1, v1);
+    }
+    const bool one_more = t + n_waves < t_end;
+    if (one_more) ask(t + n_waves, k1, v1);
+    take(t, k0, v0);
+    if (one_more) take(t + n_waves, k1, v1);
   }
 
   // join the lane groups: lanes with the same `sub` hold the same columns
@@ -527,7 +572,7 @@ __global__ void attn_decode_merge_kernel(DecodeArgs p) {
 DEFINE_LAST_ERROR(mlxlm_last_error)
 
 template <typename T, int CPK>
-static void launch(const DecodeArgs& p, int n_rows, int n_waves, int key_tile, hipStream_t stream) {
+static void launch(const DecodeArgs& p, int n_rows, int n_waves, hipStream_t stream) {
   // reading blocks for the CUs that the rows leave idle, if there are eight or more
   int extra_y = 0;
   if (p.ahead && p.ahead_chunks > 0) {
@@ -536,10 +581,7 @@ static void launch(const DecodeArgs& p, int n_rows, int n_waves, int key_tile, h
   }
   const size_t lds = p.table_in_lds ? (size_t)p.max_blocks * sizeof(int) : 0;
   const dim3 grid(n_rows, p.n_heads + extra_y, p.n_splits), block(64 * n_waves);
-  if (key_tile == 64 && CPK < 32)  // (32 lanes a key: 64 keys would be 64 loads a lane in flight)
-    hipLaunchKernelGGL((attn_decode_kernel<T, (CPK < 32 ? CPK : 16), 64>), grid, block, lds, stream, p);
-  else
-    hipLaunchKernelGGL((attn_decode_kernel<T, CPK, 32>), grid, block, lds, stream, p);
+  hipLaunchKernelGGL((attn_decode_kernel<T, CPK>), grid, block, lds, stream, p);
   if (p.n_splits > 1 && !p.join_here)
     hipLaunchKernelGGL((attn_decode_merge_kernel<T, CPK>), dim3(n_rows, p.n_heads), dim3(16 / sizeof(T) * CPK), 0, stream, p);
 }
@@ -548,7 +590,7 @@ static void launch(const DecodeArgs& p, int n_rows, int n_waves, int key_tile, h
 // item i of `rows` is row i and belongs to request i (every request of the step brings one token),
 // which saves the kernel two trips to memory.  dtype DT_BF16 with head_dim 32, 64, 128 or 256, DT_F32
 // with 16, 32, 64 or 128, and pages that hold whole loads (page_size a multiple of the keys in 1 KB).
-// key_tile: 32 or 64 keys a wave at a time (0: 32).  join_in_kernel: 0, a second kernel joins the
+// key_tile: 0, 32 or 64 (accepted, of no effect: a wave takes 16 keys at a time).  join_in_kernel: 0, a second kernel joins the
 // n_splits parts of a (row, head); 1, the block that finishes a (row, head) last does (up to
 // 65,536 (row, head)s; part_o and part_ml are still where the parts pass through); 2, the same,
 // and n_splits is only the most a row takes: a short row takes fewer, by its own length.
@@ -567,8 +609,7 @@ static int decode_rows_launch(void* out, const void* q, int ldq, int ldo, const 
     FAIL("attn_decode: softcap %g, a distance table of %d entries a head", (double)shape->softcap, shape->n_dist);
   if (keep_first < 0) FAIL("attn_decode: keep_first %d must not be negative", keep_first);
   if (gate && ldg < n_heads * head_dim) FAIL("attn_decode: the gate's row stride %d is smaller than its rows", ldg);
-  if (key_tile == 0) key_tile = 32;
-  if (key_tile != 32 && key_tile != 64) FAIL("attn_decode: a wave takes 32 or 64 keys at a time, not %d", key_tile);
+  if (key_tile != 0 && key_tile != 32 && key_tile != 64) FAIL("attn_decode: key_tile %d is not 0, 32 or 64", key_tile);
   if (dtype != DT_F32 && dtype != DT_BF16) FAIL("attn_decode: unknown dtype code %d", dtype);
   const int epl = dtype == DT_F32 ? 4 : 8;  // elements in a lane's 16 bytes
   if (n_waves < 1 || n_waves > MAX_WAVES) FAIL("attn_decode: %d waves a block, must be 1 to %d", n_waves, MAX_WAVES);
@@ -616,24 +657,25 @@ static int decode_rows_launch(void* out, const void* q, int ldq, int ldo, const 
   if (join_in_kernel < 0 || join_in_kernel > 2) FAIL("attn_decode: join_in_kernel %d is not 0, 1 or 2", join_in_kernel);
   p.join_here = n_splits > 1 && (long)n_rows * n_heads <= JOIN_MAX_ITEMS ? join_in_kernel : 0;
   p.table_in_lds = max_blocks > 0 && max_blocks <= 8192;  // (32 KB of LDS at most)
+  p.page_shift = (page_size & (page_size - 1)) == 0 ? __builtin_ctz(page_size) : -1;
   if (dtype == DT_BF16) {
     if (cpk == 4)
-      launch<uint16_t, 4>(p, n_rows, n_waves, key_tile, stream);
+      launch<uint16_t, 4>(p, n_rows, n_waves, stream);
     else if (cpk == 8)
-      launch<uint16_t, 8>(p, n_rows, n_waves, key_tile, stream);
+      launch<uint16_t, 8>(p, n_rows, n_waves, stream);
     else if (cpk == 16)
-      launch<uint16_t, 16>(p, n_rows, n_waves, key_tile, stream);
+      launch<uint16_t, 16>(p, n_rows, n_waves, stream);
     else
-      launch<uint16_t, 32>(p, n_rows, n_waves, key_tile, stream);
+      launch<uint16_t, 32>(p, n_rows, n_waves, stream);
   } else {
     if (cpk == 4)
-      launch<float, 4>(p, n_rows, n_waves, key_tile, stream);
+      launch<float, 4>(p, n_rows, n_waves, stream);
     else if (cpk == 8)
-      launch<float, 8>(p, n_rows, n_waves, key_tile, stream);
+      launch<float, 8>(p, n_rows, n_waves, stream);
     else if (cpk == 16)
-      launch<float, 16>(p, n_rows, n_waves, key_tile, stream);
+      launch<float, 16>(p, n_rows, n_waves, stream);
     else
-      launch<float, 32>(p, n_rows, n_waves, key_tile, stream);
+      launch<float, 32>(p, n_rows, n_waves, stream);
   }
   CHECK_LAUNCH("attn_decode");
   return 0;

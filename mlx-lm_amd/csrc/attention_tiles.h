@@ -43,17 +43,22 @@ __device__ __forceinline__ float head_gate_of(const Args& p, int row, int h) {
 
 // How the decode kernel (attention_decode.hip) is launched for n_rows single rows of n_heads
 // heads whose longest walk is `keys` keys (a window's and its kept first keys' at most): in how
-// many parts a row's keys go at most, the waves a block, the keys a wave takes at a time.
-// Eight waves a block (four where the rows' blocks alone are more than the CUs, or the keys no
-// more than four waves' tiles); tiles of 32 keys, of 64 where the blocks are more than three a CU
-// and the walk is 640 keys or more; splits only where a wave would walk 96 keys or more, as many
-// as leave it a tile, and no more than give every block a compute unit at once.
+// many parts a row's keys go at most, and the waves a block (`key_tile` is always 32: callers of the
+// kernel may still name 32 or 64, its tiles are of ATTN_DECODE_TILE_KEYS whatever they say).
+// Eight waves a block; four where the rows' blocks alone are more than the CUs (64 rows of 25 heads
+// at contexts of 300 to 1,001: 49.2 us, 49.7 with eight, 53.5 with two; 24 rows 20.4 and 22.6), or the keys no
+// more than four waves' tiles; sixteen where blocks that have a CU each walk 2,048 keys or more (8 rows at
+// 4,000 to 8,001: 57.1 us, 59.3 with eight).  Splits only where a wave would walk 64 keys or more, as many as
+// leave it 32, and no more than give every block a compute unit at once (one row at 700 keys: 8.1 us in two, 8.7
+// whole; at 6,000: 13.4 in eight).
 #define ATTN_DECODE_ROW_WAVES 8
-#define ATTN_DECODE_SPLIT_KEYS_A_WAVE 96
+#define ATTN_DECODE_TILE_KEYS 16
+#define ATTN_DECODE_SPLIT_KEYS_A_WAVE 64
+#define ATTN_DECODE_KEYS_A_PART 32
 static inline void attn_decode_row_work(int n_compute_units, int n_rows, int n_heads, int head_dim, long keys,
                                         int* n_splits, int* n_waves, int* key_tile) {
   const long c = keys;
-  const long tiles = c + 31 < 32 ? 1 : (c + 31) / 32;
+  const long tiles = c < 1 ? 1 : (c + ATTN_DECODE_TILE_KEYS - 1) / ATTN_DECODE_TILE_KEYS;
   const long blocks = n_rows * n_heads < 1 ? 1 : (long)n_rows * n_heads;
   int nw = blocks > n_compute_units ? 4 : ATTN_DECODE_ROW_WAVES;
   const int fewest = head_dim > 128 ? 4 : 2;  // (the block's threads write a column of the head each)
@@ -61,17 +66,11 @@ static inline void attn_decode_row_work(int n_compute_units, int n_rows, int n_h
   const long keys_a_wave = c / nw;
   long ns = 1;
   if (keys_a_wave >= ATTN_DECODE_SPLIT_KEYS_A_WAVE) {
-    ns = keys_a_wave / 32;
+    ns = keys_a_wave / ATTN_DECODE_KEYS_A_PART;
     if (n_compute_units / blocks < ns) ns = n_compute_units / blocks;
     if (ns > 64) ns = 64;
     if (ns < 1) ns = 1;
   }
+  if (ns == 1 && blocks <= n_compute_units && c >= 2048) nw = 2 * ATTN_DECODE_ROW_WAVES;
   *n_splits = (int)ns, *n_waves = nw, *key_tile = 32;
-  if (blocks > 3 * n_compute_units && c >= 640) {
-    // many rows and a long walk: tiles of 64 keys, and as many waves a block as make eight a CU
-    const long want = (8L * n_compute_units + blocks - 1) / blocks;
-    nw = fewest;
-    while (nw < 8 && nw < want) nw *= 2;
-    *n_waves = nw, *key_tile = 64;
-  }
 }

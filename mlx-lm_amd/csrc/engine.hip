@@ -733,19 +733,9 @@ struct Attention : Mixer {
 
   int scatter_for(EngCtx* ctx, int slot, EngScatter* sc) const;
 
-  // (n_splits, n_waves, keys a wave at a time) for the decode kernel.  Eight waves a block (four
-  // where the rows' blocks alone are more than the CUs, or the keys no more than four waves'
-  // tiles): measured at 1 to 64 rows and contexts of 100 to 7,000, eight were level with or ahead
-  // of sixteen everywhere.  Tiles of 32 keys, so that every wave has some at a context of a few
-  // hundred; of 64 where the blocks are more than three a CU and the context is 640 or more (the
-  // larger tile keeps more loads in flight; a recorded step plans for the model's positions: at
-  // 1,024 of them, 12 to 30 rows were 1 to 3 % faster with 32 over contexts of 512 to 1,022, 32
-  // rows 2 % faster with 64).  The block that finishes a (row, head) last joins its splits, which
-  // costs about as much as a tile of keys: splits only where a wave would walk 96 keys or more, as
-  // many as leave it a tile, and no more than give every block a compute unit at once (one row at
-  // 1,000 keys: 9.4 us unsplit, 7.3 in four; at 7,000: 44 unsplit, 13.6 in eight, 15.9 in twelve).
-  // This is the most a row takes; the kernel gives a shorter row fewer by the same rule, so a
-  // recorded step, planned for the model's positions, splits only the rows that are long.
+  // (n_splits, n_waves, key_tile) for the decode kernel: attn_decode_row_work's rule.  n_splits is the
+  // most a row takes; the kernel gives a shorter row fewer by the same rule, so a recorded step,
+  // planned for the model's positions, splits only the rows that are long.
   void row_work(const EngCtx* ctx, int n_rows, long max_row_context, int* n_splits, int* n_waves,
                 int* key_tile) const {
     const long c = window <= 0 ? max_row_context : (max_row_context < window + 31 ? max_row_context : window + 31);

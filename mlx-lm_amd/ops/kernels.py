@@ -830,7 +830,7 @@ def attn_decode(out, q, kv, block_table, token_req, positions, rows, n_rows, n_h
     ``ahead``: a ``PackedWeight`` whose first ``ahead_chunks`` chunks the CUs without a row read
     meanwhile, each the chunks that a block on its own die will ask for (``sum_partials_norm``).
     ``rows_are_requests``: item ``i`` of ``rows`` is row ``i`` of request ``i`` (the caller says so).
-    ``key_tile``: 32 or 64 keys a wave at a time.  ``join_in_kernel``: 0, a second kernel joins
+    ``key_tile``: 32 or 64 (of no effect: a wave takes 16 keys at a time).  ``join_in_kernel``: 0, a second kernel joins
     the ``n_splits`` parts of a (row, head); 1, the block that finishes it last does; 2, the same,
     and a short row takes fewer than ``n_splits`` by its own length."""
     lib = build.load("attention_decode")

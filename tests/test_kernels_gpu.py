@@ -438,6 +438,30 @@ def test_attn_decode(case, n_splits, n_waves):
         assert err < _attn_tol(torch.bfloat16), (key_tile, here, err)
 
 
+@pytest.mark.parametrize("hd,ps", [(32, 48), (64, 24), (128, 12), (256, 6), (64, 16)])
+@pytest.mark.parametrize("window", [0, 1, 17])
+@pytest.mark.parametrize("n_splits,n_waves,here", [(1, 4, 0), (1, 8, 0), (3, 4, 2), (2, 4, 1)])
+def test_attn_decode_at_the_tiles_edges(hd, ps, window, n_splits, n_waves, here):
+    """Contexts at the edges of tiles of 16 keys and of pages that are no power of two, one tile a wave,
+    two and more, pages that a window has given back marked -1; what no key lies in is NaN."""
+    k = _k()
+    ctx = [0, 14, 15, 16, 30, 31, 32, 33, 47, 48, 150, 1030]
+    c = PagedCase(torch.bfloat16, 2, 1, hd, ps, ctx, [1] * len(ctx), seed=hd + ps, window=window)
+    k.kv_write(c.k_new.to(DEV), c.v_new.to(DEV), c.kv, c.block_table_dev, c.token_req, c.positions)
+    if window:
+        for r, pos in enumerate(ctx):
+            c.block_table[r, : max(0, pos - window + 1) // ps] = -1
+        c.block_table_dev = c.block_table.to(DEV)
+    rows = torch.arange(c.T, dtype=torch.int32, device=DEV)
+    part_o = torch.empty(c.T * 2 * n_splits * hd, dtype=torch.float32, device=DEV)
+    part_ml = torch.empty(c.T * 2 * n_splits * 2, dtype=torch.float32, device=DEV)
+    out = torch.full((c.T, 2 * hd), float("nan")).to(torch.bfloat16).to(DEV)
+    k.attn_decode(out, c.q.to(DEV), c.kv, c.block_table_dev, c.token_req, c.positions, rows, c.T, 2, c.scale, window, n_splits,
+                  part_o, part_ml, n_waves, join_in_kernel=here)
+    err = (out.double().cpu() - c.reference()).abs().max().item()
+    assert err < _attn_tol(torch.bfloat16), err
+
+
 @pytest.mark.parametrize("case", [c for c in ATTN_CASES if c[2] in (16, 32, 64)] + [
     (8, 2, 16, 16, [700, 15, 16], [1, 1, 3], 0),
     (3, 1, 64, 4, [63, 64, 1000], [1, 2, 1], 100),
