@@ -825,15 +825,16 @@ struct Attention : Mixer {
       int n_splits = 1, n_waves = 4, key_tile = 32;
       // eight or more query heads a key head (a latent that all heads share): the kernel that takes
       // them together on the matrix cores, so a key is read and multiplied once for all of them.
-      // A block is four waves of sixteen keys at a time; a part for every 128 keys of the longest
-      // row, as many as give every CU two blocks.
+      // A block is four waves of sixteen keys at a time; a part for every 96 keys of the longest
+      // row (8 rows at up to 308 keys, planned for 512: 10.1 us in five parts, 12.2 in three), as many as
+      // give every CU two blocks.
       const int group = n_heads / n_kv_heads;
       const bool plain_scores = !terms || !(terms->head_scale || terms->slopes || terms->gate || terms->keep_first > 0 ||
                                             terms->softcap > 0.f || terms->dist_bias);
       if (plain_scores && bf16 && group >= 8 && (head_dim == 64 || head_dim == 128 || head_dim == 256)) {
         const long c = window <= 0 ? max_row_context : (max_row_context < window + 15 ? max_row_context : window + 15);
         const long blocks = (long)n_rows * n_kv_heads * ((group + 15) / 16);
-        long ns = c / 128, most = 2L * ctx->n_compute_units / (blocks < 1 ? 1 : blocks);
+        long ns = c / 96, most = 2L * ctx->n_compute_units / (blocks < 1 ? 1 : blocks);
         if (ns > most) ns = most;
         if (ns > 64) ns = 64;
         if (ns < 1) ns = 1;
