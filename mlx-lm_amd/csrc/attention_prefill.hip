@@ -22,6 +22,11 @@
 //    a thread reads the same 8 columns of two neighbouring keys and writes
 //    eight 32-bit words (two keys each).
 //  * Online softmax in 32-bit per lane; outputs leave as O^T accumulators.
+// What bounds it: the softmax's vector instructions, half of their time the exponentials (a tile of 128 queries x 64
+// keys is some 1,150 cycles of them a wave beside 512 of the matrix unit), and at few blocks the chain of one block.
+// 8,000 tokens of 25 heads of 64: 300 us, 0.68 PFLOP/s of the causal half (336 before the reference of the
+// probabilities was let lag); 2 x 1,024: 23.7 (25.0); 2 x 1,024 of 16 heads of 128: 30.9 (37.6); 690 tokens in four
+// requests of 16 heads of 256: 25 (36, when two tiles on their way did not fit the registers).
 #include "common.h"
 #include "attention_tiles.h"
 #include <type_traits>
@@ -78,8 +83,14 @@ __device__ __forceinline__ int key_of_row(int rho) {
 // POW2: the page size is a power of two (a key's page and row are a shift and a mask)
 // EXTRAS: the optional terms of PrefillArgs are looked at (the plain variant has no trace of them)
 // SHAPED (with EXTRAS): scores also pass the soft cap and take the distance table's term
-template <int HD, bool POW2, bool EXTRAS, bool SHAPED = false>
-__global__ __launch_bounds__(256, HD <= 64 ? 2 : 1) void attn_prefill_kernel(PrefillArgs p) {
+// GROUPS: groups of four waves, which take the key tiles by turns, each group with LDS of its own, and join their sums at
+// the end.  A block's walk over its keys is one tile after another (copy, barrier, products, softmax: some 1.2 us), and
+// where the blocks are few the longest walk is the kernel's time: two groups halve it.
+// (Two waves a SIMD, no fewer and no more, are named to the compiler: left alone it takes the registers of three, which
+// leaves it less to overlap, 25.5 us against 23.7 for 2 x 1,024 tokens of GPT-2 XL, 297 against 300 for 8,000.)
+template <int HD, bool POW2, bool EXTRAS, bool SHAPED, int GROUPS>
+__global__ __launch_bounds__(256 * GROUPS) __attribute__((amdgpu_waves_per_eu(HD <= 64 ? 2 : 1, HD <= 64 ? 2 : 1)))
+void attn_prefill_kernel(PrefillArgs p) {
   constexpr int KS_STRIDE = HD + 8;
   constexpr int DC = HD / 16;           // 16-column chunks of a head (QK contraction steps)
   constexpr int DT = HD / 32;           // 32-row tiles of O^T
@@ -87,10 +98,15 @@ __global__ __launch_bounds__(256, HD <= 64 ? 2 : 1) void attn_prefill_kernel(Pre
   constexpr int K_PER_T = (K_CHUNKS + 255) / 256;
   constexpr int V_ITEMS = (KT / 2) * (HD / 8);  // (key pair, 8-column chunk) items of a value tile
   constexpr int V_PER_T = (V_ITEMS + 255) / 256;
-  __shared__ __attribute__((aligned(16))) uint16_t Ks[KT * KS_STRIDE];
-  __shared__ __attribute__((aligned(16))) uint16_t Vt[HD * VT_STRIDE];
+  // tiles on their way: two, or one where a tile is so many registers that two would not fit (heads of 256)
+  constexpr int SETS = HD <= 128 ? 2 : 1, SECOND = SETS - 1;
+  constexpr int GROUP_LDS = KT * KS_STRIDE + HD * VT_STRIDE;
+  __shared__ __attribute__((aligned(16))) uint16_t tiles_lds[GROUPS * GROUP_LDS];
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int group = GROUPS > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0;
+  const int tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6;  // (within the group)
+  uint16_t* const Ks = tiles_lds + group * GROUP_LDS;
+  uint16_t* const Vt = Ks + KT * KS_STRIDE;
   // Which tile and head.  The tiles come with the most keys first, and a tile's heads are
   // neighbours in the launch, so the blocks with the longest walks start first and the short
   // ones fill in behind them (with the tiles as the fast index, a CU's two blocks were two
@@ -141,9 +157,9 @@ __global__ __launch_bounds__(256, HD <= 64 ? 2 : 1) void attn_prefill_kernel(Pre
 #pragma unroll
     for (int r = 0; r < 16; ++r) ot[dt][r] = 0.f;
 
-  // two tiles on their way (the keys' two sets as arrays of their own: as one array
-  // indexed by the set they stayed in scratch memory)
-  uint4 kreg0[K_PER_T], kreg1[K_PER_T], vreg[2][V_PER_T][2];
+  // (the keys' two sets as arrays of their own: as one array indexed by the set they stayed in
+  // scratch memory)
+  uint4 kreg0[K_PER_T], kreg1[K_PER_T], vreg[SETS][V_PER_T][2];
 
   // The request's page numbers go to LDS once: a load of keys or values then
   // depends on no other load from memory, and two tiles can be on their way
@@ -152,8 +168,8 @@ __global__ __launch_bounds__(256, HD <= 64 ? 2 : 1) void attn_prefill_kernel(Pre
   extern __shared__ int page_of[];  // [max_blocks]
   const int pg0 = k_lo / p.page_size;
   const int n_pg = (k_hi - 1) / p.page_size - pg0 + 1;
-  for (int i = tid; i < n_sink_pages; i += 256) page_of[i] = table[i];
-  for (int i = tid; i < n_pg; i += 256) page_of[n_sink_pages + i] = table[pg0 + i];
+  for (int i = threadIdx.x; i < n_sink_pages; i += 256 * GROUPS) page_of[i] = table[i];
+  for (int i = threadIdx.x; i < n_pg; i += 256 * GROUPS) page_of[n_sink_pages + i] = table[pg0 + i];
   __syncthreads();
 
   // Loads are never predicated and never zeroed: a key outside [k_lo, k_hi) is
@@ -221,18 +237,18 @@ __global__ __launch_bounds__(256, HD <= 64 ? 2 : 1) void attn_prefill_kernel(Pre
   };
 
   // One tile: its keys and values go from registers to LDS, the registers take
-  // the tile after the next, then the arithmetic.
+  // a later tile, then the arithmetic.
   // `steady` (a compile-time flag): the tile lies below every query of the block
   // and there is no window, so no wave is idle and nothing is masked; a loop of
   // such tiles has no branch inside, and the compiler lets the loads of the
   // other register set stay in flight while this one is staged.
-  // `kt_next2`: the first key of the tile after the next (its loads start here).
-  auto one_tile = [&](int kt_in, int kt_next2, const int set, auto steady) __attribute__((always_inline)) {
+  // `kt_next`: the first key of the tile whose loads start here, SETS tiles on.
+  auto one_tile = [&](int kt_in, int kt_next, const int set, auto steady) __attribute__((always_inline)) {
     constexpr bool STEADY = decltype(steady)::value;
     __syncthreads();  // the previous tile is no longer read
     stage(set);
     __syncthreads();
-    fetch(kt_next2, set);  // (beyond the last tile: harmless reads of the last key)
+    fetch(kt_next, set);  // (beyond the last tile: harmless reads of the last key)
     const bool sink = EXTRAS && kt_in >= SINK;
     const int kt = sink ? kt_in - SINK : kt_in;
     if constexpr (!STEADY) {
@@ -360,9 +376,21 @@ __global__ __launch_bounds__(256, HD <= 64 ? 2 : 1) void attn_prefill_kernel(Pre
         }
     }
     tmax = fmaxf(tmax, __shfl_xor(tmax, 32, WAVE));
-    const float m_new = fmaxf(m, tmax);
-    const float m_use = (m_new == -INFINITY) ? 0.f : m_new;  // a row with no key yet
-    const float alpha = exp2f(m - m_use);
+    // Probabilities are taken against `m`, which need not be the largest score: it follows only where a score of the
+    // wave's queries has passed it by 2^8 (a float and a bfloat16 keep as many digits of 200 as of 1, and a sum of
+    // such numbers is far from overflow).  Following every new maximum, some query of the 32 has one in most tiles, and
+    // the 32 products that rescale the outputs were paid nearly every time.
+    if (__any(tmax > m + 8.0f)) {
+      const float m_new = fmaxf(m, tmax);
+      const float alpha = exp2f(m - (m_new == -INFINITY ? 0.f : m_new));  // (a row with no key yet: zero)
+      l *= alpha;
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) ot[dt][r] *= alpha;
+      m = m_new;
+    }
+    const float m_use = (m == -INFINITY) ? 0.f : m;
     float lsum = 0.f;
     Frag8 pf[2][2];
 #pragma unroll
@@ -381,16 +409,10 @@ __global__ __launch_bounds__(256, HD <= 64 ? 2 : 1) void attn_prefill_kernel(Pre
         pf[s][c].u.z = pack_bf16x2(e[4], e[5]);
         pf[s][c].u.w = pack_bf16x2(e[6], e[7]);
       }
-    l = l * alpha + lsum;
-    m = m_new;
-    // ---- O^T = O^T * alpha + V^T P^T ---------------------------------------------
-    const bool rescale = __any(alpha != 1.0f);  // no row's maximum moved: nothing to scale
+    l += lsum;
+    // ---- O^T = O^T + V^T P^T -----------------------------------------------------
 #pragma unroll
     for (int dt = 0; dt < DT; ++dt) {
-      if (rescale) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) ot[dt][r] *= alpha;
-      }
       const uint16_t* vrow = Vt + (dt * 32 + ql) * VT_STRIDE + 8 * g;
 #pragma unroll
       for (int s = 0; s < 2; ++s)
@@ -408,32 +430,58 @@ __global__ __launch_bounds__(256, HD <= 64 ? 2 : 1) void attn_prefill_kernel(Pre
     // window's go on, whose loads are harmless reads of the last key)
     auto first_key = [&](int i) { return i < n_sink_tiles ? SINK + i * KT : kt0 + (i - n_sink_tiles) * KT; };
     const int n_all = n_sink_tiles + (k_hi - kt0 + KT - 1) / KT;
-    fetch(first_key(0), 0);
-    fetch(first_key(1), 1);
-    for (int i = 0; i < n_all; i += 2) {
-      one_tile(first_key(i), first_key(i + 2), 0, std::false_type{});
-      if (i + 1 >= n_all) break;  // uniform
-      one_tile(first_key(i + 1), first_key(i + 3), 1, std::false_type{});
+    fetch(first_key(group), 0);
+    if constexpr (SETS == 2) fetch(first_key(group + GROUPS), SECOND);
+    for (int i = 0; i < n_all; i += 2 * GROUPS) {
+      const int mine = i + group;
+      one_tile(first_key(mine), first_key(mine + SETS * GROUPS), 0, std::false_type{});
+      if (i + GROUPS >= n_all) break;  // uniform over the block
+      one_tile(first_key(mine + GROUPS), first_key(mine + (1 + SETS) * GROUPS), SECOND, std::false_type{});
     }
   } else {
-    fetch(kt0, 0);
-    fetch(kt0 + KT, 1);
-    int kt = kt0;
+    constexpr int STEP = GROUPS * KT;  // keys that the groups take at a time
+    int kt = kt0;                      // the first group's
+    const int ahead = group * KT;
+    fetch(kt + ahead, 0);
+    if constexpr (SETS == 2) fetch(kt + ahead + STEP, SECOND);
     if (p.window <= 0) {
-      for (; kt + 2 * KT - 1 <= pos0; kt += 2 * KT) {
-        one_tile(kt, kt + 2 * KT, 0, std::true_type{});
-        one_tile(kt + KT, kt + 3 * KT, 1, std::true_type{});
+      for (; kt + 2 * STEP - 1 <= pos0; kt += 2 * STEP) {
+        one_tile(kt + ahead, kt + ahead + SETS * STEP, 0, std::true_type{});
+        one_tile(kt + ahead + STEP, kt + ahead + (1 + SETS) * STEP, SECOND, std::true_type{});
       }
     }
-    for (; kt < k_hi; kt += 2 * KT) {  // the tiles around the diagonal, or all of them under a window
-      one_tile(kt, kt + 2 * KT, 0, std::false_type{});
-      if (kt + KT >= k_hi) break;  // uniform
-      one_tile(kt + KT, kt + 3 * KT, 1, std::false_type{});
+    for (; kt < k_hi; kt += 2 * STEP) {  // the tiles around the diagonal, or all of them under a window
+      one_tile(kt + ahead, kt + ahead + SETS * STEP, 0, std::false_type{});
+      if (kt + STEP >= k_hi) break;  // uniform
+      one_tile(kt + ahead + STEP, kt + ahead + (1 + SETS) * STEP, SECOND, std::false_type{});
     }
   }
 
   // the two halves of the wave hold different keys of the same query
   l += __shfl_xor(l, 32, WAVE);
+  if constexpr (GROUPS == 2) {
+    // the second group's sums go to the first through LDS, each thread's to the thread of the same queries
+    static_assert((DT * 16 + 2) * 256 * sizeof(float) <= sizeof(tiles_lds), "the sums fit where the tiles were");
+    float* const sums = (float*)tiles_lds + tid;
+    __syncthreads();  // no tile is read any more
+    if (group == 1) {
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) sums[(dt * 16 + r) * 256] = ot[dt][r];
+      sums[DT * 16 * 256] = m, sums[(DT * 16 + 1) * 256] = l;
+    }
+    __syncthreads();
+    if (group == 1) return;
+    const float m1 = sums[DT * 16 * 256], both = fmaxf(m, m1), to = both == -INFINITY ? 0.f : both;
+    const float w0 = exp2f(m - to), w1 = exp2f(m1 - to);  // (a group without a key of this query: zero)
+    l = l * w0 + sums[(DT * 16 + 1) * 256] * w1;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) ot[dt][r] = ot[dt][r] * w0 + sums[(dt * 16 + r) * 256] * w1;
+    m = both;
+  }
   if (q_live) {
     // (m is in units of log 2)
     if (p.sinks) l += exp2f(fmaf(p.sinks[h], 1.4426950408889634f, -m));
@@ -511,22 +559,37 @@ static int prefill_launch(void* out, const void* q, int ldq, int ldo, const void
   const bool shaped = p.softcap > 0.f || p.dist_bias;
   const bool extras = head_scale || slopes || gate || p.keep_first > 0 || shaped;
   if (n_tiles > 65535) FAIL("attn_prefill: %d tiles in a launch, at most 65535", n_tiles);
-  dim3 grid(n_heads, n_tiles), block(256);
   // a request's page numbers lie in LDS beside the tiles
   if (max_blocks > 7168)
     FAIL("attn_prefill: block tables of %d pages a request do not fit beside the tiles (at most 7168)", max_blocks);
   // (the kept first keys' pages lie before the window's; a page can be in both runs)
   const size_t lds = (size_t)(max_blocks + (extras ? 2 : 0)) * sizeof(int);
   const bool pow2 = p.page_shift >= 0;
-#define LAUNCH_PREFILL(HD)                                                                                  \
-  if (shaped) {                                                                                             \
-    if (pow2) hipLaunchKernelGGL((attn_prefill_kernel<HD, true, true, true>), grid, block, lds, stream, p); \
-    else hipLaunchKernelGGL((attn_prefill_kernel<HD, false, true, true>), grid, block, lds, stream, p);     \
-  } else if (extras) {                                                                                             \
-    if (pow2) hipLaunchKernelGGL((attn_prefill_kernel<HD, true, true>), grid, block, lds, stream, p);      \
-    else hipLaunchKernelGGL((attn_prefill_kernel<HD, false, true>), grid, block, lds, stream, p);          \
-  } else if (pow2) hipLaunchKernelGGL((attn_prefill_kernel<HD, true, false>), grid, block, lds, stream, p); \
-  else hipLaunchKernelGGL((attn_prefill_kernel<HD, false, false>), grid, block, lds, stream, p)
+  // Two groups a block where the blocks are no more than the CUs, so that a block's walk is the kernel's time: 512 queries
+  // on 4,000 earlier keys, 25 heads of 64 (100 blocks) 55 us beside 68, 1,000 keys of 16 heads of 32 13.2 / 16.2, 333 of
+  // 25 of 64 10.0 / 10.2.  With more blocks than CUs they are in each other's way (2 x 1,024 tokens of 25 heads, 400
+  // blocks: 26.2 / 23.6).  Heads of 128 and more take the registers of a whole SIMD a wave.
+  const bool two = head_dim <= 64 && pow2 && max_blocks <= 4096 && (long)n_heads * n_tiles <= n_compute_units();
+  const dim3 grid(n_heads, n_tiles), block(two ? 512 : 256);
+#define LAUNCH_AS(HD, POW2, GROUPS)                                                                                      \
+  do {                                                                                                                  \
+    if (shaped)                                                                                                         \
+      hipLaunchKernelGGL((attn_prefill_kernel<HD, POW2, true, true, GROUPS>), grid, block, lds, stream, p);             \
+    else if (extras)                                                                                                    \
+      hipLaunchKernelGGL((attn_prefill_kernel<HD, POW2, true, false, GROUPS>), grid, block, lds, stream, p);            \
+    else                                                                                                                \
+      hipLaunchKernelGGL((attn_prefill_kernel<HD, POW2, false, false, GROUPS>), grid, block, lds, stream, p);           \
+  } while (0)
+#define LAUNCH_PREFILL(HD)              \
+  do {                                  \
+    if (two) {                          \
+      LAUNCH_AS(HD, true, (HD <= 64 ? 2 : 1)); \
+    } else if (pow2) {                  \
+      LAUNCH_AS(HD, true, 1);           \
+    } else {                            \
+      LAUNCH_AS(HD, false, 1);          \
+    }                                   \
+  } while (0)
   if (head_dim == 32) {
     LAUNCH_PREFILL(32);
   } else if (head_dim == 64) {
@@ -537,6 +600,7 @@ static int prefill_launch(void* out, const void* q, int ldq, int ldo, const void
     LAUNCH_PREFILL(256);
   }
 #undef LAUNCH_PREFILL
+#undef LAUNCH_AS
   CHECK_LAUNCH("attn_prefill");
   return 0;
 }

@@ -585,6 +585,32 @@ def test_attn_prefill(case):
     assert err < 2.5e-2, err
 
 
+@pytest.mark.parametrize("hd,H,ctx,ql,window", [(64, 3, [0, 61], [200, 129], 0), (32, 2, [63], [300], 0), (64, 140, [5], [257], 0),
+                                              (128, 2, [0], [190], 0), (256, 2, [30], [150], 0), (64, 2, [100], [140], 50)])
+@pytest.mark.parametrize("step", [0.02, 0.4, 30.0])
+def test_attn_prefill_with_scores_that_keep_growing(hd, H, ctx, ql, window, step):
+    """Scores that grow by `step` with every key: the largest so far moves in every tile, by less than the
+    probabilities' reference may lag behind it, by about that, and by far more; with blocks fewer than the
+    compute units (their keys in two groups of waves) and more.  (The weights are rounded to bfloat16,
+    2^-9 of each, and meet values of up to 4.5.)"""
+    k = _k()
+    c = PagedCase(torch.bfloat16, H, 1, hd, 16, ctx, ql, seed=hd + H, window=window)
+    c.q = c.q * 0.01
+    c.q[:, ::hd] = 1.0
+    for r, n in enumerate(c.total):
+        c.k_full[r][:, 0, 0] = (torch.arange(n) * (step / c.scale)).to(torch.bfloat16)
+    c.k_new = torch.cat([c.k_full[r][c.ctx_lens[r] :].reshape(c.q_lens[r], -1) for r in range(len(ctx))])
+    for r in range(len(ctx)):
+        for pos in range(c.ctx_lens[r]):
+            c.pool[c.block_table[r, pos // 16], 0, :, pos % 16] = c.k_full[r][pos].to(DEV)
+    k.kv_write(c.k_new.to(DEV), c.v_new.to(DEV), c.kv, c.block_table_dev, c.token_req, c.positions)
+    tiles = c.tiles(k.attn_tile_sizes()[1])
+    out = torch.full((c.T, H * hd), float("nan")).to(torch.bfloat16).to(DEV)
+    k.attn_prefill(out, c.q.to(DEV), c.kv, c.block_table_dev, c.token_req, c.positions, tiles, tiles.shape[0], H, c.scale, window)
+    err = (out.double().cpu() - c.reference()).abs().max().item()
+    assert err < 2.5e-2, err
+
+
 def test_attn_prefill_far_key_stands_out():
     """Every query of a long portion points at one far key of its own."""
     k = _k()
