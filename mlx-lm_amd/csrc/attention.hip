@@ -457,10 +457,11 @@ __global__ __launch_bounds__(256) void attn_tile_wide_kernel(AttnArgs p) {
 
 // ---------------------------------------------------------------------------
 // attn_tile_mfma: float storage, head_dim = 64 * NV, page_size a multiple of 16.  Grid
-// (ceil(n_tiles / 4), n_heads), 256 threads; every wave takes a tile of its own and walks its
-// keys 16 at a time (no LDS, no barrier).  v_mfma_f32_16x16x4_f32 computes D = A B for A 16 x 4
-// and B 4 x 16: lane l brings A[l % 16][l / 16] and B[l / 16][l % 16] and gets
-// D[4 * (l / 16) + r][l % 16] in accumulator r.
+// (n_tiles, n_heads), 256 threads: one tile of up to 16 queries a block.  The keys go to the four
+// waves 16 at a time in turn; each keeps a softmax of its own (no barrier on the walk), and the
+// four are put together through LDS at the end.
+// v_mfma_f32_16x16x4_f32 computes D = A B for A 16 x 4 and B 4 x 16: lane l brings A[l % 16][l / 16]
+// and B[l / 16][l % 16] and gets D[4 * (l / 16) + r][l % 16] in accumulator r.
 //   scores, transposed: S^T[key][query] = sum_d K[key][d] Q[query][d].  The four floats of one
 //     16-byte load go to four instructions; which d an instruction's four slots stand for is
 //     free as long as both operands agree: lane (x = l % 16, g = l / 16) loads columns
@@ -474,14 +475,23 @@ __global__ __launch_bounds__(256) void attn_tile_wide_kernel(AttnArgs p) {
 //     is column 16 * g + 4 * r' + c, so a lane ends with 16 consecutive columns of its query.
 // Keys of a tile beyond the last one written are read from that one instead (their scores are
 // masked; a page's unwritten rows may hold anything, and 0 x NaN is NaN).
+// What bounds it: the walk is a chain of products, softmax and products again, 0.5 us of matrix
+// work in about twice that.  With a wave a tile of queries the last of a prompt's tiles walked
+// alone at the end while most of the chip idled; a tile's keys over four waves end four times
+// earlier.  Prompts of 215 + 480 + 330 tokens, 20 heads of 64: 55.7 us with a wave a tile, 31.1 with
+// four, 28.4 since the masks, shuffles and rescaling are left out where no key needs them; one of
+// 80 tokens, 12 heads: 8.6 and 5.9; two of 1,024: 162 and 107; one of 4,000: 787 and 493 (its matrix
+// work alone takes 266); two of 500, 16 heads of 128: 62 and 57.  Four waves a SIMD want at most 128
+// registers for heads of 64, which the compiler keeps only when told.
 
 template <int NV>
-__global__ __launch_bounds__(256) void attn_tile_mfma_kernel(AttnArgs p, int n_tiles) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NV == 1 ? 4 : 2))) void attn_tile_mfma_kernel(AttnArgs p) {
   constexpr int HD = 64 * NV;
   constexpr int NT = 4 * NV;  // 16-byte loads that cover a row of HD floats, per lane group
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int tile = blockIdx.x * 4 + wave;
-  if (tile >= n_tiles) return;
+  constexpr int LDP = HD + 4;  // (the 16 queries' rows begin in 16 different groups of four banks)
+  __shared__ float part_o[4][16][LDP], part_ml[4][2][16];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int tile = blockIdx.x;
   const int x = lane & 15, g = lane >> 4;
   // (the same in every lane: said so, the page numbers below come through scalar loads)
   const int row0 = __builtin_amdgcn_readfirstlane(p.items[2 * tile]);
@@ -500,7 +510,7 @@ __global__ __launch_bounds__(256) void attn_tile_mfma_kernel(AttnArgs p, int n_t
 #pragma unroll
     for (int t = 0; t < NT; ++t) qv[t] = *(const f32x4_t*)(qrow + 16 * t) * p.scale;
   }
-  const int qpos = pos0 + x;
+  const int qpos = pos0 + min(x, nq - 1);
   const int k_hi = pos0 + nq;  // one past the last key any query of the tile sees
   const int k_lo = p.window > 0 ? max(0, pos0 - p.window + 1) : 0;
   const size_t head_off = (size_t)kv_head * p.page_size * HD;
@@ -526,11 +536,14 @@ __global__ __launch_bounds__(256) void attn_tile_mfma_kernel(AttnArgs p, int n_t
   for (int i = 0; i < NT; ++i) o[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 
   // the page of the tile after next is looked up while the next tile's keys are on their way
-  int kt = (k_lo / 16) * 16;
-  const int last_block = (k_hi - 1) / p.page_size;
-  ask(kt, table[kt / p.page_size]);
-  int page_next = table[min((kt + 16) / p.page_size, last_block)];
-  for (; kt < k_hi; kt += 16) {
+  int kt = (k_lo / 16) * 16 + 16 * wave;
+  const int last_kt = ((k_hi - 1) / 16) * 16;  // where the last 16 keys begin
+  int page_next = 0;
+  if (kt < k_hi) {
+    ask(kt, table[kt / p.page_size]);
+    page_next = table[min(kt + 64, last_kt) / p.page_size];
+  }
+  for (; kt < k_hi; kt += 64) {
     f32x4_t s = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
@@ -544,37 +557,36 @@ __global__ __launch_bounds__(256) void attn_tile_mfma_kernel(AttnArgs p, int n_t
     for (int v = 0; v < NV; ++v)
 #pragma unroll
       for (int r = 0; r < 4; ++r) vc[v][r] = vf[v][r];
-    ask(min(kt + 16, ((k_hi - 1) / 16) * 16), page_next);  // the next tile (after the last: the last again)
-    page_next = table[min((kt + 32) / p.page_size, last_block)];
+    ask(min(kt + 64, last_kt), page_next);  // this wave's next keys (after its last: the tile's last)
+    page_next = table[min(kt + 128, last_kt) / p.page_size];
     __builtin_amdgcn_sched_barrier(0);  // (the loads stay here, ahead of the softmax and the second products)
 
-    bool ok[4];
-    float tmax = -INFINITY;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int key = kt + 4 * g + r;
-      ok[r] = x < nq && key <= qpos && key >= k_lo && (p.window == 0 || key > qpos - p.window);
-      tmax = fmaxf(tmax, ok[r] ? s[r] : -INFINITY);
-    }
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 16, WAVE));
-    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, WAVE));
-    const float m_new = fmaxf(m, tmax);
-    float alpha = 1.f, sum = 0.f;
-    f32x4_t pr = {0.f, 0.f, 0.f, 0.f};
-    if (m_new != -INFINITY) {
-      alpha = expf(m - m_new);
+    // (keys that every query of the tile sees, all but the last of a walk, need no mask)
+    if (kt + 15 > pos0 || (p.window > 0 && kt <= pos0 + nq - 1 - p.window)) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        pr[r] = ok[r] ? expf(s[r] - m_new) : 0.f;
-        sum += pr[r];
+        const int key = kt + 4 * g + r;
+        if (key > qpos || (p.window > 0 && key <= qpos - p.window)) s[r] = -INFINITY;
       }
     }
-    sum += __shfl_xor(sum, 16, WAVE);
-    sum += __shfl_xor(sum, 32, WAVE);
-    l = l * alpha + sum;
-    m = m_new;
+    float tmax = fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]));
+    if (__any(tmax > m)) {  // (few of a long walk's tiles hold a new greatest score: no shuffles for the others)
+      tmax = fmaxf(tmax, __shfl_xor(tmax, 16, WAVE));
+      tmax = fmaxf(tmax, __shfl_xor(tmax, 32, WAVE));
+      const float m_new = fmaxf(m, tmax);
+      const float alpha = m_new == -INFINITY ? 1.f : expf(m - m_new);
+      l *= alpha;
+      m = m_new;
 #pragma unroll
-    for (int i = 0; i < NT; ++i) o[i] *= alpha;
+      for (int i = 0; i < NT; ++i) o[i] *= alpha;
+    }
+    const float ref = m == -INFINITY ? 0.f : m;  // (a query that has seen nothing yet, or nothing above -infinity)
+    f32x4_t pr;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      pr[r] = expf(s[r] - ref);
+      l += pr[r];
+    }
 #pragma unroll
     for (int v = 0; v < NV; ++v)
 #pragma unroll
@@ -586,15 +598,37 @@ __global__ __launch_bounds__(256) void attn_tile_mfma_kernel(AttnArgs p, int n_t
       }
   }
 
-  if (x < nq) {
-    const float inv = head_gate_of(p, row0 + x, h) / with_sink(p, h, m, l);
-    float* orow = (float*)p.out + (size_t)(row0 + x) * p.ldo + h * HD + 16 * g;
+  l += __shfl_xor(l, 16, WAVE);  // (each lane group has summed its own keys)
+  l += __shfl_xor(l, 32, WAVE);
+  // the four waves' sums, put on the greatest of their references
+  if (g == 0) part_ml[wave][0][x] = m, part_ml[wave][1][x] = l;
 #pragma unroll
-    for (int v = 0; v < NV; ++v)
+  for (int v = 0; v < NV; ++v)
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
-        *(f32x4_t*)(orow + 64 * v + 4 * r) =
-            f32x4_t{o[4 * v][r], o[4 * v + 1][r], o[4 * v + 2][r], o[4 * v + 3][r]} * inv;
+    for (int r = 0; r < 4; ++r)
+      *(f32x4_t*)&part_o[wave][x][64 * v + 16 * g + 4 * r] =
+          f32x4_t{o[4 * v][r], o[4 * v + 1][r], o[4 * v + 2][r], o[4 * v + 3][r]};
+  __syncthreads();
+  const int y = threadIdx.x >> 4;  // a thread's query; its columns: 4 * (threadIdx.x % 16) + 64 * v
+  if (y < nq) {
+    float big = -INFINITY, total = 0.f;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) big = fmaxf(big, part_ml[w][0][y]);
+    float weight[4];
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      weight[w] = part_ml[w][0][y] == -INFINITY ? 0.f : expf(part_ml[w][0][y] - big);
+      total += weight[w] * part_ml[w][1][y];
+    }
+    const float inv = head_gate_of(p, row0 + y, h) / with_sink(p, h, big, total);
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      const int d = 64 * v + 4 * x;
+      f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int w = 0; w < 4; ++w) acc += *(const f32x4_t*)&part_o[w][y][d] * weight[w];
+      *(f32x4_t*)((float*)p.out + (size_t)(row0 + y) * p.ldo + h * HD + d) = acc * inv;
+    }
   }
 }
 
@@ -893,11 +927,11 @@ static int tile_launch(void* out, const void* q, int ldq, int ldo, const void* k
   if (fill_shape(p, "attn_tile", shape)) return 1;
   if (!has_extras(p) && dtype == DT_F32 && (head_dim == 64 || head_dim == 128) && page_size % 16 == 0 && ldq % 4 == 0 &&
       ldo % 4 == 0 && (((uintptr_t)q | (uintptr_t)out) & 15) == 0) {
-    dim3 grid((n_tiles + 3) / 4, n_heads), block(256);
+    dim3 grid(n_tiles, n_heads), block(256);
     if (head_dim == 64)
-      hipLaunchKernelGGL(attn_tile_mfma_kernel<1>, grid, block, 0, stream, p, n_tiles);
+      hipLaunchKernelGGL(attn_tile_mfma_kernel<1>, grid, block, 0, stream, p);
     else
-      hipLaunchKernelGGL(attn_tile_mfma_kernel<2>, grid, block, 0, stream, p, n_tiles);
+      hipLaunchKernelGGL(attn_tile_mfma_kernel<2>, grid, block, 0, stream, p);
     CHECK_LAUNCH("attn_tile");
     return 0;
   }

@@ -370,6 +370,35 @@ def test_attn_tile_float32_far_key_stands_out():
         assert (out.double().cpu() - c.reference()).abs().max().item() < _attn_tol(torch.float32), far
 
 
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("ctx,ql,window", [([0, 15, 16], [1, 1, 1], 0), ([0, 48, 63], [64, 17, 2], 0), ([127, 0], [66, 65], 0),
+                                           ([100], [140], 33), ([190, 3], [20, 90], 64)])
+@pytest.mark.parametrize("step", [0.0, 0.4, 30.0])
+def test_attn_tile_float32_keys_shared_by_four_waves(hd, ctx, ql, window, step):
+    """Walks of 1 to 4 times 64 keys and one around, windows that leave waves without a key, and scores that
+    do not grow, grow in every tile of keys, or leave the last key alone.  (A weight's exponent is a difference
+    of scores up to 30 * 260: rounded to 2^-24 of that, 4.6e-4, and meets values of up to 4.5 where two weights
+    count, which a step of 30 does not leave; at 0.4, 6.2e-6 each.)"""
+    k = _k()
+    H = 3
+    c = PagedCase(torch.float32, H, 1, hd, 16, ctx, ql, seed=hd, window=window)
+    if step:
+        c.q = c.q * 0.01
+        c.q[:, ::hd] = 1.0
+        for r, n in enumerate(c.total):
+            c.k_full[r][:, 0, 0] = torch.arange(n) * (step / c.scale)
+        c.k_new = torch.cat([c.k_full[r][c.ctx_lens[r] :].reshape(c.q_lens[r], -1) for r in range(len(ctx))])
+        for r in range(len(ctx)):
+            for pos in range(c.ctx_lens[r]):
+                c.pool[c.block_table[r, pos // 16], 0, :, pos % 16] = c.k_full[r][pos].to(DEV)
+    k.kv_write(c.k_new.to(DEV), c.v_new.to(DEV), c.kv, c.block_table_dev, c.token_req, c.positions)
+    tiles = c.tiles()
+    out = torch.full((c.T, H * hd), float("nan"), dtype=torch.float32, device=DEV)
+    k.attn_tile(out, c.q.to(DEV), c.kv, c.block_table_dev, c.token_req, c.positions, tiles, tiles.shape[0], H, c.scale, window)
+    err = (out.double().cpu() - c.reference()).abs().max().item()
+    assert err < (1e-4 if step < 1 else 1e-3), err
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_kv_write_from_rows_that_are_not_aligned(dtype):
     """Sources that start in the middle of a 16-byte piece take the element-wise kernel: same pages."""
