@@ -304,19 +304,23 @@ __global__ __launch_bounds__(64 * SKF_MAX_WAVES) void gemm_f32_skinny_kernel(Gem
 DEFINE_LAST_ERROR(mlxlm_last_error)
 
 // What a tile shape costs in microseconds: its products at the speed of a CU's matrix units (2.5e-4 an output and 64
-// columns; a block alone on its CU, one wave a SIMD, a fifth more), blocks that share a CU one after another, and a
-// fixed part for the first step's way and the epilogue.  Against the times of 6 numbers of rows from 80 to 2,048 and ten
-// matrices of widths 768 to 1,600, each with K in 1 to 8 parts, the choice is within 3 % of the best on average.
+// columns, 8 % more in the smallest tiles, which read most, 3 % more in the largest; a block alone on its CU, one wave a
+// SIMD, a fifth more), blocks that share a CU one after another, and a fixed part for the first step's way and the
+// epilogue.  Against the times of 11 numbers of rows from 80 to 2,048 and ten matrices of widths 768 to 1,600, each with
+// K in 1 to 8 parts, the choice is within 0.7 % of the best on average and 7 % at worst (1.7 % and 13 % with every tile
+// at the same rate).
 struct F32Price {
   int variant, bm, bn;
+  double rate;
 };
-static const F32Price F32_PRICES[] = {
-    {1, F32Tile64x128::BM, F32Tile64x128::BN}, {2, F32Tile64::BM, F32Tile64::BN}, {4, F32Tile32x64::BM, F32Tile32x64::BN}};
+static const F32Price F32_PRICES[] = {{1, F32Tile64x128::BM, F32Tile64x128::BN, 1.03},
+                                      {2, F32Tile64::BM, F32Tile64::BN, 1.0},
+                                      {4, F32Tile32x64::BM, F32Tile32x64::BN, 1.08}};
 static double price(const F32Price& s, int M, int N, int K, int n_splits) {
   const long tiles = (long)((M + s.bm - 1) / s.bm) * ((N + s.bn - 1) / s.bn);
   const long n = (tiles * n_splits + n_compute_units() - 1) / n_compute_units();
   const int chunks = ((K + 63) / 64 + n_splits - 1) / n_splits;
-  return 4.0 + (n == 1 ? 1.2 : 1.0) * n * chunks * (2.5e-4 * s.bm * s.bn);
+  return 4.0 + (n == 1 ? 1.2 : 1.0) * n * chunks * (2.5e-4 * s.rate * s.bm * s.bn);
 }
 static int cheapest_shape(int M, int N, int K, int n_splits, double* us) {
   int variant = 0;
@@ -351,7 +355,7 @@ extern "C" int gemm_f32_splits(int M, int N, int K, int fused, int force) {
       double us = 0.0;
       cheapest_shape(M, N, K, s, &us);
       if (s > 1) us += (fused ? 1.0 : 2.5) + 8.0 * (fused ? s - 1 : s) * (double)M * N / 3e6;
-      if (s == 1 || us < 0.95 * best_us) want = s, best_us = us;
+      if (s == 1 || us < 0.99 * best_us) want = s, best_us = us;
     }
   }
   if (want < 1) want = 1;
