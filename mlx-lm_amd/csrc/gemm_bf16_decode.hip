@@ -408,33 +408,39 @@ __global__ __launch_bounds__(NW * 64) void gemm_bf16_decode_kernel(DecodeGemmArg
 
 // ---------------------------------------------------------------------------
 // 17 to 64 rows.  The weights still stream exactly once and all of a block's are in flight from
-// its first instruction on: a block of four waves owns 32 output features (two packed chunks)
-// and a slice of K of at most 28 k-blocks; wave w takes the slice's k-blocks w, w + 4, ... and
-// holds their weights in registers (seven k-blocks of two chunks: 112 registers a lane).  The
-// activations are the MFMA's other operand, two or three tiles of 16 rows, read straight from
-// memory (the L2s: every block reads the same rows) a k-block ahead; no LDS on the way.  They
-// come row-major or, much faster, in the packed order (packed_at: a wave's load is then 1 KB of
-// consecutive bytes instead of sixteen pieces of 64: GPT-2 XL's four products at 48 rows took
-// 15.8 / 17.3 / 12.8 / 17.0 us from rows and 10.8 / 12.4 / 8.0 / 11.8 packed), which the kernels
-// that make these rows write where the host asks them to (the sum-and-norm, decode attention,
-// this kernel's own epilogue).  The four waves' tiles are summed in their order through LDS and
-// finished as in the kernel above.  The tile kernels of gemm_bf16.hip need K split over some 220
-// blocks at these sizes and a second kernel for the sum; here the wide products are one launch of
-// 150 or 200 blocks, and the narrow ones split K in two or four.  49 to 64 rows go as two groups
-// of two tiles, a block each, eight block ids apart: both on one die, so that the second finds
-// the weights in that die's L2 (the fetch counter shows them read from memory once).
-// (Other shapes measured at 64 rows of GPT-2 XL's sizes, packed rows, a decode step of twelve
-// layers: four tiles a block with 32 features and four or eight waves 1.34 and 1.29 ms, with 16
-// features 1.58, sixteen waves that hold everything after one trip to memory 1.65; two groups
-// 1.28; the tile kernels with K split and their second kernels 1.33.)
-#define RW 4          // waves a block
+// its first instructions on: a block owns 32 output features (two packed chunks) and a slice of K
+// of at most 28 k-blocks; its waves take the slice's k-blocks in turn and hold their weights in
+// registers (four waves seven k-blocks of two chunks, 112 registers a lane, eight waves four).  The
+// activations are the MFMA's other operand, one to four tiles of 16 rows, read straight from
+// memory (the L2s: every block reads the same rows), the first k-blocks' ahead of the weights; no
+// LDS on the way.  They come row-major or, much faster, in the packed order (packed_at: a wave's
+// load is then 1 KB of consecutive bytes instead of sixteen pieces of 64), which the kernels that
+// make these rows write where the host asks them to (the sum-and-norm, decode attention, this
+// kernel's own epilogue).  The waves' tiles are summed in their order through LDS and finished as
+// in the kernel above.  The tile kernels of gemm_bf16.hip need K split over some 220 blocks at
+// these sizes and a second kernel for the sum; here the wide products are one launch of 150 or 200
+// blocks, and the narrow ones split K in two or four.
+// What bounds it: the trips to the L2s and to memory, which follow one another in a wave, and the
+// registers that hide them; the weights alone would take 2.5 to 3.5 us of these times.  Packed
+// rows, features x K (parts of K), weights from memory, us on an MI355X; before = a block of two
+// tiles with rows and weights the other way round and a branch on the order of the rows at every
+// k-block, which kept the loads apart:
+//                          17 rows        32 rows        48 rows        64 rows
+//   4,800 x 1,600 (1)    8.1 ->  7.5    8.2 ->  7.6    9.8 ->  8.4   11.4 ->  8.9
+//   1,600 x 1,600 (2)    6.1 ->  4.7    6.1 ->  4.7    7.6 ->  5.3    5.9 ->  5.4
+//   6,400 x 1,600 (1)    8.8 ->  8.1    8.8 ->  8.1   10.3 ->  8.8   11.7 ->  9.2
+//   1,600 x 6,400 (4)    8.3 ->  7.8    8.6 ->  8.1   10.1 ->  8.6   11.8 ->  9.3
+//   3,840 x 1,280 (1)    7.1 ->  5.6    7.0 ->  5.6    8.5 ->  6.4    6.9 ->  6.5
+//   1,280 x 5,120 (3)    7.6 ->  5.9    7.8 ->  6.1    9.2 ->  6.9    8.0 ->  7.1
+//   2,304 x   768 (2)    5.9 ->  4.8    5.9 ->  4.8    7.4 ->  5.1    8.6 ->  5.3
+#define RW 4          // waves a block of one or two tiles of rows; twice as many with three or four
 #define R_FEATURES 32 // output features a block
-#define R_HELD 7      // k-blocks whose weights a wave holds
+#define R_HELD 7      // k-blocks whose weights one of RW waves holds
 #define ROWS_MAX_M 64
-#define ROWS_GROUP_FROM 49    // from this many rows on: groups of 32 rows, a block each
 #define ROWS_WANT_BLOCKS 100  // a split of K where the features give fewer blocks than this
-// R_TILES: tiles of 16 rows; FT: chunks of 16 features a block; WAVES: waves a block; HELD: k-blocks a wave holds
-template <int R_TILES, int FT, int WAVES, int HELD>
+// R_TILES: tiles of 16 rows; FT: chunks of 16 features a block; WAVES: waves a block; HELD: k-blocks a wave
+// holds; AHEAD: k-blocks whose rows are on their way
+template <int R_TILES, int FT, int WAVES, int HELD, int AHEAD>
 __global__ __launch_bounds__(WAVES * 64) void gemm_bf16_rows_kernel(DecodeGemmArgs p) {
   __shared__ float red[WAVES][R_TILES * FT][256];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -452,6 +458,30 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_bf16_rows_kernel(DecodeGemmAr
   const int n_fb = (p.N + 15) / 16;
   const int koff = (lane >> 4) * 16;
 
+  // the activations of a k-block: lane l holds row l % 16 of each tile, 16 columns from
+  // (l / 16) * 16 on (rows beyond M repeat the last; what they give is not stored)
+  const int m_tiles = (p.M + 15) / 16;
+  const uint16_t* abase[R_TILES];
+#pragma unroll
+  for (int rt = 0; rt < R_TILES; ++rt)
+    abase[rt] = p.a_packed ? p.A + (size_t)min(t0 + rt, m_tiles - 1) * n_chunks_all * 1024 + lane * 8
+                           : input_of(p, n0) + (size_t)min((t0 + rt) * 16 + (lane & 15), p.M - 1) * p.lda;
+  auto load_a = [&](Frag (&a)[R_TILES][2], int i) {
+    const int c = c_begin + min(wave + WAVES * i, n_chunks - 1);
+    const int k = c * 64 + koff;
+    const int first = p.a_packed ? c * 1024 : min(k, p.K - 8);
+    const int second = p.a_packed ? c * 1024 + 512 : min(k + 8, p.K - 8);
+#pragma unroll
+    for (int rt = 0; rt < R_TILES; ++rt) {
+      a[rt][0].u = *(const uint4*)(abase[rt] + first);
+      a[rt][1].u = *(const uint4*)(abase[rt] + second);
+    }
+  };
+  // (the first k-blocks' rows before the weights: loads come back in order, and the L2s' answers need not wait
+  // for memory's)
+  Frag a[AHEAD][R_TILES][2];
+#pragma unroll
+  for (int i = 0; i < AHEAD; ++i) load_a(a[i], i);
   // the weights, all at once (k-blocks beyond the slice repeat its last one and are not used)
   Frag w[HELD][FT][2];
 #pragma unroll
@@ -465,30 +495,6 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_bf16_rows_kernel(DecodeGemmAr
       w[i][ft][1].u = *(const uint4*)(t + 512);
     }
   }
-  // the activations of a k-block: lane l holds row l % 16 of each tile, 16 columns from
-  // (l / 16) * 16 on (rows beyond M repeat the last; what they give is not stored)
-  const uint16_t* arow[R_TILES];
-#pragma unroll
-  for (int rt = 0; rt < R_TILES; ++rt) arow[rt] = input_of(p, n0) + (size_t)min((t0 + rt) * 16 + (lane & 15), p.M - 1) * p.lda;
-  const int m_tiles = (p.M + 15) / 16;
-  auto load_a = [&](Frag (&a)[R_TILES][2], int i) {
-    const int c = c_begin + min(wave + WAVES * i, n_chunks - 1);
-    const int k = c * 64 + koff;
-    if (p.a_packed) {
-#pragma unroll
-      for (int rt = 0; rt < R_TILES; ++rt) {
-        const uint16_t* t = p.A + ((size_t)min(t0 + rt, m_tiles - 1) * n_chunks_all + c) * 1024 + lane * 8;
-        a[rt][0].u = *(const uint4*)t;
-        a[rt][1].u = *(const uint4*)(t + 512);
-      }
-    } else {
-#pragma unroll
-      for (int rt = 0; rt < R_TILES; ++rt) {
-        a[rt][0].u = *(const uint4*)(arow[rt] + min(k, p.K - 8));
-        a[rt][1].u = *(const uint4*)(arow[rt] + min(k + 8, p.K - 8));
-      }
-    }
-  };
   f32x4_t acc[R_TILES][FT];
 #pragma unroll
   for (int rt = 0; rt < R_TILES; ++rt)
@@ -532,14 +538,10 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_bf16_rows_kernel(DecodeGemmAr
       e_page[k] = (kv ? p.block_table : some_ints)[kv ? (size_t)req * p.max_blocks + e_pos[k] / p.page_size : 0];
     }
   }
-  Frag a0[R_TILES][2], a1[R_TILES][2];
-  load_a(a0, 0);
 #pragma unroll
-  for (int i = 0; i < HELD; i += 2) {
-    if (i + 1 < HELD) load_a(a1, i + 1);
-    multiply(a0, i);
-    if (i + 2 < HELD) load_a(a0, i + 2);
-    if (i + 1 < HELD) multiply(a1, i + 1);
+  for (int i = 0; i < HELD; ++i) {
+    multiply(a[i % AHEAD], i);
+    if (i + AHEAD < HELD) load_a(a[i % AHEAD], i + AHEAD);
   }
 
   // ---- sum the waves' tiles in their order, then the epilogue -----------------
@@ -959,20 +961,26 @@ static int rows_launch(void* out, const void* A, int lda, const void* W, const f
     if (ws_floats < (size_t)n_splits * M * N)
       FAIL("gemm_bf16_rows: workspace of %zu floats is too small for %d splits of %d x %d", ws_floats, n_splits, M, N);
   }
-  p.row_groups = M >= ROWS_GROUP_FROM ? (M + 31) / 32 : 1;
+  // Tiles of 16 rows a block: as few as leave a block to a compute unit at most (they are done sooner: 48 and 64 rows
+  // of 3,840 x 1,280 6.4 and 6.5 us with two, 7.1 and 7.6 with all), all of them where even two a block give more
+  // blocks than units (6,400 x 1,600 at 64 rows: 9.2, with two 9.8, with one 11.2).  Up to two tiles four waves that
+  // hold seven k-blocks and ask for four k-blocks' rows at first; with more the rows' registers are short, and eight
+  // waves that hold four and ask one ahead are faster (48 rows of 4,800 x 1,600: 8.4 against 8.8).
   // (the grid holds whole eights of feature blocks, so that a group's blocks and the next group's
   // are on the same dies; the surplus blocks return at once)
-  const int fbs = ((N + R_FEATURES - 1) / R_FEATURES + 7) / 8 * 8;
-  const dim3 grid(fbs * p.row_groups, n_splits), block(RW * 64);
-  // (eight waves of four k-blocks each where a block takes all the rows: a wave's trips to the L2s for
-  // its rows follow one another, and four are fewer than seven; a decode step of GPT-2 XL's sizes
-  // at 32 and at 48 rows 2 and 4 % shorter, with the groups of 49 to 64 rows 3 % longer)
-  if (p.row_groups > 1)
-    hipLaunchKernelGGL((gemm_bf16_rows_kernel<2, 2, RW, R_HELD>), grid, block, 0, stream, p);
-  else if (M <= 32)
-    hipLaunchKernelGGL((gemm_bf16_rows_kernel<2, 2, 2 * RW, 4>), grid, dim3(2 * RW * 64), 0, stream, p);
+  const int f_blocks = (N + R_FEATURES - 1) / R_FEATURES, tiles = (M + 15) / 16;
+  const auto fits = [&](int t) { return (long)((tiles + t - 1) / t) * f_blocks * n_splits <= n_compute_units(); };
+  const int per_block = fits(1) ? 1 : fits(2) || tiles == 2 ? 2 : tiles;
+  p.row_groups = (tiles + per_block - 1) / per_block;
+  const dim3 grid((f_blocks + 7) / 8 * 8 * p.row_groups, n_splits);
+  if (per_block == 1)
+    hipLaunchKernelGGL((gemm_bf16_rows_kernel<1, 2, RW, R_HELD, 4>), grid, dim3(RW * 64), 0, stream, p);
+  else if (per_block == 2)
+    hipLaunchKernelGGL((gemm_bf16_rows_kernel<2, 2, RW, R_HELD, 4>), grid, dim3(RW * 64), 0, stream, p);
+  else if (per_block == 3)
+    hipLaunchKernelGGL((gemm_bf16_rows_kernel<3, 2, 2 * RW, 4, 1>), grid, dim3(2 * RW * 64), 0, stream, p);
   else
-    hipLaunchKernelGGL((gemm_bf16_rows_kernel<3, 2, 2 * RW, 4>), grid, dim3(2 * RW * 64), 0, stream, p);
+    hipLaunchKernelGGL((gemm_bf16_rows_kernel<4, 2, 2 * RW, 4, 1>), grid, dim3(2 * RW * 64), 0, stream, p);
   CHECK_LAUNCH("gemm_bf16_rows");
   return 0;
 }

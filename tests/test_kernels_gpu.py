@@ -1114,6 +1114,23 @@ def test_gemm_bf16_rows_kernel_in_parts_and_with_the_cache_scatter(M, N, K):
             assert written.any() and torch.isnan(c.pool[~written].float()).all()
 
 
+@pytest.mark.parametrize("M", [17, 31, 32, 33, 47, 48, 49, 64])
+@pytest.mark.parametrize("N,splits", [(1600, 1), (2050, 1), (2720, 1), (2080, 2), (4096, 1), (4128, 1), (1344, 4)])
+@pytest.mark.parametrize("K", [1304, 1792])
+def test_rows_of_17_to_64_in_blocks_of_one_to_four_tiles(M, N, splits, K):
+    """Feature blocks and parts of K that leave a compute unit a block of one tile of 16 rows, of two (the second
+    group of three tiles is then half empty), or only of all the tiles; waves with and without a full hand of
+    k-blocks.  (Products of 16-bit numbers summed in 32 bits: the result's own rounding is 2^-9.)"""
+    k = _k()
+    a = _rand((M, K), torch.bfloat16, M)
+    w = _rand((N, K), torch.bfloat16, N, 0.1)
+    bias = _rand((N,), torch.float32, 12)
+    ref = plain.linear(a.double().cpu(), w.double().cpu(), bias.double().cpu())
+    out = torch.full((M, N), 7.0, dtype=torch.bfloat16, device=DEV)
+    k.linear(out, a, k.PackedWeight(w, keep_rows=False), bias, splits=splits)
+    assert torch.allclose(out.double().cpu(), ref, rtol=2**-8, atol=1e-3)
+
+
 @pytest.mark.parametrize("M,N,K", [(17, 48, 64), (33, 257, 1536), (64, 4800, 1600), (40, 1600, 6400), (49, 333, 1608),
                                    (48, 80, 1600), (20, 100, 520), (32, 4800, 1600), (63, 1600, 1792), (50, 6400, 1600)])
 def test_rows_in_the_packed_order_into_and_out_of_the_product_of_17_to_64_rows(M, N, K):
