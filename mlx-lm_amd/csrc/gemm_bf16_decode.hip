@@ -309,24 +309,43 @@ __global__ __launch_bounds__(NW * 64) void gemm_bf16_decode_kernel(DecodeGemmArg
     }
   } else {
     load_pass(w0, 0);  // in flight while the activations are copied
-    const uint16_t* in = input_of(p, n0);
-    // four independent loads a thread and round: one trip to L2 instead of four in a row
+    // Wave w copies rows w and w + 8, four pieces of 16 bytes a lane and row at a time, all on their way together:
+    // one trip to L2.  The empty statement says that they are all wanted there: otherwise each load is moved down
+    // to the store that needs it, and each store waits for its own trip, after the weights' (pieces dealt to the
+    // threads, up to four trips at 8 rows and eight at 16; us before and now at 1 / 8 / 16 rows: 4,800 x 1,600
+    // 6.4 / 7.2 / 8.4 and 6.4 / 7.0 / 7.8; 1,600 x 1,600 4.2 / 4.8 / 5.3 and 4.1 / 4.4 / 4.8; 1,024 x 1,024 3.5 / 3.9 / 4.3
+    // and 3.5 / 3.7 / 3.9; 1,024 x 2,688 in two parts 4.3 / 4.7 / 5.2 and 4.2 / 4.4 / 4.6).  The rows asked for ahead of
+    // the weights, whose number is not known when this is compiled, are waited for together with them and cost more.
+    static_assert(2 * NW >= 16, "the waves' two rows cover all rows");
+    typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
+    const int row = __builtin_amdgcn_readfirstlane(wave);
+    const uint16_t* in = input_of(p, n0) + kb + lane * 8;
+    uint16_t* to = As + lane * 8;
     const int per_row = (min(p.K, kb + n_chunks * 64) - kb) / 8;
-    const int total = p.M * per_row;
-    for (int c0 = tid; c0 < total; c0 += 4 * NW * 64) {
-      uint4 t[4];
+    if (p.M == 1) {  // (a piece a thread; one wave with four made a step of batch 1 through 48 layers 1.84 ms, this 1.80)
+      for (int c = tid; c < per_row; c += NW * 64)
+        *(u32x4_t*)(to + row * 512 + (c - tid) * 8) = *(const u32x4_t*)(in + row * 512 + (c - tid) * 8);
+    }
+    for (int first = 0; p.M > 1 && row < p.M && first < per_row; first += 256) {
+      u32x4_t t[2][4];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int c = min(c0 + j * NW * 64, total - 1);
-        const int r = c / per_row, k = (c - r * per_row) * 8;
-        t[j] = *(const uint4*)(in + (size_t)r * p.lda + kb + k);
-      }
+      for (int h = 0; h < 2; ++h)
+        if (row + NW * h < p.M) {
+          const uint16_t* from = in + (size_t)(row + NW * h) * p.lda + first * 8;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int c = c0 + j * NW * 64;
-        const int r = c / per_row, k = (c - r * per_row) * 8;
-        if (c < total) *(uint4*)(As + r * p.a_stride + k) = t[j];
-      }
+          for (int i = 0; i < 4; ++i)
+            if (first + lane + 64 * i < per_row) t[h][i] = *(const u32x4_t*)(from + 512 * i);
+        }
+      asm volatile("" : "+v"(t[0][0]), "+v"(t[0][1]), "+v"(t[0][2]), "+v"(t[0][3]), "+v"(t[1][0]), "+v"(t[1][1]),
+                   "+v"(t[1][2]), "+v"(t[1][3]));
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+        if (row + NW * h < p.M) {
+          uint16_t* into = to + (row + NW * h) * p.a_stride + first * 8;
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (first + lane + 64 * i < per_row) *(u32x4_t*)(into + 512 * i) = t[h][i];
+        }
     }
   }
   // What the epilogue takes from memory (the bias, and the stream's old value where the product

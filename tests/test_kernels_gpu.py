@@ -1114,6 +1114,23 @@ def test_gemm_bf16_rows_kernel_in_parts_and_with_the_cache_scatter(M, N, K):
             assert written.any() and torch.isnan(c.pool[~written].float()).all()
 
 
+@pytest.mark.parametrize("M", [1, 2, 7, 8, 9, 16])
+@pytest.mark.parametrize("K,splits", [(8, 1), (504, 1), (512, 1), (520, 1), (2040, 1), (2056, 1), (4104, 1), (4104, 2), (5120, 2)])
+def test_decode_product_copies_every_row_whole(M, K, splits):
+    """Rows that end inside, at and beyond a wave's piece of 64 x 8 columns, its four of them, and a block's parts of
+    K; one row, a row a wave, two rows a wave.  (Products of 16-bit numbers summed in 32 bits: the result's own
+    rounding is 2^-9.)"""
+    k = _k()
+    N = 48
+    a = _rand((M, K), torch.bfloat16, M)
+    w = _rand((N, K), torch.bfloat16, K, 0.1)
+    bias = _rand((N,), torch.float32, 12)
+    ref = plain.linear(a.double().cpu(), w.double().cpu(), bias.double().cpu())
+    out = torch.full((M, N), 7.0, dtype=torch.bfloat16, device=DEV)
+    k.linear(out, a, k.PackedWeight(w, keep_rows=False), bias, splits=splits)
+    assert torch.allclose(out.double().cpu(), ref, rtol=2**-8, atol=1e-3)
+
+
 @pytest.mark.parametrize("M", [17, 31, 32, 33, 47, 48, 49, 64])
 @pytest.mark.parametrize("N,splits", [(1600, 1), (2050, 1), (2720, 1), (2080, 2), (4096, 1), (4128, 1), (1344, 4)])
 @pytest.mark.parametrize("K", [1304, 1792])
