@@ -83,6 +83,20 @@ __device__ __forceinline__ float uniform01(unsigned long long key, unsigned int 
   return ((float)(x >> 8) + 0.5f) * (1.0f / 16777216.0f);
 }
 
+// Gumbel noise -log(-log u) of the same 24 bits n, u = (n + 0.5) / 2^24.  The tokens that win have u close to 1, where
+// the 24 bits of a float do not hold n + 0.5 and a logarithm's last bit is much of its value (the noise was wrong by
+// 0.001 to 0.1 there, and infinite for the largest n): -log u comes from 1 - u, which is exact, and a few terms of its
+// series (the next is 1.2e-8 of the sum at 1/64), and through the hardware's log2 only where u is further from 1.
+__device__ __forceinline__ float gumbel(unsigned long long key, unsigned int index) {
+  unsigned int x = fmix32((index + 1u) * 0x9E3779B1u ^ (unsigned int)key);
+  x = fmix32(x + (unsigned int)(key >> 32)) >> 8;
+  const float rest = ((float)(0xffffffu - x) + 0.5f) * (1.0f / 16777216.0f);
+  const float u = ((float)x + 0.5f) * (1.0f / 16777216.0f);
+  const float near = rest * (1.f + rest * (0.5f + rest * (0.33333333f + rest * 0.25f)));
+  const float minus_log_u = rest < 1.f / 64 ? near : -0.69314718f * __log2f(u);
+  return -0.69314718f * __log2f(minus_log_u);
+}
+
 struct Kept {
   float lo, hi;
   const int* special;
@@ -421,11 +435,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_rows_kernel(SampleArgs 
   const unsigned long long key = draw_key(a.seed[r], (unsigned int)a.counter[r]);
   bv = -INFINITY, bi = 0x7fffffff;
   auto consider = [&](int i, float lp) {
-    // Gumbel noise -log(-log u) through the hardware's log2 (u has 24 bits; v_log_f32 is good to
-    // an ulp of its result)
-    const float u = uniform01(key, (unsigned int)i);
-    const float g = -0.69314718f * __log2f(-0.69314718f * __log2f(u));
-    const float v = lp * inv_temp + g;
+    const float v = lp * inv_temp + gumbel(key, (unsigned int)i);
     if (v > bv || (v == bv && i < bi)) bv = v, bi = i;
   };
   if (cand && (n_cand == V || kept.lo > noncand_max)) {

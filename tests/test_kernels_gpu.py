@@ -776,6 +776,43 @@ def test_sample_temperature_distribution():
     assert (freq - q).abs().max() < 0.02
 
 
+def _noise_bits(seed, counter, n):
+    """The 24 bits that the sampling kernel hashes for tokens 0 .. n - 1 (``csrc/sampling.hip``)."""
+    import numpy as np
+
+    m, x = (1 << 64) - 1, (seed + 0x9E3779B97F4A7C15 * (counter + 1)) & ((1 << 64) - 1)
+    x = (x ^ x >> 30) * 0xBF58476D1CE4E5B9 & m
+    x = (x ^ x >> 27) * 0x94D049BB133111EB & m
+    key = x ^ x >> 31
+
+    def mix(v):
+        v = (v ^ v >> np.uint32(16)) * np.uint32(0x85EBCA6B)
+        v = (v ^ v >> np.uint32(13)) * np.uint32(0xC2B2AE35)
+        return v ^ v >> np.uint32(16)
+
+    i = np.arange(1, n + 1, dtype=np.uint32) * np.uint32(0x9E3779B1)
+    return mix(mix(i ^ np.uint32(key & 0xFFFFFFFF)) + np.uint32(key >> 32)) >> np.uint32(8)
+
+
+def test_sample_noise_of_the_tokens_that_win():
+    """Noise is -log(-log u), u = (n + 0.5) / 2^24, also where u is closest to 1 and the noise largest: 17.3, no more
+    (a token 60 below the others stays unlikely whatever its n), and the token of the greatest sum is drawn
+    wherever the second is 1e-4 behind (sums of up to 30 in 32 bits: 2e-6 each, and the hardware's log2)."""
+    import numpy as np
+
+    V = 4096
+    top = next((c, int(b.argmax())) for c in range(100000) if (b := _noise_bits(5, c, V)).max() == 0xFFFFFF)
+    counters = [top[0]] + list(range(300))
+    logits = torch.zeros(len(counters), V, device=DEV)
+    logits[0, top[1]] = -60.0
+    tok, _, _ = _sample(logits, temp=1.0, seed=5, counter=counters)
+    for row, c in enumerate(counters):
+        u = (_noise_bits(5, c, V).astype(np.float64) + 0.5) / 2**24
+        score = -np.log(-np.log(u)) + logits[row].double().cpu().numpy()
+        first, second = np.argsort(-score)[:2]
+        assert int(tok[row]) == first or score[first] - score[second] < 1e-4, (row, c)
+
+
 def test_sample_filters_match_reference_vectors():
     # vectors of the reference's tests/test_sample_utils.py:19-105
     p = torch.tensor([0.9, 1e-9, 1e-9, 0.1])
