@@ -366,14 +366,15 @@ static int finish_parts(EngCtx* ctx, const EngMat& out, float* ws, int n_splits,
 // Whether the kernel for 17 to 64 rows takes the product of M rows with w, and with K in how many
 // parts (*n_splits; 0: it does not).
 // (A matrix of more blocks than two a CU, the vocabulary's, would take that kernel several rounds,
-// each with its own wait for memory: the tiles stream it 6 us faster.  Beyond 32 rows it wins
-// only where K is long enough for the tiles to split it: at widths 768 and 1,024 a decode
-// step of 48 rows is 4 to 5 % slower through it, at 1,280 the same, at 1,600 4 % faster.)
+// each with its own wait for memory: the tiles stream it 6 us faster.  Beyond 32 rows it takes
+// K from 768 on, the shortest it was measured at: a step of 40 / 48 / 64 requests, contexts of 100
+// to 400, takes GPT-2 small (K 768 and 3,072) 0.640 / 0.665 / 0.715 ms and large (1,280 and 5,120)
+// 1.96 / 2.02 / 2.24; with the tiles where K is below 1,536, 0.650 / 0.679 / 0.723 and 2.24 / 2.33 / 2.59.)
 static int rows_parts(const EngCtx* ctx, int M, const EngWeight& w, int variant, int splits, int* n_splits) {
   *n_splits = 0;
   const int N = w.N, K = w.K;
   if (!(w.dtype == DT_BF16 && variant == 0 && M > DECODE_MAX_ROWS && M <= ROWS_MAX_ROWS && w.packed &&
-        (M <= 32 || K >= 1536) && (N + 31) / 32 <= 2 * ctx->n_compute_units))
+        (M <= 32 || K >= 768) && (N + 31) / 32 <= 2 * ctx->n_compute_units))
     return 0;
   int n = 0;
   if (splits == 0)

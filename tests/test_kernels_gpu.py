@@ -1168,6 +1168,24 @@ def test_decode_product_copies_every_row_whole(M, K, splits):
     assert torch.allclose(out.double().cpu(), ref, rtol=2**-8, atol=1e-3)
 
 
+@pytest.mark.parametrize("M", [33, 48, 49, 64])
+@pytest.mark.parametrize("N,K", [(2304, 768), (768, 768), (768, 3072), (3840, 1280), (1000, 1528), (64, 64)])
+def test_products_of_33_to_64_rows_with_a_short_k(M, N, K):
+    """Left to choose, narrow matrices at these rows too: into the stream and as activations.  (As above.)"""
+    k = _k()
+    a = _rand((M, K), torch.bfloat16, M)
+    w = _rand((N, K), torch.bfloat16, N, 0.1)
+    bias = _rand((N,), torch.float32, 12)
+    packed = k.PackedWeight(w, keep_rows=False)
+    ref = plain.linear(a.double().cpu(), w.double().cpu(), bias.double().cpu())
+    out = torch.full((M, N), 7.0, dtype=torch.bfloat16, device=DEV)
+    k.linear(out, a, packed, bias)
+    assert torch.allclose(out.double().cpu(), ref, rtol=2**-8, atol=1e-3)
+    stream = torch.ones((M, N), dtype=torch.float32, device=DEV)
+    k.linear(stream, a, packed, bias, accumulate=True)
+    assert torch.allclose(stream.double().cpu(), 1 + ref, rtol=1e-5, atol=1e-3)
+
+
 @pytest.mark.parametrize("M", [17, 31, 32, 33, 47, 48, 49, 64])
 @pytest.mark.parametrize("N,splits", [(1600, 1), (2050, 1), (2720, 1), (2080, 2), (4096, 1), (4128, 1), (1344, 4)])
 @pytest.mark.parametrize("K", [1304, 1792])
