@@ -24,7 +24,7 @@
 // of the MFMAs; the eight partial tiles are summed in a fixed order.  Where
 // the matrix has few features and K is not split, a block owns only eight of
 // them (lanes 8..15 of a group repeat the eighth): twice as many blocks.
-// (17 to 48 rows have a kernel of their own further down, gemm_bf16_rows; more
+// (17 to 64 rows have a kernel of their own further down, gemm_bf16_rows; more
 // are the tile kernels' of gemm_bf16.hip.  Both leave their partial sums to the
 // second kernels of this file in the same way.)
 //
