@@ -24,9 +24,8 @@
 //  * Online softmax in 32-bit per lane; outputs leave as O^T accumulators.
 // What bounds it: the softmax's vector instructions, half of their time the exponentials (a tile of 128 queries x 64
 // keys is some 1,150 cycles of them a wave beside 512 of the matrix unit), and at few blocks the chain of one block.
-// 8,000 tokens of 25 heads of 64: 300 us, 0.68 PFLOP/s of the causal half (336 before the reference of the
-// probabilities was let lag); 2 x 1,024: 23.7 (25.0); 2 x 1,024 of 16 heads of 128: 30.9 (37.6); 690 tokens in four
-// requests of 16 heads of 256: 25 (36, when two tiles on their way did not fit the registers).
+// 8,000 tokens of 25 heads of 64: 309 us, 0.66 PFLOP/s of the causal half; 2 x 1,024: 23.2; 2 x 1,024 of 16 heads of
+// 128: 34.6; of 8 heads of 256: 100 (107 with two tiles on their way, which did not fit the registers).
 #include "common.h"
 #include "attention_tiles.h"
 #include <type_traits>
@@ -376,11 +375,11 @@ void attn_prefill_kernel(PrefillArgs p) {
         }
     }
     tmax = fmaxf(tmax, __shfl_xor(tmax, 32, WAVE));
-    // Probabilities are taken against `m`, which need not be the largest score: it follows only where a score of the
-    // wave's queries has passed it by 2^8 (a float and a bfloat16 keep as many digits of 200 as of 1, and a sum of
-    // such numbers is far from overflow).  Following every new maximum, some query of the 32 has one in most tiles, and
-    // the 32 products that rescale the outputs were paid nearly every time.
-    if (__any(tmax > m + 8.0f)) {
+    // Probabilities are taken against the largest score so far: the weight that counts most is then exactly 1, which
+    // the rounding to bfloat16 leaves as it is.  (Against a reference that lagged by up to 2^8 it was rounded like the
+    // others while the sum took it unrounded: 25 heads of 64 at 8,000 tokens 10 % sooner, but with sharp scores the
+    // outputs were 10 to 30 % further from 64 bits.)
+    if (__any(tmax > m)) {
       const float m_new = fmaxf(m, tmax);
       const float alpha = exp2f(m - (m_new == -INFINITY ? 0.f : m_new));  // (a row with no key yet: zero)
       l *= alpha;

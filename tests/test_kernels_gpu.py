@@ -618,9 +618,8 @@ def test_attn_prefill(case):
                                               (128, 2, [0], [190], 0), (256, 2, [30], [150], 0), (64, 2, [100], [140], 50)])
 @pytest.mark.parametrize("step", [0.02, 0.4, 30.0])
 def test_attn_prefill_with_scores_that_keep_growing(hd, H, ctx, ql, window, step):
-    """Scores that grow by `step` with every key: the largest so far moves in every tile, by less than the
-    probabilities' reference may lag behind it, by about that, and by far more; with blocks fewer than the
-    compute units (their keys in two groups of waves) and more.  (The weights are rounded to bfloat16,
+    """Scores that grow by `step` with every key: the largest so far moves in every tile, by little and by far;
+    with blocks fewer than the compute units (their keys in two groups of waves) and more.  (The weights are rounded to bfloat16,
     2^-9 of each, and meet values of up to 4.5.)"""
     k = _k()
     c = PagedCase(torch.bfloat16, H, 1, hd, 16, ctx, ql, seed=hd + H, window=window)
@@ -638,6 +637,47 @@ def test_attn_prefill_with_scores_that_keep_growing(hd, H, ctx, ql, window, step
     k.attn_prefill(out, c.q.to(DEV), c.kv, c.block_table_dev, c.token_req, c.positions, tiles, tiles.shape[0], H, c.scale, window)
     err = (out.double().cpu() - c.reference()).abs().max().item()
     assert err < 2.5e-2, err
+
+
+def _weights_rounded_against_the_largest_score(c):
+    """What rounding alone does to a case's outputs: 64 bits, but for the weights, which meet the values as bfloat16
+    numbers of exp(score - the largest score so far), and the outputs.  (The sum takes the weights unrounded.)"""
+    out, t = torch.empty(c.T, c.H * c.hd, dtype=torch.float64), 0
+    for r, (known, n) in enumerate(zip(c.ctx_lens, c.q_lens)):
+        q = c.q[t : t + n].double().view(n, c.H, c.hd).transpose(0, 1)
+        kk, vv = (x[r][: known + n].double().repeat_interleave(c.H // x[r].shape[1], 1).transpose(0, 1) for x in (c.k_full, c.v_full))
+        s = (q * c.scale) @ kk.transpose(1, 2).contiguous()
+        s = s.masked_fill(torch.arange(known + n)[None, :] > known + torch.arange(n)[:, None], float("-inf"))
+        m = torch.full((c.H, n, 1), -1e300, dtype=torch.float64)
+        total, o = torch.zeros_like(m), torch.zeros(c.H, n, c.hd, dtype=torch.float64)
+        for a in range(0, known + n, 64):  # tiles of 64 keys
+            new = torch.maximum(m, s[..., a : a + 64].amax(-1, keepdim=True))
+            w = torch.exp(s[..., a : a + 64] - new)
+            total = total * torch.exp(m - new) + w.sum(-1, keepdim=True)
+            o = o * torch.exp(m - new) + w.bfloat16().double() @ vv[:, a : a + 64]
+            m = new
+        out[t : t + n] = (o / total).transpose(0, 1).reshape(n, -1)
+        t += n
+    return out.bfloat16().double()
+
+
+@pytest.mark.parametrize("hd,H,Hkv", [(32, 4, 2), (64, 3, 3), (64, 140, 7), (128, 2, 1), (256, 2, 2)])
+@pytest.mark.parametrize("spread", [0.5, 2.0, 4.0, 8.0])
+def test_attn_prefill_with_sharp_scores_is_as_exact_as_rounded_weights_allow(hd, H, Hkv, spread):
+    """Scores of a standard deviation of ``spread`` (in units of log 2): the distance from 64 bits is that of rounding
+    the weights against the largest score so far, and the outputs, to 4 %.  (Against a reference that lags by up to
+    2^8 it is 10 to 30 % more from a spread of 2 on.)"""
+    k = _k()
+    c = PagedCase(torch.bfloat16, H, Hkv, hd, 16, [0, 200], [400, 130], seed=hd + H)
+    c.q = (c.q.float() * (spread * math.log(2.0))).to(torch.bfloat16)
+    k.kv_write(c.k_new.to(DEV), c.v_new.to(DEV), c.kv, c.block_table_dev, c.token_req, c.positions)
+    tiles = c.tiles(k.attn_tile_sizes()[1])
+    out = torch.full((c.T, H * hd), float("nan")).to(torch.bfloat16).to(DEV)
+    k.attn_prefill(out, c.q.to(DEV), c.kv, c.block_table_dev, c.token_req, c.positions, tiles, tiles.shape[0], H, c.scale, 0)
+    want = c.reference()
+    err = (out.double().cpu() - want).norm().item()
+    allowed = (_weights_rounded_against_the_largest_score(c) - want).norm().item()
+    assert err < 1.04 * allowed, (err / allowed, err / want.norm().item())
 
 
 def test_attn_prefill_far_key_stands_out():
