@@ -85,10 +85,12 @@ __device__ __forceinline__ int key_of_row(int rho) {
 // GROUPS: groups of four waves, which take the key tiles by turns, each group with LDS of its own, and join their sums at
 // the end.  A block's walk over its keys is one tile after another (copy, barrier, products, softmax: some 1.2 us), and
 // where the blocks are few the longest walk is the kernel's time: two groups halve it.
-// (Two waves a SIMD, no fewer and no more, are named to the compiler: left alone it takes the registers of three, which
-// leaves it less to overlap, 25.5 us against 23.7 for 2 x 1,024 tokens of GPT-2 XL, 297 against 300 for 8,000.)
+// (With heads of 64 two waves a SIMD, no fewer and no more, are named to the compiler: left alone it takes the registers
+// of three, which leaves it less to overlap, 24.6 us against 23.4 for 2 x 1,024 tokens of 25 heads and 80 against 73 for
+// 512 on 4,000 earlier keys, though 295 against 309 for 8,000.  Heads of 32 run three where blocks are many: 16 heads at
+// 8,000 tokens 133 us, 141 with two.)
 template <int HD, bool POW2, bool EXTRAS, bool SHAPED, int GROUPS>
-__global__ __launch_bounds__(256 * GROUPS) __attribute__((amdgpu_waves_per_eu(HD <= 64 ? 2 : 1, HD <= 64 ? 2 : 1)))
+__global__ __launch_bounds__(256 * GROUPS) __attribute__((amdgpu_waves_per_eu(HD <= 64 ? 2 : 1, HD == 32 ? 8 : HD == 64 ? 2 : 1)))
 void attn_prefill_kernel(PrefillArgs p) {
   constexpr int KS_STRIDE = HD + 8;
   constexpr int DC = HD / 16;           // 16-column chunks of a head (QK contraction steps)
@@ -377,7 +379,7 @@ void attn_prefill_kernel(PrefillArgs p) {
     tmax = fmaxf(tmax, __shfl_xor(tmax, 32, WAVE));
     // Probabilities are taken against the largest score so far: the weight that counts most is then exactly 1, which
     // the rounding to bfloat16 leaves as it is.  (Against a reference that lagged by up to 2^8 it was rounded like the
-    // others while the sum took it unrounded: 25 heads of 64 at 8,000 tokens 10 % sooner, but with sharp scores the
+    // others while the sum took it unrounded: 25 heads of 64 at 8,000 tokens in 294 us instead of 309, but with sharp scores the
     // outputs were 10 to 30 % further from 64 bits.)
     if (__any(tmax > m)) {
       const float m_new = fmaxf(m, tmax);
