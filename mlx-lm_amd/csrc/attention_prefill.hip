@@ -84,11 +84,18 @@ __device__ __forceinline__ int key_of_row(int rho) {
 // SHAPED (with EXTRAS): scores also pass the soft cap and take the distance table's term
 // GROUPS: groups of four waves, which take the key tiles by turns, each group with LDS of its own, and join their sums at
 // the end.  A block's walk over its keys is one tile after another (copy, barrier, products, softmax: some 1.2 us), and
-// where the blocks are few the longest walk is the kernel's time: two groups halve it.
+// where the blocks are few the longest walk is the kernel's time: two groups halve it.  A walk of fewer than
+// TWO_GROUPS_FROM tiles is left to the first group: joining the sums costs about as much as a tile (25 heads of 64, both
+// groups and the first alone: 17 tokens, one tile, 5.3 and 4.5 us; 192, three, 8.6 and 7.7; 300, five, 10.1 and 9.5; 333,
+// six, 10.6 and 10.9; 333 under a window of 200, six at most, 11.7 and 13.1.  16 heads of 32: 192 tokens 6.4 and 5.9; 200,
+// four tiles, 6.5 and 7.2).  That the other waves were there at all costs up to 0.4 us (128 tokens: 7.5, in a block of four
+// waves 7.1), but how long the walks are is not known where the kernel is launched: a recorded step runs at other lengths.
 // (With heads of 64 two waves a SIMD, no fewer and no more, are named to the compiler: left alone it takes the registers
 // of three, which leaves it less to overlap, 24.6 us against 23.4 for 2 x 1,024 tokens of 25 heads and 80 against 73 for
 // 512 on 4,000 earlier keys, though 295 against 309 for 8,000.  Heads of 32 run three where blocks are many: 16 heads at
 // 8,000 tokens 133 us, 141 with two.)
+template <int HD>
+static constexpr int TWO_GROUPS_FROM = HD == 32 ? 4 : 6;
 template <int HD, bool POW2, bool EXTRAS, bool SHAPED, int GROUPS>
 __global__ __launch_bounds__(256 * GROUPS) __attribute__((amdgpu_waves_per_eu(HD <= 64 ? 2 : 1, HD == 32 ? 8 : HD == 64 ? 2 : 1)))
 void attn_prefill_kernel(PrefillArgs p) {
@@ -150,6 +157,9 @@ void attn_prefill_kernel(PrefillArgs p) {
   const int sink_hi = EXTRAS ? min(p.window > 0 ? p.keep_first : 0, k_lo) : 0;
   const int n_sink_tiles = (sink_hi + KT - 1) / KT;
   const int n_sink_pages = sink_hi > 0 ? (sink_hi - 1) / p.page_size + 1 : 0;
+  // (in a short walk the second group's waves end here: barriers count the waves that are left)
+  const int groups = GROUPS > 1 && n_sink_tiles + (k_hi - kt0 + KT - 1) / KT >= TWO_GROUPS_FROM<HD> ? GROUPS : 1;
+  if (GROUPS > 1 && group >= groups) return;
 
   float m = -INFINITY, l = 0.f;
   f32x16_t ot[DT];
@@ -169,8 +179,8 @@ void attn_prefill_kernel(PrefillArgs p) {
   extern __shared__ int page_of[];  // [max_blocks]
   const int pg0 = k_lo / p.page_size;
   const int n_pg = (k_hi - 1) / p.page_size - pg0 + 1;
-  for (int i = threadIdx.x; i < n_sink_pages; i += 256 * GROUPS) page_of[i] = table[i];
-  for (int i = threadIdx.x; i < n_pg; i += 256 * GROUPS) page_of[n_sink_pages + i] = table[pg0 + i];
+  for (int i = threadIdx.x; i < n_sink_pages; i += 256 * groups) page_of[i] = table[i];
+  for (int i = threadIdx.x; i < n_pg; i += 256 * groups) page_of[n_sink_pages + i] = table[pg0 + i];
   __syncthreads();
 
   // Loads are never predicated and never zeroed: a key outside [k_lo, k_hi) is
@@ -432,37 +442,37 @@ void attn_prefill_kernel(PrefillArgs p) {
     auto first_key = [&](int i) { return i < n_sink_tiles ? SINK + i * KT : kt0 + (i - n_sink_tiles) * KT; };
     const int n_all = n_sink_tiles + (k_hi - kt0 + KT - 1) / KT;
     fetch(first_key(group), 0);
-    if constexpr (SETS == 2) fetch(first_key(group + GROUPS), SECOND);
-    for (int i = 0; i < n_all; i += 2 * GROUPS) {
+    if constexpr (SETS == 2) fetch(first_key(group + groups), SECOND);
+    for (int i = 0; i < n_all; i += 2 * groups) {
       const int mine = i + group;
-      one_tile(first_key(mine), first_key(mine + SETS * GROUPS), 0, std::false_type{});
-      if (i + GROUPS >= n_all) break;  // uniform over the block
-      one_tile(first_key(mine + GROUPS), first_key(mine + (1 + SETS) * GROUPS), SECOND, std::false_type{});
+      one_tile(first_key(mine), first_key(mine + SETS * groups), 0, std::false_type{});
+      if (i + groups >= n_all) break;  // uniform over the block
+      one_tile(first_key(mine + groups), first_key(mine + (1 + SETS) * groups), SECOND, std::false_type{});
     }
   } else {
-    constexpr int STEP = GROUPS * KT;  // keys that the groups take at a time
-    int kt = kt0;                      // the first group's
+    const int step = groups * KT;  // keys that the groups take at a time
+    int kt = kt0;                  // the first group's
     const int ahead = group * KT;
     fetch(kt + ahead, 0);
-    if constexpr (SETS == 2) fetch(kt + ahead + STEP, SECOND);
+    if constexpr (SETS == 2) fetch(kt + ahead + step, SECOND);
     if (p.window <= 0) {
-      for (; kt + 2 * STEP - 1 <= pos0; kt += 2 * STEP) {
-        one_tile(kt + ahead, kt + ahead + SETS * STEP, 0, std::true_type{});
-        one_tile(kt + ahead + STEP, kt + ahead + (1 + SETS) * STEP, SECOND, std::true_type{});
+      for (; kt + 2 * step - 1 <= pos0; kt += 2 * step) {
+        one_tile(kt + ahead, kt + ahead + SETS * step, 0, std::true_type{});
+        one_tile(kt + ahead + step, kt + ahead + (1 + SETS) * step, SECOND, std::true_type{});
       }
     }
-    for (; kt < k_hi; kt += 2 * STEP) {  // the tiles around the diagonal, or all of them under a window
-      one_tile(kt + ahead, kt + ahead + SETS * STEP, 0, std::false_type{});
-      if (kt + STEP >= k_hi) break;  // uniform
-      one_tile(kt + ahead + STEP, kt + ahead + (1 + SETS) * STEP, SECOND, std::false_type{});
+    for (; kt < k_hi; kt += 2 * step) {  // the tiles around the diagonal, or all of them under a window
+      one_tile(kt + ahead, kt + ahead + SETS * step, 0, std::false_type{});
+      if (kt + step >= k_hi) break;  // uniform
+      one_tile(kt + ahead + step, kt + ahead + (1 + SETS) * step, SECOND, std::false_type{});
     }
   }
 
   // the two halves of the wave hold different keys of the same query
   l += __shfl_xor(l, 32, WAVE);
-  if constexpr (GROUPS == 2) {
+  if (GROUPS == 2 && groups == 2) {
     // the second group's sums go to the first through LDS, each thread's to the thread of the same queries
-    static_assert((DT * 16 + 2) * 256 * sizeof(float) <= sizeof(tiles_lds), "the sums fit where the tiles were");
+    static_assert(GROUPS == 1 || (DT * 16 + 2) * 256 * sizeof(float) <= sizeof(tiles_lds), "the sums fit where the tiles were");
     float* const sums = (float*)tiles_lds + tid;
     __syncthreads();  // no tile is read any more
     if (group == 1) {
@@ -566,10 +576,10 @@ static int prefill_launch(void* out, const void* q, int ldq, int ldo, const void
   // (the kept first keys' pages lie before the window's; a page can be in both runs)
   const size_t lds = (size_t)(max_blocks + (extras ? 2 : 0)) * sizeof(int);
   const bool pow2 = p.page_shift >= 0;
-  // Two groups a block where the blocks are no more than the CUs, so that a block's walk is the kernel's time: 512 queries
-  // on 4,000 earlier keys, 25 heads of 64 (100 blocks) 55 us beside 68, 1,000 keys of 16 heads of 32 13.2 / 16.2, 333 of
-  // 25 of 64 10.0 / 10.2.  With more blocks than CUs they are in each other's way (2 x 1,024 tokens of 25 heads, 400
-  // blocks: 26.2 / 23.6).  Heads of 128 and more take the registers of a whole SIMD a wave.
+  // Two groups a block where the blocks are no more than the CUs, so that a block's walk is the kernel's time: 1,024 tokens
+  // of 25 heads of 64 (200 blocks) 19.1 us beside 21.3, 512 on 4,000 earlier keys 57 / 72, of 16 heads of 32 43 / 58.  With
+  // more blocks than CUs they are in each other's way (2 x 1,024 tokens of 25 heads, 400 blocks: 25.5 / 23.1; 4 x 512:
+  // 20.7 / 15.2).  Heads of 128 and more take the registers of a whole SIMD a wave.
   const bool two = head_dim <= 64 && pow2 && max_blocks <= 4096 && (long)n_heads * n_tiles <= n_compute_units();
   const dim3 grid(n_heads, n_tiles), block(two ? 512 : 256);
 #define LAUNCH_AS(HD, POW2, GROUPS)                                                                                      \

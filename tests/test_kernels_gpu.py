@@ -264,7 +264,7 @@ class PagedCase:
         self.ctx_lens, self.q_lens = ctx_lens, q_lens
         self.scale = head_dim**-0.5
 
-    def reference(self):
+    def reference(self, keep_first=0):
         out = torch.empty(self.T, self.H * self.hd, dtype=torch.float64)
         t = 0
         for r, (c, n) in enumerate(zip(self.ctx_lens, self.q_lens)):
@@ -274,6 +274,7 @@ class PagedCase:
             kk = self.k_full[r][: c + n].double().permute(1, 0, 2)
             vv = self.v_full[r][: c + n].double().permute(1, 0, 2)
             mask = plain.causal_mask(n, c, self.window if self.window else None)
+            mask |= plain.causal_mask(n, c) & (torch.arange(c + n) < keep_first)
             o = plain.attention(q, kk, vv, self.scale, mask)
             out[t : t + n] = plain.merge_heads(o)
             t += n
@@ -678,6 +679,30 @@ def test_attn_prefill_with_sharp_scores_is_as_exact_as_rounded_weights_allow(hd,
     err = (out.double().cpu() - want).norm().item()
     allowed = (_weights_rounded_against_the_largest_score(c) - want).norm().item()
     assert err < 1.04 * allowed, (err / allowed, err / want.norm().item())
+
+
+@pytest.mark.parametrize("hd,edge", [(32, 4), (64, 6)])
+@pytest.mark.parametrize("window,keep", [(0, 0), (150, 0), (150, 70)])
+@pytest.mark.parametrize("ps", [16, 48])
+def test_attn_prefill_walks_around_the_one_that_two_groups_share(hd, edge, window, keep, ps):
+    """Walks of one tile of 64 keys up to two more than the one from which a block's second group of waves takes
+    part, a key less and more each, windows and kept first keys among them, in a launch of few blocks; with pages
+    that are no power of two a block has one group.  (The weights are rounded to bfloat16, 2^-9 of each, and meet
+    values of up to 4.5.)"""
+    k = _k()
+    walks = sorted({64 * t + d for t in range(1, edge + 3) for d in (-1, 0, 1)})
+    ql = [20 + 7 * (i % 16) for i in range(len(walks))]
+    ql = [min(n, w) for n, w in zip(ql, walks)]
+    c = PagedCase(torch.bfloat16, 2, 1, hd, ps, [w - n for w, n in zip(walks, ql)], ql, seed=hd + window, window=window)
+    k.kv_write(c.k_new.to(DEV), c.v_new.to(DEV), c.kv, c.block_table_dev, c.token_req, c.positions)
+    tiles = c.tiles(k.attn_tile_sizes()[1])
+    assert 2 * tiles.shape[0] <= 256
+    terms = k.ScoreTerms(keep_first=keep) if keep else None
+    out = torch.full((c.T, 2 * hd), float("nan")).to(torch.bfloat16).to(DEV)
+    k.attn_prefill(out, c.q.to(DEV), c.kv, c.block_table_dev, c.token_req, c.positions, tiles, tiles.shape[0], 2, c.scale, window, terms)
+    want = c.reference(keep)
+    err = (out.double().cpu() - want).abs().max().item()
+    assert err < 2.5e-2, err
 
 
 def test_attn_prefill_far_key_stands_out():
