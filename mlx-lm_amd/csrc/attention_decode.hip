@@ -88,8 +88,10 @@ __device__ __forceinline__ float gate_at(const DecodeArgs& p, int row, int col) 
 
 #define MAX_WAVES 16
 
-// Sixteen bytes that nobody on this die asks for again
-__device__ __forceinline__ uint4 load_once(const void* at) {
+// Sixteen bytes, with the streaming hint where nobody asks for them again
+template <bool ONCE>
+__device__ __forceinline__ uint4 load16(const void* at) {
+  if (!ONCE) return *(const uint4*)at;
   const u32x4_t v = __builtin_nontemporal_load((const u32x4_t*)at);
   return make_uint4(v.x, v.y, v.z, v.w);
 }
@@ -106,11 +108,11 @@ __device__ __forceinline__ size_t out_at(const DecodeArgs& p, int row, int col) 
 
 // What bounds this kernel: the keys and values come from memory once, and at many rows or long contexts that is the
 // time (64 rows of 25 heads of 64 at contexts of 300 to 1,001 are 266 MB: 49 us, 5.4 TB/s; a plain stream reads 6.4, with
-// the streaming hint 7.2).  So they are read with that hint (8 to 10 % here); a tile is small and the next one
-// on its way while it is taken, so that a wave's registers are few and many waves have something in flight (tiles of
-// 32 or 64 keys, one at a time, with a lookup and two divisions a lane and key: 54 to 58 us, 13.4 against 12.2 for 8 rows,
-// 25.3 against 22.1 for 16 rows of 16 heads of 128, 16.9 against 14.9 for 8 rows of float keys).  At few rows and short
-// contexts what is left is the chain: table and query, keys, the waves' join.
+// the streaming hint 7.2).  So they are read with that hint where no two heads share them (8 to 10 % here); a tile is
+// small and the next one on its way while it is taken, so that a wave's registers are few and many waves have something
+// in flight (tiles of 32 or 64 keys, one at a time, with a lookup and two divisions a lane and key: 54 to 58 us, 13.4 against
+// 12.2 for 8 rows, 25.3 against 22.1 for 16 rows of 16 heads of 128, 16.9 against 14.9 for 8 rows of float keys).  At few
+// rows and short contexts what is left is the chain: table and query, keys, the waves' join.
 
 // 16 bytes of a row as floats, and a float back as an element
 __device__ __forceinline__ void unpack(const uint4& v, float (&f)[8], const uint16_t*) {
@@ -153,8 +155,13 @@ __device__ __forceinline__ bool last_to_arrive(unsigned* counter, unsigned n_par
   return *s_last != 0;
 }
 
-// T: uint16_t (bfloat16 bits) or float.  CPK lanes per key: head_dim = EPL * CPK.
-template <typename T, int CPK>
+// T: uint16_t (bfloat16 bits) or float.  CPK lanes per key: head_dim = EPL * CPK.  ONCE: every key is read by one block
+// (as many key heads as query heads), with the streaming hint.  Where query heads share a key head, blocks that read the
+// same keys find them in the die's L2 or on their way to it, and a hinted line is gone by then: 64 rows of 28 query heads
+// of 128 over 4 key heads 819 us at contexts of 6,000 to 8,001 and 107 at 700 to 1,300, 691 and 79 without the hint; 32 of
+// 32 over 8 396 and 294; float, 64 of 16 of 128 over 4 938 and 686.  (At few rows and short contexts it is the hint that is
+// ahead there too, by 3 to 8 %: 8 rows of 16 of 64 over 4, 60 to 500 keys, 7.3 and 7.9 us.)
+template <typename T, int CPK, bool ONCE>
 __global__ __launch_bounds__(64 * (CPK >= 16 ? MAX_WAVES / 2 : MAX_WAVES)) void attn_decode_kernel(DecodeArgs p) {
   constexpr int EPL = 16 / sizeof(T);  // elements a lane holds of a key
   constexpr int HD = EPL * CPK;
@@ -278,8 +285,8 @@ __global__ __launch_bounds__(64 * (CPK >= 16 ? MAX_WAVES / 2 : MAX_WAVES)) void 
 #pragma unroll
     for (int j = 0; j < NL; ++j) {
       const size_t at = (size_t)page[j] * p.page_stride + head_off + in_page[j];
-      kv[j] = load_once(k_pages + at);
-      vv[j] = load_once(v_pages + at);
+      kv[j] = load16<ONCE>(k_pages + at);
+      vv[j] = load16<ONCE>(v_pages + at);
     }
   };
   auto take = [&](int t, const uint4 (&kv)[NL], const uint4 (&vv)[NL]) __attribute__((always_inline)) {
@@ -581,7 +588,10 @@ static void launch(const DecodeArgs& p, int n_rows, int n_waves, hipStream_t str
   }
   const size_t lds = p.table_in_lds ? (size_t)p.max_blocks * sizeof(int) : 0;
   const dim3 grid(n_rows, p.n_heads + extra_y, p.n_splits), block(64 * n_waves);
-  hipLaunchKernelGGL((attn_decode_kernel<T, CPK>), grid, block, lds, stream, p);
+  if (p.n_heads == p.n_kv_heads)
+    hipLaunchKernelGGL((attn_decode_kernel<T, CPK, true>), grid, block, lds, stream, p);
+  else
+    hipLaunchKernelGGL((attn_decode_kernel<T, CPK, false>), grid, block, lds, stream, p);
   if (p.n_splits > 1 && !p.join_here)
     hipLaunchKernelGGL((attn_decode_merge_kernel<T, CPK>), dim3(n_rows, p.n_heads), dim3(16 / sizeof(T) * CPK), 0, stream, p);
 }
