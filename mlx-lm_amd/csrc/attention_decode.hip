@@ -174,7 +174,7 @@ __global__ __launch_bounds__(64 * (CPK >= 16 ? MAX_WAVES / 2 : MAX_WAVES)) void 
   extern __shared__ int page_of[];  // [max_blocks] with table_in_lds
 
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int n_waves = blockDim.x >> 6;
+  int n_waves = blockDim.x >> 6;
   if (blockIdx.y >= p.n_heads) {  // a reading block (uniform)
     if (blockIdx.z != 0) return;
     // blocks go to the dies in turn, in the order x, y, z: this one is on die `lin % 8`, and
@@ -212,7 +212,9 @@ __global__ __launch_bounds__(64 * (CPK >= 16 ? MAX_WAVES / 2 : MAX_WAVES)) void 
   const int kv_head = h / (p.n_heads / p.n_kv_heads);
   const int* table = p.block_table + (size_t)req * p.max_blocks;
   if (p.table_in_lds) {
-    for (int i = tid; i < p.max_blocks; i += blockDim.x) page_of[i] = table[i];
+    const int threads = min((int)blockDim.x, 64 * ATTN_DECODE_ROW_WAVES);  // (the others may be about to end)
+    if (tid < threads)
+      for (int i = tid; i < p.max_blocks; i += threads) page_of[i] = table[i];
   }
   const int pos = __builtin_amdgcn_readfirstlane(p.positions[row]);
   const int sub = lane % CPK;  // which EPL columns of the key
@@ -232,6 +234,11 @@ __global__ __launch_bounds__(64 * (CPK >= 16 ? MAX_WAVES / 2 : MAX_WAVES)) void 
 
   const int k_hi = pos + 1;
   const int k_lo = p.window > 0 ? max(0, pos - p.window + 1) : 0;
+  // (sixteen waves are for long rows: the others' blocks go on with eight; barriers count the waves that are left)
+  if (n_waves > ATTN_DECODE_ROW_WAVES && k_hi - k_lo < ATTN_DECODE_WIDE_ROW_FROM) {
+    if (wave >= ATTN_DECODE_ROW_WAVES) return;
+    n_waves = ATTN_DECODE_ROW_WAVES;
+  }
   const int kt0 = (k_lo / TILE) * TILE;
   // the kept first keys [0, sink_hi) that the window has left behind come first, in tiles of their own
   const int sink_hi = min(p.keep_first, k_lo);

@@ -47,11 +47,15 @@ __device__ __forceinline__ float head_gate_of(const Args& p, int row, int h) {
 // kernel may still name 32 or 64, its tiles are of ATTN_DECODE_TILE_KEYS whatever they say).
 // Eight waves a block; four where the rows' blocks alone are more than the CUs (64 rows of 25 heads
 // at contexts of 300 to 1,001: 49.2 us, 49.7 with eight, 53.5 with two; 24 rows 20.4 and 22.6), or the keys no
-// more than four waves' tiles; sixteen where blocks that have a CU each walk 2,048 keys or more (8 rows at
-// 4,000 to 8,001: 57.1 us, 59.3 with eight).  Splits only where a wave would walk 64 keys or more, as many as
+// more than four waves' tiles; sixteen where blocks that have a CU each may walk 2,048 keys or more (8 rows at
+// 4,000 to 8,001: 57.1 us, 59.3 with eight).  A recorded step is planned for its class's longest, and a row of fewer
+// than ATTN_DECODE_WIDE_ROW_FROM keys lets its block's second eight waves end (8 rows of 25 heads of 64 at 60 to 500
+// keys: 9.1 us with sixteen, 8.4 with eight; 500 to 900 12.0 and 11.4; 900 to 1,300 15.1 and 14.6, of 6 rows 13.9 and
+// 14.2; 1,300 to 1,900 of 6 rows 17.4 and 18.2).  Splits only where a wave would walk 64 keys or more, as many as
 // leave it 32, and no more than give every block a compute unit at once (one row at 700 keys: 8.1 us in two, 8.7
 // whole; at 6,000: 13.4 in eight).
 #define ATTN_DECODE_ROW_WAVES 8
+#define ATTN_DECODE_WIDE_ROW_FROM 1024
 #define ATTN_DECODE_TILE_KEYS 16
 #define ATTN_DECODE_SPLIT_KEYS_A_WAVE 64
 #define ATTN_DECODE_KEYS_A_PART 32

@@ -492,6 +492,28 @@ def test_attn_decode_at_the_tiles_edges(hd, ps, window, n_splits, n_waves, here)
     assert err < _attn_tol(torch.bfloat16), err
 
 
+@pytest.mark.parametrize("dtype,hd", [(torch.bfloat16, 32), (torch.bfloat16, 64), (torch.float32, 16), (torch.float32, 32)])
+@pytest.mark.parametrize("window", [0, 600])
+@pytest.mark.parametrize("n_splits,here", [(1, 0), (3, 0), (3, 1), (3, 2)])
+@pytest.mark.parametrize("n_kv_heads", [1, 2])
+def test_attn_decode_of_sixteen_waves_of_which_eight_end(dtype, hd, window, n_splits, here, n_kv_heads):
+    """Rows on both sides of the length below which half of a block's sixteen waves end at once, in one launch, whole
+    and in parts, long block tables among them (more pages than the eight waves have threads)."""
+    k = _k()
+    H, ps = 2, 16
+    ctx = [0, 15, 16, 300, 1022, 1023, 1024, 1100, 9000]
+    c = PagedCase(dtype, H, n_kv_heads, hd, ps, ctx, [1] * len(ctx), seed=hd, window=window)
+    k.kv_write(c.k_new.to(DEV), c.v_new.to(DEV), c.kv, c.block_table_dev, c.token_req, c.positions)
+    rows = torch.arange(c.T, dtype=torch.int32, device=DEV)
+    part_o = torch.empty(c.T * H * n_splits * hd, dtype=torch.float32, device=DEV)
+    part_ml = torch.empty(c.T * H * n_splits * 2, dtype=torch.float32, device=DEV)
+    out = torch.full((c.T, H * hd), float("nan")).to(dtype).to(DEV)
+    k.attn_decode(out, c.q.to(DEV), c.kv, c.block_table_dev, c.token_req, c.positions, rows, c.T, H, c.scale, window, n_splits,
+                  part_o, part_ml, 16, rows_are_requests=True, join_in_kernel=here)
+    err = (out.double().cpu() - c.reference()).abs().max().item()
+    assert err < _attn_tol(dtype), err
+
+
 @pytest.mark.parametrize("case", [c for c in ATTN_CASES if c[2] in (16, 32, 64)] + [
     (8, 2, 16, 16, [700, 15, 16], [1, 1, 3], 0),
     (3, 1, 64, 4, [63, 64, 1000], [1, 2, 1], 100),
