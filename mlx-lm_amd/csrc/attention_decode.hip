@@ -9,7 +9,7 @@
 // (mlx_lm/models/base.py:132-139 with mask=None, mlx_lm/generate.py:1414).
 //
 // Work split: grid (rows, heads, n_splits), 1 to 16 waves a block.  The row's
-// keys [k_lo, k_hi) are cut into tiles of 16; the tiles are dealt to the splits
+// keys [k_lo, k_hi) are cut into tiles of 16 (of 32 where a load brings 16); the tiles are dealt to the splits
 // in runs and, inside a block, to the waves in turn; a wave asks for its next tile before it takes one.  With few rows in a step
 // it is the many waves of a block, joined through LDS, that give the GPU
 // enough to do; the parts of splits are joined by the block of a (row, head) that
@@ -165,7 +165,10 @@ template <typename T, int CPK, bool ONCE>
 __global__ __launch_bounds__(64 * (CPK >= 16 ? MAX_WAVES / 2 : MAX_WAVES)) void attn_decode_kernel(DecodeArgs p) {
   constexpr int EPL = 16 / sizeof(T);  // elements a lane holds of a key
   constexpr int HD = EPL * CPK;
-  constexpr int TILE = ATTN_DECODE_TILE_KEYS;
+  // two loads of keys at least: where 1 KB holds sixteen keys, a tile of one load left a wave twice the trips (bfloat16,
+  // 8 heads of 32, 500 keys, one row: 6.4 us, 5.8 with two loads; 4 rows at 60 to 500 6.5 and 5.9; 16 at 3,000 to 8,000 28.3
+  // and 22.7; float, 8 heads of 16, 32 rows at 300 to 1,000 10.2 and 8.7; a row of 50 keys 4.1 and 4.3)
+  constexpr int TILE = CPK < 8 ? 2 * ATTN_DECODE_TILE_KEYS : ATTN_DECODE_TILE_KEYS;
   constexpr int KPL = 64 / CPK;    // keys per load instruction
   constexpr int NL = TILE / KPL;   // loads per tile
   __shared__ float Ms[MAX_WAVES], Ls[MAX_WAVES];
