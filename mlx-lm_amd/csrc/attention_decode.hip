@@ -610,10 +610,10 @@ static void launch(const DecodeArgs& p, int n_rows, int n_waves, hipStream_t str
 // item i of `rows` is row i and belongs to request i (every request of the step brings one token),
 // which saves the kernel two trips to memory.  dtype DT_BF16 with head_dim 32, 64, 128 or 256, DT_F32
 // with 16, 32, 64 or 128, and pages that hold whole loads (page_size a multiple of the keys in 1 KB).
-// key_tile: 0, 32 or 64 (accepted, of no effect: a wave takes 16 keys at a time).  join_in_kernel: 0, a second kernel joins the
-// n_splits parts of a (row, head); 1, the block that finishes a (row, head) last does (up to
-// 65,536 (row, head)s; part_o and part_ml are still where the parts pass through); 2, the same,
-// and n_splits is only the most a row takes: a short row takes fewer, by its own length.
+// join_in_kernel: 0, a second kernel joins the n_splits parts of a (row, head); 1, the block that
+// finishes a (row, head) last does (up to 65,536 (row, head)s; part_o and part_ml are still where
+// the parts pass through); 2, the same, and n_splits is only the most a row takes: a short row
+// takes fewer, by its own length.
 // Launches that join in the kernel and overlap on one GPU race (they share the counters).
 static int decode_rows_launch(void* out, const void* q, int ldq, int ldo, const void* k_pages,
                               const void* v_pages, size_t page_stride, const int* block_table,
@@ -621,15 +621,14 @@ static int decode_rows_launch(void* out, const void* q, int ldq, int ldo, const 
                               const int* rows, int n_rows, int n_heads, int n_kv_heads, int head_dim,
                               int page_size, int window, float scale, int n_splits, float* part_o,
                               float* part_ml, int n_waves, const void* ahead, size_t ahead_chunk_bytes,
-                              int ahead_chunks, int rows_are_requests, int dtype, int key_tile,
-                              int join_in_kernel, const float* head_scale, const float* slopes,
+                              int ahead_chunks, int rows_are_requests, int dtype, int join_in_kernel,
+                              const float* head_scale, const float* slopes,
                               const void* gate, int ldg, int keep_first, const AttnTerms* shape, hipStream_t stream) {
   if (n_rows <= 0) return 0;
   if (shape && (shape->softcap < 0.f || (shape->dist_bias && shape->n_dist <= 0)))
     FAIL("attn_decode: softcap %g, a distance table of %d entries a head", (double)shape->softcap, shape->n_dist);
   if (keep_first < 0) FAIL("attn_decode: keep_first %d must not be negative", keep_first);
   if (gate && ldg < n_heads * head_dim) FAIL("attn_decode: the gate's row stride %d is smaller than its rows", ldg);
-  if (key_tile != 0 && key_tile != 32 && key_tile != 64) FAIL("attn_decode: key_tile %d is not 0, 32 or 64", key_tile);
   if (dtype != DT_F32 && dtype != DT_BF16) FAIL("attn_decode: unknown dtype code %d", dtype);
   const int epl = dtype == DT_F32 ? 4 : 8;  // elements in a lane's 16 bytes
   if (n_waves < 1 || n_waves > MAX_WAVES) FAIL("attn_decode: %d waves a block, must be 1 to %d", n_waves, MAX_WAVES);
@@ -708,13 +707,13 @@ extern "C" int attn_decode_rows_biased(void* out, const void* q, int ldq, int ld
                                        const int* rows, int n_rows, int n_heads, int n_kv_heads, int head_dim,
                                        int page_size, int window, float scale, int n_splits, float* part_o,
                                        float* part_ml, int n_waves, const void* ahead, size_t ahead_chunk_bytes,
-                                       int ahead_chunks, int rows_are_requests, int dtype, int key_tile,
+                                       int ahead_chunks, int rows_are_requests, int dtype,
                                        int join_in_kernel, const float* head_scale, const float* slopes,
                                        const void* gate, int ldg, int keep_first, hipStream_t stream) {
   return decode_rows_launch(out, q, ldq, ldo, k_pages, v_pages, page_stride, block_table, max_blocks, token_req,
                             positions, rows, n_rows, n_heads, n_kv_heads, head_dim, page_size, window, scale,
                             n_splits, part_o, part_ml, n_waves, ahead, ahead_chunk_bytes, ahead_chunks,
-                            rows_are_requests, dtype, key_tile, join_in_kernel, head_scale, slopes, gate, ldg,
+                            rows_are_requests, dtype, join_in_kernel, head_scale, slopes, gate, ldg,
                             keep_first, nullptr, stream);
 }
 
@@ -725,12 +724,12 @@ extern "C" int attn_decode_rows_terms(void* out, const void* q, int ldq, int ldo
                                       const int* rows, int n_rows, int n_heads, int n_kv_heads, int head_dim,
                                       int page_size, int window, float scale, int n_splits, float* part_o,
                                       float* part_ml, int n_waves, const void* ahead, size_t ahead_chunk_bytes,
-                                      int ahead_chunks, int rows_are_requests, int dtype, int key_tile,
+                                      int ahead_chunks, int rows_are_requests, int dtype,
                                       int join_in_kernel, const AttnTerms* t, hipStream_t stream) {
   return decode_rows_launch(out, q, ldq, ldo, k_pages, v_pages, page_stride, block_table, max_blocks, token_req,
                             positions, rows, n_rows, n_heads, n_kv_heads, head_dim, page_size, window, scale,
                             n_splits, part_o, part_ml, n_waves, ahead, ahead_chunk_bytes, ahead_chunks,
-                            rows_are_requests, dtype, key_tile, join_in_kernel, t ? t->head_scale : nullptr,
+                            rows_are_requests, dtype, join_in_kernel, t ? t->head_scale : nullptr,
                             t ? t->slopes : nullptr, t ? t->gate : nullptr, t ? t->ldg : 0, t ? t->keep_first : 0, t,
                             stream);
 }
@@ -741,12 +740,12 @@ extern "C" int attn_decode_rows(void* out, const void* q, int ldq, int ldo, cons
                                 const int* rows, int n_rows, int n_heads, int n_kv_heads, int head_dim,
                                 int page_size, int window, float scale, int n_splits, float* part_o,
                                 float* part_ml, int n_waves, const void* ahead, size_t ahead_chunk_bytes,
-                                int ahead_chunks, int rows_are_requests, int dtype, int key_tile,
+                                int ahead_chunks, int rows_are_requests, int dtype,
                                 int join_in_kernel, hipStream_t stream) {
   return attn_decode_rows_biased(out, q, ldq, ldo, k_pages, v_pages, page_stride, block_table, max_blocks, token_req,
                                  positions, rows, n_rows, n_heads, n_kv_heads, head_dim, page_size, window, scale,
                                  n_splits, part_o, part_ml, n_waves, ahead, ahead_chunk_bytes, ahead_chunks,
-                                 rows_are_requests, dtype, key_tile, join_in_kernel, nullptr, nullptr, nullptr, 0, 0,
+                                 rows_are_requests, dtype, join_in_kernel, nullptr, nullptr, nullptr, 0, 0,
                                  stream);
 }
 

@@ -43,8 +43,7 @@ __device__ __forceinline__ float head_gate_of(const Args& p, int row, int h) {
 
 // How the decode kernel (attention_decode.hip) is launched for n_rows single rows of n_heads
 // heads whose longest walk is `keys` keys (a window's and its kept first keys' at most): in how
-// many parts a row's keys go at most, and the waves a block (`key_tile` is always 32: callers of the
-// kernel may still name 32 or 64, its tiles are of ATTN_DECODE_TILE_KEYS whatever they say).
+// many parts a row's keys go at most, and the waves a block.
 // Eight waves a block; four where the rows' blocks alone are more than the CUs (64 rows of 25 heads
 // at contexts of 300 to 1,001: 49.2 us, 49.7 with eight, 53.5 with two; 24 rows 20.4 and 22.6), or the keys no
 // more than four waves' tiles; sixteen where blocks that have a CU each may walk 2,048 keys or more (8 rows at
@@ -60,7 +59,7 @@ __device__ __forceinline__ float head_gate_of(const Args& p, int row, int h) {
 #define ATTN_DECODE_SPLIT_KEYS_A_WAVE 64
 #define ATTN_DECODE_KEYS_A_PART 32
 static inline void attn_decode_row_work(int n_compute_units, int n_rows, int n_heads, int head_dim, long keys,
-                                        int* n_splits, int* n_waves, int* key_tile) {
+                                        int* n_splits, int* n_waves) {
   const long c = keys;
   const long tiles = c < 1 ? 1 : (c + ATTN_DECODE_TILE_KEYS - 1) / ATTN_DECODE_TILE_KEYS;
   const long blocks = n_rows * n_heads < 1 ? 1 : (long)n_rows * n_heads;
@@ -76,5 +75,5 @@ static inline void attn_decode_row_work(int n_compute_units, int n_rows, int n_h
     if (ns < 1) ns = 1;
   }
   if (ns == 1 && blocks <= n_compute_units && c >= 2048) nw = 2 * ATTN_DECODE_ROW_WAVES;
-  *n_splits = (int)ns, *n_waves = nw, *key_tile = 32;
+  *n_splits = (int)ns, *n_waves = nw;
 }

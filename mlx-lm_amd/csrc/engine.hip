@@ -110,7 +110,7 @@ typedef int (*fn_attn_row)(void*, const void*, int, int, const void*, const void
                            float*, float*, int, hipStream_t);
 typedef int (*fn_attn_decode)(void*, const void*, int, int, const void*, const void*, size_t, const int*, int,
                               const int*, const int*, const int*, int, int, int, int, int, int, float, int,
-                              float*, float*, int, const void*, size_t, int, int, int, int, int, hipStream_t);
+                              float*, float*, int, const void*, size_t, int, int, int, int, hipStream_t);
 typedef int (*fn_attn_decode_group)(void*, const void*, int, int, const void*, const void*, size_t, const int*, int,
                                     const int*, const int*, const int*, int, int, int, int, int, int, float, int,
                                     float*, float*, int, const AttnTerms*, hipStream_t);
@@ -127,7 +127,7 @@ typedef int (*fn_attn_row_terms)(void*, const void*, int, int, const void*, cons
                                  float*, float*, int, const AttnTerms*, hipStream_t);
 typedef int (*fn_attn_decode_terms)(void*, const void*, int, int, const void*, const void*, size_t, const int*, int,
                                     const int*, const int*, const int*, int, int, int, int, int, int, float, int,
-                                    float*, float*, int, const void*, size_t, int, int, int, int, int,
+                                    float*, float*, int, const void*, size_t, int, int, int, int,
                                     const AttnTerms*, hipStream_t);
 typedef int (*fn_attn_prefill_terms)(void*, const void*, int, int, const void*, const void*, size_t, const int*,
                                      int, const int*, const int*, const int*, int, int, int, int, int, int, float,
@@ -734,13 +734,13 @@ struct Attention : Mixer {
 
   int scatter_for(EngCtx* ctx, int slot, EngScatter* sc) const;
 
-  // (n_splits, n_waves, key_tile) for the decode kernel: attn_decode_row_work's rule.  n_splits is the
+  // (n_splits, n_waves) for the decode kernel: attn_decode_row_work's rule.  n_splits is the
   // most a row takes; the kernel gives a shorter row fewer by the same rule, so a recorded step,
   // planned for the model's positions, splits only the rows that are long.
-  void row_work(const EngCtx* ctx, int n_rows, long max_row_context, int* n_splits, int* n_waves,
-                int* key_tile) const {
-    const long c = window <= 0 ? max_row_context : (max_row_context < window + 31 ? max_row_context : window + 31);
-    attn_decode_row_work(ctx->n_compute_units, n_rows, n_heads, head_dim, c, n_splits, n_waves, key_tile);
+  void row_work(const EngCtx* ctx, int n_rows, long max_row_context, int* n_splits, int* n_waves) const {
+    const long most = window + ATTN_DECODE_TILE_KEYS - 1;  // (a window may begin at a tile's last key)
+    const long c = window <= 0 || max_row_context < most ? max_row_context : most;
+    attn_decode_row_work(ctx->n_compute_units, n_rows, n_heads, head_dim, c, n_splits, n_waves);
   }
 
   // How many ways to split a row's keys so that the general row kernel's launch fills the GPU.
@@ -823,7 +823,7 @@ struct Attention : Mixer {
       const int key_bytes = head_dim * (bf16 ? 2 : 4);
       const bool fast = (key_bytes == 64 || key_bytes == 128 || key_bytes == 256 || key_bytes == 512) &&
                         kv.page_size % (1024 / key_bytes) == 0;
-      int n_splits = 1, n_waves = 4, key_tile = 32;
+      int n_splits = 1, n_waves = 4;
       // eight or more query heads a key head (a latent that all heads share): the kernel that takes
       // them together on the matrix cores, so a key is read and multiplied once for all of them.
       // A block is four waves of sixteen keys at a time; a part for every 96 keys of the longest
@@ -852,7 +852,7 @@ struct Attention : Mixer {
         return 0;
       }
       if (fast)
-        row_work(ctx, n_rows, max_row_context, &n_splits, &n_waves, &key_tile);
+        row_work(ctx, n_rows, max_row_context, &n_splits, &n_waves);
       else
         n_splits = row_splits(ctx, n_rows, max_row_context);
       if (ctx->stats && n_splits > ctx->stats->key_splits_most) ctx->stats->key_splits_most = n_splits;
@@ -883,13 +883,13 @@ struct Attention : Mixer {
                  kv.block_table, kv.max_blocks, kv.token_req, kv.positions, rows, n_rows, n_heads, n_kv_heads, head_dim,
                  kv.page_size, window, scale, n_splits, (float*)part_o.p, (float*)part_ml.p, n_waves,
                  ahead ? ahead->packed : nullptr, ahead ? ahead->chunk_bytes : (size_t)0, chunks, rows_are_requests,
-                 q.dtype, key_tile, 2, terms, ctx->stream);
+                 q.dtype, 2, terms, ctx->stream);
         else
           KERNEL(k_attn_decode, ctx, out.p, q.p, q.ld, out_packed ? 0 : out.ld, kv.k, kv.v, kv.page_stride, kv.block_table,
                  kv.max_blocks, kv.token_req, kv.positions, rows, n_rows, n_heads, n_kv_heads, head_dim,
                  kv.page_size, window, scale, n_splits, (float*)part_o.p, (float*)part_ml.p, n_waves,
                  ahead ? ahead->packed : nullptr, ahead ? ahead->chunk_bytes : (size_t)0, chunks, rows_are_requests,
-                 q.dtype, key_tile, 2, ctx->stream);
+                 q.dtype, 2, ctx->stream);
       } else if (terms) {
         KERNEL(k_attn_row_terms, ctx, out.p, q.p, q.ld, out.ld, kv.k, kv.v, kv.page_stride, kv.block_table,
                kv.max_blocks, kv.token_req, kv.positions, rows, n_rows, n_heads, n_kv_heads, head_dim,

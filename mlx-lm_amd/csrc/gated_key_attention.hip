@@ -95,7 +95,7 @@ typedef int (*fn_attn_prefill_biased)(void*, const void*, int, int, const void*,
                                       const float*, const float*, const void*, int, int, hipStream_t);
 typedef int (*fn_attn_decode_biased)(void*, const void*, int, int, const void*, const void*, size_t, const int*, int,
                                      const int*, const int*, const int*, int, int, int, int, int, int, float, int,
-                                     float*, float*, int, const void*, size_t, int, int, int, int, int, const float*,
+                                     float*, float*, int, const void*, size_t, int, int, int, int, const float*,
                                      const float*, const void*, int, int, hipStream_t);
 typedef const char* (*fn_error)();
 #define ROW_KERNEL_MAX_HEAD_DIM 144  // beyond it the tile kernel takes single rows too
@@ -242,11 +242,12 @@ struct GatedKeyAttention : Mixer {
       if (n_rows) {
         const int key_bytes = head_dim * (bf16 ? 2 : 4);
         const bool fast = (key_bytes == 64 || key_bytes == 128 || key_bytes == 256) && kv.page_size % (1024 / key_bytes) == 0;
-        int n_splits = 1, n_waves = 4, key_tile = 32;
+        int n_splits = 1, n_waves = 4;
         if (fast) {
           long keys = longest;
-          if (window > 0 && keys > window + keep_first + 62) keys = window + keep_first + 62;
-          attn_decode_row_work(ctx->n_compute_units, n_rows, n_heads, head_dim, keys, &n_splits, &n_waves, &key_tile);
+          const long most = window + keep_first + 2 * (ATTN_DECODE_TILE_KEYS - 1);  // (two runs, each in tiles of its own)
+          if (window > 0 && keys > most) keys = most;
+          attn_decode_row_work(ctx->n_compute_units, n_rows, n_heads, head_dim, keys, &n_splits, &n_waves);
         } else {
           n_splits = row_splits(ctx, n_rows, longest);
         }
@@ -262,7 +263,7 @@ struct GatedKeyAttention : Mixer {
           if (attn_decode(o.p, qkg.p, qkg.ld, o.ld, kv.k, kv.v, kv.page_stride, kv.block_table, kv.max_blocks, kv.token_req,
                           kv.positions, rows, n_rows, n_heads, n_kv_heads, head_dim, kv.page_size, window, 1.f, n_splits,
                           (float*)part_o.p, (float*)part_ml.p, n_waves, nullptr, 0, 0, rows_are_requests, ctx->dtype,
-                          key_tile, 2, head_scale, slopes, gate, qkg.ld, keep_first, ctx->stream))
+                          2, head_scale, slopes, gate, qkg.ld, keep_first, ctx->stream))
             return host->fail("%s", decode_error());
         } else {
           if (attn_row(o.p, qkg.p, qkg.ld, o.ld, kv.k, kv.v, kv.page_stride, kv.block_table, kv.max_blocks, kv.token_req,
