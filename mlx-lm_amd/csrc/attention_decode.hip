@@ -161,7 +161,10 @@ __device__ __forceinline__ bool last_to_arrive(unsigned* counter, unsigned n_par
 // of 128 over 4 key heads 819 us at contexts of 6,000 to 8,001 and 107 at 700 to 1,300, 691 and 79 without the hint; 32 of
 // 32 over 8 396 and 294; float, 64 of 16 of 128 over 4 938 and 686.  (At few rows and short contexts it is the hint that is
 // ahead there too, by 3 to 8 %: 8 rows of 16 of 64 over 4, 60 to 500 keys, 7.3 and 7.9 us.)
-template <typename T, int CPK, bool ONCE>
+// SHAPED: scores also pass the soft cap and take the distance table's term.  A kernel of its own because a short walk waits
+// for its instructions: the loop below holds the arithmetic four times, each with a tanh a load, and beside blocks that
+// read weights ahead (2 rows of 25 heads of 64 at 60 to 500 keys) a launch took 9.3 us with them in and takes 8.9.
+template <typename T, int CPK, bool ONCE, bool SHAPED>
 __global__ __launch_bounds__(64 * (CPK >= 16 ? MAX_WAVES / 2 : MAX_WAVES)) void attn_decode_kernel(DecodeArgs p) {
   constexpr int EPL = 16 / sizeof(T);  // elements a lane holds of a key
   constexpr int HD = EPL * CPK;
@@ -313,9 +316,9 @@ __global__ __launch_bounds__(64 * (CPK >= 16 ? MAX_WAVES / 2 : MAX_WAVES)) void 
       for (int i = 0; i < EPL; ++i) d += qf[i] * kf[i];
       d = group_sum<CPK>(d);  // over the key's lanes
       const int key = kt + j * KPL + kin;
-      if (p.softcap > 0.f) d = p.softcap * tanhf(d / p.softcap);
+      if (SHAPED && p.softcap > 0.f) d = p.softcap * tanhf(d / p.softcap);
       d -= slope * (float)(pos - key);
-      if (p.dist_bias) d += p.dist_bias[(size_t)h * p.n_dist + min(max(pos - key, 0), p.n_dist - 1)];
+      if (SHAPED && p.dist_bias) d += p.dist_bias[(size_t)h * p.n_dist + min(max(pos - key, 0), p.n_dist - 1)];
       s[j] = (key >= t_lo && key < t_hi) ? d : -INFINITY;
       tmax = fmaxf(tmax, s[j]);
     }
@@ -598,10 +601,15 @@ static void launch(const DecodeArgs& p, int n_rows, int n_waves, hipStream_t str
   }
   const size_t lds = p.table_in_lds ? (size_t)p.max_blocks * sizeof(int) : 0;
   const dim3 grid(n_rows, p.n_heads + extra_y, p.n_splits), block(64 * n_waves);
-  if (p.n_heads == p.n_kv_heads)
-    hipLaunchKernelGGL((attn_decode_kernel<T, CPK, true>), grid, block, lds, stream, p);
+  const bool once = p.n_heads == p.n_kv_heads, shaped = p.softcap > 0.f || p.dist_bias;
+  if (once && !shaped)
+    hipLaunchKernelGGL((attn_decode_kernel<T, CPK, true, false>), grid, block, lds, stream, p);
+  else if (!shaped)
+    hipLaunchKernelGGL((attn_decode_kernel<T, CPK, false, false>), grid, block, lds, stream, p);
+  else if (once)
+    hipLaunchKernelGGL((attn_decode_kernel<T, CPK, true, true>), grid, block, lds, stream, p);
   else
-    hipLaunchKernelGGL((attn_decode_kernel<T, CPK, false>), grid, block, lds, stream, p);
+    hipLaunchKernelGGL((attn_decode_kernel<T, CPK, false, true>), grid, block, lds, stream, p);
   if (p.n_splits > 1 && !p.join_here)
     hipLaunchKernelGGL((attn_decode_merge_kernel<T, CPK>), dim3(n_rows, p.n_heads), dim3(16 / sizeof(T) * CPK), 0, stream, p);
 }
