@@ -639,7 +639,7 @@ extern "C" int gemm_bf16_splits(int M, int N, int K, int fused, int force) {
   return (n_blocks + per - 1) / per;  // no empty part
 }
 
-// variant: 0 = choose, 1 (and 7) = 128 x 128 tiles, 2 = skinny kernel, 3 = 256 x 256 tiles, 4 = 256 x 192
+// variant: 0 = choose, 1 = 128 x 128 tiles, 2 = skinny kernel, 3 = 256 x 256 tiles, 4 = 256 x 192
 // tiles, 5 = 64 x 128 tiles, 6 = 32 x 128 tiles, 8 = 256 x 128 tiles.  n_splits > 1 (variants 1, 5 and 6 only): no
 // epilogue, the partial sums go to ws.  ldw == 0: W is in the decode kernels' packed order
 // (tiles of 16 features x 64 k, zero padded), which all kernels here read as well as rows.
@@ -711,7 +711,6 @@ extern "C" int gemm_bf16_scatter(void* out, const void* A, const void* W, const 
     double us = 0.0;
     variant = M < TILE_MIN_ROWS ? 2 : cheapest_shape(M, N, K, 1, &us);
   }
-  if (variant == 7) variant = 1;
   if (variant == 2) {
     if (M > SK_MAXM) FAIL("gemm_bf16: the skinny kernel takes at most %d rows, got %d", SK_MAXM, M);
     dim3 grid((N + 15) / 16), block(256);
