@@ -196,8 +196,9 @@ __device__ __forceinline__ void finish4(const DecodeGemmArgs& p, int m, int n, f
 
 // LN: norm the rows of X in the prologue (K <= 2048: a lane holds its share of
 // a row in NV float4).  MULTI: K is longer than one pass of NW * U k-blocks
-// (2048); only then is the second set of weight registers needed.
-template <bool LN, bool MULTI>
+// (2048); only then is the second set of weight registers needed.  FEW: how rows that need no norm are copied; a
+// kernel each because a launch of 3 to 5 us waits for its instructions too (both ways in one cost 0.1 to 0.2 us).
+template <bool LN, bool MULTI, bool FEW>
 __global__ __launch_bounds__(NW * 64) void gemm_bf16_decode_kernel(DecodeGemmArgs p) {
   constexpr int NV = LN_MAX_V;
   constexpr int UU = MULTI ? 2 * U : U;  // k-blocks per pass and wave: long rows keep more in flight
@@ -309,43 +310,59 @@ __global__ __launch_bounds__(NW * 64) void gemm_bf16_decode_kernel(DecodeGemmArg
     }
   } else {
     load_pass(w0, 0);  // in flight while the activations are copied
-    // Wave w copies rows w and w + 8, four pieces of 16 bytes a lane and row at a time, all on their way together:
-    // one trip to L2.  The empty statement says that they are all wanted there: otherwise each load is moved down
-    // to the store that needs it, and each store waits for its own trip, after the weights' (pieces dealt to the
-    // threads, up to four trips at 8 rows and eight at 16; us before and now at 1 / 8 / 16 rows: 4,800 x 1,600
-    // 6.4 / 7.2 / 8.4 and 6.4 / 7.0 / 7.8; 1,600 x 1,600 4.2 / 4.8 / 5.3 and 4.1 / 4.4 / 4.8; 1,024 x 1,024 3.5 / 3.9 / 4.3
-    // and 3.5 / 3.7 / 3.9; 1,024 x 2,688 in two parts 4.3 / 4.7 / 5.2 and 4.2 / 4.4 / 4.6).  The rows asked for ahead of
-    // the weights, whose number is not known when this is compiled, are waited for together with them and cost more.
-    static_assert(2 * NW >= 16, "the waves' two rows cover all rows");
+    // The loads of a round are all on their way together: one trip to the L2s.  The empty statements say that they
+    // are all wanted there: otherwise each load is moved down to the store that needs it, and each store waits for its
+    // own trip, after the weights'.
     typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
-    const int row = __builtin_amdgcn_readfirstlane(wave);
-    const uint16_t* in = input_of(p, n0) + kb + lane * 8;
-    uint16_t* to = As + lane * 8;
     const int per_row = (min(p.K, kb + n_chunks * 64) - kb) / 8;
-    if (p.M == 1) {  // (a piece a thread; one wave with four made a step of batch 1 through 48 layers 1.84 ms, this 1.80)
-      for (int c = tid; c < per_row; c += NW * 64)
-        *(u32x4_t*)(to + row * 512 + (c - tid) * 8) = *(const u32x4_t*)(in + row * 512 + (c - tid) * 8);
-    }
-    for (int first = 0; p.M > 1 && row < p.M && first < per_row; first += 256) {
-      u32x4_t t[2][4];
+    if constexpr (FEW) {  // pieces of 16 bytes dealt to the threads, two at a time
+      const uint16_t* in = input_of(p, n0) + kb;
+      const int total = p.M * per_row;
+#pragma unroll 1
+      for (int c0 = tid; c0 < total; c0 += 2 * NW * 64) {
+        u32x4_t t[2];
+        int at[2];
 #pragma unroll
-      for (int h = 0; h < 2; ++h)
-        if (row + NW * h < p.M) {
-          const uint16_t* from = in + (size_t)(row + NW * h) * p.lda + first * 8;
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-            if (first + lane + 64 * i < per_row) t[h][i] = *(const u32x4_t*)(from + 512 * i);
+        for (int j = 0; j < 2; ++j) {
+          const int c = min(c0 + j * NW * 64, total - 1), r = c / per_row, k = (c - r * per_row) * 8;
+          at[j] = r * p.a_stride + k;
+          t[j] = *(const u32x4_t*)(in + (size_t)r * p.lda + k);
         }
-      asm volatile("" : "+v"(t[0][0]), "+v"(t[0][1]), "+v"(t[0][2]), "+v"(t[0][3]), "+v"(t[1][0]), "+v"(t[1][1]),
-                   "+v"(t[1][2]), "+v"(t[1][3]));
+        asm volatile("" : "+v"(t[0]), "+v"(t[1]));
 #pragma unroll
-      for (int h = 0; h < 2; ++h)
-        if (row + NW * h < p.M) {
-          uint16_t* into = to + (row + NW * h) * p.a_stride + first * 8;
+        for (int j = 0; j < 2; ++j)
+          if (c0 + j * NW * 64 < total) *(u32x4_t*)(As + at[j]) = t[j];
+      }
+    } else {  // wave w copies rows w and w + 8, four pieces a lane and row at a time
+      // (pieces dealt to the threads, up to four trips at 8 rows and eight at 16; us so and as here at 8 / 16 rows:
+      // 4,800 x 1,600 7.2 / 8.4 and 7.0 / 7.8; 1,600 x 1,600 4.8 / 5.3 and 4.4 / 4.8; 1,024 x 2,688 in two parts 4.7 / 5.2 and
+      // 4.4 / 4.6.  The rows asked for ahead of the weights, whose number is not known when this is compiled, are
+      // waited for together with them and cost more.)
+      static_assert(2 * NW >= 16, "the waves' two rows cover all rows");
+      const int row = __builtin_amdgcn_readfirstlane(wave);
+      const uint16_t* in = input_of(p, n0) + kb + lane * 8;
+      uint16_t* to = As + lane * 8;
+      for (int first = 0; row < p.M && first < per_row; first += 256) {
+        u32x4_t t[2][4];
 #pragma unroll
-          for (int i = 0; i < 4; ++i)
-            if (first + lane + 64 * i < per_row) *(u32x4_t*)(into + 512 * i) = t[h][i];
-        }
+        for (int h = 0; h < 2; ++h)
+          if (row + NW * h < p.M) {
+            const uint16_t* from = in + (size_t)(row + NW * h) * p.lda + first * 8;
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+              if (first + lane + 64 * i < per_row) t[h][i] = *(const u32x4_t*)(from + 512 * i);
+          }
+        asm volatile("" : "+v"(t[0][0]), "+v"(t[0][1]), "+v"(t[0][2]), "+v"(t[0][3]), "+v"(t[1][0]), "+v"(t[1][1]),
+                     "+v"(t[1][2]), "+v"(t[1][3]));
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+          if (row + NW * h < p.M) {
+            uint16_t* into = to + (row + NW * h) * p.a_stride + first * 8;
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+              if (first + lane + 64 * i < per_row) *(u32x4_t*)(into + 512 * i) = t[h][i];
+          }
+      }
     }
   }
   // What the epilogue takes from memory (the bias, and the stream's old value where the product
@@ -894,11 +911,17 @@ static int decode_launch(
   p.a_stride = a_stride_for(range);
   const size_t lds = (size_t)M * p.a_stride * 2;
   const bool multi = p.chunks_per_split > NW * U;
-  const int which = ln ? 2 : (multi ? 1 : 0);
-  void (*kernels[3])(DecodeGemmArgs) = {gemm_bf16_decode_kernel<false, false>,
-                                        gemm_bf16_decode_kernel<false, true>,
-                                        gemm_bf16_decode_kernel<true, false>};
-  static size_t granted[3] = {0, 0, 0};
+  // One or two rows leave most of the waves that copy a row each without one, and up to a piece of 16 bytes a thread
+  // the dealt pieces take one trip too, in fewer instructions (768 x 768: 5 rows 3.8 -> 3.7 us, 8 rows 4.0 -> 3.8; a step of
+  // two requests of GPT-2 XL 1,866 -> 1,830, of large 1,247 -> 1,230; with up to two pieces a thread 4 requests of XL
+  // take 1,913 instead of 1,883).
+  const bool few = !ln && (M <= 2 || M * (range / 8) <= NW * 64);
+  const int which = ln ? 0 : 1 + (multi ? 1 : 0) + (few ? 2 : 0);
+  void (*kernels[5])(DecodeGemmArgs) = {
+      gemm_bf16_decode_kernel<true, false, false>, gemm_bf16_decode_kernel<false, false, false>,
+      gemm_bf16_decode_kernel<false, true, false>, gemm_bf16_decode_kernel<false, false, true>,
+      gemm_bf16_decode_kernel<false, true, true>};
+  static size_t granted[5] = {0, 0, 0, 0, 0};
   const size_t fixed = sizeof(float) * (NW * 256 + (ln ? 2 * LN_MAX_V * 256 : 4));
   if (lds + fixed > 64 * 1024 && granted[which] < lds) {
     hipError_t e = hipFuncSetAttribute((const void*)kernels[which],

@@ -1238,11 +1238,12 @@ def test_gemm_bf16_rows_kernel_in_parts_and_with_the_cache_scatter(M, N, K):
             assert written.any() and torch.isnan(c.pool[~written].float()).all()
 
 
-@pytest.mark.parametrize("M", [1, 2, 7, 8, 9, 16])
-@pytest.mark.parametrize("K,splits", [(8, 1), (504, 1), (512, 1), (520, 1), (2040, 1), (2056, 1), (4104, 1), (4104, 2), (5120, 2)])
+@pytest.mark.parametrize("M", [1, 2, 3, 4, 7, 8, 9, 16])
+@pytest.mark.parametrize("K,splits", [(8, 1), (256, 1), (264, 1), (504, 1), (512, 1), (520, 1), (1024, 1), (1032, 1), (1360, 1), (1368, 1),
+                                      (2040, 1), (2056, 1), (4104, 1), (4104, 2), (5120, 2), (8200, 1), (12296, 1)])
 def test_decode_product_copies_every_row_whole(M, K, splits):
     """Rows that end inside, at and beyond a wave's piece of 64 x 8 columns, its four of them, and a block's parts of
-    K; one row, a row a wave, two rows a wave.  (Products of 16-bit numbers summed in 32 bits: the result's own
+    K; one row, a row a wave, two rows a wave; as many pieces as threads, one less and one more; two rounds of them.  (Products of 16-bit numbers summed in 32 bits: the result's own
     rounding is 2^-9.)"""
     k = _k()
     N = 48
