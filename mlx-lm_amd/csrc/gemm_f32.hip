@@ -143,6 +143,7 @@ __global__ __launch_bounds__(S::THREADS, 2) void gemm_f32_tile_kernel(GemmArgs p
     slot = slot == STAGES - 1 ? 0 : slot + 1;
   }
   multiply(1);
+  copies_arrived<0>();  // (what was asked for beyond the end)
 
   // Epilogue.  Accumulator r of tile (i, j): row 16 * i + x, feature 16 * j + 4 * g + r.  What is read (bias, the
   // residual stream to add to) is read for a row of tiles before anything of it is stored: a load that comes after a

@@ -9,7 +9,9 @@
 // every copy in flight before any LDS read.  It has no output register, so nothing can be overwritten by one in
 // flight; its two waits (for M0) stand in the same block.  What the compiler counts for its own loads stays right: copies
 // it does not know of only make its waits longer.  Who uses this waits with `copies_arrived` and a barrier before a
-// slot is read, and lets no wave write a slot that another may still read.
+// slot is read, and lets no wave write a slot that another may still read.  No wave ends, or uses the ring's LDS for
+// something else, with copies of its own in flight: what was asked for last is waited for with copies_arrived<0>, also
+// where nobody wants it.
 #pragma once
 #include "common.h"
 
