@@ -28,8 +28,8 @@ struct GemmArgs {
   int lda, ldw, ldo;
   int flags;
   // blockIdx.y takes part y of K's chunks of 64 columns (`per_split` of them) and leaves its sums
-  // in ws[y][M][N], without bias or epilogue
-  int n_splits, per_split;
+  // in ws[y][ws_rows][N], without bias or epilogue
+  int n_splits, per_split, ws_rows;
   float* ws;
 };
 
@@ -149,7 +149,7 @@ __global__ __launch_bounds__(S::THREADS, 2) void gemm_f32_tile_kernel(GemmArgs p
   // residual stream to add to) is read for a row of tiles before anything of it is stored: a load that comes after a
   // store to memory it might alias waits for it.
   const bool parts = p.n_splits > 1;
-  float* const out = parts ? p.ws + (size_t)blockIdx.z * p.M * p.N : p.out;
+  float* const out = parts ? p.ws + (size_t)blockIdx.z * p.ws_rows * p.N : p.out;
   const int ldo = parts ? p.N : p.ldo;
   const bool vec = ldo % 4 == 0 && ((uintptr_t)out & 15) == 0;
 #pragma unroll
@@ -289,7 +289,7 @@ __global__ __launch_bounds__(64 * SKF_MAX_WAVES) void gemm_f32_skinny_kernel(Gem
       float v = parts[b * 256 + tid];
       for (int w = 1; w < n_waves; ++w) v += parts[(w * RB + b) * 256 + tid];
       if (p.n_splits > 1) {
-        p.ws[((size_t)blockIdx.y * p.M + m) * p.N + n] = v;  // added up, and finished, by the caller's second kernel
+        p.ws[((size_t)blockIdx.y * p.ws_rows + m) * p.N + n] = v;  // added up, and finished, by the caller's second kernel
         continue;
       }
       if (p.bias) v += p.bias[n];
@@ -371,6 +371,24 @@ static void launch_tiles(const GemmArgs& p, hipStream_t stream) {
   hipLaunchKernelGGL(gemm_f32_tile_kernel<S>, grid, block, 0, stream, p);
 }
 
+static void launch(const GemmArgs& p, int variant, hipStream_t stream) {
+  if (variant == 1) return launch_tiles<F32Tile64x128>(p, stream);
+  if (variant == 2) return launch_tiles<F32Tile64>(p, stream);
+  if (variant == 4) return launch_tiles<F32Tile32x64>(p, stream);
+  // where the blocks are fewer than the compute units, more waves each
+  const int blocks = (p.N + 15) / 16;
+  const int waves = blocks * p.n_splits < n_compute_units() ? SKF_WAVES_FEW : SKF_WAVES_MANY;
+  const dim3 grid(blocks, p.n_splits), block(64 * waves);
+  if (p.M <= 16)
+    hipLaunchKernelGGL(gemm_f32_skinny_kernel<1>, grid, block, 0, stream, p);
+  else if (p.M <= 32)
+    hipLaunchKernelGGL(gemm_f32_skinny_kernel<2>, grid, block, 0, stream, p);
+  else if (p.M <= 48)
+    hipLaunchKernelGGL(gemm_f32_skinny_kernel<3>, grid, block, 0, stream, p);
+  else
+    hipLaunchKernelGGL(gemm_f32_skinny_kernel<4>, grid, block, 0, stream, p);
+}
+
 // variant: 0 = choose, 1 = tiles of 64 x 128, 2 = of 64 x 64, 4 = of 32 x 64, 3 = the kernel for up to
 // 64 rows.  n_splits > 1: K in that many parts, whose sums go to ws[part][M][N] (ws_floats floats at least) for sum_partials of gemm_bf16_decode.hip to add up
 // and finish; out is not written then.
@@ -382,7 +400,7 @@ extern "C" int gemm_f32(void* out, const void* A, const void* W, const float* bi
   p.W = (const float*)W;
   p.bias = bias;
   p.out = (float*)out;
-  p.M = M, p.N = N, p.K = K;
+  p.M = M, p.N = N, p.K = K, p.ws_rows = M;
   p.lda = lda, p.ldw = ldw, p.ldo = ldo;
   p.flags = flags;
   p.n_splits = 1, p.per_split = (K + SKF_CHUNK - 1) / SKF_CHUNK, p.ws = nullptr;
@@ -407,30 +425,19 @@ extern "C" int gemm_f32(void* out, const void* A, const void* W, const float* bi
   double us = 0.0;
   if (variant == 0) variant = M <= SKF_MAX_ROWS ? 3 : cheapest_shape(M, N, K, n_splits, &us);
   if (variant != 3 && p.per_split * (n_splits - 1) * SKF_CHUNK >= K) FAIL("gemm_f32: %d parts of K=%d leave one empty", n_splits, K);
-  if (variant != 3 && !(fits_copy_buffer(((size_t)127 * lda + K) * 4) && fits_copy_buffer(((size_t)127 * ldw + K) * 4)))
-    FAIL("gemm_f32: rows of K=%d floats, %d and %d apart, are too long", K, lda, ldw);
-  if (variant == 1) {
-    launch_tiles<F32Tile64x128>(p, stream);
-  } else if (variant == 2) {
-    launch_tiles<F32Tile64>(p, stream);
-  } else if (variant == 4) {
-    launch_tiles<F32Tile32x64>(p, stream);
-  } else if (variant == 3) {
-    if (M > SKF_MAX_ROWS) FAIL("gemm_f32: the kernel for few rows takes at most %d, got %d", SKF_MAX_ROWS, M);
-    // where the blocks are fewer than the compute units, more waves each
-    const int blocks = (N + 15) / 16;
-    const int waves = blocks * p.n_splits < n_compute_units() ? SKF_WAVES_FEW : SKF_WAVES_MANY;
-    const dim3 grid(blocks, p.n_splits), block(64 * waves);
-    if (M <= 16)
-      hipLaunchKernelGGL(gemm_f32_skinny_kernel<1>, grid, block, 0, stream, p);
-    else if (M <= 32)
-      hipLaunchKernelGGL(gemm_f32_skinny_kernel<2>, grid, block, 0, stream, p);
-    else if (M <= 48)
-      hipLaunchKernelGGL(gemm_f32_skinny_kernel<3>, grid, block, 0, stream, p);
-    else
-      hipLaunchKernelGGL(gemm_f32_skinny_kernel<4>, grid, block, 0, stream, p);
-  } else {
-    FAIL("gemm_f32: unknown variant %d", variant);
+  if (variant == 3 && M > SKF_MAX_ROWS)
+    FAIL("gemm_f32: the kernel for few rows takes at most %d, got %d", SKF_MAX_ROWS, M);
+  if (variant < 1 || variant > 4) FAIL("gemm_f32: unknown variant %d", variant);
+  // Rows some 8 million floats apart or more are beyond the 32-bit offsets of a tile's copies: the kernel for few
+  // rows, which has pointers, takes them 64 at a time.  More tiles of rows than a grid holds go in several launches.
+  if (!(fits_copy_buffer(((size_t)127 * lda + K) * 4) && fits_copy_buffer(((size_t)127 * ldw + K) * 4))) variant = 3;
+  const int most = variant == 3 ? SKF_MAX_ROWS : 65535 * (variant == 4 ? F32Tile32x64::BM : F32Tile64::BM);
+  static_assert(F32Tile64x128::BM == F32Tile64::BM, "both tiles' rows");
+  for (int left = M; left > 0; left -= most) {
+    p.M = left < most ? left : most;
+    launch(p, variant, stream);
+    p.A += (size_t)most * lda, p.out += (size_t)most * ldo;
+    if (p.ws) p.ws += (size_t)most * N;
   }
   CHECK_LAUNCH("gemm_f32");
   return 0;

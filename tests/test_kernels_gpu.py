@@ -130,6 +130,38 @@ def test_gemm_f32_tiles_at_the_ring_s_edges(M, N, K):
                 assert (wide[:, N:] == 0.5).all()
 
 
+@pytest.mark.parametrize("M,N,far", [(70, 33, "a"), (129, 20, "a"), (70, 70, "w"), (65, 9, "a")])
+@pytest.mark.parametrize("splits", [None, 2])
+def test_gemm_f32_rows_far_apart(M, N, far, splits):
+    """Rows (or features) more than 8 million floats apart: a tile of them is beyond 32-bit offsets.  (The bound of the
+    test above.)"""
+    k = _k()
+    K, apart = 192, 8_500_000
+    tall = torch.empty((M if far == "a" else N) * apart, device=DEV).view(-1, apart)[:, :K]
+    a, w = _rand((M, K), torch.float32, 10), _rand((N, K), torch.float32, 11, 0.1)
+    tall.copy_(a if far == "a" else w)
+    bias = _rand((N,), torch.float32, 12)
+    ref = plain.linear(a.double().cpu(), w.double().cpu(), bias.double().cpu())
+    tol = (K + 4) * 2.0**-24 * ((a.double().abs() @ w.double().abs().t()).max().item() + bias.abs().max().item() + 1)
+    for variant in (0, 1, 4):
+        out = torch.full((M, N), 0.5, device=DEV)
+        k.linear(out, tall if far == "a" else a, tall if far == "w" else w, bias, accumulate=True, variant=variant, splits=splits)
+        assert (out.double().cpu() - ref - 0.5).abs().max().item() < tol, variant
+
+
+def test_gemm_f32_more_rows_than_a_grid_of_tiles():
+    """More tiles of 32 rows than a grid's second dimension holds, whole and in parts of K."""
+    k = _k()
+    M, N, K = 65535 * 32 + 70, 1, 68
+    a, w = _rand((M, K), torch.float32, 10), _rand((N, K), torch.float32, 11, 0.1)
+    ref = a.double() @ w.double().t().contiguous()
+    tol = (K + 4) * 2.0**-24 * ((a.double().abs() @ w.double().abs().t().contiguous()).max().item() + 1)
+    for variant, splits in ((0, None), (4, None), (4, 2)):
+        out = torch.full((M, N), float("nan"), device=DEV)
+        k.linear(out, a, w, variant=variant, splits=splits)
+        assert (out.double() - ref).abs().max().item() < tol, (variant, splits)
+
+
 @pytest.mark.parametrize("N,K", [(1, 4), (7, 508), (9, 512), (17, 516), (40, 1024), (33, 1028), (100, 1600),
                                  (24, 2052), (4100, 520), (4097, 1600)])
 def test_gemm_f32_few_rows(N, K):
