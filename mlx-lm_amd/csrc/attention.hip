@@ -20,7 +20,8 @@
 //    of 64 staged in LDS; any head_dim that is a multiple of 16 up to 256 (wider heads, up to 1024:
 //    attn_tile_wide, which stages keys and values 256 columns at a time).
 //    Float caches with head_dim 64 or 128 in pages of whole 16 keys take
-//    attn_tile_mfma instead: a wave a tile, v_mfma_f32_16x16x4_f32, no LDS.
+//    attn_tile_mfma instead: v_mfma_f32_16x16x4_f32, a tile's keys over the block's four waves, LDS
+//    only for the waves' sums.
 //  * attn_row: one query per block, its keys split over the block's four
 //    waves and over `n_splits` blocks; attn_merge joins the splits.
 #include "common.h"

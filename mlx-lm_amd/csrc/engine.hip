@@ -53,7 +53,8 @@ extern "C" int eng_compute_units(void) { return n_compute_units(); }
 #define ROW_SPLIT_KEYS_A_WAVE ATTN_DECODE_SPLIT_KEYS_A_WAVE
 
 // The context length from which a decode step may split a row's keys over blocks (what a recorded
-// step's planning length is chosen by: below it no step launches splits).
+// step's planning length is chosen by: below it no step of the kernel for rows on their own launches
+// splits; the kernel that takes a key head's query heads together makes parts from 192 keys on).
 extern "C" int eng_rows_split_from(void) { return ROW_WAVES * ROW_SPLIT_KEYS_A_WAVE; }
 
 extern "C" void eng_attn_tile_sizes(int* tile, int* prefill_tile) {
