@@ -172,6 +172,9 @@ __global__ __launch_bounds__(64 * (CPK >= 16 ? MAX_WAVES / 2 : MAX_WAVES)) void 
   // 8 heads of 32, 500 keys, one row: 6.4 us, 5.8 with two loads; 4 rows at 60 to 500 6.5 and 5.9; 16 at 3,000 to 8,000 28.3
   // and 22.7; float, 8 heads of 16, 32 rows at 300 to 1,000 10.2 and 8.7; a row of 50 keys 4.1 and 4.3)
   constexpr int TILE = CPK < 8 ? 2 * ATTN_DECODE_TILE_KEYS : ATTN_DECODE_TILE_KEYS;
+  // (keys of 64 bytes a wave has sooner than the parts are joined: one row of 754 keys, float, 12 heads of 16, 6.7 us whole and
+  // 7.5 in two parts; bfloat16, 8 heads of 32, 6.8 and 7.6; 4 rows at 512 to 1,000 7.6 and 8.0)
+  constexpr int SPLIT_FROM = CPK < 8 ? ATTN_DECODE_SPLIT_KEYS_A_WAVE * 3 / 2 : ATTN_DECODE_SPLIT_KEYS_A_WAVE;
   constexpr int KPL = 64 / CPK;    // keys per load instruction
   constexpr int NL = TILE / KPL;   // loads per tile
   __shared__ float Ms[MAX_WAVES], Ls[MAX_WAVES];
@@ -256,7 +259,7 @@ __global__ __launch_bounds__(64 * (CPK >= 16 ? MAX_WAVES / 2 : MAX_WAVES)) void 
   int n_splits = p.n_splits;
   if (p.join_here == 2) {
     const int keys_a_wave = (k_hi - kt0 + n_sink_tiles * TILE) / n_waves;
-    n_splits = keys_a_wave >= ATTN_DECODE_SPLIT_KEYS_A_WAVE ? min(n_splits, keys_a_wave / ATTN_DECODE_KEYS_A_PART) : 1;
+    n_splits = keys_a_wave >= SPLIT_FROM ? min(n_splits, keys_a_wave / ATTN_DECODE_KEYS_A_PART) : 1;
     if (split >= n_splits) return;  // (the whole block)
   }
   const int per_split = (n_tiles + n_splits - 1) / n_splits;
