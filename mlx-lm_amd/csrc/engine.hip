@@ -348,15 +348,20 @@ extern "C" int eng_linear_norms_itself(const EngCtx* ctx, int M, int N, int K, i
   return takes(M, K, 1, n_splits) != 0;
 }
 
+// Whether a product's parts may wait for whoever reads `out` next to add them up.
+// (allowed == 2: it does, also where the product writes its float32 rows instead of adding to them; `out`
+// itself is not touched then)
+static bool may_stay_pending(const EngMat& out, int gelu, bool accumulate, const EngScatter* sc, const EngPending* pending, bool out_packed) {
+  const bool writes_plain = !accumulate && !gelu && !sc && !out_packed && out.dtype == DT_F32 && out.ld == out.cols;
+  return pending && ((accumulate && pending->allowed) || (writes_plain && pending->allowed == 2));
+}
+
 // What follows a product that left K in parts in the workspace: the sum stays pending where it
 // goes into the residual stream and the caller allows that (the next norm adds it), otherwise
 // the second kernel adds the parts and runs the epilogue.
 static int finish_parts(EngCtx* ctx, const EngMat& out, float* ws, int n_splits, const float* bias, int gelu,
                         bool accumulate, const EngScatter* sc, EngPending* pending, bool out_packed = false) {
-  // (allowed == 2: whoever reads `out` next adds the parts up itself, also where the product
-  // writes its float32 rows instead of adding to them; `out` itself is not touched then)
-  const bool writes_plain = !accumulate && !gelu && !sc && !out_packed && out.dtype == DT_F32 && out.ld == out.cols;
-  if (pending && ((accumulate && pending->allowed) || (writes_plain && pending->allowed == 2))) {
+  if (may_stay_pending(out, gelu, accumulate, sc, pending, out_packed)) {
     pending->target = (float*)out.p, pending->rows = out.rows, pending->cols = out.cols, pending->ld = out.ld;
     pending->ws = ws, pending->n_splits = n_splits, pending->bias = bias;
     return 0;
@@ -368,20 +373,31 @@ static int finish_parts(EngCtx* ctx, const EngMat& out, float* ws, int n_splits,
 // parts (*n_splits; 0: it does not).
 // (A matrix of more blocks than two a CU, the vocabulary's, would take that kernel several rounds,
 // each with its own wait for memory: the tiles stream it 6 us faster.  Beyond 32 rows it takes
-// K from 768 on, the shortest it was measured at: a step of 40 / 48 / 64 requests, contexts of 100
+// K from 768 on: at 512 and 640 it would take K in parts and be behind (33 to 64 rows, 512 to 2,560 features, a product alone
+// 6.4 to 8.2 us, the tiles 5.6 to 6.3); at 768 the product alone is level and in a step, where the norm adds the parts up,
+// ahead; at 384 and less, in one part, it would be 0.2 to 0.7 us ahead (4.5 us), which no model here asks for.  A step of 40 / 48 / 64 requests, contexts of 100
 // to 400, takes GPT-2 small (K 768 and 3,072) 0.640 / 0.665 / 0.715 ms and large (1,280 and 5,120)
 // 1.96 / 2.02 / 2.24; with the tiles where K is below 1,536, 0.650 / 0.679 / 0.723 and 2.24 / 2.33 / 2.59.)
-static int rows_parts(const EngCtx* ctx, int M, const EngWeight& w, int variant, int splits, int* n_splits) {
+// `fused`: a sum of parts would be left to the norm that follows.  Where nobody takes it, parts cost a second kernel, more
+// than they save: K goes whole if the kernel holds it (1,024 x 1,024 at 17 / 48 / 64 rows 7.3 / 9.2 / 9.4 us in two parts,
+// 5.0 / 5.0 / 5.1 whole; the tiles 8.2 and 8.6 at the latter two).
+static int rows_parts(const EngCtx* ctx, int M, const EngWeight& w, int variant, int splits, bool fused, int* n_splits) {
   *n_splits = 0;
   const int N = w.N, K = w.K;
   if (!(w.dtype == DT_BF16 && variant == 0 && M > DECODE_MAX_ROWS && M <= ROWS_MAX_ROWS && w.packed &&
         (M <= 32 || K >= 768) && (N + 31) / 32 <= 2 * ctx->n_compute_units))
     return 0;
   int n = 0;
-  if (splits == 0)
-    QUERY(k_rows_splits, n, M, N, K, ctx->force_splits);
-  else
+  if (splits != 0) {
     n = split_count((K + 63) / 64, splits);
+  } else {
+    QUERY(k_rows_splits, n, M, N, K, ctx->force_splits);
+    if (n > 1 && !fused && ctx->force_splits <= 0) {
+      int whole = 0;
+      QUERY(k_rows_takes, whole, M, K, 1);
+      if (whole) n = 1;
+    }
+  }
   if (n > 1 && (!ctx->split_ws || (size_t)n > ctx->split_ws_floats / ((size_t)M * N))) n = 0;  // (the tiles then)
   if (n >= 1) {
     int takes = 0;
@@ -395,7 +411,7 @@ static int rows_parts(const EngCtx* ctx, int M, const EngWeight& w, int variant,
 // That product reads its rows fastest in the packed order: who makes the rows may write them so.
 static bool wants_packed(const EngCtx* ctx, int M, const EngWeight* w) {
   int n = 0;
-  return w && rows_parts(ctx, M, *w, 0, 0, &n) == 0 && n >= 1;
+  return w && rows_parts(ctx, M, *w, 0, 0, true, &n) == 0 && n >= 1;
 }
 
 extern "C" int eng_wants_packed_rows(const EngCtx* ctx, const EngWeight* w, int n_rows) {
@@ -438,7 +454,7 @@ static int linear(EngCtx* ctx, const EngMat& out, const EngValue& a, const EngWe
   const size_t ws_floats = ctx->split_ws_floats;
   if (a.packed || out_packed) {
     int n = 0;
-    if (M > 0) TRY(rows_parts(ctx, M, w, variant, splits, &n));
+    if (M > 0) TRY(rows_parts(ctx, M, w, variant, splits, true, &n));
     if (n < 1) FAIL("linear: rows in the packed order are for the product of 17 to 64 rows only");
   }
 
@@ -479,7 +495,7 @@ static int linear(EngCtx* ctx, const EngMat& out, const EngValue& a, const EngWe
   {
     // 17 to 64 rows: the kernel that holds a block's weights in registers, if the sizes fit it
     int n_splits = 0;
-    TRY(rows_parts(ctx, M, w, variant, splits, &n_splits));
+    TRY(rows_parts(ctx, M, w, variant, splits, may_stay_pending(out, gelu, accumulate, sc, pending, out_packed), &n_splits));
     if (n_splits >= 1) {
       if (n_splits > 1 && pending) TRY(settle(ctx, pending));  // the workspace is about to be written again
       KERNEL(k_gemm_rows, ctx, out.p, A.p, a.packed ? 0 : A.ld, w.packed, bias, M, N, K, out_packed ? 0 : out.ld,
