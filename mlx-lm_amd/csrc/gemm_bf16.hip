@@ -139,6 +139,7 @@ using Tile256 = TileShape<2, 4, 4, 2, 2, 4, 2>;
 using Tile256x192 = TileShape<4, 2, 2, 3, 2, 4, 2>;
 using Tile256x128 = TileShape<4, 2, 2, 2, 3, 4, 2>;
 using Tile128 = TileShape<2, 4, 2, 1, 4, 8, 2>;
+using Tile128Pair = TileShape<2, 4, 2, 1, 2, 8, 4>;  // two blocks a CU (pairs_of_blocks below)
 using Tile64x128 = TileShape<2, 4, 1, 1, 3, 8, 4>;  // two blocks a CU, as the next
 using Tile32x128 = TileShape<1, 4, 1, 1, 4, 8, 2>;
 
@@ -575,7 +576,7 @@ static void launch_tiles(const GemmArgs& p, hipStream_t stream) {
 // a k-block where two blocks share the CU (shapes that fit twice), `launch` once.  Fitted to the times of 16 numbers of
 // rows from 20 to 8,000 against 18 matrices of widths from 768 to 2,048, K up to 6,400, each with K in 1 to 8 parts; the
 // shape and parts chosen from these prices are within 2 % of the best on average (at worst 1.35 times: 20 to 64 rows to
-// 10,880 features, which only one kind of design asks of these kernels).
+// 10,880 features, a gated feed-forward 2,048 wide, which the kernel for few rows cannot hold).
 struct TilePrice {
   int variant, bm, bn, per_cu;
   double launch, tile, kblock, pair;
@@ -610,6 +611,17 @@ static int cheapest_shape(int M, int N, int K, int n_splits, double* us) {
   return variant;
 }
 
+// Matrices of more columns of tiles than CUs (a vocabulary's) at rows that would leave half or more of the last 256-row
+// tile empty: blocks of 128 x 128, two a CU, one of which reads weights or stores while the other multiplies.  The prices
+// were fitted to narrower matrices and do not show it.  32-bit logits, us, by the prices and so: 50,257 x 768 at 65 / 128 /
+// 333 rows 27.5 / 36.1 / 76.8 and 24.5 / 31.8 / 70.8 (26.3 / 33.7 / 66.1 with the kernel before the LDS ring, which had two
+// such blocks a CU too); 50,257 x 1,600 43.0 / 53.6 / 107 and 38.9 / 49.3 / 106 (46.4 / 54.1 / 98.4); 50,304 x 1,024 26.5 / 31.5 /
+// 60.7 and 24.3 / 27.6 / 55.1 (28.8 / 31.6 / 58.3).  Not at 170, 256 and 512 rows (50,257 x 768 40.4 / 47.3 / 86.3 and 46.8 / 56.3 /
+// 98.4), nor where every CU has one tile (32,000 x 2,048 at 128 rows 30.8 and 36.9).
+static bool pairs_of_blocks(int M, int N) {
+  return ((M > 64 && M <= 128) || (M > 256 && M <= 384)) && (N + 127) / 128 > n_compute_units();
+}
+
 // Into how many parts the kernels with tiles 128 wide should split K (1: no split).  Few rows
 // give few tiles (up to 128 rows of GPT-2 XL's projections are 13 to 50 tiles for 256 CUs), and a
 // tile's walk through K takes the same time whether 50 or 500 of them run; a split shortens the
@@ -639,7 +651,7 @@ extern "C" int gemm_bf16_splits(int M, int N, int K, int fused, int force) {
   return (n_blocks + per - 1) / per;  // no empty part
 }
 
-// variant: 0 = choose, 1 = 128 x 128 tiles, 2 = skinny kernel, 3 = 256 x 256 tiles, 4 = 256 x 192
+// variant: 0 = choose, 1 = 128 x 128 tiles, 7 = the same two blocks a CU, 2 = skinny kernel, 3 = 256 x 256 tiles, 4 = 256 x 192
 // tiles, 5 = 64 x 128 tiles, 6 = 32 x 128 tiles, 8 = 256 x 128 tiles.  n_splits > 1 (variants 1, 5 and 6 only): no
 // epilogue, the partial sums go to ws.  ldw == 0: W is in the decode kernels' packed order
 // (tiles of 16 features x 64 k, zero padded), which all kernels here read as well as rows.
@@ -709,7 +721,7 @@ extern "C" int gemm_bf16_scatter(void* out, const void* A, const void* W, const 
   }
   if (variant == 0) {
     double us = 0.0;
-    variant = M < TILE_MIN_ROWS ? 2 : cheapest_shape(M, N, K, 1, &us);
+    variant = M < TILE_MIN_ROWS ? 2 : pairs_of_blocks(M, N) ? 7 : cheapest_shape(M, N, K, 1, &us);
   }
   if (variant == 2) {
     if (M > SK_MAXM) FAIL("gemm_bf16: the skinny kernel takes at most %d rows, got %d", SK_MAXM, M);
@@ -725,6 +737,8 @@ extern "C" int gemm_bf16_scatter(void* out, const void* A, const void* W, const 
       hipLaunchKernelGGL(gemm_bf16_skinny_kernel<4>, grid, block, 0, stream, p);
   } else if (variant == 1) {
     launch_tiles<Tile128, true>(p, stream);
+  } else if (variant == 7) {
+    launch_tiles<Tile128Pair, false>(p, stream);
   } else if (variant == 5) {
     launch_tiles<Tile64x128, true>(p, stream);
   } else if (variant == 6) {

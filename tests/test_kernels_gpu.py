@@ -207,7 +207,8 @@ def test_gemm_bf16(M, N, K, mode):
     w = _rand((N, K), torch.bfloat16, 11, 0.1)
     bias = _rand((N,), torch.float32, 12)
     ref = plain.linear(a.double().cpu(), w.double().cpu(), bias.double().cpu())
-    variants = (1, 2, 3, 4, 5, 6, 8) if M <= 64 else (1, 3, 4, 5, 6, 8)  # tiles of 128 x 128, skinny, 256 x 256, 256 x 192, 64 x 128, 32 x 128, 256 x 128
+    # tiles of 128 x 128, skinny, 256 x 256, 256 x 192, 64 x 128, 32 x 128, 128 x 128 two blocks a compute unit, 256 x 128
+    variants = (1, 2, 3, 4, 5, 6, 7, 8) if M <= 64 else (1, 3, 4, 5, 6, 7, 8)
     for variant in variants:
         if mode == "accumulate":
             out = _rand((M, N), torch.float32, 13)
@@ -1129,7 +1130,7 @@ def test_gemm_bf16_reads_weights_kept_in_packed_order_only(M, N, K):
     packed = k.PackedWeight(w.clone(), keep_rows=False)
     assert packed.w is None and not packed.c.w
     ref = plain.linear(a.double().cpu(), w.double().cpu(), bias.double().cpu())
-    variants = [(v, None) for v in ((1, 2, 3, 4, 5, 6, 8) if M <= 64 else (1, 3, 4, 5, 6, 8))]
+    variants = [(v, None) for v in ((1, 2, 3, 4, 5, 6, 7, 8) if M <= 64 else (1, 3, 4, 5, 6, 7, 8))]
     if M > 16 and K >= 192:
         variants += [(1, 3), (5, 2), (6, 3), (0, 2)]  # K in parts
     variants.append((0, None))  # the library's own choice
@@ -1164,7 +1165,7 @@ def test_gemm_bf16_tiles_at_the_ring_s_edges(M, N, K, packed):
     tol = K * 2.0**-24 * (a.double().abs() @ w.double().abs().t()).max().item() + 1e-6
     weights = k.PackedWeight(w.contiguous(), keep_rows=False) if packed else w
     parts = [s for s in (2, 3) if s <= (K + 63) // 64]
-    for variant, splits in [(v, None) for v in (1, 3, 4, 5, 6, 8)] + [(v, s) for v in (1, 5, 6) for s in parts]:
+    for variant, splits in [(v, None) for v in (1, 3, 4, 5, 6, 7, 8)] + [(v, s) for v in (1, 5, 6) for s in parts]:
         out = torch.full((M, N), 7.0, dtype=torch.float32, device=DEV)
         k.linear(out, a, weights, bias, variant=variant, splits=splits)
         err = (out.double().cpu() - ref).abs().max().item()
@@ -1289,14 +1290,16 @@ def test_decode_product_copies_every_row_whole(M, K, splits):
 
 
 @pytest.mark.parametrize("M", [33, 48, 49, 64])
-@pytest.mark.parametrize("N,K", [(2304, 768), (768, 768), (768, 3072), (3840, 1280), (1000, 1528), (64, 64)])
+@pytest.mark.parametrize("N,K", [(2304, 768), (768, 768), (768, 3072), (3840, 1280), (1000, 1528), (640, 760), (64, 64)])
 def test_products_of_33_to_64_rows_with_a_short_k(M, N, K):
-    """Left to choose, narrow matrices at these rows too: into the stream and as activations.  (As above.)"""
+    """Left to choose, narrow matrices at these rows too: into the stream and as activations, by the kernel that holds
+    its weights in registers from K = 768 on and by the tiles below.  (As above.)"""
     k = _k()
     a = _rand((M, K), torch.bfloat16, M)
     w = _rand((N, K), torch.bfloat16, N, 0.1)
     bias = _rand((N,), torch.float32, 12)
     packed = k.PackedWeight(w, keep_rows=False)
+    assert k.wants_packed_rows(packed, M) == (K >= 768) and k.wants_packed_rows(packed, 32)
     ref = plain.linear(a.double().cpu(), w.double().cpu(), bias.double().cpu())
     out = torch.full((M, N), 7.0, dtype=torch.bfloat16, device=DEV)
     k.linear(out, a, packed, bias)
@@ -1636,7 +1639,7 @@ def test_projection_scatters_keys_and_values(M, dtype, splits):
         assert torch.isnan(pool[page, 0, :, row + 1 :].float()).all()
 
 
-@pytest.mark.parametrize("variant", [0, 1, 3, 4, 5, 6, 8])
+@pytest.mark.parametrize("variant", [0, 1, 3, 4, 5, 6, 7, 8])
 @pytest.mark.parametrize("packed", [False, True])
 def test_tile_products_scatter_keys_and_values_themselves(variant, packed):
     """The many-row product writes keys and values into their pages from its own epilogue (every tile
