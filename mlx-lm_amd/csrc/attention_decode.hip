@@ -164,8 +164,12 @@ __device__ __forceinline__ bool last_to_arrive(unsigned* counter, unsigned n_par
 // SHAPED: scores also pass the soft cap and take the distance table's term.  A kernel of its own because a short walk waits
 // for its instructions: the loop below holds the arithmetic four times, each with a tanh a load, and beside blocks that
 // read weights ahead (2 rows of 25 heads of 64 at 60 to 500 keys) a launch took 9.3 us with them in and takes 8.9.
+// Five waves a SIMD at most for bfloat16 heads of 64 with a key head each: without the tanh's registers seven fit, all blocks
+// of 64 rows of 25 heads start at once and rows of unequal length end unevenly (a step of GPT-2 XL at 64 requests, contexts of
+// 300 to 1,001, 4.74 ms with seven, 4.54 with five).  Heads that share keys are 1 to 6 % ahead with seven.
 template <typename T, int CPK, bool ONCE, bool SHAPED>
-__global__ __launch_bounds__(64 * (CPK >= 16 ? MAX_WAVES / 2 : MAX_WAVES)) void attn_decode_kernel(DecodeArgs p) {
+__global__ __launch_bounds__(64 * (CPK >= 16 ? MAX_WAVES / 2 : MAX_WAVES))
+__attribute__((amdgpu_waves_per_eu(CPK >= 16 ? 2 : 4, CPK == 8 && sizeof(T) == 2 && ONCE ? 5 : 8))) void attn_decode_kernel(DecodeArgs p) {
   constexpr int EPL = 16 / sizeof(T);  // elements a lane holds of a key
   constexpr int HD = EPL * CPK;
   // two loads of keys at least: where 1 KB holds sixteen keys, a tile of one load left a wave twice the trips (bfloat16,
