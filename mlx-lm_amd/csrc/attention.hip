@@ -482,7 +482,8 @@ __global__ __launch_bounds__(256) void attn_tile_wide_kernel(AttnArgs p) {
 // earlier.  Prompts of 215 + 480 + 330 tokens, 20 heads of 64: 55.7 us with a wave a tile, 31.1 with
 // four, 28.4 since the masks, shuffles and rescaling are left out where no key needs them; one of
 // 80 tokens, 12 heads: 8.6 and 5.9; two of 1,024: 162 and 107; one of 4,000: 787 and 493 (its matrix
-// work alone takes 266); two of 500, 16 heads of 128: 62 and 57.  Four waves a SIMD want at most 128
+// work alone takes 266); two of 500, 16 heads of 128: 62 and 57 (but 2,000 under a
+// window of 256, where every walk is short and blocks are many, 73 and 78; 20 heads of 64 55 and 48).  Four waves a SIMD want at most 128
 // registers for heads of 64, which the compiler keeps only when told.
 
 template <int NV>

@@ -373,14 +373,15 @@ static int finish_parts(EngCtx* ctx, const EngMat& out, float* ws, int n_splits,
 // parts (*n_splits; 0: it does not).
 // (A matrix of more blocks than two a CU, the vocabulary's, would take that kernel several rounds,
 // each with its own wait for memory: the tiles stream it 6 us faster.  Beyond 32 rows it takes
-// K from 768 on: at 512 and 640 it would take K in parts and be behind (33 to 64 rows, 512 to 2,560 features, a product alone
-// 6.4 to 8.2 us, the tiles 5.6 to 6.3); at 768 the product alone is level and in a step, where the norm adds the parts up,
-// ahead; at 384 and less, in one part, it would be 0.2 to 0.7 us ahead (4.5 us), which no model here asks for.  A step of 40 / 48 / 64 requests, contexts of 100
+// K from 768 on.  Below, where a sum is left to the norm, it would take K in parts: 33 to 64 rows at K 512 and 640,
+// 512 to 2,560 features, 6.4 to 8.2 us with the second kernel, the tiles 5.6 to 6.3.  With K whole it would be ahead there
+// too (4.5 us at K 256 and 384, the tiles 4.6 to 5.3); no model here is so narrow.  From 768 on, a step of 40 / 48 / 64 requests, contexts of 100
 // to 400, takes GPT-2 small (K 768 and 3,072) 0.640 / 0.665 / 0.715 ms and large (1,280 and 5,120)
 // 1.96 / 2.02 / 2.24; with the tiles where K is below 1,536, 0.650 / 0.679 / 0.723 and 2.24 / 2.33 / 2.59.)
 // `fused`: a sum of parts would be left to the norm that follows.  Where nobody takes it, parts cost a second kernel, more
 // than they save: K goes whole if the kernel holds it (1,024 x 1,024 at 17 / 48 / 64 rows 7.3 / 9.2 / 9.4 us in two parts,
-// 5.0 / 5.0 / 5.1 whole; the tiles 8.2 and 8.6 at the latter two).
+// 5.3 whole, the tiles 8.2 and 8.6 at the latter two; 2,304 x 768 7.6 / 7.9 / 8.3 and 5.0 / 5.1 / 5.5; 1,600 x 1,600 7.8 / 8.6 /
+// 8.5 and 5.5 / 5.6 / 5.6).
 static int rows_parts(const EngCtx* ctx, int M, const EngWeight& w, int variant, int splits, bool fused, int* n_splits) {
   *n_splits = 0;
   const int N = w.N, K = w.K;

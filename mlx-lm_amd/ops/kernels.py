@@ -326,13 +326,11 @@ force_splits = 0
 
 def splits_alone(n_rows):
     """``splits`` for a product of ``n_rows`` rows whose partial sums nobody else would add (a part
-    written in Python has no norm behind it that takes them): 17 to 64 rows go unsplit, since the
-    second kernel that adds the parts costs more there than the split saves as long as the kernel for
-    these rows holds all of K (up to 1,792: 1,024 x 1,024 at 17 / 48 / 64 rows 5.0 / 5.0 / 5.1 us unsplit,
-    7.3 / 9.2 / 9.4 in the library's parts; 3,072 x 1,024 5.3 / 6.6 / 6.7 and 8.3 / 8.8 / 9.5).  Longer K goes to
-    tiles unsplit, which is ahead for wide matrices (10,880 x 2,048 16 us, 19 to 28 in parts) and level
-    at 2,048 x 2,048 (10.1 and 8.2 to 9.9), behind for narrow ones of long K (2,048 x 5,440 20 to 25, 11 to
-    15 in parts).  Otherwise the library chooses."""
+    written in Python has no norm behind it that takes them): 17 to 64 rows go unsplit, as the
+    library does by itself as long as the kernel for these rows holds all of K (up to 1,792). Longer
+    K goes to tiles unsplit, which is ahead of the library's parts for wide matrices (10,880 x 2,048 16 us,
+    19 to 28 in parts), 0 to 2 us behind at 2,048 x 2,048 (10.1; 8.2 to 9.9) and behind for narrow ones
+    of long K (2,048 x 5,440 20 to 25, 11 to 15 in parts). Otherwise the library chooses."""
     return 1 if DECODE_MAX_ROWS < n_rows <= 64 else None
 
 
