@@ -84,6 +84,12 @@ typedef struct {
   long key_splits_most;  // the most parts that a row kernel split a row's keys into
 } EngStats;
 
+// What the one launch of a decode step of one or two rows needs of an engine (decode_chain.h), made once.
+typedef struct {
+  const void* layers;  // the layers' table on the device (eng_chain_table)
+  void* memory[2];     // the launch's own for one row and for two (eng_chain_sizes)
+} EngChain;
+
 // One step's batch as the parts see it.
 typedef struct {
   hipStream_t stream;
@@ -110,6 +116,7 @@ typedef struct {
   const EngWeight* read_ahead;
   EngStats* stats;
   void* py;  // the Python side's own handle of this step (opaque here)
+  const EngChain* chain;  // null: every layer's launches of its own
 } EngCtx;
 
 // What a callback part's method gets and gives.
@@ -177,6 +184,10 @@ void eng_free(EngPart* part);
 
 // Each returns 0, or 1 with the text in mlxlm_last_error() (2: a callback kept a Python exception).
 int eng_model_forward(EngPart* model, EngCtx* ctx);
+// 1 if the model's layers over these cache slots can run as one launch, with the bytes of the layers' table and of the
+// launch's memory for one and for two rows (0: not for so many); eng_chain_table writes the table to host memory.
+int eng_chain_sizes(EngPart* model, const EngSlot* slots, int n_slots, size_t* table_bytes, size_t* one_row, size_t* two_rows);
+int eng_chain_table(EngPart* model, const EngSlot* slots, int n_slots, void* table);
 int eng_block_forward(EngPart* block, EngCtx* ctx, const EngMat* h, int cache_slot, int writes_cache,
                       int state_slot);
 int eng_norm_forward(EngPart* norm, EngCtx* ctx, const EngMat* x, const int* rows, int n_rows, int lazy,

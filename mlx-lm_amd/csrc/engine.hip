@@ -13,6 +13,7 @@
 #include "engine.h"
 #include "engine_parts.h"
 #include "attention_tiles.h"
+#include "decode_chain.h"
 
 #include <stdarg.h>
 #include <string.h>
@@ -161,6 +162,11 @@ static Entry<fn_attn_tile_terms> k_attn_tile_terms("attention", "attn_tile_terms
 static Entry<fn_attn_row_terms> k_attn_row_terms("attention", "attn_row_terms");
 static Entry<fn_attn_decode_terms> k_attn_decode_terms("attention_decode", "attn_decode_rows_terms");
 static Entry<fn_attn_prefill_terms> k_attn_prefill_terms("attention_prefill", "attn_prefill_terms");
+static Entry<int (*)(const ChainDims*, int)> k_chain_takes("decode_chain", "decode_chain_takes");
+static Entry<size_t (*)(const ChainDims*, int)> k_chain_bytes("decode_chain", "decode_chain_bytes");
+static Entry<int (*)(const ChainDims*, int, const void*, void*, const float*, float*, int, const int*, int, const int*, const int*, int,
+                     unsigned, hipStream_t)>
+    k_chain("decode_chain", "decode_chain");
 
 // Launch through an entry: a missing library or a refused call becomes this library's error.
 #define KERNEL(entry, ctx, ...)                                                                  \
@@ -1074,6 +1080,77 @@ struct Model : EngPart {
   Head* head;
   Model() : EngPart(KIND_MODEL) {}
 
+  // Whether the layers are alike and of the kind that one launch takes (decode_chain.h), over these cache slots;
+  // with `table`, the layers' pointers for it, in the schedule's order.
+  bool chain_of(const EngSlot* slots, int n_slots, ChainDims* d, std::vector<ChainLayer>* table) const {
+    *d = ChainDims{};
+    std::vector<char> seen(n_slots > 0 ? n_slots : 0, 0);
+    for (const Run& run : schedule) {
+      auto* block = dynamic_cast<PreNormBlock*>(layers[run.layer]);
+      if (!block || !run.writes || run.state >= 0 || run.cache < 0 || run.cache >= n_slots || seen[run.cache]) return false;
+      seen[run.cache] = 1;
+      auto* n1 = dynamic_cast<LayerNorm*>(block->mixer_norm);
+      auto* n2 = block->ffn ? dynamic_cast<LayerNorm*>(block->ffn_norm) : nullptr;
+      auto* at = dynamic_cast<Attention*>(block->mixer);
+      auto* mlp = block->ffn ? dynamic_cast<GeluMlp*>(block->ffn) : nullptr;
+      if (!n1 || !n2 || !at || !mlp || (at->position && at->position->rotates()) || at->window > 0) return false;
+      if (at->head_dim != CHAIN_HEAD_DIM || at->width != width || n1->width != width || n2->width != width || mlp->width != width) return false;
+      const EngSlot& s = slots[run.cache];
+      if (s.group < 0 || s.dtype != DT_BF16 || s.page_stride != s.v_page_stride || s.n_kv_heads != at->n_kv_heads ||
+          s.head_dim != CHAIN_HEAD_DIM || s.v_head_dim != CHAIN_HEAD_DIM || s.group != slots[schedule[0].cache].group)
+        return false;
+      const EngWeight* w[4] = {&at->qkv_w, &at->out_w, &mlp->fc_w, &mlp->proj_w};
+      const int n[4] = {at->q_width + 2 * at->kv_width, width, mlp->inner, width}, k[4] = {width, at->q_width, width, mlp->inner};
+      const float* b[4] = {at->qkv_b, at->out_b, mlp->fc_b, mlp->proj_b};
+      for (int i = 0; i < 4; ++i)
+        if (!w[i]->packed || w[i]->dtype != DT_BF16 || w[i]->N != n[i] || w[i]->K != k[i] || (uintptr_t)w[i]->packed % 16 || (uintptr_t)b[i] % 16)
+          return false;
+      for (const LayerNorm* n : {n1, n2})
+        if (!n->gamma || !n->beta || (uintptr_t)n->gamma % 16 || (uintptr_t)n->beta % 16) return false;
+      if ((uintptr_t)s.k % 16 || (uintptr_t)s.v % 16 || s.page_stride % 8) return false;
+      if (d->n_layers == 0) {
+        d->width = width, d->inner = mlp->inner, d->n_heads = at->n_heads, d->n_kv_heads = at->n_kv_heads;
+        d->page_size = s.page_size, d->page_stride = s.page_stride;
+        d->eps1 = n1->eps, d->eps2 = n2->eps, d->scale = at->scale;
+      } else if (d->inner != mlp->inner || d->n_heads != at->n_heads || d->n_kv_heads != at->n_kv_heads || d->page_size != s.page_size ||
+                 d->page_stride != s.page_stride || d->eps1 != n1->eps || d->eps2 != n2->eps || d->scale != at->scale) {
+        return false;
+      }
+      d->n_layers++;
+      if (table) {
+        ChainLayer t = {{w[0]->packed, w[1]->packed, w[2]->packed, w[3]->packed},
+                        {b[0], b[1], b[2], b[3]},
+                        {n1->gamma, n2->gamma},
+                        {n1->beta, n2->beta},
+                        s.k,
+                        s.v};
+        table->push_back(t);
+      }
+    }
+    return d->n_layers > 0;
+  }
+
+  // All layers of a step whose one or two requests bring a token each, as one launch; the stream after them
+  // lies in *out then.  At three rows its hand-overs, whose words every block reads, would cost what the launches do; a row's
+  // keys must fit the registers of the block that takes a head of it.
+  int chained(EngCtx* ctx, const EngMat& h, EngMat* out, bool* done) const {
+    *done = false;
+    const int rows = ctx->n_tokens;
+    if (!ctx->chain || rows < 1 || rows > CHAIN_MOST_ROWS || ctx->n_requests != rows || ctx->dtype != DT_BF16 || ctx->force_splits > 0 ||
+        !ctx->chain->memory[rows - 1])
+      return 0;
+    ChainDims d;
+    if (!chain_of(ctx->slots, ctx->n_slots, &d, nullptr)) return 0;
+    const Attention* at = static_cast<const Attention*>(static_cast<const PreNormBlock*>(layers[schedule[0].layer])->mixer);
+    if (ctx->counts[at->array_base + ARR_MAX_ROW_CONTEXT] - 1 > CHAIN_MOST_KEYS || ctx->counts[at->array_base + ARR_ROWS] != rows) return 0;
+    const int group = ctx->slots[schedule[0].cache].group;
+    TRY(take(ctx, rows, width, DT_F32, out));
+    KERNEL(k_chain, ctx, &d, rows, ctx->chain->layers, ctx->chain->memory[rows - 1], (const float*)h.p, (float*)out->p, width,
+           ctx->block_tables[group], ctx->table_width[group], ctx->token_req, ctx->positions, 0, 0u, ctx->stream);
+    *done = true;
+    return 0;
+  }
+
   int forward(EngCtx* ctx) {
     if (ctx->stats) ctx->stats->steps++;
     EngMat h;
@@ -1083,7 +1160,12 @@ struct Model : EngPart {
     if (positions) TRY(positions->embedding_term(ctx, &add, &add_index));
     TRY(embedding->forward(ctx, h, add, add_index));
     EngPending* pending = &ctx->pending;
+    EngMat after;
+    bool done = false;
+    TRY(chained(ctx, h, &after, &done));
+    if (done) h = after;
     for (const Run& run : schedule) {
+      if (done) break;
       Block* block = layers[run.layer];
       // a block that does not know of pending sums gets the stream with everything added
       pending->allowed = block->handles_pending;
@@ -1277,6 +1359,27 @@ extern "C" int eng_model_forward(EngPart* model, EngCtx* ctx) {
   return m ? m->forward(ctx) : 1;
 }
 
+extern "C" int eng_chain_sizes(EngPart* model, const EngSlot* slots, int n_slots, size_t* table_bytes, size_t* one_row, size_t* two_rows) {
+  Model* m = as<Model>(model, KIND_MODEL, "eng_chain_sizes");
+  ChainDims d;
+  if (!m || !m->chain_of(slots, n_slots, &d, nullptr)) return 0;
+  auto takes = k_chain_takes.get();
+  auto bytes = k_chain_bytes.get();
+  if (!takes || !bytes) return 0;
+  *table_bytes = sizeof(ChainLayer) * d.n_layers;
+  *one_row = takes(&d, 1) ? bytes(&d, 1) : 0, *two_rows = takes(&d, 2) ? bytes(&d, 2) : 0;
+  return *one_row || *two_rows;
+}
+
+extern "C" int eng_chain_table(EngPart* model, const EngSlot* slots, int n_slots, void* table) {
+  Model* m = as<Model>(model, KIND_MODEL, "eng_chain_table");
+  ChainDims d;
+  std::vector<ChainLayer> t;
+  if (!m || !m->chain_of(slots, n_slots, &d, &t)) FAIL("eng_chain_table: not a model that runs as one launch");
+  memcpy(table, t.data(), t.size() * sizeof(ChainLayer));
+  return 0;
+}
+
 extern "C" int eng_block_forward(EngPart* block, EngCtx* ctx, const EngMat* h, int cache_slot,
                                  int writes_cache, int state_slot) {
   Block* b = as<Block>(block, KIND_BLOCK, "eng_block_forward");
@@ -1376,7 +1479,7 @@ extern "C" int eng_read_ahead_pays(const EngCtx* ctx, const EngWeight* w, int n_
 extern "C" int eng_struct_sizes(long* out, int n) {
   const long sizes[] = {sizeof(EngMat),     sizeof(EngWeight), sizeof(EngValue), sizeof(EngPending),
                         sizeof(EngSlot),    sizeof(EngScratch), sizeof(EngStats), sizeof(EngCtx),
-                        sizeof(EngCall),    sizeof(EngScatter), sizeof(EngLinear),
+                        sizeof(EngCall),    sizeof(EngScatter), sizeof(EngLinear), sizeof(EngChain),
                         (long)offsetof(EngCtx, pending), (long)offsetof(EngCall, nbytes)};
   const int have = (int)(sizeof(sizes) / sizeof(sizes[0]));
   for (int i = 0; i < n && i < have; ++i) out[i] = sizes[i];

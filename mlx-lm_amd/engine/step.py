@@ -1,5 +1,6 @@
 """The step function: one batch of (request, its next tokens) through the model."""
 
+import ctypes
 from collections import OrderedDict
 from dataclasses import dataclass
 from typing import List, Sequence
@@ -75,6 +76,7 @@ class Engine:
         # decode steps are recorded as graphs where every part launches kernels only
         self.use_graphs = use_graphs and all(getattr(p, "graph_safe", False) for p in self.decoder.parts())
         self._graphs = {}
+        self._chain = None
         self._length_classers = None  # the parts that put recorded decode steps into classes of length
         # Other steps whose shape keeps coming back (portions of prompts of the scheduler's size, with
         # or without decoding requests beside them) are recorded too, if asked for.
@@ -107,6 +109,24 @@ class Engine:
         return table
 
     # -- buffers ---------------------------------------------------------------
+
+    def chain(self):
+        """What the one launch of a decode step of one or two rows needs (``EngChain``), made at the
+        first step: the table of the layers' pointers and the launch's own memory.  ``None`` where the
+        model's layers are not of the kind that it takes."""
+        if self._chain is None:
+            self._chain = False
+            L, model = native.lib(), self.decoder.native()
+            table_bytes, one, two = (ctypes.c_size_t() for _ in range(3))
+            n = len(self.slot_table)
+            if self.dtype == torch.bfloat16 and L.eng_chain_sizes(model, self.slot_table, n, table_bytes, one, two):
+                table = torch.empty(table_bytes.value, dtype=torch.uint8)
+                native.check(L.eng_chain_table(model, self.slot_table, n, table.data_ptr()), "the layers' table")
+                table = table.to(self.device)
+                memory = [torch.zeros(b.value, dtype=torch.uint8, device=self.device) if b.value else None for b in (one, two)]
+                self._chain = native.EngChain(native.ptr(table), (ctypes.c_void_p * 2)(*[native.ptr(m) for m in memory]))
+                self._chain_tensors = (table, memory)
+        return self._chain or None
 
     def logits_buffer(self, n_rows, vocab):
         if self._logits is None or self._logits.shape[0] < n_rows or self._logits.shape[1] != vocab:

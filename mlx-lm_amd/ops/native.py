@@ -65,6 +65,10 @@ class EngStats(Structure):
                 ("callbacks", c_long), ("steps", c_long), ("key_splits_most", c_long)]
 
 
+class EngChain(Structure):
+    _fields_ = [("layers", c_void_p), ("memory", c_void_p * 2)]
+
+
 class EngCtx(Structure):
     _fields_ = [
         ("stream", c_void_p), ("dtype", c_int), ("n_tokens", c_int), ("n_requests", c_int),
@@ -77,6 +81,7 @@ class EngCtx(Structure):
         ("scratch", POINTER(EngScratch)), ("split_ws", c_void_p), ("split_ws_floats", c_size_t),
         ("logits", c_void_p), ("logits_rows", c_long), ("pending", EngPending),
         ("read_ahead", POINTER(EngWeight)), ("stats", POINTER(EngStats)), ("py", c_void_p),
+        ("chain", POINTER(EngChain)),
     ]
 
 
@@ -162,6 +167,8 @@ def lib():
                                POINTER(c_int), POINTER(c_int), P, P]),
         "eng_free": (None, [P]),
         "eng_model_forward": (c_int, [P, POINTER(EngCtx)]),
+        "eng_chain_sizes": (c_int, [P, POINTER(EngSlot), c_int, POINTER(c_size_t), POINTER(c_size_t), POINTER(c_size_t)]),
+        "eng_chain_table": (c_int, [P, POINTER(EngSlot), c_int, P]),
         "eng_block_forward": (c_int, [P, POINTER(EngCtx), POINTER(EngMat), c_int, c_int, c_int]),
         "eng_norm_forward": (c_int, [P, POINTER(EngCtx), POINTER(EngMat), P, c_int, c_int, POINTER(EngWeight),
                                      POINTER(EngValue)]),
@@ -190,7 +197,7 @@ def lib():
         fn = getattr(L, name)
         fn.restype, fn.argtypes = res, args
     mirrored = [EngMat, EngWeight, EngValue, EngPending, EngSlot, EngScratch, EngStats, EngCtx, EngCall,
-                EngScatter, EngLinear]
+                EngScatter, EngLinear, EngChain]
     want = [ctypes.sizeof(t) for t in mirrored] + [EngCtx.pending.offset, EngCall.nbytes.offset]
     got = (c_long * len(want))()
     L.eng_struct_sizes.argtypes = [POINTER(c_long), c_int]

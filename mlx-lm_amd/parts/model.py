@@ -173,6 +173,8 @@ class DecoderModel:
         if ctx.n_wanted:
             logits = ctx.logits_out(ctx.n_wanted, self.vocab_size)
             ctx.c.logits, ctx.c.logits_rows = logits.data_ptr(), logits.shape[0]
+        chain = ctx.engine.chain()
+        ctx.c.chain = ctypes.pointer(chain) if chain is not None else None
         with ctx.enter():
             rc = native.lib().eng_model_forward(self.native(), ctypes.byref(ctx.c))
         native.check(rc, "the model's step")

@@ -1,0 +1,152 @@
+"""All layers of a decode step of one or two rows in one launch (csrc/decode_chain.hip) against the
+same layers in float64."""
+
+import ctypes
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+BF = torch.bfloat16
+_i, _vp = ctypes.c_int, ctypes.c_void_p
+
+
+class Dims(ctypes.Structure):
+    _fields_ = [(n, _i) for n in ("n_layers", "width", "inner", "n_heads", "n_kv_heads", "page_size")] + [
+        ("page_stride", ctypes.c_size_t), ("eps1", ctypes.c_float), ("eps2", ctypes.c_float), ("scale", ctypes.c_float)]
+
+
+class Layer(ctypes.Structure):
+    _fields_ = [("W", _vp * 4), ("bias", _vp * 4), ("gamma", _vp * 2), ("beta", _vp * 2), ("k", _vp), ("v", _vp)]
+
+
+def _lib():
+    from mlx_lm_amd.ops import build
+
+    lib = build.load("decode_chain")
+    lib.decode_chain_bytes.restype = ctypes.c_size_t
+    lib.mlxlm_last_error.restype = ctypes.c_char_p
+    return lib
+
+
+def _packed(w):
+    """[N, K] in tiles of 16 features x 64 k, in the order the lanes read them; features beyond N are zeros."""
+    n, k = w.shape
+    t = torch.zeros((n + 15) // 16 * 16, k, dtype=w.dtype, device=w.device)
+    t[:n] = w
+    return t.view(-1, 16, k // 64, 4, 2, 8).permute(0, 2, 4, 3, 1, 5).contiguous()
+
+
+# (layers, width, inner, heads, key heads, page size, keys before the step, blocks, patience):
+# one k-block, an odd number of them, the widest and longest that a wave holds; no key yet, a tile of keys less one, whole and
+# begun, the most keys; features a unit that do not divide the product's; query heads that share a key head; two rows
+# of very different lengths; and few blocks of little patience, which do each other's units (below four, nobody's own are
+# attention's)
+CASES = [
+    (2, 64, 64, 1, 1, 16, (0,), 0, 0),
+    (3, 64, 192, 2, 1, 8, (7, 8), 0, 0),
+    (2, 128, 256, 2, 2, 16, (9, 1024), 0, 0),
+    (2, 832, 3328, 13, 13, 16, (300,), 0, 0),
+    (2, 1600, 6400, 25, 25, 16, (700, 1001), 0, 0),
+    (2, 1600, 6400, 25, 25, 32, (1023,), 0, 0),
+    (1, 2048, 7168, 32, 8, 16, (64,), 0, 0),
+    (2, 768, 3072, 12, 12, 16, (93,), 3, 100),
+    (2, 192, 448, 3, 3, 16, (40, 3), 1, 10),
+    (2, 1280, 5120, 20, 20, 16, (100, 500), 100, 100),
+]
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: f"{c[1]}x{c[2]}-{'+'.join(map(str, c[6]))}{f'-{c[7]}blocks' if c[7] else ''}")
+def test_layers_of_a_decode_step_in_one_launch(case):
+    n_layers, D, I, H, HK, page, keys, blocks, patience = case
+    lib, R, Q, KV = _lib(), len(case[6]), case[3] * 64, case[4] * 64
+    g = torch.Generator().manual_seed(D + I + R)
+
+    def rand(*shape, std=1.0):
+        return (torch.randn(*shape, generator=g) * std).cuda()
+
+    width = max(keys) // page + 1
+    pages = torch.randperm(R * width, generator=g).to(torch.int32).view(R, width).cuda()
+    layers, held, table = [], [], (Layer * n_layers)()
+    for t in table:
+        shapes = ((Q + 2 * KV, D), (D, Q), (I, D), (D, I))
+        W, b = [rand(*s, std=s[1] ** -0.5).to(BF) for s in shapes], [rand(s[0], std=0.1) for s in shapes]
+        norms = [1 + rand(D, std=0.1), rand(D, std=0.1), 1 + rand(D, std=0.1), rand(D, std=0.1)]
+        kv = [rand(R * width, HK, page, 64).to(BF) for _ in range(2)]
+        packs = [_packed(w) for w in W]
+        held.append((packs, b, norms, kv))
+        layers.append((W, b, norms, [x.clone() for x in kv]))
+        t.W[:], t.bias[:] = [p.data_ptr() for p in packs], [x.data_ptr() for x in b]
+        t.gamma[:], t.beta[:] = [norms[0].data_ptr(), norms[2].data_ptr()], [norms[1].data_ptr(), norms[3].data_ptr()]
+        t.k, t.v = kv[0].data_ptr(), kv[1].data_ptr()
+    on_gpu = torch.frombuffer(bytearray(bytes(table)), dtype=torch.uint8).cuda()
+    d = Dims(n_layers, D, I, H, HK, page, HK * page * 64, 1e-5, 1e-5, 0.125)
+    assert lib.decode_chain_takes(ctypes.byref(d), R) == 1
+    memory = torch.zeros(lib.decode_chain_bytes(ctypes.byref(d), R), dtype=torch.uint8, device="cuda")
+    req = torch.arange(R, dtype=torch.int32, device="cuda")
+    pos = torch.tensor(keys, dtype=torch.int32, device="cuda")
+
+    def launch(h):
+        out = torch.full_like(h, float("nan"))
+        stream = _vp(torch.cuda.current_stream().cuda_stream)
+        p = [_vp(x.data_ptr()) for x in (on_gpu, memory, h, out, pages, req, pos)]
+        rc = lib.decode_chain(ctypes.byref(d), R, p[0], p[1], p[2], p[3], D, p[4], width, p[5], p[6], blocks, ctypes.c_uint(patience), stream)
+        assert rc == 0, lib.mlxlm_last_error().decode()
+        return out
+
+    def plain(h):
+        """The layers in 64 bits, and each layer's new keys and values."""
+        h, new = h.double(), []
+        for W, b, (g1, b1, g2, b2), (k_pages, v_pages) in layers:
+            def product(x, i):
+                return x @ W[i].double().T + b[i].double()
+
+            x = product(torch.nn.functional.layer_norm(h, (D,), g1.double(), b1.double(), 1e-5), 0)
+            o = []
+            for m, n in enumerate(keys):
+                k, v = ([p[pages[m].long()].permute(1, 0, 2, 3).reshape(HK, -1, 64)[:, :n].double() for p in (k_pages, v_pages)])
+                k = torch.cat([k, x[m, Q : Q + KV].view(HK, 1, 64)], 1).repeat_interleave(H // HK, 0)
+                v = torch.cat([v, x[m, Q + KV :].view(HK, 1, 64)], 1).repeat_interleave(H // HK, 0)
+                p = torch.softmax((k * x[m, :Q].view(H, 1, 64)).sum(-1) / 8, -1)
+                o.append((p.unsqueeze(-1) * v).sum(1).reshape(-1))
+            new.append(x[:, Q:])
+            h = h + product(torch.stack(o), 1)
+            h = h + product(torch.nn.functional.gelu(product(torch.nn.functional.layer_norm(h, (D,), g2.double(), b2.double(), 1e-5), 2), approximate="tanh"), 3)
+        return h, new
+
+    # Roundings to bfloat16 (2^-9 of a value) between a layer's products: the two norms' rows, q/k/v, the attention's rows,
+    # the activations.  Five a layer, each of what is then added to the stream, doubled for the step from each to the
+    # next through products whose rows are of one length: 5 x 2^-8 for all layers here, whose shares of the stream differ.
+    tol = 5 * 2.0**-8
+    runs = []
+    for turn in range(3):  # again on the same memory, with other rows, and the first rows once more
+        h = rand(R, D, std=2.0) if turn < 2 else first
+        first = h if turn == 0 else first
+        out = launch(h)
+        torch.cuda.synchronize()
+        want, new = plain(h)
+        assert ((out.double() - want).norm() / want.norm()).item() < tol, turn
+        for (_, _, _, kv), want_kv in zip(held, new):
+            for m, n in enumerate(keys):
+                at = pages[m, n // page].item()
+                got = torch.cat([kv[0][at, :, n % page].reshape(-1), kv[1][at, :, n % page].reshape(-1)]).double()
+                assert ((got - want_kv[m]).norm() / want_kv[m].norm()).item() < tol, (turn, m)
+        runs.append(out)
+    assert torch.equal(runs[0], runs[2])
+    # no other key or value was touched
+    for (_, _, _, kv), (_, _, _, before) in zip(held, layers):
+        for a, b in zip(kv, before):
+            for m, n in enumerate(keys):
+                a[pages[m, n // page].item(), :, n % page] = b[pages[m, n // page].item(), :, n % page]
+            assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("change", [dict(width=96), dict(width=2112), dict(inner=7232), dict(n_kv_heads=3), dict(n_layers=0), dict(rows=3)],
+                         ids=lambda c: next(iter(c)) + str(next(iter(c.values()))))
+def test_sizes_the_one_launch_does_not_take(change):
+    sizes = dict(n_layers=2, width=128, inner=256, n_heads=2, n_kv_heads=2, page_size=16, rows=1)
+    sizes.update(change)
+    rows = sizes.pop("rows")
+    d = Dims(*sizes.values(), 2048, 1e-5, 1e-5, 0.125)
+    assert _lib().decode_chain_takes(ctypes.byref(d), rows) == 0
