@@ -29,7 +29,9 @@
 #include "decode_chain.h"
 #include "lds_copy.h"
 
-#define CH_WAVES 8
+#define CH_WAVES 8         // waves that compute products
+#define CH_COPIERS 4       // waves that copy the next unit's weights meanwhile
+#define CH_ALL_WAVES (CH_WAVES + CH_COPIERS)  // (attention is everybody's)
 #define CH_LN_BLOCKS 4     // k-blocks (64) a wave of a normed product holds: K <= 2,048
 #define CH_PAIRS 7         // pairs of k-blocks a wave of the other products holds: K <= 7,168
 #define CH_TILES 2         // tiles of 16 features a unit of a normed product has at most
@@ -38,7 +40,7 @@
 #define CH_COPY_MOST (CH_PAIRS * CH_WAVES * 128)
 #define CH_HEAD CHAIN_HEAD_DIM
 #define CH_TAGS_A_STEP 0x10000u  // more than a step has products
-#define CH_KEY_TILES (CHAIN_MOST_KEYS / (CH_WAVES * 8))  // loads of 8 keys a wave holds
+#define CH_KEY_TILES ((CHAIN_MOST_KEYS + CH_ALL_WAVES * 8 - 1) / (CH_ALL_WAVES * 8))  // loads of 8 keys a wave holds
 
 #define CH_LDS_MOST (160 * 1024)
 #define CH_PATIENCE 20000  // 200 us: ten times what a layer's longest wait is
@@ -97,16 +99,18 @@ template <int MOST, typename F>
 __device__ __forceinline__ int words_wait(word_t (&w)[MOST], int n, uint32_t tag, uint32_t patience, F load) {
   uint64_t since = 0;
   for (;;) {
+    // (a word that this wave does not have counts as there: nothing is then carried from one round to the next in registers)
 #pragma unroll
-    for (int i = 0; i < MOST; ++i)
+    for (int i = 0; i < MOST; ++i) {
+      w[i] = (word_t)tag << 32;
       if (i < n) w[i] = load(i);
+    }
     bool there = true, late = false;
 #pragma unroll
-    for (int i = 0; i < MOST; ++i)
-      if (i < n) {
-        there = there && tag_of(w[i]) == tag;
-        late = late || tag_of(w[i]) - tag - 1u < CH_TAGS_A_STEP;
-      }
+    for (int i = 0; i < MOST; ++i) {
+      there = there && tag_of(w[i]) == tag;
+      late = late || tag_of(w[i]) - tag - 1u < CH_TAGS_A_STEP;
+    }
     if (__all(there)) return CH_THERE;
     if (__any(late)) return CH_LATE;
     const uint64_t now = wall_clock64();
@@ -119,8 +123,9 @@ __device__ __forceinline__ int words_wait(word_t (&w)[MOST], int n, uint32_t tag
 __device__ __forceinline__ int ceil_of(int a, int b) { return (a + b - 1) / b; }
 
 // What a product's unit reads that no unit of the step makes (weights, bias, the norm's scale and shift) comes
-// into LDS by copies of 1 KB: a wave copies what it reads itself.  Fragment h of tile t and k-block c of a normed
-// product lies at ((t * k-blocks + c) * 2 + h) KB, half h of pair c of a plain one at (c * 2 + h) KB.
+// into LDS by copies of 1 KB, dealt to the copying waves.  Fragment h of tile t and k-block c of a normed
+// product lies at ((t * k-blocks + c) * 2 + h) KB, half h of pair c of a plain one at (c * 2 + h) KB; scale and shift lie as
+// the computing waves read them, each its own k-blocks'.
 // (the table of layers is read by scalar loads: nothing writes it during a launch)
 typedef const __attribute__((address_space(4))) ChainLayer* layer_ptr;
 __device__ __forceinline__ layer_ptr layer_of(const ChainArgs& p, int layer) { return (layer_ptr)(uintptr_t)(p.layers + layer); }
@@ -141,22 +146,22 @@ __device__ __forceinline__ ChainUnit unit_of(const ChainArgs& p, int ph, int uni
   x.ly = layer_of(p, ph / CH_KINDS);
   return x;
 }
-__device__ __forceinline__ void copy_unit(const ChainArgs& p, const ChainUnit& x, uint32_t lds, uint32_t lds_small, int lane, int wave) {
+__device__ __forceinline__ void copy_unit(const ChainArgs& p, const ChainUnit& x, uint32_t lds, uint32_t lds_small, int lane, int copier) {
   const int g = lane >> 4;
   const ChainSize& z = p.size[x.kind];
-  const i32x4_t from = copy_buffer((const uint16_t*)x.ly->W[x.which], (size_t)((z.N + 15) / 16) * x.kblocks * 2048);
-  if (x.normed) {
-    const int k = (wave + CH_WAVES * (lane >> 4)) * 64 + (lane & 15) * 4;
-    const uint32_t at = k < z.K ? k * 4 : COPY_NOTHING;
-    copy16_to_lds(copy_buffer(x.ly->gamma[x.kind == CH_FC], (size_t)z.K * 4), at, 0, lds_small + wave * 2048);
-    copy16_to_lds(copy_buffer(x.ly->beta[x.kind == CH_FC], (size_t)z.K * 4), at, 0, lds_small + wave * 2048 + 1024);
-  }
-  if (wave == 0 && x.ly->bias[x.which])
+  const i32x4_t from = copy_buffer(x.ly->W[x.which], (size_t)((z.N + 15) / 16) * x.kblocks * 2048);
+  if (copier == 0 && x.ly->bias[x.which])
     copy16_to_lds(copy_buffer(x.ly->bias[x.which], (size_t)z.N * 4), lane < 8 && x.n0 + lane * 4 < z.N ? (x.n0 + lane * 4) * 4 : COPY_NOTHING, 0,
                   lds_small + CH_WAVES * 2048);
   if (x.normed) {
-    for (int b = 0; b < x.n_blocks; ++b) {
-      const int c = wave + CH_WAVES * b;
+    const i32x4_t gamma = copy_buffer(x.ly->gamma[x.kind == CH_FC], (size_t)z.K * 4), beta = copy_buffer(x.ly->beta[x.kind == CH_FC], (size_t)z.K * 4);
+    for (int v = copier; v < CH_WAVES; v += CH_COPIERS) {
+      const int k = (v + CH_WAVES * (lane >> 4)) * 64 + (lane & 15) * 4;
+      const uint32_t at = k < z.K ? k * 4 : COPY_NOTHING;
+      copy16_to_lds(gamma, at, 0, lds_small + v * 2048);
+      copy16_to_lds(beta, at, 0, lds_small + v * 2048 + 1024);
+    }
+    for (int c = copier; c < x.kblocks; c += CH_COPIERS)
 #pragma unroll
       for (int t = 0; t < CH_TILES; ++t)
         if (x.n0 + t * 16 < x.n_end) {
@@ -165,20 +170,30 @@ __device__ __forceinline__ void copy_unit(const ChainArgs& p, const ChainUnit& x
           copy16_to_lds(from, at, c * 2048, lds + (t * x.kblocks + c) * 2048);
           copy16_to_lds(from, at, c * 2048 + 1024, lds + (t * x.kblocks + c) * 2048 + 1024);
         }
-    }
   } else {
     // 8 features; a matrix instruction takes them at two k-blocks at once (rows 0 to 7 of the
     // weights and of the rows' columns the first, 8 to 15 the second; the products of one's
     // weights with the other's rows are not used)
     const int n = x.n0 + (lane & 7);
     const uint32_t at = (uint32_t)(n >> 4) * x.kblocks * 2048 + (g * 16 + (n & 15)) * 16, second = (lane >> 3) & 1;
-    for (int b = 0; b < x.n_pairs; ++b) {
-      const int pair = wave + CH_WAVES * b;
+    for (int pair = copier; pair < x.pairs; pair += CH_COPIERS) {
       const uint32_t at2 = !second ? at : 2 * pair + 1 < x.kblocks ? at + 2048 : COPY_NOTHING;  // (no second k-block: zeros)
       copy16_to_lds(from, at2, pair * 4096, lds + pair * 2048);
       copy16_to_lds(from, at2, pair * 4096 + 1024, lds + pair * 2048 + 1024);
     }
   }
+}
+
+// A barrier of the computing waves alone (the copying ones are held up by their copies): `arrived` counts, `target`
+// is a wave's own.
+__device__ __forceinline__ void meet(uint32_t* arrived, uint32_t& target, int lane) {
+  target += CH_WAVES;
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  if (lane == 0) atomicAdd(arrived, 1u);
+  while ((int)(*(volatile uint32_t*)arrived - target) < 0) {
+  }
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
 }
 
 // Sum (largest) over the lanes that hold the same eighth (lane % 8) of different keys.
@@ -199,10 +214,15 @@ struct ChainShared {
   float red[CH_TILES][CH_WAVES][2 * R * 16];
   __attribute__((aligned(16))) float small[CH_WAVES * 2 + 1][256];  // the norm's scale and shift, a wave's own share; the bias
   __attribute__((aligned(16))) float4 stat[R][CH_WAVES];
-  __attribute__((aligned(16))) float part[CH_WAVES][CH_HEAD];
-  float part_m[CH_WAVES], part_l[CH_WAVES];
-  int how[CH_WAVES];
+  __attribute__((aligned(16))) float part[CH_ALL_WAVES][CH_HEAD];
+  float part_m[16], part_l[16];
+  int how[CH_ALL_WAVES];
   int missing;
+  // what the block does next, for all waves: phase (-1: no more) and unit, whether its weights are in LDS, and the unit after it
+  struct {
+    int ph, unit, held, then_ph, then_unit;
+  } plan;
+  uint32_t arrived;
 };
 
 // One unit of attention: a row's head.  Old keys lie in the pages and are asked for before the step's query
@@ -215,7 +235,7 @@ __device__ __forceinline__ int chain_attention(const ChainArgs& p, ChainShared<R
   const int pos = p.positions[m];
   const int* table = p.block_table + (size_t)p.token_req[m] * p.max_blocks;
   const int tiles = ceil_of(pos, 8), e = lane & 7;
-  // a lane holds 8 of a key's 64 elements, a load 8 keys; wave w takes tiles w, w + 8, ...
+  // a lane holds 8 of a key's 64 elements, a load 8 keys; wave w takes tiles w, w + 12, ...
   const auto place = [&](int key) {
     return (size_t)table[key / p.page_size] * p.page_stride + ((size_t)kvh * p.page_size + key % p.page_size) * CH_HEAD + e * 8;
   };
@@ -225,8 +245,8 @@ __device__ __forceinline__ int chain_attention(const ChainArgs& p, ChainShared<R
   for (int t = 0; t < CH_KEY_TILES; ++t) k[t] = v[t] = (ChFrag)(0u), sc[t] = -INFINITY;
 #pragma unroll
   for (int t = 0; t < CH_KEY_TILES; ++t) {
-    if (t * CH_WAVES + wave >= tiles) break;
-    const size_t at = place(min((t * CH_WAVES + wave) * 8 + (lane >> 3), pos - 1));
+    if (t * CH_ALL_WAVES + wave >= tiles) break;
+    const size_t at = place(min((t * CH_ALL_WAVES + wave) * 8 + (lane >> 3), pos - 1));
     k[t] = *(const ChFrag*)((const uint16_t*)ly->k_pages + at), v[t] = *(const ChFrag*)((const uint16_t*)ly->v_pages + at);
   }
   asm volatile("" ::: "memory");
@@ -234,7 +254,7 @@ __device__ __forceinline__ int chain_attention(const ChainArgs& p, ChainShared<R
 
   const word_t* row = p.qkv + (size_t)m * (p.size[CH_QKV].N >> 1);
   word_t in[12];
-  const bool own = wave == CH_WAVES - 1;  // the wave that takes the step's own key
+  const bool own = wave == CH_ALL_WAVES - 1;  // the wave that takes the step's own key
   const int how = words_wait(in, own ? 12 : 4, tag - 1, patience, [&](int i) {
     const int first = i < 4 ? h * CH_HEAD : p.q_width + (i >= 8 ? p.kv_width : 0) + kvh * CH_HEAD;
     return word_load(row + ((first + e * 8) >> 1) + (i & 3));
@@ -257,9 +277,9 @@ __device__ __forceinline__ int chain_attention(const ChainArgs& p, ChainShared<R
   };
 #pragma unroll
   for (int t = 0; t < CH_KEY_TILES; ++t) {
-    if (t * CH_WAVES + wave >= tiles) break;
+    if (t * CH_ALL_WAVES + wave >= tiles) break;
     const float s = score(k[t][0], k[t][1], k[t][2], k[t][3]);
-    sc[t] = (t * CH_WAVES + wave) * 8 + (lane >> 3) < pos ? s : -INFINITY;
+    sc[t] = (t * CH_ALL_WAVES + wave) * 8 + (lane >> 3) < pos ? s : -INFINITY;
     top = fmaxf(top, sc[t]);
   }
   if (own) {
@@ -274,14 +294,14 @@ __device__ __forceinline__ int chain_attention(const ChainArgs& p, ChainShared<R
   const float base = top == -INFINITY ? 0.f : top;  // (a wave without keys)
 #pragma unroll
   for (int t = 0; t < CH_KEY_TILES; ++t) {
-    if (t * CH_WAVES + wave >= tiles) break;
+    if (t * CH_ALL_WAVES + wave >= tiles) break;
     const float w = __builtin_amdgcn_exp2f(sc[t] - base);
-      l += w;
+    l += w;
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        o[2 * j] = __builtin_fmaf(w, __uint_as_float(v[t][j] << 16), o[2 * j]);
-        o[2 * j + 1] = __builtin_fmaf(w, __uint_as_float(v[t][j] & 0xffff0000u), o[2 * j + 1]);
-      }
+    for (int j = 0; j < 4; ++j) {
+      o[2 * j] = __builtin_fmaf(w, __uint_as_float(v[t][j] << 16), o[2 * j]);
+      o[2 * j + 1] = __builtin_fmaf(w, __uint_as_float(v[t][j] & 0xffff0000u), o[2 * j + 1]);
+    }
   }
   if (own && lane < 8) {
     const float w = __builtin_amdgcn_exp2f(mine - base);
@@ -303,15 +323,16 @@ __device__ __forceinline__ int chain_attention(const ChainArgs& p, ChainShared<R
   __syncthreads();
   int worst = 0;
 #pragma unroll
-  for (int w = 0; w < CH_WAVES; ++w) worst |= sh.how[w];
+  for (int w = 0; w < CH_ALL_WAVES; ++w) worst |= sh.how[w];
   worst = __builtin_amdgcn_readfirstlane(worst);
   if (wave == 0 && worst == CH_THERE) {
-    const float m_w = sh.part_m[e], best = group_max<8>(m_w);
+    const int w16 = lane & 15;
+    const float m_w = w16 < CH_ALL_WAVES ? sh.part_m[w16] : -INFINITY, best = group_max<16>(m_w);
     const float f = m_w == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_w - best);
-    const float inv = 1.0f / group_sum<8>(f * sh.part_l[e]);
+    const float inv = 1.0f / group_sum<16>(f == 0.f ? 0.f : f * sh.part_l[w16]);
     float out = 0.f;
 #pragma unroll
-    for (int w = 0; w < CH_WAVES; ++w) out = __builtin_fmaf(lane_value(f, w), sh.part[w][lane], out);
+    for (int w = 0; w < CH_ALL_WAVES; ++w) out = __builtin_fmaf(lane_value(f, w), sh.part[w][lane], out);
     out *= inv;
     const float next = dpp_move<DPP_QUAD_SWAP1>(out);
     if ((lane & 1) == 0) word_store(p.att + (((size_t)m * p.q_width + h * CH_HEAD + lane) >> 1), pack_bf16x2(out, next), tag);
@@ -325,7 +346,7 @@ __device__ __forceinline__ int chain_attention(const ChainArgs& p, ChainShared<R
 }
 
 template <int R>
-__global__ __launch_bounds__(CH_WAVES * 64, 2) void decode_chain_kernel(ChainArgs p) {
+__global__ __launch_bounds__(CH_ALL_WAVES * 64, 3) void decode_chain_kernel(ChainArgs p) {
   __shared__ ChainShared<R> sh;
   extern __shared__ __attribute__((aligned(16))) char held_weights[];
   const uint32_t lds = lds_address(held_weights), lds_small = lds_address(sh.small);
@@ -339,51 +360,70 @@ __global__ __launch_bounds__(CH_WAVES * 64, 2) void decode_chain_kernel(ChainArg
   const int stride = attends ? p.attention_blocks : p.product_blocks;
   int i = attends ? CH_ATTN : CH_QKV, u = start;
   int help_i = -1, help_u = 0;  // a missing unit done in its stead
+  uint32_t target = 0;  // of the computing waves' own barrier
+  if (threadIdx.x == 0) sh.arrived = 0;
   for (;;) {
     // (made anew for every unit: what is computed from them would otherwise be kept in registers over the loop, 50 of them)
     int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     asm volatile("" : "+v"(lane), "+s"(wave));
-    while (i < n_phases && u >= p.size[i % CH_KINDS].units) u = start, i += attends ? CH_KINDS : i % CH_KINDS == CH_QKV ? 2 : 1;
-    if (i >= n_phases) break;
-    const int ph = help_i >= 0 ? help_i : i, unit = help_i >= 0 ? help_u : u;
+    const bool copies = wave >= CH_WAVES;
+    if (wave == 0) {
+      const auto settle = [&](int& at_i, int& at_u) {  // to the next phase that has a unit of this block's
+        while (at_i < n_phases && at_u >= p.size[at_i % CH_KINDS].units)
+          at_u = start, at_i += attends ? CH_KINDS : at_i % CH_KINDS == CH_QKV ? 2 : 1;
+      };
+      settle(i, u);
+      int then_i = i, then_u = u;
+      if (help_i < 0) then_u += stride, settle(then_i, then_u);
+      if (lane == 0) {
+        sh.plan.ph = i >= n_phases ? -1 : help_i >= 0 ? help_i : i, sh.plan.unit = help_i >= 0 ? help_u : u, sh.plan.held = held;
+        sh.plan.then_ph = !attends && then_i < n_phases ? then_i : -1, sh.plan.then_unit = then_u;
+      }
+      held = !attends && then_i < n_phases;
+    }
+    if (copies) copies_arrived<0>();
+    __syncthreads();
+    const int ph = __builtin_amdgcn_readfirstlane(sh.plan.ph), unit = __builtin_amdgcn_readfirstlane(sh.plan.unit);
+    const int then_ph = __builtin_amdgcn_readfirstlane(sh.plan.then_ph), then_unit = __builtin_amdgcn_readfirstlane(sh.plan.then_unit);
+    const bool in_lds = __builtin_amdgcn_readfirstlane(sh.plan.held) != 0;
+    if (ph < 0) break;
     const int kind = ph % CH_KINDS, layer = ph / CH_KINDS;
     const uint32_t tag = tag_base + ph;
     int worst;
     if (kind == CH_ATTN) {
       worst = chain_attention<R>(p, sh, layer, unit, tag, patience, lane, wave);
       __syncthreads();
+      if (wave == 0) held = false;
+      if (copies) continue;
     } else {
+      if (!in_lds) {
+        if (copies) {
+          copy_unit(p, unit_of(p, ph, unit, wave), lds, lds_small, lane, wave - CH_WAVES);
+          copies_arrived<0>();
+        }
+        __syncthreads();
+      }
+      if (copies) {
+        __syncthreads();  // (the computing waves have read what lies in LDS)
+        if (then_ph >= 0) copy_unit(p, unit_of(p, then_ph, then_unit, wave), lds, lds_small, lane, wave - CH_WAVES);
+        continue;
+      }
       const ChainUnit at_hand = unit_of(p, ph, unit, wave);
-      const layer_ptr ly = at_hand.ly;
       const ChainSize& z = p.size[kind];
       const bool normed = at_hand.normed, first = ph == 0, last = ph == n_phases - 1;
       const int g = lane >> 4, kblocks = at_hand.kblocks, pairs = at_hand.pairs, n_blocks = at_hand.n_blocks, n_pairs = at_hand.n_pairs;
       const int n0 = at_hand.n0, n_end = at_hand.n_end;
       const bool odd = kblocks & 1;  // the last pair has no second k-block: its lanes repeat the first, and count as zeros
       const bool short_pair = odd && n_pairs > 0 && wave + CH_WAVES * (n_pairs - 1) == pairs - 1;
-      // the block's unit after this one
-      int then_i = i, then_u = u;
-      if (help_i < 0) {
-        then_u += stride;
-        while (then_i < n_phases && then_u >= p.size[then_i % CH_KINDS].units)
-          then_u = start, then_i += attends ? CH_KINDS : then_i % CH_KINDS == CH_QKV ? 2 : 1;
-      }
-      const bool ahead = !attends && then_i < n_phases;
 
-      // ---- what needs nobody ------------------------------------------------------------------
-      copies_arrived<0>();
-      if (!held) {
-        copy_unit(p, at_hand, lds, lds_small, lane, wave);
-        copies_arrived<0>();
-      }
-      held = ahead;
+      // ---- what the copying waves brought ---------------------------------------------------------
       // wave 0 writes the outputs: one feature a lane into the stream, else two neighbours a lane
       const int o_m = normed ? lane >> 4 : lane >> 3;
       const int o_f = normed ? (lane & 15) * 2 : lane & 7;
       const bool mine = wave == 0 && o_m < R && n0 + o_f < n_end;
       float2 bias = make_float2(0.f, 0.f);
       float old = 0.f;
-      if (wave == 0 && ly->bias[at_hand.which]) bias.x = sh.small[CH_WAVES * 2][o_f], bias.y = sh.small[CH_WAVES * 2][o_f + 1];
+      if (wave == 0 && at_hand.ly->bias[at_hand.which]) bias.x = sh.small[CH_WAVES * 2][o_f], bias.y = sh.small[CH_WAVES * 2][o_f + 1];
       float gm[CH_LN_BLOCKS], bt[CH_LN_BLOCKS];
 #pragma unroll
       for (int b = 0; b < CH_LN_BLOCKS; ++b) gm[b] = sh.small[wave * 2][b * 64 + lane], bt[b] = sh.small[wave * 2 + 1][b * 64 + lane];
@@ -412,10 +452,7 @@ __global__ __launch_bounds__(CH_WAVES * 64, 2) void decode_chain_kernel(ChainArg
       }
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       __builtin_amdgcn_sched_barrier(0);
-      // The block's next weights, all of them, ahead of the wait for this unit's rows.  (The barrier: what one wave copies
-      // for the next unit may lie where another has just read.)
-      ring_barrier();
-      if (ahead) copy_unit(p, unit_of(p, then_i, then_u, wave), lds, lds_small, lane, wave);
+      __syncthreads();  // the copying waves go on with the next unit's
 
       // ---- the rows, and the products ----------------------------------------------------------
       int how = CH_THERE;
@@ -432,9 +469,9 @@ __global__ __launch_bounds__(CH_WAVES * 64, 2) void decode_chain_kernel(ChainArg
               x[r][b] = b < n_blocks ? p.h[(size_t)r * p.ldh + (wave + CH_WAVES * b) * 64 + lane] : 0.f;
         } else {
           word_t in[R * CH_LN_BLOCKS];
-          const word_t* from = (kind == CH_QKV ? p.h2 : p.h1) + wave * 64 + lane;
+          const word_t* from = (kind == CH_QKV ? p.h2 : p.h1) + wave * 64;
           how |= words_wait(in, n_blocks * R, tag - 1, patience, [&](int j) {  // (word j: row j % R of block j / R)
-            return word_load(from + (size_t)(j % R) * z.K + (j / R) * (CH_WAVES * 64));
+            return word_load(from + ((j % R) * z.K + (j / R) * (CH_WAVES * 64)) + (uint32_t)lane);
           });
 #pragma unroll
           for (int r = 0; r < R; ++r)
@@ -459,7 +496,7 @@ __global__ __launch_bounds__(CH_WAVES * 64, 2) void decode_chain_kernel(ChainArg
           qq = wave_sum(qq);
           if (lane == 0) sh.stat[r][wave] = make_float4(s, wmean, qq, (float)(n_blocks * 64));
         }
-        __syncthreads();
+        meet(&sh.arrived, target, lane);
         const float inv_k = 1.0f / (float)z.K;
 #pragma unroll
         for (int r = 0; r < R; ++r) {
@@ -493,12 +530,12 @@ __global__ __launch_bounds__(CH_WAVES * 64, 2) void decode_chain_kernel(ChainArg
         // tag is made this one); then word j: row (j - 1) % R of pair (j - 1) / R
         const int whole = short_pair && lane >= 32 ? n_pairs - 1 : n_pairs;  // pairs that this lane's words exist of
         word_t in[R * CH_PAIRS + 1];
-        const word_t* from = (kind == CH_OUT ? p.att : p.act) + wave * 64 + lane;
+        const word_t* from = (kind == CH_OUT ? p.att : p.act) + wave * 64;
         const bool from_rows = kind == CH_OUT && layer == 0;
         const size_t old_at = (size_t)min(o_m, R - 1) * z.N + min(n0 + o_f, z.N - 1);
         if (wave == 0 && from_rows) old = p.h[(size_t)min(o_m, R - 1) * p.ldh + min(n0 + o_f, z.N - 1)];
         how |= words_wait(in, whole * R + 1, tag - 1, patience, [&](int j) {
-          if (j > 0) return word_load(from + (size_t)((j - 1) % R) * (z.K >> 1) + ((j - 1) / R) * (CH_WAVES * 64));
+          if (j > 0) return word_load(from + ((j - 1) % R * (z.K >> 1) + (j - 1) / R * (CH_WAVES * 64)) + (uint32_t)lane);
           if (wave != 0 || from_rows) return (word_t)(tag - 1) << 32;
           return kind == CH_OUT ? word_load(p.h2 + old_at) + ((word_t)2 << 32) : word_load(p.h1 + old_at) + ((word_t)1 << 32);
         });
@@ -532,7 +569,7 @@ __global__ __launch_bounds__(CH_WAVES * 64, 2) void decode_chain_kernel(ChainArg
 #pragma unroll
             for (int r = 0; r < 4; ++r) sh.red[t][wave][((lane >> 3 & 1) * R + (lane & 7)) * 16 + 4 * g + r] = acc[t][r];
       if (lane == 0) sh.how[wave] = how;
-      __syncthreads();
+      meet(&sh.arrived, target, lane);
       worst = 0;
 #pragma unroll
       for (int v = 0; v < CH_WAVES; ++v) worst |= sh.how[v];
@@ -557,15 +594,11 @@ __global__ __launch_bounds__(CH_WAVES * 64, 2) void decode_chain_kernel(ChainArg
           word_store((kind == CH_FC ? p.act : p.qkv) + (((size_t)o_m * z.N + n) >> 1), pack_bf16x2(v0, v1), tag);
         }
       }
-      // (the next unit's weights are asked for only once the outputs are on their way: in the other order
-      // these wait behind them)
-      __syncthreads();
     }
     if (worst != CH_MISSING) {
-      // (a block that helped has its own unit's weights to ask for again)
-      if (help_i >= 0) held = false;
-      // (done, or somebody else's so long ago that later words lie in its place)
-      if (help_i < 0) u += stride;
+      // (done, or somebody else's so long ago that later words lie in its place; a block that helped has its own unit's
+      // weights to ask for again)
+      if (help_i < 0) u += stride; else held = false;
       help_i = -1;
       continue;
     }
@@ -582,21 +615,20 @@ __global__ __launch_bounds__(CH_WAVES * 64, 2) void decode_chain_kernel(ChainArg
       const word_t* words = qk == CH_QKV ? p.qkv : qk == CH_ATTN ? p.att : qk == CH_OUT ? p.h1 : qk == CH_FC ? p.act : p.h2;
       const int turn = (int)(blockIdx.x % (unsigned)zq.units);
       if (threadIdx.x == 0) sh.missing = 0x7fffffff;
-      __syncthreads();
+      meet(&sh.arrived, target, lane);
       for (int j = threadIdx.x; j < per * R; j += CH_WAVES * 64) {
         const uint32_t off = tag_of(word_load(words + j)) - (tag_base + q);
         if (off < CH_TAGS_A_STEP) continue;
         const int of = qk == CH_ATTN ? (j / per) * p.n_heads + (j % per) * 2 / CH_HEAD : (j % per) * (pairs_of ? 2 : 1) / zq.features;
         atomicMin(&sh.missing, (of - turn + zq.units) % zq.units);
       }
-      __syncthreads();
+      meet(&sh.arrived, target, lane);
       const int found = __builtin_amdgcn_readfirstlane(sh.missing);
-      __syncthreads();
+      meet(&sh.arrived, target, lane);
       if (found == 0x7fffffff) break;
       help_i = q, help_u = (found + turn) % zq.units;
     }
   }
-  copies_arrived<0>();
 }
 
 // (a launch of its own ahead of the step's: no block may see the tag change)
@@ -702,9 +734,9 @@ extern "C" int decode_chain(const ChainDims* d, int rows, const void* layers, vo
   hipLaunchKernelGGL(chain_step_kernel, dim3(1), dim3(1), 0, stream, (uint32_t*)memory, (uint32_t)(d->n_layers * CH_KINDS + 1));
   CHECK_LAUNCH("decode_chain");
   if (rows == 1)
-    hipLaunchKernelGGL(decode_chain_kernel<1>, dim3(deal.blocks), dim3(CH_WAVES * 64), deal.lds, stream, a);
+    hipLaunchKernelGGL(decode_chain_kernel<1>, dim3(deal.blocks), dim3(CH_ALL_WAVES * 64), deal.lds, stream, a);
   else
-    hipLaunchKernelGGL(decode_chain_kernel<2>, dim3(deal.blocks), dim3(CH_WAVES * 64), deal.lds, stream, a);
+    hipLaunchKernelGGL(decode_chain_kernel<2>, dim3(deal.blocks), dim3(CH_ALL_WAVES * 64), deal.lds, stream, a);
   CHECK_LAUNCH("decode_chain");
   return 0;
 }
