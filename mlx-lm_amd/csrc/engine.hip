@@ -82,7 +82,8 @@ typedef int (*fn_embed)(void*, const void*, const int*, const void*, const int*,
 typedef int (*fn_layernorm)(void*, const float*, const int*, const float*, const float*, float, int, int, int,
                             hipStream_t);
 typedef int (*fn_gemm_f32)(void*, const void*, const void*, const float*, int, int, int, int, int, int, int,
-                           int, int, float*, size_t, hipStream_t);
+                           int, int, float*, size_t, void*, void*, size_t, const int*, int, const int*, const int*, int, int,
+                           int, int, hipStream_t);
 typedef int (*fn_gemm_bf16)(void*, const void*, const void*, const float*, int, int, int, int, int, int, int,
                             int, int, float*, size_t, void*, void*, size_t, const int*, int, const int*,
                             const int*, int, int, int, int, hipStream_t);
@@ -138,7 +139,8 @@ typedef int (*fn_attn_prefill_terms)(void*, const void*, int, int, const void*, 
 static Entry<fn_embed> k_embed("embed", "embed_scale_add");
 static Entry<fn_layernorm> k_layernorm("norm", "layernorm");
 static Entry<int (*)(void*, const float*, int, const int*, const float*, float, int, int, int, hipStream_t)> k_rmsnorm("rmsnorm", "rmsnorm");
-static Entry<fn_gemm_f32> k_gemm_f32("gemm_f32", "gemm_f32");
+static Entry<fn_gemm_f32> k_gemm_f32("gemm_f32", "gemm_f32_scatter");
+static Entry<int (*)(int, int)> k_gemm_f32_scatters("gemm_f32", "gemm_f32_scatters");
 static Entry<fn_int5> k_gemm_f32_splits("gemm_f32", "gemm_f32_splits");
 static Entry<fn_gemm_bf16> k_gemm_bf16("gemm_bf16", "gemm_bf16_scatter");
 static Entry<fn_int5> k_gemm_bf16_splits("gemm_bf16", "gemm_bf16_splits");
@@ -533,9 +535,16 @@ static int linear(EngCtx* ctx, const EngMat& out, const EngValue& a, const EngWe
       if (n_splits < 1) n_splits = 1;
       if (n_splits > 1 && pending) TRY(settle(ctx, pending));  // the workspace is about to be written again
     }
+    // (few rows' keys and values go to their pages from the product's own epilogue, others from the finished rows, below)
+    int scatters = 0;
+    if (sc && (variant == 0 || variant == 3)) QUERY(k_gemm_f32_scatters, scatters, M, n_splits);
+    const EngScatter* own = scatters ? sc : nullptr;
     KERNEL(k_gemm_f32, ctx, out.p, A.p, w.w, bias, M, N, K, A.ld, w.ldw, out.ld, flags, variant, n_splits,
-           n_splits > 1 ? ws : nullptr, n_splits > 1 ? ws_floats : (size_t)0, ctx->stream);
-    // (keys and values go to their pages from the finished rows, below)
+           n_splits > 1 ? ws : nullptr, n_splits > 1 ? ws_floats : (size_t)0, own ? own->k : nullptr, own ? own->v : nullptr,
+           own ? own->page_stride : (size_t)0, own ? own->block_table : nullptr, own ? own->max_blocks : 0,
+           own ? own->token_req : nullptr, own ? own->positions : nullptr, own ? own->q_width : 0, own ? own->kv_width : 0,
+           own ? own->head_dim : 0, own ? own->page_size : 0, ctx->stream);
+    if (own) return 0;
     if (n_splits > 1) TRY(finish_parts(ctx, out, ws, n_splits, bias, gelu, accumulate, nullptr, pending));
   } else {
     // Few rows give the tile kernel few tiles: K is split then as for the decode kernels,

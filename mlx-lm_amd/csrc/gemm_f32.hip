@@ -31,7 +31,24 @@ struct GemmArgs {
   // in ws[y][ws_rows][N], without bias or epilogue
   int n_splits, per_split, ws_rows;
   float* ws;
+  // the kernel for few rows: the features from q_width on are keys and values, which go to their pages too (k_pages null:
+  // none do)
+  float* k_pages;
+  float* v_pages;
+  size_t page_stride;
+  const int* block_table;
+  const int* token_req;
+  const int* positions;
+  int max_blocks, q_width, kv_width, head_dim, page_size;
 };
+
+// Where feature n (from q_width on) of row m lies in its page.
+__device__ __forceinline__ float* page_place(const GemmArgs& p, int m, int n) {
+  const int c = n - p.q_width, cc = c < p.kv_width ? c : c - p.kv_width, head = cc / p.head_dim;
+  const int pos = p.positions[m], page = p.block_table[(size_t)p.token_req[m] * p.max_blocks + pos / p.page_size];
+  return (c < p.kv_width ? p.k_pages : p.v_pages) + (size_t)page * p.page_stride + ((size_t)head * p.page_size + pos % p.page_size) * p.head_dim +
+         (cc - head * p.head_dim);
+}
 
 // Many rows: WAVES_M x WAVES_N waves a block, each with TM x TN tiles of 16 x 16 outputs.
 // v_mfma_f32_16x16x4_f32 computes D = A B for A 16 x 4 and B 4 x 16: lane l brings A[l % 16][l / 16] and
@@ -298,6 +315,7 @@ __global__ __launch_bounds__(64 * SKF_MAX_WAVES) void gemm_f32_skinny_kernel(Gem
         p.out[idx] += v;
       else
         p.out[idx] = activate<false>(p.flags, v);
+      if (p.k_pages && n >= p.q_width) *page_place(p, m, n) = v;
     }
   }
 }
@@ -389,13 +407,21 @@ static void launch(const GemmArgs& p, int variant, hipStream_t stream) {
     hipLaunchKernelGGL(gemm_f32_skinny_kernel<4>, grid, block, 0, stream, p);
 }
 
+// 1 if gemm_f32_scatter puts the keys and values of so many rows into their pages.  (Up to 64 rows: a step of 8 rows of
+// GPT-2 large 2,199 -> 2,098 us without the 36 launches that did it.  A tile's epilogue does not: its pieces of 16 bytes a
+// row, each at a place of its own, cost more than the launch that writes whole heads, 15,002 -> 15,122 us for 1,050 rows.)
+extern "C" int gemm_f32_scatters(int M, int n_splits) { return M >= 1 && M <= SKF_MAX_ROWS && n_splits == 1; }
+
 // variant: 0 = choose, 1 = tiles of 64 x 128, 2 = of 64 x 64, 4 = of 32 x 64, 3 = the kernel for up to
 // 64 rows.  n_splits > 1: K in that many parts, whose sums go to ws[part][M][N] (ws_floats floats at least) for sum_partials of gemm_bf16_decode.hip to add up
 // and finish; out is not written then.
-extern "C" int gemm_f32(void* out, const void* A, const void* W, const float* bias, int M, int N,
-                        int K, int lda, int ldw, int ldo, int flags, int variant, int n_splits, float* ws,
-                        size_t ws_floats, hipStream_t stream) {
-  GemmArgs p;
+// k_pages: the features from q_width on go to the pages of the key/value cache too (mlx_lm/models/cache.py:352-354).
+extern "C" int gemm_f32_scatter(void* out, const void* A, const void* W, const float* bias, int M, int N,
+                                int K, int lda, int ldw, int ldo, int flags, int variant, int n_splits, float* ws,
+                                size_t ws_floats, void* k_pages, void* v_pages, size_t page_stride, const int* block_table,
+                                int max_blocks, const int* token_req, const int* positions, int q_width, int kv_width,
+                                int head_dim, int page_size, hipStream_t stream) {
+  GemmArgs p = {};
   p.A = (const float*)A;
   p.W = (const float*)W;
   p.bias = bias;
@@ -422,6 +448,16 @@ extern "C" int gemm_f32(void* out, const void* A, const void* W, const float* bi
     if (!ws || ws_floats < (size_t)n_splits * M * N) FAIL("gemm_f32: the parts' workspace is too small");
     p.n_splits = n_splits, p.per_split = per, p.ws = ws;
   }
+  if (k_pages) {
+    if (!gemm_f32_scatters(M, n_splits) || (variant != 0 && variant != 3) || (flags & (FLAG_ACCUMULATE | FLAG_ACT_ANY)))
+      FAIL("gemm_f32: the cache scatter is the kernel for few rows', with a plain epilogue and K whole");
+    if (!v_pages || !block_table || !token_req || !positions || head_dim <= 0 || page_size <= 0 || max_blocks <= 0 ||
+        kv_width % head_dim != 0 || q_width + 2 * kv_width != N)
+      FAIL("gemm_f32: the cache scatter's pointers or widths (q_width %d + 2 * kv_width %d, N=%d)", q_width, kv_width, N);
+    p.k_pages = (float*)k_pages, p.v_pages = (float*)v_pages, p.page_stride = page_stride;
+    p.block_table = block_table, p.max_blocks = max_blocks, p.token_req = token_req, p.positions = positions;
+    p.q_width = q_width, p.kv_width = kv_width, p.head_dim = head_dim, p.page_size = page_size;
+  }
   double us = 0.0;
   if (variant == 0) variant = M <= SKF_MAX_ROWS ? 3 : cheapest_shape(M, N, K, n_splits, &us);
   if (variant != 3 && p.per_split * (n_splits - 1) * SKF_CHUNK >= K) FAIL("gemm_f32: %d parts of K=%d leave one empty", n_splits, K);
@@ -441,4 +477,11 @@ extern "C" int gemm_f32(void* out, const void* A, const void* W, const float* bi
   }
   CHECK_LAUNCH("gemm_f32");
   return 0;
+}
+
+extern "C" int gemm_f32(void* out, const void* A, const void* W, const float* bias, int M, int N,
+                        int K, int lda, int ldw, int ldo, int flags, int variant, int n_splits, float* ws,
+                        size_t ws_floats, hipStream_t stream) {
+  return gemm_f32_scatter(out, A, W, bias, M, N, K, lda, ldw, ldo, flags, variant, n_splits, ws, ws_floats, nullptr, nullptr, 0, nullptr, 0,
+                          nullptr, nullptr, 0, 0, 0, 0, stream);
 }
