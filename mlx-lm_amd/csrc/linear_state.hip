@@ -400,42 +400,45 @@ __global__ __launch_bounds__(256) void state_chunks_kernel(ScanArgs a, int C, Sp
 // With a bonus the queries read the state ahead of their own token: their side of every exponent is
 // L_(t-1) (zero at the chunk's first token), still <= 0 against L_j for j < t and against L_b, and
 // a pair (t, t) has the bonus in place of an exponential.
+#define CHANNEL_THREADS 512
+#define CHANNEL_AHEAD (4096 / CHANNEL_THREADS)  // loads of each operand that a thread has on their way: a chunk of 64 x 64 in one trip
 template <typename T>
-__global__ __launch_bounds__(256) void channel_chunks_kernel(ScanArgs a, int C, SpanArgs sp) {
+__global__ __launch_bounds__(CHANNEL_THREADS) void channel_chunks_kernel(ScanArgs a, int C, SpanArgs sp) {
+  constexpr int NT = CHANNEL_THREADS, NW = NT / 64;
   extern __shared__ float lds[];
   __shared__ float Rs[64];
   __shared__ unsigned char pair_t[136], pair_j[136];
   const int N = a.N, P = a.P, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int Np = (N + 15) & ~15, Pp = (P + 15) & ~15, CP = C + 4;
+  const int Np = (N + 15) & ~15, Pp = (P + 15) & ~15, CP = C + 4, PS = Pp + 4;  // (rows four banks apart)
   const int h = blockIdx.x;
   const int r = sp.mode == WHOLE ? blockIdx.y : sp.span_req[blockIdx.y];
   float* QT = lds;
   float* KT = QT + (size_t)Np * CP;
   float* LT = KT + (size_t)Np * CP;
   float* V = LT + (size_t)Np * CP;
-  float* O = V + (size_t)C * Pp;
-  float* AT = O + (size_t)C * Pp;
+  float* O = V + (size_t)C * PS;
+  float* AT = O + (size_t)C * PS;
   float* S = AT + (size_t)C * CP;
-  float* Lsum = S + (size_t)Np * Pp;  // [Np] the log decay of every channel over the span so far
+  float* Lsum = S + (size_t)Np * PS;  // [Np] the log decay of every channel over the span so far
   const int start = a.seq_start[r];
   const int lo = sp.mode == WHOLE ? 0 : sp.span_start[blockIdx.y];
   const int n = sp.mode == WHOLE ? a.seq_len[r] : min(a.seq_len[r], lo + sp.span);
   float* Sg = sp.mode == WHOLE ? a.state + (size_t)a.slot_ids[r] * a.state_stride + a.state_offset + (size_t)h * N * P
                                : sp.span_state + ((size_t)blockIdx.y * a.H + h) * N * P;
-  for (int base = 0; base < Np * Pp; base += 256 * 8) {
+  for (int base = 0; base < Np * Pp; base += NT * 8) {
     float sv[8];
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
-      const int i = min(base + u * 256 + tid, Np * Pp - 1), kn = min(i / Pp, N - 1), p = min(i % Pp, P - 1);
+      const int i = min(base + u * NT + tid, Np * Pp - 1), kn = min(i / Pp, N - 1), p = min(i % Pp, P - 1);
       sv[u] = sp.mode != SPAN_STATES ? Sg[(size_t)kn * P + p] : 0.f;
     }
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
-      const int i = base + u * 256 + tid;
-      if (i < Np * Pp) S[i] = i / Pp < N && i % Pp < P ? sv[u] : 0.f;
+      const int i = base + u * NT + tid;
+      if (i < Np * Pp) S[(size_t)(i / Pp) * PS + i % Pp] = i / Pp < N && i % Pp < P ? sv[u] : 0.f;
     }
   }
-  for (int i = tid; i < Np; i += 256) Lsum[i] = 0.f;
+  for (int i = tid; i < Np; i += NT) Lsum[i] = 0.f;
   if (tid < 136) {  // the pairs (t, j <= t) of a tile of sixteen tokens, row by row
     int t = 0;
     while ((t + 1) * (t + 2) / 2 <= tid) ++t;
@@ -450,10 +453,10 @@ __global__ __launch_bounds__(256) void channel_chunks_kernel(ScanArgs a, int C, 
     const int m = min(C, n - c0);
     const size_t row0 = (size_t)(start + c0);
     const bool gates_ahead = outputs && a.gate && P <= 64;
-    float gv[16];
+    float gv[64 / NW];
 #pragma unroll
-    for (int u = 0; u < 16; ++u)
-      gv[u] = gates_ahead ? a.gate[(row0 + min(wave + 4 * u, m - 1)) * a.ldg + (size_t)h * P + min(lane, P - 1)] : 0.f;
+    for (int u = 0; u < 64 / NW; ++u)
+      gv[u] = gates_ahead ? a.gate[(row0 + min(wave + NW * u, m - 1)) * a.ldg + (size_t)h * P + min(lane, P - 1)] : 0.f;
     {
       const int total = C * N, v_total = C * P, most = max(total, v_total);
       const float* qb = a.q + row0 * a.ldq + (size_t)h * N;
@@ -461,11 +464,11 @@ __global__ __launch_bounds__(256) void channel_chunks_kernel(ScanArgs a, int C, 
       const float* ab = a.chan_a + row0 * a.ldca + (size_t)h * N;
       const float* vb = a.v + row0 * a.ldv + (size_t)h * P;
       bool first = true;
-      for (int base = 0; base < most; base += 256 * 16) {
-        float qv[16], kv[16], av[16], vv[16];
+      for (int base = 0; base < most; base += NT * CHANNEL_AHEAD) {
+        float qv[CHANNEL_AHEAD], kv[CHANNEL_AHEAD], av[CHANNEL_AHEAD], vv[CHANNEL_AHEAD];
 #pragma unroll
-        for (int u = 0; u < 16; ++u) {
-          const int e = base + u * 256 + tid;
+        for (int u = 0; u < CHANNEL_AHEAD; ++u) {
+          const int e = base + u * NT + tid;
           const int eq = min(e, total - 1), t = eq / N, i = eq - t * N, tc = min(t, m - 1);
           qv[u] = qb[(size_t)tc * a.ldq + i], kv[u] = kb[(size_t)tc * a.ldk + i], av[u] = ab[(size_t)tc * a.ldca + i];
           const int ev = min(e, v_total - 1), tv = ev / P;
@@ -473,12 +476,12 @@ __global__ __launch_bounds__(256) void channel_chunks_kernel(ScanArgs a, int C, 
         }
         if (first) {
           __syncthreads();  // the chunk before is done with every array (and S is loaded)
-          for (int e = tid; e < C * CP; e += 256) AT[e] = 0.f;
+          for (int e = tid; e < C * CP; e += NT) AT[e] = 0.f;
         }
         first = false;
 #pragma unroll
-        for (int u = 0; u < 16; ++u) {
-          const int e = base + u * 256 + tid;
+        for (int u = 0; u < CHANNEL_AHEAD; ++u) {
+          const int e = base + u * NT + tid;
           if (e < total) {
             const int t = e / N, i = e - t * N;
             const float la = a.chan_logit ? -a.chan_mult * softplus_f(-av[u]) : av[u];
@@ -487,34 +490,38 @@ __global__ __launch_bounds__(256) void channel_chunks_kernel(ScanArgs a, int C, 
           }
           if (e < v_total) {
             const int t = e / P;
-            V[(size_t)t * Pp + (e - t * P)] = t < m ? vv[u] : 0.f;
+            V[(size_t)t * PS + (e - t * P)] = t < m ? vv[u] : 0.f;
           }
         }
       }
-      for (int e = tid; e < C * (Np - N); e += 256) {  // the padding
+      for (int e = tid; e < C * (Np - N); e += NT) {  // the padding
         const int t = e / (Np - N), i = N + e % (Np - N);
         QT[(size_t)i * CP + t] = 0.f, KT[(size_t)i * CP + t] = 0.f, LT[(size_t)i * CP + t] = 0.f;
       }
-      for (int e = tid; e < C * (Pp - P); e += 256) V[(size_t)(e / (Pp - P)) * Pp + P + e % (Pp - P)] = 0.f;
+      for (int e = tid; e < C * (Pp - P); e += NT) V[(size_t)(e / (Pp - P)) * PS + P + e % (Pp - P)] = 0.f;
     }
     __syncthreads();
-    for (int i = tid; i < N; i += 256) {  // a channel's running sum, token after token
+    for (int i = tid; i < N; i += NT) {  // a channel's running sum, token after token, eight on their way at a time
       float acc = 0.f;
-      for (int t = 0; t < C; ++t) {
-        acc += LT[(size_t)i * CP + t];
-        LT[(size_t)i * CP + t] = acc;
+      for (int t0 = 0; t0 < C; t0 += 8) {  // (C is 16, 32 or 64)
+        float4* at = (float4*)(LT + (size_t)i * CP + t0);
+        float4 x = at[0], y = at[1];
+        x.x = acc += x.x, x.y = acc += x.y, x.z = acc += x.z, x.w = acc += x.w;
+        y.x = acc += y.x, y.y = acc += y.y, y.z = acc += y.z, y.w = acc += y.w;
+        at[0] = x, at[1] = y;
       }
       Lsum[i] += acc;
     }
     __syncthreads();
     if (outputs) {
-      // the diagonal tiles: lanes 4p .. 4p + 3 share pair p, a quarter of the channels each
-      const int items = ct * 136 * 4, quarter = Np / 4, part = tid & 3;
-      for (int base = 0; base < items; base += 256) {
+      // the diagonal tiles: lanes 4p .. 4p + 3 share pair p, every fourth channel each (four neighbouring rows of LDS are
+      // four groups of banks; a quarter of the channels each met in one)
+      const int items = ct * 136 * 4, part = tid & 3;
+      for (int base = 0; base < items; base += NT) {
         const int item = base + tid, pr = min(item, items - 1) >> 2, tile = pr / 136, pp = pr - tile * 136;
         const int t = tile * 16 + pair_t[pp], j = tile * 16 + pair_j[pp];
         float acc = 0.f;
-        for (int i = part * quarter; i < (part + 1) * quarter; ++i) {
+        for (int i = part; i < Np; i += 4) {
           const float* row = QT + (size_t)i * CP;
           const float* lrow = LT + (size_t)i * CP;
           const float f = bonus && t == j ? bonus[min(i, N - 1)] : expf(at_query(lrow, t) - lrow[j]);
@@ -526,7 +533,7 @@ __global__ __launch_bounds__(256) void channel_chunks_kernel(ScanArgs a, int C, 
       }
       // the tiles below the diagonal
       const int below = ct * (ct - 1) / 2;
-      for (int tile = wave; tile < below; tile += 4) {
+      for (int tile = wave; tile < below; tile += NW) {
         int tt = 1;
         while (tt * (tt + 1) / 2 <= tile) ++tt;
         const int t0 = tt * 16, j0 = (tile - tt * (tt - 1) / 2) * 16;
@@ -544,7 +551,7 @@ __global__ __launch_bounds__(256) void channel_chunks_kernel(ScanArgs a, int C, 
     }
     __syncthreads();
     const bool state_needed = sp.mode != SPAN_OUTPUTS || c0 + C < n;
-    for (int e = tid; e < Np * C; e += 256) {
+    for (int e = tid; e < Np * C; e += NT) {
       const int i = e / C, t = e - i * C;
       const size_t at = (size_t)i * CP + t;
       const float l = LT[at];
@@ -553,47 +560,47 @@ __global__ __launch_bounds__(256) void channel_chunks_kernel(ScanArgs a, int C, 
     }
     __syncthreads();
     // O[t][p] = sum_j AT[j][t] V[j][p] + sum_i QT[i][t] S[i][p]
-    for (int tile = wave; outputs && tile < ct * pt; tile += 4) {
+    for (int tile = wave; outputs && tile < ct * pt; tile += NW) {
       const int t0 = (tile / pt) * 16, p0 = (tile % pt) * 16;
       f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
       const int j_end = min((m + 3) & ~3, t0 + 16);
       for (int j = 0; j < j_end; j += 4)
-        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(AT[(size_t)(j + lg) * CP + t0 + lr], V[(size_t)(j + lg) * Pp + p0 + lr], acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(AT[(size_t)(j + lg) * CP + t0 + lr], V[(size_t)(j + lg) * PS + p0 + lr], acc, 0, 0, 0);
       for (int i = 0; i < Np; i += 4)
-        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(QT[(size_t)(i + lg) * CP + t0 + lr], S[(size_t)(i + lg) * Pp + p0 + lr], acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(QT[(size_t)(i + lg) * CP + t0 + lr], S[(size_t)(i + lg) * PS + p0 + lr], acc, 0, 0, 0);
 #pragma unroll
-      for (int x = 0; x < 4; ++x) O[(size_t)(t0 + 4 * lg + x) * Pp + p0 + lr] = acc[x];
+      for (int x = 0; x < 4; ++x) O[(size_t)(t0 + 4 * lg + x) * PS + p0 + lr] = acc[x];
     }
     __syncthreads();
     // S[i][:] = exp(L_C[i]) S[i][:] + sum_j KT[i][j] V[j][:]
-    for (int tile = wave; state_needed && tile < nt * pt; tile += 4) {
+    for (int tile = wave; state_needed && tile < nt * pt; tile += NW) {
       const int i0 = (tile / pt) * 16, p0 = (tile % pt) * 16;
       f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
       const int j_end = (m + 3) & ~3;
       for (int j = 0; j < j_end; j += 4)
-        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(KT[(size_t)(i0 + lr) * CP + j + lg], V[(size_t)(j + lg) * Pp + p0 + lr], acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(KT[(size_t)(i0 + lr) * CP + j + lg], V[(size_t)(j + lg) * PS + p0 + lr], acc, 0, 0, 0);
 #pragma unroll
       for (int x = 0; x < 4; ++x) {
         const int i = i0 + 4 * lg + x;
-        float* sp_ = S + (size_t)i * Pp + p0 + lr;
+        float* sp_ = S + (size_t)i * PS + p0 + lr;
         *sp_ = expf(LT[(size_t)i * CP + C - 1]) * *sp_ + acc[x];
       }
     }
     // the rows on their way out: a wave a token
     if (outputs && a.unit_rms)
-      for (int t = wave; t < m; t += 4) {
+      for (int t = wave; t < m; t += NW) {
         float ss = 0.f;
-        for (int pc = lane; pc < P; pc += 64) ss += O[(size_t)t * Pp + pc] * O[(size_t)t * Pp + pc];
+        for (int pc = lane; pc < P; pc += 64) ss += O[(size_t)t * PS + pc] * O[(size_t)t * PS + pc];
         ss = wave_sum(ss);
         if (lane == 0) Rs[t] = 1.0f / sqrtf(ss / (float)P + a.eps);
       }
     if (gates_ahead || (outputs && !a.gate && P <= 64)) {
       const float nw = a.norm_w && a.unit_rms ? a.norm_w[(size_t)h * a.norm_stride + min(lane, P - 1)] : 1.f;
 #pragma unroll
-      for (int u = 0; u < 16; ++u) {
-        const int t = wave + 4 * u;
+      for (int u = 0; u < 64 / NW; ++u) {
+        const int t = wave + NW * u;
         if (t >= m || lane >= P) continue;
-        float o = O[(size_t)t * Pp + lane];
+        float o = O[(size_t)t * PS + lane];
         if (a.unit_rms) o *= Rs[t] * nw;
         if (a.gate) o *= silu_f(gv[u]);
         ((T*)a.out)[(row0 + t) * a.ldo + (size_t)h * P + lane] = from_f32<T>(o);
@@ -602,16 +609,16 @@ __global__ __launch_bounds__(256) void channel_chunks_kernel(ScanArgs a, int C, 
       for (int pb = 0; outputs && pb < P; pb += 64) {
         const int pc = min(pb + lane, P - 1);
         const float nw = a.norm_w && a.unit_rms ? a.norm_w[(size_t)h * a.norm_stride + pc] : 1.f;
-        for (int tb = wave; tb < m; tb += 32) {
+        for (int tb = wave; tb < m; tb += 8 * NW) {
           float g8[8];
 #pragma unroll
           for (int u = 0; u < 8; ++u)
-            g8[u] = a.gate ? a.gate[(row0 + min(tb + 4 * u, m - 1)) * a.ldg + (size_t)h * P + pc] : 0.f;
+            g8[u] = a.gate ? a.gate[(row0 + min(tb + NW * u, m - 1)) * a.ldg + (size_t)h * P + pc] : 0.f;
 #pragma unroll
           for (int u = 0; u < 8; ++u) {
-            const int t = tb + 4 * u;
+            const int t = tb + NW * u;
             if (t >= m || pb + lane >= P) continue;
-            float o = O[(size_t)t * Pp + pc];
+            float o = O[(size_t)t * PS + pc];
             if (a.unit_rms) o *= Rs[t] * nw;
             if (a.gate) o *= silu_f(g8[u]);
             ((T*)a.out)[(row0 + t) * a.ldo + (size_t)h * P + pc] = from_f32<T>(o);
@@ -622,9 +629,9 @@ __global__ __launch_bounds__(256) void channel_chunks_kernel(ScanArgs a, int C, 
   }
   __syncthreads();
   if (sp.mode == SPAN_OUTPUTS) return;
-  for (int i = tid; i < N * P; i += 256) Sg[i] = S[(size_t)(i / P) * Pp + i % P];
+  for (int i = tid; i < N * P; i += NT) Sg[i] = S[(size_t)(i / P) * PS + i % P];
   if (sp.mode == SPAN_STATES)  // (span_decay has a value for every channel here)
-    for (int i = tid; i < N; i += 256) sp.span_decay[((size_t)blockIdx.y * a.H + h) * N + i] = expf(Lsum[i]);
+    for (int i = tid; i < N; i += NT) sp.span_decay[((size_t)blockIdx.y * a.H + h) * N + i] = expf(Lsum[i]);
 }
 
 // Block (head, request, 256 elements of the state), a thread an element: span_state[s] becomes
@@ -756,7 +763,7 @@ static size_t chunk_floats(int N, int P, int C) {
 // The same for the kernel with a decay per key channel.
 static size_t channel_chunk_floats(int N, int P, int C) {
   const size_t Np = (N + 15) & ~15, Pp = (P + 15) & ~15, CP = C + 4;
-  return 3 * Np * CP + 2 * (size_t)C * Pp + (size_t)C * CP + Np * Pp + Np;
+  return 3 * Np * CP + 2 * (size_t)C * (Pp + 4) + (size_t)C * CP + Np * (Pp + 4) + Np;
 }
 
 // 1 if chunks of tokens fit a block's LDS for a state of N x P (`by_channel`: a decay per key channel).
@@ -828,9 +835,9 @@ extern "C" int state_scan(const ScanArgs* args, int chunked, int span, int n_spa
 #define CHUNKS(GRID)                                                                                \
   do {                                                                                              \
     if (by_channel && a.out_dtype == DT_F32)                                                        \
-      hipLaunchKernelGGL(channel_chunks_kernel<float>, GRID, block, bytes, stream, turned, C, sp);       \
+      hipLaunchKernelGGL(channel_chunks_kernel<float>, GRID, dim3(CHANNEL_THREADS), bytes, stream, turned, C, sp);       \
     else if (by_channel)                                                                            \
-      hipLaunchKernelGGL(channel_chunks_kernel<bf16>, GRID, block, bytes, stream, turned, C, sp);        \
+      hipLaunchKernelGGL(channel_chunks_kernel<bf16>, GRID, dim3(CHANNEL_THREADS), bytes, stream, turned, C, sp);        \
     else if (a.out_dtype == DT_F32)                                                                 \
       hipLaunchKernelGGL(state_chunks_kernel<float>, GRID, block, bytes, stream, turned, C, sp);         \
     else                                                                                            \
