@@ -400,16 +400,22 @@ __global__ __launch_bounds__(256) void state_chunks_kernel(ScanArgs a, int C, Sp
 // With a bonus the queries read the state ahead of their own token: their side of every exponent is
 // L_(t-1) (zero at the chunk's first token), still <= 0 against L_j for j < t and against L_b, and
 // a pair (t, t) has the bonus in place of an exponential.
+// What bounds it: a chunk is a chain of short phases (loads, running sums, tiles, products) with barriers between, and one
+// block's LDS leaves room for no second block on a compute unit, so only the block's own waves cover a
+// phase's latency.  A span's launch for its end state / for its outputs (us, 8 prompts of 40 to 300 tokens, 16 heads of 64 x 64): 56 / 135 with
+// four waves, 36 / 81 with eight, rows of LDS four floats longer than P (neighbouring rows shared their banks), the
+// channels of a pair interleaved over its lanes and the running sum taken eight tokens a trip; 38 / 76 with sixteen waves,
+// whose 128 registers a thread spill 21.
 #define CHANNEL_THREADS 512
 #define CHANNEL_AHEAD (4096 / CHANNEL_THREADS)  // loads of each operand that a thread has on their way: a chunk of 64 x 64 in one trip
 template <typename T>
-__global__ __launch_bounds__(CHANNEL_THREADS) void channel_chunks_kernel(ScanArgs a, int C, SpanArgs sp) {
+__global__ __launch_bounds__(CHANNEL_THREADS) void channel_chunks_kernel(ScanArgs a, int C, int PS, SpanArgs sp) {
   constexpr int NT = CHANNEL_THREADS, NW = NT / 64;
   extern __shared__ float lds[];
   __shared__ float Rs[64];
   __shared__ unsigned char pair_t[136], pair_j[136];
   const int N = a.N, P = a.P, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int Np = (N + 15) & ~15, Pp = (P + 15) & ~15, CP = C + 4, PS = Pp + 4;  // (rows four banks apart)
+  const int Np = (N + 15) & ~15, Pp = (P + 15) & ~15, CP = C + 4;  // (PS: a row of V, O and S, channel_row_floats)
   const int h = blockIdx.x;
   const int r = sp.mode == WHOLE ? blockIdx.y : sp.span_req[blockIdx.y];
   float* QT = lds;
@@ -760,16 +766,25 @@ static size_t chunk_floats(int N, int P, int C) {
   const size_t Np = (N + 15) & ~15, Pp = (P + 15) & ~15, CP = C + 4;
   return 2 * Np * CP + (size_t)C * Np + 2 * (size_t)C * Pp + (size_t)C * CP + Np * Pp;
 }
-// The same for the kernel with a decay per key channel.
-static size_t channel_chunk_floats(int N, int P, int C) {
-  const size_t Np = (N + 15) & ~15, Pp = (P + 15) & ~15, CP = C + 4;
-  return 3 * Np * CP + 2 * (size_t)C * (Pp + 4) + (size_t)C * CP + Np * (Pp + 4) + Np;
+// The same for the kernel with a decay per key channel, where rows of P values lie PS floats apart.
+static size_t channel_chunk_floats(int N, int PS, int C) {
+  const size_t Np = (N + 15) & ~15, CP = C + 4;
+  return 3 * Np * CP + 2 * (size_t)C * PS + (size_t)C * CP + Np * PS + Np;
+}
+// PS: rows four banks apart, unless just that makes chunks of C tokens too many for the LDS (a shorter chunk, or none, costs more
+// than the rows' shared banks).
+static int channel_row_floats(int N, int P, int C) {
+  const int Pp = (P + 15) & ~15;
+  return channel_chunk_floats(N, Pp + 4, C) * sizeof(float) <= SCAN_MAX_LDS ? Pp + 4 : Pp;
+}
+// Bytes of LDS of chunks of C tokens.
+static size_t chunk_bytes(bool by_channel, int N, int P, int C) {
+  return (by_channel ? channel_chunk_floats(N, channel_row_floats(N, P, C), C) : chunk_floats(N, P, C)) * sizeof(float);
 }
 
 // 1 if chunks of tokens fit a block's LDS for a state of N x P (`by_channel`: a decay per key channel).
 extern "C" int state_chunks_takes(int N, int P, int by_channel) {
-  return N > 0 && P > 0 && P <= 256 &&
-         (by_channel ? channel_chunk_floats(N, P, 16) : chunk_floats(N, P, 16)) * sizeof(float) <= SCAN_MAX_LDS;
+  return N > 0 && P > 0 && P <= 256 && chunk_bytes(by_channel, N, P, 16) <= SCAN_MAX_LDS;
 }
 
 // `chunked`: the kernel that takes a chunk of tokens at a time (for steps in which some request
@@ -811,7 +826,7 @@ extern "C" int state_scan(const ScanArgs* args, int chunked, int span, int n_spa
   const bool by_channel = a.chan_a != nullptr;
   if (chunked && !(by_channel && (a.k_scale || a.skip || a.rot_dims)))
     for (int c = 64; c >= 16 && !C; c /= 2)
-      if ((by_channel ? channel_chunk_floats(a.N, a.P, c) : chunk_floats(a.N, a.P, c)) * sizeof(float) <= SCAN_MAX_LDS) C = c;
+      if (chunk_bytes(by_channel, a.N, a.P, c) <= SCAN_MAX_LDS) C = c;
   if (C) {
     ScanArgs turned = a;  // (the chunked kernel itself turns nothing)
     if (a.rot_dims) {
@@ -830,14 +845,15 @@ extern "C" int state_scan(const ScanArgs* args, int chunked, int span, int n_spa
       (void)hipFuncSetAttribute((const void*)channel_chunks_kernel<bf16>, hipFuncAttributeMaxDynamicSharedMemorySize, SCAN_MAX_LDS);
       chunks_raised = true;
     }
-    const size_t bytes = (by_channel ? channel_chunk_floats(a.N, a.P, C) : chunk_floats(a.N, a.P, C)) * sizeof(float);
+    const size_t bytes = chunk_bytes(by_channel, a.N, a.P, C);
+    const int row_floats = by_channel ? channel_row_floats(a.N, a.P, C) : 0;
     SpanArgs sp = {WHOLE, 0, nullptr, nullptr, nullptr, nullptr};
 #define CHUNKS(GRID)                                                                                \
   do {                                                                                              \
     if (by_channel && a.out_dtype == DT_F32)                                                        \
-      hipLaunchKernelGGL(channel_chunks_kernel<float>, GRID, dim3(CHANNEL_THREADS), bytes, stream, turned, C, sp);       \
+      hipLaunchKernelGGL(channel_chunks_kernel<float>, GRID, dim3(CHANNEL_THREADS), bytes, stream, turned, C, row_floats, sp); \
     else if (by_channel)                                                                            \
-      hipLaunchKernelGGL(channel_chunks_kernel<bf16>, GRID, dim3(CHANNEL_THREADS), bytes, stream, turned, C, sp);        \
+      hipLaunchKernelGGL(channel_chunks_kernel<bf16>, GRID, dim3(CHANNEL_THREADS), bytes, stream, turned, C, row_floats, sp); \
     else if (a.out_dtype == DT_F32)                                                                 \
       hipLaunchKernelGGL(state_chunks_kernel<float>, GRID, block, bytes, stream, turned, C, sp);         \
     else                                                                                            \

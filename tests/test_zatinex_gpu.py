@@ -262,6 +262,13 @@ def test_a_state_that_decays_by_key_channel_in_portions_of_two_requests(N, P, H,
     assert (state[[1, 3]] == 3.0).all() and (state[:, :7] == 3.0).all()
 
 
+@pytest.mark.parametrize("chunked", [True, "spans"])
+@pytest.mark.parametrize("N,P,H", [(16, 224, 1), (144, 112, 2), (208, 112, 1), (304, 16, 2), (496, 16, 1)])
+def test_states_whose_chunks_fit_only_in_rows_without_padding(N, P, H, chunked):
+    """Chunks of 64, 32 and 16 tokens whose rows of LDS lie side by side, as four more floats a row would not fit."""
+    test_a_state_that_decays_by_key_channel_in_portions_of_two_requests(N, P, H, chunked)
+
+
 def test_a_token_far_back_in_a_state_that_decays_by_channel():
     """Half of the key channels keep nearly everything and the query of the last of 1,200 tokens
     lies along the key of token 3 on those: the output is that token's value, and the state after
