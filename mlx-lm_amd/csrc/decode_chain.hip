@@ -5,12 +5,16 @@
 //
 // What bounds it: so few rows cost a layer five launches of 4 to 10 us, each 1.7 us from the last
 // one's end, then a trip for its rows, then its weights from memory, then the drain.  In one launch a
-// block copies its next unit's weights into LDS (keys and values, which no product of the step makes, into
-// registers) while it waits for the rows of the unit at hand, and a hand-over between two products is one store and
-// one load that meet in memory: 1.2 us.  A layer of GPT-2's sizes (us, one row, with its five launches / here; two rows):
-// width 768 at 93 keys 26 / 16.3 (18.6), 1,280 at 500 34 / 19.9, 1,600 at 700 37 / 23.0 (26.0).  Of the 23 the weights'
-// 61 MB are 9.6 at the memory's rate: a unit's copies (100 KB at the 25 KB a us that a compute unit draws) are longer than a
-// hand-over in three of the five, and the rows that a wave asks for come behind them.
+// hand-over between two products is one store and one load that meet in memory, 1.2 us, and the next unit's
+// weights come into LDS meanwhile (keys and values, which no product of the step makes, into registers).  A wave
+// that issues those copies stands still until the memory has taken them, 3 to 4 us for the 100 KB of a unit (a compute
+// unit draws some 25 KB a us), and rows that it asks for come behind them: so CH_COPIERS waves of the block do nothing
+// else, and the others never wait for more than their rows.  A layer of GPT-2's sizes in us, with its five launches /
+// here with the computing waves copying too / with two waves to copy / with four (as it is):
+//   width   768 at  93 keys, one row    26 / 16.3 / 16.4 / 15.7   (two rows, in one launch only: 18.6 / - / 17.9)
+//   width 1,280 at 500 keys, one row    34 / 19.9 / 19.0 / 17.1
+//   width 1,600 at 700 keys, one row    37 / 23.0 / 21.3 / 19.5   (two rows: 26.0 / 23.4 / 22.0)
+// Of the 19.5 the weights' 61 MB are 9.6 at the memory's rate and the five hand-overs 6.
 //
 // Hand-over.  What one product hands to the next lies in words of eight bytes, 4 of payload (a float32
 // of the stream, or two bfloat16) and 4 of tag; a tag belongs to one product of one step.  A word is
