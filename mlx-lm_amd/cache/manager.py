@@ -107,6 +107,7 @@ class CacheManager:
             elif need is not None:
                 raise TypeError(f"cache slot {slot}: unknown need {need!r}")
         self._free_state_slots = list(range(max_requests - 1, -1, -1))
+        self._state_rows = None  # the rows of all state tensors cleared at once (on a GPU)
         self.requests: Dict[object, RequestCache] = {}
         self.kept: List[KeptPages] = []  # detached and neither attached again nor dropped
         if device is not None:
@@ -130,6 +131,11 @@ class CacheManager:
             self.state_storage[slot] = torch.zeros(
                 (self.max_requests, *need.shape), dtype=getattr(torch, need.dtype), device=self.device
             )
+        storages = list(self.state_storage.values())
+        if len(storages) > 1 and all(t.is_cuda and t.numel() for t in storages):
+            from ..ops.kernels import RowsCleared
+
+            self._state_rows = RowsCleared(storages)
 
     # -- sizes ---------------------------------------------------------------
 
@@ -164,9 +170,16 @@ class CacheManager:
         self._serial = getattr(self, "_serial", 0) + 1
         rc = RequestCache(request_id, slot, blocks=[[] for _ in self.groups], serial=self._serial)
         self.requests[request_id] = rc
-        for storage in self.state_storage.values():
-            storage[slot].zero_()
+        self._clear_state(slot)
         return rc
+
+    def _clear_state(self, state_slot):
+        # (a launch a tensor keeps the host some 10 us each, 64 of them for eight requests of a model with eight such tensors)
+        if self._state_rows is not None:
+            self._state_rows.clear(state_slot)
+            return
+        for storage in self.state_storage.values():
+            storage[state_slot].zero_()
 
     def reserve(self, request_id, n_new):
         """Make sure positions ``length .. length+n_new-1`` have pages in every group.
@@ -404,11 +417,11 @@ class CacheManager:
     def set_state(self, request_id, state=None):
         """A live request's rows of the state tensors: as ``state`` (cache slot -> row) has them, or zero."""
         rc = self.requests[request_id]
+        if state is None:
+            self._clear_state(rc.state_slot)
+            return
         for slot, storage in self.state_storage.items():
-            if state is None:
-                storage[rc.state_slot].zero_()
-            else:
-                storage[rc.state_slot].copy_(state[slot])
+            storage[rc.state_slot].copy_(state[slot])
 
     def drop(self, kept):
         """Give back the pages of a ``KeptPages`` that nobody goes on from."""

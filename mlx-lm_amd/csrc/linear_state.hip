@@ -738,6 +738,28 @@ __global__ __launch_bounds__(256) void conv_state_update_kernel(const float* __r
 }
 
 // A block a (row, group).
+// Row `row` of every tensor of `table` (base, bytes a row) set to zero: blockIdx.y is the tensor.  A new request's rows
+// are 10 KB to a few MB over all tensors, less than the launches that clear them one by one cost their host.
+struct RowsOf {
+  char* base;
+  size_t bytes;
+};
+template <typename W>
+__device__ inline void clear_row(char* row, size_t bytes) {
+  for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < bytes / sizeof(W); i += (size_t)gridDim.x * 256) ((W*)row)[i] = W{};
+}
+__global__ __launch_bounds__(256) void clear_rows_kernel(const RowsOf* __restrict__ table, int row) {
+  const RowsOf t = table[blockIdx.y];
+  char* p = t.base + (size_t)row * t.bytes;
+  const size_t low = (size_t)p | t.bytes;
+  if (low % 16 == 0)
+    clear_row<float4>(p, t.bytes);
+  else if (low % 4 == 0)
+    clear_row<float>(p, t.bytes);
+  else
+    clear_row<char>(p, t.bytes);
+}
+
 template <typename T>
 __global__ __launch_bounds__(256) void gated_group_rmsnorm_kernel(const float* __restrict__ y, int ldy,
                                                                   const float* __restrict__ z, int ldz,
@@ -913,6 +935,17 @@ extern "C" int conv_state_update(const float* u, int ldu, int conv_col, int taps
   hipLaunchKernelGGL(conv_state_update_kernel, grid, block, 0, stream, u, ldu, conv_col, taps, C, state, state_stride,
                      conv_offset, seq_start, seq_len, slot_ids);
   CHECK_LAUNCH("conv_state_update");
+  return 0;
+}
+
+// `most_bytes`: of a row of any of the tensors.
+extern "C" int clear_rows(const void* table, int n_tensors, size_t most_bytes, int row, hipStream_t stream) {
+  if (n_tensors <= 0 || most_bytes == 0) return 0;
+  if (!table || row < 0 || n_tensors > 65535) FAIL("clear_rows: row %d of %d tensors", row, n_tensors);
+  const size_t blocks = (most_bytes / 16 + 1023) / 1024;  // four stores of 16 bytes a thread
+  dim3 grid(blocks < 1 ? 1 : blocks > 1024 ? 1024 : (unsigned)blocks, n_tensors);
+  hipLaunchKernelGGL(clear_rows_kernel, grid, dim3(256), 0, stream, (const RowsOf*)table, row);
+  CHECK_LAUNCH("clear_rows");
   return 0;
 }
 

@@ -1371,6 +1371,25 @@ def conv_state_update(u, conv_col, taps, n_channels, state, conv_offset, seq_sta
     build.check(lib, rc, "conv_state_update")
 
 
+class RowsCleared:
+    """``clear(row)`` sets that row of every one of the contiguous ``tensors`` (one device, ``[rows, ...]``,
+    of any types) to zero, in one launch."""
+
+    def __init__(self, tensors):
+        _need(all(t.is_cuda and t.is_contiguous() and t.device == tensors[0].device for t in tensors), "clear_rows: contiguous tensors of one GPU")
+        self.n_rows = min(t.shape[0] for t in tensors)
+        sizes = [(t.data_ptr(), t.numel() // t.shape[0] * t.element_size()) for t in tensors]
+        self.tensors, self.most = list(tensors), max(n for _, n in sizes)
+        self.table = torch.tensor(sizes, dtype=torch.int64).to(tensors[0].device)
+
+    def clear(self, row):
+        _need(0 <= row < self.n_rows, "clear_rows: no such row")
+        lib = build.load("linear_state")
+        with torch.cuda.device(self.table.device):
+            rc = lib.clear_rows(_ptr(self.table), _c_int(len(self.tensors)), _c_size_t(self.most), _c_int(row), _stream())
+        build.check(lib, rc, "clear_rows")
+
+
 def gated_group_rmsnorm(out, y, z, weight, groups, eps):
     """``out = RMSnorm(y * silu(z))`` in ``groups`` equal parts of a row, times ``weight``."""
     lib = build.load("linear_state")
