@@ -739,7 +739,8 @@ __global__ __launch_bounds__(256) void conv_state_update_kernel(const float* __r
 
 // A block a (row, group).
 // Row `row` of every tensor of `table` (base, bytes a row) set to zero: blockIdx.y is the tensor.  A new request's rows
-// are 10 KB to a few MB over all tensors, less than the launches that clear them one by one cost their host.
+// are 10 KB to a few MB over all tensors, less than the launches that clear them one by one cost their host: eight requests of
+// a model with eight tensors were 64 fills of 1.9 us some 10 us apart, a pass of theirs 7,491 us, and 7,312 with eight launches.
 struct RowsOf {
   char* base;
   size_t bytes;
