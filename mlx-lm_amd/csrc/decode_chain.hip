@@ -28,8 +28,12 @@
 // No block relies on another one running.  A unit (8 to 32 features of a product, or a row's head and part
 // of the keys) belongs to a block by its number; a wave that has waited `patience` for its words gives up, and its
 // block looks for the missing units and does one itself, then tries again.  A unit done twice stores the
-// same words twice; a unit done so late that its words' places hold a later product's is seen by their tags and
-// left alone.  So a single resident block would finish the launch, whatever holds the rest of the GPU.
+// same words twice.  A block that falls behind others on the way (its unit done by them meanwhile, and a later product's
+// words in the places that it reads) sees that by their tags, and where it had read its rows already, its late words change
+// nothing: a word is stored by an atomic maximum, whose high half is the tag, so what a place holds only gets later.  (With
+// plain stores a late word could put back an older product's, which nobody then missed where its own product's
+// successor was complete: the residual's old value would have been waited for without end.)  So a single resident block
+// would finish the launch, whatever holds the rest of the GPU.
 #include "decode_chain.h"
 #include "lds_copy.h"
 
@@ -87,8 +91,9 @@ __device__ __forceinline__ f32x4_t mfma(ChFrag a, ChFrag b, f32x4_t c) {
 __device__ __forceinline__ word_t word_load(const word_t* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+// (a maximum: a place that holds a later product's word keeps it)
 __device__ __forceinline__ void word_store(word_t* p, uint32_t payload, uint32_t tag) {
-  __hip_atomic_store(p, ((word_t)tag << 32) | payload, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  (void)__hip_atomic_fetch_max(p, ((word_t)tag << 32) | payload, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 __device__ __forceinline__ void word_store(word_t* p, float payload, uint32_t tag) { word_store(p, __float_as_uint(payload), tag); }
 __device__ __forceinline__ uint32_t tag_of(word_t w) { return (uint32_t)(w >> 32); }
@@ -113,7 +118,7 @@ __device__ __forceinline__ int words_wait(word_t (&w)[MOST], int n, uint32_t tag
 #pragma unroll
     for (int i = 0; i < MOST; ++i) {
       there = there && tag_of(w[i]) == tag;
-      late = late || tag_of(w[i]) - tag - 1u < CH_TAGS_A_STEP;
+      late = late || tag_of(w[i]) > tag;
     }
     if (__all(there)) return CH_THERE;
     if (__any(late)) return CH_LATE;
@@ -621,8 +626,7 @@ __global__ __launch_bounds__(CH_ALL_WAVES * 64, 3) void decode_chain_kernel(Chai
       if (threadIdx.x == 0) sh.missing = 0x7fffffff;
       meet(&sh.arrived, target, lane);
       for (int j = threadIdx.x; j < per * R; j += CH_WAVES * 64) {
-        const uint32_t off = tag_of(word_load(words + j)) - (tag_base + q);
-        if (off < CH_TAGS_A_STEP) continue;
+        if (tag_of(word_load(words + j)) >= tag_base + q) continue;
         const int of = qk == CH_ATTN ? (j / per) * p.n_heads + (j % per) * 2 / CH_HEAD : (j % per) * (pairs_of ? 2 : 1) / zq.features;
         atomicMin(&sh.missing, (of - turn + zq.units) % zq.units);
       }
@@ -635,8 +639,16 @@ __global__ __launch_bounds__(CH_ALL_WAVES * 64, 3) void decode_chain_kernel(Chai
   }
 }
 
-// (a launch of its own ahead of the step's: no block may see the tag change)
-__global__ void chain_step_kernel(uint32_t* base, uint32_t by) { *base += by; }
+// (a launch of its own ahead of the step's: no block may see the tag change.)  Tags only grow, as the words' maximum wants
+// it: where 32 bits end, after some 18 million steps of 48 layers, the words start from zeros again.
+__global__ __launch_bounds__(256) void chain_step_kernel(uint32_t* base, uint32_t by, word_t* words, int n_words) {
+  const uint32_t old = *base;
+  const bool again = old > 0u - 2 * CH_TAGS_A_STEP;
+  __syncthreads();
+  if (again)
+    for (int i = threadIdx.x; i < n_words; i += 256) words[i] = 0;
+  if (threadIdx.x == 0) *base = again ? by : old + by;
+}
 
 DEFINE_LAST_ERROR(mlxlm_last_error)
 
@@ -712,7 +724,7 @@ extern "C" int decode_chain(const ChainDims* d, int rows, const void* layers, vo
   deal_of(d, rows, &deal);
   ChainArgs a = {};
   size_t at[CH_KINDS];
-  words_of(d, rows, at);
+  const size_t n_words = words_of(d, rows, at);
   word_t* words = (word_t*)memory;
   a.layers = (const ChainLayer*)layers, a.n_layers = d->n_layers;
   for (int i = 0; i < CH_KINDS; ++i) a.size[i] = deal.size[i];
@@ -735,7 +747,8 @@ extern "C" int decode_chain(const ChainDims* d, int rows, const void* layers, vo
     if (e != hipSuccess) FAIL("decode_chain: cannot get %zu bytes of LDS: %s", deal.lds, hipGetErrorString(e));
     granted[rows - 1] = deal.lds;
   }
-  hipLaunchKernelGGL(chain_step_kernel, dim3(1), dim3(1), 0, stream, (uint32_t*)memory, (uint32_t)(d->n_layers * CH_KINDS + 1));
+  hipLaunchKernelGGL(chain_step_kernel, dim3(1), dim3(256), 0, stream, (uint32_t*)memory, (uint32_t)(d->n_layers * CH_KINDS + 1),
+                     words + at[0], (int)(n_words - at[0]));
   CHECK_LAUNCH("decode_chain");
   if (rows == 1)
     hipLaunchKernelGGL(decode_chain_kernel<1>, dim3(deal.blocks), dim3(CH_ALL_WAVES * 64), deal.lds, stream, a);

@@ -150,3 +150,71 @@ def test_sizes_the_one_launch_does_not_take(change):
     rows = sizes.pop("rows")
     d = Dims(*sizes.values(), 2048, 1e-5, 1e-5, 0.125)
     assert _lib().decode_chain_takes(ctypes.byref(d), rows) == 0
+
+
+def _one_layer(rows=1):
+    """(dims, the layers' table on the device and all it points to, launch) of one layer of width 128 without keys in the cache."""
+    lib, D, I, Q = _lib(), 128, 256, 128
+    g = torch.Generator().manual_seed(rows)
+    W = [_packed((torch.randn(*s, generator=g) * s[1] ** -0.5).to(BF).cuda()) for s in ((3 * Q, D), (D, Q), (I, D), (D, I))]
+    ones, zeros = torch.ones(D, device="cuda"), torch.zeros(D, device="cuda")
+    kv = [torch.zeros(rows, 2, 16, 64, dtype=BF, device="cuda") for _ in range(2)]
+    table = (Layer * 1)()
+    table[0].W[:], table[0].gamma[:], table[0].beta[:] = [w.data_ptr() for w in W], [ones.data_ptr()] * 2, [zeros.data_ptr()] * 2
+    table[0].k, table[0].v = kv[0].data_ptr(), kv[1].data_ptr()
+    on_gpu = torch.frombuffer(bytearray(bytes(table)), dtype=torch.uint8).cuda()
+    d = Dims(1, D, I, 2, 2, 16, 2 * 16 * 64, 1e-5, 1e-5, 0.125)
+    memory = torch.zeros(lib.decode_chain_bytes(ctypes.byref(d), rows) // 8, dtype=torch.int64, device="cuda")
+    index = torch.arange(rows, dtype=torch.int32, device="cuda")
+    pos = torch.zeros(rows, dtype=torch.int32, device="cuda")
+    h = torch.randn(rows, D, generator=g).cuda()
+    held = (W, ones, zeros, kv, on_gpu, index, pos, h)
+
+    def launch():
+        out = torch.full_like(h, float("nan"))
+        p = [_vp(x.data_ptr()) for x in (on_gpu, memory, h, out, index, index, pos)]
+        rc = lib.decode_chain(ctypes.byref(d), rows, p[0], p[1], p[2], p[3], D, p[4], 1, p[5], p[6], 0, ctypes.c_uint(0),
+                              _vp(torch.cuda.current_stream().cuda_stream))
+        assert rc == 0, lib.mlxlm_last_error().decode()
+        torch.cuda.synchronize()
+        return out
+
+    return memory, launch, held
+
+
+def _places(rows, N, Q, D, I):
+    """(first word, words) of q/k/v, attention's rows, the stream after attention, the activations, the stream."""
+    at, out = 32, []
+    for n in (N // 2, Q // 2, D, I // 2, D):
+        out.append(slice(at, at + n * rows))
+        at += (n * rows + 31) // 32 * 32
+    return out
+
+
+@pytest.mark.parametrize("rows", [1, 2])
+def test_late_words_leave_a_later_product_s_alone(rows):
+    """Where the places of a product hold words of a later one, as they do for a block that fell behind the others after it
+    had read its rows, they stay: an older word put back would be waited past by nobody and waited for without end."""
+    memory, launch, _held = _one_layer(rows)
+    launch()
+    qkv, att, h1, act, h2 = _places(rows, 3 * 128, 128, 128, 256)
+    base = memory[0].item() & 0xFFFFFFFF
+    assert base == 6 and (memory[h1] >> 32 == base + 2).all() and (memory[act] >> 32 == base + 3).all()
+    later = (base + 1000 << 32) + 12345  # (its readers see that their unit is long done: the launch ends)
+    memory[h1], memory[act] = later, later
+    out = launch()
+    assert (memory[qkv] >> 32 == base + 6).all() and (memory[att] >> 32 == base + 7).all()  # computed, and stored over older ones
+    assert (memory[h1] == later).all() and (memory[act] == later).all() and out.isnan().all()
+
+
+def test_tags_where_their_bits_end():
+    """The counter of tags goes past its last step: the words start from zeros again and every step's output is the same."""
+    memory, launch, _held = _one_layer()
+    want = launch()
+    memory[0] = 0xFFFFFFFF - 2 * 0x10000 - 13
+    bases = []
+    for _ in range(6):
+        assert torch.equal(launch(), want)
+        bases.append(memory[0].item() & 0xFFFFFFFF)
+    turn = next(i for i, b in enumerate(bases) if b == 6)
+    assert bases == [0xFFFFFFFF - 2 * 0x10000 - 13 + 6 * (i + 1) for i in range(turn)] + [6 * (i + 1) for i in range(6 - turn)] and 0 < turn < 5
