@@ -34,7 +34,7 @@ int decode_chain_takes(const ChainDims* d, int rows);
 size_t decode_chain_bytes(const ChainDims* d, int rows);
 // h_out = the stream `h` ([rows][width] float32, row stride ldh, both) after all layers; the rows' keys and values go to
 // their pages.  `layers` lies on the device.  `blocks` and `patience` (ticks of 10 ns): 0, or for tests a smaller
-// grid, and how long a block waits for another's unit before it does it itself.
+// grid, and how long a block waits for another's unit before the units are dealt anew among the blocks that run.
 int decode_chain(const ChainDims* d, int rows, const void* layers, void* memory, const float* h, float* h_out, int ldh,
                  const int* block_table, int max_blocks, const int* token_req, const int* positions, int blocks,
                  unsigned patience, hipStream_t stream);

@@ -26,14 +26,20 @@
 // be as many bytes as its weights.
 //
 // No block relies on another one running.  A unit (8 to 32 features of a product, or a row's head and part
-// of the keys) belongs to a block by its number; a wave that has waited `patience` for its words gives up, and its
-// block looks for the missing units and does one itself, then tries again.  A unit done twice stores the
+// of the keys) belongs to a block by its number.  A wave that has waited `patience` for its words gives up: its block then
+// counts the blocks that run (each says so in a word of its own) and takes its share of all units among those, from the first
+// phase that lacks one; what is missing even so is done by whoever waits for it.  A unit done twice stores the
 // same words twice.  A block that falls behind others on the way (its unit done by them meanwhile, and a later product's
 // words in the places that it reads) sees that by their tags, and where it had read its rows already, its late words change
 // nothing: a word is stored by an atomic maximum, whose high half is the tag, so what a place holds only gets later.  (With
 // plain stores a late word could put back an older product's, which nobody then missed where its own product's
 // successor was complete: the residual's old value would have been waited for without end.)  So a single resident block
-// would finish the launch, whatever holds the rest of the GPU.
+// would finish the launch, whatever holds the rest of the GPU.  A step of XL at 700 keys with 0 / 64 / 128 / 224 of 256 compute
+// units held by another stream's kernel for longer than the step (us): 1,005 / 2,149 / 2,098 / 6,168; where units kept their first
+// owners 1,004 / 16,494 / 16,877 / until they were free; each layer's own launches 1,851 / 2,174 / 2,323 / 5,149.  GPT-2 small at 93
+// keys pays for the first wait: 253 / 491 / 567 / 1,095 against 349 / 340 / 370 / 609.  (Blocks of twelve waves of
+// 168 registers leave no room beside them: two engines' steps on two streams follow each other, a pair of XL steps 1,999
+// against 2,266; beside an XL step of 8 rows the step of one row takes 989 instead of 2,384, and the pair 3,094 instead of 2,722.)
 #include "decode_chain.h"
 #include "lds_copy.h"
 
@@ -51,7 +57,13 @@
 #define CH_KEY_TILES ((CHAIN_MOST_KEYS + CH_ALL_WAVES * 8 - 1) / (CH_ALL_WAVES * 8))  // loads of 8 keys a wave holds
 
 #define CH_LDS_MOST (160 * 1024)
-#define CH_PATIENCE 20000  // 200 us: ten times what a layer's longest wait is
+// Ticks of 10 ns.  200 us: some five times the longest wait of any size (a head's, for a layer of width
+// 2,048, 38 us); 100 and 60 were 0.1 ms better for held compute units and worse beside short kernels, whose places come free
+// (XL beside large products, nine steps of ten within 1.4 ms, then 1.75 and 1.9).  Dealt anew, a wait is a phase's, and 30 us
+// are enough: with 10 a step of 2.3 ms took 2.8 (blocks that wait for a head did others' units).
+#define CH_PATIENCE 20000
+#define CH_PATIENCE_ANEW 3000u
+#define CH_UNITS_MOST 4096u  // a phase has fewer: 3 x 7,168 features of q, k and v, 8 a unit
 
 enum { CH_QKV = 0, CH_ATTN, CH_OUT, CH_FC, CH_PROJ, CH_KINDS };
 
@@ -64,6 +76,7 @@ struct ChainArgs {
   int n_layers;
   ChainSize size[CH_KINDS];
   int product_blocks, attention_blocks;  // attention's are the later ones
+  word_t* present;  // a word a block: tag_base's once it runs
   const uint32_t* tag_base;
   uint32_t patience;   // ticks of 10 ns
   float eps1, eps2, scale;
@@ -226,11 +239,16 @@ struct ChainShared {
   __attribute__((aligned(16))) float part[CH_ALL_WAVES][CH_HEAD];
   float part_m[16], part_l[16];
   int how[CH_ALL_WAVES];
-  int missing;
+  uint32_t missing;
   // what the block does next, for all waves: phase (-1: no more) and unit, whether its weights are in LDS, and the unit after it
   struct {
-    int ph, unit, held, then_ph, then_unit;
+    int ph, unit, held, then_ph, then_unit, anew;
   } plan;
+  // Dealt anew: this block's place among those that run and their number, a missing unit that it does in its own's stead, and
+  // the unit whose weights are in LDS or on their way
+  struct {
+    int start, stride, help_i, help_u, held_ph, held_unit;
+  } anew;
   uint32_t arrived;
 };
 
@@ -354,41 +372,300 @@ __device__ __forceinline__ int chain_attention(const ChainArgs& p, ChainShared<R
   return worst;
 }
 
+extern __shared__ __attribute__((aligned(16))) char held_weights[];
+
+// A unit of a product.  Computing waves return how their wait for rows ended; copying ones leave with the weights of the unit
+// after it on their way.
+template <int R>
+__device__ __forceinline__ int chain_product(const ChainArgs& p, ChainShared<R>& sh, int ph, int unit, bool in_lds, int then_ph, int then_unit,
+                                             uint32_t tag, uint32_t patience, uint32_t& target, int lane, int wave) {
+  const uint32_t lds = lds_address(held_weights), lds_small = lds_address(sh.small);
+  const int kind = ph % CH_KINDS, layer = ph / CH_KINDS;
+  const bool copies = wave >= CH_WAVES;
+  if (!in_lds) {
+    if (copies) {
+      copy_unit(p, unit_of(p, ph, unit, wave), lds, lds_small, lane, wave - CH_WAVES);
+      copies_arrived<0>();
+    }
+    __syncthreads();
+  }
+  if (copies) {
+    __syncthreads();  // (the computing waves have read what lies in LDS)
+    if (then_ph >= 0) copy_unit(p, unit_of(p, then_ph, then_unit, wave), lds, lds_small, lane, wave - CH_WAVES);
+    return CH_THERE;
+  }
+  const ChainUnit at_hand = unit_of(p, ph, unit, wave);
+  const ChainSize& z = p.size[kind];
+  const bool normed = at_hand.normed, first = ph == 0, last = ph == p.n_layers * CH_KINDS - 1;
+  const int g = lane >> 4, kblocks = at_hand.kblocks, pairs = at_hand.pairs, n_blocks = at_hand.n_blocks, n_pairs = at_hand.n_pairs;
+  const int n0 = at_hand.n0, n_end = at_hand.n_end;
+  const bool odd = kblocks & 1;  // the last pair has no second k-block: its lanes repeat the first, and count as zeros
+  const bool short_pair = odd && n_pairs > 0 && wave + CH_WAVES * (n_pairs - 1) == pairs - 1;
+
+  // ---- what the copying waves brought ---------------------------------------------------------
+  // wave 0 writes the outputs: one feature a lane into the stream, else two neighbours a lane
+  const int o_m = normed ? lane >> 4 : lane >> 3;
+  const int o_f = normed ? (lane & 15) * 2 : lane & 7;
+  const bool mine = wave == 0 && o_m < R && n0 + o_f < n_end;
+  float2 bias = make_float2(0.f, 0.f);
+  float old = 0.f;
+  if (wave == 0 && at_hand.ly->bias[at_hand.which]) bias.x = sh.small[CH_WAVES * 2][o_f], bias.y = sh.small[CH_WAVES * 2][o_f + 1];
+  float gm[CH_LN_BLOCKS], bt[CH_LN_BLOCKS];
+#pragma unroll
+  for (int b = 0; b < CH_LN_BLOCKS; ++b) gm[b] = sh.small[wave * 2][b * 64 + lane], bt[b] = sh.small[wave * 2 + 1][b * 64 + lane];
+  ChFrag w[CH_HELD][2];
+#pragma unroll
+  for (int b = 0; b < CH_HELD; ++b) w[b][0] = w[b][1] = (ChFrag)(0u);
+  if (normed) {
+#pragma unroll
+    for (int t = 0; t < CH_TILES; ++t)
+      if (n0 + t * 16 < n_end)
+#pragma unroll
+        for (int b = 0; b < CH_LN_BLOCKS; ++b)
+          if (b < n_blocks) {
+            const char* at = held_weights + (t * kblocks + wave + CH_WAVES * b) * 2048 + lane * 16;
+            w[t * CH_LN_BLOCKS + b][0] = *(const ChFrag*)at, w[t * CH_LN_BLOCKS + b][1] = *(const ChFrag*)(at + 1024);
+          }
+    asm volatile("; weights of a normed product" ::: "memory");  // (the branches' ends differ: merged, w would be indexed by a variable)
+  } else {
+#pragma unroll
+    for (int b = 0; b < CH_PAIRS; ++b)
+      if (b < n_pairs) {
+        const char* at = held_weights + (wave + CH_WAVES * b) * 2048 + lane * 16;
+        w[b][0] = *(const ChFrag*)at, w[b][1] = *(const ChFrag*)(at + 1024);
+      }
+    asm volatile("; weights of a plain product" ::: "memory");
+  }
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+  __syncthreads();  // the copying waves go on with the next unit's
+
+  // ---- the rows, and the products ----------------------------------------------------------
+  int how = CH_THERE;
+  f32x4_t acc[CH_TILES];
+#pragma unroll
+  for (int t = 0; t < CH_TILES; ++t) acc[t] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+  if (normed) {
+    float x[R][CH_LN_BLOCKS];
+    if (first) {
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int b = 0; b < CH_LN_BLOCKS; ++b)
+          x[r][b] = b < n_blocks ? p.h[(size_t)r * p.ldh + (wave + CH_WAVES * b) * 64 + lane] : 0.f;
+    } else {
+      word_t in[R * CH_LN_BLOCKS];
+      const word_t* from = (kind == CH_QKV ? p.h2 : p.h1) + wave * 64;
+      how |= words_wait(in, n_blocks * R, tag - 1, patience, [&](int j) {  // (word j: row j % R of block j / R)
+        return word_load(from + ((j % R) * z.K + (j / R) * (CH_WAVES * 64)) + (uint32_t)lane);
+      });
+#pragma unroll
+      for (int r = 0; r < R; ++r)
+#pragma unroll
+        for (int b = 0; b < CH_LN_BLOCKS; ++b) x[r][b] = b < n_blocks ? f32_of(in[b * R + r]) : 0.f;
+    }
+    // The wave's own mean and squares around it, then all waves' joined in one exchange (squares around
+    // a wave's mean are as exact as around the row's): n (mean_w - mean)^2 comes on top.
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      float s = 0.f;
+#pragma unroll
+      for (int b = 0; b < CH_LN_BLOCKS; ++b) s += x[r][b];
+      s = wave_sum(s);
+      const float wmean = s * (n_blocks == 4 ? 0x1p-8f : n_blocks == 3 ? 1.f / 192.f : n_blocks == 2 ? 0x1p-7f : 0x1p-6f);
+      float qq = 0.f;
+#pragma unroll
+      for (int b = 0; b < CH_LN_BLOCKS; ++b) {
+        const float d = x[r][b] - wmean;
+        qq += b < n_blocks ? d * d : 0.f;
+      }
+      qq = wave_sum(qq);
+      if (lane == 0) sh.stat[r][wave] = make_float4(s, wmean, qq, (float)(n_blocks * 64));
+    }
+    meet(&sh.arrived, target, lane);
+    const float inv_k = 1.0f / (float)z.K;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const float4 st = sh.stat[r][lane & 7];
+      const float mean = group_sum<8>(st.x) * inv_k;
+      const float d = st.y - mean;
+      const float var = group_sum<8>(st.z + st.w * d * d) * inv_k + (kind == CH_QKV ? p.eps1 : p.eps2);
+      float rstd = __builtin_amdgcn_rsqf(var);
+      rstd = rstd * (1.5f - 0.5f * var * rstd * rstd);  // (the instruction is an ulp off, one step is not)
+#pragma unroll
+      for (int b = 0; b < CH_LN_BLOCKS; ++b)
+        if (b < n_blocks)
+          sh.xs[r][(wave + CH_WAVES * b) * 64 + lane] = f32_to_bf16_bits((x[r][b] - mean) * rstd * gm[b] + bt[b]);
+    }
+    // (a wave reads back only what it wrote itself)
+    const uint16_t* xr = sh.xs[min(lane & 15, R - 1)] + g * 16;
+#pragma unroll
+    for (int b = 0; b < CH_LN_BLOCKS; ++b) {
+      const int c = wave + CH_WAVES * b;
+      if (b < n_blocks) {
+        const ChFrag a0 = *(const ChFrag*)(xr + c * 64), a1 = *(const ChFrag*)(xr + c * 64 + 8);
+#pragma unroll
+        for (int t = 0; t < CH_TILES; ++t) {
+          acc[t] = mfma(w[t * CH_LN_BLOCKS + b][0], a0, acc[t]);
+          acc[t] = mfma(w[t * CH_LN_BLOCKS + b][1], a1, acc[t]);
+        }
+      }
+    }
+  } else {
+    // word 0: the stream's old value, wave 0's alone (complete long before the rows, and waited for all the same: its
+    // tag is made this one); then word j: row (j - 1) % R of pair (j - 1) / R
+    const int whole = short_pair && lane >= 32 ? n_pairs - 1 : n_pairs;  // pairs that this lane's words exist of
+    word_t in[R * CH_PAIRS + 1];
+    const word_t* from = (kind == CH_OUT ? p.att : p.act) + wave * 64;
+    const bool from_rows = kind == CH_OUT && layer == 0;
+    const size_t old_at = (size_t)min(o_m, R - 1) * z.N + min(n0 + o_f, z.N - 1);
+    if (wave == 0 && from_rows) old = p.h[(size_t)min(o_m, R - 1) * p.ldh + min(n0 + o_f, z.N - 1)];
+    how |= words_wait(in, whole * R + 1, tag - 1, patience, [&](int j) {
+      if (j > 0) return word_load(from + ((j - 1) % R * (z.K >> 1) + (j - 1) / R * (CH_WAVES * 64)) + (uint32_t)lane);
+      if (wave != 0 || from_rows) return (word_t)(tag - 1) << 32;
+      return kind == CH_OUT ? word_load(p.h2 + old_at) + ((word_t)2 << 32) : word_load(p.h1 + old_at) + ((word_t)1 << 32);
+    });
+    if (wave == 0 && !from_rows) old = f32_of(in[0]);
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+      for (int b = 0; b < CH_PAIRS; ++b)
+        if (b < whole) *(uint32_t*)(sh.xs[r] + (wave + CH_WAVES * b) * 128 + lane * 2) = (uint32_t)in[b * R + r + 1];
+    const int r = min(lane & 7, R - 1), second = (lane >> 3) & 1;
+#pragma unroll
+    for (int b = 0; b < CH_PAIRS; ++b) {
+      const int pair = wave + CH_WAVES * b;
+      if (pair < pairs) {
+        const bool repeats = odd && pair == pairs - 1 && second;
+        const uint16_t* from = sh.xs[r] + pair * 128 + (repeats ? 0 : second * 64) + g * 16;
+        ChFrag x0 = *(const ChFrag*)from, x1 = *(const ChFrag*)(from + 8);
+        if (repeats) x0 = x1 = (ChFrag)(0u);
+        acc[0] = mfma(w[b][0], x0, acc[0]);
+        acc[0] = mfma(w[b][1], x1, acc[0]);
+      }
+    }
+  }
+
+  // ---- the waves' tiles are added by wave 0 in a fixed order; element: row t / 16, feature t % 16 ----
+  // (only rows that are there are kept: column m, and for the pairs' second k-blocks column m + 8)
+#pragma unroll
+  for (int t = 0; t < CH_TILES; ++t)
+    if (t == 0 || n0 + t * 16 < n_end)
+      if ((lane & 7) < R)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) sh.red[t][wave][((lane >> 3 & 1) * R + (lane & 7)) * 16 + 4 * g + r] = acc[t][r];
+  if (lane == 0) sh.how[wave] = how;
+  meet(&sh.arrived, target, lane);
+  int worst = 0;
+#pragma unroll
+  for (int v = 0; v < CH_WAVES; ++v) worst |= sh.how[v];
+  worst = __builtin_amdgcn_readfirstlane(worst);
+  if (mine && worst == CH_THERE) {
+    if (!normed) {
+      float v = 0.f;
+#pragma unroll
+      for (int k = 0; k < CH_WAVES; ++k) v += sh.red[0][k][o_m * 16 + o_f] + sh.red[0][k][(o_m + R) * 16 + o_f + 8];
+      v = old + (v + bias.x);
+      if (last)
+        p.h_out[(size_t)o_m * p.ldh + n0 + o_f] = v;
+      else
+        word_store((kind == CH_OUT ? p.h1 : p.h2) + (size_t)o_m * z.N + n0 + o_f, v, tag);
+    } else {
+      const int tile = o_f >> 4, f = o_f & 15, n = n0 + o_f;
+      float v0 = 0.f, v1 = 0.f;
+#pragma unroll
+      for (int k = 0; k < CH_WAVES; ++k) v0 += sh.red[tile][k][o_m * 16 + f], v1 += sh.red[tile][k][o_m * 16 + f + 1];
+      v0 += bias.x, v1 += bias.y;
+      if (kind == CH_FC) v0 = gelu_tanh_fast(v0), v1 = gelu_tanh_fast(v1);
+      word_store((kind == CH_FC ? p.act : p.qkv) + (((size_t)o_m * z.N + n) >> 1), pack_bf16x2(v0, v1), tag);
+    }
+  }
+  return worst;
+}
+
+// A plan for a block that waited for `patience`, or came so late that its unit's places held a later product's words: every
+// phase's units, attention's too, are dealt among the blocks that run, counted again a layer, as others may come.  (Wave 0's.  Its
+// state lies in LDS: in registers it would cost the ordinary step 2 % at two rows.)
+template <int R>
+__device__ __forceinline__ void plan_anew(const ChainArgs& p, ChainShared<R>& sh, uint32_t tag_base, int& i, int& u, int lane) {
+  const int n_phases = p.n_layers * CH_KINDS;
+  int start = __builtin_amdgcn_readfirstlane(sh.anew.start), stride = __builtin_amdgcn_readfirstlane(sh.anew.stride);
+  int held_ph = __builtin_amdgcn_readfirstlane(sh.anew.held_ph), held_unit = __builtin_amdgcn_readfirstlane(sh.anew.held_unit);
+  const int help_i = __builtin_amdgcn_readfirstlane(sh.anew.help_i), help_u = __builtin_amdgcn_readfirstlane(sh.anew.help_u);
+  // The last phase's units stay their first owners': nobody would miss one.  (The first blocks are those with a second unit of
+  // a product, so the heads go to the last.)
+  const auto first_unit = [&](int at_i) {
+    if (at_i == n_phases - 1) return (int)blockIdx.x < p.product_blocks ? (int)blockIdx.x : 0x7fff;
+    return at_i % CH_KINDS == CH_ATTN ? stride - 1 - start : start;
+  };
+  const auto settle = [&](int& at_i, int& at_u) {  // to the next phase that has a unit of this block's
+    while (at_i < n_phases && at_u >= p.size[at_i % CH_KINDS].units) ++at_i, at_u = first_unit(at_i);
+  };
+  if (start >= 0) settle(i, u);
+  if (help_i < 0 && (start < 0 || (i < n_phases && i % CH_KINDS == CH_QKV && u == start))) {
+    if (start < 0) {  // a phase that has begun: those ahead of the one before it are whole
+      const word_t* words = lane == CH_QKV ? p.qkv : lane == CH_ATTN ? p.att : lane == CH_OUT ? p.h1 : lane == CH_FC ? p.act : p.h2;
+      int front = (int)(tag_of(word_load(words)) - tag_base);
+#pragma unroll
+      for (int d = 1; d < 8; d *= 2) front = max(front, __shfl_xor(front, d, 64));
+      i = max(__builtin_amdgcn_readfirstlane(front) - 1, 0);
+    }
+    int before = 0, here = 0;  // (the block's own word may still be on its way)
+    for (int b = 0; b < (int)gridDim.x; b += 64) {
+      const int of = b + lane;
+      const uint64_t runs = __ballot(of == (int)blockIdx.x || (of < (int)gridDim.x && tag_of(word_load(p.present + min(of, (int)gridDim.x - 1))) == tag_base));
+      here += __popcll(runs), before += __popcll(runs & __ballot(of < (int)blockIdx.x));
+    }
+    start = before, stride = here, u = first_unit(i);
+    settle(i, u);
+  }
+  int then_i = i, then_u = u;
+  if (help_i < 0) then_u += i != n_phases - 1 ? stride : p.product_blocks, settle(then_i, then_u);
+  const int ph = i >= n_phases ? -1 : help_i >= 0 ? help_i : i, unit = help_i >= 0 ? help_u : u;
+  const bool in_lds = ph == held_ph && unit == held_unit, copying = ph % CH_KINDS != CH_ATTN;
+  if (copying) {  // the next product's weights come meanwhile (a head's unit leaves them where they are)
+    held_ph = then_i, held_unit = then_u;
+    while (held_ph < n_phases && held_ph % CH_KINDS == CH_ATTN) held_unit += stride, settle(held_ph, held_unit);
+    if (held_ph >= n_phases) held_ph = -1;
+  }
+  if (lane == 0) {
+    sh.plan.ph = ph, sh.plan.unit = unit, sh.plan.held = in_lds;
+    sh.plan.then_ph = copying ? held_ph : -1, sh.plan.then_unit = held_unit;
+    sh.anew.start = start, sh.anew.stride = stride, sh.anew.held_ph = held_ph, sh.anew.held_unit = held_unit;
+  }
+}
+
 template <int R>
 __global__ __launch_bounds__(CH_ALL_WAVES * 64, 3) void decode_chain_kernel(ChainArgs p) {
   __shared__ ChainShared<R> sh;
-  extern __shared__ __attribute__((aligned(16))) char held_weights[];
-  const uint32_t lds = lds_address(held_weights), lds_small = lds_address(sh.small);
   bool held = false;  // the weights of the unit at hand are in LDS, or on their way
+  bool anew = false;  // dealt anew (plan_anew)
   const int n_phases = p.n_layers * CH_KINDS;
   const uint32_t tag_base = *p.tag_base;
-  uint32_t patience = p.patience;
   const bool attends = (int)blockIdx.x >= p.product_blocks;
   // this block's next unit: `u` of phase `i` (layer i / 5, kind i % 5)
   const int start = attends ? blockIdx.x - p.product_blocks : blockIdx.x;
   const int stride = attends ? p.attention_blocks : p.product_blocks;
   int i = attends ? CH_ATTN : CH_QKV, u = start;
-  int help_i = -1, help_u = 0;  // a missing unit done in its stead
+  const auto settle = [&] {  // to the next phase that has a unit of this block's
+    while (i < n_phases && u >= p.size[i % CH_KINDS].units) u = start, i += attends ? CH_KINDS : i % CH_KINDS == CH_QKV ? 2 : 1;
+  };
+  settle();
   uint32_t target = 0;  // of the computing waves' own barrier
-  if (threadIdx.x == 0) sh.arrived = 0;
+  if (threadIdx.x == 0) sh.arrived = 0, sh.plan.anew = 0, word_store(p.present + blockIdx.x, 0u, tag_base);
   for (;;) {
     // (made anew for every unit: what is computed from them would otherwise be kept in registers over the loop, 50 of them)
     int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     asm volatile("" : "+v"(lane), "+s"(wave));
     const bool copies = wave >= CH_WAVES;
-    if (wave == 0) {
-      const auto settle = [&](int& at_i, int& at_u) {  // to the next phase that has a unit of this block's
-        while (at_i < n_phases && at_u >= p.size[at_i % CH_KINDS].units)
-          at_u = start, at_i += attends ? CH_KINDS : at_i % CH_KINDS == CH_QKV ? 2 : 1;
-      };
-      settle(i, u);
-      int then_i = i, then_u = u;
-      if (help_i < 0) then_u += stride, settle(then_i, then_u);
-      if (lane == 0) {
-        sh.plan.ph = i >= n_phases ? -1 : help_i >= 0 ? help_i : i, sh.plan.unit = help_i >= 0 ? help_u : u, sh.plan.held = held;
-        sh.plan.then_ph = !attends && then_i < n_phases ? then_i : -1, sh.plan.then_unit = then_u;
-      }
-      held = !attends && then_i < n_phases;
+    if (wave == 0 && !anew) {
+      const int ph = i < n_phases ? i : -1, unit = u;
+      u += stride, settle();
+      const bool more = !attends && i < n_phases;
+      if (lane == 0) sh.plan.ph = ph, sh.plan.unit = unit, sh.plan.held = held, sh.plan.then_ph = more ? i : -1, sh.plan.then_unit = u;
+      held = more;
+    } else if (wave == 0) {
+      plan_anew<R>(p, sh, tag_base, i, u, lane);
     }
     if (copies) copies_arrived<0>();
     __syncthreads();
@@ -396,245 +673,48 @@ __global__ __launch_bounds__(CH_ALL_WAVES * 64, 3) void decode_chain_kernel(Chai
     const int then_ph = __builtin_amdgcn_readfirstlane(sh.plan.then_ph), then_unit = __builtin_amdgcn_readfirstlane(sh.plan.then_unit);
     const bool in_lds = __builtin_amdgcn_readfirstlane(sh.plan.held) != 0;
     if (ph < 0) break;
-    const int kind = ph % CH_KINDS, layer = ph / CH_KINDS;
-    const uint32_t tag = tag_base + ph;
+    const uint32_t patience = __builtin_amdgcn_readfirstlane(sh.plan.anew) ? min(p.patience, CH_PATIENCE_ANEW) : p.patience;
     int worst;
-    if (kind == CH_ATTN) {
-      worst = chain_attention<R>(p, sh, layer, unit, tag, patience, lane, wave);
+    if (ph % CH_KINDS == CH_ATTN) {
+      worst = chain_attention<R>(p, sh, ph / CH_KINDS, unit, tag_base + ph, patience, lane, wave);
       __syncthreads();
-      if (wave == 0) held = false;
-      if (copies) continue;
     } else {
-      if (!in_lds) {
-        if (copies) {
-          copy_unit(p, unit_of(p, ph, unit, wave), lds, lds_small, lane, wave - CH_WAVES);
-          copies_arrived<0>();
-        }
-        __syncthreads();
-      }
-      if (copies) {
-        __syncthreads();  // (the computing waves have read what lies in LDS)
-        if (then_ph >= 0) copy_unit(p, unit_of(p, then_ph, then_unit, wave), lds, lds_small, lane, wave - CH_WAVES);
-        continue;
-      }
-      const ChainUnit at_hand = unit_of(p, ph, unit, wave);
-      const ChainSize& z = p.size[kind];
-      const bool normed = at_hand.normed, first = ph == 0, last = ph == n_phases - 1;
-      const int g = lane >> 4, kblocks = at_hand.kblocks, pairs = at_hand.pairs, n_blocks = at_hand.n_blocks, n_pairs = at_hand.n_pairs;
-      const int n0 = at_hand.n0, n_end = at_hand.n_end;
-      const bool odd = kblocks & 1;  // the last pair has no second k-block: its lanes repeat the first, and count as zeros
-      const bool short_pair = odd && n_pairs > 0 && wave + CH_WAVES * (n_pairs - 1) == pairs - 1;
-
-      // ---- what the copying waves brought ---------------------------------------------------------
-      // wave 0 writes the outputs: one feature a lane into the stream, else two neighbours a lane
-      const int o_m = normed ? lane >> 4 : lane >> 3;
-      const int o_f = normed ? (lane & 15) * 2 : lane & 7;
-      const bool mine = wave == 0 && o_m < R && n0 + o_f < n_end;
-      float2 bias = make_float2(0.f, 0.f);
-      float old = 0.f;
-      if (wave == 0 && at_hand.ly->bias[at_hand.which]) bias.x = sh.small[CH_WAVES * 2][o_f], bias.y = sh.small[CH_WAVES * 2][o_f + 1];
-      float gm[CH_LN_BLOCKS], bt[CH_LN_BLOCKS];
-#pragma unroll
-      for (int b = 0; b < CH_LN_BLOCKS; ++b) gm[b] = sh.small[wave * 2][b * 64 + lane], bt[b] = sh.small[wave * 2 + 1][b * 64 + lane];
-      ChFrag w[CH_HELD][2];
-#pragma unroll
-      for (int b = 0; b < CH_HELD; ++b) w[b][0] = w[b][1] = (ChFrag)(0u);
-      if (normed) {
-#pragma unroll
-        for (int t = 0; t < CH_TILES; ++t)
-          if (n0 + t * 16 < n_end)
-#pragma unroll
-            for (int b = 0; b < CH_LN_BLOCKS; ++b)
-              if (b < n_blocks) {
-                const char* at = held_weights + (t * kblocks + wave + CH_WAVES * b) * 2048 + lane * 16;
-                w[t * CH_LN_BLOCKS + b][0] = *(const ChFrag*)at, w[t * CH_LN_BLOCKS + b][1] = *(const ChFrag*)(at + 1024);
-              }
-        asm volatile("; weights of a normed product" ::: "memory");  // (the branches' ends differ: merged, w would be indexed by a variable)
-      } else {
-#pragma unroll
-        for (int b = 0; b < CH_PAIRS; ++b)
-          if (b < n_pairs) {
-            const char* at = held_weights + (wave + CH_WAVES * b) * 2048 + lane * 16;
-            w[b][0] = *(const ChFrag*)at, w[b][1] = *(const ChFrag*)(at + 1024);
-          }
-        asm volatile("; weights of a plain product" ::: "memory");
-      }
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      __builtin_amdgcn_sched_barrier(0);
-      __syncthreads();  // the copying waves go on with the next unit's
-
-      // ---- the rows, and the products ----------------------------------------------------------
-      int how = CH_THERE;
-      f32x4_t acc[CH_TILES];
-#pragma unroll
-      for (int t = 0; t < CH_TILES; ++t) acc[t] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-      if (normed) {
-        float x[R][CH_LN_BLOCKS];
-        if (first) {
-#pragma unroll
-          for (int r = 0; r < R; ++r)
-#pragma unroll
-            for (int b = 0; b < CH_LN_BLOCKS; ++b)
-              x[r][b] = b < n_blocks ? p.h[(size_t)r * p.ldh + (wave + CH_WAVES * b) * 64 + lane] : 0.f;
-        } else {
-          word_t in[R * CH_LN_BLOCKS];
-          const word_t* from = (kind == CH_QKV ? p.h2 : p.h1) + wave * 64;
-          how |= words_wait(in, n_blocks * R, tag - 1, patience, [&](int j) {  // (word j: row j % R of block j / R)
-            return word_load(from + ((j % R) * z.K + (j / R) * (CH_WAVES * 64)) + (uint32_t)lane);
-          });
-#pragma unroll
-          for (int r = 0; r < R; ++r)
-#pragma unroll
-            for (int b = 0; b < CH_LN_BLOCKS; ++b) x[r][b] = b < n_blocks ? f32_of(in[b * R + r]) : 0.f;
-        }
-        // The wave's own mean and squares around it, then all waves' joined in one exchange (squares around
-        // a wave's mean are as exact as around the row's): n (mean_w - mean)^2 comes on top.
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-          float s = 0.f;
-#pragma unroll
-          for (int b = 0; b < CH_LN_BLOCKS; ++b) s += x[r][b];
-          s = wave_sum(s);
-          const float wmean = s * (n_blocks == 4 ? 0x1p-8f : n_blocks == 3 ? 1.f / 192.f : n_blocks == 2 ? 0x1p-7f : 0x1p-6f);
-          float qq = 0.f;
-#pragma unroll
-          for (int b = 0; b < CH_LN_BLOCKS; ++b) {
-            const float d = x[r][b] - wmean;
-            qq += b < n_blocks ? d * d : 0.f;
-          }
-          qq = wave_sum(qq);
-          if (lane == 0) sh.stat[r][wave] = make_float4(s, wmean, qq, (float)(n_blocks * 64));
-        }
-        meet(&sh.arrived, target, lane);
-        const float inv_k = 1.0f / (float)z.K;
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-          const float4 st = sh.stat[r][lane & 7];
-          const float mean = group_sum<8>(st.x) * inv_k;
-          const float d = st.y - mean;
-          const float var = group_sum<8>(st.z + st.w * d * d) * inv_k + (kind == CH_QKV ? p.eps1 : p.eps2);
-          float rstd = __builtin_amdgcn_rsqf(var);
-          rstd = rstd * (1.5f - 0.5f * var * rstd * rstd);  // (the instruction is an ulp off, one step is not)
-#pragma unroll
-          for (int b = 0; b < CH_LN_BLOCKS; ++b)
-            if (b < n_blocks)
-              sh.xs[r][(wave + CH_WAVES * b) * 64 + lane] = f32_to_bf16_bits((x[r][b] - mean) * rstd * gm[b] + bt[b]);
-        }
-        // (a wave reads back only what it wrote itself)
-        const uint16_t* xr = sh.xs[min(lane & 15, R - 1)] + g * 16;
-#pragma unroll
-        for (int b = 0; b < CH_LN_BLOCKS; ++b) {
-          const int c = wave + CH_WAVES * b;
-          if (b < n_blocks) {
-            const ChFrag a0 = *(const ChFrag*)(xr + c * 64), a1 = *(const ChFrag*)(xr + c * 64 + 8);
-#pragma unroll
-            for (int t = 0; t < CH_TILES; ++t) {
-              acc[t] = mfma(w[t * CH_LN_BLOCKS + b][0], a0, acc[t]);
-              acc[t] = mfma(w[t * CH_LN_BLOCKS + b][1], a1, acc[t]);
-            }
-          }
-        }
-      } else {
-        // word 0: the stream's old value, wave 0's alone (complete long before the rows, and waited for all the same: its
-        // tag is made this one); then word j: row (j - 1) % R of pair (j - 1) / R
-        const int whole = short_pair && lane >= 32 ? n_pairs - 1 : n_pairs;  // pairs that this lane's words exist of
-        word_t in[R * CH_PAIRS + 1];
-        const word_t* from = (kind == CH_OUT ? p.att : p.act) + wave * 64;
-        const bool from_rows = kind == CH_OUT && layer == 0;
-        const size_t old_at = (size_t)min(o_m, R - 1) * z.N + min(n0 + o_f, z.N - 1);
-        if (wave == 0 && from_rows) old = p.h[(size_t)min(o_m, R - 1) * p.ldh + min(n0 + o_f, z.N - 1)];
-        how |= words_wait(in, whole * R + 1, tag - 1, patience, [&](int j) {
-          if (j > 0) return word_load(from + ((j - 1) % R * (z.K >> 1) + (j - 1) / R * (CH_WAVES * 64)) + (uint32_t)lane);
-          if (wave != 0 || from_rows) return (word_t)(tag - 1) << 32;
-          return kind == CH_OUT ? word_load(p.h2 + old_at) + ((word_t)2 << 32) : word_load(p.h1 + old_at) + ((word_t)1 << 32);
-        });
-        if (wave == 0 && !from_rows) old = f32_of(in[0]);
-#pragma unroll
-        for (int r = 0; r < R; ++r)
-#pragma unroll
-          for (int b = 0; b < CH_PAIRS; ++b)
-            if (b < whole) *(uint32_t*)(sh.xs[r] + (wave + CH_WAVES * b) * 128 + lane * 2) = (uint32_t)in[b * R + r + 1];
-        const int r = min(lane & 7, R - 1), second = (lane >> 3) & 1;
-#pragma unroll
-        for (int b = 0; b < CH_PAIRS; ++b) {
-          const int pair = wave + CH_WAVES * b;
-          if (pair < pairs) {
-            const bool repeats = odd && pair == pairs - 1 && second;
-            const uint16_t* from = sh.xs[r] + pair * 128 + (repeats ? 0 : second * 64) + g * 16;
-            ChFrag x0 = *(const ChFrag*)from, x1 = *(const ChFrag*)(from + 8);
-            if (repeats) x0 = x1 = (ChFrag)(0u);
-            acc[0] = mfma(w[b][0], x0, acc[0]);
-            acc[0] = mfma(w[b][1], x1, acc[0]);
-          }
-        }
-      }
-
-      // ---- the waves' tiles are added by wave 0 in a fixed order; element: row t / 16, feature t % 16 ----
-      // (only rows that are there are kept: column m, and for the pairs' second k-blocks column m + 8)
-#pragma unroll
-      for (int t = 0; t < CH_TILES; ++t)
-        if (t == 0 || n0 + t * 16 < n_end)
-          if ((lane & 7) < R)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) sh.red[t][wave][((lane >> 3 & 1) * R + (lane & 7)) * 16 + 4 * g + r] = acc[t][r];
-      if (lane == 0) sh.how[wave] = how;
-      meet(&sh.arrived, target, lane);
-      worst = 0;
-#pragma unroll
-      for (int v = 0; v < CH_WAVES; ++v) worst |= sh.how[v];
-      worst = __builtin_amdgcn_readfirstlane(worst);
-      if (mine && worst == CH_THERE) {
-        if (!normed) {
-          float v = 0.f;
-#pragma unroll
-          for (int k = 0; k < CH_WAVES; ++k) v += sh.red[0][k][o_m * 16 + o_f] + sh.red[0][k][(o_m + R) * 16 + o_f + 8];
-          v = old + (v + bias.x);
-          if (last)
-            p.h_out[(size_t)o_m * p.ldh + n0 + o_f] = v;
-          else
-            word_store((kind == CH_OUT ? p.h1 : p.h2) + (size_t)o_m * z.N + n0 + o_f, v, tag);
-        } else {
-          const int tile = o_f >> 4, f = o_f & 15, n = n0 + o_f;
-          float v0 = 0.f, v1 = 0.f;
-#pragma unroll
-          for (int k = 0; k < CH_WAVES; ++k) v0 += sh.red[tile][k][o_m * 16 + f], v1 += sh.red[tile][k][o_m * 16 + f + 1];
-          v0 += bias.x, v1 += bias.y;
-          if (kind == CH_FC) v0 = gelu_tanh_fast(v0), v1 = gelu_tanh_fast(v1);
-          word_store((kind == CH_FC ? p.act : p.qkv) + (((size_t)o_m * z.N + n) >> 1), pack_bf16x2(v0, v1), tag);
-        }
-      }
+      worst = chain_product<R>(p, sh, ph, unit, in_lds, then_ph, then_unit, tag_base + ph, patience, target, lane, wave);
     }
-    if (worst != CH_MISSING) {
-      // (done, or somebody else's so long ago that later words lie in its place; a block that helped has its own unit's
-      // weights to ask for again)
-      if (help_i < 0) u += stride; else held = false;
-      help_i = -1;
+    if (copies) continue;
+    if (!anew) {
+      if (worst == CH_THERE) continue;
+      anew = true;
+      if (threadIdx.x == 0) sh.anew.start = -1, sh.anew.help_i = -1, sh.anew.held_ph = -1, sh.plan.anew = 1;
       continue;
     }
-    // Somebody's unit is missing: back to the last phase that lacks nothing, and of the one after it a
-    // missing unit from this block's place on.  Whoever had to look once waits less from then on.
-    patience = min(patience, 400u);
-    help_i = -1;
-    held = false;
+    if (worst != CH_MISSING) {  // (done, or somebody else's long ago: later words lie in the places that it reads)
+      if (wave == 0 && __builtin_amdgcn_readfirstlane(sh.anew.help_i) < 0)
+        u += i != n_phases - 1 ? __builtin_amdgcn_readfirstlane(sh.anew.stride) : p.product_blocks;
+      if (threadIdx.x == 0) sh.anew.help_i = -1;
+      continue;
+    }
+    // Somebody's unit is missing: back to the last phase that lacks nothing, and of the one after it one missing unit, a
+    // different one from block to block (the next after a block's own number was the same one for all that looked).
+    if (threadIdx.x == 0) sh.anew.help_i = -1;
     for (int q = ph - 1; q >= 0; --q) {
       const int qk = q % CH_KINDS;
       const ChainSize zq = p.size[qk];
       const bool pairs_of = qk != CH_OUT && qk != CH_PROJ;
       const int per = (qk == CH_ATTN ? p.q_width : zq.N) >> (pairs_of ? 1 : 0);
       const word_t* words = qk == CH_QKV ? p.qkv : qk == CH_ATTN ? p.att : qk == CH_OUT ? p.h1 : qk == CH_FC ? p.act : p.h2;
-      const int turn = (int)(blockIdx.x % (unsigned)zq.units);
-      if (threadIdx.x == 0) sh.missing = 0x7fffffff;
+      if (threadIdx.x == 0) sh.missing = 0xffffffffu;
       meet(&sh.arrived, target, lane);
       for (int j = threadIdx.x; j < per * R; j += CH_WAVES * 64) {
         if (tag_of(word_load(words + j)) >= tag_base + q) continue;
         const int of = qk == CH_ATTN ? (j / per) * p.n_heads + (j % per) * 2 / CH_HEAD : (j % per) * (pairs_of ? 2 : 1) / zq.features;
-        atomicMin(&sh.missing, (of - turn + zq.units) % zq.units);
+        atomicMin(&sh.missing, (((uint32_t)of * 0x9e3779b1u + blockIdx.x * 0x85ebca6bu) * 0xc2b2ae35u & ~(CH_UNITS_MOST - 1u)) | (uint32_t)of);
       }
       meet(&sh.arrived, target, lane);
-      const int found = __builtin_amdgcn_readfirstlane(sh.missing);
+      const uint32_t found = __builtin_amdgcn_readfirstlane(sh.missing);
       meet(&sh.arrived, target, lane);
-      if (found == 0x7fffffff) break;
-      help_i = q, help_u = (found + turn) % zq.units;
+      if (found == 0xffffffffu) break;
+      if (threadIdx.x == 0) sh.anew.help_i = q, sh.anew.help_u = found & (CH_UNITS_MOST - 1);
     }
   }
 }
@@ -701,16 +781,17 @@ extern "C" int decode_chain_takes(const ChainDims* d, int rows) {
   return deal_of(d, rows, &deal) ? 1 : 0;
 }
 
-// The launch's memory: the tag, then the words of each product in turn.
-static size_t words_of(const ChainDims* d, int rows, size_t (&at)[CH_KINDS]) {
+// The launch's memory: the tag, then the words of each product in turn, then the blocks'.
+static size_t words_of(const ChainDims* d, int rows, size_t (&at)[CH_KINDS + 1]) {
   const int q_width = d->n_heads * CH_HEAD, kv_width = d->n_kv_heads * CH_HEAD;
   const size_t n[CH_KINDS] = {(size_t)(q_width + 2 * kv_width) / 2, (size_t)q_width / 2, (size_t)d->width, (size_t)d->inner / 2, (size_t)d->width};
   size_t total = 32;
   for (int i = 0; i < CH_KINDS; ++i) at[i] = total, total += (n[i] * rows + 31) / 32 * 32;
-  return total;
+  at[CH_KINDS] = total;
+  return total + n_compute_units();
 }
 extern "C" size_t decode_chain_bytes(const ChainDims* d, int rows) {
-  size_t at[CH_KINDS];
+  size_t at[CH_KINDS + 1];
   return words_of(d, rows, at) * sizeof(word_t);
 }
 
@@ -723,7 +804,7 @@ extern "C" int decode_chain(const ChainDims* d, int rows, const void* layers, vo
   ChainDeal deal;
   deal_of(d, rows, &deal);
   ChainArgs a = {};
-  size_t at[CH_KINDS];
+  size_t at[CH_KINDS + 1];
   const size_t n_words = words_of(d, rows, at);
   word_t* words = (word_t*)memory;
   a.layers = (const ChainLayer*)layers, a.n_layers = d->n_layers;
@@ -737,6 +818,7 @@ extern "C" int decode_chain(const ChainDims* d, int rows, const void* layers, vo
   a.eps1 = d->eps1, a.eps2 = d->eps2, a.scale = d->scale * 1.4426950408889634f;
   a.h = h, a.h_out = h_out, a.ldh = ldh;
   a.qkv = words + at[CH_QKV], a.att = words + at[CH_ATTN], a.h1 = words + at[CH_OUT], a.act = words + at[CH_FC], a.h2 = words + at[CH_PROJ];
+  a.present = words + at[CH_KINDS];
   a.n_heads = d->n_heads, a.n_kv_heads = d->n_kv_heads, a.q_width = d->n_heads * CH_HEAD, a.kv_width = d->n_kv_heads * CH_HEAD;
   a.page_size = d->page_size, a.page_stride = d->page_stride;
   a.block_table = block_table, a.max_blocks = max_blocks, a.token_req = token_req, a.positions = positions;

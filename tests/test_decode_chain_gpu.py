@@ -55,9 +55,18 @@ CASES = [
     (2, 192, 448, 3, 3, 16, (40, 3), 1, 10),
     (2, 1280, 5120, 20, 20, 16, (100, 500), 100, 100),
 ]
+# ... and units dealt anew among the blocks that run, from the first wait on: all of them (there are more than a product's units,
+# or fewer), and five, of which one began as attention's
+CASES += [
+    (3, 64, 192, 2, 1, 8, (7, 8), 0, 1),
+    (2, 832, 3328, 13, 13, 16, (300,), 0, 1),
+    (3, 1600, 6400, 25, 25, 16, (700, 1001), 0, 1),
+    (1, 2048, 7168, 32, 8, 16, (64,), 0, 1),
+    (3, 768, 3072, 12, 12, 16, (93, 20), 5, 1),
+]
 
 
-@pytest.mark.parametrize("case", CASES, ids=lambda c: f"{c[1]}x{c[2]}-{'+'.join(map(str, c[6]))}{f'-{c[7]}blocks' if c[7] else ''}")
+@pytest.mark.parametrize("case", CASES, ids=lambda c: f"{c[1]}x{c[2]}-{'+'.join(map(str, c[6]))}{f'-{c[7]}blocks' if c[7] else ''}{'-anew' if c[8] == 1 else ''}")
 def test_layers_of_a_decode_step_in_one_launch(case):
     n_layers, D, I, H, HK, page, keys, blocks, patience = case
     lib, R, Q, KV = _lib(), len(case[6]), case[3] * 64, case[4] * 64
