@@ -766,6 +766,11 @@ static bool deal_of(const ChainDims* d, int rows, ChainDeal* deal) {
       if (fixed + held > CH_LDS_MOST) z.features = 16, held = (size_t)kb * 2048;
     }
     z.units = (z.N + z.features - 1) / z.features;
+    // Two rows of width 1,664 and more leave LDS for 16 features a unit only, and blocks with two units a product wait for both
+    // (us a step of 12 layers at 3 / 500 / 1,000 keys, here against each layer's launches: width 1,728 of inner size 6,784 558 /
+    // 563 / 570 against 474 / 513 / 532, width 2,048 of 2,048 432 / 438 / 444 against 417 / 450 / 469; width 1,600 316 / 319 /
+    // 328 against 455 / 494 / 513).  One row is ahead there too (2,048 of 6,656: 450 / 454 / 460 against 502 / 529 / 563).
+    if (rows > 1 && (i == CH_QKV || i == CH_FC) && z.units > products) return false;
     if (held > deal->lds) deal->lds = held;
   }
   return fixed + deal->lds <= CH_LDS_MOST;

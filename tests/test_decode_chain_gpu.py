@@ -151,7 +151,8 @@ def test_layers_of_a_decode_step_in_one_launch(case):
             assert torch.equal(a, b)
 
 
-@pytest.mark.parametrize("change", [dict(width=96), dict(width=2112), dict(inner=7232), dict(n_kv_heads=3), dict(n_layers=0), dict(rows=3)],
+@pytest.mark.parametrize("change", [dict(width=96), dict(width=2112), dict(inner=7232), dict(n_kv_heads=3), dict(n_layers=0), dict(rows=3),
+                                    dict(width=1664, inner=6656, n_heads=26, n_kv_heads=26, rows=2)],
                          ids=lambda c: next(iter(c)) + str(next(iter(c.values()))))
 def test_sizes_the_one_launch_does_not_take(change):
     sizes = dict(n_layers=2, width=128, inner=256, n_heads=2, n_kv_heads=2, page_size=16, rows=1)
@@ -227,3 +228,10 @@ def test_tags_where_their_bits_end():
         bases.append(memory[0].item() & 0xFFFFFFFF)
     turn = next(i for i, b in enumerate(bases) if b == 6)
     assert bases == [0xFFFFFFFF - 2 * 0x10000 - 13 + 6 * (i + 1) for i in range(turn)] + [6 * (i + 1) for i in range(6 - turn)] and 0 < turn < 5
+
+
+@pytest.mark.parametrize("width,rows", [(1664, 1), (2048, 1), (1600, 2), (64, 2)])
+def test_widest_sizes_the_one_launch_takes(width, rows):
+    """Two rows only where every block has one unit of a product: two units a block are slower than each layer's launches."""
+    d = Dims(2, width, min(4 * width, 6656), width // 64, width // 64, 16, width * 16, 1e-5, 1e-5, 0.125)
+    assert _lib().decode_chain_takes(ctypes.byref(d), rows) == 1
