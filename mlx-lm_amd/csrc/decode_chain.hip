@@ -40,6 +40,8 @@
 // keys pays for the first wait: 253 / 491 / 567 / 1,095 against 349 / 340 / 370 / 609.  (Blocks of twelve waves of
 // 168 registers leave no room beside them: two engines' steps on two streams follow each other, a pair of XL steps 1,999
 // against 2,266; beside an XL step of 8 rows the step of one row takes 989 instead of 2,384, and the pair 3,094 instead of 2,722.)
+#include <atomic>
+
 #include "decode_chain.h"
 #include "lds_copy.h"
 
@@ -57,6 +59,7 @@
 #define CH_KEY_TILES ((CHAIN_MOST_KEYS + CH_ALL_WAVES * 8 - 1) / (CH_ALL_WAVES * 8))  // loads of 8 keys a wave holds
 
 #define CH_LDS_MOST (160 * 1024)
+#define CH_DEVICES 64  // whose grants of LDS are remembered (others ask at each launch)
 // Ticks of 10 ns.  200 us: some five times the longest wait of any size (a head's, for a layer of width
 // 2,048, 38 us); 100 and 60 were 0.1 ms better for held compute units and worse beside short kernels, whose places come free
 // (XL beside large products, nine steps of ten within 1.4 ms, then 1.75 and 1.9).  Dealt anew, a wait is a phase's, and 30 us
@@ -828,11 +831,15 @@ extern "C" int decode_chain(const ChainDims* d, int rows, const void* layers, vo
   a.page_size = d->page_size, a.page_stride = d->page_stride;
   a.block_table = block_table, a.max_blocks = max_blocks, a.token_req = token_req, a.positions = positions;
   const void* kernel = rows == 1 ? (const void*)decode_chain_kernel<1> : (const void*)decode_chain_kernel<2>;
-  static size_t granted[CHAIN_MOST_ROWS] = {0, 0};
-  if (granted[rows - 1] < deal.lds) {
-    hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)deal.lds);
-    if (e != hipSuccess) FAIL("decode_chain: cannot get %zu bytes of LDS: %s", deal.lds, hipGetErrorString(e));
-    granted[rows - 1] = deal.lds;
+  // (granted a device at a time: one process may hold engines on several; and always the most, as threads may grant side by side)
+  static std::atomic<bool> granted[CH_DEVICES][CHAIN_MOST_ROWS];
+  int device = 0;
+  if (hipGetDevice(&device) != hipSuccess || device < 0) FAIL("decode_chain: no current device");
+  if (device >= CH_DEVICES || !granted[device][rows - 1]) {
+    const int most = CH_LDS_MOST - (int)(rows == 1 ? sizeof(ChainShared<1>) : sizeof(ChainShared<2>));
+    hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, most);
+    if (e != hipSuccess) FAIL("decode_chain: cannot get %d bytes of LDS: %s", most, hipGetErrorString(e));
+    if (device < CH_DEVICES) granted[device][rows - 1] = true;
   }
   hipLaunchKernelGGL(chain_step_kernel, dim3(1), dim3(256), 0, stream, (uint32_t*)memory, (uint32_t)(d->n_layers * CH_KINDS + 1),
                      words + at[0], (int)(n_words - at[0]));
