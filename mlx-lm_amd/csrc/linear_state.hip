@@ -411,7 +411,7 @@ __global__ __launch_bounds__(256) void state_chunks_kernel(ScanArgs a, int C, Sp
 template <typename T>
 __global__ __launch_bounds__(CHANNEL_THREADS) void channel_chunks_kernel(ScanArgs a, int C, int PS, SpanArgs sp) {
   constexpr int NT = CHANNEL_THREADS, NW = NT / 64;
-  extern __shared__ float lds[];
+  extern __shared__ __attribute__((aligned(16))) float lds[];  // (the running sum takes four floats at a time)
   __shared__ float Rs[64];
   __shared__ unsigned char pair_t[136], pair_j[136];
   const int N = a.N, P = a.P, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
