@@ -400,32 +400,38 @@ __global__ __launch_bounds__(256) void state_chunks_kernel(ScanArgs a, int C, Sp
 // With a bonus the queries read the state ahead of their own token: their side of every exponent is
 // L_(t-1) (zero at the chunk's first token), still <= 0 against L_j for j < t and against L_b, and
 // a pair (t, t) has the bonus in place of an exponential.
-// What bounds it: a chunk is a chain of short phases (loads, running sums, tiles, products) with barriers between, and one
-// block's LDS leaves room for no second block on a compute unit, so only the block's own waves cover a
-// phase's latency.  A span's launch for its end state / for its outputs (us, 8 prompts of 40 to 300 tokens, 16 heads of 64 x 64): 56 / 135 with
-// four waves, 36 / 81 with eight, rows of LDS four floats longer than P (neighbouring rows shared their banks), the
-// channels of a pair interleaved over its lanes and the running sum taken eight tokens a trip; 38 / 76 with sixteen waves,
-// whose 128 registers a thread spill 21.
-#define CHANNEL_THREADS 512
-#define CHANNEL_AHEAD (4096 / CHANNEL_THREADS)  // loads of each operand that a thread has on their way: a chunk of 64 x 64 in one trip
-template <typename T>
-__global__ __launch_bounds__(CHANNEL_THREADS) void channel_chunks_kernel(ScanArgs a, int C, int PS, SpanArgs sp) {
-  constexpr int NT = CHANNEL_THREADS, NW = NT / 64;
+// What bounds it: a chunk is a chain of short phases (loads, running sums, tiles, products) with barriers between.  Where one
+// block's LDS leaves room for no second block on a compute unit, only the block's own waves cover a phase's latency: a span's
+// launch for its end state / for its outputs took (us, 8 prompts of 40 to 300 tokens, 16 heads of 64 x 64) 56 / 135 with four
+// waves and takes 36 / 81 with eight, the channels of a pair interleaved over its lanes and the running sum taken eight tokens a trip;
+// 38 / 76 with sixteen waves, whose 128 registers a thread spill 21.  Where LDS has room for two, the registers of eight
+// waves (160 a thread) still keep a compute unit to one block, those of four (212) to two that cover each other: four waves then, if
+// there are more blocks than compute units.  All launches of a call (us), four / eight waves:
+//   heads x state     64 prompts of 20 tokens    8 prompts in spans of 64     8 whole
+//   16 of 16 x 16         57 /  71                   54 /  63               144 /  89 (128 blocks: one a compute unit)
+//    8 of 32 x 32         43 /  49                   61 /  43 (152 blocks)  197 / 119
+//   64 of 32 x 32        310 / 378                  219 / 256               214 / 191
+//   16 of 48 x 48        204 / 128                  152 / 102               266 / 162 (LDS for one block)
+//   16 of 64 x 64        255 / 157                  185 / 122               325 / 196 (the same)
+// (Rows of LDS four floats longer than P, so that neighbouring rows do not share their banks, measured the same everywhere.)
+template <typename T, int NT>
+__global__ __launch_bounds__(NT) void channel_chunks_kernel(ScanArgs a, int C, SpanArgs sp) {
+  constexpr int NW = NT / 64, CHANNEL_AHEAD = 4096 / NT;  // loads of each operand that a thread has on their way: a chunk of 64 x 64 in one trip
   extern __shared__ __attribute__((aligned(16))) float lds[];  // (the running sum takes four floats at a time)
   __shared__ float Rs[64];
   __shared__ unsigned char pair_t[136], pair_j[136];
   const int N = a.N, P = a.P, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int Np = (N + 15) & ~15, Pp = (P + 15) & ~15, CP = C + 4;  // (PS: a row of V, O and S, channel_row_floats)
+  const int Np = (N + 15) & ~15, Pp = (P + 15) & ~15, CP = C + 4;
   const int h = blockIdx.x;
   const int r = sp.mode == WHOLE ? blockIdx.y : sp.span_req[blockIdx.y];
   float* QT = lds;
   float* KT = QT + (size_t)Np * CP;
   float* LT = KT + (size_t)Np * CP;
   float* V = LT + (size_t)Np * CP;
-  float* O = V + (size_t)C * PS;
-  float* AT = O + (size_t)C * PS;
+  float* O = V + (size_t)C * Pp;
+  float* AT = O + (size_t)C * Pp;
   float* S = AT + (size_t)C * CP;
-  float* Lsum = S + (size_t)Np * PS;  // [Np] the log decay of every channel over the span so far
+  float* Lsum = S + (size_t)Np * Pp;  // [Np] the log decay of every channel over the span so far
   const int start = a.seq_start[r];
   const int lo = sp.mode == WHOLE ? 0 : sp.span_start[blockIdx.y];
   const int n = sp.mode == WHOLE ? a.seq_len[r] : min(a.seq_len[r], lo + sp.span);
@@ -441,7 +447,7 @@ __global__ __launch_bounds__(CHANNEL_THREADS) void channel_chunks_kernel(ScanArg
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
       const int i = base + u * NT + tid;
-      if (i < Np * Pp) S[(size_t)(i / Pp) * PS + i % Pp] = i / Pp < N && i % Pp < P ? sv[u] : 0.f;
+      if (i < Np * Pp) S[i] = i / Pp < N && i % Pp < P ? sv[u] : 0.f;
     }
   }
   for (int i = tid; i < Np; i += NT) Lsum[i] = 0.f;
@@ -496,7 +502,7 @@ __global__ __launch_bounds__(CHANNEL_THREADS) void channel_chunks_kernel(ScanArg
           }
           if (e < v_total) {
             const int t = e / P;
-            V[(size_t)t * PS + (e - t * P)] = t < m ? vv[u] : 0.f;
+            V[(size_t)t * Pp + (e - t * P)] = t < m ? vv[u] : 0.f;
           }
         }
       }
@@ -504,7 +510,7 @@ __global__ __launch_bounds__(CHANNEL_THREADS) void channel_chunks_kernel(ScanArg
         const int t = e / (Np - N), i = N + e % (Np - N);
         QT[(size_t)i * CP + t] = 0.f, KT[(size_t)i * CP + t] = 0.f, LT[(size_t)i * CP + t] = 0.f;
       }
-      for (int e = tid; e < C * (Pp - P); e += NT) V[(size_t)(e / (Pp - P)) * PS + P + e % (Pp - P)] = 0.f;
+      for (int e = tid; e < C * (Pp - P); e += NT) V[(size_t)(e / (Pp - P)) * Pp + P + e % (Pp - P)] = 0.f;
     }
     __syncthreads();
     for (int i = tid; i < N; i += NT) {  // a channel's running sum, token after token, eight on their way at a time
@@ -571,11 +577,11 @@ __global__ __launch_bounds__(CHANNEL_THREADS) void channel_chunks_kernel(ScanArg
       f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
       const int j_end = min((m + 3) & ~3, t0 + 16);
       for (int j = 0; j < j_end; j += 4)
-        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(AT[(size_t)(j + lg) * CP + t0 + lr], V[(size_t)(j + lg) * PS + p0 + lr], acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(AT[(size_t)(j + lg) * CP + t0 + lr], V[(size_t)(j + lg) * Pp + p0 + lr], acc, 0, 0, 0);
       for (int i = 0; i < Np; i += 4)
-        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(QT[(size_t)(i + lg) * CP + t0 + lr], S[(size_t)(i + lg) * PS + p0 + lr], acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(QT[(size_t)(i + lg) * CP + t0 + lr], S[(size_t)(i + lg) * Pp + p0 + lr], acc, 0, 0, 0);
 #pragma unroll
-      for (int x = 0; x < 4; ++x) O[(size_t)(t0 + 4 * lg + x) * PS + p0 + lr] = acc[x];
+      for (int x = 0; x < 4; ++x) O[(size_t)(t0 + 4 * lg + x) * Pp + p0 + lr] = acc[x];
     }
     __syncthreads();
     // S[i][:] = exp(L_C[i]) S[i][:] + sum_j KT[i][j] V[j][:]
@@ -584,11 +590,11 @@ __global__ __launch_bounds__(CHANNEL_THREADS) void channel_chunks_kernel(ScanArg
       f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
       const int j_end = (m + 3) & ~3;
       for (int j = 0; j < j_end; j += 4)
-        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(KT[(size_t)(i0 + lr) * CP + j + lg], V[(size_t)(j + lg) * PS + p0 + lr], acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(KT[(size_t)(i0 + lr) * CP + j + lg], V[(size_t)(j + lg) * Pp + p0 + lr], acc, 0, 0, 0);
 #pragma unroll
       for (int x = 0; x < 4; ++x) {
         const int i = i0 + 4 * lg + x;
-        float* sp_ = S + (size_t)i * PS + p0 + lr;
+        float* sp_ = S + (size_t)i * Pp + p0 + lr;
         *sp_ = expf(LT[(size_t)i * CP + C - 1]) * *sp_ + acc[x];
       }
     }
@@ -596,7 +602,7 @@ __global__ __launch_bounds__(CHANNEL_THREADS) void channel_chunks_kernel(ScanArg
     if (outputs && a.unit_rms)
       for (int t = wave; t < m; t += NW) {
         float ss = 0.f;
-        for (int pc = lane; pc < P; pc += 64) ss += O[(size_t)t * PS + pc] * O[(size_t)t * PS + pc];
+        for (int pc = lane; pc < P; pc += 64) ss += O[(size_t)t * Pp + pc] * O[(size_t)t * Pp + pc];
         ss = wave_sum(ss);
         if (lane == 0) Rs[t] = 1.0f / sqrtf(ss / (float)P + a.eps);
       }
@@ -606,7 +612,7 @@ __global__ __launch_bounds__(CHANNEL_THREADS) void channel_chunks_kernel(ScanArg
       for (int u = 0; u < 64 / NW; ++u) {
         const int t = wave + NW * u;
         if (t >= m || lane >= P) continue;
-        float o = O[(size_t)t * PS + lane];
+        float o = O[(size_t)t * Pp + lane];
         if (a.unit_rms) o *= Rs[t] * nw;
         if (a.gate) o *= silu_f(gv[u]);
         ((T*)a.out)[(row0 + t) * a.ldo + (size_t)h * P + lane] = from_f32<T>(o);
@@ -624,7 +630,7 @@ __global__ __launch_bounds__(CHANNEL_THREADS) void channel_chunks_kernel(ScanArg
           for (int u = 0; u < 8; ++u) {
             const int t = tb + NW * u;
             if (t >= m || pb + lane >= P) continue;
-            float o = O[(size_t)t * PS + pc];
+            float o = O[(size_t)t * Pp + pc];
             if (a.unit_rms) o *= Rs[t] * nw;
             if (a.gate) o *= silu_f(g8[u]);
             ((T*)a.out)[(row0 + t) * a.ldo + (size_t)h * P + pc] = from_f32<T>(o);
@@ -635,7 +641,7 @@ __global__ __launch_bounds__(CHANNEL_THREADS) void channel_chunks_kernel(ScanArg
   }
   __syncthreads();
   if (sp.mode == SPAN_OUTPUTS) return;
-  for (int i = tid; i < N * P; i += NT) Sg[i] = S[(size_t)(i / P) * PS + i % P];
+  for (int i = tid; i < N * P; i += NT) Sg[i] = S[(size_t)(i / P) * Pp + i % P];
   if (sp.mode == SPAN_STATES)  // (span_decay has a value for every channel here)
     for (int i = tid; i < N; i += NT) sp.span_decay[((size_t)blockIdx.y * a.H + h) * N + i] = expf(Lsum[i]);
 }
@@ -789,20 +795,14 @@ static size_t chunk_floats(int N, int P, int C) {
   const size_t Np = (N + 15) & ~15, Pp = (P + 15) & ~15, CP = C + 4;
   return 2 * Np * CP + (size_t)C * Np + 2 * (size_t)C * Pp + (size_t)C * CP + Np * Pp;
 }
-// The same for the kernel with a decay per key channel, where rows of P values lie PS floats apart.
-static size_t channel_chunk_floats(int N, int PS, int C) {
-  const size_t Np = (N + 15) & ~15, CP = C + 4;
-  return 3 * Np * CP + 2 * (size_t)C * PS + (size_t)C * CP + Np * PS + Np;
-}
-// PS: rows four banks apart, unless just that makes chunks of C tokens too many for the LDS (a shorter chunk, or none, costs more
-// than the rows' shared banks).
-static int channel_row_floats(int N, int P, int C) {
-  const int Pp = (P + 15) & ~15;
-  return channel_chunk_floats(N, Pp + 4, C) * sizeof(float) <= SCAN_MAX_LDS ? Pp + 4 : Pp;
+// The same for the kernel with a decay per key channel.
+static size_t channel_chunk_floats(int N, int P, int C) {
+  const size_t Np = (N + 15) & ~15, Pp = (P + 15) & ~15, CP = C + 4;
+  return 3 * Np * CP + 2 * (size_t)C * Pp + (size_t)C * CP + Np * Pp + Np;
 }
 // Bytes of LDS of chunks of C tokens.
 static size_t chunk_bytes(bool by_channel, int N, int P, int C) {
-  return (by_channel ? channel_chunk_floats(N, channel_row_floats(N, P, C), C) : chunk_floats(N, P, C)) * sizeof(float);
+  return (by_channel ? channel_chunk_floats(N, P, C) : chunk_floats(N, P, C)) * sizeof(float);
 }
 
 // 1 if chunks of tokens fit a block's LDS for a state of N x P (`by_channel`: a decay per key channel).
@@ -864,19 +864,27 @@ extern "C" int state_scan(const ScanArgs* args, int chunked, int span, int n_spa
     if (!chunks_raised) {
       (void)hipFuncSetAttribute((const void*)state_chunks_kernel<float>, hipFuncAttributeMaxDynamicSharedMemorySize, SCAN_MAX_LDS);
       (void)hipFuncSetAttribute((const void*)state_chunks_kernel<bf16>, hipFuncAttributeMaxDynamicSharedMemorySize, SCAN_MAX_LDS);
-      (void)hipFuncSetAttribute((const void*)channel_chunks_kernel<float>, hipFuncAttributeMaxDynamicSharedMemorySize, SCAN_MAX_LDS);
-      (void)hipFuncSetAttribute((const void*)channel_chunks_kernel<bf16>, hipFuncAttributeMaxDynamicSharedMemorySize, SCAN_MAX_LDS);
+      (void)hipFuncSetAttribute((const void*)channel_chunks_kernel<float, 256>, hipFuncAttributeMaxDynamicSharedMemorySize, SCAN_MAX_LDS);
+      (void)hipFuncSetAttribute((const void*)channel_chunks_kernel<bf16, 256>, hipFuncAttributeMaxDynamicSharedMemorySize, SCAN_MAX_LDS);
+      (void)hipFuncSetAttribute((const void*)channel_chunks_kernel<float, 512>, hipFuncAttributeMaxDynamicSharedMemorySize, SCAN_MAX_LDS);
+      (void)hipFuncSetAttribute((const void*)channel_chunks_kernel<bf16, 512>, hipFuncAttributeMaxDynamicSharedMemorySize, SCAN_MAX_LDS);
       chunks_raised = true;
     }
     const size_t bytes = chunk_bytes(by_channel, a.N, a.P, C);
-    const int row_floats = by_channel ? channel_row_floats(a.N, a.P, C) : 0;
+    // (eight waves a block where LDS keeps a compute unit to one block, or there is but one for each: channel_chunks_kernel)
+    const bool shared_units = 2 * (bytes + 1024) <= 160 * 1024;
     SpanArgs sp = {WHOLE, 0, nullptr, nullptr, nullptr, nullptr};
 #define CHUNKS(GRID)                                                                                \
   do {                                                                                              \
-    if (by_channel && a.out_dtype == DT_F32)                                                        \
-      hipLaunchKernelGGL(channel_chunks_kernel<float>, GRID, dim3(CHANNEL_THREADS), bytes, stream, turned, C, row_floats, sp); \
+    const bool four_waves = shared_units && (long)GRID.x * GRID.y > n_compute_units();              \
+    if (by_channel && a.out_dtype == DT_F32 && four_waves)                                          \
+      hipLaunchKernelGGL((channel_chunks_kernel<float, 256>), GRID, dim3(256), bytes, stream, turned, C, sp); \
+    else if (by_channel && a.out_dtype == DT_F32)                                                   \
+      hipLaunchKernelGGL((channel_chunks_kernel<float, 512>), GRID, dim3(512), bytes, stream, turned, C, sp); \
+    else if (by_channel && four_waves)                                                              \
+      hipLaunchKernelGGL((channel_chunks_kernel<bf16, 256>), GRID, dim3(256), bytes, stream, turned, C, sp);  \
     else if (by_channel)                                                                            \
-      hipLaunchKernelGGL(channel_chunks_kernel<bf16>, GRID, dim3(CHANNEL_THREADS), bytes, stream, turned, C, row_floats, sp); \
+      hipLaunchKernelGGL((channel_chunks_kernel<bf16, 512>), GRID, dim3(512), bytes, stream, turned, C, sp);  \
     else if (a.out_dtype == DT_F32)                                                                 \
       hipLaunchKernelGGL(state_chunks_kernel<float>, GRID, block, bytes, stream, turned, C, sp);         \
     else                                                                                            \

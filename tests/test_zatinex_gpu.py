@@ -264,8 +264,15 @@ def test_a_state_that_decays_by_key_channel_in_portions_of_two_requests(N, P, H,
 
 @pytest.mark.parametrize("chunked", [True, "spans"])
 @pytest.mark.parametrize("N,P,H", [(16, 224, 1), (144, 112, 2), (208, 112, 1), (304, 16, 2), (496, 16, 1)])
-def test_states_whose_chunks_fit_only_in_rows_without_padding(N, P, H, chunked):
-    """Chunks of 64, 32 and 16 tokens whose rows of LDS lie side by side, as four more floats a row would not fit."""
+def test_states_whose_chunks_just_fit(N, P, H, chunked):
+    """Chunks of 64, 32 and 16 tokens that leave less of the LDS than four floats a row."""
+    test_a_state_that_decays_by_key_channel_in_portions_of_two_requests(N, P, H, chunked)
+
+
+@pytest.mark.parametrize("chunked", [True, "spans"])
+@pytest.mark.parametrize("N,P,H", [(8, 8, 150), (32, 32, 130), (5, 33, 140)])
+def test_states_of_which_a_compute_unit_holds_several(N, P, H, chunked):
+    """More blocks than compute units, several of which fit one: blocks of four waves instead of eight."""
     test_a_state_that_decays_by_key_channel_in_portions_of_two_requests(N, P, H, chunked)
 
 
