@@ -535,9 +535,11 @@ static int linear(EngCtx* ctx, const EngMat& out, const EngValue& a, const EngWe
       if (n_splits < 1) n_splits = 1;
       if (n_splits > 1 && pending) TRY(settle(ctx, pending));  // the workspace is about to be written again
     }
-    // (few rows' keys and values go to their pages from the product's own epilogue, others from the finished rows, below)
+    // (few rows' keys and values go to their pages from the product's own epilogue, others from the finished rows, below: also
+    // columns that the pages' heads do not take all of)
     int scatters = 0;
-    if (sc && (variant == 0 || variant == 3)) QUERY(k_gemm_f32_scatters, scatters, M, n_splits);
+    if (sc && (variant == 0 || variant == 3) && sc->n_kv_heads * sc->head_dim == sc->kv_width)
+      QUERY(k_gemm_f32_scatters, scatters, M, n_splits);
     const EngScatter* own = scatters ? sc : nullptr;
     KERNEL(k_gemm_f32, ctx, out.p, A.p, w.w, bias, M, N, K, A.ld, w.ldw, out.ld, flags, variant, n_splits,
            n_splits > 1 ? ws : nullptr, n_splits > 1 ? ws_floats : (size_t)0, own ? own->k : nullptr, own ? own->v : nullptr,

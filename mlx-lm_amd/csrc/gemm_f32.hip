@@ -454,6 +454,8 @@ extern "C" int gemm_f32_scatter(void* out, const void* A, const void* W, const f
     if (!v_pages || !block_table || !token_req || !positions || head_dim <= 0 || page_size <= 0 || max_blocks <= 0 ||
         kv_width % head_dim != 0 || q_width + 2 * kv_width != N)
       FAIL("gemm_f32: the cache scatter's pointers or widths (q_width %d + 2 * kv_width %d, N=%d)", q_width, kv_width, N);
+    if (head_dim < 4 || head_dim > 256 || head_dim % 4 != 0 || page_stride < (size_t)kv_width * page_size)  // (as kv_write has it)
+      FAIL("gemm_f32: heads of %d, or a page stride smaller than a page", head_dim);
     p.k_pages = (float*)k_pages, p.v_pages = (float*)v_pages, p.page_stride = page_stride;
     p.block_table = block_table, p.max_blocks = max_blocks, p.token_req = token_req, p.positions = positions;
     p.q_width = q_width, p.kv_width = kv_width, p.head_dim = head_dim, p.page_size = page_size;

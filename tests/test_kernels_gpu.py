@@ -1639,6 +1639,19 @@ def test_projection_scatters_keys_and_values(M, dtype, splits):
         assert torch.isnan(pool[page, 0, :, row + 1 :].float()).all()
 
 
+@pytest.mark.parametrize("hd", [2, 6, 260])
+def test_heads_that_no_cache_write_takes(hd):
+    """float32 products of few rows, which fill the pages themselves, refuse the head sizes that the cache write of more rows does."""
+    k = _k()
+    for M in (5, 80):
+        c = PagedCase(torch.float32, 2, 1, hd, 16, [3] * M, [1] * M, seed=M)
+        w, a = _rand((4 * hd, 96), torch.float32, 3, 0.2), _rand((M, 96), torch.float32, 5)
+        out, before = torch.empty(M, 4 * hd, device=DEV), c.pool.clone()
+        with pytest.raises(RuntimeError, match="head"):
+            k.linear(out, a, w, scatter=k.KVScatter(c.kv, c.block_table_dev, c.token_req, c.positions, 2 * hd))
+        assert torch.equal(c.pool.isnan(), before.isnan())
+
+
 @pytest.mark.parametrize("variant", [0, 1, 3, 4, 5, 6, 7, 8])
 @pytest.mark.parametrize("packed", [False, True])
 def test_tile_products_scatter_keys_and_values_themselves(variant, packed):
