@@ -82,6 +82,7 @@ typedef struct {
 typedef struct {
   long launches, settle_normed, settle_plain, callbacks, steps;
   long key_splits_most;  // the most parts that a row kernel split a row's keys into
+  long chained;          // steps whose layers were one launch (a recorded one counts when it is recorded)
 } EngStats;
 
 // What the one launch of a decode step of one or two rows needs of an engine (decode_chain.h), made once.

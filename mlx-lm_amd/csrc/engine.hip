@@ -1158,6 +1158,7 @@ struct Model : EngPart {
     TRY(take(ctx, rows, width, DT_F32, out));
     KERNEL(k_chain, ctx, &d, rows, ctx->chain->layers, ctx->chain->memory[rows - 1], (const float*)h.p, (float*)out->p, width,
            ctx->block_tables[group], ctx->table_width[group], ctx->token_req, ctx->positions, 0, 0u, ctx->stream);
+    if (ctx->stats) ctx->stats->chained++;
     *done = true;
     return 0;
   }

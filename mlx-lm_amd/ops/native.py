@@ -62,7 +62,7 @@ class EngScratch(Structure):
 
 class EngStats(Structure):
     _fields_ = [("launches", c_long), ("settle_normed", c_long), ("settle_plain", c_long),
-                ("callbacks", c_long), ("steps", c_long), ("key_splits_most", c_long)]
+                ("callbacks", c_long), ("steps", c_long), ("key_splits_most", c_long), ("chained", c_long)]
 
 
 class EngChain(Structure):
