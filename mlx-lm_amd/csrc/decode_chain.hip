@@ -10,11 +10,11 @@
 // that issues those copies stands still until the memory has taken them, 3 to 4 us for the 100 KB of a unit (a compute
 // unit draws some 25 KB a us), and rows that it asks for come behind them: so CH_COPIERS waves of the block do nothing
 // else, and the others never wait for more than their rows.  A layer of GPT-2's sizes in us, with its five launches /
-// here with the computing waves copying too / with two waves to copy / with four (as it is):
-//   width   768 at  93 keys, one row    26 / 16.3 / 16.4 / 15.7   (two rows, in one launch only: 18.6 / - / 17.9)
-//   width 1,280 at 500 keys, one row    34 / 19.9 / 19.0 / 17.1
-//   width 1,600 at 700 keys, one row    37 / 23.0 / 21.3 / 19.5   (two rows: 26.0 / 23.4 / 22.0)
-// Of the 19.5 the weights' 61 MB are 9.6 at the memory's rate and the five hand-overs 6.
+// here with the computing waves copying too / with two waves to copy / with four / and the next unit looked up once (as it is):
+//   width   768 at  93 keys, one row    26 / 16.3 / 16.4 / 15.7 / 15.0   (two rows, in one launch only: 18.6 / - / 17.9 / 17.8)
+//   width 1,280 at 500 keys, one row    34 / 19.9 / 19.0 / 17.1 / 16.9
+//   width 1,600 at 700 keys, one row    37 / 23.0 / 21.3 / 19.5 / 18.9   (two rows: 26.0 / 23.4 / 22.0 / 21.9)
+// Of the 18.9 the weights' 61 MB are 9.6 at the memory's rate and the five hand-overs 6.
 //
 // Hand-over.  What one product hands to the next lies in words of eight bytes, 4 of payload (a float32
 // of the stream, or two bfloat16) and 4 of tag; a tag belongs to one product of one step.  A word is

@@ -1142,8 +1142,9 @@ struct Model : EngPart {
   }
 
   // All layers of a step whose one or two requests bring a token each, as one launch; the stream after them
-  // lies in *out then.  At three rows its hand-overs, whose words every block reads, would cost what the launches do; a row's
-  // keys must fit the registers of the block that takes a head of it.
+  // lies in *out then.  At three rows its hand-overs, whose words every block reads, would cost what the launches do (two rows only
+  // of widths whose products leave each block one unit: decode_chain_takes); a row's keys must fit the registers of the block that
+  // takes a head of it.
   int chained(EngCtx* ctx, const EngMat& h, EngMat* out, bool* done) const {
     *done = false;
     const int rows = ctx->n_tokens;

@@ -407,8 +407,9 @@ static void launch(const GemmArgs& p, int variant, hipStream_t stream) {
     hipLaunchKernelGGL(gemm_f32_skinny_kernel<4>, grid, block, 0, stream, p);
 }
 
-// 1 if gemm_f32_scatter puts the keys and values of so many rows into their pages.  (Up to 64 rows: a step of 8 rows of
-// GPT-2 large 2,199 -> 2,098 us without the 36 launches that did it.  A tile's epilogue does not: its pieces of 16 bytes a
+// 1 if gemm_f32_scatter puts the keys and values of so many rows into their pages.  (Up to 64 rows: a step of GPT-2 large at 30 to
+// 60 keys without the 36 launches that did it, 1 / 8 / 16 / 17 / 32 / 64 rows, 1,705 -> 1,595, 1,909 -> 1,800, 2,190 -> 2,072, 2,362 ->
+// 2,283, 2,850 -> 2,744, 4,585 -> 4,534 us; of small with 12, 514 -> 492 to 1,361 -> 1,350.  A tile's epilogue does not: its pieces of 16 bytes a
 // row, each at a place of its own, cost more than the launch that writes whole heads, 15,002 -> 15,122 us for 1,050 rows.)
 extern "C" int gemm_f32_scatters(int M, int n_splits) { return M >= 1 && M <= SKF_MAX_ROWS && n_splits == 1; }
 

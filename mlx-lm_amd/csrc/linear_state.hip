@@ -743,7 +743,6 @@ __global__ __launch_bounds__(256) void conv_state_update_kernel(const float* __r
   }
 }
 
-// A block a (row, group).
 // Row `row` of every tensor of `table` (base, bytes a row) set to zero: blockIdx.y is the tensor.  A new request's rows
 // are 10 KB to a few MB over all tensors, less than the launches that clear them one by one cost their host: eight requests of
 // a model with eight tensors were 64 fills of 1.9 us some 10 us apart, a pass of theirs 7,491 us, and 7,312 with eight launches.
@@ -767,6 +766,7 @@ __global__ __launch_bounds__(256) void clear_rows_kernel(const RowsOf* __restric
     clear_row<char>(p, t.bytes);
 }
 
+// A block a (row, group).
 template <typename T>
 __global__ __launch_bounds__(256) void gated_group_rmsnorm_kernel(const float* __restrict__ y, int ldy,
                                                                   const float* __restrict__ z, int ldz,
