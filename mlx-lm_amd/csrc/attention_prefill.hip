@@ -22,12 +22,16 @@
 //    a thread reads the same 8 columns of two neighbouring keys and writes
 //    eight 32-bit words (two keys each).
 //  * Online softmax in 32-bit per lane; outputs leave as O^T accumulators.
-// What bounds it: the softmax's vector instructions, half of their time the exponentials (a tile of 128 queries x 64
-// keys is some 1,150 cycles of them a wave beside 512 of the matrix unit), and at few blocks the chain of one block.
-// 8,000 tokens of 25 heads of 64: 309 us, 0.66 PFLOP/s of the causal half; 2 x 1,024: 23.2; 2 x 1,024 of 16 heads of
-// 128: 34.6; of 8 heads of 256: 100 (107 with two tiles on their way, which did not fit the registers).
+// Heads of 64 without optional terms of a score have a kernel of their own, attn_prefill_ring_kernel, with the same
+// products and the same softmax: tiles go into LDS as they lie in the pages, by copies, and the values are transposed
+// on their way out of it.
+// What bounds it: the softmax's vector instructions (here some 1,150 cycles of them a wave and tile of 64 keys beside 512 of
+// the matrix unit, a third of them addresses and the values' transposition), and at few blocks the chain of one block.
+// 2 x 1,024 tokens of 16 heads of 128: 34.6 us; of 8 heads of 256: 100 (107 with two tiles on their way, which did not fit
+// the registers).
 #include "common.h"
 #include "attention_tiles.h"
+#include "lds_copy.h"
 #include <type_traits>
 
 struct PrefillArgs {
@@ -88,11 +92,11 @@ __device__ __forceinline__ int key_of_row(int rho) {
 // TWO_GROUPS_FROM tiles is left to the first group: joining the sums costs about as much as a tile (25 heads of 64, both
 // groups and the first alone: 17 tokens, one tile, 5.3 and 4.5 us; 192, three, 8.6 and 7.7; 300, five, 10.1 and 9.5; 333,
 // six, 10.6 and 10.9; 333 under a window of 200, six at most, 11.7 and 13.1.  16 heads of 32: 192 tokens 6.4 and 5.9; 200,
-// four tiles, 6.5 and 7.2).  That the other waves were there at all costs up to 0.4 us (128 tokens: 7.5, in a block of four
-// waves 7.1), but how long the walks are is not known where the kernel is launched: a recorded step runs at other lengths.
+// four tiles, 6.5 and 7.2; the kernel for heads of 64 without terms, five tiles 10.1 and 9.8, six 9.3 and 9.6.)  That the
+// other waves were there at all costs up to 0.4 us (128 tokens: 7.0, in a block of four
+// waves 6.8), but how long the walks are is not known where the kernel is launched: a recorded step runs at other lengths.
 // (With heads of 64 two waves a SIMD, no fewer and no more, are named to the compiler: left alone it takes the registers
-// of three, which leaves it less to overlap, 24.6 us against 23.4 for 2 x 1,024 tokens of 25 heads and 80 against 73 for
-// 512 on 4,000 earlier keys, though 295 against 309 for 8,000.  Heads of 32 run three where blocks are many: 16 heads at
+// of three, which leaves it less to overlap.  Heads of 32 run three where blocks are many: 16 heads at
 // 8,000 tokens 133 us, 141 with two.)
 template <int HD>
 static constexpr int TWO_GROUPS_FROM = HD == 32 ? 4 : 6;
@@ -519,6 +523,397 @@ void attn_prefill_kernel(PrefillArgs p) {
   }
 }
 
+// ---------------------------------------------------------------------------
+// Heads of 64 without optional terms of a score, in pages of a power of two of sixteen keys or more: one page then holds
+// the sixteen keys of a tile that a wave copies.
+//
+// The same blocks, walks and arithmetic as above.  What differs is how a tile comes to its products, so that the vector
+// unit has little to do but the softmax:
+//  * Keys and values go from the pages to LDS by copies (lds_copy.h), two copies of a kilobyte a wave and tile for
+//    each, into rings of three tiles, asked for two tiles ahead; a page's place is three scalar instructions out of a table in LDS.
+//    Before, a tile went through registers: a dozen integer instructions an address and 24 to transpose the values.
+//  * Values are transposed by the LDS read (ds_read_b64_tr_b16: four keys of a column a lane).  A lane's eight scores of a
+//    chunk are keys 4 g .. + 3 and 8 + 4 g .. + 3 of it, and two such reads bring the values of just these.
+//  * A row's pieces of 16 bytes lie permuted (piece ^ (row / 2 % 8) of keys, piece ^ 4 (row / 2 % 2) of values), so that the
+//    sixteen rows of a read of keys, and the four rows x 64 bytes of a read of values, meet all banks: no conflict is counted.
+//  * The next tile's scores are begun while this one's probabilities are made, in the registers that are free by then, so
+//    that a wave needs 153 registers and three blocks share a CU.  (With the scores in two sets of registers, a whole tile ahead, 232:
+//    two blocks, 272 us for 8,000 tokens instead of 251.)
+// 25 heads of 64, us, the kernel above and this one: 8,000 tokens 315 and 251 (0.82 PFLOP/s of the causal half), under a window of
+// 1,000 112 and 84; 2 x 1,024 24.5 and 21.2; 1,024 19.6 and 17.2; 512 on 4,000 earlier keys 58.5 and 49; 512 12.3 and 11.4; 333 10.1
+// and 9.4; 128 7.6 and 7.0; 17 4.7 and 4.8.  What bounds it: vector instructions, 74 % of the CUs' cycles beside 41 % for the
+// products (8,000 tokens at 1.88 GHz); at few blocks the way to the first tile and the walk's steps of some 1 us.
+
+typedef short i16x4_t __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) i16x4_t* lds_i16x4_p;
+union FragHalves {
+  i16x4_t h[2];
+  bf16x8_t v;
+};
+// Four keys of one column a lane: lane l of each sixteen names four columns (8 bytes) of key l / 4 and gets column l of
+// all four keys.
+__device__ __forceinline__ i16x4_t read_transposed(uint32_t at) {
+  return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_p)(uintptr_t)at);
+}
+__device__ __forceinline__ bf16x8_t read_piece(uint32_t at) {
+  return *(const __attribute__((address_space(3))) bf16x8_t*)(uintptr_t)at;
+}
+// the larger of a value and the one of the lane 32 away (the maximum as an instruction: fmaxf first makes its operands
+// canonical, which these are)
+__device__ __forceinline__ float max_of_halves(float v) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  float larger;
+  asm("v_max_f32 %0, %1, %2" : "=v"(larger) : "v"(r[0]), "v"(r[1]));
+  return larger;
+}
+
+template <int HD, int GROUPS>
+__global__ __launch_bounds__(256 * GROUPS) __attribute__((amdgpu_waves_per_eu(GROUPS == 1 ? 3 : 2, GROUPS == 1 ? 3 : 2)))
+void attn_prefill_ring_kernel(PrefillArgs p) {
+  constexpr int DC = HD / 16, DT = HD / 32;
+  constexpr int ROW = HD * 2, WAVE_KEYS = KT / 4, COPIES = WAVE_KEYS * ROW / 1024;  // bytes a key; keys and copies a wave and tile
+  constexpr int SLOTS = 3, TILE = KT * ROW, GROUP_LDS = 2 * SLOTS * TILE;
+  static_assert(HD == 64, "the permutations of a row's pieces are those of rows of 128 bytes");
+  __shared__ __attribute__((aligned(1024))) char ring[GROUPS * GROUP_LDS];
+  extern __shared__ size_t page_at[];  // [max_blocks]: byte offsets of this head's part of the request's pages, from the first tile's on
+
+  const int group = GROUPS > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0;
+  const int tid = threadIdx.x & 255, lane = tid & 63;  // (within the group)
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int h = blockIdx.x, tile = blockIdx.y;
+  const int row0 = p.tiles[2 * tile];
+  const int nq = p.tiles[2 * tile + 1];
+  const int kv_head = h / (p.n_heads / p.n_kv_heads);
+  const int pos0 = __builtin_amdgcn_readfirstlane(p.positions[row0]), request = __builtin_amdgcn_readfirstlane(p.token_req[row0]);
+  asm volatile("" ::"s"(pos0), "s"(request));  // (one wait for the two: left alone, the second load stands behind the first's use)
+  const int* table = p.block_table + (size_t)request * p.max_blocks;
+
+  const int ql = lane & 31, g = lane >> 5;
+  const int qi = wave * 32 + ql;  // this lane's query within the tile
+  const bool q_live = qi < nq;
+  const int qpos = pos0 + qi;
+  const int q_lo = p.window > 0 ? max(0, qpos - p.window + 1) : 0;
+
+  // (a lane without a query takes the last one's: nothing of it is stored)
+  Frag8 qf[DC];
+  {
+    const uint16_t* qrow = p.q + (size_t)(row0 + min(qi, nq - 1)) * p.ldq + h * HD + 8 * g;
+#pragma unroll
+    for (int dc = 0; dc < DC; ++dc) qf[dc].u = *(const uint4*)(qrow + dc * 16);
+  }
+
+  const int k_hi = pos0 + nq;  // one past the last key any query of the tile sees
+  const int k_lo = p.window > 0 ? max(0, pos0 - p.window + 1) : 0;
+  const int kt0 = (k_lo / KT) * KT;
+  const int n_tiles = (k_hi - kt0 + KT - 1) / KT;
+  // (in a short walk the second group's waves end here: barriers count the waves that are left)
+  const int groups = GROUPS > 1 && n_tiles >= TWO_GROUPS_FROM<HD> ? GROUPS : 1;
+  if (GROUPS > 1 && group >= groups) return;
+  const int n_steps = (n_tiles + groups - 1) / groups;
+  // keys this wave's queries can see end here (a wave without queries: none)
+  const int wave_hi = wave * 32 < nq ? min(k_hi, pos0 + wave * 32 + 32) : 0;
+  const int wave_q0 = pos0 + wave * 32;  // position of the wave's first query
+  const float c2 = p.scale * 1.4426950408889634f;  // scores to units of log 2
+
+  const int shift = p.page_shift, row_mask = p.page_size - 1;
+  const int pg0 = kt0 >> shift, n_pg = ((k_hi - 1) >> shift) - pg0 + 1, first_page = k_lo >> shift;
+  for (int i = threadIdx.x; i < n_pg; i += 256 * groups)
+    page_at[i] = ((size_t)(uint32_t)table[max(pg0 + i, first_page)] * p.page_stride + (size_t)(kv_head << shift) * HD) * 2;
+  __syncthreads();
+
+  // (the queries are waited for here, ahead of the copies: the compiler, which does not count those, would wait for all)
+#pragma unroll
+  for (int dc = 0; dc < DC; ++dc) asm volatile("" : "+v"(qf[dc].v));
+
+  // Copies: this wave brings keys 16 wave .. + 15 of each tile, which lie in one page.  Of keys in pages before the
+  // window's first and of keys beyond the last nothing is read, and zeros come.
+  const uint32_t ring_at = lds_address(ring) + group * GROUP_LDS;
+  const uint32_t copy_at = __builtin_amdgcn_readfirstlane(ring_at + wave * COPIES * 1024);
+  const int row8 = lane >> 3;
+  const uint32_t k_from0 = row8 * ROW + (((lane & 7) ^ (row8 >> 1)) * 16), k_from1 = row8 * ROW + (((lane & 7) ^ (4 + (row8 >> 1))) * 16);
+  const uint32_t v_from = row8 * ROW + (((lane & 7) ^ (4 * ((row8 >> 1) & 1))) * 16);
+  auto first_key = [&](int t) __attribute__((always_inline)) { return kt0 + (t * groups + group) * KT; };
+  auto page_entry = [&](int t) __attribute__((always_inline)) {
+    return page_at[min(((first_key(t) + wave * WAVE_KEYS) >> shift) - pg0, n_pg - 1)];
+  };
+  // where this wave's keys of tile t lie in the pages, and how many bytes of them there are
+  struct Source {
+    uint32_t lo, hi;
+    int bytes;
+  };
+  auto source = [&](int t, size_t entry) __attribute__((always_inline)) {
+    const int key = first_key(t) + wave * WAVE_KEYS;
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)entry), hi = __builtin_amdgcn_readfirstlane((uint32_t)(entry >> 32));
+    const size_t at = (((size_t)hi << 32) | lo) + (uint32_t)((key & row_mask) * ROW);
+    int keys;  // (as scalar instructions: the compiler takes the vector unit's median)
+    asm("s_max_i32 %0, %1, 0\n\ts_min_i32 %0, %0, %2" : "=&s"(keys) : "s"(k_hi - key), "n"(WAVE_KEYS) : "scc");
+    return Source{(uint32_t)at, (uint32_t)(at >> 32), (key >> shift) < first_page ? 0 : keys * ROW};
+  };
+  // (what a copy's descriptor is made of is the same in all lanes; the compiler loses sight of that)
+  auto copy = [&](const uint16_t* pages, const Source& s, uint32_t from0, uint32_t from1, uint32_t to) __attribute__((always_inline)) {
+    const size_t at = (size_t)pages + (((size_t)s.hi << 32) | s.lo);
+    const i32x4_t buffer = {__builtin_amdgcn_readfirstlane((int)(uint32_t)at), __builtin_amdgcn_readfirstlane((int)((at >> 32) & 0xffffu)),
+                            __builtin_amdgcn_readfirstlane(s.bytes), BUFFER_WORD3};
+    copy_pair_to_lds(buffer, from0, from1, __builtin_amdgcn_readfirstlane(to));
+  };
+  auto copy_k = [&](const Source& s, int slot) __attribute__((always_inline)) { copy(p.k_pages, s, k_from0, k_from1, copy_at + slot * TILE); };
+  auto copy_v = [&](const Source& s, int slot) __attribute__((always_inline)) { copy(p.v_pages, s, v_from, v_from, copy_at + (SLOTS + slot) * TILE); };
+
+  float m = -INFINITY, l = 0.f;
+  f32x16_t ot[DT];
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) ot[dt][r] = 0.f;
+
+  // where this lane reads: keys (rows of S^T's first operand) and, transposed, values
+  uint32_t k_read[DC], v_read[DT];
+#pragma unroll
+  for (int dc = 0; dc < DC; ++dc) k_read[dc] = ring_at + ql * ROW + (((2 * dc + g) ^ ((ql >> 1) & 7)) * 16);
+  const int vrow = 4 * g + ((lane & 15) >> 2);
+#pragma unroll
+  for (int dt = 0; dt < DT; ++dt)
+    v_read[dt] = ring_at + SLOTS * TILE + vrow * ROW +
+                 (((4 * dt + 2 * ((lane >> 4) & 1) + ((lane & 3) >> 1)) ^ (4 * ((vrow >> 1) & 1))) * 16) + (lane & 1) * 8;
+
+  // (an address whose origin the compiler does not see: what is added to it goes into the reads' offsets)
+  auto opaque = [](uint32_t at) __attribute__((always_inline)) {
+    asm("" : "+v"(at));
+    return at;
+  };
+  auto read_k = [&](bf16x8_t (&kf)[2], uint32_t at) __attribute__((always_inline)) {  // of both subtiles
+#pragma unroll
+    for (int s = 0; s < 2; ++s) kf[s] = read_piece(at + s * 32 * ROW);
+  };
+  auto read_v = [&](bf16x8_t (&vf)[DT], int c, const uint32_t (&at)[DT]) __attribute__((always_inline)) {  // of keys 16 c .. + 15
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) {
+      FragHalves f;
+#pragma unroll
+      for (int e = 0; e < 2; ++e) f.h[e] = read_transposed(at[dt] + (16 * c + 8 * e) * ROW);
+      vf[dt] = f.v;
+    }
+  };
+  const f32x16_t NO_SUMS = {};
+  auto scores = [&](f32x16_t (&sn)[2], int slot) __attribute__((always_inline)) {
+    bf16x8_t kf[DC][2];
+#pragma unroll
+    for (int dc = 0; dc < DC; ++dc) read_k(kf[dc], opaque(k_read[dc] + slot * TILE));
+#pragma unroll
+    for (int dc = 0; dc < DC; ++dc)
+#pragma unroll
+      for (int s = 0; s < 2; ++s) sn[s] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[dc][s], qf[dc].v, dc == 0 ? NO_SUMS : sn[s], 0, 0, 0);
+  };
+  auto rescale = [&](float tmax) __attribute__((always_inline)) {
+    if (__any(tmax > m)) {
+      const float m_new = fmaxf(m, tmax);
+      const float alpha = __builtin_amdgcn_exp2f(m - (m_new == -INFINITY ? 0.f : m_new));  // (a row with no key yet: zero)
+      l *= alpha;
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) ot[dt][r] *= alpha;
+      m = m_new;
+    }
+  };
+
+  // One step: the softmax and the output's products of tile t out of its scores `st`, and the scores of tile t + 1 to `sn`.
+  auto whole = [&](int kt) __attribute__((always_inline)) { return kt + KT - 1 <= wave_q0 && (p.window <= 0 || kt >= wave_q0 + 31 - p.window + 1); };
+  // A tile that every query of the wave sees whole, with another one behind it.  Eight pieces of four scores' probabilities;
+  // the products go beside them as their operands are there: the first subtile's registers take the next tile's scores
+  // when its probabilities are made, the second's at the end.
+  auto steady_step = [&](f32x16_t (&st)[2], int kslot, int vslot) __attribute__((always_inline)) {
+    bf16x8_t kf[DC][2], vf[4][DT];
+    float tmax = -INFINITY;
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int r = 0; r < 16; r += 2) tmax = fmaxf(fmaxf(st[s][r], st[s][r + 1]), tmax);
+    uint32_t v_at[DT], k_at[DC];
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt) v_at[dt] = opaque(v_read[dt] + vslot * TILE);
+#pragma unroll
+    for (int dc = 0; dc < DC; ++dc) k_at[dc] = opaque(k_read[dc] + kslot * TILE);
+    read_v(vf[0], 0, v_at);
+    rescale(max_of_halves(tmax * c2));  // (c2 > 0: the largest score stays the largest)
+    const float m_use = m == -INFINITY ? 0.f : m;
+    __builtin_amdgcn_sched_barrier(0);
+    Frag8 pf[4];
+    float part[4];
+    auto output = [&](int c) __attribute__((always_inline)) {
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) ot[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[c][dt], pf[c].v, ot[dt], 0, 0, 0);
+    };
+    auto score = [&](int s, int dc) __attribute__((always_inline)) {
+      st[s] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[dc][s], qf[dc].v, dc == 0 ? NO_SUMS : st[s], 0, 0, 0);
+    };
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      float e[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        e[i] = __builtin_amdgcn_exp2f(fmaf(st[j >> 2][4 * (j & 3) + i], c2, -m_use));
+        part[i] = j == 0 ? e[i] : part[i] + e[i];
+      }
+      if (j & 1)
+        pf[j >> 1].u.z = pack_bf16x2(e[0], e[1]), pf[j >> 1].u.w = pack_bf16x2(e[2], e[3]);
+      else
+        pf[j >> 1].u.x = pack_bf16x2(e[0], e[1]), pf[j >> 1].u.y = pack_bf16x2(e[2], e[3]);
+      // (what is multiplied is read from LDS two pieces earlier)
+      if (j == 1) read_v(vf[1], 1, v_at);
+      if (j >= 2 && j < 6) kf[j - 2][0] = read_piece(k_at[j - 2]);
+      if (j == 4) read_v(vf[2], 2, v_at);
+      if (j == 6) read_v(vf[3], 3, v_at);
+      if (j == 2) output(0);
+      if (j == 4) output(1);
+      if (j >= 4) score(0, j - 4);
+      if (j == 6) output(2);
+      if (j >= 6) kf[j - 6][1] = read_piece(k_at[j - 6] + 32 * ROW);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    kf[2][1] = read_piece(k_at[2] + 32 * ROW);
+    kf[3][1] = read_piece(k_at[3] + 32 * ROW);
+    output(3);
+#pragma unroll
+    for (int dc = 0; dc < DC; ++dc) score(1, dc);
+    l += (part[0] + part[1]) + (part[2] + part[3]);
+  };
+  // Any tile; the next one's scores take the place of its own at the end.
+  auto step = [&](f32x16_t (&st)[2], int t, int kslot, int vslot) __attribute__((always_inline)) {
+    const int kt = first_key(t);
+    const bool now = kt < wave_hi, next = first_key(t + 1) < wave_hi;
+    if (now) {
+      float tmax = -INFINITY;
+      if (!whole(kt)) {
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            const int key = kt + 32 * s + 8 * (r >> 2) + 4 * g + (r & 3);
+            st[s][r] = q_live && key <= qpos && key >= q_lo ? st[s][r] : -INFINITY;
+          }
+      }
+#pragma unroll
+      for (int s = 0; s < 2; ++s)
+#pragma unroll
+        for (int r = 0; r < 16; r += 2) tmax = fmaxf(fmaxf(st[s][r], st[s][r + 1]), tmax);
+      rescale(max_of_halves(tmax * c2));
+      const float m_use = m == -INFINITY ? 0.f : m;
+      Frag8 pf[4];
+      float part[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) part[i] = 0.f;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        float e[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          e[i] = __builtin_amdgcn_exp2f(fmaf(st[c >> 1][8 * (c & 1) + i], c2, -m_use));
+          part[i & 3] += e[i];
+        }
+        pf[c].u = make_uint4(pack_bf16x2(e[0], e[1]), pack_bf16x2(e[2], e[3]), pack_bf16x2(e[4], e[5]), pack_bf16x2(e[6], e[7]));
+      }
+      l += (part[0] + part[1]) + (part[2] + part[3]);
+      uint32_t v_at[DT];
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) v_at[dt] = opaque(v_read[dt] + vslot * TILE);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        bf16x8_t vf[DT];
+        read_v(vf, c, v_at);
+#pragma unroll
+        for (int dt = 0; dt < DT; ++dt) ot[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[dt], pf[c].v, ot[dt], 0, 0, 0);
+      }
+    }
+    if (next) scores(st, kslot);
+  };
+
+  // What is on its way when step t begins: K(t + 2), V(t + 1) and all before.  A step asks for V(t + 2) and K(t + 3),
+  // into the slots of K(t) and V(t - 1), which every wave has read when the step's barrier is passed.
+  static_assert(COPIES == 2, "a pair of copies a tile");
+  Source ahead;  // of tile t + 2
+#pragma unroll
+  for (int t = 0; t < 3; ++t) {
+    ahead = source(t, page_entry(t));
+    copy_k(ahead, t);
+    if (t < 2) copy_v(ahead, t);
+  }
+  size_t entry = page_entry(3);  // of tile t + 3, read from LDS a step ahead
+  f32x16_t sa[2];
+  copies_arrived<4 * COPIES>();  // K(0): behind it V(0), K(1), V(1), K(2)
+  ring_barrier();
+  if (first_key(0) < wave_hi) scores(sa, 0);
+  int slot = 0;  // of K(t) and V(t)
+  auto turn = [&](f32x16_t (&st)[2], int t, auto steady) __attribute__((always_inline)) {
+    copies_arrived<2 * COPIES>();  // K(t + 1) and V(t): behind them K(t + 2) and V(t + 1)
+    ring_barrier();
+    const int before = slot == 0 ? SLOTS - 1 : slot - 1, after = slot == SLOTS - 1 ? 0 : slot + 1;
+    copy_v(ahead, before);
+    ahead = source(t + 3, entry);
+    copy_k(ahead, slot);
+    entry = page_entry(t + 4);
+    if constexpr (decltype(steady)::value)
+      steady_step(st, after, slot);
+    else
+      step(st, t, after, slot);
+    slot = after;
+  };
+  // The steps from `from` up to `to` are of tiles that every query of the wave sees whole, with another one behind.  (The waves of a block go through theirs each on its own; what they share is a barrier a step.)
+  const int key0 = first_key(0), step_keys = groups * KT;
+  const int seen_from = p.window > 0 ? max(wave_q0 + 32 - p.window - key0, 0) : 0;
+  const int from = (seen_from + step_keys - 1) / step_keys;
+  const int seen_to = min(wave_q0 + 1 - KT, wave_hi - 1 - step_keys) - key0;  // the last one's first key
+  const int to = seen_to < 0 ? 0 : seen_to / step_keys + 1;
+  for (int t = 0; t < n_steps; ++t) {
+    if (t >= from)
+      for (; t < to; ++t) turn(sa, t, std::true_type{});
+    turn(sa, t, std::false_type{});
+  }
+  copies_arrived<0>();  // (what was asked for beyond the last tile)
+
+  // the two halves of the wave hold different keys of the same query
+  l += __shfl_xor(l, 32, WAVE);
+  if (GROUPS == 2 && groups == 2) {
+    // the second group's sums go to the first through LDS, each thread's to the thread of the same queries
+    static_assert(GROUPS == 1 || (DT * 16 + 2) * 256 * sizeof(float) <= sizeof(ring), "the sums fit where the tiles were");
+    float* const sums = (float*)ring + tid;
+    __syncthreads();  // no tile is read any more
+    if (group == 1) {
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) sums[(dt * 16 + r) * 256] = ot[dt][r];
+      sums[DT * 16 * 256] = m, sums[(DT * 16 + 1) * 256] = l;
+    }
+    __syncthreads();
+    if (group == 1) return;
+    const float m1 = sums[DT * 16 * 256], both = fmaxf(m, m1), to = both == -INFINITY ? 0.f : both;
+    const float w0 = exp2f(m - to), w1 = exp2f(m1 - to);  // (a group without a key of this query: zero)
+    l = l * w0 + sums[(DT * 16 + 1) * 256] * w1;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) ot[dt][r] = ot[dt][r] * w0 + sums[(dt * 16 + r) * 256] * w1;
+    m = both;
+  }
+  if (q_live) {
+    // (m is in units of log 2)
+    if (p.sinks) l += exp2f(fmaf(p.sinks[h], 1.4426950408889634f, -m));
+    const float inv = head_gate_of(p, row0 + qi, h) / l;
+    uint16_t* orow = p.out + (size_t)(row0 + qi) * p.ldo + h * HD;
+#pragma unroll
+    for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        // accumulators 4j .. 4j+3: head columns dt*32 + 8j + 4g + (0..3)
+        uint2 o;
+        o.x = pack_bf16x2(ot[dt][4 * j] * inv, ot[dt][4 * j + 1] * inv);
+        o.y = pack_bf16x2(ot[dt][4 * j + 2] * inv, ot[dt][4 * j + 3] * inv);
+        *(uint2*)(orow + dt * 32 + 8 * j + 4 * g) = o;
+      }
+  }
+}
+
 DEFINE_LAST_ERROR(mlxlm_last_error)
 
 // tiles: n_tiles pairs (first flat row, number of rows 1..128); the rows of a
@@ -576,11 +971,13 @@ static int prefill_launch(void* out, const void* q, int ldq, int ldo, const void
   // (the kept first keys' pages lie before the window's; a page can be in both runs)
   const size_t lds = (size_t)(max_blocks + (extras ? 2 : 0)) * sizeof(int);
   const bool pow2 = p.page_shift >= 0;
+  const bool ring = head_dim == 64 && !extras && p.page_shift >= 4;
   // Two groups a block where the blocks are no more than the CUs, so that a block's walk is the kernel's time: 1,024 tokens
   // of 25 heads of 64 (200 blocks) 19.1 us beside 21.3, 512 on 4,000 earlier keys 57 / 72, of 16 heads of 32 43 / 58.  With
   // more blocks than CUs they are in each other's way (2 x 1,024 tokens of 25 heads, 400 blocks: 25.5 / 23.1; 4 x 512:
-  // 20.7 / 15.2).  Heads of 128 and more take the registers of a whole SIMD a wave.
-  const bool two = head_dim <= 64 && pow2 && max_blocks <= 4096 && (long)n_heads * n_tiles <= n_compute_units();
+  // 20.7 / 15.2).  The kernel for heads of 64 without terms, one row of figures each: 1,024 16.9 / 18.4, 512 on 4,000 49 / 59.4;
+  // 2 x 1,024 23.2 / 20.8, 4 x 512 18.4 / 13.5.  Heads of 128 and more take the registers of a whole SIMD a wave.
+  const bool two = head_dim <= 64 && pow2 && (extras || head_dim != 64 || ring) && max_blocks <= 4096 && (long)n_heads * n_tiles <= n_compute_units();
   const dim3 grid(n_heads, n_tiles), block(two ? 512 : 256);
 #define LAUNCH_AS(HD, POW2, GROUPS)                                                                                      \
   do {                                                                                                                  \
@@ -588,20 +985,26 @@ static int prefill_launch(void* out, const void* q, int ldq, int ldo, const void
       hipLaunchKernelGGL((attn_prefill_kernel<HD, POW2, true, true, GROUPS>), grid, block, lds, stream, p);             \
     else if (extras)                                                                                                    \
       hipLaunchKernelGGL((attn_prefill_kernel<HD, POW2, true, false, GROUPS>), grid, block, lds, stream, p);            \
-    else                                                                                                                \
+    else if constexpr (HD != 64 || !POW2)                                                                               \
       hipLaunchKernelGGL((attn_prefill_kernel<HD, POW2, false, false, GROUPS>), grid, block, lds, stream, p);           \
   } while (0)
 #define LAUNCH_PREFILL(HD)              \
   do {                                  \
-    if (two) {                          \
-      LAUNCH_AS(HD, true, (HD <= 64 ? 2 : 1)); \
-    } else if (pow2) {                  \
-      LAUNCH_AS(HD, true, 1);           \
-    } else {                            \
+    if (!pow2 || (HD == 64 && !extras)) { \
       LAUNCH_AS(HD, false, 1);          \
+    } else if (two) {                   \
+      LAUNCH_AS(HD, true, (HD <= 64 ? 2 : 1)); \
+    } else {                            \
+      LAUNCH_AS(HD, true, 1);           \
     }                                   \
   } while (0)
-  if (head_dim == 32) {
+  if (ring) {
+    const size_t table = (size_t)max_blocks * sizeof(size_t);
+    if (two)
+      hipLaunchKernelGGL((attn_prefill_ring_kernel<64, 2>), grid, block, table, stream, p);
+    else
+      hipLaunchKernelGGL((attn_prefill_ring_kernel<64, 1>), grid, block, table, stream, p);
+  } else if (head_dim == 32) {
     LAUNCH_PREFILL(32);
   } else if (head_dim == 64) {
     LAUNCH_PREFILL(64);

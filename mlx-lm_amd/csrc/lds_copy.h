@@ -36,6 +36,17 @@ __device__ __forceinline__ void copy16_to_lds(i32x4_t buffer, uint32_t from, uin
                : "memory", "m0");
 }
 
+// Two copies of neighbouring kilobytes: the second one's bytes come from `from1` + 1024 and go to `to` + 1024 (the
+// instruction's offset counts on both sides).  The five states waited for are those between a vector instruction that
+// writes a scalar register and a memory instruction that reads it: the buffer may come straight from v_readfirstlane.
+__device__ __forceinline__ void copy_pair_to_lds(i32x4_t buffer, uint32_t from0, uint32_t from1, uint32_t to) {
+  asm volatile(
+      "s_mov_b32 m0, %0\n\ts_nop 4\n\tbuffer_load_dwordx4 %1, %3, 0 offen lds\n\tbuffer_load_dwordx4 %2, %3, 0 offen offset:1024 lds"
+      :
+      : "s"(to), "v"(from0), "v"(from1), "s"(buffer)
+      : "memory", "m0");
+}
+
 // Every copy of this wave but the newest N has arrived, and its LDS reads are done: with a barrier behind it, what all
 // waves copied can be read, and what all waves have read may be written.
 template <int N>

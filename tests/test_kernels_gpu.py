@@ -760,6 +760,32 @@ def test_attn_prefill_walks_around_the_one_that_two_groups_share(hd, edge, windo
     assert err < 2.5e-2, err
 
 
+@pytest.mark.parametrize("ps", [8, 16, 64, 256])
+@pytest.mark.parametrize("H,Hkv", [(3, 1), (90, 9)])
+@pytest.mark.parametrize("window", [0, 65, 300])
+def test_attn_prefill_heads_of_64_over_tiles_and_pages(ps, H, Hkv, window):
+    """Heads of 64, which read tiles of 64 keys by copies of a page's rows: portions of one query up to two tiles of queries
+    that end a key before, at and behind a tile of keys, a wave's sixteen keys and a page, with blocks fewer than the
+    compute units (two groups of waves) and more, windows whose first page is not the first; block tables as long as a
+    launch takes for either.  Free rows of pages hold NaN and unused entries of the tables name no page."""
+    k = _k()
+    total = [63, 64, 65, 80, 145, 256, 449, 703]
+    ql = [1, 33, 65, 80, 128, 129, 200, 17]
+    c = PagedCase(torch.bfloat16, H, Hkv, 64, ps, [t - n for t, n in zip(total, ql)], ql, seed=ps + H, window=window)
+    k.kv_write(c.k_new.to(DEV), c.v_new.to(DEV), c.kv, c.block_table_dev, c.token_req, c.positions)
+    tiles = c.tiles(k.attn_tile_sizes()[1])
+    few = H * tiles.shape[0] <= 256
+    table = torch.full((len(total), 4096 if few else 7168), -1, dtype=torch.int32, device=DEV)
+    table[:, : c.block_table_dev.shape[1]] = c.block_table_dev
+    want = c.reference()
+    for bt in (c.block_table_dev, table):
+        out = torch.full((c.T, H * 64), float("nan")).to(torch.bfloat16).to(DEV)
+        k.attn_prefill(out, c.q.to(DEV), c.kv, bt, c.token_req, c.positions, tiles, tiles.shape[0], H, c.scale, window)
+        err = (out.double().cpu() - want).abs().max().item()
+        # (the weights are rounded to bfloat16, 2^-9 of each, and meet values of up to 4.5)
+        assert err < 2.5e-2, err
+
+
 def test_attn_prefill_far_key_stands_out():
     """Every query of a long portion points at one far key of its own."""
     k = _k()
