@@ -107,7 +107,7 @@ __device__ __forceinline__ size_t out_at(const DecodeArgs& p, int row, int col) 
 }
 
 // What bounds this kernel: the keys and values come from memory once, and at many rows or long contexts that is the
-// time (64 rows of 25 heads of 64 at contexts of 300 to 1,001 are 266 MB: 49 us, 5.4 TB/s; a plain stream reads 6.4, with
+// time (64 rows of 25 heads of 64 at contexts of 300 to 1,001 are 266 MB: 46.7 us, 5.7 TB/s; a plain stream reads 6.4, with
 // the streaming hint 7.2).  So they are read with that hint where no two heads share them (8 to 10 % here); a tile is
 // small and the next one on its way while it is taken, so that a wave's registers are few and many waves have something
 // in flight (tiles of 32 or 64 keys, one at a time, with a lookup and two divisions a lane and key: 54 to 58 us, 13.4 against
@@ -215,7 +215,11 @@ __attribute__((amdgpu_waves_per_eu(CPK >= 16 ? 2 : 4, CPK == 8 && sizeof(T) == 2
     asm volatile("" ::"v"(seen));  // the loads stay although nobody wants the values
     return;
   }
-  const int item = blockIdx.x, h = blockIdx.y, split = blockIdx.z;
+  // A row's heads are neighbours in the launch.  Blocks go to the compute units in turn, so with the rows as the fast index
+  // and 64 rows every 256th block was the same row's: a unit had the longest row's heads and no others.  25 heads of 64,
+  // us, rows fast and heads fast: 64 rows at 300 to 1,001 keys 47.7 and 46.7, 48 at 16 to 1,000 32.3 and 30.5, 16 at 500 to 8,001 100
+  // and 90, 8 at 4,000 to 8,001 57.9 and 56.5; rows of one length, 24 of 550 and 8 of 6,000, 18.0 and 18.0, 48.3 and 49.
+  const int lin = blockIdx.x + gridDim.x * blockIdx.y, item = lin / p.n_heads, h = lin - item * p.n_heads, split = blockIdx.z;
   // Which row, whose pages, at which position: looked up one after the other these are three
   // trips to memory before the first key can be asked for, in a kernel that otherwise makes one
   // or two.  In a decode step item i is row i of request i, and the request's page numbers go to
