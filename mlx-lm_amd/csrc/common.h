@@ -118,6 +118,8 @@ __device__ __forceinline__ float gelu_tanh_fast(float x) {
   return x * __builtin_amdgcn_rcpf(1.0f + e);
 }
 
+__device__ __forceinline__ float silu_f(float z) { return z / (1.0f + expf(-z)); }
+
 // The activations that a product's epilogue can apply, chosen by two of its flag bits
 // (the same bits in every product kernel): tanh-GELU, or the square of the ReLU.
 #define FLAG_ACT_GELU 1

@@ -2,7 +2,8 @@
 //   router_choice   s = softmax(z) over all router outputs, or the logistic function of each; the `top`
 //                   largest of s + correction are chosen (the lower index on a tie), out of all or out
 //                   of the best groups of neighbours; their weights are s itself.
-//   silu_mul        act = silu(gate) * up for rows [gate | up]   (a dense gated feed-forward)
+//   silu_mul        act = silu(gate) * up for rows [gate | up]   (a dense gated feed-forward), or for
+//                   rows of eight gate columns and the same eight of up by turns
 //   route_and_gate  both of these in one launch, for a step of few tokens whose router, gate and up
 //                   came out of one product as float rows
 //   expert_rows_up / expert_rows_down
@@ -24,8 +25,6 @@
 //                   beyond the tiles that there are leave at once, so nothing comes to the host.
 // The router's softmax, the choice and the weights are 32-bit; products accumulate in 32-bit.
 #include "common.h"
-
-__device__ __forceinline__ float silu_f(float z) { return z / (1.0f + expf(-z)); }
 
 // An expert's activation of its gate and up columns:
 //   EXPERT_SILU     silu(g) u
@@ -211,6 +210,23 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(const T* __restrict__ gu,
   const T* row = gu + (size_t)r * ld;
   const float z = to_f32(row[f]);
   out[(size_t)r * ldo + f] = from_f32<T>((GELU ? gelu_tanh(z) : silu_f(z)) * to_f32(row[F + f]));
+}
+
+// The same for bfloat16 rows of eight gate columns and the same eight of up by turns: 16 bytes of each a thread.
+template <bool GELU>
+__global__ __launch_bounds__(256) void silu_mul_turns_kernel(const uint16_t* __restrict__ gu, int ld, uint16_t* __restrict__ out, int ldo, int F) {
+  const int f = (blockIdx.y * 256 + threadIdx.x) * 8, r = blockIdx.x;
+  if (f >= F) return;
+  const u32x4_t* in = (const u32x4_t*)(gu + (size_t)r * ld + 2 * f);
+  const u32x4_t g = in[0], u = in[1];
+  u32x4_t o;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const float g0 = __uint_as_float(g[i] << 16), g1 = __uint_as_float(g[i] & 0xffff0000u);
+    const float u0 = __uint_as_float(u[i] << 16), u1 = __uint_as_float(u[i] & 0xffff0000u);
+    o[i] = pack_bf16x2((GELU ? gelu_tanh(g0) : silu_f(g0)) * u0, (GELU ? gelu_tanh(g1) : silu_f(g1)) * u1);
+  }
+  *(u32x4_t*)(out + (size_t)r * ldo + f) = o;
 }
 
 // ROWS dot products of one vector b with ROWS rows a[r] over a lane's share of K, all loads of a step on
@@ -798,6 +814,22 @@ static int act_mul_launch(const void* gu, int ld, void* out, int ldo, int n_rows
       hipLaunchKernelGGL((silu_mul_kernel<bf16, false>), grid, block, 0, stream, (const bf16*)gu, ld, (bf16*)out, ldo, n_rows, F);
   }
   CHECK_LAUNCH("silu_mul");
+  return 0;
+}
+
+// act_mul of bfloat16 rows in which eight gate columns and the same eight of up stand by turns (F a multiple of 8; rows and
+// pointers of 16 bytes).
+extern "C" int act_mul_turns(const void* gu, int ld, void* out, int ldo, int n_rows, int F, int activation, hipStream_t stream) {
+  if (n_rows <= 0 || F <= 0) return 0;
+  if (activation != 0 && activation != 1) FAIL("act_mul_turns: unknown activation code %d", activation);
+  if (!gu || !out || (((uintptr_t)gu | (uintptr_t)out) & 15) || F % 8 != 0 || ld % 8 != 0 || ldo % 8 != 0 || ld < 2 * F || ldo < F)
+    FAIL("act_mul_turns: rows of %d for 2 x %d, output rows of %d, in whole pieces of 16 bytes", ld, F, ldo);
+  const dim3 grid(n_rows, (F / 8 + 255) / 256), block(256);
+  if (activation)
+    hipLaunchKernelGGL(silu_mul_turns_kernel<true>, grid, block, 0, stream, (const uint16_t*)gu, ld, (uint16_t*)out, ldo, F);
+  else
+    hipLaunchKernelGGL(silu_mul_turns_kernel<false>, grid, block, 0, stream, (const uint16_t*)gu, ld, (uint16_t*)out, ldo, F);
+  CHECK_LAUNCH("act_mul_turns");
   return 0;
 }
 

@@ -50,6 +50,7 @@
 #define FLAG_ACCUMULATE 2
 #define FLAG_OUT_F32 4
 #define FLAG_KV 8
+#define FLAG_GATED 64       // (GATED kernels) features of a block of 16: eight of the gate, then the same eight of what it gates
 #define FLAG_OUT_PACKED 16  // a bfloat16 out in tiles of 16 rows x 64 columns, in the weights' packed order
 
 #define NW 8        // waves per block
@@ -198,7 +199,10 @@ __device__ __forceinline__ void finish4(const DecodeGemmArgs& p, int m, int n, f
 // a row in NV float4).  MULTI: K is longer than one pass of NW * U k-blocks
 // (2048); only then is the second set of weight registers needed.  FEW: how rows that need no norm are copied; a
 // kernel each because a launch of 3 to 5 us waits for its instructions too (both ways in one cost 0.1 to 0.2 us).
-template <bool LN, bool MULTI, bool FEW>
+// GATED: the features come in pairs of eight, gate and what it gates, and out gets act(gate) * other (N / 2 columns):
+// both lie in one block's tile.  The activation's own launch took 3.9 us a layer beside a product of 6.5 (8 rows of 1,024 to
+// 2 x 2,688), the product with it takes what it took without.
+template <bool LN, bool MULTI, bool FEW, bool GATED = false>
 __global__ __launch_bounds__(NW * 64) void gemm_bf16_decode_kernel(DecodeGemmArgs p) {
   constexpr int NV = LN_MAX_V;
   constexpr int UU = MULTI ? 2 * U : U;  // k-blocks per pass and wave: long rows keep more in flight
@@ -424,6 +428,19 @@ __global__ __launch_bounds__(NW * 64) void gemm_bf16_decode_kernel(DecodeGemmArg
   if (tid < 256) {
 #pragma unroll
     for (int w = 0; w < NW; ++w) v += red[w][tid];
+  }
+  if constexpr (GATED) {
+    if (tid >= 128) return;  // (feature f's other is feature f + 8 of the same row: element tid + 128)
+    float other = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) other += red[w][tid + 128];
+    // (both as a product of more rows leaves them, so that a row's result does not depend on how many there are)
+    v = bits_to_f32(f32_to_bf16_bits(v)), other = bits_to_f32(f32_to_bf16_bits(other));
+    const int m = (tid >> 2) & 15;
+    if (m < p.M)
+      ((uint16_t*)p.out)[(size_t)m * p.ldo + n0 / 2 + 4 * (tid >> 6) + (tid & 3)] =
+          f32_to_bf16_bits(((p.flags & FLAG_GELU) ? gelu_tanh(v) : silu_f(v)) * other);
+    return;
   }
   if (tid < 256) {
     // element tid = 4 * L + r of the MFMA tile: feature 4 * (L / 16) + r, row L % 16
@@ -846,7 +863,7 @@ static int fill_epilogue(DecodeGemmArgs& p, const char* who, void* out, const fl
            q_width, kv_width, N, head_dim);
     if (flags & (FLAG_OUT_F32 | FLAG_ACT_ANY)) FAIL("%s: the cache scatter writes bfloat16, no activation", who);
     if (ldo < q_width) FAIL("%s: ldo=%d smaller than q_width=%d", who, ldo, q_width);
-  } else if (ldo < N && !(flags & FLAG_OUT_PACKED)) {
+  } else if (ldo < ((flags & FLAG_GATED) ? N / 2 : N) && !(flags & FLAG_OUT_PACKED)) {
     FAIL("%s: ldo=%d smaller than N=%d", who, ldo, N);
   }
   p.bias = bias, p.out = out, p.M = M, p.N = N, p.ldo = ldo, p.flags = flags;
@@ -895,7 +912,8 @@ static int decode_launch(
   p.K = K, p.lda = lda, p.ldx = ldx, p.ldw = ldw;
   // Few features and no split of K: blocks of eight features (half of each MFMA
   // tile is idle, which costs nothing here) put twice as many CUs to work.
-  p.rows = (n_splits == 1 && (N + 15) / 16 < few_blocks()) ? 8 : 16;
+  const bool gated = flags & FLAG_GATED;
+  p.rows = (n_splits == 1 && (N + 15) / 16 < few_blocks() && !gated) ? 8 : 16;
   p.n_splits = n_splits, p.chunks_per_split = chunks_per_split(K, n_splits);
   p.ws = ws;
   if (n_splits > 1) {
@@ -916,12 +934,14 @@ static int decode_launch(
   // two requests of GPT-2 XL 1,866 -> 1,830, of large 1,247 -> 1,230; with up to two pieces a thread 4 requests of XL
   // take 1,913 instead of 1,883).
   const bool few = !ln && (M <= 2 || M * (range / 8) <= NW * 64);
-  const int which = ln ? 0 : 1 + (multi ? 1 : 0) + (few ? 2 : 0);
-  void (*kernels[5])(DecodeGemmArgs) = {
+  const int which = (ln ? 0 : 1 + (multi ? 1 : 0) + (few ? 2 : 0)) + (gated ? 5 : 0);
+  void (*kernels[10])(DecodeGemmArgs) = {
       gemm_bf16_decode_kernel<true, false, false>, gemm_bf16_decode_kernel<false, false, false>,
       gemm_bf16_decode_kernel<false, true, false>, gemm_bf16_decode_kernel<false, false, true>,
-      gemm_bf16_decode_kernel<false, true, true>};
-  static size_t granted[5] = {0, 0, 0, 0, 0};
+      gemm_bf16_decode_kernel<false, true, true>, gemm_bf16_decode_kernel<true, false, false, true>,
+      gemm_bf16_decode_kernel<false, false, false, true>, gemm_bf16_decode_kernel<false, true, false, true>,
+      gemm_bf16_decode_kernel<false, false, true, true>, gemm_bf16_decode_kernel<false, true, true, true>};
+  static size_t granted[10] = {};
   const size_t fixed = sizeof(float) * (NW * 256 + (ln ? 2 * LN_MAX_V * 256 : 4));
   if (lds + fixed > 64 * 1024 && granted[which] < lds) {
     hipError_t e = hipFuncSetAttribute((const void*)kernels[which],
@@ -940,9 +960,20 @@ extern "C" int gemm_bf16_decode(
     int ldo, int flags, void* k_pages, void* v_pages, size_t page_stride, const int* block_table,
     int max_blocks, const int* token_req, const int* positions, int q_width, int kv_width,
     int head_dim, int page_size, int n_splits, float* ws, size_t ws_floats, hipStream_t stream) {
-  return decode_launch(out, A, lda, X, ldx, gamma, beta, eps, W, bias, M, N, K, ldw, ldo, flags, k_pages, v_pages, page_stride,
+  return decode_launch(out, A, lda, X, ldx, gamma, beta, eps, W, bias, M, N, K, ldw, ldo, flags & ~FLAG_GATED, k_pages, v_pages, page_stride,
                        block_table, max_blocks, token_req, positions, q_width, kv_width, head_dim, page_size, n_splits, ws,
                        ws_floats, nullptr, stream);
+}
+
+// out[m, f] = act(gate) * other of up to 16 rows and F features each (bfloat16 rows of stride ldo): W holds 2 F features in
+// the packed order, eight of the gate and the same eight of the other by turns (F a multiple of 8).  The rows are A, or X to be
+// normed first, as in gemm_bf16_decode; `activation` 0: silu, 1: the tanh form of gelu.
+extern "C" int gemm_bf16_decode_gated(void* out, const void* A, int lda, const float* X, int ldx, const float* gamma, const float* beta,
+                                      float eps, const void* W, int M, int F, int K, int ldo, int activation, hipStream_t stream) {
+  if (F <= 0 || F % 8 != 0) FAIL("gemm_bf16_decode_gated: %d features are not whole groups of eight", F);
+  if (activation != 0 && activation != 1) FAIL("gemm_bf16_decode_gated: unknown activation code %d", activation);
+  return decode_launch(out, A, lda, X, ldx, gamma, beta, eps, W, nullptr, M, 2 * F, K, 0, ldo, FLAG_GATED | (activation ? FLAG_GELU : 0),
+                       nullptr, nullptr, 0, nullptr, 0, nullptr, nullptr, 0, 0, 0, 0, 1, nullptr, 0, nullptr, stream);
 }
 
 // 1 if gemm_bf16_rows takes these sizes

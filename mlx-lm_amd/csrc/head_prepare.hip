@@ -26,7 +26,6 @@
 //   head_gate       x[t, h, :] *= sigmoid(g[t, h]), in place.
 #include "common.h"
 
-__device__ __forceinline__ float silu_f(float z) { return z / (1.0f + expf(-z)); }
 
 #define PREPARE_CONV_MAX_DIM 256  // the widest head that passes a convolution
 

@@ -22,7 +22,6 @@
 // and of the gated norm may be bfloat16.  Sums run in a fixed order.
 #include "common.h"
 
-__device__ __forceinline__ float silu_f(float z) { return z / (1.0f + expf(-z)); }
 __device__ __forceinline__ float softplus_f(float z) { return fmaxf(z, 0.f) + log1pf(expf(-fabsf(z))); }
 
 struct ScanArgs {

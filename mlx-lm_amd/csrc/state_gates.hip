@@ -10,7 +10,6 @@
 //                   together), float rows in, the compute dtype out; a block a row.
 #include "common.h"
 
-__device__ __forceinline__ float silu_f(float z) { return z / (1.0f + expf(-z)); }
 
 __global__ __launch_bounds__(256) void silu_columns_kernel(float* __restrict__ u, int ld, int col, int n) {
   const int c = blockIdx.y * 256 + threadIdx.x;

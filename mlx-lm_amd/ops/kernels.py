@@ -1490,6 +1490,46 @@ def silu_mul(out, gate_up, activation="silu"):
     return out
 
 
+def gate_in_turns(gate, up):
+    """``gate`` and ``up`` (``[F, K]``, ``F`` a multiple of 8) as one matrix: eight rows of the one and the same eight of the
+    other by turns, so that a product kernel's block of sixteen features holds both of every column it gates."""
+    F, K = gate.shape
+    return torch.stack([gate.view(F // 8, 8, K), up.view(F // 8, 8, K)], 1).view(2 * F, K)
+
+
+def gated_linear(alloc, out, x, w, activation="silu"):
+    """``out = act(x @ gate.T) * (x @ up.T)`` for a ``PackedWeight`` of ``gate_in_turns``.
+
+    Up to 16 rows (where the decode kernel takes them whole) in one launch, more in two,
+    with rows ``[x.shape[0], 2 F]`` from ``alloc(shape, dtype)`` between; rounded alike."""
+    M, K = x.shape
+    F = out.shape[1]
+    ldo = _rows2d(out, "out")
+    _need(isinstance(w, PackedWeight) and w.shape == (2 * F, K) and F % 8 == 0, "gated_linear: weights")
+    _need(out.dtype == torch.bfloat16 and x.dtype == torch.bfloat16 and out.shape[0] == M, "gated_linear: shapes")
+    _need(activation in GATE_ACTIVATIONS, f"gated_linear: activation {activation!r} (known: {sorted(GATE_ACTIVATIONS)})")
+    code = GATE_ACTIVATIONS[activation]
+    if 0 < M <= DECODE_MAX_ROWS and force_splits <= 0:
+        lib = build.load("gemm_bf16_decode")
+        lazy = isinstance(x, NormedInput) and lib.gemm_bf16_decode_takes(_c_int(M), _c_int(K), _c_int(1), _c_int(1))
+        if lazy or lib.gemm_bf16_decode_takes(_c_int(M), _c_int(K), _c_int(0), _c_int(1)):
+            if lazy:
+                _dev(x.x, "x", torch.float32)
+                rows = (None, _c_int(0), _ptr(x.x), _c_int(x.x.stride(0)), _ptr(x.gamma), None if x.rms else _ptr(x.beta), _c_float(x.eps))
+            else:
+                a = normed(x)
+                rows = (_ptr(a), _c_int(_rows2d(a, "x")), None, _c_int(0), None, None, _c_float(0.0))
+            rc = lib.gemm_bf16_decode_gated(_ptr(out), *rows, _ptr(w.packed), _c_int(M), _c_int(F), _c_int(K), _c_int(ldo), _c_int(code), _stream())
+            build.check(lib, rc, "gated_linear")
+            return out
+    both = alloc((M, 2 * F), torch.bfloat16)
+    linear(both, x, w, splits=splits_alone(M))
+    lib = build.load("experts")
+    rc = lib.act_mul_turns(_ptr(both), _c_int(_rows2d(both, "both")), _ptr(out), _c_int(ldo), _c_int(M), _c_int(F), _c_int(code), _stream())
+    build.check(lib, rc, "gated_linear")
+    return out
+
+
 EXPERT_ACTIVATIONS = {"silu": 0, "clamped": 1}
 
 

@@ -121,9 +121,10 @@ class Relu2MLP(FeedForward):
 class GatedMLP(OutputProduct, FeedForward):
     """``down(act(gate(x)) * up(x))``, dense, no biases; ``activation``: ``silu`` or ``gelu_tanh``.
 
-    One product gives ``[gate | up]``; the activation and the product of the two halves are one
-    kernel (``silu_mul``, which the experts' shared expert uses too); the second product adds into
-    ``residual`` (or writes it: ``OutputProduct``).  No counterpart in mlx_lm/models/gpt2.py, whose MLP (:71-80) has no gate.
+    One product gives gate and up; the activation and the product of the two are that product's
+    epilogue in a step of few bfloat16 tokens (``gated_linear``: packed weights, gate and up by turns),
+    one kernel more otherwise (``silu_mul`` on ``[gate | up]`` where the weights are rows); the second product adds
+    into ``residual`` (or writes it: ``OutputProduct``).  No counterpart in mlx_lm/models/gpt2.py, whose MLP (:71-80) has no gate.
     """
 
     graph_safe = True  # launches kernels only: a step of such parts can be recorded
@@ -155,17 +156,22 @@ class GatedMLP(OutputProduct, FeedForward):
             zeros = gate.new_zeros(pad, self.width)
             gate, up = torch.cat([gate, zeros]), torch.cat([up, zeros])
             down = torch.cat([down, down.new_zeros(self.width, pad)], dim=1)
-        self.gate_up_w = kernels.for_decode(torch.cat([gate, up]).contiguous())
+        # (packed weights: by turns, as gated_linear has them)
+        packs = gate.is_cuda and gate.dtype == torch.bfloat16
+        self.gate_up_w = kernels.for_decode(kernels.gate_in_turns(gate, up) if packs else torch.cat([gate, up]).contiguous())
         self.down_w = kernels.for_decode(down.contiguous())
         self.first_weight = self.gate_up_w
 
     def forward(self, ctx, x, residual):
         T, F = x.shape[0], self.inner_padded
         mark = ctx.scratch_mark()
-        gate_up = ctx.scratch((T, 2 * F), ctx.dtype)
-        kernels.linear(gate_up, x, self.gate_up_w, splits=kernels.splits_alone(T))
         act = ctx.scratch((T, F), ctx.dtype)
-        kernels.silu_mul(act, gate_up, self.activation)
+        if isinstance(self.gate_up_w, kernels.PackedWeight):
+            kernels.gated_linear(ctx.scratch, act, x, self.gate_up_w, self.activation)
+        else:
+            gate_up = ctx.scratch((T, 2 * F), ctx.dtype)
+            kernels.linear(gate_up, x, self.gate_up_w, splits=kernels.splits_alone(T))
+            kernels.silu_mul(act, gate_up, self.activation)
         self.output(residual, act, self.down_w)
         ctx.scratch_release(mark)
 

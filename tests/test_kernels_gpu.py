@@ -760,6 +760,44 @@ def test_attn_prefill_walks_around_the_one_that_two_groups_share(hd, edge, windo
     assert err < 2.5e-2, err
 
 
+@pytest.mark.parametrize("M", [1, 2, 3, 8, 9, 16, 17, 64, 65, 130])
+@pytest.mark.parametrize("F,K", [(8, 64), (24, 200), (1200, 520), (2688, 1024), (40, 2048), (72, 2568)])
+@pytest.mark.parametrize("rows,activation", [("plain", "silu"), ("rms", "silu"), ("layer", "gelu_tanh")])
+def test_gated_product(M, F, K, rows, activation):
+    """A gate and what it gates out of one product of weights by turns, in one launch up to 16 rows (the rows normed in it
+    where it holds them, K up to 2,048) and in two beyond, against 64 bits: rows rounded to bfloat16 once (a norm's), both
+    products and the output (a rounding is 2^-8 of a value at most; the gate's counts up to twice).  The bits are those of the
+    product and the activation apart."""
+    k = _k()
+    g = torch.Generator().manual_seed(M + F + K)
+    gate, up = ((torch.randn(F, K, generator=g) * K ** -0.5).to(torch.bfloat16) for _ in range(2))
+    w = k.PackedWeight(k.gate_in_turns(gate.to(DEV), up.to(DEV)), keep_rows=False)
+    x = torch.randn(M, K, generator=g)
+    alloc = lambda shape, dtype: torch.empty(shape, dtype=dtype, device=DEV)
+    if rows == "plain":
+        a = x.to(torch.bfloat16)
+        given = a.to(DEV)
+    else:
+        gamma, beta = torch.rand(K, generator=g) + 0.5, torch.randn(K, generator=g) * 0.1
+        given = k.NormedInput(alloc, x.to(DEV), gamma.to(DEV), None if rows == "rms" else beta.to(DEV), 1e-5, torch.bfloat16, rms=rows == "rms")
+        xd = x.double() if rows == "rms" else x.double() - x.double().mean(1, keepdim=True)
+        a = xd / torch.sqrt((xd * xd).mean(1, keepdim=True) + 1e-5) * gamma.double() + (0 if rows == "rms" else beta.double())
+        a = a.to(torch.bfloat16)
+    out = torch.full((M, F + 8), float("nan"), dtype=torch.bfloat16, device=DEV)
+    k.gated_linear(alloc, out[:, :F], given, w, activation)
+    z, u = a.double() @ gate.double().T, a.double() @ up.double().T
+    want = (z * torch.sigmoid(z) if activation == "silu" else 0.5 * z * (1 + torch.tanh(math.sqrt(2 / math.pi) * (z + 0.044715 * z ** 3)))) * u
+    err = ((out[:, :F].double().cpu() - want).norm() / want.norm()).item()
+    # (32-bit sums 1e-5; a norm's rounding may fall on the other side of a tie: a step of 2^-8 in few of the rows' values)
+    assert err < 2 ** -8 * (4 + (0.01 if rows == "plain" else 0.3)), err
+    both = torch.empty(M, 2 * F, dtype=torch.bfloat16, device=DEV)
+    k.linear(both, given, w, splits=1 if M <= 64 else None)
+    apart = torch.empty(M, F, dtype=torch.bfloat16, device=DEV)
+    k.silu_mul(apart, both.view(M, F // 8, 2, 8).transpose(1, 2).reshape(M, 2 * F), activation)
+    assert torch.equal(out[:, :F], apart)
+    assert torch.isnan(out[:, F:].float()).all()
+
+
 @pytest.mark.parametrize("ps", [8, 16, 64, 256])
 @pytest.mark.parametrize("H,Hkv", [(3, 1), (90, 9)])
 @pytest.mark.parametrize("window", [0, 65, 300])
