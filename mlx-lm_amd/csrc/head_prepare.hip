@@ -155,9 +155,172 @@ __device__ __forceinline__ void prepare_head(const PrepareArgs& a, long item, in
   }
 }
 
-template <typename T>
-__global__ __launch_bounds__(256) void head_prepare_kernel(PrepareArgs a) {
-  prepare_head<T>(a, (long)blockIdx.x * 4 + (threadIdx.x >> 6), threadIdx.x & 63);
+// The same for heads of up to 64 CPL columns, convolutions of up to four taps and norms over a head: what every mixer here
+// but those with wider heads or a norm over the whole projection has.  A wave takes R neighbouring rows of a head.
+//
+// What bounds it: at few rows the trips to memory that follow one another, at many rows the same trips, paid once a row and head by
+// the kernel above (which looks up a request, its first row, its state row and a page one after another, then takes the
+// taps and the norm's weights a load at a time: 1,357 rows of 32 heads of 64 and 8 of 128 through four taps 48 us, 8 rows 8.8; 1,357
+// rows of 16 heads of 224 and the latent 18.5).  Here what does not depend on the row's request (the rows with the R + 3 inputs that R outputs
+// need, taps, weights, angles) is on its way together with the request and the position, then first row, state row and page
+// together, then (only where a request's first rows are among them) the state: 27, 6.4 and 15.5 us.  The sums, and so the bits,
+// are those of the kernel above.
+#define PREPARE_TAPS 4
+template <typename T, int R, int CPL>
+__device__ __forceinline__ void prepare_rows(const PrepareArgs& a, int row0, int h, int lane, float* mine) {
+  const int first_col = a.src_col + h * a.src_stride;
+  const bool conv = a.conv_w != nullptr, pages = a.block_table != nullptr;
+  const int back = conv ? a.taps - 1 : 0;  // rows before a row that it needs
+  // lane r (of each R) looks things up for row row0 + r
+  const int my_row = min(row0 + lane % R, a.n_rows - 1);
+  int req = 0, position = 0;
+  if (conv || pages) req = a.token_req[my_row];
+  if (a.rot_dims || pages) position = a.positions[my_row];
+  int col[CPL];
+  float u[R + PREPARE_TAPS - 1][CPL], w[PREPARE_TAPS][CPL], weight[CPL], freq[CPL];
+#pragma unroll
+  for (int c = 0; c < CPL; ++c) col[c] = min(lane + 64 * c, a.dim - 1);  // (columns beyond the head: the last one's values, not used)
+#pragma unroll
+  for (int i = 0; i < R + PREPARE_TAPS - 1; ++i) {
+    if (i < PREPARE_TAPS - 1 - back) continue;  // (uniform)
+    const float* s = a.src + (size_t)min(max(row0 - (PREPARE_TAPS - 1) + i, 0), a.n_rows - 1) * a.lds + first_col;
+#pragma unroll
+    for (int c = 0; c < CPL; ++c) u[i][c] = s[col[c]];
+  }
+  if (conv)
+#pragma unroll
+    for (int j = 0; j < PREPARE_TAPS; ++j)
+      if (j < a.taps)
+#pragma unroll
+        for (int c = 0; c < CPL; ++c) w[j][c] = a.conv_w[(size_t)(first_col + col[c]) * a.taps + (a.taps - 1 - j)];
+  const int half = a.rot_dims / 2;
+#pragma unroll
+  for (int c = 0; c < CPL; ++c) {
+    weight[c] = a.norm_dim > 0 && a.norm_w ? a.norm_w[min(col[c], a.norm_dim - 1)] : 1.f;
+    if (a.rot_dims) {
+      const int rel = min(max(col[c] - a.rot_off, 0), a.rot_dims - 1);
+      freq[c] = a.inv_freq[a.interleaved ? rel >> 1 : rel < half ? rel : rel - half];
+    }
+  }
+  int local = 0, slot = 0, page = 0;
+  if (conv) local = my_row - a.seq_start[req], slot = a.slot_ids[req];
+  if (pages) page = a.block_table[(size_t)req * a.max_blocks + position / a.page_size];
+
+  float v[R][CPL];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    if (!conv) {
+#pragma unroll
+      for (int c = 0; c < CPL; ++c) v[r][c] = u[PREPARE_TAPS - 1 + r][c];
+      continue;
+    }
+    const int at_start = __builtin_amdgcn_readlane(local, r);  // rows of the request before this one in this step
+    float in[PREPARE_TAPS][CPL];
+#pragma unroll
+    for (int j = 0; j < PREPARE_TAPS; ++j)
+#pragma unroll
+      for (int c = 0; c < CPL; ++c) in[j][c] = u[PREPARE_TAPS - 1 + r - j][c];
+    if (at_start < back) {  // (uniform) inputs of earlier steps, the latest last
+      const float* old = a.conv_state + (size_t)__builtin_amdgcn_readlane(slot, r) * a.conv_state_stride + a.conv_offset + first_col;
+#pragma unroll
+      for (int j = 1; j < PREPARE_TAPS; ++j)
+        if (j < a.taps && at_start - j < 0)
+#pragma unroll
+          for (int c = 0; c < CPL; ++c) in[j][c] = old[(size_t)(back + at_start - j) * a.conv_channels + col[c]];
+    }
+#pragma unroll
+    for (int c = 0; c < CPL; ++c) v[r][c] = 0.f;
+#pragma unroll
+    for (int j = PREPARE_TAPS - 1; j >= 0; --j)  // the oldest input first
+      if (j < a.taps)
+#pragma unroll
+        for (int c = 0; c < CPL; ++c) v[r][c] += w[j][c] * in[j][c];
+  }
+  if (a.norm_dim > 0) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      float q = 0.f;
+#pragma unroll
+      for (int c = 0; c < CPL; ++c)
+        if (lane + 64 * c < a.norm_dim) q += v[r][c] * v[r][c];
+      const float rstd = 1.0f / sqrtf(wave_sum(q) / (float)a.norm_dim + a.eps);
+#pragma unroll
+      for (int c = 0; c < CPL; ++c)
+        if (lane + 64 * c < a.norm_dim) v[r][c] = v[r][c] * rstd * weight[c];
+    }
+  }
+  if (a.rot_dims) {
+    // a column's partner is another lane's: through the wave's own piece of LDS
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+      for (int c = 0; c < CPL; ++c) mine[(r * CPL + c) * 64 + lane] = v[r][c];
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int c = 0; c < CPL; ++c) {
+      const int k = lane + 64 * c, rel = k - a.rot_off;
+      const bool turns = rel >= 0 && rel < a.rot_dims && k < a.dim;
+      if (!__any(turns)) continue;
+      const bool first = a.interleaved ? !(rel & 1) : rel < half;  // this column is the pair's first member
+      const int partner = a.interleaved ? (first ? k + 1 : k - 1) : first ? k + half : k - half;
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        float sn, cs;
+        sincosf((float)__builtin_amdgcn_readlane(position, r) * freq[c], &sn, &cs);
+        sn *= a.rot_mult, cs *= a.rot_mult;
+        const float other = mine[r * CPL * 64 + (turns ? partner : k)];
+        const float turned = first ? v[r][c] * cs - other * sn : v[r][c] * cs + other * sn;
+        v[r][c] = turns ? turned : v[r][c];
+      }
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    if (row0 + r >= a.n_rows) break;
+    const int pos = __builtin_amdgcn_readlane(position, r);
+    size_t base = (size_t)(row0 + r) * a.ldd, head = a.dst_stride;
+    if (pages) {
+      base = (size_t)__builtin_amdgcn_readlane(page, r) * a.page_stride + (size_t)(pos % a.page_size) * a.dst_stride;
+      head = (size_t)a.page_size * a.dst_stride;
+    }
+    for (int k = 0; k < a.copies; ++k) {
+      T* out = (T*)a.dst + base + (size_t)(a.dst_head ? a.dst_head[k * a.n_heads + h] : h) * head;
+#pragma unroll
+      for (int c = 0; c < CPL; ++c)
+        if (lane + 64 * c < a.dst_fill) out[lane + 64 * c] = from_f32<T>(lane + 64 * c < a.dim ? v[r][c] : 0.f);
+    }
+  }
+  if (R == 1 && conv && a.conv_single && a.taps > 1) {
+    // every request brings one token: this wave alone has its request's inputs of this head's channels and moves them up by one
+    float* old = a.conv_state + (size_t)__builtin_amdgcn_readlane(slot, 0) * a.conv_state_stride + a.conv_offset + first_col;
+#pragma unroll
+    for (int c = 0; c < CPL; ++c) {
+      if (lane + 64 * c >= a.dim) continue;
+      float next[PREPARE_TAPS];
+#pragma unroll
+      for (int j = 0; j + 2 < PREPARE_TAPS; ++j)
+        if (j + 2 < a.taps) next[j] = old[(size_t)(j + 1) * a.conv_channels + lane + 64 * c];
+#pragma unroll
+      for (int j = 0; j + 2 < PREPARE_TAPS; ++j)
+        if (j + 2 < a.taps) old[(size_t)j * a.conv_channels + lane + 64 * c] = next[j];
+      old[(size_t)(a.taps - 2) * a.conv_channels + lane + 64 * c] = u[PREPARE_TAPS - 1][c];
+    }
+  }
+}
+template <typename T, int R>
+__device__ __forceinline__ void prepare_any(const PrepareArgs& a, long item, int lane, float* mine) {
+  if (item >= (long)((a.n_rows + R - 1) / R) * a.n_heads) return;  // whole waves leave; no barrier follows
+  const int row0 = (int)(item / a.n_heads) * R, h = (int)(item % a.n_heads);
+  if (a.dst_fill <= 64)
+    prepare_rows<T, R, 1>(a, row0, h, lane, mine);
+  else if (a.dst_fill <= 128)
+    prepare_rows<T, R, 2>(a, row0, h, lane, mine);
+  else
+    prepare_rows<T, R, 4>(a, row0, h, lane, mine);
+}
+static bool prepared_in_rows(const PrepareArgs& a) {
+  return a.dst_fill <= 256 && a.norm_whole == 0 && (!a.conv_w || a.taps <= PREPARE_TAPS);
 }
 
 // Several preparations in one launch (a mixer's queries, keys and values): the blocks of each
@@ -174,6 +337,15 @@ __global__ __launch_bounds__(256) void head_prepare_many_kernel(PrepareMany m) {
   int s = 0;
   while (s + 1 < m.n && blockIdx.x >= m.first_block[s + 1]) ++s;
   prepare_head<T>(m.seg[s], (long)(blockIdx.x - m.first_block[s]) * 4 + (threadIdx.x >> 6), threadIdx.x & 63);
+}
+
+template <typename T, int R>
+__global__ __launch_bounds__(256) void head_prepare_rows_kernel(PrepareMany m) {
+  __shared__ float turning[4][R * 256];
+  int s = 0;
+  while (s + 1 < m.n && blockIdx.x >= m.first_block[s + 1]) ++s;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  prepare_any<T, R>(m.seg[s], (long)(blockIdx.x - m.first_block[s]) * 4 + wave, threadIdx.x & 63, turning[wave]);
 }
 
 // A wave a (row, head).
@@ -237,19 +409,27 @@ static int prepare_args_fit(const PrepareArgs& a) {
   return 0;
 }
 
-extern "C" int head_prepare(const PrepareArgs* args, int dst_dtype, hipStream_t stream) {
-  const PrepareArgs& a = *args;
-  if (a.n_rows <= 0 || a.n_heads <= 0) return 0;
-  if (prepare_args_fit(a)) return 1;
-  if (dst_dtype != DT_F32 && dst_dtype != DT_BF16) FAIL("head_prepare: unknown dtype code %d", dst_dtype);
-  const long items = (long)a.n_rows * a.n_heads;
-  dim3 grid((unsigned)((items + 3) / 4)), block(256);
-  if (dst_dtype == DT_F32)
-    hipLaunchKernelGGL(head_prepare_kernel<float>, grid, block, 0, stream, a);
+// Rows a wave takes where there are many: eight leave a wave's lookups an eighth a row.  Fewer rows than 128 would not give
+// the compute units a block each (16 heads: 128 / 8 x 16 / 4 = 64 blocks, with three preparations a launch 160).
+#define PREPARE_ROWS 8
+#define PREPARE_ROWS_FROM 128
+template <typename T>
+static void launch_many(PrepareMany& m, bool in_rows, hipStream_t stream) {
+  bool many = in_rows;
+  for (int i = 0; i < m.n; ++i) many = many && m.seg[i].n_rows >= PREPARE_ROWS_FROM && !(m.seg[i].conv_w && m.seg[i].conv_single);
+  const int R = many ? PREPARE_ROWS : 1;
+  unsigned blocks = 0;
+  for (int i = 0; i < m.n; ++i) {
+    m.first_block[i] = blocks;
+    blocks += (unsigned)(((long)((m.seg[i].n_rows + R - 1) / R) * m.seg[i].n_heads + 3) / 4);
+  }
+  for (int i = m.n; i <= PREPARE_MOST; ++i) m.first_block[i] = blocks;
+  if (many)
+    hipLaunchKernelGGL((head_prepare_rows_kernel<T, PREPARE_ROWS>), dim3(blocks), dim3(256), 0, stream, m);
+  else if (in_rows)
+    hipLaunchKernelGGL((head_prepare_rows_kernel<T, 1>), dim3(blocks), dim3(256), 0, stream, m);
   else
-    hipLaunchKernelGGL(head_prepare_kernel<bf16>, grid, block, 0, stream, a);
-  CHECK_LAUNCH("head_prepare");
-  return 0;
+    hipLaunchKernelGGL(head_prepare_many_kernel<T>, dim3(blocks), dim3(256), 0, stream, m);
 }
 
 // `n` preparations (1 to 4) whose outputs are all of `dst_dtype`, in one launch.
@@ -258,23 +438,25 @@ extern "C" int head_prepare_many(const PrepareArgs* args, int n, int dst_dtype, 
   if (dst_dtype != DT_F32 && dst_dtype != DT_BF16) FAIL("head_prepare: unknown dtype code %d", dst_dtype);
   PrepareMany m;
   m.n = 0;
-  unsigned blocks = 0;
+  bool in_rows = true;
   for (int i = 0; i < n; ++i) {
     const PrepareArgs& a = args[i];
     if (a.n_rows <= 0 || a.n_heads <= 0) continue;
     if (prepare_args_fit(a)) return 1;
-    m.seg[m.n] = a, m.first_block[m.n] = blocks;
-    blocks += (unsigned)(((long)a.n_rows * a.n_heads + 3) / 4);
-    ++m.n;
+    in_rows = in_rows && prepared_in_rows(a);
+    m.seg[m.n++] = a;
   }
   if (m.n == 0) return 0;
-  for (int i = m.n; i <= PREPARE_MOST; ++i) m.first_block[i] = blocks;
   if (dst_dtype == DT_F32)
-    hipLaunchKernelGGL(head_prepare_many_kernel<float>, dim3(blocks), dim3(256), 0, stream, m);
+    launch_many<float>(m, in_rows, stream);
   else
-    hipLaunchKernelGGL(head_prepare_many_kernel<bf16>, dim3(blocks), dim3(256), 0, stream, m);
+    launch_many<bf16>(m, in_rows, stream);
   CHECK_LAUNCH("head_prepare_many");
   return 0;
+}
+
+extern "C" int head_prepare(const PrepareArgs* args, int dst_dtype, hipStream_t stream) {
+  return head_prepare_many(args, 1, dst_dtype, stream);
 }
 
 extern "C" int diff_combine(const void* att, int lda, int head_stride, const int* first, const int* second, float lambda,

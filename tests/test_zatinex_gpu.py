@@ -146,6 +146,70 @@ def test_heads_normed_turned_and_placed(dtype):
     assert (dst2.double().cpu()[:, :14] - want2).abs().max() <= tol and (dst2[:, 14:] == 0).all()
 
 
+@pytest.mark.parametrize("rows", [5, 127, 128, 131, 300])
+@pytest.mark.parametrize("dim,fill,norm,rot_off,rot_dims,taps", [(64, 64, 64, 0, 64, 4), (64, 64, 0, 0, 0, 3), (100, 128, 90, 90, 10, 2),
+                                                                 (224, 256, 192, 192, 32, None), (130, 136, 130, 2, 128, 4), (40, 64, 40, 0, 8, 5)])
+@pytest.mark.parametrize("interleaved", [False, True])
+def test_heads_prepared_in_runs_of_rows(rows, dim, fill, norm, rot_off, rot_dims, taps, interleaved):
+    """Runs of rows of one wave around where they begin (128 rows) and end (a remainder), requests of one to three rows (fewer
+    than the taps) and longer ones in a run, earlier inputs in the state; heads of one, two and four columns a lane, a head with
+    more taps than a run takes; rows of a matrix and, in the same launch, a cache's pages."""
+    from mlx_lm_amd.ops import kernels
+
+    H, ps = 3, 16
+    g = torch.Generator().manual_seed(rows + dim)
+    lens = []
+    while sum(lens) < rows:
+        lens.append(min([1, 3, 2, 40, 1, 1, 77, 9][len(lens) % 8], rows - sum(lens)))
+    R, C = len(lens), H * dim + 4
+    known = torch.randint(0, 50, (R,), generator=g).tolist()
+    src = torch.randn(rows, C, generator=g)
+    nw = 1 + 0.3 * torch.randn(max(norm, 1), generator=g)
+    freq = 10.0 ** -torch.rand(max(rot_dims // 2, 1), generator=g)
+    req = sum([[r] * n for r, n in enumerate(lens)], [])
+    starts = [sum(lens[:r]) for r in range(R)]
+    pos = [known[r] + i - starts[r] for i, r in enumerate(req)]
+    slots = torch.randperm(R, generator=g).tolist()
+    t = taps or 1
+    state = torch.randn(R, 5 + (t - 1) * C, generator=g)
+    w = torch.randn(C, t, generator=g)
+    options = dict(dst_stride=fill, dst_fill=fill, norm_dim=norm, norm_weight=nw.cuda() if norm else None, eps=1e-4, rot_off=rot_off,
+                   rot_dims=rot_dims, inv_freq=freq.cuda() if rot_dims else None, rot_mult=0.9, positions=_ints(pos), interleaved=interleaved)
+    if taps:
+        options["conv"] = kernels.ConvolutionAhead(w.cuda(), state.cuda(), 5, _ints(req), _ints(starts), _ints(slots), single=False)
+    x = src.double()
+    if taps:
+        parts = []
+        for r, n in enumerate(lens):
+            old = state[slots[r], 5:].double().view(t - 1, C)
+            parts.append(plain.causal_conv(torch.cat([old, x[starts[r] : starts[r] + n]]), w.double())[t - 1 :])
+        x = torch.cat(parts)
+    want = x[:, : H * dim].reshape(rows, H, dim).clone()
+    if norm:
+        want[..., :norm] = plain.rms_norm(want[..., :norm], nw.double(), 1e-4)
+    if rot_dims:
+        a = (torch.tensor(pos)[:, None].float() * freq[None]).double()[:, None]  # (the angle is a 32-bit product)
+        part = want[..., rot_off : rot_off + rot_dims]
+        one, two = (part[..., 0::2], part[..., 1::2]) if interleaved else (part[..., : rot_dims // 2], part[..., rot_dims // 2 :])
+        first, second = 0.9 * (one * a.cos() - two * a.sin()), 0.9 * (two * a.cos() + one * a.sin())
+        want[..., rot_off : rot_off + rot_dims] = torch.stack([first, second], -1).flatten(-2) if interleaved else torch.cat([first, second], -1)
+    blocks = [(k + n + ps - 1) // ps for k, n in zip(known, lens)]
+    pool = torch.full((sum(blocks), 2, H, ps, fill), 7.0, device="cuda")
+    kv = kernels.PagedKV(pool[:, 0], pool[:, 1])
+    table, at = torch.full((R, max(blocks)), -1, dtype=torch.int32), 0
+    for r, n in enumerate(blocks):
+        table[r, :n] = torch.arange(at, at + n)
+        at += n
+    out = torch.full((rows, H * fill + 3), 7.0, device="cuda")
+    pages = kernels.PagesOut(kv, True, table.cuda(), _ints(req), _ints(pos))
+    kernels.head_prepare_many((out, src.cuda(), 0, H, dim, options), (pages, src.cuda(), 0, H, dim, options))
+    got = out.double().cpu()[:, : H * fill].view(rows, H, fill)
+    scale = want.abs().max()
+    assert (got[..., :dim] - want).abs().max() <= 1e-5 * scale and (got[..., dim:] == 0).all() and (out[:, H * fill :] == 7.0).all()
+    placed = torch.stack([pool[table[r, p // ps], 1, :, p % ps] for r, p in zip(req, pos)]).double().cpu()
+    assert torch.equal(placed, got) and (pool[:, 0] == 7.0).all()
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_two_maps_joined_and_heads_gated(dtype):
     from mlx_lm_amd.ops import kernels
