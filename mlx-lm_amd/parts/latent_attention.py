@@ -132,9 +132,8 @@ class LatentAttention(ProjectsFirst, Mixer):
                                                                eps=self.eps, **rot)))
         kernels.head_prepare_many(*calls)  # (queries and the latent in one launch)
         att = ctx.scratch((T, H * hd), ctx.dtype)
-        kernels.attend(ctx, att, q, cache, H, 1, hd, self.scale, self.window)
-        if self.gate:
-            kernels.head_gate(att, hd, H, u[:, Q:Q + H])
+        terms = kernels.ScoreTerms(head_gate=u[:, Q:Q + H]) if self.gate else None  # (on the attention's way out, in 32 bits)
+        kernels.attend(ctx, att, q, cache, H, 1, hd, self.scale, self.window, terms)
         kernels.linear(residual, att, self.out_w, accumulate=True, splits=kernels.splits_alone(T))
         ctx.scratch_release(mark)
 
