@@ -232,8 +232,11 @@ class PackedWeight:
         self.shape, self.dtype, self.device = tuple(w.shape), w.dtype, w.device
         N, K = w.shape
         Np, Kp = (N + 15) // 16 * 16, (K + 63) // 64 * 64
-        padded = torch.zeros((Np, Kp), dtype=w.dtype, device=w.device)
-        padded[:N, :K] = w
+        if (Np, Kp) == (N, K):
+            padded = w.contiguous()
+        else:
+            padded = torch.zeros((Np, Kp), dtype=w.dtype, device=w.device)
+            padded[:N, :K] = w
         # (block, feature, k-block, k group, half, 8) -> (block, k-block, half, k group, feature, 8)
         t = padded.view(Np // 16, 16, Kp // 64, 4, 2, 8).permute(0, 2, 4, 3, 1, 5)
         self.packed = t.contiguous().view(-1)
