@@ -118,32 +118,43 @@ __device__ __forceinline__ bool tile_of_block(int tiles_m, int tiles_n, int& tm,
   return true;
 }
 
-// The shape of a block: WAVES_M x WAVES_N waves, each with TM x TN MFMA tiles of 32 x 32, and a ring of STAGES k-blocks
-// in LDS.  What bounds this kernel is how fast a CU is fed from the L2s (some 32 to 39 bytes a cycle arrive, measured with
+// The shape of a block: WAVES_M x WAVES_N waves, each with TM x TN MFMA tiles of 32 x 32, and rings in LDS of SLOTS_A
+// k-blocks of the rows and SLOTS_B of the weights.  What bounds this kernel is how fast a CU is fed from the L2s (some 32 to 39 bytes a cycle arrive, measured with
 // the products taken out), so the larger the tile, the fewer bytes per product: 256 x 256 where the matrix gives a tile
 // to every CU, smaller ones where it does not; `price` below chooses.  Eight waves (but for 32 rows): two a SIMD cover each
 // other's waits for LDS; four waves of 64 x 64 were level or up to 12 % behind.
-template <int WAVES_M_, int WAVES_N_, int TM_, int TN_, int STAGES_, int PANEL_, int WAVES_PER_SIMD_>
+// The widest shapes have room for two k-blocks of both and what is left goes to the weights, which come from memory while
+// the rows lie in the L2s; their copies are asked for a few at a time between products (SPREAD): a wave that asks waits
+// until its copies are taken, 64 KB a k-block, and right behind the barrier all waves did so at once, the matrix units idle.  Zeros, so that
+// power does not limit, 256 x 256, a k-block: products alone 0.87 us, copies alone 0.96, both 1.28 and now 1.10; from memory, rows x features x K:
+// 2,048 x 4,800 x 1,600 37.4 -> 33.6 us, x 6,400 x 1,600 47.4 -> 43.8, 8,000 x 4,800 x 1,600 128.3 -> 124, 8,000 x 1,280 x 5,120 111 -> 104.  The
+// smaller shapes were level or up to 3 % slower with either (128 x 128 with five slots, 64 x 128 with six: what they wait for is not depth).
+template <int WAVES_M_, int WAVES_N_, int TM_, int TN_, int SLOTS_A_, int PANEL_, int WAVES_PER_SIMD_, int SLOTS_B_ = SLOTS_A_, bool SPREAD_ = false>
 struct TileShape {
-  static constexpr int WAVES_M = WAVES_M_, WAVES_N = WAVES_N_, TM = TM_, TN = TN_, STAGES = STAGES_;
+  static constexpr int WAVES_M = WAVES_M_, WAVES_N = WAVES_N_, TM = TM_, TN = TN_, SLOTS_A = SLOTS_A_, SLOTS_B = SLOTS_B_;
+  static constexpr bool SPREAD = SPREAD_;
   static constexpr int PANEL = PANEL_, WAVES_PER_SIMD = WAVES_PER_SIMD_;  // PANEL: rows of tiles that share a die's L2
   static constexpr int WAVES = WAVES_M * WAVES_N, THREADS = 64 * WAVES;
   static constexpr int BM = WAVES_M * TM * 32, BN = WAVES_N * TN * 32;
   static constexpr int PA = BM / 8 / WAVES, PB = BN / 8 / WAVES;  // copies of 1 KB a wave asks for per k-block
   static constexpr int COPIES = PA + PB;
-  static constexpr int STAGE_BYTES = (BM + BN) * BK * 2;
+  static constexpr int A_BYTES = BM * BK * 2, B_BYTES = BN * BK * 2, RING = SLOTS_A * A_BYTES + SLOTS_B * B_BYTES;
+  // as many slots for both: a k-block's rows and weights side by side, one address for both; else a ring behind the other
+  static constexpr bool ALIKE = SLOTS_A == SLOTS_B;
+  static constexpr int A_STRIDE = ALIKE ? A_BYTES + B_BYTES : A_BYTES, B_STRIDE = ALIKE ? A_STRIDE : B_BYTES;
+  static constexpr int B_BASE = ALIKE ? A_BYTES : SLOTS_A * A_BYTES;
   static_assert(BM % (8 * WAVES) == 0 && BN % (8 * WAVES) == 0, "a wave copies whole kilobytes");
-  static_assert(STAGES * STAGE_BYTES <= 160 * 1024, "the ring fits a CU's LDS");
+  static_assert(RING <= 160 * 1024, "the rings fit a CU's LDS");
 };
-using Tile256 = TileShape<2, 4, 4, 2, 2, 4, 2>;
-using Tile256x192 = TileShape<4, 2, 2, 3, 2, 4, 2>;
-using Tile256x128 = TileShape<4, 2, 2, 2, 3, 4, 2>;
+using Tile256 = TileShape<2, 4, 4, 2, 2, 4, 2, 3, true>;
+using Tile256x192 = TileShape<4, 2, 2, 3, 2, 4, 2, 4, true>;
+using Tile256x128 = TileShape<4, 2, 2, 2, 3, 4, 2, 4, true>;
 using Tile128 = TileShape<2, 4, 2, 1, 4, 8, 2>;
 using Tile128Pair = TileShape<2, 4, 2, 1, 2, 8, 4>;  // two blocks a CU (pairs_of_blocks below)
 using Tile64x128 = TileShape<2, 4, 1, 1, 3, 8, 4>;  // two blocks a CU, as the next
 using Tile32x128 = TileShape<1, 4, 1, 1, 4, 8, 2>;
 
-// Pipeline: k-block kb is multiplied out of one slot of the ring while those up to kb + STAGES - 1 are on their way into
+// Pipeline: k-block kb is multiplied out of one slot of each ring while the next ones are on their way into
 // the others (lds_copy.h); one wait by count and one barrier a k-block.  Nothing passes through registers but the operands,
 // which are read a quarter of a k-block (16 columns) ahead of their products: left to the compiler, each read stood next
 // to its product (2,048 x 4,800 x 1,600: 36.0 us, 34.0 read ahead; 8,000 x 1,600 x 6,400: 178.7 and 167.0).  Before, the k-blocks went through
@@ -155,9 +166,9 @@ using Tile32x128 = TileShape<1, 4, 1, 1, 4, 8, 2>;
 // PACKED: W lies in the decode kernels' packed order.
 template <typename S, bool SPLIT, bool PACKED>
 __global__ __launch_bounds__(S::THREADS, S::WAVES_PER_SIMD) void gemm_bf16_tile_kernel(GemmArgs p) {
-  constexpr int BM = S::BM, BN = S::BN, TM = S::TM, TN = S::TN, PA = S::PA, PB = S::PB, STAGES = S::STAGES;
+  constexpr int BM = S::BM, BN = S::BN, TM = S::TM, TN = S::TN, PA = S::PA, PB = S::PB;
   // (one buffer: the epilogue uses it again for the output tiles)
-  __shared__ __attribute__((aligned(1024))) uint16_t smem[STAGES * S::STAGE_BYTES / 2];
+  __shared__ __attribute__((aligned(1024))) uint16_t smem[S::RING / 2];
 
   int tm, tn;
   if (!tile_of_block<S::PANEL>((p.M + BM - 1) / BM, (p.N + BN - 1) / BN, tm, tn)) return;
@@ -208,23 +219,34 @@ __global__ __launch_bounds__(S::THREADS, S::WAVES_PER_SIMD) void gemm_bf16_tile_
     }
   }
   const uint32_t ring = lds_address(smem);
-  const uint32_t a_to = ring + wave * PA * 1024, b_to = ring + BM * BK * 2 + wave * PB * 1024;
+  const uint32_t a_to = ring + wave * PA * 1024, b_to = ring + S::B_BASE + wave * PB * 1024;
+  // What a round asks for: rows' k-block ka into slot sa and weights' k-block kb into slot sb, copy by copy.
   // (k-blocks beyond the last are asked for too, as nothing: the waits then count the same copies in every round)
-  auto ask = [&](int kb, int slot) __attribute__((always_inline)) {
-    const bool live = kb < n_blocks;
-    const int k_left = live ? p.K - (kb_lo + kb) * BK : 0;  // columns from this k-block on
-    const uint32_t at = (uint32_t)slot * S::STAGE_BYTES;
-    const uint32_t k2 = (uint32_t)(kb_lo + kb) * (BK * 2), w2 = PACKED ? k2 * 16 : k2;
-#pragma unroll
-    for (int i = 0; i < PA; ++i) copy16_to_lds(a_buf, piece_of(wave * PA + i) * 8 < k_left ? a_from[i] : COPY_NOTHING, k2, a_to + at + i * 1024);
-#pragma unroll
-    for (int i = 0; i < PB; ++i) 
-      copy16_to_lds(b_buf, (PACKED ? live : piece_of(wave * PB + i) * 8 < k_left) ? b_from[i] : COPY_NOTHING, w2, b_to + at + i * 1024);
+  struct Round {
+    int k_left_a, k_left_b;  // columns from the k-block on
+    uint32_t a_at, a_k, b_at, b_k;
+  };
+  auto round_of = [&](int ka, int sa, int kb, int sb) __attribute__((always_inline)) {
+    Round q;
+    q.k_left_a = ka < n_blocks ? p.K - (kb_lo + ka) * BK : 0;
+    q.k_left_b = S::ALIKE ? q.k_left_a : kb < n_blocks ? p.K - (kb_lo + kb) * BK : 0;
+    q.a_at = (uint32_t)sa * S::A_STRIDE, q.b_at = S::ALIKE ? q.a_at : (uint32_t)sb * S::B_STRIDE;
+    q.a_k = (uint32_t)(kb_lo + ka) * (BK * 2), q.b_k = (uint32_t)(kb_lo + kb) * (BK * 2 * (PACKED ? 16 : 1));
+    return q;
+  };
+  auto ask = [&](const Round& q, int i) __attribute__((always_inline)) {
+    if (i < PA) {
+      copy16_to_lds(a_buf, piece_of(wave * PA + i) * 8 < q.k_left_a ? a_from[i < PA ? i : 0] : COPY_NOTHING, q.a_k, a_to + q.a_at + i * 1024);
+    } else {
+      const int j = i < PA ? 0 : i - PA;
+      copy16_to_lds(b_buf, (PACKED ? q.k_left_b > 0 : piece_of(wave * PB + j) * 8 < q.k_left_b) ? b_from[j] : COPY_NOTHING, q.b_k,
+                    b_to + q.b_at + j * 1024);
+    }
   };
 
   const int row32 = lane & 31, hi = lane >> 5;
   const char* const a_row = (const char*)smem + (wm * TM * 32 + row32) * 128;
-  const char* const b_row = (const char*)smem + BM * BK * 2 +
+  const char* const b_row = (const char*)smem + S::B_BASE +
                             (PACKED ? ((wn * TN * 2 + (row32 >> 4)) * 2 + hi) * 1024 + (row32 & 15) * 16 : (wn * TN * 32 + row32) * 128);
 
   // Without a split the tiles are accumulated transposed (the weights' rows as the MFMA's rows):
@@ -238,9 +260,10 @@ __global__ __launch_bounds__(S::THREADS, S::WAVES_PER_SIMD) void gemm_bf16_tile_
   // The operands of 16 columns (a quarter of a k-block) go to registers one quarter ahead of their products, also
   // across the barrier: a k-block's last quarter is multiplied after the barrier that lets the next one be read.
   bf16x8_t fa[2][TM], fb[2][TN];
-  auto read_quarter = [&](int set, int slot, int q) __attribute__((always_inline)) {
-    const char* af = a_row + slot * S::STAGE_BYTES;
-    const char* bf = b_row + slot * S::STAGE_BYTES;
+  int slot_a = 0, slot_b = 0;
+  auto read_quarter = [&](int set, int q) __attribute__((always_inline)) {
+    const char* af = a_row + slot_a * S::A_STRIDE;
+    const char* bf = b_row + (S::ALIKE ? slot_a : slot_b) * S::B_STRIDE;
     const int s = ((2 * q + hi) ^ ((row32 >> 1) & 7)) * 16;
 #pragma unroll
     for (int i = 0; i < TM; ++i) fa[set][i] = *(const bf16x8_t*)(af + i * 32 * 128 + s);
@@ -248,32 +271,59 @@ __global__ __launch_bounds__(S::THREADS, S::WAVES_PER_SIMD) void gemm_bf16_tile_
     for (int j = 0; j < TN; ++j) fb[set][j] = *(const bf16x8_t*)(PACKED ? bf + j * 4096 + q * 256 : bf + j * 32 * 128 + s);
     __builtin_amdgcn_sched_barrier(0);
   };
-  auto multiply = [&](int set) __attribute__((always_inline)) {
+  // The products of a quarter; with SPREAD copies `from` up to `to` of a round go between them.
+  constexpr int TAKES = S::SPREAD ? (S::COPIES + 1) / 2 : S::COPIES;  // copies asked for beside a quarter's products, or at once
+  auto multiply = [&](int set, const Round& round, int from, int to) __attribute__((always_inline)) {
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
-      for (int j = 0; j < TN; ++j) acc[i][j] = mfma_tile(fa[set][i], fb[set][j], acc[i][j]);
+      for (int j = 0; j < TN; ++j) {
+        acc[i][j] = mfma_tile(fa[set][i], fb[set][j], acc[i][j]);
+        const int done = i * TN + j, n = to - from;
+        if ((done + 1) * n / (TM * TN) > done * n / (TM * TN)) {
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int c = done * n / (TM * TN); c < (done + 1) * n / (TM * TN); ++c) ask(round, from + c);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
     __builtin_amdgcn_sched_barrier(0);
   };
 
+  constexpr int SA = S::SLOTS_A, SB = S::SLOTS_B, AHEAD = SA > SB ? SA : SB;
 #pragma unroll
-  for (int s = 0; s < STAGES - 1; ++s) ask(s, s);
-  int slot = 0;
-  for (int kb = 0; kb < n_blocks; ++kb) {
-    copies_arrived<(STAGES - 2) * S::COPIES>();
-    ring_barrier();  // k-block kb is whole, and nobody reads the slot of k-block kb - 1 any more
-    read_quarter(0, slot, 0);
-    ask(kb + STAGES - 1, slot == 0 ? STAGES - 1 : slot - 1);
-    if (kb > 0) multiply(1);
-    read_quarter(1, slot, 1);
-    multiply(0);
-    read_quarter(0, slot, 2);
-    multiply(1);
-    read_quarter(1, slot, 3);
-    multiply(0);
-    slot = slot == STAGES - 1 ? 0 : slot + 1;
+  for (int t = 1 - AHEAD; t < 0; ++t) {  // as rounds before the first would have it
+    const Round q = round_of(t + SA - 1, t + SA - 1, t + SB - 1, t + SB - 1);
+#pragma unroll
+    for (int i = t + SA - 1 >= 0 ? 0 : PA; i < (t + SB - 1 >= 0 ? S::COPIES : PA); ++i) ask(q, i);
   }
-  multiply(1);
+  // A round asks for rows SA - 1 and weights SB - 1 k-blocks ahead, the rows first.  When k-block kb begins, its rows came
+  // with round kb - SA + 1 and its weights with round kb - SB + 1: so many copies were asked for behind both.
+  constexpr int BEHIND_A = PB + (SA - 2) * S::COPIES, BEHIND_B = (SB - 2) * S::COPIES;
+  const Round none = round_of(0, 0, 0, 0);
+  for (int kb = 0; kb < n_blocks; ++kb) {
+    copies_arrived<(BEHIND_A < BEHIND_B ? BEHIND_A : BEHIND_B)>();
+    ring_barrier();  // k-block kb is whole, and nobody reads the slots of k-block kb - 1 any more
+    read_quarter(0, 0);
+    const int next_a = slot_a == 0 ? SA - 1 : slot_a - 1, next_b = S::ALIKE ? next_a : slot_b == 0 ? SB - 1 : slot_b - 1;
+    const Round q = round_of(kb + SA - 1, next_a, kb + SB - 1, next_b);
+    if (!S::SPREAD || kb == 0) {
+#pragma unroll
+      for (int i = 0; i < TAKES; ++i) ask(q, i);
+      if (kb > 0) multiply(1, none, 0, 0);
+    } else {
+      multiply(1, q, 0, TAKES);
+    }
+    read_quarter(1, 1);
+    multiply(0, q, TAKES, S::COPIES);
+    read_quarter(0, 2);
+    multiply(1, none, 0, 0);
+    read_quarter(1, 3);
+    multiply(0, none, 0, 0);
+    slot_a = slot_a == SA - 1 ? 0 : slot_a + 1;
+    if constexpr (!S::ALIKE) slot_b = slot_b == SB - 1 ? 0 : slot_b + 1;
+  }
+  multiply(1, none, 0, 0);
   copies_arrived<0>();  // (what was asked for beyond the end: the epilogue writes where it goes)
 
   if constexpr (SPLIT) {  // the partial sums as they are; sum_partials adds them and runs the epilogue
@@ -576,15 +626,16 @@ static void launch_tiles(const GemmArgs& p, hipStream_t stream) {
 // a k-block where two blocks share the CU (shapes that fit twice), `launch` once.  Fitted to the times of 16 numbers of
 // rows from 20 to 8,000 against 18 matrices of widths from 768 to 2,048, K up to 6,400, each with K in 1 to 8 parts; the
 // shape and parts chosen from these prices are within 2 % of the best on average (at worst 1.35 times: 20 to 64 rows to
-// 10,880 features, a gated feed-forward 2,048 wide, which the kernel for few rows cannot hold).
+// 10,880 features, a gated feed-forward 2,048 wide, which the kernel for few rows cannot hold).  With K whole, 333 to 8,000 rows
+// against sixteen matrices, they choose the fastest shape everywhere.
 struct TilePrice {
   int variant, bm, bn, per_cu;
   double launch, tile, kblock, pair;
   bool splits;  // K may be split over blocks
 };
 static const TilePrice TILE_PRICES[] = {
-    {3, Tile256::BM, Tile256::BN, 1, 0.0, 7.78, 1.39, 0.0, false},
-    {4, Tile256x192::BM, Tile256x192::BN, 1, 0.0, 7.26, 1.17, 0.0, false},
+    {3, Tile256::BM, Tile256::BN, 1, 0.0, 7.78, 1.3, 0.0, false},
+    {4, Tile256x192::BM, Tile256x192::BN, 1, 0.0, 7.26, 1.0, 0.0, false},
     {8, Tile256x128::BM, Tile256x128::BN, 1, 0.0, 7.6, 0.7, 0.0, false},
     {1, Tile128::BM, Tile128::BN, 1, 0.0, 4.33, 0.49, 0.0, true},
     {5, Tile64x128::BM, Tile64x128::BN, 2, 0.52, 2.81, 0.38, 0.77, true},
