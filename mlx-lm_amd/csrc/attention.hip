@@ -221,10 +221,10 @@ __global__ __launch_bounds__(256) void kv_write_vec_kernel(const T* __restrict__
     const int col = c * VN;
     const int h = col / head_dim, d = col - h * head_dim;
     const size_t dst = (size_t)page * page_stride + ((size_t)h * page_size + row) * head_dim + d;
-    const uint4 kk = *(const uint4*)(k_src + (size_t)t * ld_src + col);
-    const uint4 vv = *(const uint4*)(v_src + (size_t)t * ld_src + col);
-    *(uint4*)(k_pages + dst) = kk;
-    *(uint4*)(v_pages + dst) = vv;
+    const u32x4_t kk = *(const u32x4_t*)(k_src + (size_t)t * ld_src + col);
+    const u32x4_t vv = *(const u32x4_t*)(v_src + (size_t)t * ld_src + col);
+    store_through(k_pages + dst, kk);  // (megabytes for a prompt: not left to the kernel's end)
+    store_through(v_pages + dst, vv);
   }
 }
 
@@ -629,7 +629,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NV == 1 ? 4
       f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int w = 0; w < 4; ++w) acc += *(const f32x4_t*)&part_o[w][y][d] * weight[w];
-      *(f32x4_t*)((float*)p.out + (size_t)(row0 + y) * p.ldo + h * HD + d) = acc * inv;
+      store_through((float*)p.out + (size_t)(row0 + y) * p.ldo + h * HD + d, __builtin_bit_cast(u32x4_t, acc * inv));
     }
   }
 }

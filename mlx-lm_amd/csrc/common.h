@@ -185,6 +185,15 @@ __device__ __forceinline__ void store_through(__amdgpu_buffer_rsrc_t r, uint32_t
 __device__ __forceinline__ void store_through(__amdgpu_buffer_rsrc_t r, uint32_t byte_offset, float v) {
   __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned int, v), r, (int)byte_offset, 0, POLICY_THROUGH);
 }
+__device__ __forceinline__ void store_through(__amdgpu_buffer_rsrc_t r, uint32_t byte_offset, const float4& v) {
+  store_through(r, byte_offset, u32x4_t{__float_as_uint(v.x), __float_as_uint(v.y), __float_as_uint(v.z), __float_as_uint(v.w)});
+}
+// The same at any address, for where no one buffer of 4 GB holds the places (cache pages).  In assembly, as the compiler
+// takes a policy for 16 bytes on buffer stores only; nothing waits for it but the kernel's end.  (The wait states: what
+// is stored lies in registers that the next instruction may write.)  The address is a multiple of 16.
+__device__ __forceinline__ void store_through(void* at, u32x4_t v) {
+  asm volatile("global_store_dwordx4 %0, %1, off sc0 sc1\n\ts_nop 1" ::"v"(at), "v"(v) : "memory");
+}
 static inline bool fits_through_buffer(size_t bytes) { return bytes < ((size_t)1 << 32); }
 
 // ---------------------------------------------------------------------------
