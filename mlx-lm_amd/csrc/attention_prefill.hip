@@ -36,6 +36,7 @@
 
 struct PrefillArgs {
   uint16_t* out;
+  int out_by_16;  // a head's row of out is whole pieces of 16 bytes
   const uint16_t* q;
   const uint16_t* k_pages;
   const uint16_t* v_pages;
@@ -539,7 +540,7 @@ void attn_prefill_kernel(PrefillArgs p) {
 //  * The next tile's scores are begun while this one's probabilities are made, in the registers that are free by then, so
 //    that a wave needs 153 registers and three blocks share a CU.  (With the scores in two sets of registers, a whole tile ahead, 232:
 //    two blocks, 272 us for 8,000 tokens instead of 251.)
-// 25 heads of 64, us, the kernel above and this one: 8,000 tokens 315 and 251 (0.82 PFLOP/s of the causal half), under a window of
+// 25 heads of 64, us, the kernel above and this one (while its outputs left as the other's do; now: at its end): 8,000 tokens 315 and 251 (0.82 PFLOP/s of the causal half), under a window of
 // 1,000 112 and 84; 2 x 1,024 24.5 and 21.2; 1,024 19.6 and 17.2; 512 on 4,000 earlier keys 58.5 and 49; 512 12.3 and 11.4; 333 10.1
 // and 9.4; 128 7.6 and 7.0; 17 4.7 and 4.8.  What bounds it: vector instructions, 74 % of the CUs' cycles beside 41 % for the
 // products (8,000 tokens at 1.88 GHz); at few blocks the way to the first tile and the walk's steps of some 1 us.
@@ -896,21 +897,41 @@ void attn_prefill_ring_kernel(PrefillArgs p) {
       for (int r = 0; r < 16; ++r) ot[dt][r] = ot[dt][r] * w0 + sums[(dt * 16 + r) * 256] * w1;
     m = both;
   }
-  if (q_live) {
-    // (m is in units of log 2)
-    if (p.sinks) l += exp2f(fmaf(p.sinks[h], 1.4426950408889634f, -m));
-    const float inv = head_gate_of(p, row0 + qi, h) / l;
-    uint16_t* orow = p.out + (size_t)(row0 + qi) * p.ldo + h * HD;
+  // (m is in units of log 2)
+  if (p.sinks) l += exp2f(fmaf(p.sinks[h], 1.4426950408889634f, -m));
+  const float inv = head_gate_of(p, row0 + min(qi, nq - 1), h) / l;
+  // The outputs leave through LDS, as whole rows of 128 bytes that go through to memory: stored as they lie here, pieces of
+  // 8 bytes of 32 rows, they had to stay in the L2s and were written back at the kernel's end (2 x 1,024 tokens of 25 heads
+  // 22.2 -> 21.1 us, 512 11.5 -> 10.6, 8,000 271 -> 264, under a window of 1,000 97 -> 86.5; 17 4.8 -> 5.0).
+  constexpr int OUT_ROW = ROW + 16;  // bytes from row to row in LDS: sixteen rows' pieces on different banks
+  static_assert(4 * 32 * OUT_ROW <= GROUP_LDS, "the outputs fit where the tiles were");
+  if (GROUPS == 1) __syncthreads();  // no tile is read any more (of two groups: where the second one's tiles were, which end above)
+  char* const rows_at = ring + (GROUPS - 1) * GROUP_LDS + wave * 32 * OUT_ROW;
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
+  for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        // accumulators 4j .. 4j+3: head columns dt*32 + 8j + 4g + (0..3)
-        uint2 o;
-        o.x = pack_bf16x2(ot[dt][4 * j] * inv, ot[dt][4 * j + 1] * inv);
-        o.y = pack_bf16x2(ot[dt][4 * j + 2] * inv, ot[dt][4 * j + 3] * inv);
-        *(uint2*)(orow + dt * 32 + 8 * j + 4 * g) = o;
-      }
+    for (int j = 0; j < 4; ++j) {
+      // accumulators 4j .. 4j+3: head columns dt*32 + 8j + 4g + (0..3)
+      uint2 o;
+      o.x = pack_bf16x2(ot[dt][4 * j] * inv, ot[dt][4 * j + 1] * inv);
+      o.y = pack_bf16x2(ot[dt][4 * j + 2] * inv, ot[dt][4 * j + 3] * inv);
+      *(uint2*)(rows_at + ql * OUT_ROW + (dt * 32 + 8 * j + 4 * g) * 2) = o;
+    }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();  // (a wave's rows are its own, and its LDS accesses keep their order)
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+  for (int s = 0; s < 4; ++s) {
+    const int row = s * 8 + row8, q = wave * 32 + row;
+    if (q >= nq) continue;
+    const u32x4_t o = *(const u32x4_t*)(rows_at + row * OUT_ROW + (lane & 7) * 16);
+    uint16_t* const to = p.out + (size_t)(row0 + q) * p.ldo + h * HD + (lane & 7) * 8;
+    if (p.out_by_16) {
+      store_through(to, o);
+    } else {
+      *(uint2*)to = make_uint2(o.x, o.y);
+      *(uint2*)(to + 4) = make_uint2(o.z, o.w);
+    }
   }
 }
 
@@ -947,6 +968,7 @@ static int prefill_launch(void* out, const void* q, int ldq, int ldo, const void
   if (page_stride >= ((size_t)1 << 32)) FAIL("attn_prefill: a page of %zu elements is too large", page_stride);
   PrefillArgs p;
   p.out = (uint16_t*)out, p.q = (const uint16_t*)q;
+  p.out_by_16 = ldo % 8 == 0 && !((uintptr_t)out & 15);
   p.k_pages = (const uint16_t*)k_pages, p.v_pages = (const uint16_t*)v_pages;
   p.block_table = block_table, p.token_req = token_req, p.positions = positions, p.tiles = tiles;
   p.page_stride = page_stride, p.ldq = ldq, p.ldo = ldo, p.max_blocks = max_blocks;

@@ -824,6 +824,27 @@ def test_attn_prefill_heads_of_64_over_tiles_and_pages(ps, H, Hkv, window):
         assert err < 2.5e-2, err
 
 
+@pytest.mark.parametrize("ql", [[17, 128, 1], [700, 65]])
+def test_attn_prefill_heads_of_64_into_rows_of_any_place(ql):
+    """Rows of heads of 64 leave in pieces of 16 bytes where they lie on such, in halves of them where the stride or the
+    first row does not: the same bits, and nothing beside them, with one group of waves a block and with two."""
+    k = _k()
+    H = 40 if len(ql) == 3 else 90  # (120 blocks; 630: more than there are compute units)
+    c = PagedCase(torch.bfloat16, H, H // 10, 64, 16, [0] * len(ql), ql, seed=3)
+    k.kv_write(c.k_new.to(DEV), c.v_new.to(DEV), c.kv, c.block_table_dev, c.token_req, c.positions)
+    tiles, outs = c.tiles(k.attn_tile_sizes()[1]), []
+    for before, behind in ((0, 0), (8, 8), (0, 4), (4, 4)):
+        wide = torch.full((c.T, before + H * 64 + behind), float("nan")).to(torch.bfloat16).to(DEV)
+        out = wide[:, before : before + H * 64]
+        k.attn_prefill(out, c.q.to(DEV), c.kv, c.block_table_dev, c.token_req, c.positions, tiles, tiles.shape[0], H, c.scale, 0)
+        outs.append(out)
+        assert torch.isnan(wide[:, :before].float()).all() and torch.isnan(wide[:, before + H * 64 :].float()).all()
+    # (the weights are rounded to bfloat16, 2^-9 of each, and meet values of up to 4.5)
+    assert (outs[0].double().cpu() - c.reference()).abs().max().item() < 2.5e-2
+    for out in outs[1:]:
+        assert torch.equal(out, outs[0])
+
+
 def test_attn_prefill_far_key_stands_out():
     """Every query of a long portion points at one far key of its own."""
     k = _k()
