@@ -31,6 +31,7 @@
 // the registers).
 #include "common.h"
 #include "attention_tiles.h"
+#include "attention_decode_row.h"
 #include "lds_copy.h"
 #include <type_traits>
 
@@ -568,20 +569,20 @@ __device__ __forceinline__ float max_of_halves(float v) {
   return larger;
 }
 
+// Head h of tile `tile`'s queries.  ring: LDS for the tiles, ring_bytes(GROUPS) of it; page_at: [max_blocks], byte offsets of this
+// head's part of the request's pages, from the first tile's on.
+constexpr int ring_bytes(int groups) { return groups * 2 * 3 * KT * 128; }
 template <int HD, int GROUPS>
-__global__ __launch_bounds__(256 * GROUPS) __attribute__((amdgpu_waves_per_eu(GROUPS == 1 ? 3 : 2, GROUPS == 1 ? 3 : 2)))
-void attn_prefill_ring_kernel(PrefillArgs p) {
+__device__ __forceinline__ void attend_tile(const PrefillArgs& p, int h, int tile, char* ring, size_t* page_at) {
   constexpr int DC = HD / 16, DT = HD / 32;
   constexpr int ROW = HD * 2, WAVE_KEYS = KT / 4, COPIES = WAVE_KEYS * ROW / 1024;  // bytes a key; keys and copies a wave and tile
   constexpr int SLOTS = 3, TILE = KT * ROW, GROUP_LDS = 2 * SLOTS * TILE;
   static_assert(HD == 64, "the permutations of a row's pieces are those of rows of 128 bytes");
-  __shared__ __attribute__((aligned(1024))) char ring[GROUPS * GROUP_LDS];
-  extern __shared__ size_t page_at[];  // [max_blocks]: byte offsets of this head's part of the request's pages, from the first tile's on
+  static_assert(GROUPS * GROUP_LDS == ring_bytes(GROUPS), "the kernels' LDS");
 
   const int group = GROUPS > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0;
   const int tid = threadIdx.x & 255, lane = tid & 63;  // (within the group)
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int h = blockIdx.x, tile = blockIdx.y;
   const int row0 = p.tiles[2 * tile];
   const int nq = p.tiles[2 * tile + 1];
   const int kv_head = h / (p.n_heads / p.n_kv_heads);
@@ -876,7 +877,7 @@ void attn_prefill_ring_kernel(PrefillArgs p) {
   l += __shfl_xor(l, 32, WAVE);
   if (GROUPS == 2 && groups == 2) {
     // the second group's sums go to the first through LDS, each thread's to the thread of the same queries
-    static_assert(GROUPS == 1 || (DT * 16 + 2) * 256 * sizeof(float) <= sizeof(ring), "the sums fit where the tiles were");
+    static_assert(GROUPS == 1 || (DT * 16 + 2) * 256 * sizeof(float) <= GROUPS * GROUP_LDS, "the sums fit where the tiles were");
     float* const sums = (float*)ring + tid;
     __syncthreads();  // no tile is read any more
     if (group == 1) {
@@ -935,18 +936,52 @@ void attn_prefill_ring_kernel(PrefillArgs p) {
   }
 }
 
+template <int HD, int GROUPS>
+__global__ __launch_bounds__(256 * GROUPS) __attribute__((amdgpu_waves_per_eu(GROUPS == 1 ? 3 : 2, GROUPS == 1 ? 3 : 2)))
+void attn_prefill_ring_kernel(PrefillArgs p) {
+  __shared__ __attribute__((aligned(1024))) char ring[ring_bytes(GROUPS)];
+  extern __shared__ size_t page_at[];
+  attend_tile<HD, GROUPS>(p, blockIdx.x, blockIdx.y, ring, page_at);
+}
+
+// A prompt's portion and the rows that decode beside it in one launch: first the tiles' blocks, a few long ones bound by their
+// instructions, then the rows', many that wait for memory, both in blocks of four waves, three a CU.  One after the other, as
+// two launches, the second waited for the last block of the first.  25 heads, us, two launches and one: 24 rows at 200 to
+// 900 keys beside 512 tokens 32.1 and 22.5 (the rows alone 20.7), beside 16 24.6 and 20.4, beside 1,000 38.1 and 26.4; 48 rows at 16 to 900
+// beside 512 41.7 and 31.8; 11 rows at 30 to 60 beside 1,000 22.8 and 19.6.  What bounds it: the rows' keys, then the tiles' walks.
+template <int HD>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) void attn_mixed_kernel(PrefillArgs p, DecodeArgs rows, int n_tiles) {
+  __shared__ __attribute__((aligned(1024))) char ring[ring_bytes(1)];
+  extern __shared__ size_t page_at[];
+  const int lin = blockIdx.x, item = lin / p.n_heads, h = lin - item * p.n_heads;  // (a row's heads are neighbours, as in the decode kernel)
+  if (item < n_tiles) {
+    attend_tile<HD, 1>(p, h, item, ring, page_at);
+  } else {
+    attend_row<uint16_t, HD / 8, true, false, 4>(rows, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), 4, item - n_tiles, h, 0);
+  }
+}
+
 DEFINE_LAST_ERROR(mlxlm_last_error)
 
 // tiles: n_tiles pairs (first flat row, number of rows 1..128); the rows of a
 // tile are consecutive tokens of one request at consecutive positions.
 // bfloat16 only, head_dim 32, 64, 128 or 256.
+// The longest walk that attn_mixed takes a portion's tiles on: they go by one group of waves a block here, and where few rows
+// stand beside a long walk that costs what the launch saves (512 tokens on 1,500 earlier keys beside 11 rows at 30 to 60: 32.5
+// as two launches, 32.7 as one; beside 24 rows at 200 to 2,000 64.8 and 44.8; 1,024 on 1,024 beside 24 at 30 to 60 33.8 and 32.4).
+#define MIXED_MOST_KEYS 2048
+// And the longest row where the decode kernel would give rows eight waves or parts, which are sooner done alone: one row of 700
+// keys beside 16 / 512 / 1,000 tokens 13.1, 19.9, 26.1 (eight waves) and 11.0, 12.2, 19.1 in one launch; four at 200 to 900 14.6,
+// 21.5, 27.7 and 13.5, 14.3, 19.2; eight at 200 to 1,000 16.3, 22.9, 29.3 and 15.7, 16.2, 19.6: level beside the fewest tokens.
+#define MIXED_MOST_ROW_KEYS 1024
+
 static int prefill_launch(void* out, const void* q, int ldq, int ldo, const void* k_pages,
                           const void* v_pages, size_t page_stride, const int* block_table,
                           int max_blocks, const int* token_req, const int* positions,
                           const int* tiles, int n_tiles, int n_heads, int n_kv_heads,
                           int head_dim, int page_size, int window, float scale,
                           const float* head_scale, const float* slopes, const void* gate, int ldg,
-                          int keep_first, const AttnTerms* shape, hipStream_t stream) {
+                          int keep_first, const AttnTerms* shape, hipStream_t stream, const int* rows = nullptr, int n_rows = 0) {
   if (n_tiles <= 0) return 0;
   if (shape && (shape->softcap < 0.f || (shape->dist_bias && shape->n_dist <= 0)))
     FAIL("attn_prefill: softcap %g, a distance table of %d entries a head", (double)shape->softcap, shape->n_dist);
@@ -1020,7 +1055,16 @@ static int prefill_launch(void* out, const void* q, int ldq, int ldo, const void
       LAUNCH_AS(HD, true, 1);           \
     }                                   \
   } while (0)
-  if (ring) {
+  if (rows) {  // (attn_mixed has looked at what the rows need beyond this)
+    if (!ring) FAIL("attn_mixed: pages of %d keys", page_size);
+    DecodeArgs d = {};
+    d.out = out, d.q = q, d.k_pages = k_pages, d.v_pages = v_pages;
+    d.block_table = block_table, d.token_req = token_req, d.positions = positions, d.rows = rows;
+    d.page_stride = page_stride, d.ldq = ldq, d.ldo = ldo, d.max_blocks = max_blocks;
+    d.n_heads = n_heads, d.n_kv_heads = n_kv_heads, d.page_size = page_size, d.window = window, d.n_splits = 1;
+    d.scale = scale, d.out_head_dim = head_dim, d.table_in_lds = 1, d.page_shift = p.page_shift;
+    hipLaunchKernelGGL((attn_mixed_kernel<64>), dim3((unsigned)(n_heads * (n_tiles + n_rows))), dim3(256), (size_t)max_blocks * sizeof(size_t), stream, p, d, n_tiles);
+  } else if (ring) {
     const size_t table = (size_t)max_blocks * sizeof(size_t);
     if (two)
       hipLaunchKernelGGL((attn_prefill_ring_kernel<64, 2>), grid, block, table, stream, p);
@@ -1039,6 +1083,28 @@ static int prefill_launch(void* out, const void* q, int ldq, int ldo, const void
 #undef LAUNCH_AS
   CHECK_LAUNCH("attn_prefill");
   return 0;
+}
+
+// 1 if attn_mixed takes a step's tiles and rows, of which the longest reads `row_keys`: bfloat16 heads of 64 with a key head
+// each; rows that the decode kernel would give four waves a block too (more (row, head)s than CUs), or short ones.
+extern "C" int attn_mixed_takes(int n_tiles, int n_rows, int n_heads, int n_kv_heads, int head_dim, int page_size, int max_blocks,
+                                long row_keys) {
+  return n_tiles > 0 && n_rows > 0 && n_tiles + n_rows <= 65535 && head_dim == 64 && n_heads == n_kv_heads && page_size >= 16 &&
+         (page_size & (page_size - 1)) == 0 && (long)max_blocks * page_size <= MIXED_MOST_KEYS &&
+         ((long)n_rows * n_heads > n_compute_units() || row_keys <= MIXED_MOST_ROW_KEYS);
+}
+
+// attn_prefill's tiles and attn_decode_rows' rows, of one step, in one launch.
+extern "C" int attn_mixed(void* out, const void* q, int ldq, int ldo, const void* k_pages, const void* v_pages, size_t page_stride,
+                          const int* block_table, int max_blocks, const int* token_req, const int* positions, const int* tiles, int n_tiles,
+                          const int* rows, int n_rows, int n_heads, int n_kv_heads, int head_dim, int page_size, int window, float scale,
+                          hipStream_t stream) {
+  if (!attn_mixed_takes(n_tiles, n_rows, n_heads, n_kv_heads, head_dim, page_size, max_blocks, 0))
+    FAIL("attn_mixed: %d tiles and %d rows of %d heads of %d over %d, %d pages of %d keys", n_tiles, n_rows, n_heads, head_dim, n_kv_heads,
+         max_blocks, page_size);
+  if (!rows || max_blocks <= 0 || ldo < n_heads * head_dim) FAIL("attn_mixed: null pointer or stride");
+  return prefill_launch(out, q, ldq, ldo, k_pages, v_pages, page_stride, block_table, max_blocks, token_req, positions, tiles, n_tiles, n_heads,
+                        n_kv_heads, head_dim, page_size, window, scale, nullptr, nullptr, nullptr, 0, 0, nullptr, stream, rows, n_rows);
 }
 
 // attn_prefill_biased: with the optional terms of PrefillArgs (null or 0 where one is absent).

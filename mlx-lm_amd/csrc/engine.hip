@@ -122,6 +122,9 @@ typedef int (*fn_attn_prefill)(void*, const void*, int, int, const void*, const 
                                hipStream_t);
 
 // (the same with the optional score terms: an AttnTerms ahead of the stream)
+typedef int (*fn_attn_mixed)(void*, const void*, int, int, const void*, const void*, size_t, const int*, int, const int*, const int*, const int*,
+                             int, const int*, int, int, int, int, int, int, float, hipStream_t);
+typedef int (*fn_attn_mixed_takes)(int, int, int, int, int, int, int, long);
 typedef int (*fn_attn_tile_terms)(void*, const void*, int, int, const void*, const void*, size_t, const int*, int,
                                   const int*, const int*, const int*, int, int, int, int, int, int, float, int,
                                   const AttnTerms*, hipStream_t);
@@ -160,6 +163,8 @@ static Entry<fn_attn_row> k_attn_row("attention", "attn_row");
 static Entry<fn_attn_decode> k_attn_decode("attention_decode", "attn_decode_rows");
 static Entry<fn_attn_decode_group> k_attn_decode_group("attention_decode", "attn_decode_group");
 static Entry<fn_attn_prefill> k_attn_prefill("attention_prefill", "attn_prefill");
+static Entry<fn_attn_mixed> k_attn_mixed("attention_prefill", "attn_mixed");
+static Entry<fn_attn_mixed_takes> k_attn_mixed_takes("attention_prefill", "attn_mixed_takes");
 static Entry<fn_attn_tile_terms> k_attn_tile_terms("attention", "attn_tile_terms");
 static Entry<fn_attn_row_terms> k_attn_row_terms("attention", "attn_row_terms");
 static Entry<fn_attn_decode_terms> k_attn_decode_terms("attention_decode", "attn_decode_rows_terms");
@@ -834,6 +839,17 @@ struct Attention : Mixer {
       return 0;
     }
     const bool mfma_sizes = bf16 && (head_dim == 32 || head_dim == 64 || head_dim == 128 || head_dim == 256);
+    if (n_big_tiles && n_rows && bf16 && !terms && !out_packed) {  // a portion beside rows that decode: both in one launch
+      int takes = 0;
+      QUERY(k_attn_mixed_takes, takes, n_big_tiles, n_rows, n_heads, n_kv_heads, head_dim, kv.page_size, kv.max_blocks,
+            window > 0 && window < max_row_context ? (long)window : max_row_context);
+      if (takes) {
+        if (ctx->stats && ctx->stats->key_splits_most < 1) ctx->stats->key_splits_most = 1;
+        KERNEL(k_attn_mixed, ctx, out.p, q.p, q.ld, out.ld, kv.k, kv.v, kv.page_stride, kv.block_table, kv.max_blocks, kv.token_req,
+               kv.positions, big_tiles, n_big_tiles, rows, n_rows, n_heads, n_kv_heads, head_dim, kv.page_size, window, scale, ctx->stream);
+        return 0;
+      }
+    }
     if (n_tiles && terms) {
       if (mfma_sizes)
         KERNEL(k_attn_prefill_terms, ctx, out.p, q.p, q.ld, out.ld, kv.k, kv.v, kv.page_stride, kv.block_table,

@@ -818,6 +818,26 @@ def attn_prefill(out, q, kv, block_table, token_req, positions, tiles, n_tiles, 
     return out
 
 
+def attn_mixed(out, q, kv, block_table, token_req, positions, tiles, n_tiles, rows, n_rows, n_heads, scale, window=0):
+    """``attn_prefill``'s tiles and, of the same step, rows that decode (as ``attn_decode`` by four waves a block, in one part), in
+    one launch: bfloat16 heads of 64 with a key head each, pages of a power of two of 16 keys or more, tables of up to 2,048 keys."""
+    lib = build.load("attention_prefill")
+    ldq, ldo = _rows2d(q, "q"), _rows2d(out, "out")
+    _need(q.dtype == torch.bfloat16 and out.dtype == q.dtype, "attn_mixed: bfloat16 only")
+    _need(q.shape[1] == n_heads * kv.head_dim and out.shape[1] == q.shape[1], "attn_mixed: rows of n_heads*head_dim")
+    _attn_common(q, kv, block_table, token_req, positions)
+    _dev(tiles, "tiles", torch.int32)
+    _dev(rows, "rows", torch.int32)
+    _need(tiles.numel() >= 2 * n_tiles and rows.numel() >= n_rows, "attn_mixed: lists too short")
+    rc = lib.attn_mixed(
+        _ptr(out), _ptr(q), _c_int(ldq), _c_int(ldo), _ptr(kv.k), _ptr(kv.v), _c_size_t(kv.page_stride), _ptr(block_table),
+        _c_int(block_table.shape[1]), _ptr(token_req), _ptr(positions), _ptr(tiles), _c_int(n_tiles), _ptr(rows), _c_int(n_rows),
+        _c_int(n_heads), _c_int(kv.n_kv_heads), _c_int(kv.head_dim), _c_int(kv.page_size), _c_int(window), _c_float(scale), _stream(),
+    )
+    build.check(lib, rc, "attn_mixed")
+    return out
+
+
 def attn_decode_takes(q_dtype, kv):
     """Whether the register-streaming decode kernel takes this cache geometry."""
     if q_dtype not in (torch.bfloat16, torch.float32):

@@ -197,6 +197,34 @@ def test_mixed_batches_with_few_pages(folders, dtype, name, sharp):
         _close(torch.cat(got[rid]), want, dtype, f"mixed, request {rid}")
 
 
+@pytest.mark.parametrize("record", [False, True])
+def test_portions_beside_decoding_rows_of_heads_of_64(tmp_path, monkeypatch, record):
+    """Heads of 64 in bfloat16, where a portion and the rows beside it share a launch of attention: logits of both against
+    the plain implementation, steps of one shape run again (recorded where that is asked for)."""
+    from mlx_lm_amd.engine import Engine, StepEntry
+    from mlx_lm_amd.utils import load_model
+
+    config = dict(helpers.TINY_C, n_embd=128, n_head=2, n_inner=256)
+    monkeypatch.setitem(helpers.TINY, "HEADS64", (config, 11, "b"))
+    _, weights = helpers.make_folder(str(tmp_path), "HEADS64", 8.0)
+    model, _ = load_model(str(tmp_path), dtype="bfloat16")
+    eng = Engine(model, dtype="bfloat16", page_size=16, max_tokens=6000, max_requests=16, record_prompt_steps=record)
+    rows = {f"r{i}": helpers.random_tokens(n, config["vocab_size"], i) for i, n in enumerate((20, 64, 65, 129, 200, 301, 440))}
+    for rid, toks in rows.items():
+        eng.add_request(rid)
+        eng.step([StepEntry(rid, toks[:-4], [0])])
+    want = {rid: _plain_logits(weights, config, toks, "bfloat16") for rid, toks in rows.items()}
+    for step in range(4):
+        portion = helpers.random_tokens(130, config["vocab_size"], 50 + step)
+        eng.add_request("portion")
+        entries = [StepEntry(rid, [toks[len(toks) - 4 + step]], [0]) for rid, toks in rows.items()]
+        logits = eng.step(entries + [StepEntry("portion", portion, [0, 64, 129])])
+        for i, rid in enumerate(rows):
+            _close(logits[i], want[rid][len(rows[rid]) - 4 + step], "bfloat16", f"{rid}, step {step}")
+        _close(logits[len(rows) :], _plain_logits(weights, config, portion, "bfloat16")[[0, 64, 129]], "bfloat16", f"portion {step}")
+        eng.end_request("portion")
+
+
 @pytest.mark.parametrize("dtype", ["bfloat16", "float32"])
 @pytest.mark.parametrize("name,sharp", [("B", 8.0), ("C", 0.0)])
 @pytest.mark.parametrize("use_graphs", [False, True])

@@ -1,5 +1,6 @@
 """Each HIP kernel alone against a plain torch reference, at sizes of its own."""
 
+import ctypes
 import math
 
 import pytest
@@ -843,6 +844,49 @@ def test_attn_prefill_heads_of_64_into_rows_of_any_place(ql):
     assert (outs[0].double().cpu() - c.reference()).abs().max().item() < 2.5e-2
     for out in outs[1:]:
         assert torch.equal(out, outs[0])
+
+
+@pytest.mark.parametrize("ps", [16, 64])
+@pytest.mark.parametrize("window", [0, 33, 200])
+@pytest.mark.parametrize("rows,portions", [
+    ([1] * 11, [(0, 1)]), ([1, 2, 15, 16, 17, 63, 64, 65, 300, 511, 700], [(0, 128), (130, 129), (5, 17)]),
+    ([200 + 29 * i for i in range(24)], [(0, 512)]), ([40] * 64, [(700, 300), (0, 65)])])
+def test_attn_mixed(rows, portions, window, ps):
+    """Portions' tiles and rows that decode in one launch: the rows bit for bit as the decode kernel alone makes them with four
+    waves, both against 64 bits; queries that are in no list stay untouched."""
+    k = _k()
+    H = 25
+    ctx = [n - 1 for n in rows] + [c for c, _ in portions] + [3]
+    ql = [1] * len(rows) + [n for _, n in portions] + [1]  # (the last request's row is left out)
+    c = PagedCase(torch.bfloat16, H, H, 64, ps, ctx, ql, seed=len(rows) + window, window=window)
+    k.kv_write(c.k_new.to(DEV), c.v_new.to(DEV), c.kv, c.block_table_dev, c.token_req, c.positions)
+    tiles, first = [], len(rows)
+    for _, n in portions:
+        tiles += [(first + t, min(128, n - t)) for t in range(0, n, 128)]
+        first += n
+    tiles = torch.tensor(tiles, dtype=torch.int32, device=DEV)
+    list_ = torch.arange(len(rows) - 1, -1, -1, dtype=torch.int32, device=DEV)
+    out, alone = (torch.full((c.T, H * 64), float("nan")).to(torch.bfloat16).to(DEV) for _ in range(2))
+    k.attn_mixed(out, c.q.to(DEV), c.kv, c.block_table_dev, c.token_req, c.positions, tiles, tiles.shape[0], list_, len(rows), H, c.scale, window)
+    k.attn_decode(alone, c.q.to(DEV), c.kv, c.block_table_dev, c.token_req, c.positions, list_, len(rows), H, c.scale, window, n_waves=4)
+    assert torch.equal(out[: len(rows)], alone[: len(rows)])
+    assert torch.isnan(out[-1].float()).all()
+    # (the weights are rounded to bfloat16, 2^-9 of each, and meet values of up to 4.5)
+    assert (out[:-1].double().cpu() - c.reference()[:-1]).abs().max().item() < 2.5e-2
+
+
+def test_attn_mixed_refuses_what_it_does_not_take():
+    from mlx_lm_amd.ops import build
+
+    lib = build.load("attention_prefill")
+    def takes(**other):
+        a = dict(dict(n_tiles=4, n_rows=8, n_heads=25, n_kv_heads=25, head_dim=64, page_size=16, max_blocks=64, keys=1024), **other)
+        return lib.attn_mixed_takes(*(ctypes.c_int(v) for v in list(a.values())[:-1]), ctypes.c_long(a["keys"]))
+
+    assert takes() == takes(n_rows=11, keys=2048) == takes(max_blocks=128) == 1
+    for other in [dict(n_tiles=0), dict(n_rows=0), dict(n_kv_heads=5), dict(head_dim=128), dict(page_size=48), dict(page_size=8),
+                  dict(max_blocks=129), dict(keys=1025)]:
+        assert takes(**other) == 0, other
 
 
 def test_attn_prefill_far_key_stands_out():
