@@ -627,8 +627,9 @@ __device__ __forceinline__ void attend_tile(const PrefillArgs& p, int h, int til
 #pragma unroll
   for (int dc = 0; dc < DC; ++dc) asm volatile("" : "+v"(qf[dc].v));
 
-  // Copies: this wave brings keys 16 wave .. + 15 of each tile, which lie in one page.  Of keys in pages before the
-  // window's first and of keys beyond the last nothing is read, and zeros come.
+  // Copies: this wave brings keys 16 wave .. + 15 of each tile, which lie in one page.  Of keys beyond the last, and of the
+  // first tile's keys before the first that any query sees, nothing is read, and zeros come: such keys enter the products with a
+  // weight of zero, and what lies there (another request's keys, infinities) must not make NaN of it.
   const uint32_t ring_at = lds_address(ring) + group * GROUP_LDS;
   const uint32_t copy_at = __builtin_amdgcn_readfirstlane(ring_at + wave * COPIES * 1024);
   const int row8 = lane >> 3;
@@ -649,7 +650,7 @@ __device__ __forceinline__ void attend_tile(const PrefillArgs& p, int h, int til
     const size_t at = (((size_t)hi << 32) | lo) + (uint32_t)((key & row_mask) * ROW);
     int keys;  // (as scalar instructions: the compiler takes the vector unit's median)
     asm("s_max_i32 %0, %1, 0\n\ts_min_i32 %0, %0, %2" : "=&s"(keys) : "s"(k_hi - key), "n"(WAVE_KEYS) : "scc");
-    return Source{(uint32_t)at, (uint32_t)(at >> 32), (key >> shift) < first_page ? 0 : keys * ROW};
+    return Source{(uint32_t)at, (uint32_t)(at >> 32), keys * ROW};
   };
   // (what a copy's descriptor is made of is the same in all lanes; the compiler loses sight of that)
   auto copy = [&](const uint16_t* pages, const Source& s, uint32_t from0, uint32_t from1, uint32_t to) __attribute__((always_inline)) {
@@ -834,8 +835,15 @@ __device__ __forceinline__ void attend_tile(const PrefillArgs& p, int h, int til
   // into the slots of K(t) and V(t - 1), which every wave has read when the step's barrier is passed.
   static_assert(COPIES == 2, "a pair of copies a tile");
   Source ahead;  // of tile t + 2
+  // (only the first tile holds keys before k_lo: rows `unseen` and less of this wave's sixteen)
+  const int unseen = k_lo - first_key(0) - wave * WAVE_KEYS;
+  constexpr uint32_t NOTHING = COPY_NOTHING - 1024;  // (the second copy adds its kilobyte)
+  auto seen = [&](uint32_t from, int row) __attribute__((always_inline)) { return row < unseen ? NOTHING : from; };
+  ahead = source(0, page_entry(0));
+  copy(p.k_pages, ahead, seen(k_from0, row8), seen(k_from1, 8 + row8), copy_at);
+  copy(p.v_pages, ahead, seen(v_from, row8), seen(v_from, 8 + row8), copy_at + SLOTS * TILE);
 #pragma unroll
-  for (int t = 0; t < 3; ++t) {
+  for (int t = 1; t < 3; ++t) {
     ahead = source(t, page_entry(t));
     copy_k(ahead, t);
     if (t < 2) copy_v(ahead, t);

@@ -889,6 +889,32 @@ def test_attn_mixed_refuses_what_it_does_not_take():
         assert takes(**other) == 0, other
 
 
+@pytest.mark.parametrize("hd,ps", [(32, 16), (64, 8), (64, 16), (64, 64), (64, 256), (128, 16)])
+@pytest.mark.parametrize("H,mixed", [(2, False), (90, False), (2, True)])
+@pytest.mark.parametrize("window", [1, 17, 40, 100])
+def test_attn_prefill_keys_behind_every_window_do_not_count(hd, ps, H, mixed, window):
+    """Keys that have left the windows of all queries of a tile, in the pages and tiles of keys that the first key seen
+    shares with them, are infinite and NaN, keys and values: nothing of them reaches an output."""
+    if mixed and (hd != 64 or ps < 16):
+        pytest.skip("a launch of both is for heads of 64 in pages of sixteen keys or more")
+    k = _k()
+    starts, ql = [window + 1, 63 + window, 150, 300, 333], [1, 1, 90, 128, 17]  # (a tile of queries a request)
+    rows = 3 if mixed else 0
+    c = PagedCase(torch.bfloat16, H, H, hd, ps, [20, 64, 130][:rows] + starts, [1] * rows + ql, seed=hd + ps + window, window=window)
+    k.kv_write(c.k_new.to(DEV), c.v_new.to(DEV), c.kv, c.block_table_dev, c.token_req, c.positions)
+    for r, start in enumerate(starts, rows):
+        for p in range(start - window + 1):  # (the first query sees start - window + 1 .. start)
+            c.pool[c.block_table[r, p // ps], :, :, p % ps] = (float("inf"), float("nan"), -float("inf"))[p % 3]
+    tiles, out = c.tiles(k.attn_tile_sizes()[1])[rows:].contiguous(), torch.empty(c.T, H * hd, dtype=torch.bfloat16, device=DEV)
+    at = (c.q.to(DEV), c.kv, c.block_table_dev, c.token_req, c.positions, tiles, len(ql))
+    if mixed:
+        k.attn_mixed(out, *at, torch.arange(rows, dtype=torch.int32, device=DEV), rows, H, c.scale, window)
+    else:
+        k.attn_prefill(out, *at, H, c.scale, window)
+    # (the weights are rounded to bfloat16, 2^-9 of each, and meet values of up to 4.5)
+    assert (out.double().cpu() - c.reference()).abs().max().item() < 2.5e-2
+
+
 def test_attn_prefill_far_key_stands_out():
     """Every query of a long portion points at one far key of its own."""
     k = _k()
