@@ -25,7 +25,8 @@
 
 // T: uint16_t (bfloat16 bits) or float.  CPK lanes per key: head_dim = EPL * CPK.  ONCE: every key is read by one block
 // (as many key heads as query heads), with the streaming hint.  Where query heads share a key head, blocks that read the
-// same keys find them in the die's L2 or on their way to it, and a hinted line is gone by then: 64 rows of 28 query heads
+// same keys find them in the die's L2 or on their way to it (which is why their rows are the fast index, below), and a hinted line
+// is gone by then: 64 rows of 28 query heads
 // of 128 over 4 key heads 819 us at contexts of 6,000 to 8,001 and 107 at 700 to 1,300, 691 and 79 without the hint; 32 of
 // 32 over 8 396 and 294; float, 64 of 16 of 128 over 4 938 and 686.  (At few rows and short contexts it is the hint that is
 // ahead there too, by 3 to 8 %: 8 rows of 16 of 64 over 4, 60 to 500 keys, 7.3 and 7.9 us.)
@@ -66,12 +67,21 @@ __attribute__((amdgpu_waves_per_eu(CPK >= 16 ? 2 : 4, CPK == 8 && sizeof(T) == 2
     asm volatile("" ::"v"(seen));  // the loads stay although nobody wants the values
     return;
   }
-  // A row's heads are neighbours in the launch.  Blocks go to the compute units in turn, so with the rows as the fast index
-  // and 64 rows every 256th block was the same row's: a unit had the longest row's heads and no others.  25 heads of 64,
-  // us, rows fast and heads fast: 64 rows at 300 to 1,001 keys 47.7 and 46.7, 48 at 16 to 1,000 32.3 and 30.5, 16 at 500 to 8,001 100
-  // and 90, 8 at 4,000 to 8,001 57.9 and 56.5; rows of one length, 24 of 550 and 8 of 6,000, 18.0 and 18.0, 48.3 and 49.
-  const int lin = blockIdx.x + gridDim.x * blockIdx.y, item = lin / p.n_heads;
-  attend_row<T, CPK, ONCE, SHAPED, MAX_WAVES>(p, wave, n_waves, item, lin - item * p.n_heads, blockIdx.z);
+  // With a key head each, a row's heads are neighbours in the launch.  Blocks go to the compute units in turn, so with the rows as
+  // the fast index and 64 rows every 256th block was the same row's: a unit had the longest row's heads and no others.  25 heads of
+  // 64, us, rows fast and heads fast: 64 rows at 300 to 1,001 keys 47.7 and 46.7, 48 at 16 to 1,000 32.3 and 30.5, 16 at 500 to
+  // 8,001 100 and 90, 8 at 4,000 to 8,001 57.9 and 56.5; rows of one length, 24 of 550 and 8 of 6,000, 18.0 and 18.0, 48.3 and 49.
+  // Where heads share keys the rows are the fast index: blocks go to the eight dies in turn too, and at a multiple of eight rows the
+  // heads of a group are on one die, whose L2 has the keys after the first.  As neighbours they are on as many dies, each of
+  // which reads the keys; rows fast and heads fast: 32 heads of 128 over 8, 8 rows at 60 to 500 keys 9.9 and 12.3, at 4,000 to
+  // 8,001 83.5 and 126, 12 at 500 to 3,000 57.6 and 60.0, 64 at 300 to 1,001 71.3 and 108, at 2,000 to 6,000 397 and 628; 28 over 4,
+  // the same, 10.0 / 11.5, 83 / 107, 57 / 62, 58 / 92, 388 / 553; float, 24 of 128 over 8, 64 at 300 to 1,001 110 and 161.
+  int item = blockIdx.x, h = blockIdx.y;
+  if constexpr (ONCE) {
+    const int lin = blockIdx.x + gridDim.x * blockIdx.y;
+    item = lin / p.n_heads, h = lin - item * p.n_heads;
+  }
+  attend_row<T, CPK, ONCE, SHAPED, MAX_WAVES>(p, wave, n_waves, item, h, blockIdx.z);
 }
 
 // attn_decode_group: bfloat16, the query heads that share a key head taken together.  Where many
