@@ -1036,13 +1036,15 @@ static int prefill_launch(void* out, const void* q, int ldq, int ldo, const void
   // (the kept first keys' pages lie before the window's; a page can be in both runs)
   const size_t lds = (size_t)(max_blocks + (extras ? 2 : 0)) * sizeof(int);
   const bool pow2 = p.page_shift >= 0;
+  // (pages of one to eight keys, of which a copy of sixteen would take several, keep the general kernel and its shifts: by
+  // divisions, and so without two groups, 25 heads in pages of eight took 82.7 us for 512 on 4,000 earlier keys, 57.9 with, 8,000 361 / 328)
   const bool ring = head_dim == 64 && !extras && p.page_shift >= 4;
   // Two groups a block where the blocks are no more than the CUs, so that a block's walk is the kernel's time: 1,024 tokens
   // of 25 heads of 64 (200 blocks) 19.1 us beside 21.3, 512 on 4,000 earlier keys 57 / 72, of 16 heads of 32 43 / 58.  With
   // more blocks than CUs they are in each other's way (2 x 1,024 tokens of 25 heads, 400 blocks: 25.5 / 23.1; 4 x 512:
   // 20.7 / 15.2).  The kernel for heads of 64 without terms, one row of figures each: 1,024 16.9 / 18.4, 512 on 4,000 49 / 59.4;
   // 2 x 1,024 23.2 / 20.8, 4 x 512 18.4 / 13.5.  Heads of 128 and more take the registers of a whole SIMD a wave.
-  const bool two = head_dim <= 64 && pow2 && (extras || head_dim != 64 || ring) && max_blocks <= 4096 && (long)n_heads * n_tiles <= n_compute_units();
+  const bool two = head_dim <= 64 && pow2 && max_blocks <= 4096 && (long)n_heads * n_tiles <= n_compute_units();
   const dim3 grid(n_heads, n_tiles), block(two ? 512 : 256);
 #define LAUNCH_AS(HD, POW2, GROUPS)                                                                                      \
   do {                                                                                                                  \
@@ -1050,17 +1052,17 @@ static int prefill_launch(void* out, const void* q, int ldq, int ldo, const void
       hipLaunchKernelGGL((attn_prefill_kernel<HD, POW2, true, true, GROUPS>), grid, block, lds, stream, p);             \
     else if (extras)                                                                                                    \
       hipLaunchKernelGGL((attn_prefill_kernel<HD, POW2, true, false, GROUPS>), grid, block, lds, stream, p);            \
-    else if constexpr (HD != 64 || !POW2)                                                                               \
+    else                                                                                                                \
       hipLaunchKernelGGL((attn_prefill_kernel<HD, POW2, false, false, GROUPS>), grid, block, lds, stream, p);           \
   } while (0)
 #define LAUNCH_PREFILL(HD)              \
   do {                                  \
-    if (!pow2 || (HD == 64 && !extras)) { \
-      LAUNCH_AS(HD, false, 1);          \
-    } else if (two) {                   \
+    if (two) {                          \
       LAUNCH_AS(HD, true, (HD <= 64 ? 2 : 1)); \
-    } else {                            \
+    } else if (pow2) {                  \
       LAUNCH_AS(HD, true, 1);           \
+    } else {                            \
+      LAUNCH_AS(HD, false, 1);          \
     }                                   \
   } while (0)
   if (rows) {  // (attn_mixed has looked at what the rows need beyond this)
