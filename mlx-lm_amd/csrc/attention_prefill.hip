@@ -560,10 +560,13 @@ __device__ __forceinline__ i16x4_t read_transposed(uint32_t at) {
 __device__ __forceinline__ bf16x8_t read_piece(uint32_t at) {
   return *(const __attribute__((address_space(3))) bf16x8_t*)(uintptr_t)at;
 }
-// the larger of a value and the one of the lane 32 away (the maximum as an instruction: fmaxf first makes its operands
-// canonical, which these are)
+// The larger of a value and the one of the lane 32 away (the maximum as an instruction: fmaxf first makes its operands
+// canonical, which these are).  The swap exchanges halves of two registers and says nothing of one register with itself, so
+// the second operand is made a value of its own, which the compiler cannot put where the first one lies.
 __device__ __forceinline__ float max_of_halves(float v) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  uint32_t mine = __float_as_uint(v), copy = mine;
+  asm("" : "+v"(copy));
+  const auto r = __builtin_amdgcn_permlane32_swap(mine, copy, false, false);
   float larger;
   asm("v_max_f32 %0, %1, %2" : "=v"(larger) : "v"(r[0]), "v"(r[1]));
   return larger;
