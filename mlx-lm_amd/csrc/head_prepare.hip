@@ -156,7 +156,7 @@ __device__ __forceinline__ void prepare_head(const PrepareArgs& a, long item, in
 }
 
 // The same for heads of up to 64 CPL columns, convolutions of up to four taps and norms over a head: what every mixer here
-// but those with wider heads or a norm over the whole projection has.  A wave takes R neighbouring rows of a head.
+// but those with wider heads or a norm over the whole projection has.  A wave takes R neighbouring rows of a head, one or eight.
 //
 // What bounds it: at few rows the trips to memory that follow one another, at many rows the same trips, paid once a row and head by
 // the kernel above (which looks up a request, its first row, its state row and a page one after another, then takes the
@@ -409,14 +409,25 @@ static int prepare_args_fit(const PrepareArgs& a) {
   return 0;
 }
 
-// Rows a wave takes where there are many: eight leave a wave's lookups an eighth a row.  Fewer rows than 128 would not give
-// the compute units a block each (16 heads: 128 / 8 x 16 / 4 = 64 blocks, with three preparations a launch 160).
+// Rows a wave takes where there are many: eight leave a wave's lookups an eighth a row, but its eight rows follow one another
+// (norms and turns), 3.5 to 4.5 us of them.  So runs are for launches that give every compute unit several waves of them, eight
+// with a convolution, whose inputs a run shares, twelve without.  us, a row and runs of eight, (row, head)s: through four taps 2 heads
+// of 64, 2,000 rows (4,000) 4.5 and 7.1, 8,000 (16,000) 11.2 and 9.6; 32 heads, 128 rows (4,096) 4.5 and 7.2, 300 (9,600) 7.0 and
+// 8.4, 512 (16,384) 10.2 and 9.3, 2,000 31.1 and 21.0; without, 16 heads of 224, 300 rows (4,800) 5.4 and 8.7, 1,000 (16,000) 11.3 and
+// 12.2, 2,000 (32,000) 19.0 and 17.9, 8,000 62 and 48; one head of 224, 128 rows 3.4 and 7.6, 8,000 7.2 and 9.5.
 #define PREPARE_ROWS 8
-#define PREPARE_ROWS_FROM 128
+#define PREPARE_RUNS_A_CU 12
+#define PREPARE_CONV_RUNS_A_CU 8
 template <typename T>
 static void launch_many(PrepareMany& m, bool in_rows, hipStream_t stream) {
-  bool many = in_rows;
-  for (int i = 0; i < m.n; ++i) many = many && m.seg[i].n_rows >= PREPARE_ROWS_FROM && !(m.seg[i].conv_w && m.seg[i].conv_single);
+  bool many = in_rows, conv = false;
+  long runs = 0;
+  for (int i = 0; i < m.n; ++i) {
+    many = many && !(m.seg[i].conv_w && m.seg[i].conv_single);
+    conv = conv || m.seg[i].conv_w;
+    runs += (long)((m.seg[i].n_rows + PREPARE_ROWS - 1) / PREPARE_ROWS) * m.seg[i].n_heads;
+  }
+  many = many && runs >= (long)(conv ? PREPARE_CONV_RUNS_A_CU : PREPARE_RUNS_A_CU) * n_compute_units();
   const int R = many ? PREPARE_ROWS : 1;
   unsigned blocks = 0;
   for (int i = 0; i < m.n; ++i) {

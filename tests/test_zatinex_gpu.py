@@ -146,17 +146,33 @@ def test_heads_normed_turned_and_placed(dtype):
     assert (dst2.double().cpu()[:, :14] - want2).abs().max() <= tol and (dst2[:, 14:] == 0).all()
 
 
+PREPARED = [(64, 64, 64, 0, 64, 4), (64, 64, 0, 0, 0, 3), (100, 128, 90, 90, 10, 2), (224, 256, 192, 192, 32, None), (130, 136, 130, 2, 128, 4),
+            (40, 64, 40, 0, 8, 5)]
+
+
 @pytest.mark.parametrize("rows", [5, 127, 128, 131, 300])
-@pytest.mark.parametrize("dim,fill,norm,rot_off,rot_dims,taps", [(64, 64, 64, 0, 64, 4), (64, 64, 0, 0, 0, 3), (100, 128, 90, 90, 10, 2),
-                                                                 (224, 256, 192, 192, 32, None), (130, 136, 130, 2, 128, 4), (40, 64, 40, 0, 8, 5)])
+@pytest.mark.parametrize("dim,fill,norm,rot_off,rot_dims,taps", PREPARED)
 @pytest.mark.parametrize("interleaved", [False, True])
 def test_heads_prepared_in_runs_of_rows(rows, dim, fill, norm, rot_off, rot_dims, taps, interleaved):
-    """Runs of rows of one wave around where they begin (128 rows) and end (a remainder), requests of one to three rows (fewer
-    than the taps) and longer ones in a run, earlier inputs in the state; heads of one, two and four columns a lane, a head with
-    more taps than a run takes; rows of a matrix and, in the same launch, a cache's pages."""
+    """Few heads, a row of a head a wave: requests of one to three rows (fewer than the taps) and longer ones, earlier inputs in
+    the state; heads of one, two and four columns a lane, a head with more taps than such a wave takes; rows of a matrix and, in
+    the same launch, a cache's pages."""
+    _heads_prepared(3, rows, dim, fill, norm, rot_off, rot_dims, taps, interleaved)
+
+
+@pytest.mark.parametrize("rows", [119, 120, 121, 128, 131, 300])
+@pytest.mark.parametrize("dim,fill,norm,rot_off,rot_dims,taps", PREPARED)
+def test_heads_prepared_in_runs_of_eight_rows(rows, dim, fill, norm, rot_off, rot_dims, taps):
+    """So many heads that a launch of 121 rows on gives every compute unit (256) eight waves of eight rows each (two preparations
+    of 64 heads through a convolution), or twelve (96 heads without one): around where runs begin, with and without a
+    remainder, requests' ends within a run."""
+    _heads_prepared(64 if taps else 96, rows, dim, fill, norm, rot_off, rot_dims, taps, rows % 2 == 0)
+
+
+def _heads_prepared(H, rows, dim, fill, norm, rot_off, rot_dims, taps, interleaved):
     from mlx_lm_amd.ops import kernels
 
-    H, ps = 3, 16
+    ps = 16
     g = torch.Generator().manual_seed(rows + dim)
     lens = []
     while sum(lens) < rows:
