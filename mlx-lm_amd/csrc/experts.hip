@@ -212,21 +212,26 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(const T* __restrict__ gu,
   out[(size_t)r * ldo + f] = from_f32<T>((GELU ? gelu_tanh(z) : silu_f(z)) * to_f32(row[F + f]));
 }
 
-// The same for bfloat16 rows of eight gate columns and the same eight of up by turns: 16 bytes of each a thread.
-template <bool GELU>
+// The same for bfloat16 rows of eight gate columns and the same eight of up by turns: V of each a thread, eight (16 bytes) where
+// that gives every SIMD a wave, else two: eight activations one after another are 0.3 to 0.5 us of a launch of some 3.  With the product
+// ahead, us, eight a thread and two: 130 rows of 128 (K 1,024) 9.8 and 9.4, 64 of 256 (512) 7.9 and 7.3, 130 of 2,688 (1,024) 11.1 and
+// 10.8; a value a thread in rows [gate | up] 9.3, 7.4, 10.8, and 56.6 for 130 rows of 11,008 (4,096), 55.0 with eight.
+template <bool GELU, int V>
 __global__ __launch_bounds__(256) void silu_mul_turns_kernel(const uint16_t* __restrict__ gu, int ld, uint16_t* __restrict__ out, int ldo, int F) {
-  const int f = (blockIdx.y * 256 + threadIdx.x) * 8, r = blockIdx.x;
+  static_assert(V == 2 || V == 8, "words of two columns, whole turns of eight");
+  typedef uint32_t piece_t __attribute__((ext_vector_type(V / 2)));
+  const int f = (blockIdx.y * 256 + threadIdx.x) * V, r = blockIdx.x;
   if (f >= F) return;
-  const u32x4_t* in = (const u32x4_t*)(gu + (size_t)r * ld + 2 * f);
-  const u32x4_t g = in[0], u = in[1];
-  u32x4_t o;
+  const uint16_t* const in = gu + (size_t)r * ld + 2 * (f & ~7) + (f & 7);
+  const piece_t g = *(const piece_t*)in, u = *(const piece_t*)(in + 8);
+  piece_t o;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
+  for (int i = 0; i < V / 2; ++i) {
     const float g0 = __uint_as_float(g[i] << 16), g1 = __uint_as_float(g[i] & 0xffff0000u);
     const float u0 = __uint_as_float(u[i] << 16), u1 = __uint_as_float(u[i] & 0xffff0000u);
     o[i] = pack_bf16x2((GELU ? gelu_tanh(g0) : silu_f(g0)) * u0, (GELU ? gelu_tanh(g1) : silu_f(g1)) * u1);
   }
-  *(u32x4_t*)(out + (size_t)r * ldo + f) = o;
+  *(piece_t*)(out + (size_t)r * ldo + f) = o;
 }
 
 // ROWS dot products of one vector b with ROWS rows a[r] over a lane's share of K, all loads of a step on
@@ -824,11 +829,12 @@ extern "C" int act_mul_turns(const void* gu, int ld, void* out, int ldo, int n_r
   if (activation != 0 && activation != 1) FAIL("act_mul_turns: unknown activation code %d", activation);
   if (!gu || !out || (((uintptr_t)gu | (uintptr_t)out) & 15) || F % 8 != 0 || ld % 8 != 0 || ldo % 8 != 0 || ld < 2 * F || ldo < F)
     FAIL("act_mul_turns: rows of %d for 2 x %d, output rows of %d, in whole pieces of 16 bytes", ld, F, ldo);
-  const dim3 grid(n_rows, (F / 8 + 255) / 256), block(256);
-  if (activation)
-    hipLaunchKernelGGL(silu_mul_turns_kernel<true>, grid, block, 0, stream, (const uint16_t*)gu, ld, (uint16_t*)out, ldo, F);
-  else
-    hipLaunchKernelGGL(silu_mul_turns_kernel<false>, grid, block, 0, stream, (const uint16_t*)gu, ld, (uint16_t*)out, ldo, F);
+  const bool wide = (long)n_rows * (F / 8) >= 4L * 64 * n_compute_units();
+  void (*const kernel)(const uint16_t*, int, uint16_t*, int, int) =
+      wide ? (activation ? silu_mul_turns_kernel<true, 8> : silu_mul_turns_kernel<false, 8>)
+           : (activation ? silu_mul_turns_kernel<true, 2> : silu_mul_turns_kernel<false, 2>);
+  const int items = F / (wide ? 8 : 2);
+  hipLaunchKernelGGL(kernel, dim3(n_rows, (items + 255) / 256), dim3(256), 0, stream, (const uint16_t*)gu, ld, (uint16_t*)out, ldo, F);
   CHECK_LAUNCH("act_mul_turns");
   return 0;
 }

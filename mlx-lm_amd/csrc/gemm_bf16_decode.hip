@@ -201,7 +201,10 @@ __device__ __forceinline__ void finish4(const DecodeGemmArgs& p, int m, int n, f
 // kernel each because a launch of 3 to 5 us waits for its instructions too (both ways in one cost 0.1 to 0.2 us).
 // GATED: the features come in pairs of eight, gate and what it gates, and out gets act(gate) * other (N / 2 columns):
 // both lie in one block's tile.  The activation's own launch took 3.9 us a layer beside a product of 6.5 (8 rows of 1,024 to
-// 2 x 2,688), the product with it takes what it took without.
+// 2 x 2,688), the product with it takes what it took without.  Blocks of sixteen features and K whole cost less than that
+// launch also where the plain product takes eight features or parts of K; both launches and this one, us, 1 / 8 rows: 512 features of
+// K 1,024 5.4 and 3.4 / 5.6 and 3.6, 256 of 4,096 6.6 and 5.2 / 7.4 and 5.6, 1,024 of 4,096 8.8 and 7.0 / 11.4 and 7.6, 1,536 of 2,048 7.4 and
+// 5.2 / 10.7 and 5.6, 128 of 8,192 8.4 and 7.1 (eight rows do not fit), 11,008 of 4,096 43.0 and 40.5 / 47.4 and 44.6.
 template <bool LN, bool MULTI, bool FEW, bool GATED = false>
 __global__ __launch_bounds__(NW * 64) void gemm_bf16_decode_kernel(DecodeGemmArgs p) {
   constexpr int NV = LN_MAX_V;

@@ -799,6 +799,23 @@ def test_gated_product(M, F, K, rows, activation):
     assert torch.isnan(out[:, F:].float()).all()
 
 
+@pytest.mark.parametrize("M", [17, 195, 196, 400])
+@pytest.mark.parametrize("F", [8, 2688])
+@pytest.mark.parametrize("activation", ["silu", "gelu_tanh"])
+def test_gated_product_activation_of_many_rows(M, F, activation):
+    """The activation's launch behind a product by turns, around where a thread takes eight columns instead of two (196 rows of 2,688:
+    a wave for each of 1,024 SIMDs): the bits of the same activation on rows [gate | up], and nothing beside its rows."""
+    k = _k()
+    g = torch.Generator().manual_seed(M + F)
+    gate, up = (torch.randn(F, 64, generator=g).to(torch.bfloat16).to(DEV) for _ in range(2))
+    x = torch.randn(M, 64, generator=g).to(torch.bfloat16).to(DEV)
+    rows, both = torch.full((M, F + 8), 3.0, dtype=torch.bfloat16, device=DEV), torch.empty(M, 2 * F, dtype=torch.bfloat16, device=DEV)
+    k.gated_linear(lambda shape, dtype: both, rows[:, :F], x, k.PackedWeight(k.gate_in_turns(gate, up)), activation)
+    apart = torch.empty(M, F, dtype=torch.bfloat16, device=DEV)
+    k.silu_mul(apart, both.view(M, F // 8, 2, 8).transpose(1, 2).reshape(M, 2 * F), activation)
+    assert torch.equal(rows[:, :F], apart) and (rows[:, F:] == 3.0).all()
+
+
 @pytest.mark.parametrize("ps", [8, 16, 64, 256])
 @pytest.mark.parametrize("H,Hkv", [(3, 1), (90, 9)])
 @pytest.mark.parametrize("window", [0, 65, 300])
