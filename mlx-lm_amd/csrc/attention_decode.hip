@@ -23,6 +23,11 @@
 // waves) at the end.
 #include "attention_decode_row.h"
 
+// Where the parts of a (row, head) are counted that the kernel joins itself: all launches on a GPU share the counters, so launches that
+// join and overlap on one GPU race.
+#define JOIN_MAX_ITEMS 65536
+static __device__ unsigned join_counters[JOIN_MAX_ITEMS];
+
 // T: uint16_t (bfloat16 bits) or float.  CPK lanes per key: head_dim = EPL * CPK.  ONCE: every key is read by one block
 // (as many key heads as query heads), with the streaming hint.  Where query heads share a key head, blocks that read the
 // same keys find them in the die's L2 or on their way to it (which is why their rows are the fast index, below), and a hinted line
@@ -81,7 +86,7 @@ __attribute__((amdgpu_waves_per_eu(CPK >= 16 ? 2 : 4, CPK == 8 && sizeof(T) == 2
     const int lin = blockIdx.x + gridDim.x * blockIdx.y;
     item = lin / p.n_heads, h = lin - item * p.n_heads;
   }
-  attend_row<T, CPK, ONCE, SHAPED, MAX_WAVES>(p, wave, n_waves, item, h, blockIdx.z);
+  attend_row<T, CPK, ONCE, SHAPED, MAX_WAVES, true>(p, wave, n_waves, item, h, blockIdx.z, join_counters);
 }
 
 // attn_decode_group: bfloat16, the query heads that share a key head taken together.  Where many

@@ -112,10 +112,7 @@ __device__ __forceinline__ void put(float* at, float v) { *at = v; }
 // Joining a row's parts inside the kernel.  The parts' sums pass between blocks on different
 // dies, whose L2s do not see each other's lines: they are written and read at agent scope (past
 // the die's L2), and a counter a (row, head) says when all are there.  The counters are zero
-// between launches (the block that arrives last puts its counter back); all launches on a GPU
-// share them, so launches that overlap on one GPU race.
-#define JOIN_MAX_ITEMS 65536
-static __device__ unsigned join_counters[JOIN_MAX_ITEMS];
+// between launches (the block that arrives last puts its counter back).
 __device__ __forceinline__ void put_shared(float* at, float v) {
   __hip_atomic_store(at, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -138,9 +135,10 @@ __device__ __forceinline__ bool last_to_arrive(unsigned* counter, unsigned n_par
 
 // (see attn_decode_kernel) The keys of `item`'s head h, part `split` of them, by up to WAVES waves, n_waves of them here.  (The
 // caller asks for the block's size, ahead of its branches: asked for here it was one more trip, 0.2 to 0.9 % of a decode step.)
-// The launch's dynamic LDS holds max_blocks page numbers with table_in_lds.
-template <typename T, int CPK, bool ONCE, bool SHAPED, int WAVES>
-__device__ __forceinline__ void attend_row(const DecodeArgs& p, int wave, int n_waves, int item, int h, int split) {
+// The launch's dynamic LDS holds max_blocks page numbers with table_in_lds.  PARTS: a row may be in several (p.n_splits);
+// join_counters: a counter a (row, head), for parts that are joined here.
+template <typename T, int CPK, bool ONCE, bool SHAPED, int WAVES, bool PARTS>
+__device__ __forceinline__ void attend_row(const DecodeArgs& p, int wave, int n_waves, int item, int h, int split, unsigned* join_counters) {
   constexpr int EPL = 16 / sizeof(T);  // elements a lane holds of a key
   constexpr int HD = EPL * CPK;
   // two loads of keys at least: where 1 KB holds sixteen keys, a tile of one load left a wave twice the trips (bfloat16,
@@ -202,8 +200,8 @@ __device__ __forceinline__ void attend_row(const DecodeArgs& p, int wave, int n_
   // Joined here, a row may take fewer splits than the launch has: as many as leave a wave
   // ATTN_DECODE_KEYS_A_PART keys, and one if a wave has few anyway (joining costs about 32 keys'
   // time).  Blocks of the splits it does not take have nothing to do.
-  int n_splits = p.n_splits;
-  if (p.join_here == 2) {
+  int n_splits = PARTS ? p.n_splits : 1;
+  if (PARTS && p.join_here == 2) {
     const int keys_a_wave = (k_hi - kt0 + n_sink_tiles * TILE) / n_waves;
     n_splits = keys_a_wave >= SPLIT_FROM ? min(n_splits, keys_a_wave / ATTN_DECODE_KEYS_A_PART) : 1;
     if (split >= n_splits) return;  // (the whole block)
@@ -335,7 +333,7 @@ __device__ __forceinline__ void attend_row(const DecodeArgs& p, int wave, int n_
     L += Ls[i] * w;
     if (tid < HD) acc += Os[i][tid] * w;
   }
-  if (n_splits > 1 && p.join_here) {  // (uniform over the block)
+  if (PARTS && n_splits > 1 && p.join_here) {  // (uniform over the block)
     const size_t first = ((size_t)item * p.n_heads + h) * p.n_splits;
     if (tid < HD) put_shared(p.part_o + (first + split) * HD + tid, acc);
     if (tid == 0) put_shared(p.part_ml + (first + split) * 2, M), put_shared(p.part_ml + (first + split) * 2 + 1, L);
@@ -366,7 +364,7 @@ __device__ __forceinline__ void attend_row(const DecodeArgs& p, int wave, int n_
     return;
   }
   if (tid < HD) {
-    if (n_splits == 1) {
+    if (!PARTS || n_splits == 1) {
       put((T*)p.out + out_at(p, row, h * HD + tid),
           acc / with_sink(p, h, M, L) * head_gate_of(p, row, h) * gate_at<T>(p, row, h * HD + tid));
     } else {

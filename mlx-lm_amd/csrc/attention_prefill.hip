@@ -968,7 +968,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
   if (item < n_tiles) {
     attend_tile<HD, 1>(p, h, item, ring, page_at);
   } else {
-    attend_row<uint16_t, HD / 8, true, false, 4>(rows, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), 4, item - n_tiles, h, 0);
+    attend_row<uint16_t, HD / 8, true, false, 4, false>(rows, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), 4, item - n_tiles, h, 0, nullptr);
   }
 }
 
