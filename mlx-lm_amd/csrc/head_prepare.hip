@@ -23,9 +23,9 @@
 //   diff_combine    o = a1 - lambda a2 per head, where a1 and a2 are two heads of an attention's
 //                   output (tables say which), divided by its root mean square and multiplied by
 //                   `mult`.
-//   head_gate       x[t, h, :] *= sigmoid(g[t, h]), in place.
+//   head_gate       x[t, h, :] *= sigmoid(g[t, h]), in place, for heads that are there already (the latent attention's gate is a
+//                   term of its attention kernels).
 #include "common.h"
-
 
 #define PREPARE_CONV_MAX_DIM 256  // the widest head that passes a convolution
 

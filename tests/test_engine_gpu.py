@@ -199,8 +199,9 @@ def test_mixed_batches_with_few_pages(folders, dtype, name, sharp):
 
 @pytest.mark.parametrize("record", [False, True])
 def test_portions_beside_decoding_rows_of_heads_of_64(tmp_path, monkeypatch, record):
-    """Heads of 64 in bfloat16, where a portion and the rows beside it share a launch of attention: logits of both against
-    the plain implementation, steps of one shape run again (recorded where that is asked for)."""
+    """Heads of 64 in bfloat16, where a portion and the rows beside it share a launch of attention (a launch a layer less than in
+    pages of 48 keys, which keep two): logits of both against the plain implementation, steps of one shape run again
+    (recorded where that is asked for)."""
     from mlx_lm_amd.engine import Engine, StepEntry
     from mlx_lm_amd.utils import load_model
 
@@ -208,21 +209,27 @@ def test_portions_beside_decoding_rows_of_heads_of_64(tmp_path, monkeypatch, rec
     monkeypatch.setitem(helpers.TINY, "HEADS64", (config, 11, "b"))
     _, weights = helpers.make_folder(str(tmp_path), "HEADS64", 8.0)
     model, _ = load_model(str(tmp_path), dtype="bfloat16")
-    eng = Engine(model, dtype="bfloat16", page_size=16, max_tokens=6000, max_requests=16, record_prompt_steps=record)
     rows = {f"r{i}": helpers.random_tokens(n, config["vocab_size"], i) for i, n in enumerate((20, 64, 65, 129, 200, 301, 440))}
-    for rid, toks in rows.items():
-        eng.add_request(rid)
-        eng.step([StepEntry(rid, toks[:-4], [0])])
     want = {rid: _plain_logits(weights, config, toks, "bfloat16") for rid, toks in rows.items()}
-    for step in range(4):
-        portion = helpers.random_tokens(130, config["vocab_size"], 50 + step)
-        eng.add_request("portion")
-        entries = [StepEntry(rid, [toks[len(toks) - 4 + step]], [0]) for rid, toks in rows.items()]
-        logits = eng.step(entries + [StepEntry("portion", portion, [0, 64, 129])])
-        for i, rid in enumerate(rows):
-            _close(logits[i], want[rid][len(rows[rid]) - 4 + step], "bfloat16", f"{rid}, step {step}")
-        _close(logits[len(rows) :], _plain_logits(weights, config, portion, "bfloat16")[[0, 64, 129]], "bfloat16", f"portion {step}")
-        eng.end_request("portion")
+    launches = {}
+    for page_size in (48, 16):
+        eng = Engine(model, dtype="bfloat16", page_size=page_size, max_tokens=6000, max_requests=16, record_prompt_steps=record)
+        for rid, toks in rows.items():
+            eng.add_request(rid)
+            eng.step([StepEntry(rid, toks[:-4], [0])])
+        before = eng.stats.launches
+        for step in range(4):
+            portion = helpers.random_tokens(130, config["vocab_size"], 50 + step)
+            eng.add_request("portion")
+            entries = [StepEntry(rid, [toks[len(toks) - 4 + step]], [0]) for rid, toks in rows.items()]
+            logits = eng.step(entries + [StepEntry("portion", portion, [0, 64, 129])])
+            for i, rid in enumerate(rows):
+                _close(logits[i], want[rid][len(rows[rid]) - 4 + step], "bfloat16", f"{rid}, step {step}, pages of {page_size}")
+            _close(logits[len(rows) :], _plain_logits(weights, config, portion, "bfloat16")[[0, 64, 129]], "bfloat16", f"portion {step}")
+            eng.end_request("portion")
+        launches[page_size] = eng.stats.launches - before
+    if not record:  # (a step that is replayed counts none)
+        assert launches[16] == launches[48] - 4 * config["n_layer"]
 
 
 @pytest.mark.parametrize("dtype", ["bfloat16", "float32"])

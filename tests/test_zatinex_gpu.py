@@ -248,6 +248,51 @@ def test_two_maps_joined_and_heads_gated(dtype):
     assert (x.double().cpu().view(T, H, hd) - want).abs().max() <= tol
 
 
+@pytest.mark.parametrize("kernel,dtype,H,d,splits", [
+    ("prefill", torch.bfloat16, 16, 256, 1), ("prefill", torch.bfloat16, 5, 64, 1), ("group", torch.bfloat16, 16, 256, 1),
+    ("group", torch.bfloat16, 16, 256, 4), ("group", torch.bfloat16, 12, 64, 3), ("decode", torch.bfloat16, 4, 256, 1), ("decode", torch.bfloat16, 4, 256, 3),
+    ("tile", torch.float32, 16, 256, 1), ("tile", torch.bfloat16, 4, 40, 1), ("row", torch.float32, 6, 80, 3)])
+def test_the_heads_gate_on_attentions_way_out(kernel, dtype, H, d, splits):
+    """Attention of many heads over one key head (a latent's), each head's output times the sigmoid of its column of a
+    wider float32 matrix and nothing else beside the scores; gates that all but close a head and that leave it as it is."""
+    from mlx_lm_amd.ops import kernels
+    from test_pafutar_gpu import _paged
+
+    offset, n_q = 300, {"tile": 16, "prefill": 150}.get(kernel, 3)
+    n = offset + n_q
+    g = torch.Generator().manual_seed(d + H)
+    q, k, v = (torch.randn(*shape, generator=g).to(dtype) for shape in ((n_q, H, d), (n, 1, d), (n, 1, d)))
+    gate = torch.randn(n_q, H, generator=g) * 2
+    gate[0, 0], gate[-1, -1], gate[1, 0] = -30.0, 30.0, -120.0
+    s = torch.einsum("ihd,jd->hij", q.double(), k[:, 0].double()) / d**0.5
+    i, j = torch.arange(n_q)[:, None] + offset, torch.arange(n)[None, :]
+    want = torch.einsum("hij,jd->ihd", torch.softmax(s.masked_fill((j > i)[None], float("-inf")), -1), v[:, 0].double())
+    want = (want * torch.sigmoid(gate.double())[:, :, None]).reshape(n_q, H * d)
+
+    kv, block_table = _paged(k, v, 16, dtype, seed=d)
+    qd = q.reshape(n_q, H * d).cuda()
+    out = torch.empty_like(qd)
+    wide = torch.full((n_q, H + 7), float("nan"))
+    wide[:, 3 : 3 + H] = gate
+    terms = kernels.ScoreTerms(head_gate=wide.cuda()[:, 3 : 3 + H])
+    tables = (block_table, torch.zeros(n_q, dtype=torch.int32, device="cuda"), (torch.arange(n_q, dtype=torch.int32) + offset).cuda())
+    items, parts = torch.arange(n_q, dtype=torch.int32).cuda(), [torch.empty(n_q * H * splits * m, device="cuda") for m in (d, 2)]
+    if kernel == "tile":
+        kernels.attn_tile(out, qd, kv, *tables, _ints([0, n_q]), 1, H, d**-0.5, 0, terms)
+    elif kernel == "prefill":
+        kernels.attn_prefill(out, qd, kv, *tables, _ints([128, n_q - 128, 0, 128]), 2, H, d**-0.5, 0, terms)
+    elif kernel == "row":
+        kernels.attn_row(out, qd, kv, *tables, items, n_q, H, d**-0.5, 0, splits, *parts, terms)
+    elif kernel == "group":
+        kernels.attn_decode_group(out, qd, kv, *tables, items, n_q, H, d**-0.5, 0, splits, *parts, terms=terms)
+    else:
+        kernels.attn_decode(out, qd, kv, *tables, items, n_q, H, d**-0.5, 0, splits, *parts, n_waves=4, terms=terms)
+    # (bfloat16: weights rounded to 2^-9 of each, outputs to 2^-9 of themselves, of values of up to 4.5)
+    assert (out.double().cpu() - want).abs().max() <= (2e-5 if dtype == torch.float32 else 2.5e-2)
+    tiny = want.view(n_q, H, d)[0, 0].abs().max()
+    assert tiny < 1e-12 and out.view(n_q, H, d)[0, 0].abs().max() <= 2 * tiny
+
+
 @pytest.mark.parametrize("taps", [1, 2, 4, 7])
 def test_the_convolution_on_the_way_into_the_heads(taps):
     """``head_prepare`` with a convolution ahead: two requests in portions of 2, 1, 1, 6 and 3 tokens
