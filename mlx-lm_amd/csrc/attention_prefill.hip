@@ -532,19 +532,20 @@ void attn_prefill_kernel(PrefillArgs p) {
 // The same blocks, walks and arithmetic as above.  What differs is how a tile comes to its products, so that the vector
 // unit has little to do but the softmax:
 //  * Keys and values go from the pages to LDS by copies (lds_copy.h), two copies of a kilobyte a wave and tile for
-//    each, into rings of three tiles, asked for two tiles ahead; a page's place is three scalar instructions out of a table in LDS.
+//    each, into rings of three tiles, keys asked for three tiles ahead and values two; a page's place is three scalar instructions out of a table in LDS.
 //    Before, a tile went through registers: a dozen integer instructions an address and 24 to transpose the values.
 //  * Values are transposed by the LDS read (ds_read_b64_tr_b16: four keys of a column a lane).  A lane's eight scores of a
 //    chunk are keys 4 g .. + 3 and 8 + 4 g .. + 3 of it, and two such reads bring the values of just these.
 //  * A row's pieces of 16 bytes lie permuted (piece ^ (row / 2 % 8) of keys, piece ^ 4 (row / 2 % 2) of values), so that the
 //    sixteen rows of a read of keys, and the four rows x 64 bytes of a read of values, meet all banks: no conflict is counted.
 //  * The next tile's scores are begun while this one's probabilities are made, in the registers that are free by then, so
-//    that a wave needs 153 registers and three blocks share a CU.  (With the scores in two sets of registers, a whole tile ahead, 232:
-//    two blocks, 272 us for 8,000 tokens instead of 251.)
-// 25 heads of 64, us, the kernel above and this one (while its outputs left as the other's do; now: at its end): 8,000 tokens 315 and 251 (0.82 PFLOP/s of the causal half), under a window of
-// 1,000 112 and 84; 2 x 1,024 24.5 and 21.2; 1,024 19.6 and 17.2; 512 on 4,000 earlier keys 58.5 and 49; 512 12.3 and 11.4; 333 10.1
-// and 9.4; 128 7.6 and 7.0; 17 4.7 and 4.8.  What bounds it: vector instructions, 74 % of the CUs' cycles beside 41 % for the
-// products (8,000 tokens at 1.88 GHz); at few blocks the way to the first tile and the walk's steps of some 1 us.
+//    that a wave needs fewer registers than the 168 of three waves a SIMD and three blocks share a CU.  (With the scores in two sets of
+//    registers, a whole tile ahead, 232: two blocks, 8 % more for 8,000 tokens.)
+// 25 heads of 64 in pages of sixteen, us, the kernel above and this one: 8,000 tokens 317 and 259 (0.79 PFLOP/s of the causal half), under
+// a window of 1,000 110 and 87; 2 x 1,024 23.7 and 20.2; 512 on 4,000 earlier keys 58.9 and 49.9; 512 12.8 and 10.9; 333 10.4 and
+// 9.4; eight portions of 128 on 300 earlier keys under a window of 77 12.0 and 11.1; 40 on 500 under one of 100 8.4 and 8.4; 17 4.7 and
+// 4.9 (its outputs' way through LDS, below).  What bounds it: vector instructions, 74 % of the CUs' cycles beside 41 % for the products
+// (8,000 tokens at 1.88 GHz); at few blocks the way to the first tile and the walk's steps of some 1 us.
 
 typedef short i16x4_t __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) i16x4_t* lds_i16x4_p;
@@ -914,7 +915,7 @@ __device__ __forceinline__ void attend_tile(const PrefillArgs& p, int h, int til
   const float inv = head_gate_of(p, row0 + min(qi, nq - 1), h) / l;
   // The outputs leave through LDS, as whole rows of 128 bytes that go through to memory: stored as they lie here, pieces of
   // 8 bytes of 32 rows, they had to stay in the L2s and were written back at the kernel's end (2 x 1,024 tokens of 25 heads
-  // 22.2 -> 21.1 us, 512 11.5 -> 10.6, 8,000 271 -> 264, under a window of 1,000 97 -> 86.5; 17 4.8 -> 5.0).
+  // 22.2 -> 21.1 us, 512 11.5 -> 10.6, 8,000 271 -> 264, under a window of 1,000 97 -> 86.5; 17 4.8 -> 5.0: that sitting's figures).
   constexpr int OUT_ROW = ROW + 16;  // bytes from row to row in LDS: sixteen rows' pieces on different banks
   static_assert(4 * 32 * OUT_ROW <= GROUP_LDS, "the outputs fit where the tiles were");
   if (GROUPS == 1) __syncthreads();  // no tile is read any more (of two groups: where the second one's tiles were, which end above)
@@ -974,18 +975,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3))) voi
 
 DEFINE_LAST_ERROR(mlxlm_last_error)
 
-// tiles: n_tiles pairs (first flat row, number of rows 1..128); the rows of a
-// tile are consecutive tokens of one request at consecutive positions.
-// bfloat16 only, head_dim 32, 64, 128 or 256.
-// The longest walk that attn_mixed takes a portion's tiles on: they go by one group of waves a block here, and where few rows
-// stand beside a long walk that costs what the launch saves (512 tokens on 1,500 earlier keys beside 11 rows at 30 to 60: 32.5
-// as two launches, 32.7 as one; beside 24 rows at 200 to 2,000 64.8 and 44.8; 1,024 on 1,024 beside 24 at 30 to 60 33.8 and 32.4).
+// The longest table that attn_mixed takes (the walks themselves are not known where a step is recorded).  Its tiles go by one group of
+// waves a block, and where few short rows stand beside a walk of some 2,000 keys that costs what the launch saves or a little
+// more; us, two launches and one, 512 tokens on 1,500 earlier keys: beside 11 rows at 30 to 60 keys, 25 heads, 32.5 and 32.3, 4 heads
+// 30.0 and 31.0; beside 8 at 200 to 1,000 38.4 and 32.6, 33.5 and 30.9; beside 24 at 200 to 900 47.3 and 35.6, 34.5 and 31.1; at 200 to 2,000
+// 64.8 and 44.8, 25 heads; 1,000 on 1,024 beside 24 at 30 to 60 34.7 and 32.2, 29.4 and 30.1; 16 on 2,000 beside 11 at 30 to 60 29.0 and
+// 27.1, 27.6 and 26.3.  Longer walks are not measured in one launch.
 #define MIXED_MOST_KEYS 2048
 // And the longest row where the decode kernel would give rows eight waves or parts, which are sooner done alone: one row of 700
 // keys beside 16 / 512 / 1,000 tokens 13.1, 19.9, 26.1 (eight waves) and 11.0, 12.2, 19.1 in one launch; four at 200 to 900 14.6,
-// 21.5, 27.7 and 13.5, 14.3, 19.2; eight at 200 to 1,000 16.3, 22.9, 29.3 and 15.7, 16.2, 19.6: level beside the fewest tokens.
+// 21.5, 27.7 and 13.5, 14.3, 19.2; eight at 200 to 1,000 16.3, 22.9, 29.3 and 15.7, 16.2, 19.6: level beside the fewest tokens
+// (of 2 heads, whose rows go in parts alone, 12.5 and 13.2 beside 16).
 #define MIXED_MOST_ROW_KEYS 1024
 
+// tiles: n_tiles pairs (first flat row, number of rows 1..128); the rows of a
+// tile are consecutive tokens of one request at consecutive positions.
+// bfloat16 only, head_dim 32, 64, 128 or 256.
 static int prefill_launch(void* out, const void* q, int ldq, int ldo, const void* k_pages,
                           const void* v_pages, size_t page_stride, const int* block_table,
                           int max_blocks, const int* token_req, const int* positions,
