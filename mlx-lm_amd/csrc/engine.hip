@@ -83,7 +83,7 @@ typedef int (*fn_layernorm)(void*, const float*, const int*, const float*, const
                             hipStream_t);
 typedef int (*fn_gemm_f32)(void*, const void*, const void*, const float*, int, int, int, int, int, int, int,
                            int, int, float*, size_t, void*, void*, size_t, const int*, int, const int*, const int*, int, int,
-                           int, int, hipStream_t);
+                           int, int, const int*, float*, size_t, hipStream_t);
 typedef int (*fn_gemm_bf16)(void*, const void*, const void*, const float*, int, int, int, int, int, int, int,
                             int, int, float*, size_t, void*, void*, size_t, const int*, int, const int*,
                             const int*, int, int, int, int, hipStream_t);
@@ -144,6 +144,7 @@ static Entry<fn_layernorm> k_layernorm("norm", "layernorm");
 static Entry<int (*)(void*, const float*, int, const int*, const float*, float, int, int, int, hipStream_t)> k_rmsnorm("rmsnorm", "rmsnorm");
 static Entry<fn_gemm_f32> k_gemm_f32("gemm_f32", "gemm_f32_scatter");
 static Entry<int (*)(int, int)> k_gemm_f32_scatters("gemm_f32", "gemm_f32_scatters");
+static Entry<size_t (*)(int, int, int, int, int)> k_gemm_f32_room("gemm_f32", "gemm_f32_room");
 static Entry<fn_int5> k_gemm_f32_splits("gemm_f32", "gemm_f32_splits");
 static Entry<fn_gemm_bf16> k_gemm_bf16("gemm_bf16", "gemm_bf16_scatter");
 static Entry<fn_int5> k_gemm_bf16_splits("gemm_bf16", "gemm_bf16_splits");
@@ -546,11 +547,22 @@ static int linear(EngCtx* ctx, const EngMat& out, const EngValue& a, const EngWe
     if (sc && (variant == 0 || variant == 3) && sc->n_kv_heads * sc->head_dim == sc->kv_width)
       QUERY(k_gemm_f32_scatters, scatters, M, n_splits);
     const EngScatter* own = scatters ? sc : nullptr;
+    // (rows that the tiles want cut are cut into scratch memory, which the next launches of the stream may have again)
+    EngMat room = {};
+    const size_t mark = ctx->scratch ? ctx->scratch->offset : 0;
+    size_t room_floats = 0;
+    QUERY(k_gemm_f32_room, room_floats, M, N, K, variant, n_splits);
+    if (room_floats) TRY(take(ctx, (int)((room_floats + 1023) / 1024), 1024, DT_F32, &room));
     KERNEL(k_gemm_f32, ctx, out.p, A.p, w.w, bias, M, N, K, A.ld, w.ldw, out.ld, flags, variant, n_splits,
            n_splits > 1 ? ws : nullptr, n_splits > 1 ? ws_floats : (size_t)0, own ? own->k : nullptr, own ? own->v : nullptr,
            own ? own->page_stride : (size_t)0, own ? own->block_table : nullptr, own ? own->max_blocks : 0,
            own ? own->token_req : nullptr, own ? own->positions : nullptr, own ? own->q_width : 0, own ? own->kv_width : 0,
-           own ? own->head_dim : 0, own ? own->page_size : 0, ctx->stream);
+           own ? own->head_dim : 0, own ? own->page_size : 0, w.exponents,
+           (float*)room.p, room_floats, ctx->stream);
+    if (room_floats) {
+      ctx->scratch->offset = mark;
+      if (ctx->stats) ctx->stats->launches++;  // the one that cuts them
+    }
     if (own) return 0;
     if (n_splits > 1) TRY(finish_parts(ctx, out, ws, n_splits, bias, gelu, accumulate, nullptr, pending));
   } else {

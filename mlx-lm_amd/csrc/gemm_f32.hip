@@ -1,11 +1,13 @@
-// Linear layer in true 32-bit: float operands, float products and sums
-// (v_mfma_f32_16x16x4_f32; no reduced-precision matrix mode, no float cut
-// into shorter pieces).
+// Linear layer on float operands with float sums:
 //   out[m, n] = epilogue( sum_k A[m, k] * W[n, k] + bias[n] )
 // A is [M, K], W is [N, K], both contiguous along k.  Epilogues: plain,
 // tanh-GELU, or accumulate into the residual stream.  Any M, N; K % 4 == 0.
 // The 32-bit twin of gemm_bf16.hip; replaces the same nn.Linear calls
 // (mlx_lm/models/gpt2.py:41-42,52,68,76-80,167).
+//
+// Three ways, chosen by rows and prices: up to 64 rows a kernel that streams the weights once and tiles of few blocks both multiply with
+// v_mfma_f32_16x16x4_f32, a sixteenth of bfloat16's rate; where tiles are many, each float is cut into two half-precision
+// numbers (22 to 24 of its 24 bits) and three products of them stand for one, with smaller errors against 64 bits than the former.
 //
 // Up to 64 rows (decode steps) take a kernel of their own, which streams W
 // once through v_mfma_f32_16x16x4_f32, 16 features a block: a 64 x 64 tile
@@ -14,6 +16,7 @@
 // units, K goes in parts and a second kernel (the caller's) adds them up.
 #include "common.h"
 #include "lds_copy.h"
+#include "tile_order.h"
 
 #define FLAG_GELU FLAG_ACT_GELU
 #define FLAG_RELU2 FLAG_ACT_RELU2  // the square of the ReLU instead
@@ -31,6 +34,11 @@ struct GemmArgs {
   // in ws[y][ws_rows][N], without bias or epilogue
   int n_splits, per_split, ws_rows;
   float* ws;
+  // the tiles' rows, cut (cut_rows_kernel), ldc floats apart, and the rows' and features' exponents
+  const float* cut;
+  const int* a_exponents;
+  const int* w_exponents;
+  int ldc;
   int through;  // out and a part of ws are below 4 GB: the tiles' stores go through to memory
   // the kernel for few rows: the features from q_width on are keys and values, which go to their pages too (k_pages null:
   // none do)
@@ -213,6 +221,312 @@ __global__ __launch_bounds__(S::THREADS, 2) void gemm_f32_tile_kernel(GemmArgs p
   }
 }
 
+// Many rows, cut operands.  x = 2^-s (h + l), h the half-precision number nearest to 2^s x and l the one nearest to what h
+// leaves: 11 bits each and a sign, so that h + l is x's 24 bits in three of four cases and misses by its last one in the fourth.  x y is then
+// h h' + h l' + l h', three of v_mfma_f32_32x32x16_f16 (16 times the rate of the float instruction: 5 times its products); l l', 2^-22 of x y at
+// most, is left out.  One power of two a row of A and of W puts the row's greatest value between 2^14 and 2^15: half precision
+// then reaches 2^-39 below it before l loses bits.  h h' and the two smaller products are summed apart, each 16 columns an instruction, so a sum is rounded a
+// quarter as often as with the float instruction (4 columns each): 2-norm of the error over the result's, normal rows against weights of 0.02,
+// K = 768 / 1,280 / 5,120, 1.9e-7 / 2.4e-7 / 4.6e-7 against 5.0e-7 / 6.4e-7 / 1.3e-6; largest error over the sum of magnitudes, in 2^-24, 1.4 to 3.1 against
+// 3.5 to 8.9 (K from 512 to 6,400, 65 to 4,000 rows).  At K = 16 the cut's own error shows (8.8e-8 against 7.4e-8), hence CUT_FROM_K.
+//
+// cut_rows_kernel finds the exponents and lays the rows out cut, a row's octet of columns as 16 bytes of h and 16 of l where its 32
+// bytes were, so that a tile copies both operands alike; the features' exponents are found when weights are laid out.  The weights, which would
+// take as much memory again, are cut in registers, 16 columns ahead of their products (24 vector instructions for 8 columns of 32 features, which
+// fit between a wave's 12 products); six products of three bfloat16 numbers each, exact without exponents, took 106 us instead of 68
+// for 1,050 x 5,120 x 1,280.
+//
+// What bounds it: at 2,048 rows and more the power (with zeros instead of numbers 4,096 x 4,096 x 1,280 takes three quarters of the time), below
+// the tiles' number and what a CU gets out of the L2s.  us, rows x features x K, with the launch that cuts and with the float instruction's
+// tiles: 300 x 3,840 x 1,280 31.7 (37.2), 1,050 x 3,840 x 1,280 56 (93), 1,050 x 5,120 x 1,280 68 (114), 1,050 x 1,280 x 5,120 in parts 78 (111), 2,048 x 6,400 x
+// 1,600 167 (316: 133 -> 252 TFLOP/s).  Where blocks are few the launch ahead is not made up for: 200 x 1,280 x 1,280 15.5 (13.3), 1,050 x 768 x 768
+// 20.2 (18.8); `price` draws the line.
+//
+// Four waves a block, two by two, each with TM x TN tiles of 32 x 32 outputs.
+template <int TM_, int TN_, int STAGES_, int PANEL_>
+struct CutShape {
+  static constexpr int TM = TM_, TN = TN_, STAGES = STAGES_, PANEL = PANEL_, WAVES = 4, THREADS = 256, STEP = 32;
+  static constexpr int BM = 2 * TM * 32, BN = 2 * TN * 32;
+  static constexpr int PA = BM / 8 / WAVES, PB = BN / 8 / WAVES, COPIES = PA + PB;  // copies of eight rows a wave and step
+  static constexpr int STAGE_BYTES = (BM + BN) * STEP * 4;
+};
+using CutTile128 = CutShape<2, 2, 2, 8>;
+using CutTile64x128 = CutShape<1, 2, 3, 8>;
+using CutTile64 = CutShape<1, 1, 3, 8>;
+
+// Columns from which operands may be cut.
+#define CUT_FROM_K 256
+
+typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
+
+// Two floats, already scaled, as two half-precision numbers each: the nearest one and what it leaves.
+__device__ __forceinline__ void cut_pair(float y0, float y1, uint32_t& high, uint32_t& low) {
+  const f16x2_t h = __builtin_convertvector((hw_f32x2_t{y0, y1}), f16x2_t);
+  const f16x2_t l = __builtin_convertvector((hw_f32x2_t{__builtin_fmaf((float)h.x, -1.f, y0), __builtin_fmaf((float)h.y, -1.f, y1)}), f16x2_t);
+  high = __builtin_bit_cast(uint32_t, h), low = __builtin_bit_cast(uint32_t, l);
+}
+struct Cut {
+  u32x4_t high, low;  // eight halves each
+};
+__device__ __forceinline__ Cut cut(f32x4_t a, f32x4_t b, float scale) {
+  a *= scale, b *= scale;
+  uint32_t h[4], l[4];
+  cut_pair(a.x, a.y, h[0], l[0]), cut_pair(a.z, a.w, h[1], l[1]);
+  cut_pair(b.x, b.y, h[2], l[2]), cut_pair(b.z, b.w, h[3], l[3]);
+  return Cut{u32x4_t{h[0], h[1], h[2], h[3]}, u32x4_t{l[0], l[1], l[2], l[3]}};
+}
+__device__ __forceinline__ f32x16_t mfma(u32x4_t a, u32x4_t b, f32x16_t c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
+}
+__device__ __forceinline__ bool finite(float v) { return (__float_as_uint(v) & 0x7f800000u) != 0x7f800000u; }
+__device__ __forceinline__ float power_of_2(int e) { return __uint_as_float((uint32_t)(e + 127) << 23); }
+
+// Ahead of the products: the rows' greatest values, whose exponents say what a row is scaled by (so that its greatest
+// value lies from 2^14 up to 2^15), and A's rows scaled and cut.  A wave a row: first A's, then W's.  A cut row has the place of the
+// row itself: where eight floats were lie eight high halves and eight low ones, up to whole steps of 32 columns.
+struct CutArgs {
+  const float* A;
+  const float* W;
+  int M, N, K, lda, ldw, ldc;
+  u32x4_t* cut;
+  int* exponents;  // [M], then [N]
+};
+__global__ __launch_bounds__(256) void cut_rows_kernel(CutArgs p) {
+  const int row = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+  if (row >= p.M + p.N) return;
+  const bool is_a = row < p.M;
+  const float* from = is_a ? p.A + (size_t)row * p.lda : p.W + (size_t)(row - p.M) * p.ldw;
+  constexpr int AHEAD = 6;
+  uint32_t most = 0;
+  for (int k0 = lane * 4; k0 < p.K; k0 += 256 * AHEAD) {
+    u32x4_t v[AHEAD];
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) v[i] = *(const u32x4_t*)(from + min(k0 + 256 * i, p.K - 4));  // (again the last ones: no other maximum)
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i)
+      most = max(max(max(most, v[i].x & 0x7fffffffu), max(v[i].y & 0x7fffffffu, v[i].z & 0x7fffffffu)), v[i].w & 0x7fffffffu);
+  }
+  // (without their signs floats are ordered as integers are, infinities and NaN behind all others)
+#pragma unroll
+  for (int d = 32; d; d >>= 1) most = max(most, (uint32_t)__shfl_xor((int)most, d, 64));
+  const int e = (int)(most >> 23);
+  const int up = most == 0 || e == 255 ? 0 : min(14 + 127 - e, 126);
+  if (lane == 0) p.exponents[row] = up;
+  if (!is_a) return;
+  const float scale = power_of_2(up);
+  u32x4_t* to = p.cut + (size_t)row * (p.ldc / 4);
+  for (int k = lane * 8; k < p.ldc; k += 512) {
+    f32x4_t a = {0.f, 0.f, 0.f, 0.f}, b = a;
+    if (k < p.K) a = *(const f32x4_t*)(from + k);
+    if (k + 4 < p.K) b = *(const f32x4_t*)(from + k + 4);
+    const Cut c = cut(a, b, scale);
+    to[k / 4] = c.high, to[k / 4 + 1] = c.low;
+  }
+}
+
+template <typename S>
+__global__ __launch_bounds__(S::THREADS, 2) void gemm_f32_cut_kernel(GemmArgs p) {
+  constexpr int BM = S::BM, BN = S::BN, TM = S::TM, TN = S::TN, PA = S::PA, PB = S::PB, STAGES = S::STAGES;
+  __shared__ __attribute__((aligned(1024))) float smem[STAGES * S::STAGE_BYTES / 4];
+  int tm, tn;
+  if (!tile_of_block<S::PANEL>((p.M + BM - 1) / BM, (p.N + BN - 1) / BN, tm, tn)) return;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int x = lane & 31, hi = lane >> 5;
+  const int wm = wave >> 1, wn = wave & 1;
+  const int m0 = tm * BM, n0 = tn * BN;
+  const int k_lo = blockIdx.y * p.per_split * 64, k_end = min(p.K, k_lo + p.per_split * 64);
+  const int n_steps = (k_end - k_lo + S::STEP - 1) / S::STEP;
+
+  // the block's rows and features, each a buffer of its own from the block's first on: what lies beyond the matrix lies
+  // beyond the buffer, or is sent there
+  const int a_rows = min(BM, p.M - m0), b_rows = min(BN, p.N - n0);
+  const i32x4_t a_buf = copy_buffer(p.cut + (size_t)m0 * p.ldc, (size_t)a_rows * p.ldc * 4);
+  const i32x4_t b_buf = copy_buffer(p.W + (size_t)n0 * p.ldw, ((size_t)(b_rows - 1) * p.ldw + p.K) * 4);
+  const int row8 = lane >> 3;
+  auto piece_of = [&](int copy) __attribute__((always_inline)) { return (lane & 7) ^ ((copy & 1) * 4 + (row8 >> 1)); };
+  uint32_t a_from[PA], b_from[PB];
+#pragma unroll
+  for (int i = 0; i < PA; ++i) {
+    const int c = wave * PA + i, row = c * 8 + row8;
+    a_from[i] = row < a_rows ? (uint32_t)(((size_t)row * p.ldc + piece_of(c) * 4) * 4) : COPY_NOTHING;
+  }
+#pragma unroll
+  for (int i = 0; i < PB; ++i) {
+    const int c = wave * PB + i, row = c * 8 + row8;
+    b_from[i] = row < b_rows ? (uint32_t)(((size_t)row * p.ldw + piece_of(c) * 4) * 4) : COPY_NOTHING;
+  }
+  const uint32_t ring = lds_address(smem);
+  // (steps beyond the last are asked for too, as nothing: the waits then count the same copies in every round)
+  auto ask = [&](int t, int slot) __attribute__((always_inline)) {
+    const int k = k_lo + t * S::STEP, left = t < n_steps ? k_end - k : 0;
+    const uint32_t k4 = t < n_steps ? (uint32_t)k * 4u : 0u, at = ring + (uint32_t)slot * S::STAGE_BYTES;
+#pragma unroll
+    for (int i = 0; i < PA; ++i)
+      copy16_to_lds(a_buf, left > 0 ? a_from[i] : COPY_NOTHING, k4, at + (wave * PA + i) * 1024);
+#pragma unroll
+    for (int i = 0; i < PB; ++i)
+      copy16_to_lds(b_buf, piece_of(wave * PB + i) * 4 < left ? b_from[i] : COPY_NOTHING, k4, at + BM * 128 + (wave * PB + i) * 1024);
+  };
+
+  // the features' scales
+  float scale[TN];
+#pragma unroll
+  for (int j = 0; j < TN; ++j) scale[j] = power_of_2(p.w_exponents[min(n0 + (wn * TN + j) * 32 + x, p.N - 1)]);
+
+  // the products of the high parts, and those with a low part
+  f32x16_t acc[TM][TN], low[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = low[i][j][r] = 0.f;
+  const char* const a_row = (const char*)smem + (wm * TM * 32 + x) * 128;
+  const char* const b_row = (const char*)smem + BM * 128 + (wn * TN * 32 + x) * 128;
+  // the operands of 16 columns go to registers that many columns ahead of their products, also across the barrier
+  Cut a[2][TM], b[2][TN];
+  f32x4_t raw[TN][2];
+  auto read_half = [&](int h, int slot) __attribute__((always_inline)) {
+    const int s0 = ((4 * h + 2 * hi) ^ ((x >> 1) & 7)) * 16, s1 = s0 ^ 16;
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      raw[j][0] = *(const f32x4_t*)(b_row + slot * S::STAGE_BYTES + j * 4096 + s0);
+      raw[j][1] = *(const f32x4_t*)(b_row + slot * S::STAGE_BYTES + j * 4096 + s1);
+    }
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      a[h][i].high = *(const u32x4_t*)(a_row + slot * S::STAGE_BYTES + i * 4096 + s0);
+      a[h][i].low = *(const u32x4_t*)(a_row + slot * S::STAGE_BYTES + i * 4096 + s1);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto cut_half = [&](int h) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < TN; ++j) b[h][j] = cut(raw[j][0], raw[j][1], scale[j]);
+  };
+  auto multiply = [&](int h) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) acc[i][j] = mfma(b[h][j].high, a[h][i].high, acc[i][j]);
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) low[i][j] = mfma(b[h][j].high, a[h][i].low, low[i][j]);
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j) low[i][j] = mfma(b[h][j].low, a[h][i].high, low[i][j]);
+  };
+#pragma unroll
+  for (int t = 0; t < STAGES - 1; ++t) ask(t, t);
+  int slot = 0;
+  for (int t = 0; t < n_steps; ++t) {
+    copies_arrived<(STAGES - 2) * S::COPIES>();
+    ring_barrier();  // step t is whole, and nobody reads the slot of step t - 1 any more
+    read_half(0, slot);
+    ask(t + STAGES - 1, slot == 0 ? STAGES - 1 : slot - 1);
+    if (t > 0) multiply(1);
+    cut_half(0);
+    __builtin_amdgcn_sched_barrier(0);
+    read_half(1, slot);
+    multiply(0);
+    cut_half(1);
+    __builtin_amdgcn_sched_barrier(0);
+    slot = slot == STAGES - 1 ? 0 : slot + 1;
+  }
+  multiply(1);
+  copies_arrived<0>();  // (what was asked for beyond the end)
+
+  // A row's sums leave their scales behind.  What is not finite is computed again with the 32-bit instructions, out of the operands
+  // themselves: an infinity's parts would give NaN, and the sums' own infinities and NaN come out as those instructions have them.
+  bool whole = true;
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      acc[i][j] += low[i][j];
+#pragma unroll
+      for (int r = 0; r < 16; ++r) whole = whole && finite(acc[i][j][r]);
+    }
+  const bool again = __any(!whole);
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+    const int m = min(m0 + (wm * TM + i) * 32 + x, p.M - 1);
+    const int down = -p.a_exponents[m];
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      const int nt = n0 + (wn * TN + j) * 32;
+      f32x16_t sum;
+      if (again) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) sum[r] = 0.f;
+        const float* ap = p.A + (size_t)m * p.lda;
+        const float* wp = p.W + (size_t)min(nt + x, p.N - 1) * p.ldw;
+        for (int k = k_lo + hi; k < k_end; k += 2) sum = __builtin_amdgcn_mfma_f32_32x32x2f32(wp[k], ap[k], sum, 0, 0, 0);
+      }
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const float v = ldexpf(acc[i][j][r], down - p.w_exponents[min(nt + 8 * (r >> 2) + 4 * hi + (r & 3), p.N - 1)]);
+        acc[i][j][r] = again && !finite(acc[i][j][r]) ? sum[r] : v;
+      }
+    }
+  }
+
+  // Epilogue.  Accumulator r of tile (i, j): row 32 * i + x, feature 32 * j + 8 * (r / 4) + 4 * hi + r % 4.  What is read (bias, the
+  // residual stream to add to) is read for a tile before anything of it is stored: a load that comes after a
+  // store to memory it might alias waits for it.
+  const bool parts = p.n_splits > 1;
+  float* const out = parts ? p.ws + (size_t)blockIdx.y * p.ws_rows * p.N : p.out;
+  const int ldo = parts ? p.N : p.ldo;
+  const bool vec = ldo % 4 == 0 && ((uintptr_t)out & 15) == 0;
+  // (through to memory, as far as a buffer reaches: 1,050 x 1,280 x 5,120 in three parts 114.8 -> 113.5 us, two parts of
+  // 1,280 columns 34.7 -> 33.9, the wide ones level)
+  const __amdgpu_buffer_rsrc_t out_buf = through_buffer(out, ((size_t)(p.M - 1) * ldo + p.N) * 4);
+#pragma unroll
+  for (int i = 0; i < TM; ++i) {
+    const int m = m0 + (wm * TM + i) * 32 + x;
+    if (m >= p.M) continue;
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      f32x4_t v[4];
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int n = n0 + (wn * TN + j) * 32 + 8 * g + 4 * hi;
+        v[g] = f32x4_t{acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
+        if (parts) continue;
+        const bool add = p.flags & FLAG_ACCUMULATE, whole = vec && n + 4 <= p.N;
+        f32x4_t old = {0.f, 0.f, 0.f, 0.f};
+        if (add && whole) old = *(const f32x4_t*)(p.out + (size_t)m * ldo + n);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int nc = min(n + r, p.N - 1);
+          const float bias = p.bias ? p.bias[nc] : 0.f;
+          if (add)
+            v[g][r] = (whole ? old[r] : p.out[(size_t)m * ldo + nc]) + (v[g][r] + bias);
+          else
+            v[g][r] = activate<false>(p.flags, v[g][r] + bias);
+        }
+      }
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int n = n0 + (wn * TN + j) * 32 + 8 * g + 4 * hi;
+        if (vec && n + 4 <= p.N) {
+          if (p.through)
+            store_through(out_buf, (uint32_t)(((size_t)m * ldo + n) * 4), __builtin_bit_cast(u32x4_t, v[g]));
+          else
+            *(f32x4_t*)(out + (size_t)m * ldo + n) = v[g];
+        } else {
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (n + r < p.N) out[(size_t)m * ldo + n + r] = v[g][r];
+        }
+      }
+    }
+  }
+}
+
 #define SKF_WAVES_FEW 8   // waves a block where the blocks are fewer than the compute units
 #define SKF_WAVES_MANY 4  // and where every unit has a block or more (8: 12.1 us instead of 10.6 for 4,800 features of 1,600)
 #define SKF_MAX_WAVES 8
@@ -329,29 +643,43 @@ __global__ __launch_bounds__(64 * SKF_MAX_WAVES) void gemm_f32_skinny_kernel(Gem
 
 DEFINE_LAST_ERROR(mlxlm_last_error)
 
-// What a tile shape costs in microseconds: its products at the speed of a CU's matrix units (2.5e-4 an output and 64
-// columns, 8 % more in the smallest tiles, which read most, 3 % more in the largest; a block alone on its CU, one wave a
+// What a tile shape costs in microseconds.  The 32-bit instructions' tiles: their products at the speed of a CU's matrix units (2.5e-4 an
+// output and 64 columns, 8 % more in the smallest tiles, which read most, 3 % more in the largest; a block alone on its CU, one wave a
 // SIMD, a fifth more), blocks that share a CU one after another, and a fixed part for the first step's way and the
 // epilogue.  Against the times of 11 numbers of rows from 80 to 2,048 and ten matrices of widths 768 to 1,600, each with
 // K in 1 to 8 parts, the choice is within 0.7 % of the best on average and 7 % at worst (1.7 % and 13 % with every tile
 // at the same rate).
+// Tiles of cut operands: `base` once, `tile` for each round of blocks that share a CU (`per_cu` of them), each 64 columns of K
+// as many blocks as then share the CU (`chunk[0]` one, `chunk[1]` two, `chunk[2]` three), and the launch ahead that cuts the rows. Fitted to the times of
+// as many rows from 65 on and 15 matrices of widths 768 to 1,600.
 struct F32Price {
   int variant, bm, bn;
-  double rate;
+  double rate;  // (0: cut operands)
+  int per_cu;
+  double base, tile, chunk[3];
 };
-static const F32Price F32_PRICES[] = {{1, F32Tile64x128::BM, F32Tile64x128::BN, 1.03},
-                                      {2, F32Tile64::BM, F32Tile64::BN, 1.0},
-                                      {4, F32Tile32x64::BM, F32Tile32x64::BN, 1.08}};
+static const F32Price F32_PRICES[] = {{1, F32Tile64x128::BM, F32Tile64x128::BN, 1.03, 0, 0, 0, {}},
+                                      {2, F32Tile64::BM, F32Tile64::BN, 1.0, 0, 0, 0, {}},
+                                      {4, F32Tile32x64::BM, F32Tile32x64::BN, 1.08, 0, 0, 0, {}},
+                                      {5, CutTile128::BM, CutTile128::BN, 0, 2, 0.0, 13.2, {1.53, 2.94, 0.0}},
+                                      {6, CutTile64x128::BM, CutTile64x128::BN, 0, 2, 5.0, 6.3, {1.03, 1.91, 0.0}},
+                                      {7, CutTile64::BM, CutTile64::BN, 0, 3, 5.7, 4.3, {0.69, 1.11, 1.6}}};
+static inline bool is_cut(int variant) { return variant >= 5 && variant <= 7; }
 static double price(const F32Price& s, int M, int N, int K, int n_splits) {
   const long tiles = (long)((M + s.bm - 1) / s.bm) * ((N + s.bn - 1) / s.bn);
-  const long n = (tiles * n_splits + n_compute_units() - 1) / n_compute_units();
-  const int chunks = ((K + 63) / 64 + n_splits - 1) / n_splits;
-  return 4.0 + (n == 1 ? 1.2 : 1.0) * n * chunks * (2.5e-4 * s.rate * s.bm * s.bn);
+  const int cus = n_compute_units(), chunks = ((K + 63) / 64 + n_splits - 1) / n_splits;
+  // the busiest CU (of a die's run of tiles where operands are cut)
+  const long n = is_cut(s.variant) ? ((tiles + N_DIES - 1) / N_DIES * n_splits + cus / N_DIES - 1) / (cus / N_DIES) : (tiles * n_splits + cus - 1) / cus;
+  if (!is_cut(s.variant)) return 4.0 + (n == 1 ? 1.2 : 1.0) * n * chunks * (2.5e-4 * s.rate * s.bm * s.bn);
+  const long full = n / s.per_cu, left = n % s.per_cu;
+  return s.base + s.tile * (full + (left ? 1 : 0)) + chunks * (full * s.chunk[s.per_cu - 1] + (left ? s.chunk[left - 1] : 0.0)) +
+         2.3e-6 * M * K;
 }
 static int cheapest_shape(int M, int N, int K, int n_splits, double* us) {
   int variant = 0;
   for (const F32Price& s : F32_PRICES) {
-    const double t = price(s, M, N, K, n_splits);
+    if (is_cut(s.variant) && K < CUT_FROM_K) continue;
+    const double t = price(s, M, N, K, n_splits) * (is_cut(s.variant) ? 1.04 : 1.0);  // (to be ahead for certain)
     if (!variant || t < *us) variant = s.variant, *us = t;
   }
   return variant;
@@ -395,11 +723,20 @@ static void launch_tiles(const GemmArgs& p, hipStream_t stream) {
   dim3 grid((p.N + S::BN - 1) / S::BN, (p.M + S::BM - 1) / S::BM, p.n_splits), block(S::THREADS);
   hipLaunchKernelGGL(gemm_f32_tile_kernel<S>, grid, block, 0, stream, p);
 }
+template <typename S>
+static void launch_cut_tiles(const GemmArgs& p, hipStream_t stream) {
+  const long tiles = (long)((p.M + S::BM - 1) / S::BM) * ((p.N + S::BN - 1) / S::BN);
+  dim3 grid((unsigned)((tiles + N_DIES - 1) / N_DIES * N_DIES), p.n_splits), block(S::THREADS);  // a run of tiles for each die
+  hipLaunchKernelGGL(gemm_f32_cut_kernel<S>, grid, block, 0, stream, p);
+}
 
 static void launch(const GemmArgs& p, int variant, hipStream_t stream) {
   if (variant == 1) return launch_tiles<F32Tile64x128>(p, stream);
   if (variant == 2) return launch_tiles<F32Tile64>(p, stream);
   if (variant == 4) return launch_tiles<F32Tile32x64>(p, stream);
+  if (variant == 5) return launch_cut_tiles<CutTile128>(p, stream);
+  if (variant == 6) return launch_cut_tiles<CutTile64x128>(p, stream);
+  if (variant == 7) return launch_cut_tiles<CutTile64>(p, stream);
   // where the blocks are fewer than the compute units, more waves each
   const int blocks = (p.N + 15) / 16;
   const int waves = blocks * p.n_splits < n_compute_units() ? SKF_WAVES_FEW : SKF_WAVES_MANY;
@@ -420,15 +757,42 @@ static void launch(const GemmArgs& p, int variant, hipStream_t stream) {
 // row, each at a place of its own, cost more than the launch that writes whole heads, 15,002 -> 15,122 us for 1,050 rows.)
 extern "C" int gemm_f32_scatters(int M, int n_splits) { return M >= 1 && M <= SKF_MAX_ROWS && n_splits == 1; }
 
+static inline int cut_stride(int K) { return (K + 31) / 32 * 32; }
+static inline bool fits_tiles(int lda, int ldw, int K, bool cut) {
+  return (cut ? fits_copy_buffer((size_t)128 * cut_stride(K) * 4) : fits_copy_buffer(((size_t)127 * lda + K) * 4)) &&
+         fits_copy_buffer(((size_t)127 * ldw + K) * 4);
+}
+static int choose(int M, int N, int K, int variant, int n_splits) {
+  double us = 0.0;
+  return variant != 0 ? variant : M <= SKF_MAX_ROWS ? 3 : cheapest_shape(M, N, K, n_splits, &us);
+}
+// Floats of memory that gemm_f32_scatter needs for a product of these sizes: its rows cut, and an exponent a row and feature (0: tiles of
+// cut operands don't take it).
+extern "C" size_t gemm_f32_room(int M, int N, int K, int variant, int n_splits) {
+  return M > 0 && is_cut(choose(M, N, K, variant, n_splits)) ? (size_t)M * cut_stride(K) + (size_t)M + N : 0;
+}
+
+static void cut_rows(const CutArgs& c, hipStream_t stream) {
+  hipLaunchKernelGGL(cut_rows_kernel, dim3((unsigned)(((long)c.M + c.N + 3) / 4)), dim3(256), 0, stream, c);
+}
+// What the rows of W are scaled by, powers of two: made once for weights that are kept.
+extern "C" int gemm_f32_exponents(int* out, const float* W, int N, int K, int ldw, hipStream_t stream) {
+  if (N <= 0 || K <= 0 || K % 4 != 0 || ldw % 4 != 0 || ldw < K) FAIL("gemm_f32: bad sizes N=%d K=%d ldw=%d", N, K, ldw);
+  if (!out || !W || ((uintptr_t)W & 15)) FAIL("gemm_f32: W must be 16-byte aligned");
+  cut_rows(CutArgs{nullptr, W, 0, N, K, 0, ldw, 0, nullptr, out}, stream);
+  CHECK_LAUNCH("gemm_f32_exponents");
+  return 0;
+}
+
 // variant: 0 = choose, 1 = tiles of 64 x 128, 2 = of 64 x 64, 4 = of 32 x 64, 3 = the kernel for up to
-// 64 rows.  n_splits > 1: K in that many parts, whose sums go to ws[part][M][N] (ws_floats floats at least) for sum_partials of gemm_bf16_decode.hip to add up
+// 64 rows, 5 = tiles of cut operands of 128 x 128, 6 = of 64 x 128, 7 = of 64 x 64.  n_splits > 1: K in that many parts, whose sums go to ws[part][M][N] (ws_floats floats at least) for sum_partials of gemm_bf16_decode.hip to add up
 // and finish; out is not written then.
 // k_pages: the features from q_width on go to the pages of the key/value cache too (mlx_lm/models/cache.py:352-354).
 extern "C" int gemm_f32_scatter(void* out, const void* A, const void* W, const float* bias, int M, int N,
                                 int K, int lda, int ldw, int ldo, int flags, int variant, int n_splits, float* ws,
                                 size_t ws_floats, void* k_pages, void* v_pages, size_t page_stride, const int* block_table,
                                 int max_blocks, const int* token_req, const int* positions, int q_width, int kv_width,
-                                int head_dim, int page_size, hipStream_t stream) {
+                                int head_dim, int page_size, const int* w_exponents, float* room, size_t room_floats, hipStream_t stream) {
   GemmArgs p = {};
   p.A = (const float*)A;
   p.W = (const float*)W;
@@ -468,15 +832,26 @@ extern "C" int gemm_f32_scatter(void* out, const void* A, const void* W, const f
     p.block_table = block_table, p.max_blocks = max_blocks, p.token_req = token_req, p.positions = positions;
     p.q_width = q_width, p.kv_width = kv_width, p.head_dim = head_dim, p.page_size = page_size;
   }
-  double us = 0.0;
-  if (variant == 0) variant = M <= SKF_MAX_ROWS ? 3 : cheapest_shape(M, N, K, n_splits, &us);
+  variant = choose(M, N, K, variant, n_splits);
   if (variant != 3 && p.per_split * (n_splits - 1) * SKF_CHUNK >= K) FAIL("gemm_f32: %d parts of K=%d leave one empty", n_splits, K);
   if (variant == 3 && M > SKF_MAX_ROWS)
     FAIL("gemm_f32: the kernel for few rows takes at most %d, got %d", SKF_MAX_ROWS, M);
-  if (variant < 1 || variant > 4) FAIL("gemm_f32: unknown variant %d", variant);
+  if (variant < 1 || variant > 7) FAIL("gemm_f32: unknown variant %d", variant);
+  const size_t room_wanted = gemm_f32_room(M, N, K, variant, n_splits);
   // Rows some 8 million floats apart or more are beyond the 32-bit offsets of a tile's copies: the kernel for few
   // rows, which has pointers, takes them 64 at a time.  More tiles of rows than a grid holds go in several launches.
-  if (!(fits_copy_buffer(((size_t)127 * lda + K) * 4) && fits_copy_buffer(((size_t)127 * ldw + K) * 4))) variant = 3;
+  if (!fits_tiles(lda, ldw, K, is_cut(variant))) variant = 3;
+  if (is_cut(variant)) {
+    if (!room || ((uintptr_t)room & 15) || room_floats < room_wanted)
+      FAIL("gemm_f32: tiles of cut operands need %zu floats of aligned memory", room_wanted);
+    int* const exponents = (int*)(room + (size_t)M * cut_stride(K));
+    p.cut = room, p.ldc = cut_stride(K), p.a_exponents = exponents, p.w_exponents = w_exponents ? w_exponents : exponents + M;
+    cut_rows(CutArgs{p.A, p.W, M, w_exponents ? 0 : N, K, lda, ldw, p.ldc, (u32x4_t*)room, exponents}, stream);
+    p.through = fits_through_buffer((size_t)M * (n_splits > 1 ? N : ldo) * 4);
+    launch(p, variant, stream);
+    CHECK_LAUNCH("gemm_f32");
+    return 0;
+  }
   const int most = variant == 3 ? SKF_MAX_ROWS : 65535 * (variant == 4 ? F32Tile32x64::BM : F32Tile64::BM);
   static_assert(F32Tile64x128::BM == F32Tile64::BM, "both tiles' rows");
   for (int left = M; left > 0; left -= most) {
@@ -488,11 +863,4 @@ extern "C" int gemm_f32_scatter(void* out, const void* A, const void* W, const f
   }
   CHECK_LAUNCH("gemm_f32");
   return 0;
-}
-
-extern "C" int gemm_f32(void* out, const void* A, const void* W, const float* bias, int M, int N,
-                        int K, int lda, int ldw, int ldo, int flags, int variant, int n_splits, float* ws,
-                        size_t ws_floats, hipStream_t stream) {
-  return gemm_f32_scatter(out, A, W, bias, M, N, K, lda, ldw, ldo, flags, variant, n_splits, ws, ws_floats, nullptr, nullptr, 0, nullptr, 0,
-                          nullptr, nullptr, 0, 0, 0, 0, stream);
 }

@@ -32,6 +32,7 @@ GEMM_KV = 8
 # Up to this many rows a bfloat16 product goes to the decode kernels, which stream the weights
 # once and fuse the norm and the cache scatter; more rows go to the tile kernels.
 DECODE_MAX_ROWS = 16
+F32_FEW_ROWS = 64  # rows that the 32-bit product's streaming kernel takes
 
 
 # torch's current stream as a raw handle.  torch.cuda.current_stream() builds a Stream object
@@ -298,7 +299,7 @@ def weight_struct(w):
         return w.c
     ld = _rows2d(w, "w")
     w.dtype in DT or _fail(f"weight dtype {w.dtype} not supported")
-    return native.EngWeight(w.data_ptr(), None, w.shape[0], w.shape[1], ld, DT[w.dtype], 0, 0, 0)
+    return native.EngWeight(w.data_ptr(), None, w.shape[0], w.shape[1], ld, DT[w.dtype], 0, 0, 0, native.ptr(getattr(w, "row_exponents", None)))
 
 
 def read_ahead_pays(w, n_rows, with_norm=False):
@@ -313,10 +314,27 @@ def read_ahead_pays(w, n_rows, with_norm=False):
 
 def for_decode(w, keep_rows=False):
     """``w`` in the packed order where the product kernels can use it (bfloat16 on the GPU),
-    instead of the row-major matrix unless ``keep_rows``; anything else is returned as it is."""
+    instead of the row-major matrix unless ``keep_rows``; float32 rows with their ``row_exponents``; anything
+    else is returned as it is."""
     if isinstance(w, torch.Tensor) and w.is_cuda and w.dtype == torch.bfloat16 and w.dim() == 2:
         return PackedWeight(w, keep_rows=keep_rows)
+    if isinstance(w, torch.Tensor) and w.is_cuda and w.dtype == torch.float32 and w.dim() == 2 and _reads_by_fours(w):
+        w = w.detach()
+        w.row_exponents = row_exponents(w)
     return w
+
+
+def _reads_by_fours(w):
+    return w.numel() > 0 and w.stride(1) == 1 and w.shape[1] % 4 == 0 and w.stride(0) % 4 == 0 and w.data_ptr() % 16 == 0
+
+
+def row_exponents(w):
+    """What the tiles of the 32-bit product scale each row of ``w`` ``[N, K]`` by, as powers of two (csrc/gemm_f32.hip): found once
+    where weights are laid out, ahead of every product for other tensors."""
+    lib = build.load("gemm_f32")
+    out = torch.empty(w.shape[0], dtype=torch.int32, device=w.device)
+    build.check(lib, lib.gemm_f32_exponents(_ptr(out), _ptr(w), w.shape[0], w.shape[1], _rows2d(w, "w"), _stream()), "gemm_f32_exponents")
+    return out
 
 
 _SPLIT_WS = {}
@@ -539,6 +557,13 @@ def linear(out, a, w, bias=None, gelu=False, accumulate=False, variant=0, scatte
         _fail(f"linear: unknown activation {activation!r} (known: {sorted(k for k in ACTIVATIONS if k)})")
     code = ACTIVATIONS[activation] or int(bool(gelu))
     call.gelu, call.accumulate, call.variant, call.splits = code, int(accumulate), int(variant), int(splits or 0)
+    if call.w.dtype == DT[torch.float32] and not ctx.scratch and (a.shape[0] > F32_FEW_ROWS or variant >= 5):
+        # outside a step there is no scratch memory for the rows that the tiles cut (a context of the call's own: others, on other
+        # streams, share the bare one)
+        room = torch.empty(4 * (a.shape[0] * ((K + 31) // 32 * 32 + 1) + N) + 4096, dtype=torch.uint8, device=out.device)
+        scratch = native.EngScratch(room.data_ptr(), room.numel(), 0, 0, 1, 0)
+        ctx = native.EngCtx.from_buffer_copy(ctx)
+        ctx.scratch = ctypes.pointer(scratch)
     rc = L.eng_linear(ctypes.byref(ctx), ctypes.byref(call), ctypes.byref(pending.c) if pending is not None else None)
     native.check(rc, "linear")
     return out

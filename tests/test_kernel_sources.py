@@ -35,4 +35,4 @@ def test_copies_into_lds_are_waited_for_before_a_wave_ends():
                 seen.append(name)
                 last = body.rindex("ask(")
                 assert "copies_arrived<0>()" in body[last:], (os.path.basename(path), name)
-    assert {"gemm_bf16_tile_kernel", "gemm_f32_tile_kernel"} <= set(seen)
+    assert {"gemm_bf16_tile_kernel", "gemm_f32_tile_kernel", "gemm_f32_cut_kernel"} <= set(seen)

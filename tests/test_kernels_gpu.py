@@ -131,6 +131,71 @@ def test_gemm_f32_tiles_at_the_ring_s_edges(M, N, K):
                 assert (wide[:, N:] == 0.5).all()
 
 
+def _cut_tolerance(a, w, K):
+    """K roundings of a partial sum, and a cut's: an operand's last bit each (2^-23), the low parts' product (2^-22), half precision's
+    least steps below the rows' greatest values (2^-39)."""
+    mags = (a.double().abs() @ w.double().abs().t().contiguous()).cpu()
+    least = a.double().abs().amax(1)[:, None].cpu() * w.double().abs().amax(1)[None, :].cpu() * K * 2.0**-38
+    return (K + 10) * 2.0**-24 * mags + least
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 1, 4), (65, 60, 32), (64, 129, 68), (127, 128, 100), (129, 257, 520), (300, 70, 1284)])
+def test_gemm_f32_cut_operands(M, N, K):
+    """Tiles of cut operands at the edges of tiles, steps of 32 columns and rows of eight: rows and features from 1e-30 to 1e30, columns that
+    differ by 2^12, NaN around the operands, K whole and in parts, exponents known ahead or found by the call (the same bits)."""
+    k = _k()
+    a = torch.full((M + 40, K + 12), float("nan"), device=DEV)[:M, :K]
+    w = torch.full((N + 40, K + 12), float("nan"), device=DEV)[:N, :K]
+    steep = torch.logspace(0, -12, K, base=2.0, device=DEV)
+    a.copy_(_rand((M, K), torch.float32, 10) * torch.logspace(-30, 30, M, device=DEV)[:, None] * steep)
+    w.copy_(_rand((N, K), torch.float32, 11) * torch.logspace(3, -3, N, device=DEV)[:, None] * steep.flip(0))
+    a[0, 0] = 0.0
+    if M > 2:
+        a[1] = 0.0
+    known = k.for_decode(w)
+    ref, tol = (a.double() @ w.double().t().contiguous()).cpu(), _cut_tolerance(a, w, K)
+    for variant in (5, 6, 7):
+        for splits in [None] + [s for s in (2, 3) if s <= (K + 63) // 64]:
+            wide = torch.full((M, N + 3), 0.5, device=DEV)
+            k.linear(wide[:, :N], a, w, variant=variant, splits=splits)
+            assert ((wide[:, :N].double().cpu() - ref).abs() <= tol).all(), (variant, splits)
+            assert (wide[:, N:] == 0.5).all()
+            again = torch.empty(M, N, device=DEV)
+            k.linear(again, a, known, variant=variant, splits=splits)
+            assert torch.equal(again, wide[:, :N]), (variant, splits)
+
+
+def test_gemm_f32_cut_operands_that_are_not_finite():
+    """Infinities and NaN come out as sums of products have them, sums beyond the greatest float as infinities, and what else is in
+    their tiles stays as it was, bit by bit."""
+    k = _k()
+    M, N, K = 150, 140, 288
+    a, w = _rand((M, K), torch.float32, 10), _rand((N, K), torch.float32, 11)
+    clean = {}
+    for variant in (5, 6, 7):
+        clean[variant] = torch.empty(M, N, device=DEV)
+        k.linear(clean[variant], a, w, variant=variant)
+    a[3, 17], a[40, 0], a[100, 287] = float("inf"), float("nan"), float("-inf")
+    a[70], w[33] = 3e38, w[33].abs() + 2.0
+    w[90, 5], w[91, 200] = float("inf"), float("nan")
+    # (torch's own sum in 64 bits, as a float: every product that is not finite comes from an operand above or from row 70)
+    want = (a.double().cpu() @ w.double().cpu().t()).float()
+    for variant in (5, 6, 7):
+        for splits in (None, 3):
+            out = torch.empty(M, N, device=DEV)
+            k.linear(out, a, w, variant=variant, splits=splits)
+            got = out.cpu()
+            rows, cols = [i for i in range(M) if i not in (3, 40, 70, 100)], [j for j in range(N) if j not in (33, 90, 91)]
+            if splits is None:
+                assert torch.equal(out[rows][:, cols], clean[variant][rows][:, cols]), variant
+            for i in (3, 40, 100):
+                assert torch.equal(got[i].isnan(), want[i].isnan()) and torch.equal(got[i].isinf(), want[i].isinf()), (variant, i)
+                assert (got[i][want[i].isinf()] == want[i][want[i].isinf()]).all(), (variant, i)
+            for j in (90, 91):
+                assert torch.equal(got[rows][:, j].isnan(), want[rows][:, j].isnan()) and (got[rows][:, j][want[rows][:, j].isinf()] == want[rows][:, j][want[rows][:, j].isinf()]).all(), (variant, j)
+            assert got[70, 33].isposinf(), variant
+
+
 @pytest.mark.parametrize("M,N,far", [(70, 33, "a"), (129, 20, "a"), (70, 70, "w"), (65, 9, "a")])
 @pytest.mark.parametrize("splits", [None, 2])
 def test_gemm_f32_rows_far_apart(M, N, far, splits):
