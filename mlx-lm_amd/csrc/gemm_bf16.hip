@@ -55,6 +55,7 @@ struct GemmArgs {
   // tiles of 16 features x 64 k (1024 elements), zero padded, w_kblocks of them a feature block;
   // in a tile the 8 values k = 16 g + 8 h + 0..7 of feature f lie at ((4 h + g) * 16 + f) * 8.
   int w_packed, w_kblocks;
+  int tile_blocks;  // blocks of the grid's first dimension that have tiles: those behind them read weights ahead (read_weights)
 };
 
 // Element offset of the 16-byte piece `piece` (k = 8 piece ..) of feature row n in k-block 0.
@@ -101,36 +102,75 @@ __device__ __forceinline__ void store_out(const GemmArgs& p, int m, int n, float
 // the products taken out), so the larger the tile, the fewer bytes per product: 256 x 256 where the matrix gives a tile
 // to every CU, smaller ones where it does not; `price` below chooses.  Eight waves (but for 32 rows): two a SIMD cover each
 // other's waits for LDS; four waves of 64 x 64 were level or up to 12 % behind.
+// COPIERS: waves beside those that only copy (Tile128Fed).
 // The widest shapes have room for two k-blocks of both and what is left goes to the weights, which come from memory while
 // the rows lie in the L2s; their copies are asked for a few at a time between products (SPREAD): a wave that asks waits
 // until its copies are taken, 64 KB a k-block, and right behind the barrier all waves did so at once, the matrix units idle.  Zeros, so that
 // power does not limit, 256 x 256, a k-block: products alone 0.87 us, copies alone 0.96, both 1.28 and now 1.10; from memory, rows x features x K:
 // 2,048 x 4,800 x 1,600 37.4 -> 33.6 us, x 6,400 x 1,600 47.4 -> 43.8, 8,000 x 4,800 x 1,600 128.3 -> 124, 8,000 x 1,280 x 5,120 111 -> 104.  The
 // smaller shapes were level or up to 3 % slower with either (128 x 128 with five slots, 64 x 128 with six: what they wait for is not depth).
-template <int WAVES_M_, int WAVES_N_, int TM_, int TN_, int SLOTS_A_, int PANEL_, int WAVES_PER_SIMD_, int SLOTS_B_ = SLOTS_A_, bool SPREAD_ = false>
+template <int WAVES_M_, int WAVES_N_, int TM_, int TN_, int SLOTS_A_, int PANEL_, int WAVES_PER_SIMD_, int SLOTS_B_ = SLOTS_A_, bool SPREAD_ = false, int COPIERS_ = 0>
 struct TileShape {
+  static constexpr int COPIERS = COPIERS_;
   static constexpr int WAVES_M = WAVES_M_, WAVES_N = WAVES_N_, TM = TM_, TN = TN_, SLOTS_A = SLOTS_A_, SLOTS_B = SLOTS_B_;
   static constexpr bool SPREAD = SPREAD_;
   static constexpr int PANEL = PANEL_, WAVES_PER_SIMD = WAVES_PER_SIMD_;  // PANEL: rows of tiles that share a die's L2
-  static constexpr int WAVES = WAVES_M * WAVES_N, THREADS = 64 * WAVES;
+  static constexpr int WAVES = WAVES_M * WAVES_N, THREADS = 64 * (WAVES + COPIERS), ASKERS = COPIERS ? COPIERS : WAVES;
   static constexpr int BM = WAVES_M * TM * 32, BN = WAVES_N * TN * 32;
-  static constexpr int PA = BM / 8 / WAVES, PB = BN / 8 / WAVES;  // copies of 1 KB a wave asks for per k-block
+  static constexpr int PA = BM / 8 / ASKERS, PB = BN / 8 / ASKERS;  // copies of 1 KB a wave asks for per k-block
   static constexpr int COPIES = PA + PB;
   static constexpr int A_BYTES = BM * BK * 2, B_BYTES = BN * BK * 2, RING = SLOTS_A * A_BYTES + SLOTS_B * B_BYTES;
   // as many slots for both: a k-block's rows and weights side by side, one address for both; else a ring behind the other
   static constexpr bool ALIKE = SLOTS_A == SLOTS_B;
   static constexpr int A_STRIDE = ALIKE ? A_BYTES + B_BYTES : A_BYTES, B_STRIDE = ALIKE ? A_STRIDE : B_BYTES;
   static constexpr int B_BASE = ALIKE ? A_BYTES : SLOTS_A * A_BYTES;
-  static_assert(BM % (8 * WAVES) == 0 && BN % (8 * WAVES) == 0, "a wave copies whole kilobytes");
+  static_assert(BM % (8 * ASKERS) == 0 && BN % (8 * ASKERS) == 0, "a wave copies whole kilobytes");
   static_assert(RING <= 160 * 1024, "the rings fit a CU's LDS");
 };
 using Tile256 = TileShape<2, 4, 4, 2, 2, 4, 2, 3, true>;
 using Tile256x192 = TileShape<4, 2, 2, 3, 2, 4, 2, 4, true>;
 using Tile256x128 = TileShape<4, 2, 2, 2, 3, 4, 2, 4, true>;
 using Tile128 = TileShape<2, 4, 2, 1, 4, 8, 2>;
+// beside readers (read_weights), where what is copied comes from the L2s, four more waves that only copy: those that multiply
+// then wait for no copy to be taken (2,048 x 1,600 x 6,400 51.1 -> 47.0 us, 150 x 4,800 x 1,600 13.6 -> 12.6; without readers 0 to 5 % slower)
+using Tile128Fed = TileShape<2, 4, 2, 1, 4, 8, 3, 4, false, 4>;
 using Tile128Pair = TileShape<2, 4, 2, 1, 2, 8, 4>;  // two blocks a CU (pairs_of_blocks below)
 using Tile64x128 = TileShape<2, 4, 1, 1, 3, 8, 4>;  // two blocks a CU, as the next
 using Tile32x128 = TileShape<1, 4, 1, 1, 4, 8, 2>;
+
+// Weights read ahead by compute units that have no tile.  A compute unit gets some 25 to 40 GB/s of what its die's L2 does not hold, and
+// the k-blocks of a column of tiles are such to each block that meets them first: with weights from memory 333 x 4,800 x 1,600 (tiles
+// of 128 x 128, 114 blocks) took 16.5 us, out of the last-level cache 13.4, however many slots the ring had.  So blocks behind the
+// tiles', as many a die as it has units left, read their die's columns in the order in which the tiles will want them, four pieces of a k-block on their way
+// each, into nothing: the tiles' copies find them in the L2.  They end by themselves with the last piece and nobody waits for
+// them.  us, rows x features x K, without and with: 333 x 6,400 x 1,600 16.7 -> 14.4, 2,048 x 1,600 x 6,400 53.7 -> 47.1, 1,000 x 1,600 x 1,600 (64 x 128)
+// 13.3 -> 10.6, 200 x 4,800 x 1,600 (64 x 128) 13.8 -> 10.9, 100 x 5,440 x 1,024 (32 x 128) 8.1 -> 7.3.
+template <typename S>
+__device__ __forceinline__ void read_weights(const GemmArgs& p, int kb_lo, int n_blocks) {
+  const int tiles_n = (p.N + S::BN - 1) / S::BN;
+  const int reader = ((int)blockIdx.x - p.tile_blocks) / N_DIES, readers = ((int)gridDim.x - p.tile_blocks) / N_DIES;
+  int first, columns;
+  if (!columns_of_die<S::PANEL>((p.M + S::BM - 1) / S::BM, tiles_n, blockIdx.x % N_DIES, first, columns)) return;
+  columns = min(columns, readers);  // (a reader that had more to read would still be at it when the tiles are done)
+  const int n_fb = (p.N + 15) / 16, pieces = n_blocks * columns;  // a k-block of a column of tiles
+  constexpr int LOADS = (S::BN * 8 + S::THREADS - 1) / S::THREADS, GROUP = 4;
+  for (int i = reader; i < pieces; i += GROUP * readers) {
+    u32x4_t v[GROUP][LOADS];
+#pragma unroll
+    for (int g = 0; g < GROUP; ++g) {
+      const int at = min(i + g * readers, pieces - 1), kb = kb_lo + at / columns, fb = (first + at % columns) % tiles_n * (S::BN / 16);
+#pragma unroll
+      for (int l = 0; l < LOADS; ++l) {
+        const int t = min(l * S::THREADS + (int)threadIdx.x, S::BN * 8 - 1);
+        v[g][l] = *(const u32x4_t*)(p.W + ((size_t)min(fb + (t >> 7), n_fb - 1) * p.w_kblocks + kb) * 1024 + (t & 127) * 8);
+      }
+    }
+#pragma unroll
+    for (int g = 0; g < GROUP; ++g)
+#pragma unroll
+      for (int l = 0; l < LOADS; ++l) asm volatile("" ::"v"(v[g][l]));  // (read, and forgotten)
+  }
+}
 
 // Pipeline: k-block kb is multiplied out of one slot of each ring while the next ones are on their way into
 // the others (lds_copy.h); one wait by count and one barrier a k-block.  Nothing passes through registers but the operands,
@@ -148,6 +188,10 @@ __global__ __launch_bounds__(S::THREADS, S::WAVES_PER_SIMD) void gemm_bf16_tile_
   // (one buffer: the epilogue uses it again for the output tiles)
   __shared__ __attribute__((aligned(1024))) uint16_t smem[S::RING / 2];
 
+  if (PACKED && (int)blockIdx.x >= p.tile_blocks) {
+    const int lo = SPLIT ? blockIdx.y * p.blocks_per_split : 0, all = (p.K + BK - 1) / BK;
+    return read_weights<S>(p, lo, SPLIT ? min(all, lo + p.blocks_per_split) - lo : all);
+  }
   int tm, tn;
   if (!tile_of_block<S::PANEL>((p.M + BM - 1) / BM, (p.N + BN - 1) / BN, tm, tn)) return;
   const int tid = threadIdx.x;
@@ -174,6 +218,7 @@ __global__ __launch_bounds__(S::THREADS, S::WAVES_PER_SIMD) void gemm_bf16_tile_
   // different groups of banks (s ^ (r % 8), which gives only eight, made a read take twice as long).  Packed weights need none of that: half a tile of 16 features x 64 k is a copy as it lies, and
   // sixteen lanes read 256 bytes in a row.  Rows beyond the matrix lie beyond the buffer's end, columns beyond K are
   // sent there.
+  const int asker = S::COPIERS ? wave - S::WAVES : wave;
   const i32x4_t a_buf = copy_buffer(p.A, ((size_t)(p.M - 1) * p.lda + p.K) * 2);
   const i32x4_t b_buf = copy_buffer(p.W, PACKED ? (size_t)((p.N + 15) / 16) * p.w_kblocks * 2048
                                                 : ((size_t)(p.N - 1) * p.ldw + p.K) * 2);
@@ -182,12 +227,12 @@ __global__ __launch_bounds__(S::THREADS, S::WAVES_PER_SIMD) void gemm_bf16_tile_
   uint32_t a_from[PA], b_from[PB];
 #pragma unroll
   for (int i = 0; i < PA; ++i) {
-    const int row = m0 + (wave * PA + i) * 8 + row8;
-    a_from[i] = row < p.M ? (uint32_t)(((size_t)row * p.lda + piece_of(wave * PA + i) * 8) * 2) : COPY_NOTHING;
+    const int row = m0 + (asker * PA + i) * 8 + row8;
+    a_from[i] = row < p.M ? (uint32_t)(((size_t)row * p.lda + piece_of(asker * PA + i) * 8) * 2) : COPY_NOTHING;
   }
 #pragma unroll
   for (int i = 0; i < PB; ++i) {
-    const int g = wave * PB + i;
+    const int g = asker * PB + i;
     if constexpr (PACKED) {
       const int fb = n0 / 16 + (g >> 1);
       b_from[i] = fb < (p.N + 15) / 16 ? (uint32_t)(((size_t)fb * p.w_kblocks * 1024 + (g & 1) * 512 + lane * 8) * 2) : COPY_NOTHING;
@@ -197,7 +242,7 @@ __global__ __launch_bounds__(S::THREADS, S::WAVES_PER_SIMD) void gemm_bf16_tile_
     }
   }
   const uint32_t ring = lds_address(smem);
-  const uint32_t a_to = ring + wave * PA * 1024, b_to = ring + S::B_BASE + wave * PB * 1024;
+  const uint32_t a_to = ring + asker * PA * 1024, b_to = ring + S::B_BASE + asker * PB * 1024;
   // What a round asks for: rows' k-block ka into slot sa and weights' k-block kb into slot sb, copy by copy.
   // (k-blocks beyond the last are asked for too, as nothing: the waits then count the same copies in every round)
   struct Round {
@@ -214,10 +259,10 @@ __global__ __launch_bounds__(S::THREADS, S::WAVES_PER_SIMD) void gemm_bf16_tile_
   };
   auto ask = [&](const Round& q, int i) __attribute__((always_inline)) {
     if (i < PA) {
-      copy16_to_lds(a_buf, piece_of(wave * PA + i) * 8 < q.k_left_a ? a_from[i < PA ? i : 0] : COPY_NOTHING, q.a_k, a_to + q.a_at + i * 1024);
+      copy16_to_lds(a_buf, piece_of(asker * PA + i) * 8 < q.k_left_a ? a_from[i < PA ? i : 0] : COPY_NOTHING, q.a_k, a_to + q.a_at + i * 1024);
     } else {
       const int j = i < PA ? 0 : i - PA;
-      copy16_to_lds(b_buf, (PACKED ? q.k_left_b > 0 : piece_of(wave * PB + j) * 8 < q.k_left_b) ? b_from[j] : COPY_NOTHING, q.b_k,
+      copy16_to_lds(b_buf, (PACKED ? q.k_left_b > 0 : piece_of(asker * PB + j) * 8 < q.k_left_b) ? b_from[j] : COPY_NOTHING, q.b_k,
                     b_to + q.b_at + j * 1024);
     }
   };
@@ -238,7 +283,8 @@ __global__ __launch_bounds__(S::THREADS, S::WAVES_PER_SIMD) void gemm_bf16_tile_
   // The operands of 16 columns (a quarter of a k-block) go to registers one quarter ahead of their products, also
   // across the barrier: a k-block's last quarter is multiplied after the barrier that lets the next one be read.
   bf16x8_t fa[2][TM], fb[2][TN];
-  int slot_a = 0, slot_b = 0;
+  int slot_a = 0;
+  [[maybe_unused]] int slot_b = 0;
   auto read_quarter = [&](int set, int q) __attribute__((always_inline)) {
     const char* af = a_row + slot_a * S::A_STRIDE;
     const char* bf = b_row + (S::ALIKE ? slot_a : slot_b) * S::B_STRIDE;
@@ -269,40 +315,79 @@ __global__ __launch_bounds__(S::THREADS, S::WAVES_PER_SIMD) void gemm_bf16_tile_
   };
 
   constexpr int SA = S::SLOTS_A, SB = S::SLOTS_B, AHEAD = SA > SB ? SA : SB;
+  if constexpr (S::COPIERS > 0) {
+    static_assert(S::ALIKE && !S::SPREAD, "waves that only copy");
+    if (wave >= S::WAVES) {
 #pragma unroll
-  for (int t = 1 - AHEAD; t < 0; ++t) {  // as rounds before the first would have it
-    const Round q = round_of(t + SA - 1, t + SA - 1, t + SB - 1, t + SB - 1);
+      for (int t = 0; t < SA - 1; ++t) {
+        const Round q = round_of(t, t, t, t);
 #pragma unroll
-    for (int i = t + SA - 1 >= 0 ? 0 : PA; i < (t + SB - 1 >= 0 ? S::COPIES : PA); ++i) ask(q, i);
-  }
-  // A round asks for rows SA - 1 and weights SB - 1 k-blocks ahead, the rows first.  When k-block kb begins, its rows came
-  // with round kb - SA + 1 and its weights with round kb - SB + 1: so many copies were asked for behind both.
-  constexpr int BEHIND_A = PB + (SA - 2) * S::COPIES, BEHIND_B = (SB - 2) * S::COPIES;
-  const Round none = round_of(0, 0, 0, 0);
-  for (int kb = 0; kb < n_blocks; ++kb) {
-    copies_arrived<(BEHIND_A < BEHIND_B ? BEHIND_A : BEHIND_B)>();
-    ring_barrier();  // k-block kb is whole, and nobody reads the slots of k-block kb - 1 any more
-    read_quarter(0, 0);
-    const int next_a = slot_a == 0 ? SA - 1 : slot_a - 1, next_b = S::ALIKE ? next_a : slot_b == 0 ? SB - 1 : slot_b - 1;
-    const Round q = round_of(kb + SA - 1, next_a, kb + SB - 1, next_b);
-    if (!S::SPREAD || kb == 0) {
+        for (int i = 0; i < S::COPIES; ++i) ask(q, i);
+      }
+      for (int kb = 0; kb < n_blocks; ++kb) {
+        copies_arrived<(SA - 2) * S::COPIES>();
+        ring_barrier();  // k-block kb is whole, and nobody reads the slot of k-block kb - 1 any more
+        const int next = slot_a == 0 ? SA - 1 : slot_a - 1;
+        const Round q = round_of(kb + SA - 1, next, kb + SA - 1, next);
 #pragma unroll
-      for (int i = 0; i < TAKES; ++i) ask(q, i);
-      if (kb > 0) multiply(1, none, 0, 0);
-    } else {
-      multiply(1, q, 0, TAKES);
+        for (int i = 0; i < S::COPIES; ++i) ask(q, i);
+        slot_a = slot_a == SA - 1 ? 0 : slot_a + 1;
+      }
+      copies_arrived<0>();  // (what was asked for beyond the end: the epilogue writes where it goes)
+      if (!SPLIT) __syncthreads();
+      return;
     }
-    read_quarter(1, 1);
-    multiply(0, q, TAKES, S::COPIES);
-    read_quarter(0, 2);
+    const Round none = round_of(0, 0, 0, 0);
+    for (int kb = 0; kb < n_blocks; ++kb) {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      ring_barrier();
+      read_quarter(0, 0);
+      if (kb > 0) multiply(1, none, 0, 0);
+      read_quarter(1, 1);
+      multiply(0, none, 0, 0);
+      read_quarter(0, 2);
+      multiply(1, none, 0, 0);
+      read_quarter(1, 3);
+      multiply(0, none, 0, 0);
+      slot_a = slot_a == SA - 1 ? 0 : slot_a + 1;
+    }
     multiply(1, none, 0, 0);
-    read_quarter(1, 3);
-    multiply(0, none, 0, 0);
-    slot_a = slot_a == SA - 1 ? 0 : slot_a + 1;
-    if constexpr (!S::ALIKE) slot_b = slot_b == SB - 1 ? 0 : slot_b + 1;
+  } else {
+#pragma unroll
+    for (int t = 1 - AHEAD; t < 0; ++t) {  // as rounds before the first would have it
+      const Round q = round_of(t + SA - 1, t + SA - 1, t + SB - 1, t + SB - 1);
+#pragma unroll
+      for (int i = t + SA - 1 >= 0 ? 0 : PA; i < (t + SB - 1 >= 0 ? S::COPIES : PA); ++i) ask(q, i);
+    }
+    // A round asks for rows SA - 1 and weights SB - 1 k-blocks ahead, the rows first.  When k-block kb begins, its rows came
+    // with round kb - SA + 1 and its weights with round kb - SB + 1: so many copies were asked for behind both.
+    constexpr int BEHIND_A = PB + (SA - 2) * S::COPIES, BEHIND_B = (SB - 2) * S::COPIES;
+    const Round none = round_of(0, 0, 0, 0);
+    for (int kb = 0; kb < n_blocks; ++kb) {
+      copies_arrived<(BEHIND_A < BEHIND_B ? BEHIND_A : BEHIND_B)>();
+      ring_barrier();  // k-block kb is whole, and nobody reads the slots of k-block kb - 1 any more
+      read_quarter(0, 0);
+      const int next_a = slot_a == 0 ? SA - 1 : slot_a - 1, next_b = S::ALIKE ? next_a : slot_b == 0 ? SB - 1 : slot_b - 1;
+      const Round q = round_of(kb + SA - 1, next_a, kb + SB - 1, next_b);
+      if (!S::SPREAD || kb == 0) {
+#pragma unroll
+        for (int i = 0; i < TAKES; ++i) ask(q, i);
+        if (kb > 0) multiply(1, none, 0, 0);
+      } else {
+        multiply(1, q, 0, TAKES);
+      }
+      read_quarter(1, 1);
+      multiply(0, q, TAKES, S::COPIES);
+      read_quarter(0, 2);
+      multiply(1, none, 0, 0);
+      read_quarter(1, 3);
+      multiply(0, none, 0, 0);
+      slot_a = slot_a == SA - 1 ? 0 : slot_a + 1;
+      if constexpr (!S::ALIKE) slot_b = slot_b == SB - 1 ? 0 : slot_b + 1;
+    }
+    multiply(1, none, 0, 0);
+    copies_arrived<0>();  // (what was asked for beyond the end: the epilogue writes where it goes)
   }
-  multiply(1, none, 0, 0);
-  copies_arrived<0>();  // (what was asked for beyond the end: the epilogue writes where it goes)
 
   if constexpr (SPLIT) {  // the partial sums as they are; sum_partials adds them and runs the epilogue
     float* ws = p.ws + (size_t)blockIdx.y * p.M * p.N;
@@ -336,7 +421,7 @@ __global__ __launch_bounds__(S::THREADS, S::WAVES_PER_SIMD) void gemm_bf16_tile_
   // wave passes its tile through LDS, 32 rows at a time, and takes it out again with eight
   // neighbouring columns a lane: stores of 16 or 32 bytes a lane that cover whole rows of
   // the wave's tile.  The region of a wave is its own; a wave's LDS accesses keep their order.
-  constexpr int NW = S::THREADS / 64;
+  constexpr int NW = S::WAVES;
   constexpr int WCOLS = TN * 32;   // columns of a wave's tile
   constexpr int EST = WCOLS + 4;   // floats a row in LDS: sixteen-byte pieces of neighbouring rows on other banks
   static_assert(NW * 32 * EST * 4 <= (int)sizeof(smem), "the waves' output tiles fit the k-blocks' LDS");
@@ -584,9 +669,10 @@ static int check_args(const GemmArgs& p) {
 }
 
 template <typename S, bool CAN_SPLIT>
-static void launch_tiles(const GemmArgs& p, hipStream_t stream) {
+static void launch_tiles(GemmArgs p, hipStream_t stream, int readers = 0) {
   const long tiles = (long)((p.M + S::BM - 1) / S::BM) * ((p.N + S::BN - 1) / S::BN);
   dim3 grid((unsigned)((tiles + 7) / 8 * 8), p.n_splits), block(S::THREADS);  // a run of tiles for each die
+  p.tile_blocks = grid.x, grid.x += N_DIES * readers;
   if constexpr (CAN_SPLIT) {
     if (p.n_splits > 1) {
       if (p.w_packed)
@@ -602,32 +688,64 @@ static void launch_tiles(const GemmArgs& p, hipStream_t stream) {
     hipLaunchKernelGGL((gemm_bf16_tile_kernel<S, false, false>), grid, block, 0, stream, p);
 }
 
-// What a shape costs, in microseconds: `tile` for each round of tiles on a CU and `kblock` for each k-block of it, `pair`
-// a k-block where two blocks share the CU (shapes that fit twice), `launch` once.  Fitted to the times of 16 numbers of
-// rows from 20 to 8,000 against 18 matrices of widths from 768 to 2,048, K up to 6,400, each with K in 1 to 8 parts; the
-// shape and parts chosen from these prices are within 2 % of the best on average (at worst 1.35 times: 20 to 64 rows to
-// 10,880 features, a gated feed-forward 2,048 wide, which the kernel for few rows cannot hold).  With K whole, 333 to 8,000 rows
-// against sixteen matrices, they choose the fastest shape everywhere.
+// Compute units of a die that a product's tiles leave idle, for each part of K, and the columns of tiles that they would read ahead for.
+template <typename S>
+static void idle_units(int M, int N, int n_splits, int* idle, double* columns) {
+  const int tiles_m = (M + S::BM - 1) / S::BM, run = (tiles_m * ((N + S::BN - 1) / S::BN) + N_DIES - 1) / N_DIES;
+  const int left = n_compute_units() / N_DIES - run * n_splits;
+  *idle = left > 0 ? left / n_splits : 0;
+  *columns = (double)run / (tiles_m < S::PANEL ? tiles_m : S::PANEL);
+}
+
+// Compute units a die and part of K that read the weights ahead (0: none do).  Too few of them fall behind the tiles and are still
+// reading when those are done: 333 x 4,800 x 1,600 in tiles of 64 x 128 (three a die for five columns) 14.0 -> 14.5 us, 536 x 1,600 x 1,600 in
+// two parts (one for two) 8.8 -> 9.6.  Tiles of 128 x 128 want nearly two a column (536 x 4,800 x 1,600, eight for five, 15.0 -> 15.5; 470 x 6,400 x
+// 1,600, thirteen for six, 16.7 -> 14.4) and gain nothing in parts of K (25 us with 24.6 for 536 x 1,600 x 6,400 in two); the widest were
+// level or behind (1,000 x 6,400 x 1,600 in 256 x 128 24.7 -> 25.7).  More than eight (twelve) take from the tiles: 333 x 6,400 x 1,600 15.2 with twelve.
+static int readers_of(int variant, int M, int N, int n_splits, bool packed) {
+  int idle = 0;
+  double columns = 0.0;
+  if (!packed || M < TILE_MIN_ROWS || (variant == 1 && n_splits > 1)) return 0;
+  if (variant == 1)
+    idle_units<Tile128>(M, N, n_splits, &idle, &columns);
+  else if (variant == 5)
+    idle_units<Tile64x128>(M, N, n_splits, &idle, &columns);
+  else if (variant == 6)
+    idle_units<Tile32x128>(M, N, n_splits, &idle, &columns);
+  else
+    return 0;
+  const double enough = variant == 1 ? 1.83 : 0.9;
+  const int most = variant == 1 ? 8 : 12;
+  return idle < 1 || idle < enough * columns ? 0 : idle < most ? idle : most;
+}
+
+// What a shape costs, in microseconds: `launch` once, `tile` for each round of tiles on a CU and `kblock` for each k-block of it, `pair`
+// a k-block where two blocks share the CU (shapes that fit twice); where CUs that have no tile read weights ahead, `fed_tile` and
+// `fed` instead.  `full`: what a k-block costs at least where all CUs ask the L2s for one at once (fewer in proportion).  Fitted to the
+// times of 18 numbers of rows from 65 to 2,048 against 18 matrices of widths 768 to 2,048, K up to
+// 6,400, weights from 2.5 GB of memory, each with K in 1 to 8 parts; the shape and parts chosen from these prices are within 1.1 % of the best on average (at
+// worst 1.18 times; the prices before the readers, 6.7 % and 1.76).
 struct TilePrice {
   int variant, bm, bn, per_cu;
   double launch, tile, kblock, pair;
   bool splits;  // K may be split over blocks
+  double fed_tile, fed, full;
 };
 static const TilePrice TILE_PRICES[] = {
-    {3, Tile256::BM, Tile256::BN, 1, 0.0, 7.78, 1.3, 0.0, false},
-    {4, Tile256x192::BM, Tile256x192::BN, 1, 0.0, 7.26, 1.0, 0.0, false},
-    {8, Tile256x128::BM, Tile256x128::BN, 1, 0.0, 7.6, 0.7, 0.0, false},
-    {1, Tile128::BM, Tile128::BN, 1, 0.0, 4.33, 0.49, 0.0, true},
-    {5, Tile64x128::BM, Tile64x128::BN, 2, 0.52, 2.81, 0.38, 0.77, true},
-    {6, Tile32x128::BM, Tile32x128::BN, 2, 1.81, 1.98, 0.33, 0.52, true},
+    {3, Tile256::BM, Tile256::BN, 1, 0.0, 7.69, 1.042, 0.0, false, 0.0, 0.0, 0.0},
+    {4, Tile256x192::BM, Tile256x192::BN, 1, 0.0, 6.9, 0.885, 0.0, false, 0.0, 0.0, 0.0},
+    {8, Tile256x128::BM, Tile256x128::BN, 1, 0.0, 6.1, 0.65, 0.0, false, 0.0, 0.0, 0.0},
+    {1, Tile128::BM, Tile128::BN, 1, 0.21, 4.09, 0.499, 0.0, true, 4.25, 0.331, 0.686},
+    {5, Tile64x128::BM, Tile64x128::BN, 2, 3.11, 1.32, 0.363, 0.708, true, 0.49, 0.276, 0.403},
+    {6, Tile32x128::BM, Tile32x128::BN, 2, 2.83, 1.54, 0.191, 0.516, true, 0.83, 0.202, 0.316},
 };
 static double price(const TilePrice& s, int M, int N, int K, int n_splits) {
-  const long tiles = (long)((M + s.bm - 1) / s.bm) * ((N + s.bn - 1) / s.bn);
-  const int cus = n_compute_units();
-  // the busiest CU: of a die's run of tiles, or of all blocks where K is split
-  const long n = n_splits > 1 ? (tiles * n_splits + cus - 1) / cus
-                              : ((tiles + N_DIES - 1) / N_DIES + cus / N_DIES - 1) / (cus / N_DIES);
+  const long tiles = (long)((M + s.bm - 1) / s.bm) * ((N + s.bn - 1) / s.bn), cus = n_compute_units(), per_die = cus / N_DIES;
+  const long n = ((tiles + N_DIES - 1) / N_DIES * n_splits + per_die - 1) / per_die;  // the busiest CU
   const int k_blocks = ((K + BK - 1) / BK + n_splits - 1) / n_splits;
+  const double least = s.full * (tiles * n_splits < cus ? tiles * n_splits : cus) / cus;
+  if (readers_of(s.variant, M, N, n_splits, true)) return s.launch + s.fed_tile + k_blocks * (s.fed > least ? s.fed : least);
+  if (n == 1) return s.launch + s.tile + k_blocks * (s.kblock > least ? s.kblock : least);
   if (s.per_cu == 1) return s.launch + n * (s.tile + k_blocks * s.kblock);
   return s.launch + (n / 2) * (s.tile + k_blocks * s.pair) + (n % 2) * (s.tile + k_blocks * s.kblock);
 }
@@ -767,13 +885,17 @@ extern "C" int gemm_bf16_scatter(void* out, const void* A, const void* W, const 
     else
       hipLaunchKernelGGL(gemm_bf16_skinny_kernel<4>, grid, block, 0, stream, p);
   } else if (variant == 1) {
-    launch_tiles<Tile128, true>(p, stream);
+    const int readers = readers_of(variant, M, N, n_splits, p.w_packed);
+    if (readers && n_splits == 1)
+      launch_tiles<Tile128Fed, false>(p, stream, readers);
+    else
+      launch_tiles<Tile128, true>(p, stream, readers);
   } else if (variant == 7) {
     launch_tiles<Tile128Pair, false>(p, stream);
   } else if (variant == 5) {
-    launch_tiles<Tile64x128, true>(p, stream);
+    launch_tiles<Tile64x128, true>(p, stream, readers_of(variant, M, N, n_splits, p.w_packed));
   } else if (variant == 6) {
-    launch_tiles<Tile32x128, true>(p, stream);
+    launch_tiles<Tile32x128, true>(p, stream, readers_of(variant, M, N, n_splits, p.w_packed));
   } else if (variant == 3) {
     launch_tiles<Tile256, false>(p, stream);
   } else if (variant == 4) {

@@ -1,3 +1,4 @@
+// The order in which the blocks of a product take its tiles (gemm_bf16.hip, gemm_f32.hip).
 #pragma once
 #include "common.h"
 
@@ -21,5 +22,20 @@ __device__ __forceinline__ bool tile_of_block(int tiles_m, int tiles_n, int& tm,
   const int h = min(PANEL, tiles_m - panel * PANEL);
   tn = rem / h;
   tm = panel * PANEL + rem % h;
+  return true;
+}
+
+// The columns of tiles that a die's run touches, panel after panel: `n` of them from column `first` of the sequence in which panel
+// after panel brings its columns (the matrix's column is the remainder by tiles_n).
+template <int PANEL>
+__device__ __forceinline__ bool columns_of_die(int tiles_m, int tiles_n, int die, int& first, int& n) {
+  const int total = tiles_m * tiles_n, run = (total + 7) / 8;
+  if (die * run >= total) return false;
+  const auto column_of = [&](int idx) {
+    const int panel = min(idx / (PANEL * tiles_n), (tiles_m + PANEL - 1) / PANEL - 1);
+    return panel * tiles_n + (idx - panel * PANEL * tiles_n) / min(PANEL, tiles_m - panel * PANEL);
+  };
+  first = column_of(die * run);
+  n = column_of(min(total, (die + 1) * run) - 1) - first + 1;
   return true;
 }

@@ -1409,6 +1409,26 @@ def test_gemm_bf16_tiles_at_the_ring_s_edges(M, N, K, packed):
         assert err < tol, (variant, splits, err)
 
 
+@pytest.mark.parametrize("M,N,K", [(65, 129, 72), (333, 1000, 328), (1100, 300, 640), (2048, 1600, 200), (150, 4800, 136), (70, 2056, 1608)])
+def test_gemm_bf16_weights_read_ahead(M, N, K):
+    """Packed weights, which compute units without a tile read ahead and waves that only copy feed to the tiles, give the bits that
+    row-major ones give (no block reads those ahead): one row of tiles and several panels, last columns and k-blocks that are not
+    whole, more readers than columns and as many, K whole and in parts, each epilogue."""
+    k = _k()
+    a, w = _rand((M, K), torch.bfloat16, 10), _rand((N, K), torch.bfloat16, 11, 0.1)
+    bias = _rand((N,), torch.float32, 12)
+    packed = k.PackedWeight(w, keep_rows=False)
+    for variant in (1, 5, 6):
+        for splits in [None] + [s for s in (2, 5) if s <= (K + 63) // 64]:
+            for mode in ("plain", "gelu", "accumulate"):
+                got = []
+                for weights in (w, packed):
+                    out = torch.full((M, N), 0.5, dtype=torch.float32 if mode == "accumulate" else torch.bfloat16, device=DEV)
+                    k.linear(out, a, weights, bias, gelu=mode == "gelu", accumulate=mode == "accumulate", variant=variant, splits=splits)
+                    got.append(out)
+                assert torch.equal(got[0], got[1]), (variant, splits, mode)
+
+
 @pytest.mark.parametrize("M,N,K", [(17, 48, 64), (33, 257, 384), (64, 4800, 1600), (40, 1600, 6400), (64, 333, 1608),
                                    (48, 80, 200), (20, 100, 520), (32, 4800, 1600), (24, 1600, 6400), (30, 333, 1608)])
 @pytest.mark.parametrize("mode", ["plain", "gelu", "accumulate", "f32out"])
