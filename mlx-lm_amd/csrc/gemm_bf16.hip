@@ -688,6 +688,8 @@ static void launch_tiles(GemmArgs p, hipStream_t stream, int readers = 0) {
     hipLaunchKernelGGL((gemm_bf16_tile_kernel<S, false, false>), grid, block, 0, stream, p);
 }
 
+#define FEW_ROWS 64  // up to so many rows packed weights are other kernels' (gemm_bf16_decode.hip), but for a K that they do not hold
+
 // Compute units of a die that a product's tiles leave idle, for each part of K, and the columns of tiles that they would read ahead for.
 template <typename S>
 static void idle_units(int M, int N, int n_splits, int* idle, double* columns) {
@@ -705,7 +707,7 @@ static void idle_units(int M, int N, int n_splits, int* idle, double* columns) {
 static int readers_of(int variant, int M, int N, int n_splits, bool packed) {
   int idle = 0;
   double columns = 0.0;
-  if (!packed || M < TILE_MIN_ROWS || (variant == 1 && n_splits > 1)) return 0;
+  if (!packed || M <= FEW_ROWS || (variant == 1 && n_splits > 1)) return 0;
   if (variant == 1)
     idle_units<Tile128>(M, N, n_splits, &idle, &columns);
   else if (variant == 5)
@@ -723,7 +725,7 @@ static int readers_of(int variant, int M, int N, int n_splits, bool packed) {
 // a k-block where two blocks share the CU (shapes that fit twice); where CUs that have no tile read weights ahead, `fed_tile` and
 // `fed` instead.  `full`: what a k-block costs at least where all CUs ask the L2s for one at once (fewer in proportion).  Fitted to the
 // times of 18 numbers of rows from 65 to 2,048 against 18 matrices of widths 768 to 2,048, K up to
-// 6,400, weights from 2.5 GB of memory, each with K in 1 to 8 parts; the shape and parts chosen from these prices are within 1.1 % of the best on average (at
+// 6,400, weights from 2.5 GB of memory, each with K in 1 to 8 parts; the shape and parts chosen from these prices are within 1.2 % of the best on average (at
 // worst 1.18 times; the prices before the readers, 6.7 % and 1.76).
 struct TilePrice {
   int variant, bm, bn, per_cu;
@@ -736,9 +738,16 @@ static const TilePrice TILE_PRICES[] = {
     {4, Tile256x192::BM, Tile256x192::BN, 1, 0.0, 6.9, 0.885, 0.0, false, 0.0, 0.0, 0.0},
     {8, Tile256x128::BM, Tile256x128::BN, 1, 0.0, 6.1, 0.65, 0.0, false, 0.0, 0.0, 0.0},
     {1, Tile128::BM, Tile128::BN, 1, 0.21, 4.09, 0.499, 0.0, true, 4.25, 0.331, 0.686},
-    {5, Tile64x128::BM, Tile64x128::BN, 2, 3.11, 1.32, 0.363, 0.708, true, 0.49, 0.276, 0.403},
-    {6, Tile32x128::BM, Tile32x128::BN, 2, 2.83, 1.54, 0.191, 0.516, true, 0.83, 0.202, 0.316},
+    {5, Tile64x128::BM, Tile64x128::BN, 2, 3.11, 1.32, 0.363, 0.708, true, 0.49, 0.32, 0.403},
+    {6, Tile32x128::BM, Tile32x128::BN, 2, 2.83, 1.54, 0.27, 0.516, true, 0.83, 0.202, 0.316},
 };
+// Up to 64 rows, what the kernels for few rows leave (row-major weights, a longer K than they hold): no readers.
+static const TilePrice FEW_PRICES[] = {
+    {1, Tile128::BM, Tile128::BN, 1, 0.0, 4.33, 0.49, 0.0, true, 0.0, 0.0, 0.0},
+    {5, Tile64x128::BM, Tile64x128::BN, 2, 0.52, 2.81, 0.38, 0.77, true, 0.0, 0.0, 0.0},
+    {6, Tile32x128::BM, Tile32x128::BN, 2, 1.81, 1.98, 0.33, 0.52, true, 0.0, 0.0, 0.0},
+};
+
 static double price(const TilePrice& s, int M, int N, int K, int n_splits) {
   const long tiles = (long)((M + s.bm - 1) / s.bm) * ((N + s.bn - 1) / s.bn), cus = n_compute_units(), per_die = cus / N_DIES;
   const long n = ((tiles + N_DIES - 1) / N_DIES * n_splits + per_die - 1) / per_die;  // the busiest CU
@@ -752,11 +761,15 @@ static double price(const TilePrice& s, int M, int N, int K, int n_splits) {
 // The cheapest shape for K in so many parts, and its price.
 static int cheapest_shape(int M, int N, int K, int n_splits, double* us) {
   int variant = 0;
-  for (const TilePrice& s : TILE_PRICES) {
-    if (n_splits > 1 && !s.splits) continue;
+  const auto look = [&](const TilePrice& s) {
+    if (n_splits > 1 && !s.splits) return;
     const double t = price(s, M, N, K, n_splits);
     if (!variant || t < *us) variant = s.variant, *us = t;
-  }
+  };
+  if (M <= FEW_ROWS)
+    for (const TilePrice& s : FEW_PRICES) look(s);
+  else
+    for (const TilePrice& s : TILE_PRICES) look(s);
   return variant;
 }
 
@@ -788,11 +801,13 @@ extern "C" int gemm_bf16_splits(int M, int N, int K, int fused, int force) {
     best = force < n_blocks ? force : n_blocks;
   } else {
     double best_us = 0.0;
-    for (int s = 1; s <= 16 && s <= (n_blocks >= 3 ? n_blocks / 3 : 1); ++s) {
+    // (a long K of few rows goes in eight parts or more: five to eight are within 3 % of each other at 65 to 80 rows of 1,600 x 6,400)
+    const int first = M > FEW_ROWS && M <= 96 && n_blocks >= 96 ? 8 : 1;
+    for (int s = first; s <= 16 && s <= (n_blocks >= 3 ? n_blocks / 3 : 1); ++s) {
       double us = 0.0;
       cheapest_shape(M, N, K, s, &us);
       if (s > 1) us += (fused ? 1.0 : 2.5) + 8.0 * (fused ? s - 1 : s) * (double)M * N / 3e6;
-      if (s == 1 || us < 0.98 * best_us) best = s, best_us = us;
+      if (s == first || us < 0.98 * best_us) best = s, best_us = us;
     }
   }
   if (best <= 1) return 1;
