@@ -330,7 +330,8 @@ def _reads_by_fours(w):
 
 def row_exponents(w):
     """What the tiles of the 32-bit product scale each row of ``w`` ``[N, K]`` by, as powers of two (csrc/gemm_f32.hip): found once
-    where weights are laid out, ahead of every product for other tensors."""
+    where weights are laid out, ahead of every product for other tensors.  (Of rows that are changed afterwards it is asked again, as a
+    ``PackedWeight`` is made again.)"""
     lib = build.load("gemm_f32")
     out = torch.empty(w.shape[0], dtype=torch.int32, device=w.device)
     build.check(lib, lib.gemm_f32_exponents(_ptr(out), _ptr(w), w.shape[0], w.shape[1], _rows2d(w, "w"), _stream()), "gemm_f32_exponents")
