@@ -32,7 +32,6 @@ typedef struct {
   int N, K, ldw, dtype;
   size_t chunk_bytes;
   int n_chunks, pad_;
-  const int* exponents;  // float32: what each row is scaled by where it is cut (gemm_f32.hip), as powers of two; null: not known yet
 } EngWeight;
 
 // The input of a mixer or feed-forward: a matrix, or the LayerNorm of float32

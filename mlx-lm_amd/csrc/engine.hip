@@ -83,7 +83,7 @@ typedef int (*fn_layernorm)(void*, const float*, const int*, const float*, const
                             hipStream_t);
 typedef int (*fn_gemm_f32)(void*, const void*, const void*, const float*, int, int, int, int, int, int, int,
                            int, int, float*, size_t, void*, void*, size_t, const int*, int, const int*, const int*, int, int,
-                           int, int, const int*, float*, size_t, hipStream_t);
+                           int, int, float*, size_t, hipStream_t);
 typedef int (*fn_gemm_bf16)(void*, const void*, const void*, const float*, int, int, int, int, int, int, int,
                             int, int, float*, size_t, void*, void*, size_t, const int*, int, const int*,
                             const int*, int, int, int, int, hipStream_t);
@@ -557,8 +557,8 @@ static int linear(EngCtx* ctx, const EngMat& out, const EngValue& a, const EngWe
            n_splits > 1 ? ws : nullptr, n_splits > 1 ? ws_floats : (size_t)0, own ? own->k : nullptr, own ? own->v : nullptr,
            own ? own->page_stride : (size_t)0, own ? own->block_table : nullptr, own ? own->max_blocks : 0,
            own ? own->token_req : nullptr, own ? own->positions : nullptr, own ? own->q_width : 0, own ? own->kv_width : 0,
-           own ? own->head_dim : 0, own ? own->page_size : 0, w.exponents,
-           (float*)room.p, room_floats, ctx->stream);
+           own ? own->head_dim : 0, own ? own->page_size : 0, (float*)room.p,
+           room_floats, ctx->stream);
     if (room_floats) {
       ctx->scratch->offset = mark;
       if (ctx->stats) ctx->stats->launches++;  // the one that cuts them

@@ -231,7 +231,8 @@ __global__ __launch_bounds__(S::THREADS, 2) void gemm_f32_tile_kernel(GemmArgs p
 // 3.5 to 8.9 (K from 512 to 6,400, 65 to 4,000 rows).  At K = 16 the cut's own error shows (8.8e-8 against 7.4e-8), hence CUT_FROM_K.
 //
 // cut_rows_kernel finds the exponents and lays the rows out cut, a row's octet of columns as 16 bytes of h and 16 of l where its 32
-// bytes were, so that a tile copies both operands alike; the features' exponents are found when weights are laid out.  The weights, which would
+// bytes were, so that a tile copies both operands alike; the features' are found beside them, by each call: exponents that are kept are
+// wrong as soon as a caller changes its weights in place (what is asked for again overflows, or loses its low bits).  The weights, which would
 // take as much memory again, are cut in registers, 16 columns ahead of their products (24 vector instructions for 8 columns of 32 features, which
 // fit between a wave's 12 products); six products of three bfloat16 numbers each, exact without exponents, took 106 us instead of 68
 // for 1,050 x 5,120 x 1,280.
@@ -810,18 +811,6 @@ extern "C" size_t gemm_f32_room(int M, int N, int K, int variant, int n_splits) 
   return M > 0 && is_cut(choose(M, N, K, variant, n_splits)) ? (size_t)M * cut_stride(K) + (size_t)M + N : 0;
 }
 
-static void cut_rows(const CutArgs& c, hipStream_t stream) {
-  hipLaunchKernelGGL(cut_rows_kernel, dim3((unsigned)(c.M + c.N)), dim3(256), 0, stream, c);
-}
-// What the rows of W are scaled by, powers of two: made once for weights that are kept.
-extern "C" int gemm_f32_exponents(int* out, const float* W, int N, int K, int ldw, hipStream_t stream) {
-  if (N <= 0 || K <= 0 || K % 4 != 0 || ldw % 4 != 0 || ldw < K) FAIL("gemm_f32: bad sizes N=%d K=%d ldw=%d", N, K, ldw);
-  if (!out || !W || ((uintptr_t)W & 15)) FAIL("gemm_f32: W must be 16-byte aligned");
-  cut_rows(CutArgs{nullptr, W, 0, N, K, 0, ldw, 0, nullptr, out}, stream);
-  CHECK_LAUNCH("gemm_f32_exponents");
-  return 0;
-}
-
 // variant: 0 = choose, 1 = tiles of 64 x 128, 2 = of 64 x 64, 4 = of 32 x 64, 3 = the kernel for up to
 // 64 rows, 5 = tiles of cut operands of 128 x 128, 6 = of 64 x 128, 7 = of 64 x 64.  n_splits > 1: K in that many parts, whose sums go to ws[part][M][N] (ws_floats floats at least) for sum_partials of gemm_bf16_decode.hip to add up
 // and finish; out is not written then.
@@ -830,7 +819,7 @@ extern "C" int gemm_f32_scatter(void* out, const void* A, const void* W, const f
                                 int K, int lda, int ldw, int ldo, int flags, int variant, int n_splits, float* ws,
                                 size_t ws_floats, void* k_pages, void* v_pages, size_t page_stride, const int* block_table,
                                 int max_blocks, const int* token_req, const int* positions, int q_width, int kv_width,
-                                int head_dim, int page_size, const int* w_exponents, float* room, size_t room_floats, hipStream_t stream) {
+                                int head_dim, int page_size, float* room, size_t room_floats, hipStream_t stream) {
   GemmArgs p = {};
   p.A = (const float*)A;
   p.W = (const float*)W;
@@ -883,8 +872,9 @@ extern "C" int gemm_f32_scatter(void* out, const void* A, const void* W, const f
     if (!room || ((uintptr_t)room & 15) || room_floats < room_wanted)
       FAIL("gemm_f32: tiles of cut operands need %zu floats of aligned memory", room_wanted);
     int* const exponents = (int*)(room + (size_t)M * cut_stride(K));
-    p.cut = room, p.ldc = cut_stride(K), p.a_exponents = exponents, p.w_exponents = w_exponents ? w_exponents : exponents + M;
-    cut_rows(CutArgs{p.A, p.W, M, w_exponents ? 0 : N, K, lda, ldw, p.ldc, (u32x4_t*)room, exponents}, stream);
+    p.cut = room, p.ldc = cut_stride(K), p.a_exponents = exponents, p.w_exponents = exponents + M;
+    const CutArgs c = {p.A, p.W, M, N, K, lda, ldw, p.ldc, (u32x4_t*)room, exponents};
+    hipLaunchKernelGGL(cut_rows_kernel, dim3((unsigned)(M + N)), dim3(256), 0, stream, c);
     p.through = fits_through_buffer((size_t)M * (n_splits > 1 ? N : ldo) * 4);
     launch(p, variant, stream);
     CHECK_LAUNCH("gemm_f32");

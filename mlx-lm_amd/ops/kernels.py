@@ -299,7 +299,7 @@ def weight_struct(w):
         return w.c
     ld = _rows2d(w, "w")
     w.dtype in DT or _fail(f"weight dtype {w.dtype} not supported")
-    return native.EngWeight(w.data_ptr(), None, w.shape[0], w.shape[1], ld, DT[w.dtype], 0, 0, 0, native.ptr(getattr(w, "row_exponents", None)))
+    return native.EngWeight(w.data_ptr(), None, w.shape[0], w.shape[1], ld, DT[w.dtype], 0, 0, 0)
 
 
 def read_ahead_pays(w, n_rows, with_norm=False):
@@ -314,28 +314,10 @@ def read_ahead_pays(w, n_rows, with_norm=False):
 
 def for_decode(w, keep_rows=False):
     """``w`` in the packed order where the product kernels can use it (bfloat16 on the GPU),
-    instead of the row-major matrix unless ``keep_rows``; float32 rows with their ``row_exponents``; anything
-    else is returned as it is."""
+    instead of the row-major matrix unless ``keep_rows``; anything else is returned as it is."""
     if isinstance(w, torch.Tensor) and w.is_cuda and w.dtype == torch.bfloat16 and w.dim() == 2:
         return PackedWeight(w, keep_rows=keep_rows)
-    if isinstance(w, torch.Tensor) and w.is_cuda and w.dtype == torch.float32 and w.dim() == 2 and _reads_by_fours(w):
-        w = w.detach()
-        w.row_exponents = row_exponents(w)
     return w
-
-
-def _reads_by_fours(w):
-    return w.numel() > 0 and w.stride(1) == 1 and w.shape[1] % 4 == 0 and w.stride(0) % 4 == 0 and w.data_ptr() % 16 == 0
-
-
-def row_exponents(w):
-    """What the tiles of the 32-bit product scale each row of ``w`` ``[N, K]`` by, as powers of two (csrc/gemm_f32.hip): found once
-    where weights are laid out, ahead of every product for other tensors.  (Of rows that are changed afterwards it is asked again, as a
-    ``PackedWeight`` is made again.)"""
-    lib = build.load("gemm_f32")
-    out = torch.empty(w.shape[0], dtype=torch.int32, device=w.device)
-    build.check(lib, lib.gemm_f32_exponents(_ptr(out), _ptr(w), w.shape[0], w.shape[1], _rows2d(w, "w"), _stream()), "gemm_f32_exponents")
-    return out
 
 
 _SPLIT_WS = {}

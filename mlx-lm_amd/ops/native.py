@@ -36,7 +36,7 @@ class EngMat(Structure):
 
 class EngWeight(Structure):
     _fields_ = [("w", c_void_p), ("packed", c_void_p), ("N", c_int), ("K", c_int), ("ldw", c_int),
-                ("dtype", c_int), ("chunk_bytes", c_size_t), ("n_chunks", c_int), ("pad_", c_int), ("exponents", c_void_p)]
+                ("dtype", c_int), ("chunk_bytes", c_size_t), ("n_chunks", c_int), ("pad_", c_int)]
 
 
 class EngValue(Structure):

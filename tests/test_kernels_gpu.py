@@ -142,7 +142,7 @@ def _cut_tolerance(a, w, K):
 @pytest.mark.parametrize("M,N,K", [(1, 1, 4), (65, 60, 32), (64, 129, 68), (127, 128, 100), (129, 257, 520), (300, 70, 1284)])
 def test_gemm_f32_cut_operands(M, N, K):
     """Tiles of cut operands at the edges of tiles, steps of 32 columns and rows of eight: rows and features from 1e-30 to 1e30, columns that
-    differ by 2^12, NaN around the operands, K whole and in parts, exponents known ahead or found by the call (the same bits)."""
+    differ by 2^12, NaN around the operands, K whole and in parts, weights as they are and as they are laid out for a model (the same bits)."""
     k = _k()
     a = torch.full((M + 40, K + 12), float("nan"), device=DEV)[:M, :K]
     w = torch.full((N + 40, K + 12), float("nan"), device=DEV)[:N, :K]
@@ -163,6 +163,22 @@ def test_gemm_f32_cut_operands(M, N, K):
             again = torch.empty(M, N, device=DEV)
             k.linear(again, a, known, variant=variant, splits=splits)
             assert torch.equal(again, wide[:, :N]), (variant, splits)
+
+
+def test_gemm_f32_weights_that_are_changed_in_place():
+    """Weights that were laid out and multiplied with are read as they are now: features that shrink or grow afterwards, by a view that
+    counts no version, give the bits that a copy of them gives."""
+    k = _k()
+    M, N, K = 100, 130, 288
+    a, w = _rand((M, K), torch.float32, 10), _rand((N, K), torch.float32, 11)
+    kept = k.for_decode(w)
+    out, want = torch.empty(M, N, device=DEV), torch.empty(M, N, device=DEV)
+    for by in (1.0, 2.0**-30, 2.0**50):
+        w.data.mul_(torch.where(torch.arange(N, device=DEV)[:, None] % 2 == 0, by, 1.0))
+        for variant in (5, 6, 7):
+            k.linear(out, a, kept, variant=variant)
+            k.linear(want, a, w.clone(), variant=variant)
+            assert torch.equal(out, want), (by, variant)
 
 
 def test_gemm_f32_cut_operands_that_are_not_finite():
