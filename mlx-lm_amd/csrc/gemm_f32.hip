@@ -7,7 +7,8 @@
 //
 // Three ways, chosen by rows and prices: up to 64 rows a kernel that streams the weights once and tiles of few blocks both multiply with
 // v_mfma_f32_16x16x4_f32, a sixteenth of bfloat16's rate; where tiles are many, each float is cut into two half-precision
-// numbers (22 to 24 of its 24 bits) and three products of them stand for one, with smaller errors against 64 bits than the former.
+// numbers (23 or 24 of its 24 bits) and three products of them stand for one, with smaller errors against 64 bits than the former; sums
+// for which a row's range is too wide for that are computed with the float instruction.
 //
 // Up to 64 rows (decode steps) take a kernel of their own, which streams W
 // once through v_mfma_f32_16x16x4_f32, 16 features a block: a 64 x 64 tile
@@ -22,6 +23,12 @@
 #define FLAG_RELU2 FLAG_ACT_RELU2  // the square of the ReLU instead
 #define FLAG_ACCUMULATE 2
 
+// What a row is scaled by where it is cut, a power of two, and the sum (as scaled) below which its small values are in doubt (cut_rows_kernel).
+struct RowScale {
+  int up;
+  float doubt;
+};
+
 struct GemmArgs {
   const float* A;
   const float* W;
@@ -34,10 +41,10 @@ struct GemmArgs {
   // in ws[y][ws_rows][N], without bias or epilogue
   int n_splits, per_split, ws_rows;
   float* ws;
-  // the tiles' rows, cut (cut_rows_kernel), ldc floats apart, and the rows' and features' exponents
+  // the tiles' rows, cut (cut_rows_kernel), ldc floats apart, and the rows' and features' scales
   const float* cut;
-  const int* a_exponents;
-  const int* w_exponents;
+  const RowScale* a_scales;
+  const RowScale* w_scales;
   int ldc;
   int through;  // out and a part of ws are below 4 GB: the tiles' stores go through to memory
   // the kernel for few rows: the features from q_width on are keys and values, which go to their pages too (k_pages null:
@@ -221,60 +228,66 @@ __global__ __launch_bounds__(S::THREADS, 2) void gemm_f32_tile_kernel(GemmArgs p
   }
 }
 
-// Many rows, cut operands.  x = 2^-s (h + l), h the half-precision number nearest to 2^s x and l the one nearest to what h
-// leaves: 11 bits each and a sign, so that h + l is x's 24 bits in three of four cases and misses by its last one in the fourth.  x y is then
-// h h' + h l' + l h', three of v_mfma_f32_32x32x16_f16 (16 times the rate of the float instruction: 5 times its products); l l', 2^-22 of x y at
-// most, is left out.  One power of two a row of A and of W puts the row's greatest value between 2^14 and 2^15: half precision
-// then reaches 2^-39 below it before l loses bits.  h h' and the two smaller products are summed apart, each 16 columns an instruction, so a sum is rounded a
+// Many rows, cut operands.  x = 2^-s (h + 2^-12 l), h the half-precision number nearest to 2^s x and l the one nearest to 2^12 times what h
+// leaves: 11 bits each and a sign, so that the two are x's 24 bits in three of four cases and miss by its last one in the fourth.  x y is then
+// h h' + 2^-12 (h l' + l h'), three of v_mfma_f32_32x32x16_f16 (16 times the rate of the float instruction: 5 times its products); 2^-24 l l', 2^-22 of x y at
+// most, is left out.  One power of two a row of A and of W puts the row's greatest value between 2^14 and 2^15: values down to 2^-28 below it
+// then keep both halves whole (LEAST_WHOLE).  Of smaller ones a row counts how many there are, and a sum that is not well above what they can have lost
+// (one great value beside them that met a zero, say) is computed again with the 32-bit instructions (the end of gemm_f32_cut_kernel).
+// h h' and the two smaller products are summed apart, each 16 columns an instruction, so a sum is rounded a
 // quarter as often as with the float instruction (4 columns each): 2-norm of the error over the result's, normal rows against weights of 0.02,
-// K = 768 / 1,280 / 5,120, 1.9e-7 / 2.4e-7 / 4.6e-7 against 5.0e-7 / 6.4e-7 / 1.3e-6; largest error over the sum of magnitudes, in 2^-24, 1.4 to 3.1 against
-// 3.5 to 8.9 (K from 512 to 6,400, 65 to 4,000 rows).  At K = 16 the cut's own error shows (8.8e-8 against 7.4e-8), hence CUT_FROM_K.
+// K = 768 / 1,280 / 5,120, 1.9e-7 / 2.4e-7 / 4.6e-7 against 5.0e-7 / 6.4e-7 / 1.3e-6 (the same of rows that a GELU left, and 2.2e-7 / 2.8e-7 / 5.4e-7 against 5.7e-7 /
+// 7.4e-7 / 1.5e-6 with one column a thousand times the others); largest error over the sum of magnitudes, in 2^-24, 1.5 to 2.7 against
+// 4.3 to 9.3 (K from 256 to 6,400, 65 to 4,000 rows).  At K = 16 the cut's own error shows (8.6e-8 against 7.4e-8), hence CUT_FROM_K.
 //
-// cut_rows_kernel finds the exponents and lays the rows out cut, a row's octet of columns as 16 bytes of h and 16 of l where its 32
-// bytes were, so that a tile copies both operands alike; the features' are found beside them, by each call: exponents that are kept are
-// wrong as soon as a caller changes its weights in place (what is asked for again overflows, or loses its low bits).  The weights, which would
-// take as much memory again, are cut in registers, 16 columns ahead of their products (24 vector instructions for 8 columns of 32 features, which
-// fit between a wave's 12 products); six products of three bfloat16 numbers each, exact without exponents, took 106 us instead of 68
-// for 1,050 x 5,120 x 1,280.
+// cut_rows_kernel finds the powers and lays the rows out cut, a row's octet of columns as 16 bytes of h and 16 of l where its 32
+// bytes were, so that a tile copies both operands alike; the features' are found beside them, by each call: what is kept is
+// wrong as soon as a caller changes its weights in place.  (No time: the product finds the weights in the last-level cache then.)  The weights, which would
+// take as much memory again, are cut in registers, 16 columns ahead of their products (28 vector instructions for 8 columns of 32 features, between
+// a wave's products); six products of three bfloat16 numbers each, exact without scales, took 106 us instead of 68 for 1,050 x 5,120 x 1,280.
 //
 // What bounds it: at 2,048 rows and more the power (with zeros instead of numbers 4,096 x 4,096 x 1,280 takes three quarters of the time), below
-// the tiles' number and what a CU gets out of the L2s.  us, rows x features x K, with the launch that cuts and with the float instruction's
-// tiles: 300 x 3,840 x 1,280 31.7 (37.2), 1,050 x 3,840 x 1,280 56 (93), 1,050 x 5,120 x 1,280 68 (114), 1,050 x 1,280 x 5,120 in parts 78 (111), 2,048 x 6,400 x
-// 1,600 167 (316: 133 -> 252 TFLOP/s).  Where blocks are few the launch ahead is not made up for: 200 x 1,280 x 1,280 15.5 (13.3), 1,050 x 768 x 768
-// 20.2 (18.8); `price` draws the line.
+// the tiles' number and what a CU gets out of the L2s.  us, rows x features x K, with the launch that cuts (weights from memory) and in brackets with the float
+// instruction's tiles: 300 x 3,840 x 1,280 31.8 (37.2), 1,050 x 3,840 x 1,280 54 (93), 1,050 x 5,120 x 1,280 73 (114), 1,050 x 1,280 x 5,120 in five parts 71.5 (111),
+// 2,048 x 6,400 x 1,600 167 (316: 133 -> 251 TFLOP/s).  Where blocks are few the launch ahead is not made up for: 200 x 1,280 x 1,280 15.5 (13.3), 1,050 x 768 x 768
+// 20.2 (18.8); `price` draws the line.  Where every sum is computed again, 1,050 x 5,120 x 1,280 takes 390.
 //
-// Four waves a block, two by two, each with TM x TN tiles of 32 x 32 outputs.
-template <int TM_, int TN_, int STAGES_, int PANEL_>
+// Four waves a block, WAVES_M of them one below the other, each with TM x TN tiles of 32 x 32 outputs.  Side by side, so that each feature is cut by one
+// wave only: with two by two, each cutting twice as many, 1,050 x 5,120 x 1,280 76.5, x 3,840 x 1,280 59.7, 300 x 3,840 x 1,280 36.5 us.
+template <int WAVES_M_, int TM_, int TN_, int STAGES_, int PANEL_>
 struct CutShape {
+  static constexpr int WAVES_M = WAVES_M_, WAVES_N = 4 / WAVES_M_;
   static constexpr int TM = TM_, TN = TN_, STAGES = STAGES_, PANEL = PANEL_, WAVES = 4, THREADS = 256, STEP = 32;
-  static constexpr int BM = 2 * TM * 32, BN = 2 * TN * 32;
+  static constexpr int BM = WAVES_M * TM * 32, BN = WAVES_N * TN * 32;
   static constexpr int PA = BM / 8 / WAVES, PB = BN / 8 / WAVES, COPIES = PA + PB;  // copies of eight rows a wave and step
   static constexpr int STAGE_BYTES = (BM + BN) * STEP * 4;
 };
-using CutTile128 = CutShape<2, 2, 2, 8>;
-using CutTile64x128 = CutShape<1, 2, 3, 8>;
-using CutTile64 = CutShape<1, 1, 3, 8>;
+using CutTile128 = CutShape<1, 4, 1, 2, 8>;
+using CutTile64x128 = CutShape<1, 2, 1, 3, 8>;
+using CutTile64 = CutShape<2, 1, 1, 3, 8>;
 
 // Columns from which operands may be cut.
 #define CUT_FROM_K 256
+// The low halves are held so much greater: 2^15 at most beside a high half of 2^15.
+#define LOW_UP 4096.f
 
 typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
 
-// Two floats, already scaled, as two half-precision numbers each: the nearest one and what it leaves.
-__device__ __forceinline__ void cut_pair(float y0, float y1, uint32_t& high, uint32_t& low) {
-  const f16x2_t h = __builtin_convertvector((hw_f32x2_t{y0, y1}), f16x2_t);
-  const f16x2_t l = __builtin_convertvector((hw_f32x2_t{__builtin_fmaf((float)h.x, -1.f, y0), __builtin_fmaf((float)h.y, -1.f, y1)}), f16x2_t);
+// Two floats as two half-precision numbers each: the one nearest to the scaled float and LOW_UP times what it leaves.
+__device__ __forceinline__ void cut_pair(float x0, float x1, float scale, float low_scale, uint32_t& high, uint32_t& low) {
+  const f16x2_t h = __builtin_convertvector((hw_f32x2_t{x0 * scale, x1 * scale}), f16x2_t);
+  const f16x2_t l = {(_Float16)__builtin_fmaf((float)h.x, -LOW_UP, x0 * low_scale), (_Float16)__builtin_fmaf((float)h.y, -LOW_UP, x1 * low_scale)};
   high = __builtin_bit_cast(uint32_t, h), low = __builtin_bit_cast(uint32_t, l);
 }
 struct Cut {
   u32x4_t high, low;  // eight halves each
 };
 __device__ __forceinline__ Cut cut(f32x4_t a, f32x4_t b, float scale) {
-  a *= scale, b *= scale;
+  const float low_scale = scale * LOW_UP;
   uint32_t h[4], l[4];
-  cut_pair(a.x, a.y, h[0], l[0]), cut_pair(a.z, a.w, h[1], l[1]);
-  cut_pair(b.x, b.y, h[2], l[2]), cut_pair(b.z, b.w, h[3], l[3]);
+  cut_pair(a.x, a.y, scale, low_scale, h[0], l[0]), cut_pair(a.z, a.w, scale, low_scale, h[1], l[1]);
+  cut_pair(b.x, b.y, scale, low_scale, h[2], l[2]), cut_pair(b.z, b.w, scale, low_scale, h[3], l[3]);
   return Cut{u32x4_t{h[0], h[1], h[2], h[3]}, u32x4_t{l[0], l[1], l[2], l[3]}};
 }
 __device__ __forceinline__ f32x16_t mfma(u32x4_t a, u32x4_t b, f32x16_t c) {
@@ -292,6 +305,12 @@ __device__ __forceinline__ float gelu_tanh_short(float x) {
 __device__ __forceinline__ bool finite(float v) { return (__float_as_uint(v) & 0x7f800000u) != 0x7f800000u; }
 __device__ __forceinline__ float power_of_2(int e) { return __uint_as_float((uint32_t)(e + 127) << 23); }
 
+// From here on up a scaled value's two halves hold it to 2^-23 of itself.  Below, half precision's least step leaves out 2^-37, and the low
+// parts' product 2^-36 of what it is multiplied with (2^15 at most): 1.5 2^-21 a value.  A sum of 4 for each such value of its row and feature is
+// then good to 1.5 2^-23 of itself; one below that is in doubt.
+#define LEAST_WHOLE 0x1p-14f
+#define DOUBT_A_VALUE 4.f
+
 // Ahead of the products: the rows' greatest values, whose exponents say what a row is scaled by (so that its greatest
 // value lies from 2^14 up to 2^15), and A's rows scaled and cut.  A block a row, which stays in registers up to 8,192 columns: first A's, then W's.  A cut row has the place of the
 // row itself: where eight floats were lie eight high halves and eight low ones, up to whole steps of 32 columns.  (A wave a row, read
@@ -301,10 +320,11 @@ struct CutArgs {
   const float* W;
   int M, N, K, lda, ldw, ldc;
   u32x4_t* cut;
-  int* exponents;  // [M], then [N]
+  RowScale* scales;  // [M], then [N]
 };
 __global__ __launch_bounds__(256) void cut_rows_kernel(CutArgs p) {
   __shared__ uint32_t wave_most[4];
+  __shared__ int n_small;
   const int row = blockIdx.x, tid = threadIdx.x;
   const bool is_a = row < p.M;
   const float* from = is_a ? p.A + (size_t)row * p.lda : p.W + (size_t)(row - p.M) * p.ldw;
@@ -334,35 +354,44 @@ __global__ __launch_bounds__(256) void cut_rows_kernel(CutArgs p) {
 #pragma unroll
   for (int d = 32; d; d >>= 1) most = max(most, (uint32_t)__shfl_xor((int)most, d, 64));
   if ((tid & 63) == 0) wave_most[tid >> 6] = most;
+  if (tid == 0) n_small = 0;
   __syncthreads();
   most = max(max(wave_most[0], wave_most[1]), max(wave_most[2], wave_most[3]));
   const int e = (int)(most >> 23);
   const int up = most == 0 || e == 255 ? 0 : min(14 + 127 - e, 126);
-  if (tid == 0) p.exponents[row] = up;
-  if (!is_a) return;
   const float scale = power_of_2(up);
   u32x4_t* to = p.cut + (size_t)row * (p.ldc / 4);
+  int small = 0;
   for (int k0 = 0; k0 < p.ldc; k0 += CHUNK) {
     if (p.K > CHUNK) load(k0);
 #pragma unroll
     for (int i = 0; i < HELD; ++i) {
       const int k = k0 + (tid + 256 * i) * 8;
       if (k >= p.ldc) continue;
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) small += v[i][h][c] != 0.f && fabsf(v[i][h][c] * scale) < LEAST_WHOLE;
+      if (!is_a) continue;
       const Cut c = cut(v[i][0], v[i][1], scale);
       to[k / 4] = c.high, to[k / 4 + 1] = c.low;
     }
   }
+  if (small) atomicAdd(&n_small, small);
+  __syncthreads();
+  if (tid == 0) p.scales[row] = RowScale{up, most == 0 ? -INFINITY : DOUBT_A_VALUE * (float)n_small};
 }
 
 template <typename S>
 __global__ __launch_bounds__(S::THREADS, 2) void gemm_f32_cut_kernel(GemmArgs p) {
   constexpr int BM = S::BM, BN = S::BN, TM = S::TM, TN = S::TN, PA = S::PA, PB = S::PB, STAGES = S::STAGES;
   __shared__ __attribute__((aligned(1024))) float smem[STAGES * S::STAGE_BYTES / 4];
+  __shared__ __attribute__((aligned(16))) RowScale scales[BM + BN];  // the tile's rows', then its features'
   int tm, tn;
   if (!tile_of_block<S::PANEL>((p.M + BM - 1) / BM, (p.N + BN - 1) / BN, tm, tn)) return;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int x = lane & 31, hi = lane >> 5;
-  const int wm = wave >> 1, wn = wave & 1;
+  const int wm = wave / S::WAVES_N, wn = wave % S::WAVES_N;
   const int m0 = tm * BM, n0 = tn * BN;
   const int k_lo = blockIdx.y * p.per_split * 64, k_end = min(p.K, k_lo + p.per_split * 64);
   const int n_steps = (k_end - k_lo + S::STEP - 1) / S::STEP;
@@ -398,10 +427,17 @@ __global__ __launch_bounds__(S::THREADS, 2) void gemm_f32_cut_kernel(GemmArgs p)
       copy16_to_lds(b_buf, piece_of(wave * PB + i) * 4 < left ? b_from[i] : COPY_NOTHING, k4, at + BM * 128 + (wave * PB + i) * 1024);
   };
 
-  // the features' scales
+  static_assert(BM + BN <= S::THREADS, "a scale a thread");
+  if ((int)threadIdx.x < BM + BN) {
+    const int n = n0 + (int)threadIdx.x - BM;
+    RowScale s = {0, -INFINITY};
+    if ((int)threadIdx.x < a_rows) s = p.a_scales[m0 + threadIdx.x];
+    if ((int)threadIdx.x >= BM && n < p.N) s = p.w_scales[n];
+    scales[threadIdx.x] = s;
+  }
   float scale[TN];
 #pragma unroll
-  for (int j = 0; j < TN; ++j) scale[j] = power_of_2(p.w_exponents[min(n0 + (wn * TN + j) * 32 + x, p.N - 1)]);
+  for (int j = 0; j < TN; ++j) scale[j] = power_of_2(p.w_scales[min(n0 + (wn * TN + j) * 32 + x, p.N - 1)].up);
 
   // the products of the high parts, and those with a low part
   f32x16_t acc[TM][TN], low[TM][TN];
@@ -468,37 +504,52 @@ __global__ __launch_bounds__(S::THREADS, 2) void gemm_f32_cut_kernel(GemmArgs p)
   multiply(1);
   copies_arrived<0>();  // (what was asked for beyond the end)
 
-  // A row's sums leave their scales behind.  What is not finite is computed again with the 32-bit instructions, out of the operands
-  // themselves: an infinity's parts would give NaN, and the sums' own infinities and NaN come out as those instructions have them.
-  bool whole = true;
+  // A row's sums leave their scales behind.  What is not finite or in doubt is computed again with the 32-bit instructions, out of the
+  // operands themselves: an infinity's parts would give NaN, and the sums' own infinities and NaN come out as those instructions have them.
+  // (Two sums of every other column, so that each is rounded as seldom as with the instruction of four columns.)
 #pragma unroll
-  for (int i = 0; i < TM; ++i)
+  for (int j = 0; j < TN; ++j) {
+    RowScale w_scale[16];
+    float w_doubt = -INFINITY;
 #pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      acc[i][j] += low[i][j];
-#pragma unroll
-      for (int r = 0; r < 16; ++r) whole = whole && finite(acc[i][j][r]);
+    for (int r = 0; r < 16; ++r) {
+      w_scale[r] = scales[BM + (wn * TN + j) * 32 + 8 * (r >> 2) + 4 * hi + (r & 3)];
+      w_doubt = fmaxf(w_doubt, w_scale[r].doubt);
     }
-  const bool again = __any(!whole);
 #pragma unroll
-  for (int i = 0; i < TM; ++i) {
-    const int m = min(m0 + (wm * TM + i) * 32 + x, p.M - 1);
-    const int down = -p.a_exponents[m];
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      const int nt = n0 + (wn * TN + j) * 32;
-      f32x16_t sum;
-      if (again) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) sum[r] = 0.f;
-        const float* ap = p.A + (size_t)m * p.lda;
-        const float* wp = p.W + (size_t)min(nt + x, p.N - 1) * p.ldw;
-        for (int k = k_lo + hi; k < k_end; k += 2) sum = __builtin_amdgcn_mfma_f32_32x32x2f32(wp[k], ap[k], sum, 0, 0, 0);
-      }
+    for (int i = 0; i < TM; ++i) {
+      const RowScale a_scale = scales[(wm * TM + i) * 32 + x];
+      float least = INFINITY, nothing = 0.f;
+      f32x16_t s;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        const float v = ldexpf(acc[i][j][r], down - p.w_exponents[min(nt + 8 * (r >> 2) + 4 * hi + (r & 3), p.N - 1)]);
-        acc[i][j][r] = again && !finite(acc[i][j][r]) ? sum[r] : v;
+        s[r] = __builtin_fmaf(low[i][j][r], 1.f / LOW_UP, acc[i][j][r]);
+        least = fminf(least, fabsf(s[r]));
+        nothing = __builtin_fmaf(s[r], 0.f, nothing);
+        acc[i][j][r] = ldexpf(s[r], -a_scale.up - w_scale[r].up);
+      }
+      if (__any(!(nothing == 0.f && least >= a_scale.doubt + w_doubt))) {
+        f32x16_t sum[2];
+#pragma unroll
+        for (int r = 0; r < 16; ++r) sum[0][r] = sum[1][r] = 0.f;
+        const float* ap = p.A + (size_t)min(m0 + (wm * TM + i) * 32 + x, p.M - 1) * p.lda;
+        const float* wp = p.W + (size_t)min(n0 + (wn * TN + j) * 32 + x, p.N - 1) * p.ldw;
+        for (int k0 = k_lo; k0 < k_end; k0 += 32) {
+          f32x4_t av[4], wv[4];
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const int k = k0 + 8 * q + 4 * hi;
+            av[q] = wv[q] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+            if (k < k_end) av[q] = *(const f32x4_t*)(ap + k), wv[q] = *(const f32x4_t*)(wp + k);
+          }
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) sum[c & 1] = __builtin_amdgcn_mfma_f32_32x32x2f32(wv[q][c], av[q][c], sum[c & 1], 0, 0, 0);
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r)
+          if (!finite(s[r]) || fabsf(s[r]) < a_scale.doubt + w_scale[r].doubt) acc[i][j][r] = sum[0][r] + sum[1][r];
       }
     }
   }
@@ -805,10 +856,10 @@ static int choose(int M, int N, int K, int variant, int n_splits) {
   double us = 0.0;
   return variant != 0 ? variant : M <= SKF_MAX_ROWS ? 3 : cheapest_shape(M, N, K, n_splits, &us);
 }
-// Floats of memory that gemm_f32_scatter needs for a product of these sizes: its rows cut, and an exponent a row and feature (0: tiles of
+// Floats of memory that gemm_f32_scatter needs for a product of these sizes: its rows cut, and a scale a row and feature (0: tiles of
 // cut operands don't take it).
 extern "C" size_t gemm_f32_room(int M, int N, int K, int variant, int n_splits) {
-  return M > 0 && is_cut(choose(M, N, K, variant, n_splits)) ? (size_t)M * cut_stride(K) + (size_t)M + N : 0;
+  return M > 0 && is_cut(choose(M, N, K, variant, n_splits)) ? (size_t)M * cut_stride(K) + 2 * ((size_t)M + N) : 0;
 }
 
 // variant: 0 = choose, 1 = tiles of 64 x 128, 2 = of 64 x 64, 4 = of 32 x 64, 3 = the kernel for up to
@@ -871,9 +922,9 @@ extern "C" int gemm_f32_scatter(void* out, const void* A, const void* W, const f
   if (is_cut(variant)) {
     if (!room || ((uintptr_t)room & 15) || room_floats < room_wanted)
       FAIL("gemm_f32: tiles of cut operands need %zu floats of aligned memory", room_wanted);
-    int* const exponents = (int*)(room + (size_t)M * cut_stride(K));
-    p.cut = room, p.ldc = cut_stride(K), p.a_exponents = exponents, p.w_exponents = exponents + M;
-    const CutArgs c = {p.A, p.W, M, N, K, lda, ldw, p.ldc, (u32x4_t*)room, exponents};
+    RowScale* const scales = (RowScale*)(room + (size_t)M * cut_stride(K));
+    p.cut = room, p.ldc = cut_stride(K), p.a_scales = scales, p.w_scales = scales + M;
+    const CutArgs c = {p.A, p.W, M, N, K, lda, ldw, p.ldc, (u32x4_t*)room, scales};
     hipLaunchKernelGGL(cut_rows_kernel, dim3((unsigned)(M + N)), dim3(256), 0, stream, c);
     p.through = fits_through_buffer((size_t)M * (n_splits > 1 ? N : ldo) * 4);
     launch(p, variant, stream);

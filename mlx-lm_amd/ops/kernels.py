@@ -543,7 +543,7 @@ def linear(out, a, w, bias=None, gelu=False, accumulate=False, variant=0, scatte
     if call.w.dtype == DT[torch.float32] and not ctx.scratch and (a.shape[0] > F32_FEW_ROWS or variant >= 5):
         # outside a step there is no scratch memory for the rows that the tiles cut (a context of the call's own: others, on other
         # streams, share the bare one)
-        room = torch.empty(4 * (a.shape[0] * ((K + 31) // 32 * 32 + 1) + N) + 4096, dtype=torch.uint8, device=out.device)
+        room = torch.empty(4 * (a.shape[0] * ((K + 31) // 32 * 32 + 2) + 2 * N) + 4096, dtype=torch.uint8, device=out.device)
         scratch = native.EngScratch(room.data_ptr(), room.numel(), 0, 0, 1, 0)
         ctx = native.EngCtx.from_buffer_copy(ctx)
         ctx.scratch = ctypes.pointer(scratch)

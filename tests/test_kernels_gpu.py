@@ -132,11 +132,11 @@ def test_gemm_f32_tiles_at_the_ring_s_edges(M, N, K):
 
 
 def _cut_tolerance(a, w, K):
-    """K roundings of a partial sum, and a cut's: an operand's last bit each (2^-23), the low parts' product (2^-22), half precision's
-    least steps below the rows' greatest values (2^-39)."""
+    """What each output may be off by, in 2^-24 of its products' magnitudes: an operand's last bit each (2), the low parts' product (4), what
+    values far below their rows' greatest lose where the sum is still good (3), and a rounding of the sum every 16 columns, of either sign
+    (the root of their number, twice over).  Without the low halves 1,284 columns are off by three times as much and more."""
     mags = (a.double().abs() @ w.double().abs().t().contiguous()).cpu()
-    least = a.double().abs().amax(1)[:, None].cpu() * w.double().abs().amax(1)[None, :].cpu() * K * 2.0**-38
-    return (K + 10) * 2.0**-24 * mags + least
+    return (11 + 2 * math.sqrt(K / 16)) * 2.0**-24 * mags
 
 
 @pytest.mark.parametrize("M,N,K", [(1, 1, 4), (65, 60, 32), (64, 129, 68), (127, 128, 100), (129, 257, 520), (300, 70, 1284)])
@@ -163,6 +163,54 @@ def test_gemm_f32_cut_operands(M, N, K):
             again = torch.empty(M, N, device=DEV)
             k.linear(again, a, known, variant=variant, splits=splits)
             assert torch.equal(again, wide[:, :N]), (variant, splits)
+
+
+@pytest.mark.parametrize("K", [260, 1280])
+def test_gemm_f32_rows_of_wide_range(K):
+    """Great values that meet zeros or tiny weights, in rows, in features and in both, leave the sums of the others whole, whichever kernel
+    multiplies: one value of 2^8 to 2^100 beside ones and beside normal numbers, columns that fall by 2^60 against weights that
+    rise by as much, rows that are all far below one, K whole and in parts."""
+    k = _k()
+    M, N = 132, 134
+    at = K // 2
+    great = torch.cat([2.0 ** torch.arange(8, 101, 4, device=DEV)] * 6)[:M]
+    fall = torch.logspace(0, -60, K, base=2.0, device=DEV)
+    a, w = _rand((M, K), torch.float32, 10), _rand((N, K), torch.float32, 11)
+    ones = a.clone()
+    ones[:24] = 1.0
+    none, tiny = w.clone(), w.clone()
+    none[:, at], tiny[:, at] = 0.0, 1e-30
+    none[3] = 0.0
+    ones[:, at] = great
+    both_a, both_w = ones.clone(), none.clone()
+    both_a[:, at + 1], both_w[:, at + 1] = 0.0, great[0] * 2.0**40
+    cases = {"rows": (ones, none), "tiny": (ones, tiny), "features": (none, ones), "both": (both_a, both_w),
+             "fall": (a * fall, w * fall.flip(0)), "small rows": (a * 1e-38, w * fall * 1e3)}
+    for name, (a, w) in cases.items():
+        a, w = a.contiguous(), w.contiguous()
+        ref, tol = (a.double() @ w.double().t().contiguous()).cpu(), _cut_tolerance(a, w, K)
+        for variant in (0, 5, 6, 7):
+            for splits in (None, 2):
+                out = torch.empty(a.shape[0], w.shape[0], device=DEV)
+                k.linear(out, a, w, variant=variant, splits=splits)
+                over = ((out.double().cpu() - ref).abs() - tol).max().item()
+                assert over <= 2.0**-140, (name, variant, splits, over)  # (some denormal steps)
+
+
+@pytest.mark.parametrize("M,N,K", [(100, 300, 768), (300, 130, 1280), (128, 128, 5120)])
+def test_gemm_f32_cut_operands_are_no_further_off(M, N, K):
+    """Rows as models have them (normal numbers, and what a GELU leaves of them, a tenth of it tiny): the error against 64 bits, by
+    2-norm, is no larger than that of the 32-bit instructions' tiles."""
+    k = _k()
+    for name, a in (("normal", _rand((M, K), torch.float32, 10)), ("gelu", plain.gelu_tanh(_rand((M, K), torch.float32, 11, 4.0)))):
+        w = _rand((N, K), torch.float32, 12, 0.02)
+        ref = a.double() @ w.double().t().contiguous()
+        off = {}
+        for variant in (1, 5, 6, 7):
+            out = torch.empty(M, N, device=DEV)
+            k.linear(out, a, w, variant=variant)
+            off[variant] = (out.double() - ref).norm().item()
+        assert max(off[5], off[6], off[7]) <= off[1], (name, off)
 
 
 def test_gemm_f32_weights_that_are_changed_in_place():
