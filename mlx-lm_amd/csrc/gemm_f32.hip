@@ -856,10 +856,19 @@ static int choose(int M, int N, int K, int variant, int n_splits) {
   double us = 0.0;
   return variant != 0 ? variant : M <= SKF_MAX_ROWS ? 3 : cheapest_shape(M, N, K, n_splits, &us);
 }
-// Floats of memory that gemm_f32_scatter needs for a product of these sizes: its rows cut, and a scale a row and feature (0: tiles of
-// cut operands don't take it).
+// Rows that are cut at once: up to 256 MB of them (a prompt of 8,192 rows of 6,400 has 210), so that the room does not grow with the
+// rows and a grid of one block a row and feature holds them.
+static inline int cut_at_once(int M, int K) {
+  const int most = ((64 << 20) / cut_stride(K) + 127) / 128 * 128;
+  return M < most ? M : most;
+}
+#define CUT_BLOCKS (1 << 23)  // features whose scales a launch finds at most (a grid holds less than 2^32 threads)
+// Floats of memory that gemm_f32_scatter needs for a product of these sizes: as many rows as are cut at once, and a scale a row and
+// feature (0: tiles of cut operands don't take it).
 extern "C" size_t gemm_f32_room(int M, int N, int K, int variant, int n_splits) {
-  return M > 0 && is_cut(choose(M, N, K, variant, n_splits)) ? (size_t)M * cut_stride(K) + 2 * ((size_t)M + N) : 0;
+  if (M <= 0 || !is_cut(choose(M, N, K, variant, n_splits))) return 0;
+  const size_t rows = cut_at_once(M, K);
+  return rows * cut_stride(K) + 2 * (rows + N);
 }
 
 // variant: 0 = choose, 1 = tiles of 64 x 128, 2 = of 64 x 64, 4 = of 32 x 64, 3 = the kernel for up to
@@ -922,12 +931,23 @@ extern "C" int gemm_f32_scatter(void* out, const void* A, const void* W, const f
   if (is_cut(variant)) {
     if (!room || ((uintptr_t)room & 15) || room_floats < room_wanted)
       FAIL("gemm_f32: tiles of cut operands need %zu floats of aligned memory", room_wanted);
-    RowScale* const scales = (RowScale*)(room + (size_t)M * cut_stride(K));
-    p.cut = room, p.ldc = cut_stride(K), p.a_scales = scales, p.w_scales = scales + M;
-    const CutArgs c = {p.A, p.W, M, N, K, lda, ldw, p.ldc, (u32x4_t*)room, scales};
-    hipLaunchKernelGGL(cut_rows_kernel, dim3((unsigned)(M + N)), dim3(256), 0, stream, c);
-    p.through = fits_through_buffer((size_t)M * (n_splits > 1 ? N : ldo) * 4);
-    launch(p, variant, stream);
+    const int rows = cut_at_once(M, K);
+    RowScale* const scales = (RowScale*)(room + (size_t)rows * cut_stride(K));
+    p.cut = room, p.ldc = cut_stride(K), p.a_scales = scales, p.w_scales = scales + rows;
+    for (int m = 0; m < M; m += rows) {
+      p.M = M - m < rows ? M - m : rows;
+      // (the features' scales lie behind those of the first rows, which are as many as any that follow)
+      CutArgs c = {p.A, p.W, p.M, m ? 0 : N < CUT_BLOCKS ? N : CUT_BLOCKS, K, lda, ldw, p.ldc, (u32x4_t*)room, scales};
+      hipLaunchKernelGGL(cut_rows_kernel, dim3((unsigned)(c.M + c.N)), dim3(256), 0, stream, c);
+      for (int n = c.N; m == 0 && n < N; n += c.N) {
+        c.M = 0, c.N = N - n < CUT_BLOCKS ? N - n : CUT_BLOCKS, c.W = p.W + (size_t)n * ldw, c.scales = scales + rows + n;
+        hipLaunchKernelGGL(cut_rows_kernel, dim3((unsigned)c.N), dim3(256), 0, stream, c);
+      }
+      p.through = fits_through_buffer((size_t)p.M * (n_splits > 1 ? N : ldo) * 4);
+      launch(p, variant, stream);
+      p.A += (size_t)p.M * lda, p.out += (size_t)p.M * ldo;
+      if (n_splits > 1) p.ws += (size_t)p.M * N;
+    }
     CHECK_LAUNCH("gemm_f32");
     return 0;
   }

@@ -229,6 +229,28 @@ def test_gemm_f32_weights_that_are_changed_in_place():
             assert torch.equal(out, want), (by, variant)
 
 
+def test_gemm_f32_cut_operands_in_several_rounds():
+    """More rows than are cut at once: the room stays 256 MB, and every row has the bits that it has in a product of few, K whole and in
+    parts, with what the epilogue adds."""
+    k = _k()
+    M, N, K = 66_000, 40, 1024
+    a, w, bias = torch.randn(M, K, device=DEV), _rand((N, K), torch.float32, 11), _rand((N,), torch.float32, 12)
+    from mlx_lm_amd.ops import build
+
+    room = build.load("gemm_f32").gemm_f32_room
+    room.restype = ctypes.c_size_t
+    for variant in (5, 6, 7):
+        assert (1 << 26) <= room(M, N, K, variant, 1) < (1 << 26) + 2 * (M + N) + 128 * K, variant
+        assert room(2_000_000_000, N, 16_384, variant, 1) < (1 << 26) + (1 << 22), variant
+        for splits in (None, 2):
+            out = torch.full((M, N), 0.5, device=DEV)
+            k.linear(out, a, w, bias, accumulate=True, variant=variant, splits=splits)
+            for first in (0, 65_480, 65_536, M - 100):
+                part = torch.full((100, N), 0.5, device=DEV)
+                k.linear(part, a[first : first + 100], w, bias, accumulate=True, variant=variant, splits=splits)
+                assert torch.equal(out[first : first + 100], part), (variant, splits, first)
+
+
 def test_gemm_f32_cut_operands_that_are_not_finite():
     """Infinities and NaN come out as sums of products have them, sums beyond the greatest float as infinities, and what else is in
     their tiles stays as it was, bit by bit."""
