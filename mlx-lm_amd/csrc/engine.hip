@@ -433,6 +433,24 @@ extern "C" int eng_wants_packed_rows(const EngCtx* ctx, const EngWeight* w, int 
   return wants_packed(ctx, n_rows, w) ? 1 : 0;
 }
 
+// Into how many parts a float32 product splits K: where a matrix gives fewer blocks than there are compute units, or a last round of
+// few, K goes in parts, and the same second kernels add them up as for bfloat16.  (`fused`: into the next norm)
+static int f32_parts(const EngCtx* ctx, int M, int N, int K, int variant, int splits, bool fused, int* n_splits) {
+  *n_splits = 1;
+  if (!(variant == 0 || (variant == 3 && M <= F32_FEW_ROWS) || splits != 0)) return 0;
+  if (splits == 0)
+    QUERY(k_gemm_f32_splits, *n_splits, M, N, K, fused ? 1 : 0, ctx->force_splits);
+  else
+    *n_splits = split_count((K + 63) / 64, splits);
+  if (*n_splits > 1) {
+    const size_t most = ctx->split_ws ? ctx->split_ws_floats / ((size_t)M * N) : 0;
+    if ((size_t)*n_splits > most) *n_splits = (int)most;
+    if (*n_splits > 1) *n_splits = split_count((K + 63) / 64, *n_splits);
+  }
+  if (*n_splits < 1) *n_splits = 1;
+  return 0;
+}
+
 // `gelu`: the activation code of the epilogue (0 none, 1 tanh-GELU, 2 squared ReLU).
 static int linear(EngCtx* ctx, const EngMat& out, const EngValue& a, const EngWeight& w, const float* bias,
                   int gelu, bool accumulate, int variant, const EngScatter* sc, int splits,
@@ -524,34 +542,21 @@ static int linear(EngCtx* ctx, const EngMat& out, const EngValue& a, const EngWe
     }
   }
   if (w.dtype == DT_F32) {
-    // Where a matrix gives fewer blocks than there are compute units, or a last round of few, K goes
-    // in parts, and the same second kernels add them up as for bfloat16.
     int n_splits = 1;
-    if (variant == 0 || (variant == 3 && M <= F32_FEW_ROWS) || splits != 0) {
-      const int fused = (accumulate && pending && pending->allowed) ? 1 : 0;
-      if (splits == 0)
-        QUERY(k_gemm_f32_splits, n_splits, M, N, K, fused, ctx->force_splits);
-      else
-        n_splits = split_count((K + 63) / 64, splits);
-      if (n_splits > 1) {
-        const size_t most = ws ? ws_floats / ((size_t)M * N) : 0;
-        if ((size_t)n_splits > most) n_splits = (int)most;
-        if (n_splits > 1) n_splits = split_count((K + 63) / 64, n_splits);
-      }
-      if (n_splits < 1) n_splits = 1;
-      if (n_splits > 1 && pending) TRY(settle(ctx, pending));  // the workspace is about to be written again
-    }
+    TRY(f32_parts(ctx, M, N, K, variant, splits, accumulate && pending && pending->allowed, &n_splits));
+    if (n_splits > 1 && pending) TRY(settle(ctx, pending));  // the workspace is about to be written again
     // (few rows' keys and values go to their pages from the product's own epilogue, others from the finished rows, below: also
     // columns that the pages' heads do not take all of)
     int scatters = 0;
     if (sc && (variant == 0 || variant == 3) && sc->n_kv_heads * sc->head_dim == sc->kv_width)
       QUERY(k_gemm_f32_scatters, scatters, M, n_splits);
     const EngScatter* own = scatters ? sc : nullptr;
-    // (rows that the tiles want cut are cut into scratch memory, which the next launches of the stream may have again)
+    // (rows that the tiles want cut are cut into scratch memory, which the next launches of the stream may have again; without any,
+    // other tiles take them)
     EngMat room = {};
     const size_t mark = ctx->scratch ? ctx->scratch->offset : 0;
     size_t room_floats = 0;
-    QUERY(k_gemm_f32_room, room_floats, M, N, K, variant, n_splits);
+    if (ctx->scratch || variant != 0) QUERY(k_gemm_f32_room, room_floats, M, N, K, variant, n_splits);
     if (room_floats) TRY(take(ctx, (int)((room_floats + 1023) / 1024), 1024, DT_F32, &room));
     KERNEL(k_gemm_f32, ctx, out.p, A.p, w.w, bias, M, N, K, A.ld, w.ldw, out.ld, flags, variant, n_splits,
            n_splits > 1 ? ws : nullptr, n_splits > 1 ? ws_floats : (size_t)0, own ? own->k : nullptr, own ? own->v : nullptr,
@@ -609,6 +614,16 @@ static int linear(EngCtx* ctx, const EngMat& out, const EngValue& a, const EngWe
 extern "C" int eng_linear(EngCtx* ctx, const EngLinear* c, EngPending* pending) {
   return linear(ctx, c->out, c->a, c->w, c->bias, c->gelu, c->accumulate != 0, c->variant, c->scatter,
                 c->splits, pending, c->out_packed != 0);
+}
+
+// Bytes of scratch memory that eng_linear takes for the rows of this product, with a context that has some.
+extern "C" size_t eng_linear_room(const EngCtx* ctx, const EngLinear* c, const EngPending* pending) {
+  const int M = c->a.m.rows, K = c->a.m.cols, N = c->w.N;
+  int n_splits = 1;
+  if (c->w.dtype != DT_F32 || M <= 0 || N <= 0 || K <= 0) return 0;
+  if (f32_parts(ctx, M, N, K, c->variant, c->splits, c->accumulate && pending && pending->allowed, &n_splits)) return 0;
+  auto room = k_gemm_f32_room.get();
+  return room ? (room(M, N, K, c->variant, n_splits) + 1023) / 1024 * 4096 : 0;
 }
 
 // ---------------------------------------------------------------------------

@@ -765,10 +765,10 @@ static double price(const F32Price& s, int M, int N, int K, int n_splits) {
   return s.base + s.tile * (full + (left ? 1 : 0)) + chunks * (full * s.chunk[s.per_cu - 1] + (left ? s.chunk[left - 1] : 0.0)) +
          2.3e-6 * M * K;
 }
-static int cheapest_shape(int M, int N, int K, int n_splits, double* us) {
+static int cheapest_shape(int M, int N, int K, int n_splits, double* us, bool cuts = true) {
   int variant = 0;
   for (const F32Price& s : F32_PRICES) {
-    if (is_cut(s.variant) && K < CUT_FROM_K) continue;
+    if (is_cut(s.variant) && (K < CUT_FROM_K || !cuts)) continue;
     const double t = price(s, M, N, K, n_splits) * (is_cut(s.variant) ? 1.04 : 1.0);  // (to be ahead for certain)
     if (!variant || t < *us) variant = s.variant, *us = t;
   }
@@ -852,9 +852,9 @@ static inline bool fits_tiles(int lda, int ldw, int K, bool cut) {
   return (cut ? fits_copy_buffer((size_t)128 * cut_stride(K) * 4) : fits_copy_buffer(((size_t)127 * lda + K) * 4)) &&
          fits_copy_buffer(((size_t)127 * ldw + K) * 4);
 }
-static int choose(int M, int N, int K, int variant, int n_splits) {
+static int choose(int M, int N, int K, int variant, int n_splits, bool cuts = true) {
   double us = 0.0;
-  return variant != 0 ? variant : M <= SKF_MAX_ROWS ? 3 : cheapest_shape(M, N, K, n_splits, &us);
+  return variant != 0 ? variant : M <= SKF_MAX_ROWS ? 3 : cheapest_shape(M, N, K, n_splits, &us, cuts);
 }
 // Rows that are cut at once: up to 256 MB of them (a prompt of 8,192 rows of 6,400 has 210), so that the room does not grow with the
 // rows and a grid of one block a row and feature holds them.
@@ -919,7 +919,7 @@ extern "C" int gemm_f32_scatter(void* out, const void* A, const void* W, const f
     p.block_table = block_table, p.max_blocks = max_blocks, p.token_req = token_req, p.positions = positions;
     p.q_width = q_width, p.kv_width = kv_width, p.head_dim = head_dim, p.page_size = page_size;
   }
-  variant = choose(M, N, K, variant, n_splits);
+  variant = choose(M, N, K, variant, n_splits, room != nullptr);  // (0 without room: not those that need it)
   if (variant != 3 && p.per_split * (n_splits - 1) * SKF_CHUNK >= K) FAIL("gemm_f32: %d parts of K=%d leave one empty", n_splits, K);
   if (variant == 3 && M > SKF_MAX_ROWS)
     FAIL("gemm_f32: the kernel for few rows takes at most %d, got %d", SKF_MAX_ROWS, M);

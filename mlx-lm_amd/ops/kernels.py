@@ -540,13 +540,19 @@ def linear(out, a, w, bias=None, gelu=False, accumulate=False, variant=0, scatte
         _fail(f"linear: unknown activation {activation!r} (known: {sorted(k for k in ACTIVATIONS if k)})")
     code = ACTIVATIONS[activation] or int(bool(gelu))
     call.gelu, call.accumulate, call.variant, call.splits = code, int(accumulate), int(variant), int(splits or 0)
-    if call.w.dtype == DT[torch.float32] and not ctx.scratch and (a.shape[0] > F32_FEW_ROWS or variant >= 5):
-        # outside a step there is no scratch memory for the rows that the tiles cut (a context of the call's own: others, on other
-        # streams, share the bare one)
-        room = torch.empty(4 * (a.shape[0] * ((K + 31) // 32 * 32 + 2) + 2 * N) + 4096, dtype=torch.uint8, device=out.device)
-        scratch = native.EngScratch(room.data_ptr(), room.numel(), 0, 0, 1, 0)
-        ctx = native.EngCtx.from_buffer_copy(ctx)
-        ctx.scratch = ctypes.pointer(scratch)
+    if call.w.dtype == DT[torch.float32] and not ctx.scratch and (a.shape[0] > F32_FEW_ROWS or variant):
+        # rows that the tiles cut need scratch memory: the step's in its Python parts, elsewhere the call's own (in a context of the
+        # call's own: others, on other streams, share the bare one)
+        nbytes = L.eng_linear_room(ctypes.byref(ctx), ctypes.byref(call), ctypes.byref(pending.c) if pending is not None else None)
+        if nbytes:
+            step = native.step_of_part()
+            ctx = native.EngCtx.from_buffer_copy(ctx)
+            if step is not None and step._scratch.buffer.device == out.device and step.c.stream == ctx.stream:
+                ctx.scratch = step.c.scratch
+            else:
+                room = torch.empty(nbytes, dtype=torch.uint8, device=out.device)
+                scratch = native.EngScratch(room.data_ptr(), room.numel(), 0, 0, 1, 0)
+                ctx.scratch = ctypes.pointer(scratch)
     rc = L.eng_linear(ctypes.byref(ctx), ctypes.byref(call), ctypes.byref(pending.c) if pending is not None else None)
     native.check(rc, "linear")
     return out

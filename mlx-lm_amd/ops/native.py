@@ -10,6 +10,7 @@ needed, builds) a kernel library when the native side first asks for one of its 
 """
 
 import ctypes
+import threading
 import weakref
 from ctypes import POINTER, Structure, byref, c_char_p, c_float, c_int, c_long, c_size_t, c_void_p
 
@@ -114,6 +115,7 @@ _raised = []  # an exception a hook caught, to be raised again where the native 
 _py_parts = weakref.WeakValueDictionary()  # id -> part, for callback parts
 _next_id = [1]
 _running = []  # the StepContext of each native call in progress, innermost last
+_part = threading.local()  # .step: the StepContext whose Python part this thread runs
 
 
 class NativeError(RuntimeError, ValueError):
@@ -137,7 +139,11 @@ def _callback(part_id, method, cctx, call):
             ctx._scratch.grow(call.contents.nbytes)
             return 0
         part = _py_parts[part_id]
-        run_python_part(part, method, ctx, call.contents)
+        outer, _part.step = getattr(_part, "step", None), ctx
+        try:
+            run_python_part(part, method, ctx, call.contents)
+        finally:
+            _part.step = outer
         return 0
     except BaseException as e:  # noqa: BLE001
         _raised.append(e)
@@ -182,6 +188,7 @@ def lib():
         "eng_head_forward": (c_int, [P, POINTER(EngCtx), POINTER(EngValue), POINTER(EngMat)]),
         "eng_settle": (c_int, [POINTER(EngCtx)]),
         "eng_linear": (c_int, [POINTER(EngCtx), POINTER(EngLinear), POINTER(EngPending)]),
+        "eng_linear_room": (c_size_t, [POINTER(EngCtx), POINTER(EngLinear), POINTER(EngPending)]),
         "eng_linear_norms_itself": (c_int, [POINTER(EngCtx), c_int, c_int, c_int, c_int, c_int]),
         "eng_pending_settle": (c_int, [POINTER(EngCtx), POINTER(EngPending)]),
         "eng_pending_can_norm": (c_int, [POINTER(EngPending), POINTER(EngMat)]),
@@ -241,6 +248,11 @@ def made(handle, what):
     if not handle:
         check(1, what)
     return handle
+
+
+def step_of_part():
+    """The ``StepContext`` of the step whose Python part this thread is running, or ``None``."""
+    return getattr(_part, "step", None)
 
 
 class running:

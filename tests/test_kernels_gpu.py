@@ -251,6 +251,32 @@ def test_gemm_f32_cut_operands_in_several_rounds():
                 assert torch.equal(out[first : first + 100], part), (variant, splits, first)
 
 
+def test_gemm_f32_takes_room_only_for_rows_that_are_cut():
+    """A product outside a step allocates what its tiles cut and nothing where they do not cut; a context without scratch memory
+    gets tiles that need none."""
+    k = _k()
+    from mlx_lm_amd.ops import native
+
+    def allocates(M, N, K, **kw):
+        a, w, out = torch.ones(M, K, device=DEV), torch.ones(N, K, device=DEV), torch.empty(M, N, device=DEV)
+        before = torch.cuda.memory_stats()["allocation.all.allocated"]
+        k.linear(out, a, w, **kw)
+        n = torch.cuda.memory_stats()["allocation.all.allocated"] - before
+        assert (out == K).all()
+        return n
+
+    assert allocates(1050, 5120, 1280) == 1
+    assert allocates(70, 40, 512, variant=5) == 1
+    for shape, kw in (((1050, 512, 128), {}), ((70, 40, 512), {}), ((64, 5120, 1280), {}), ((1050, 5120, 1280), {"variant": 1}),
+                      ((300, 100, 512), {"variant": 2, "splits": 2})):
+        assert allocates(*shape, **kw) == 0, (shape, kw)
+    a, w, out = torch.ones(1050, 1280, device=DEV), torch.ones(5120, 1280, device=DEV), torch.empty(1050, 5120, device=DEV)
+    call = native.EngLinear()
+    call.w, call.a.m, call.out = k.weight_struct(w), native.mat(a), native.mat(out)
+    native.check(native.lib().eng_linear(ctypes.byref(k.bare_context()), ctypes.byref(call), None))
+    assert (out == 1280).all()
+
+
 def test_gemm_f32_cut_operands_that_are_not_finite():
     """Infinities and NaN come out as sums of products have them, sums beyond the greatest float as infinities, and what else is in
     their tiles stays as it was, bit by bit."""

@@ -460,6 +460,33 @@ def test_a_mixer_alone(tmp_path, name, dtype):
     eng.cache.check()
 
 
+def test_cut_rows_lie_in_the_step_s_scratch_memory(models, monkeypatch):
+    """A step's float32 products that cut their rows (here all of more than 64) take the room from the step: none of them allocates,
+    eager or recorded, and the logits stay."""
+    from mlx_lm_amd.ops import kernels
+
+    folder, config, weights = models["A"]
+    tokens = helpers.random_tokens(90, config["vocab"], seed=1)
+    want = _plain(weights, config, tokens, "float32")
+    eng = _engine(folder, "float32", n_pages=16)
+    linear, grew = kernels.linear, []
+
+    def cut(out, a, w, *args, **kw):
+        if a.shape[0] > 64:
+            kw["variant"] = 5
+        before = torch.cuda.memory_stats()["allocation.all.allocated"]
+        linear(out, a, w, *args, **kw)
+        grew.append(torch.cuda.memory_stats()["allocation.all.allocated"] - before)
+
+    monkeypatch.setattr(kernels, "linear", cut)
+    _close(_run(eng, "first", tokens, [90]), want, "float32", "first")  # (scratch memory grows here)
+    assert len(grew) >= 6
+    for again in range(4):
+        grew.clear()
+        _close(_run(eng, "again", tokens, [90]), want, "float32", f"again {again}")
+        assert not any(grew), (again, grew)
+
+
 def test_the_plain_side_notices_what_the_comparisons_are_for(models):
     """With these weights a key head taken for another, the maps swapped, the convolution's taps
     in reverse, a rotation of the wrong layout, a decay per head instead of per channel or a
