@@ -147,7 +147,7 @@ static Entry<int (*)(int, int)> k_gemm_f32_scatters("gemm_f32", "gemm_f32_scatte
 static Entry<size_t (*)(int, int, int, int, int)> k_gemm_f32_room("gemm_f32", "gemm_f32_room");
 static Entry<fn_int5> k_gemm_f32_splits("gemm_f32", "gemm_f32_splits");
 static Entry<fn_gemm_bf16> k_gemm_bf16("gemm_bf16", "gemm_bf16_scatter");
-static Entry<fn_int5> k_gemm_bf16_splits("gemm_bf16", "gemm_bf16_splits");
+static Entry<int (*)(int, int, int, int, int, size_t)> k_gemm_bf16_parts("gemm_bf16", "gemm_bf16_parts");
 static Entry<fn_gemm_decode> k_gemm_decode("gemm_bf16_decode", "gemm_bf16_decode");
 static Entry<fn_int4> k_decode_takes("gemm_bf16_decode", "gemm_bf16_decode_takes");
 static Entry<int (*)()> k_decode_few_blocks("gemm_bf16_decode", "gemm_bf16_decode_few_blocks");
@@ -579,7 +579,7 @@ static int linear(EngCtx* ctx, const EngMat& out, const EngValue& a, const EngWe
       if (splits == 0) {
         // (the second kernel stands in for one that would run anyway: the next norm, or the cache write)
         const int fused = (accumulate && pending && pending->allowed) || sc != nullptr;
-        QUERY(k_gemm_bf16_splits, n_splits, M, N, K, fused, ctx->force_splits);
+        QUERY(k_gemm_bf16_parts, n_splits, M, N, K, fused, ctx->force_splits, ws ? ws_floats : (size_t)0);
       } else {
         n_splits = split_count(n_blocks, splits);
       }

@@ -721,39 +721,62 @@ static int readers_of(int variant, int M, int N, int n_splits, bool packed) {
   return idle < 1 || idle < enough * columns ? 0 : idle < most ? idle : most;
 }
 
+// Whether they keep up with the tiles, so that those cost what fed ones do.  Tiles of 64 rows: where there is a reader for each column (65 x 10,880 x 2,048, ten
+// for eleven, 0.42 us a k-block; 160 x 8,192 x 2,048, eight for eight, 0.35).  Of 32 rows, which take half as long: from five readers for four columns on
+// (65 x 8,192 x 6,144, eight for eight, 0.31; 100 x 6,144 x 2,048, eight for six, 0.25; 65 x 6,400 x 1,600, thirteen for six, 0.23); with three or fewer, as parts
+// of K leave them, from nine for four on (65 x 1,600 x 6,400 in four parts, three for five thirds, 0.31; 100 x 1,280 x 5,120 in four, three for five quarters, 0.21) or
+// two for one (80 x 768 x 3,072 in six, 0.22).  Of 128 rows: up to the columns that the most readers have (160 x 8,192 x 2,048, 0.39; 65 x 10,880 x 2,048, eight for eleven, 0.48).
+static bool readers_keep_up(int variant, int M, int N, int n_splits) {
+  if (!readers_of(variant, M, N, n_splits, true)) return false;
+  int idle = 0;
+  double columns = 0.0;
+  if (variant == 5) {
+    idle_units<Tile64x128>(M, N, n_splits, &idle, &columns);
+    return idle >= columns;
+  }
+  if (variant == 6) {
+    idle_units<Tile32x128>(M, N, n_splits, &idle, &columns);
+    return idle >= (idle > 3 ? 1.25 : columns > 1.0 ? 2.25 : 2.0) * columns;
+  }
+  idle_units<Tile128>(M, N, n_splits, &idle, &columns);
+  return columns <= 10.0;
+}
+
 // What a shape costs, in microseconds: `launch` once, `tile` for each round of tiles on a CU and `kblock` for each k-block of it, `pair`
-// a k-block where two blocks share the CU (shapes that fit twice); where CUs that have no tile read weights ahead, `fed_tile` and
-// `fed` instead.  `full`: what a k-block costs at least where all CUs ask the L2s for one at once (fewer in proportion).  Fitted to the
-// times of 18 numbers of rows from 65 to 2,048 against 18 matrices of widths 768 to 2,048, K up to
-// 6,400, weights from 2.5 GB of memory, each with K in 1 to 8 parts; the shape and parts chosen from these prices are within 1.2 % of the best on average (at
-// worst 1.18 times; the prices before the readers, 6.7 % and 1.76).
+// a k-block where two blocks share the CU (shapes that fit twice); where CUs that have no tile read weights ahead and keep up, `fed_tile` and
+// `fed` instead.  `full`: what a k-block costs at least where all CUs ask the L2s for one at once (fewer in proportion); `full_alone` with K whole and nobody who
+// reads ahead (128 x 128, K whole: 500 x 8,192 x 6,144 0.60, 2,048 x 2,048 x 5,440 0.55; 900 x 1,280 x 5,120 in three parts, which are stored as they are, 0.77).
+// Fitted to the times of 18 numbers of rows from 65 to 2,048 against 18 matrices of widths 768 to 2,048, K up to
+// 6,400, weights from 2.5 GB of memory, each with K in 1 to 8 parts; the shape and parts chosen from these prices are within 0.6 % of the best on average (at
+// worst 1.13 times; the prices before the readers, 6.7 % and 1.76).  Fifteen numbers of rows against fourteen matrices up to 16,384 x 8,192: 1.1 %, at worst 1.2 times.
 struct TilePrice {
   int variant, bm, bn, per_cu;
   double launch, tile, kblock, pair;
   bool splits;  // K may be split over blocks
-  double fed_tile, fed, full;
+  double fed_tile, fed, full, full_alone;
 };
 static const TilePrice TILE_PRICES[] = {
-    {3, Tile256::BM, Tile256::BN, 1, 0.0, 7.69, 1.042, 0.0, false, 0.0, 0.0, 0.0},
-    {4, Tile256x192::BM, Tile256x192::BN, 1, 0.0, 6.9, 0.885, 0.0, false, 0.0, 0.0, 0.0},
-    {8, Tile256x128::BM, Tile256x128::BN, 1, 0.0, 6.1, 0.65, 0.0, false, 0.0, 0.0, 0.0},
-    {1, Tile128::BM, Tile128::BN, 1, 0.21, 4.09, 0.499, 0.0, true, 4.25, 0.331, 0.686},
-    {5, Tile64x128::BM, Tile64x128::BN, 2, 3.11, 1.32, 0.363, 0.708, true, 0.49, 0.32, 0.403},
-    {6, Tile32x128::BM, Tile32x128::BN, 2, 2.83, 1.54, 0.27, 0.516, true, 0.83, 0.202, 0.316},
+    {3, Tile256::BM, Tile256::BN, 1, 0.0, 7.69, 1.042, 0.0, false, 0.0, 0.0, 0.0, 0.0},
+    {4, Tile256x192::BM, Tile256x192::BN, 1, 0.0, 6.9, 0.885, 0.0, false, 0.0, 0.0, 0.0, 0.0},
+    {8, Tile256x128::BM, Tile256x128::BN, 1, 0.0, 6.1, 0.65, 0.0, false, 0.0, 0.0, 0.0, 0.0},
+    {1, Tile128::BM, Tile128::BN, 1, 0.21, 4.09, 0.499, 0.0, true, 4.25, 0.331, 0.686, 0.6},
+    {5, Tile64x128::BM, Tile64x128::BN, 2, 3.11, 1.32, 0.363, 0.708, true, 0.49, 0.32, 0.403, 0.403},
+    {6, Tile32x128::BM, Tile32x128::BN, 2, 2.83, 1.54, 0.27, 0.516, true, 0.83, 0.202, 0.316, 0.316},
 };
 // Up to 64 rows, what the kernels for few rows leave (row-major weights, a longer K than they hold): no readers.
 static const TilePrice FEW_PRICES[] = {
-    {1, Tile128::BM, Tile128::BN, 1, 0.0, 4.33, 0.49, 0.0, true, 0.0, 0.0, 0.0},
-    {5, Tile64x128::BM, Tile64x128::BN, 2, 0.52, 2.81, 0.38, 0.77, true, 0.0, 0.0, 0.0},
-    {6, Tile32x128::BM, Tile32x128::BN, 2, 1.81, 1.98, 0.33, 0.52, true, 0.0, 0.0, 0.0},
+    {1, Tile128::BM, Tile128::BN, 1, 0.0, 4.33, 0.49, 0.0, true, 0.0, 0.0, 0.0, 0.0},
+    {5, Tile64x128::BM, Tile64x128::BN, 2, 0.52, 2.81, 0.38, 0.77, true, 0.0, 0.0, 0.0, 0.0},
+    {6, Tile32x128::BM, Tile32x128::BN, 2, 1.81, 1.98, 0.33, 0.52, true, 0.0, 0.0, 0.0, 0.0},
 };
 
 static double price(const TilePrice& s, int M, int N, int K, int n_splits) {
   const long tiles = (long)((M + s.bm - 1) / s.bm) * ((N + s.bn - 1) / s.bn), cus = n_compute_units(), per_die = cus / N_DIES;
   const long n = ((tiles + N_DIES - 1) / N_DIES * n_splits + per_die - 1) / per_die;  // the busiest CU
   const int k_blocks = ((K + BK - 1) / BK + n_splits - 1) / n_splits;
-  const double least = s.full * (tiles * n_splits < cus ? tiles * n_splits : cus) / cus;
-  if (readers_of(s.variant, M, N, n_splits, true)) return s.launch + s.fed_tile + k_blocks * (s.fed > least ? s.fed : least);
+  const bool fed = readers_keep_up(s.variant, M, N, n_splits);
+  const double least = (n_splits == 1 && !fed ? s.full_alone : s.full) * (tiles * n_splits < cus ? tiles * n_splits : cus) / cus;
+  if (fed) return s.launch + s.fed_tile + k_blocks * (s.fed > least ? s.fed : least);
   if (n == 1) return s.launch + s.tile + k_blocks * (s.kblock > least ? s.kblock : least);
   if (s.per_cu == 1) return s.launch + n * (s.tile + k_blocks * s.kblock);
   return s.launch + (n / 2) * (s.tile + k_blocks * s.pair) + (n % 2) * (s.tile + k_blocks * s.kblock);
@@ -791,29 +814,41 @@ static bool pairs_of_blocks(int M, int N) {
 // are priced: the walk as above, the second kernel as a launch plus its bytes at 3 TB/s.
 // `fused`: the second kernel stands in for one that would run anyway (the norm that follows a
 // sum into the residual stream, the write of keys and values into their pages), so it costs only
-// the extra bytes.  A part keeps three k-blocks or more, and more parts have to be 2 % cheaper.
-// `force` > 0 asks for that many parts wherever K has them (for tests of small sizes).
-extern "C" int gemm_bf16_splits(int M, int N, int K, int fused, int force) {
+// the extra bytes.  A part keeps three k-blocks or more, and more parts have to be 2 % cheaper.  Where the second kernel would run anyway, more parts
+// of twelve k-blocks or more that all have a unit to themselves may cost 5 % more by these prices: in steps they are level or ahead (GPT-2 XL, us a step, 72 rows of
+// 1,600 x 6,400 in 5 / 6 / 8 parts 2,632 / 2,630 / 2,630, 200 rows in two and four 3,200 and 3,156; large, 260 rows of 1,280 x 5,120 in two and three 2,316 and
+// 2,206), at worst 0.7 % behind (150 rows of 1,600 x 6,400 in four and six 2,887 and 2,908).
+// `force` > 0 asks for that many parts wherever K has them (for tests of small sizes).  `ws_floats`: what the parts' sums have to fit.
+extern "C" int gemm_bf16_parts(int M, int N, int K, int fused, int force, size_t ws_floats) {
   if (M < TILE_MIN_ROWS) return 1;
   const int n_blocks = (K + BK - 1) / BK;
   int best = 1;
   if (force > 0) {
     best = force < n_blocks ? force : n_blocks;
   } else {
-    double best_us = 0.0;
-    // (a long K of few rows goes in eight parts or more: five to eight are within 3 % of each other at 65 to 80 rows of 1,600 x 6,400)
-    const int first = M > FEW_ROWS && M <= 96 && n_blocks >= 96 ? 8 : 1;
-    for (int s = first; s <= 16 && s <= (n_blocks >= 3 ? n_blocks / 3 : 1); ++s) {
+    constexpr int MOST = 16;
+    const size_t fit = ws_floats / ((size_t)M * N);
+    const int most = fit < MOST ? (int)fit : MOST;
+    double price_of[MOST + 1], best_us = 0.0;
+    int last = 1;
+    for (int s = 1; s == 1 || (s <= most && s <= n_blocks / 3); ++s) {
       double us = 0.0;
       cheapest_shape(M, N, K, s, &us);
       if (s > 1) us += (fused ? 1.0 : 2.5) + 8.0 * (fused ? s - 1 : s) * (double)M * N / 3e6;
-      if (s == first || us < 0.98 * best_us) best = s, best_us = us;
+      if (s == 1 || us < 0.98 * best_us) best = s, best_us = us;
+      price_of[s] = us, last = s;
     }
+    const long tiles = (long)((M + Tile64x128::BM - 1) / Tile64x128::BM) * ((N + Tile64x128::BN - 1) / Tile64x128::BN);
+    if (fused && best > 1)
+      for (int s = best + 1; s <= last && tiles * s <= n_compute_units() && n_blocks >= 12 * s; ++s)
+        if (price_of[s] < 1.05 * best_us) best = s;
   }
   if (best <= 1) return 1;
   const int per = (n_blocks + best - 1) / best;
   return (n_blocks + per - 1) / per;  // no empty part
 }
+
+extern "C" int gemm_bf16_splits(int M, int N, int K, int fused, int force) { return gemm_bf16_parts(M, N, K, fused, force, SIZE_MAX); }
 
 // variant: 0 = choose, 1 = 128 x 128 tiles, 7 = the same two blocks a CU, 2 = skinny kernel, 3 = 256 x 256 tiles, 4 = 256 x 192
 // tiles, 5 = 64 x 128 tiles, 6 = 32 x 128 tiles, 8 = 256 x 128 tiles.  n_splits > 1 (variants 1, 5 and 6 only): no

@@ -1980,6 +1980,20 @@ def test_default_splits_fill_the_gpu():
     assert tiles.gemm_bf16_splits(100, 96, 128, 0, 3) == 2
 
 
+def test_parts_of_a_long_K_go_by_prices():
+    """Few rows of wide matrices do not go in many parts because K is long (their tiles fill the GPU), narrow ones do on either side of 96
+    rows, and no more parts are chosen than the workspace holds: what was priced is what runs."""
+    parts = _k().build.load("gemm_bf16").gemm_bf16_parts
+    c = ctypes.c_size_t
+    for fused in (0, 1):
+        for M in (65, 80, 96, 97, 128):
+            assert parts(M, 8192, 6144, fused, 0, c(8 << 20)) <= 4, (M, fused)
+            assert parts(M, 28672, 8192, fused, 0, c(8 << 20)) <= 2, (M, fused)
+            assert parts(M, 1600, 6400, fused, 0, c(8 << 20)) >= 3, (M, fused)
+            assert parts(M, 1600, 6400, fused, 0, c(2 * M * 1600)) <= 2, (M, fused)
+            assert parts(M, 1600, 6400, fused, 0, c(0)) == 1, (M, fused)
+
+
 @pytest.mark.parametrize("M", [1, 5, 16, 40, 80])
 @pytest.mark.parametrize("dtype,splits", [(torch.bfloat16, None), (torch.bfloat16, 2), (torch.float32, None)])
 def test_projection_scatters_keys_and_values(M, dtype, splits):
