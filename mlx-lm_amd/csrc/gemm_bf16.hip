@@ -763,18 +763,23 @@ static const TilePrice TILE_PRICES[] = {
     {5, Tile64x128::BM, Tile64x128::BN, 2, 3.11, 1.32, 0.363, 0.708, true, 0.49, 0.32, 0.403, 0.403},
     {6, Tile32x128::BM, Tile32x128::BN, 2, 2.83, 1.54, 0.27, 0.516, true, 0.83, 0.202, 0.316, 0.316},
 };
-// Up to 64 rows, what the kernels for few rows leave (row-major weights, a longer K than they hold): no readers.
-static const TilePrice FEW_PRICES[] = {
+// Products that nobody reads ahead for: row-major weights, and up to 64 rows (what the kernels for few rows leave, a longer K than they hold).
+// Fitted to 16 numbers of rows from 20 to 8,000.  us, rows x features x K, row-major, by these and by the prices above: 333 x 4,800 x 1,600 14.3 and 16.7,
+// 150 x 6,400 x 1,600 12.5 and 14.6, 333 x 5,376 x 1,024 10.5 and 11.9, 65 x 10,880 x 2,048 18.0 and 19.7.
+static const TilePrice UNFED_PRICES[] = {
+    {3, Tile256::BM, Tile256::BN, 1, 0.0, 7.78, 1.3, 0.0, false, 0.0, 0.0, 0.0, 0.0},
+    {4, Tile256x192::BM, Tile256x192::BN, 1, 0.0, 7.26, 1.0, 0.0, false, 0.0, 0.0, 0.0, 0.0},
+    {8, Tile256x128::BM, Tile256x128::BN, 1, 0.0, 7.6, 0.7, 0.0, false, 0.0, 0.0, 0.0, 0.0},
     {1, Tile128::BM, Tile128::BN, 1, 0.0, 4.33, 0.49, 0.0, true, 0.0, 0.0, 0.0, 0.0},
     {5, Tile64x128::BM, Tile64x128::BN, 2, 0.52, 2.81, 0.38, 0.77, true, 0.0, 0.0, 0.0, 0.0},
     {6, Tile32x128::BM, Tile32x128::BN, 2, 1.81, 1.98, 0.33, 0.52, true, 0.0, 0.0, 0.0, 0.0},
 };
 
-static double price(const TilePrice& s, int M, int N, int K, int n_splits) {
+static double price(const TilePrice& s, int M, int N, int K, int n_splits, bool packed) {
   const long tiles = (long)((M + s.bm - 1) / s.bm) * ((N + s.bn - 1) / s.bn), cus = n_compute_units(), per_die = cus / N_DIES;
   const long n = ((tiles + N_DIES - 1) / N_DIES * n_splits + per_die - 1) / per_die;  // the busiest CU
   const int k_blocks = ((K + BK - 1) / BK + n_splits - 1) / n_splits;
-  const bool fed = readers_keep_up(s.variant, M, N, n_splits);
+  const bool fed = packed && readers_keep_up(s.variant, M, N, n_splits);
   const double least = (n_splits == 1 && !fed ? s.full_alone : s.full) * (tiles * n_splits < cus ? tiles * n_splits : cus) / cus;
   if (fed) return s.launch + s.fed_tile + k_blocks * (s.fed > least ? s.fed : least);
   if (n == 1) return s.launch + s.tile + k_blocks * (s.kblock > least ? s.kblock : least);
@@ -782,15 +787,15 @@ static double price(const TilePrice& s, int M, int N, int K, int n_splits) {
   return s.launch + (n / 2) * (s.tile + k_blocks * s.pair) + (n % 2) * (s.tile + k_blocks * s.kblock);
 }
 // The cheapest shape for K in so many parts, and its price.
-static int cheapest_shape(int M, int N, int K, int n_splits, double* us) {
+static int cheapest_shape(int M, int N, int K, int n_splits, bool packed, double* us) {
   int variant = 0;
   const auto look = [&](const TilePrice& s) {
     if (n_splits > 1 && !s.splits) return;
-    const double t = price(s, M, N, K, n_splits);
+    const double t = price(s, M, N, K, n_splits, packed);
     if (!variant || t < *us) variant = s.variant, *us = t;
   };
-  if (M <= FEW_ROWS)
-    for (const TilePrice& s : FEW_PRICES) look(s);
+  if (M <= FEW_ROWS || !packed)
+    for (const TilePrice& s : UNFED_PRICES) look(s);
   else
     for (const TilePrice& s : TILE_PRICES) look(s);
   return variant;
@@ -818,7 +823,8 @@ static bool pairs_of_blocks(int M, int N) {
 // of twelve k-blocks or more that all have a unit to themselves may cost 5 % more by these prices: in steps they are level or ahead (GPT-2 XL, us a step, 72 rows of
 // 1,600 x 6,400 in 5 / 6 / 8 parts 2,632 / 2,630 / 2,630, 200 rows in two and four 3,200 and 3,156; large, 260 rows of 1,280 x 5,120 in two and three 2,316 and
 // 2,206), at worst 0.7 % behind (150 rows of 1,600 x 6,400 in four and six 2,887 and 2,908).
-// `force` > 0 asks for that many parts wherever K has them (for tests of small sizes).  `ws_floats`: what the parts' sums have to fit.
+// `force` > 0 asks for that many parts wherever K has them (for tests of small sizes).  `ws_floats`: what the parts' sums
+// have to fit.  (Priced for packed weights; row-major ones, which only direct callers have, go in as many parts, so that both orders give the same bits.)
 extern "C" int gemm_bf16_parts(int M, int N, int K, int fused, int force, size_t ws_floats) {
   if (M < TILE_MIN_ROWS) return 1;
   const int n_blocks = (K + BK - 1) / BK;
@@ -833,7 +839,7 @@ extern "C" int gemm_bf16_parts(int M, int N, int K, int fused, int force, size_t
     int last = 1;
     for (int s = 1; s == 1 || (s <= most && s <= n_blocks / 3); ++s) {
       double us = 0.0;
-      cheapest_shape(M, N, K, s, &us);
+      cheapest_shape(M, N, K, s, true, &us);
       if (s > 1) us += (fused ? 1.0 : 2.5) + 8.0 * (fused ? s - 1 : s) * (double)M * N / 3e6;
       if (s == 1 || us < 0.98 * best_us) best = s, best_us = us;
       price_of[s] = us, last = s;
@@ -849,6 +855,12 @@ extern "C" int gemm_bf16_parts(int M, int N, int K, int fused, int force, size_t
 }
 
 extern "C" int gemm_bf16_splits(int M, int N, int K, int fused, int force) { return gemm_bf16_parts(M, N, K, fused, force, SIZE_MAX); }
+
+// The kernel (`variant` below) for a product with K whole.
+extern "C" int gemm_bf16_shape(int M, int N, int K, int packed) {
+  double us = 0.0;
+  return M < TILE_MIN_ROWS ? 2 : pairs_of_blocks(M, N) ? 7 : cheapest_shape(M, N, K, 1, packed, &us);
+}
 
 // variant: 0 = choose, 1 = 128 x 128 tiles, 7 = the same two blocks a CU, 2 = skinny kernel, 3 = 256 x 256 tiles, 4 = 256 x 192
 // tiles, 5 = 64 x 128 tiles, 6 = 32 x 128 tiles, 8 = 256 x 128 tiles.  n_splits > 1 (variants 1, 5 and 6 only): no
@@ -912,16 +924,13 @@ extern "C" int gemm_bf16_scatter(void* out, const void* A, const void* W, const 
   if (fits_through_buffer((size_t)M * ldo * 4) && fits_through_buffer((size_t)M * N * 4)) p.flags |= FLAG_THROUGH;
   if (n_splits > 1) {
     double us = 0.0;
-    if (variant == 0) variant = cheapest_shape(M, N, K, n_splits, &us);
+    if (variant == 0) variant = cheapest_shape(M, N, K, n_splits, p.w_packed, &us);
     if (variant != 1 && variant != 5 && variant != 6) FAIL("gemm_bf16: only the tiles of 128, 64 and 32 rows by 128 split K");
     if (p.blocks_per_split * (n_splits - 1) >= n_blocks) FAIL("gemm_bf16: %d splits of K=%d leave one empty", n_splits, K);
     if (!ws || ((uintptr_t)ws & 15) || ws_floats < (size_t)n_splits * M * N)
       FAIL("gemm_bf16: %d splits of %d x %d need an aligned workspace of that many floats", n_splits, M, N);
   }
-  if (variant == 0) {
-    double us = 0.0;
-    variant = M < TILE_MIN_ROWS ? 2 : pairs_of_blocks(M, N) ? 7 : cheapest_shape(M, N, K, 1, &us);
-  }
+  if (variant == 0) variant = gemm_bf16_shape(M, N, K, p.w_packed);
   if (variant == 2) {
     if (M > SK_MAXM) FAIL("gemm_bf16: the skinny kernel takes at most %d rows, got %d", SK_MAXM, M);
     dim3 grid((N + 15) / 16), block(256);

@@ -1994,6 +1994,14 @@ def test_parts_of_a_long_K_go_by_prices():
             assert parts(M, 1600, 6400, fused, 0, c(0)) == 1, (M, fused)
 
 
+def test_row_major_weights_are_not_priced_as_read_ahead():
+    """No unit reads row-major weights ahead: tiles that are the cheapest where one does are not chosen for them, nor for few rows."""
+    shape = _k().build.load("gemm_bf16").gemm_bf16_shape
+    assert [shape(*s, 1) for s in ((333, 4800, 1600), (150, 6400, 1600), (333, 5376, 1024))] == [1, 5, 1]  # 128 and 64 x 128, fed
+    assert [shape(*s, 0) for s in ((333, 4800, 1600), (150, 6400, 1600), (333, 5376, 1024))] == [5, 6, 5]  # 64 and 32 x 128
+    assert shape(64, 6400, 1600, 1) == shape(64, 6400, 1600, 0)
+
+
 @pytest.mark.parametrize("M", [1, 5, 16, 40, 80])
 @pytest.mark.parametrize("dtype,splits", [(torch.bfloat16, None), (torch.bfloat16, 2), (torch.float32, None)])
 def test_projection_scatters_keys_and_values(M, dtype, splits):
