@@ -213,6 +213,65 @@ def test_gemm_f32_cut_operands_are_no_further_off(M, N, K):
         assert max(off[5], off[6], off[7]) <= off[1], (name, off)
 
 
+@pytest.mark.parametrize("M,N,K", [(65, 60, 32), (64, 129, 68), (127, 128, 100), (129, 257, 520), (300, 513, 1608)])
+@pytest.mark.parametrize("mode", ["bias", "gelu", "relu2", "accumulate"])
+def test_gemm_f32_cut_operands_epilogues(M, N, K, mode):
+    """What the tiles of cut operands do with their sums, K whole and in parts, output rows whose pieces of four are aligned and not, and what lies
+    beside the rows.  (The sums' error, times the greatest slope of what is applied, and a rounding or two of the result.)"""
+    k = _k()
+    a, w, bias = _rand((M, K), torch.float32, 10), _rand((N, K), torch.float32, 11, 0.1), _rand((N,), torch.float32, 12)
+    old = _rand((M, N), torch.float32, 13)
+    ref = a.double().cpu() @ w.double().cpu().t() + bias.double().cpu()
+    tol = _cut_tolerance(a, w, K) + 2.0**-23 * ref.abs()
+    if mode == "gelu":
+        ref, tol = plain.gelu_tanh(ref), 1.13 * tol + 2.0**-20 * ref.abs()  # (the slope is 1.129 at most; the function itself 9e-7)
+    elif mode == "relu2":
+        ref, tol = torch.relu(ref) ** 2, 2 * (torch.relu(ref) + tol) * tol + 2.0**-23 * ref**2
+    elif mode == "accumulate":
+        ref = ref + old.double().cpu()
+        tol = tol + 2.0**-23 * (ref.abs() + old.double().cpu().abs())
+    for variant in (5, 6, 7):
+        for splits in [None] + [s for s in (2, 3) if s <= (K + 63) // 64]:
+            for pad in (0, 3):
+                wide = torch.full((M, N + pad), 0.5, device=DEV)
+                out = wide[:, :N]
+                out.copy_(old)
+                k.linear(out, a, w, bias, variant=variant, splits=splits, accumulate=mode == "accumulate",
+                         activation={"gelu": "gelu_tanh", "relu2": "relu2"}.get(mode))
+                over = ((out.double().cpu() - ref).abs() - tol).max().item()
+                assert over <= 0, (variant, splits, pad, over)
+                assert (wide[:, N:] == 0.5).all()
+
+
+def test_gemm_f32_cut_operands_gelu():
+    """The GELU of the cut tiles' epilogue over all magnitudes, by products with ones and zeros (of numbers that both halves hold): no further
+    from 64 bits than the other tiles' on any stretch, greatest, mean and 2-norm, and the same for zeros, infinities, NaN and sums beyond
+    every exponential."""
+    k = _k()
+    eye = torch.eye(256, device=DEV)
+
+    def gelu(x, variant):
+        out = torch.empty_like(x)
+        k.linear(out, x, eye, gelu=True, variant=variant)
+        return out
+
+    for lo, hi in ((-12, -5), (-5, -2), (-2, -0.5), (-0.5, 0.5), (0.5, 3), (3, 20)):
+        m, e = torch.frexp(torch.linspace(lo, hi, 1 << 18, device=DEV))
+        x = torch.ldexp((m * 2**20).round() / 2**20, e).view(-1, 256)
+        ref = plain.gelu_tanh(x.double().cpu())
+        err = {v: (gelu(x, v).double().cpu() - ref).abs() for v in (1, 5)}
+        for what in (lambda d: (d / ref.abs().clamp_min(1e-30)).max(), lambda d: (d / ref.abs().clamp_min(1e-30)).mean(), lambda d: d.norm()):
+            assert what(err[5]) <= 1.01 * what(err[1]), (lo, hi, what(err[5]).item(), what(err[1]).item())
+    inf = float("inf")
+    special = [inf, -inf, float("nan"), 0.0, -0.0, 1e3, -1e3, 1e30, -1e30, 3e38, -3e38, -14.0, -20.0, 1e-30, -1e-30]
+    x = torch.zeros(70, 256, device=DEV)
+    for i, v in enumerate(special):
+        x[i, i] = v
+    got, want = gelu(x, 5), gelu(x, 1)
+    at = torch.arange(len(special), device=DEV)
+    assert torch.equal(got[at, at].nan_to_num(7.0), want[at, at].nan_to_num(7.0)) and got[2, 2].isnan() and got[1, 1].isnan() and got[0, 0] == inf
+
+
 def test_gemm_f32_weights_that_are_changed_in_place():
     """Weights that were laid out and multiplied with are read as they are now: features that shrink or grow afterwards, by a view that
     counts no version, give the bits that a copy of them gives."""
