@@ -700,10 +700,15 @@ static void idle_units(int M, int N, int n_splits, int* idle, double* columns) {
 }
 
 // Compute units a die and part of K that read the weights ahead (0: none do).  Too few of them fall behind the tiles and are still
-// reading when those are done: 333 x 4,800 x 1,600 in tiles of 64 x 128 (three a die for five columns) 14.0 -> 14.5 us, 536 x 1,600 x 1,600 in
-// two parts (one for two) 8.8 -> 9.6.  Tiles of 128 x 128 want nearly two a column (536 x 4,800 x 1,600, eight for five, 15.0 -> 15.5; 470 x 6,400 x
-// 1,600, thirteen for six, 16.7 -> 14.4) and gain nothing in parts of K (25 us with 24.6 for 536 x 1,600 x 6,400 in two); the widest were
-// level or behind (1,000 x 6,400 x 1,600 in 256 x 128 24.7 -> 25.7).  More than eight (twelve) take from the tiles: 333 x 6,400 x 1,600 15.2 with twelve.
+// reading when those are done: 240 x 6,784 x 1,600 in tiles of 64 x 128 (five a die for seven columns) 14.2 -> 14.8 us, 536 x 1,600 x 1,600 in
+// two parts (one for two) 8.8 -> 9.6; 240 x 6,400 x 1,600 (seven for six) 14.2 -> 12.0.  Tiles of 32 x 128 gain a little from any.  Tiles of 128 x 128 want one a column, of
+// at most eight (480 x 6,400 x 1,600, seven for six, 17.0 -> 14.9, 352 x 7,680 x 1,600, nine for eight, 17.3 -> 15.0; 224 x 8,704 x 1,600, fifteen for nine of which eight are read,
+// 17.3 -> 18.4, 96 x 10,880 x 1,600 17.8 -> 18.7), but where the last row of tiles is nearly empty they have less to gain and to spare (390 x 6,400 x
+// 1,600 15.0 -> 15.4, 520 x 4,800 x 1,600, eight for five, 15.0 -> 15.2), so the line lies at nearly two a column: with one, prompts of 510 and 640 tokens of GPT-2 XL would take
+// 1.4 and 0.6 % less (4,284 -> 4,230, 4,860 -> 4,833 us), of 390, 520 and 536 1.1, 0.9 and 0.6 % more, of large 520 2 % more and 640 1.2 % less; with one and
+// a half 520 and 536 0.7 % more and 640 0.5 % less.  2,048 x 1,600 x 1,600 (1.85 a column) 16.5 -> 15.5, x 6,400 53.5 -> 48.2.  They
+// gain nothing in parts of K (25 us with 24.6 for 536 x 1,600 x 6,400 in two); the widest were
+// level or behind (1,000 x 6,400 x 1,600 in 256 x 128 24.7 -> 25.7).  More than eight (twelve) take from the tiles: 333 x 6,400 x 1,600 15.2 with twelve, 14.1 with eight.
 static int readers_of(int variant, int M, int N, int n_splits, bool packed) {
   int idle = 0;
   double columns = 0.0;
@@ -716,6 +721,7 @@ static int readers_of(int variant, int M, int N, int n_splits, bool packed) {
     idle_units<Tile32x128>(M, N, n_splits, &idle, &columns);
   else
     return 0;
+  if (variant == 1 && columns > 8.0) return 0;
   const double enough = variant == 1 ? 1.83 : 0.9;
   const int most = variant == 1 ? 8 : 12;
   return idle < 1 || idle < enough * columns ? 0 : idle < most ? idle : most;
@@ -725,7 +731,7 @@ static int readers_of(int variant, int M, int N, int n_splits, bool packed) {
 // for eleven, 0.42 us a k-block; 160 x 8,192 x 2,048, eight for eight, 0.35).  Of 32 rows, which take half as long: from five readers for four columns on
 // (65 x 8,192 x 6,144, eight for eight, 0.31; 100 x 6,144 x 2,048, eight for six, 0.25; 65 x 6,400 x 1,600, thirteen for six, 0.23); with three or fewer, as parts
 // of K leave them, from nine for four on (65 x 1,600 x 6,400 in four parts, three for five thirds, 0.31; 100 x 1,280 x 5,120 in four, three for five quarters, 0.21) or
-// two for one (80 x 768 x 3,072 in six, 0.22).  Of 128 rows: up to the columns that the most readers have (160 x 8,192 x 2,048, 0.39; 65 x 10,880 x 2,048, eight for eleven, 0.48).
+// two for one (80 x 768 x 3,072 in six, 0.22).
 static bool readers_keep_up(int variant, int M, int N, int n_splits) {
   if (!readers_of(variant, M, N, n_splits, true)) return false;
   int idle = 0;
@@ -738,8 +744,7 @@ static bool readers_keep_up(int variant, int M, int N, int n_splits) {
     idle_units<Tile32x128>(M, N, n_splits, &idle, &columns);
     return idle >= (idle > 3 ? 1.25 : columns > 1.0 ? 2.25 : 2.0) * columns;
   }
-  idle_units<Tile128>(M, N, n_splits, &idle, &columns);
-  return columns <= 10.0;
+  return true;
 }
 
 // What a shape costs, in microseconds: `launch` once, `tile` for each round of tiles on a CU and `kblock` for each k-block of it, `pair`
