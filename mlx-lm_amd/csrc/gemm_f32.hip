@@ -567,9 +567,8 @@ __global__ __launch_bounds__(S::THREADS, 2) void gemm_f32_cut_kernel(GemmArgs p)
   const int ldo = parts ? p.N : p.ldo;
   const bool vec = ldo % 4 == 0 && ((uintptr_t)out & 15) == 0;
   const bool add = p.flags & FLAG_ACCUMULATE;
-  // (through to memory, as far as a buffer reaches: 1,050 x 1,280 x 5,120 in three parts 114.8 -> 113.5 us, two parts of
-  // 1,280 columns 34.7 -> 33.9, the wide ones level)
-  const __amdgpu_buffer_rsrc_t out_buf = through_buffer(out, ((size_t)(p.M - 1) * ldo + p.N) * 4);
+  // (Stores that leave their lines in the caches: through to memory, as the other tiles' are, a prompt of 1,000 tokens of GPT-2 large in float32 took
+  // 11,170 us instead of 10,770, of XL 20,850 instead of 19,970; 1,050 x 5,120 x 1,280 alone 75.2 and 71.9.)
 #pragma unroll
   for (int j = 0; j < TN; ++j) {
     const int nt = n0 + (wn * TN + j) * 32 + 4 * hi;
@@ -608,10 +607,7 @@ __global__ __launch_bounds__(S::THREADS, 2) void gemm_f32_cut_kernel(GemmArgs p)
       for (int g = 0; g < 4; ++g) {
         const int n = nt + 8 * g;
         if (vec && n + 4 <= p.N) {
-          if (p.through)
-            store_through(out_buf, (uint32_t)(((size_t)m * ldo + n) * 4), __builtin_bit_cast(u32x4_t, v[g]));
-          else
-            *(f32x4_t*)(out + (size_t)m * ldo + n) = v[g];
+          *(f32x4_t*)(out + (size_t)m * ldo + n) = v[g];
         } else {
 #pragma unroll
           for (int r = 0; r < 4; ++r)
@@ -948,7 +944,6 @@ extern "C" int gemm_f32_scatter(void* out, const void* A, const void* W, const f
         c.M = 0, c.N = N - n < CUT_BLOCKS ? N - n : CUT_BLOCKS, c.W = p.W + (size_t)n * ldw, c.scales = scales + rows + n;
         hipLaunchKernelGGL(cut_rows_kernel, dim3((unsigned)c.N), dim3(256), 0, stream, c);
       }
-      p.through = fits_through_buffer((size_t)p.M * (n_splits > 1 ? N : ldo) * 4);
       launch(p, variant, stream);
       p.A += (size_t)p.M * lda, p.out += (size_t)p.M * ldo;
       if (n_splits > 1) p.ws += (size_t)p.M * N;
