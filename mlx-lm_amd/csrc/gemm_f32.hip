@@ -741,8 +741,9 @@ DEFINE_LAST_ERROR(mlxlm_last_error)
 // K in 1 to 8 parts, the choice is within 0.7 % of the best on average and 7 % at worst (1.7 % and 13 % with every tile
 // at the same rate).
 // Tiles of cut operands: `base` once, `tile` for each round of blocks that share a CU (`per_cu` of them), each 64 columns of K
-// as many blocks as then share the CU (`chunk[0]` one, `chunk[1]` two, `chunk[2]` three), and the launch ahead that cuts the rows. Fitted to the times of
-// as many rows from 65 on and 15 matrices of widths 768 to 1,600.
+// as many blocks as then share the CU (`chunk[0]` one, `chunk[1]` two, `chunk[2]` three), and the launch ahead that cuts the rows.  With them the choice among
+// all shapes and parts is within 2.5 % of the best on average, for as many rows from 65 on and 15 matrices of widths 768 to 1,600.  (Prices fitted to today's
+// kernels are within 1.1 %, but take K in fewer parts, longer sums: GPT-2 large, 1,050 tokens, logits off by 6.7e-7 instead of 6.1e-7.)
 struct F32Price {
   int variant, bm, bn;
   double rate;  // (0: cut operands)
