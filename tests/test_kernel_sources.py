@@ -23,9 +23,16 @@ def _kernels(text):
         yield name, text[start:at]
 
 
+def _asks_without_wait(body):
+    """The places in a kernel's body that ask for copies into LDS without a wait for all of them ahead of the next way out."""
+    outs = [m.start() for m in re.finditer(r"\breturn\b", body)] + [len(body)]
+    asks = [m.start() for m in re.finditer(r"\bask\(", body)]
+    return [at for at in asks if "copies_arrived<0>()" not in body[at : next(o for o in outs if o > at)]]
+
+
 def test_copies_into_lds_are_waited_for_before_a_wave_ends():
-    """A kernel that asks for copies beyond the end of its ring (``lds_copy.h``) waits for all of them behind its loop:
-    LDS that another block has by then must not be written."""
+    """A kernel that asks for copies beyond the end of its ring (``lds_copy.h``) waits for all of them behind its loop, on each
+    way out (waves that only copy have one of their own): LDS that another block has by then must not be written."""
     seen = []
     for path in sorted(glob.glob(os.path.join(CSRC, "*.hip"))):
         with open(path) as f:
@@ -33,6 +40,8 @@ def test_copies_into_lds_are_waited_for_before_a_wave_ends():
         for name, body in _kernels(text):
             if "copy16_to_lds(" in body:
                 seen.append(name)
-                last = body.rindex("ask(")
-                assert "copies_arrived<0>()" in body[last:], (os.path.basename(path), name)
+                assert not _asks_without_wait(body), (os.path.basename(path), name)
+                # each of the waits is needed
+                for m in re.finditer(r"copies_arrived<0>\(\);", body):
+                    assert _asks_without_wait(body[: m.start()] + body[m.end() :]), (name, m.start())
     assert {"gemm_bf16_tile_kernel", "gemm_f32_tile_kernel", "gemm_f32_cut_kernel"} <= set(seen)
