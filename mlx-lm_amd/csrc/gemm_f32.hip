@@ -242,7 +242,8 @@ __global__ __launch_bounds__(S::THREADS, 2) void gemm_f32_tile_kernel(GemmArgs p
 //
 // cut_rows_kernel finds the powers and lays the rows out cut, a row's octet of columns as 16 bytes of h and 16 of l where its 32
 // bytes were, so that a tile copies both operands alike; the features' are found beside them, by each call: what is kept is
-// wrong as soon as a caller changes its weights in place.  (No time: the product finds the weights in the last-level cache then.)  The weights, which would
+// wrong as soon as a caller changes its weights in place.  (The product finds the weights in the last-level cache then: from 600 rows on it takes no time, at 120
+// to 200 rows 1 to 4 % of a step, which the prices' last term leaves to other tiles where those are as good.)  The weights, which would
 // take as much memory again, are cut in registers, 16 columns ahead of their products (28 vector instructions for 8 columns of 32 features, between
 // a wave's products); six products of three bfloat16 numbers each, exact without scales, took 106 us instead of 68 for 1,050 x 5,120 x 1,280.
 //
@@ -317,9 +318,11 @@ __device__ __forceinline__ float power_of_2(int e) { return __uint_as_float((uin
 #define DOUBT_A_VALUE 4.f
 
 // Ahead of the products: the rows' greatest values, whose exponents say what a row is scaled by (so that its greatest
-// value lies from 2^14 up to 2^15), and A's rows scaled and cut.  A block a row, which stays in registers up to 8,192 columns: first A's, then W's.  A cut row has the place of the
-// row itself: where eight floats were lie eight high halves and eight low ones, up to whole steps of 32 columns.  (A wave a row, read
-// twice: 1,050 x 5,120 12.5 us; 10.2 so, 2,048 x 6,400 in 6 us less, 1,280 columns 5.4 either way.)
+// value lies from 2^14 up to 2^15), how many of their values are small, and A's rows scaled and cut.  A's first, a block a row, which stays in registers up to 8,192 columns.  A cut row has
+// the place of the row itself: where eight floats were lie eight high halves and eight low ones, up to whole steps of 32 columns.  (A wave a row, read
+// twice: 1,050 x 5,120 12.5 us; 10.2 so, 2,048 x 6,400 in 6 us less, 1,280 columns 5.4 either way.)  Then the features, a wave each, read once but for those that have
+// small values: they come from memory, which is what bounds this.  (Features a block each: with the product 200 x 4,800 x 1,600 36.2 us, 35.0 so, 1,050 x 1,280 x 1,280
+// in two parts 29.7 and 29.0, prompts of 400 and 1,000 tokens of GPT-2 large 6,130 and 5,965, 10,270 and 10,150.)
 struct CutArgs {
   const float* A;
   const float* W;
@@ -327,12 +330,52 @@ struct CutArgs {
   u32x4_t* cut;
   RowScale* scales;  // [M], then [N]
 };
+// How a row is scaled whose greatest value has these bits (without the sign).
+__device__ __forceinline__ int scale_up(uint32_t most) {
+  const int e = (int)(most >> 23);
+  return most == 0 || e == 255 ? 0 : min(14 + 127 - e, 126);
+}
+// A wave a feature.
+__device__ __forceinline__ void scale_of_feature(const CutArgs& p, int n, int lane) {
+  if (n >= p.N) return;
+  const float* from = p.W + (size_t)n * p.ldw;
+  constexpr int HELD = 8;
+  auto each = [&](auto see) __attribute__((always_inline)) {
+    for (int k0 = 4 * lane; k0 < p.K; k0 += 256 * HELD) {
+      f32x4_t v[HELD];
+#pragma unroll
+      for (int i = 0; i < HELD; ++i) {
+        v[i] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        if (k0 + 256 * i < p.K) v[i] = *(const f32x4_t*)(from + k0 + 256 * i);
+      }
+#pragma unroll
+      for (int i = 0; i < HELD; ++i)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) see(v[i][c]);
+    }
+  };
+  uint32_t most = 0, least = ~0u;  // (the least value that is not zero, less one)
+  each([&](float v) __attribute__((always_inline)) {
+    const uint32_t bits = __float_as_uint(v) & 0x7fffffffu;
+    most = max(most, bits), least = min(least, bits - 1u);
+  });
+#pragma unroll
+  for (int d = 32; d; d >>= 1) most = max(most, (uint32_t)__shfl_xor((int)most, d, 64)), least = min(least, (uint32_t)__shfl_xor((int)least, d, 64));
+  const int up = scale_up(most);
+  const float scale = power_of_2(up);
+  int small = 0;
+  if (least != ~0u && __uint_as_float(least + 1u) * scale < LEAST_WHOLE)  // (hardly ever)
+    each([&](float v) __attribute__((always_inline)) { small += v != 0.f && fabsf(v * scale) < LEAST_WHOLE; });
+#pragma unroll
+  for (int d = 32; d; d >>= 1) small += __shfl_xor(small, d, 64);
+  if (lane == 0) p.scales[p.M + n] = RowScale{up, most == 0 ? -INFINITY : DOUBT_A_VALUE * (float)small};
+}
 __global__ __launch_bounds__(256) void cut_rows_kernel(CutArgs p) {
   __shared__ uint32_t wave_most[4];
   __shared__ int n_small;
   const int row = blockIdx.x, tid = threadIdx.x;
-  const bool is_a = row < p.M;
-  const float* from = is_a ? p.A + (size_t)row * p.lda : p.W + (size_t)(row - p.M) * p.ldw;
+  if (row >= p.M) return scale_of_feature(p, (row - p.M) * 4 + (tid >> 6), tid & 63);
+  const float* from = p.A + (size_t)row * p.lda;
   constexpr int HELD = 4, CHUNK = 256 * 8 * HELD;
   f32x4_t v[HELD][2];
   auto load = [&](int k0) __attribute__((always_inline)) {
@@ -362,8 +405,7 @@ __global__ __launch_bounds__(256) void cut_rows_kernel(CutArgs p) {
   if (tid == 0) n_small = 0;
   __syncthreads();
   most = max(max(wave_most[0], wave_most[1]), max(wave_most[2], wave_most[3]));
-  const int e = (int)(most >> 23);
-  const int up = most == 0 || e == 255 ? 0 : min(14 + 127 - e, 126);
+  const int up = scale_up(most);
   const float scale = power_of_2(up);
   u32x4_t* to = p.cut + (size_t)row * (p.ldc / 4);
   int small = 0;
@@ -372,12 +414,12 @@ __global__ __launch_bounds__(256) void cut_rows_kernel(CutArgs p) {
 #pragma unroll
     for (int i = 0; i < HELD; ++i) {
       const int k = k0 + (tid + 256 * i) * 8;
+      if (k0 + 2048 * i >= p.ldc) break;
       if (k >= p.ldc) continue;
 #pragma unroll
       for (int h = 0; h < 2; ++h)
 #pragma unroll
         for (int c = 0; c < 4; ++c) small += v[i][h][c] != 0.f && fabsf(v[i][h][c] * scale) < LEAST_WHOLE;
-      if (!is_a) continue;
       const Cut c = cut(v[i][0], v[i][1], scale);
       to[k / 4] = c.high, to[k / 4 + 1] = c.low;
     }
@@ -765,7 +807,7 @@ static double price(const F32Price& s, int M, int N, int K, int n_splits) {
   if (!is_cut(s.variant)) return 4.0 + (n == 1 ? 1.2 : 1.0) * n * chunks * (2.5e-4 * s.rate * s.bm * s.bn);
   const long full = n / s.per_cu, left = n % s.per_cu;
   return s.base + s.tile * (full + (left ? 1 : 0)) + chunks * (full * s.chunk[s.per_cu - 1] + (left ? s.chunk[left - 1] : 0.0)) +
-         2.3e-6 * M * K;
+         (2.3e-6 * M + 0.1e-6 * N) * K;
 }
 static int cheapest_shape(int M, int N, int K, int n_splits, double* us, bool cuts = true) {
   int variant = 0;
@@ -940,10 +982,10 @@ extern "C" int gemm_f32_scatter(void* out, const void* A, const void* W, const f
       p.M = M - m < rows ? M - m : rows;
       // (the features' scales lie behind those of the first rows, which are as many as any that follow)
       CutArgs c = {p.A, p.W, p.M, m ? 0 : N < CUT_BLOCKS ? N : CUT_BLOCKS, K, lda, ldw, p.ldc, (u32x4_t*)room, scales};
-      hipLaunchKernelGGL(cut_rows_kernel, dim3((unsigned)(c.M + c.N)), dim3(256), 0, stream, c);
+      hipLaunchKernelGGL(cut_rows_kernel, dim3((unsigned)(c.M + (c.N + 3) / 4)), dim3(256), 0, stream, c);
       for (int n = c.N; m == 0 && n < N; n += c.N) {
         c.M = 0, c.N = N - n < CUT_BLOCKS ? N - n : CUT_BLOCKS, c.W = p.W + (size_t)n * ldw, c.scales = scales + rows + n;
-        hipLaunchKernelGGL(cut_rows_kernel, dim3((unsigned)c.N), dim3(256), 0, stream, c);
+        hipLaunchKernelGGL(cut_rows_kernel, dim3((unsigned)((c.N + 3) / 4)), dim3(256), 0, stream, c);
       }
       launch(p, variant, stream);
       p.A += (size_t)p.M * lda, p.out += (size_t)p.M * ldo;
