@@ -333,7 +333,7 @@ struct CutArgs {
 // How a row is scaled whose greatest value has these bits (without the sign).
 __device__ __forceinline__ int scale_up(uint32_t most) {
   const int e = (int)(most >> 23);
-  return most == 0 || e == 255 ? 0 : min(14 + 127 - e, 126);
+  return most == 0 || e == 255 ? 0 : min(14 + 127 - e, 115);  // (LOW_UP times the power is a float too)
 }
 // A wave a feature.
 __device__ __forceinline__ void scale_of_feature(const CutArgs& p, int n, int lane) {
@@ -475,6 +475,7 @@ __global__ __launch_bounds__(S::THREADS, 2) void gemm_f32_cut_kernel(GemmArgs p)
   };
 
   static_assert(BM + BN <= S::THREADS, "a scale a thread");
+  // (read behind the first step's wait and barrier)
   if ((int)threadIdx.x < BM + BN) {
     const int n = n0 + (int)threadIdx.x - BM;
     RowScale s = {0, -INFINITY};

@@ -185,7 +185,7 @@ def test_gemm_f32_rows_of_wide_range(K):
     both_a, both_w = ones.clone(), none.clone()
     both_a[:, at + 1], both_w[:, at + 1] = 0.0, great[0] * 2.0**40
     cases = {"rows": (ones, none), "tiny": (ones, tiny), "features": (none, ones), "both": (both_a, both_w),
-             "fall": (a * fall, w * fall.flip(0)), "small rows": (a * 1e-38, w * fall * 1e3)}
+             "fall": (a * fall, w * fall.flip(0)), "small rows": (a * 1e-38, w * fall * 1e3), "small": (a * 1e-33, w * 1e-4)}
     for name, (a, w) in cases.items():
         a, w = a.contiguous(), w.contiguous()
         ref, tol = (a.double() @ w.double().t().contiguous()).cpu(), _cut_tolerance(a, w, K)
